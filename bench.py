@@ -235,7 +235,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
     model.synchronize()
     load_s = time.time() - t0
 
-    # ---- warm-up (also captures the step graph; the events are recorded around it too, so that creating them and
+    # ---- warm-up (the events are recorded around it too, so that creating them and
     # recording for the first time — 30 us of host time — is not part of the timed region), then the timed region
     model.stream_mark(0)
     model.run(warmup)
@@ -258,7 +258,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
         data = model.neuron_populations[p.name].spike_recording_data
         rates[p.name] = round(sum(len(ids) for _, ids in data) / batch / p.n / ((warmup + steps) * net.dt / 1000.0), 3)
 
-    # ---- per-kernel durations: the same graph replay with HIP event nodes between the kernels of every step
+    # ---- per-kernel durations: the same steps with HIP events between the kernels of every step
     # (events on the runner's stream; durations are those of back-to-back execution)
     roofline = None
     info = model.runner_info()
@@ -284,8 +284,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
                         "us_per_step": round(region_s / steps * 1e6, 3),
                         "avg_launch_us_one_step_per_launch": round(st["step_seconds"] / max(1, st["step_launches"]) * 1e6, 3) if st["step_launches"] else None}
         elif info["single_launch_step"]:
-            # the timed region consists of this kernel only (one launch per step, back to back inside the replayed
-            # graphs, plus one 1-thread node per 100 steps), so HIP events around the region give its average duration
+            # the timed region consists of this kernel only (one launch per step, back to back), so HIP events around the region give its average duration
             avg_s = region_s / steps
             ev_per_launch = events / steps
             achieved = (ev_per_launch * bpe + neuron_bytes) / avg_s / 1e9
@@ -377,7 +376,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
                   "events_per_step": round(ev_s / args.steady_steps, 1),
                   "wall_s_per_sim_s": round(wall_s / (args.steady_steps * net.dt / 1000.0), 4),
                   "roofline": {"bound": "hbm", "kernel": ("residentKernel (one launch for all steps of the block)" if info["resident_plan"] else
-                                                          "all kernels of the block's steps (hipGraph replay)"),
+                                                          "all kernels of the block's steps"),
                                "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 6),
                                "avg_launch_us": round(region * 1e6, 3), "us_per_step": round(region / args.steady_steps * 1e6, 3),
                                "bytes_per_event": bpe, "events_per_launch": ev_s, "neuron_bytes_per_launch": nbytes * args.steady_steps, "traffic": None}}
@@ -451,7 +450,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": label, "neurons": num_neurons, "synapses": num_synapses, "dt_ms": net.dt, "seed": net.seed,
                    "stepping": ("resident plan: one launch for all timed steps, state in registers/LDS" if info["resident_plan"] else
-                                "hipGraph replay, 100 steps per graph, " + ("1 launch per step" if (info["single_launch_step"] or info["conv_step_in_one_launch"]) else
+                                "step by step, " + ("1 launch per step" if (info["single_launch_step"] or info["conv_step_in_one_launch"]) else
                                                                            "2 launches per step (synaptic kernels combined)" if (info["combined_synapse_launch"] or info["conv_on_matrix_cores"]) else
                                                                            "2-3 launches per step"))},
         "gsop_per_s": round(events / wall / 1e9, 4),
@@ -479,7 +478,7 @@ def main():
     ap.add_argument("--reference-steps", type=int, default=2000,
                     help="steps of the extra CPU leg on the reference's own SingleThreadedCPU backend (oracle/_ref/ref_driver, "
                          "only where that prebuilt driver exists; 0 disables)")
-    ap.add_argument("--profile-steps", type=int, default=2000, help="extra steps replayed with HIP event nodes around every kernel (multiple of 100)")
+    ap.add_argument("--profile-steps", type=int, default=2000, help="extra steps with HIP events around every kernel")
     ap.add_argument("--steady-steps", type=int, default=10000,
                     help="runs of fewer than 1000 timed steps: steps of the `steady_state` block that follows in the same process (0 disables)")
     ap.add_argument("--steady-warmup", type=int, default=2000, help="untimed steps before the `steady_state` block")

@@ -1,6 +1,6 @@
 // MI355X (gfx950) device layer for GeNN's per-timestep hot path: kernels + C ABI.
 //
-// This file holds the runner (launch plans, graph capture, the C entry points); the kernels live in the headers it
+// This file holds the runner (launch plans, the C entry points); the kernels live in the headers it
 // includes: genn_mi355x_device.h (descriptor tables, helpers), genn_mi355x_synapse_kernels.h, genn_mi355x_neuron_kernels.h,
 // genn_mi355x_resident_kernels.h.
 //
@@ -62,7 +62,6 @@ struct gennmi_runner
     uint32_t neuronBlocks = 0, preBlocks = 0, postBlocks = 0;
     unsigned long long *dAgg = nullptr; uint32_t *dError = nullptr; unsigned long long *dEvents = nullptr;
     uint32_t *hError = nullptr;     // the error flag: a pinned host word; dError is the same word's device address
-    StepState *dState = nullptr;
     unsigned long long epoch = 0;       // completed steps (host mirror)
     bool synapsesDone = false;          // updateSynapses ran for the current step
     bool fusedStep = false;             // zero-delay synapses are delivered by the neuron update; one launch per step
@@ -110,8 +109,6 @@ struct gennmi_runner
     uint32_t *dOrderedBitmaps = nullptr; size_t orderedBitmapWords = 0;
     std::vector<void*> orderedOwned;
     bool scatterNeeded = true;          // some presynaptic group still goes through presynapticUpdateKernel
-    // graph
-    hipGraphExec_t graphExec = nullptr; unsigned long long graphSteps = 0;
     // timing
     bool timing = false;
     double neuronTime = 0, preTime = 0, postTime = 0;
@@ -491,8 +488,6 @@ int gennmi_runner_create(gennmi_runner **runner, float dt, uint32_t batchSize)
     HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&r->dError), r->hError, 0));
     HIP_TRY(hipMalloc(&r->dEvents, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
     HIP_TRY(hipMemset(r->dEvents, 0, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
-    HIP_TRY(hipMalloc(&r->dState, sizeof(StepState)));
-    HIP_TRY(hipMemset(r->dState, 0, sizeof(StepState)));
     {
         std::lock_guard<std::mutex> lock(g_runnersMutex);
         g_runners.push_back(r);
@@ -510,7 +505,6 @@ int gennmi_runner_destroy(gennmi_runner *r)
         g_runners.erase(std::remove(g_runners.begin(), g_runners.end(), r), g_runners.end());
     }
     hipStreamSynchronize(r->stream);
-    if(r->graphExec) { hipGraphExecDestroy(r->graphExec); }
     for(hipEvent_t e : r->eventPool) { hipEventDestroy(e); }
     for(hipEvent_t e : r->marks) { if(e) { hipEventDestroy(e); } }
     for(void *q : r->owned) { hipFree(q); }
@@ -518,7 +512,7 @@ int gennmi_runner_destroy(gennmi_runner *r)
     for(void *q : r->orderedOwned) { hipFree(q); }
     hipFree(r->dOrderedSources); hipFree(r->dOrderedBitmaps);
     hipFree(r->dTile); hipFree(r->dConvTile);
-    hipFree(r->dNeuron); hipFree(r->dPre); hipFree(r->dPost); hipFree(r->dDense); hipFree(r->dProc); hipFree(r->dAgg); if(r->hError) { hipHostFree(r->hError); } hipFree(r->dEvents); hipFree(r->dState);
+    hipFree(r->dNeuron); hipFree(r->dPre); hipFree(r->dPost); hipFree(r->dDense); hipFree(r->dProc); hipFree(r->dAgg); if(r->hError) { hipHostFree(r->hError); } hipFree(r->dEvents);
     hipStreamDestroy(r->stream);
     delete r;
     return GENNMI_OK;
@@ -1147,9 +1141,6 @@ static int refreshTables(gennmi_runner *r)
         HIP_TRY(hipMemcpy(r->dPre, preTable.data(), preTable.size() * sizeof(PreGroupDev), hipMemcpyHostToDevice));
     }
     if(r->ordered) {
-        // the gather kernels receive their column views by value, so a captured step graph holds the addresses of the views
-        // just freed: it is captured again on the next replay
-        if(r->graphExec) { HIP_TRY(hipGraphExecDestroy(r->graphExec)); r->graphExec = nullptr; r->graphSteps = 0; }
         const int rc = buildOrderedViews(r);
         if(rc) { return rc; }
     }
@@ -1833,15 +1824,6 @@ static int launchConvStep(gennmi_runner *r, const StepArgs &a)
     return GENNMI_OK;
 }
 
-// one whole timestep: a single launch where the runner allows it, else synapse kernels then the neuron kernel
-static int launchStep(gennmi_runner *r, const StepArgs &a)
-{
-    if(r->fusedStep) { return launchFusedStep(r, a); }
-    if(r->convStep) { return launchConvStep(r, a); }
-    const int rc = launchSynapses(r, a, false);
-    return rc ? rc : launchNeurons(r, a, false);
-}
-
 static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed)
 {
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1862,8 +1844,7 @@ int gennmi_update_synapses(gennmi_runner *r, float t)
     if(r->failed) { return fail(GENNMI_ESTATE, "update_synapses: an earlier queued step of this runner failed, the runner cannot continue"); }
     FLUSH_QUEUED();
     { const int rc = refreshTables(r); if(rc) { return rc; } }
-    StepArgs a{};
-    a.base = nullptr; a.epoch = r->epoch; a.t = t; a.recordingTimestep = 0;
+    const StepArgs a{r->epoch, t, 0u};
     const int rc = launchSynapses(r, a, r->timing);
     if(rc) { return rc; }
     r->synapsesDone = true;
@@ -1876,8 +1857,7 @@ int gennmi_update_neurons(gennmi_runner *r, float t, uint32_t recordingTimestep)
     if(r->failed) { return fail(GENNMI_ESTATE, "update_neurons: an earlier queued step of this runner failed, the runner cannot continue"); }
     FLUSH_QUEUED();
     { const int rc = refreshSpikeSources(r); if(rc) { return rc; } }
-    StepArgs a{};
-    a.base = nullptr; a.epoch = r->epoch; a.t = t; a.recordingTimestep = recordingTimestep;
+    const StepArgs a{r->epoch, t, recordingTimestep};
     const int rc = launchNeurons(r, a, r->timing);
     if(rc) { return rc; }
     r->epoch++;
@@ -1897,9 +1877,8 @@ int gennmi_step_time(gennmi_runner *r, unsigned long long timestep, unsigned lon
 // one step, launched now
 static int stepNow(gennmi_runner *r, float t, uint32_t recordingTimestep)
 {
+    const StepArgs a{r->epoch, t, recordingTimestep};
     if(r->fusedStep || r->convStep) {
-        StepArgs a{};
-        a.base = nullptr; a.epoch = r->epoch; a.t = t; a.recordingTimestep = recordingTimestep;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if(r->timing) {
             if(r->pending.size() >= 2048) { const int rc = drainTimers(r); if(rc) { return rc; } }
@@ -1911,9 +1890,11 @@ static int stepNow(gennmi_runner *r, float t, uint32_t recordingTimestep)
         r->epoch++;
         return GENNMI_OK;
     }
-    const int rc = gennmi_update_synapses(r, t);
-    if(rc) { return rc; }
-    return gennmi_update_neurons(r, t, recordingTimestep);
+    { const int rc = launchSynapses(r, a, r->timing); if(rc) { return rc; } }
+    { const int rc = launchNeurons(r, a, r->timing); if(rc) { return rc; } }
+    r->epoch++;
+    r->synapsesDone = false;
+    return GENNMI_OK;
 }
 
 // Executes the steps a runner has queued: runs of steps whose recording rows follow one another (or that all record into row
@@ -1987,55 +1968,16 @@ int gennmi_run_steps(gennmi_runner *r, unsigned long long timestep, unsigned lon
     FLUSH_QUEUED();
     { const int rc = refreshSpikeSources(r); if(rc) { return rc; } }
     { const int rc = refreshTables(r); if(rc) { return rc; } }
-    constexpr unsigned long long CHUNK = 100;
-    // (the resident plan takes time, epoch and recording length as kernel arguments: no step state on the device to refresh,
-    // and so no copy and no wait for it ahead of the launch — 20 us of a call that launches 20 steps, and, between two
-    // events recorded around the call, 20 us that are not the kernel's)
     if(r->resident && !r->timing && numSteps >= 4) { return launchResident(r, timestep, numSteps, numRecordingTimesteps); }
-    const StepState hs{timestep, r->epoch, numRecordingTimesteps};
-    HIP_TRY(hipMemcpyAsync(r->dState, &hs, sizeof(hs), hipMemcpyHostToDevice, r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));   // hs lives on this stack frame
-    unsigned long long done = 0;
-    if(r->timing) {
-        // individually launched steps with HIP events around every kernel; nothing waits until the statistics
-        // are read, so the device stays busy and the clocks stay up
-        for(; done < numSteps; done++) {
-            const int rc = gennmi_step_time(r, timestep + done, numRecordingTimesteps);
-            if(rc) { return rc; }
-        }
-        return GENNMI_OK;
-    }
-    while(numSteps - done >= CHUNK) {
-        if(!r->graphExec) {
-            hipGraph_t graph;
-            HIP_TRY(hipStreamBeginCapture(r->stream, hipStreamCaptureModeThreadLocal));
-            int rc = GENNMI_OK;
-            for(unsigned long long k = 0; k < CHUNK && rc == GENNMI_OK; k++) {
-                StepArgs a{};
-                a.base = r->dState; a.k = k;
-                rc = launchStep(r, a);
-            }
-            advanceStepKernel<<<dim3(1), dim3(64), 0, r->stream>>>(r->dState, CHUNK);
-            const hipError_t ce = hipStreamEndCapture(r->stream, &graph);
-            if(rc) { return rc; }
-            if(ce != hipSuccess) { return fail(GENNMI_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(ce)); }
-            HIP_TRY(hipGraphInstantiate(&r->graphExec, graph, nullptr, nullptr, 0));
-            HIP_TRY(hipGraphDestroy(graph));
-            r->graphSteps = CHUNK;
-        }
-        HIP_TRY(hipGraphLaunch(r->graphExec, r->stream));
-        done += CHUNK;
-        r->epoch += CHUNK;
-    }
-    for(; done < numSteps; done++) {
-        StepArgs a{};
-        a.base = r->dState; a.k = 0;
-        const int rc = launchStep(r, a);
+    // Every step is launched as gennmi_step_time() launches it: time, epoch and recording row are kernel arguments.  (Measured
+    // against replaying captured graphs of 100 steps whose kernels read them from a device-resident state: a launch costs the
+    // host 2.5 us, less than any step's kernels take, while the graph cost every kernel a dependent load of that state before its
+    // first useful access, runs a copy and a wait for it, and steps beyond a multiple of 100 a launch that advanced it.)
+    for(unsigned long long done = 0; done < numSteps; done++) {
+        const unsigned long long ts = timestep + done;
+        const int rc = stepNow(r, (float)ts * r->dt, numRecordingTimesteps ? (uint32_t)(ts % numRecordingTimesteps) : 0u);
         if(rc) { return rc; }
-        advanceStepKernel<<<dim3(1), dim3(64), 0, r->stream>>>(r->dState, 1);
-        r->epoch++;
     }
-    HIP_TRY(hipGetLastError());
     return GENNMI_OK;
 }
 

@@ -95,7 +95,7 @@ void convStepKernel(const ConvMfmaDev * __restrict__ conv, const NeuronGroupDev 
     __shared__ uint32_t shWaveTotal[CONV_STEP_THREADS / WAVE];
     __shared__ uint32_t shPrefix;
     __shared__ unsigned long long shWaveEvents[CONV_STEP_THREADS / WAVE];
-    const Resolved st = resolve(args, dt);
+    const StepArgs st = args;
     const ConvMfmaDev &G = conv[0];
     const uint32_t ow = (uint32_t)G.g.conv[6], oc = (uint32_t)G.g.conv[7], oh = (uint32_t)G.g.conv[5];
     const uint32_t convBlocks = (oh + G.rowsPerBlock - 1) / G.rowsPerBlock;
@@ -134,7 +134,7 @@ void convStepKernel(const ConvMfmaDev * __restrict__ conv, const NeuronGroupDev 
         const uint32_t bits = spikeBits[w];
         mine += __popc(bits);
         // the bitmap's words are the recording words of the step (every word of the step is written: nothing to clear)
-        if(t.recordSpk) { t.recordSpk[((size_t)st.recT * numBatches + batch) * ((n + 31) / 32) + (firstNeuron >> 5) + w] = bits; }
+        if(t.recordSpk) { t.recordSpk[((size_t)st.recordingTimestep * numBatches + batch) * ((n + 31) / 32) + (firstNeuron >> 5) + w] = bits; }
     }
     uint32_t scan = mine;       // inclusive scan over the wave, then over the waves
     for(int off = 1; off < WAVE; off <<= 1) { const uint32_t up = __shfl_up(scan, off, WAVE); if(lane >= (uint32_t)off) { scan += up; } }

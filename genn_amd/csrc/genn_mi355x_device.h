@@ -34,46 +34,18 @@ __constant__ uint32_t c_spinLimit = SPIN_LIMIT;
 // ------------------------------------------------------------------------------------------------
 // device-side tables
 // ------------------------------------------------------------------------------------------------
-struct StepState             // device-resident; lets a captured graph be replayed unchanged
+struct StepArgs              // per launch: what a step's kernels know of time
 {
-    unsigned long long timestep;
-    unsigned long long epoch;           // number of completed steps since runner creation
-    unsigned long long numRecordingTimesteps;
+    unsigned long long epoch;           // completed steps since runner creation
+    float t;
+    uint32_t recordingTimestep;
 };
-
-struct StepArgs              // per-launch; either direct values or offsets from *base
-{
-    const StepState *base;
-    unsigned long long k;               // offset added to base->timestep / base->epoch
-    unsigned long long epoch;           // direct
-    float t;                            // direct
-    uint32_t recordingTimestep;         // direct
-};
-
-struct Resolved { float t; uint32_t recT; unsigned long long epoch; };
 
 // step counter modulo a 32-bit period: 64-bit division is a long software routine on this part, and the
 // counter fits 32 bits for the first 4e9 steps
 __device__ __forceinline__ uint32_t modStep(unsigned long long x, uint32_t d)
 {
     return (x >> 32) ? (uint32_t)(x % d) : ((uint32_t)x % d);
-}
-
-__device__ __forceinline__ Resolved resolve(const StepArgs &a, float dt)
-{
-    Resolved r;
-    if(a.base) {
-        const unsigned long long ts = a.base->timestep + a.k;
-        // const float t = timestep * DT  (generateRunner.cc:283)
-        r.t = (float)ts * dt;
-        const unsigned long long nr = a.base->numRecordingTimesteps;
-        r.recT = nr ? (((ts | nr) >> 32) ? (uint32_t)(ts % nr) : ((uint32_t)ts % (uint32_t)nr)) : 0u;
-        r.epoch = a.base->epoch + a.k;
-    }
-    else {
-        r.t = a.t; r.recT = a.recordingTimestep; r.epoch = a.epoch;
-    }
-    return r;
 }
 
 // Synapses whose dendritic delay is a multiple of the ring depth land in the slot the target reads in

@@ -144,7 +144,7 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
 // emitted spikes, and the last block of each population (which stores spkCnt), look back.
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
-                                           const Resolved &st, float dt, unsigned long long *agg, uint32_t *errorFlag)
+                                           const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
     __shared__ uint32_t shWaveCount[BLOCK / WAVE];
     __shared__ uint32_t shPrefix;
@@ -304,7 +304,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
             appendOrdered(i < n && vEvent > g.spkEvent[e].threshold, i, localBlock, G.numBlocks, (size_t)batch * totalNeuronBlocks + G.startBlock,
                           counts, counts + perArea, (uint32_t)(st.epoch + 1), g.spkEvent[e].spkEvent + (size_t)batch * n,
                           g.spkEvent[e].spkCntEvent + batch, errorFlag,
-                          g.spkEvent[e].recordSpkEvent ? g.spkEvent[e].recordSpkEvent + ((size_t)st.recT * gridDim.y + batch) * ((n + 31) / 32) : nullptr, i < n);
+                          g.spkEvent[e].recordSpkEvent ? g.spkEvent[e].recordSpkEvent + ((size_t)st.recordingTimestep * gridDim.y + batch) * ((n + 31) / 32) : nullptr, i < n);
         }
     }
 
@@ -318,7 +318,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     // the step is overwritten, so no clearing and no atomicOr (cf. backendSIMT.cc:1948-1953)
     if(g.recordSpk && (lane & 31) == 0 && i < n) {
         const uint32_t words = (n + 31) / 32;
-        g.recordSpk[((size_t)st.recT * gridDim.y + batch) * words + (i >> 5)] = (uint32_t)(ballot >> (lane & 32));
+        g.recordSpk[((size_t)st.recordingTimestep * gridDim.y + batch) * words + (i >> 5)] = (uint32_t)(ballot >> (lane & 32));
     }
     if(G.spikeBitmap && (lane & 31) == 0 && i < n) { G.spikeBitmap[((st.epoch + 1) & 1) * G.bitmapStride + (size_t)batch * ((n + 31) / 32) + (i >> 5)] = (uint32_t)(ballot >> (lane & 32)); }
     __syncthreads();
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(BLOCK)
 void neuronUpdateKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args, float dt,
                         unsigned long long *agg, uint32_t *errorFlag)
 {
-    neuronBody(blocks[blockIdx.x], blockIdx.x, gridDim.x, resolve(args, dt), dt, agg, errorFlag);
+    neuronBody(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -498,7 +498,7 @@ __device__ __forceinline__ bool plainNeuronStep(const PlainNeuron &c, float Isyn
 // (THREADS: threads of the calling work-group, all of which call; batch / numBatches: the grid's second dimension in the neuron kernels)
 template<int NPL, int THREADS = BLOCK>
 __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
-                                               const Resolved &st, float dt, unsigned long long *agg, uint32_t *errorFlag,
+                                               const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag,
                                                uint32_t batch, uint32_t numBatches)
 {
     __shared__ uint32_t shWaveCount[THREADS / WAVE];
@@ -637,7 +637,7 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
         if(i >= n) { continue; }
         if(recordSpk && (lane & 31) == 0) {
             const uint32_t words = (n + 31) / 32;
-            recordSpk[((size_t)st.recT * numBatches + batch) * words + (i >> 5)] = (uint32_t)(ballots[j] >> (lane & 32));
+            recordSpk[((size_t)st.recordingTimestep * numBatches + batch) * words + (i >> 5)] = (uint32_t)(ballots[j] >> (lane & 32));
         }
         if(spikeBitmap && (lane & 31) == 0) { spikeBitmap[((st.epoch + 1) & 1) * bitmapStride + (size_t)batch * ((n + 31) / 32) + (i >> 5)] = (uint32_t)(ballots[j] >> (lane & 32)); }
         if(source) {
@@ -678,7 +678,7 @@ template<int NPL>
 __global__ __launch_bounds__(BLOCK)
 void neuronBulkKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
-    neuronBulkBody<NPL>(blocks[blockIdx.x], blockIdx.x, gridDim.x, resolve(args, dt), dt, agg, errorFlag, blockIdx.y, gridDim.y);
+    neuronBulkBody<NPL>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag, blockIdx.y, gridDim.y);
 }
 
 // One launch per timestep for networks whose projections all go through the dendritic-delay ring: the
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(BLOCK)
 void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t numNeuronBlocks, const PreGroupDev * __restrict__ preBlocks,
                      StepArgs args, float dt, unsigned long long *agg, uint32_t *errorFlag, unsigned long long *eventCounter)
 {
-    const Resolved st = resolve(args, dt);
+    const StepArgs st = args;
     if(blockIdx.x < numNeuronBlocks) {
         // the neuron blocks are the critical path (other blocks wait for their spike counts): let their
         // instructions issue ahead of the presynaptic blocks that share the compute unit
@@ -718,7 +718,6 @@ __global__ void zeroDelayScanKernel(uint32_t numSrc, uint32_t rowStride, const u
     if(zeroLen) { zeroLen[row] = count; }
 }
 
-// Advances the device-resident step state at the end of a captured graph.
 // spike sources: (re)build the per-neuron copy of the next spike time from the arrays the user owns
 __global__ void nextSpikeTimeKernel(const uint32_t *startSpike, const uint32_t *endSpike, const float *spikeTimes, float *next, size_t count)
 {
@@ -727,11 +726,6 @@ __global__ void nextSpikeTimeKernel(const uint32_t *startSpike, const uint32_t *
         const uint32_t s = startSpike[i];
         next[i] = (s != endSpike[i]) ? spikeTimes[s] : INFINITY;
     }
-}
-
-__global__ void advanceStepKernel(StepState *state, unsigned long long steps)
-{
-    if(threadIdx.x == 0 && blockIdx.x == 0) { state->timestep += steps; state->epoch += steps; }
 }
 
 // four floats per lane; dwordx4 when both pointers are 16-byte aligned (hipMalloc'd arrays are), else scalar

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(BLOCK)
 void orderedBitmapKernel(const OrderedSourceDev * __restrict__ blocks, StepArgs args, float dt)
 {
     const OrderedSourceDev &S = blocks[blockIdx.x];
-    const Resolved st = resolve(args, dt);
+    const StepArgs st = args;
     const uint32_t batch = blockIdx.y;
     const uint32_t slots = max(1u, S.numSrcDelaySlots);
     // the slot a projection with this axonal delay reads (backendBase.cc:207-216), as in the scatter kernel
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(BLOCK)
 void presynapticOrderedKernel(OrderedGroupDev G, StepArgs args, float dt, unsigned long long *eventCounter)
 {
     const gennmi_presynaptic_update_group_t &g = G.g;
-    const Resolved st = resolve(args, dt);
+    const StepArgs st = args;
     const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint32_t idPost = blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE;
     if(idPost >= g.numTrgNeurons) { return; }

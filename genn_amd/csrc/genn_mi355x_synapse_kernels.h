@@ -46,7 +46,7 @@ __device__ __forceinline__ bool bitmapTest(GLOBAL_AS const uint32_t *bitmap, uin
 // while the spike count lives on the device.
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t blockInKernel, uint32_t batch, uint32_t numBatches,
-                                                const Resolved &st, float dt, unsigned long long *eventCounter)
+                                                const StepArgs &st, float dt, unsigned long long *eventCounter)
 {
     const gennmi_presynaptic_update_group_t &g = G.g;
     if(G.ordered) { return; }
@@ -551,7 +551,7 @@ __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float
     const bool additive = (g.wum == GENNMI_WUM_STDP);
     const bool stdp = (g.wum == GENNMI_WUM_STDP_TRACE) || additive;
     GLOBAL_AS float *weight = asGlobal(g.g) + (stdp ? (size_t)batch * g.numSrcNeurons * g.rowStride : (size_t)0);
-    const float t = stdp ? resolve(args, dt).t : 0.0f;
+    const float t = stdp ? args.t : 0.0f;
     GLOBAL_AS const float *trgST = asGlobal(g.trgST) + (size_t)batch * g.numTrgNeurons;
     GLOBAL_AS const float *postTrace = asGlobal(g.postTrace) + (size_t)batch * g.numTrgNeurons;
     GLOBAL_AS const uint32_t *trgBitmap = asGlobal(G.learn.trgBitmap) + (size_t)batch * ((g.numTrgNeurons + 31) / 32);
@@ -1025,7 +1025,7 @@ void presynapticConvMfmaKernel(const ConvMfmaDev * __restrict__ blocks, uint32_t
     // the steps too quiet for it: one launch, and the device decides which of the two does the work.
     const uint32_t numBatches = G.numBatches;
     const uint32_t batch = blockIdx.x % numBatches;
-    const Resolved st = resolve(args, dt);
+    const StepArgs st = args;
     if(blockIdx.x >= mfmaBlocks) {
         const uint32_t b = (blockIdx.x - mfmaBlocks) / numBatches;
         presynapticBody(scatter[b], b, batch, numBatches, st, dt, eventCounter);
@@ -1050,14 +1050,14 @@ __global__ void spikeBitmapFromQueueKernel(const uint32_t *spkCnt, const uint32_
 __global__ __launch_bounds__(1024)
 void presynapticUpdateKernel(const PreGroupDev * __restrict__ blocks, StepArgs args, float dt, unsigned long long *eventCounter)
 {
-    presynapticBody(blocks[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, resolve(args, dt), dt, eventCounter);
+    presynapticBody(blocks[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
 }
 
 // ------------------------------------------------------------------------------------------------
 // Postsynaptic update (learnPost): one sub-group per postsynaptic spike walks the column through
 // remap (coalesced), gathers g by synapse index.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void postsynapticBody(const PostGroupDev &G, uint32_t blockInKernel, uint32_t *shBits, const Resolved &st, float dt)
+__device__ __forceinline__ void postsynapticBody(const PostGroupDev &G, uint32_t blockInKernel, uint32_t *shBits, const StepArgs &st, float dt)
 {
     const gennmi_postsynaptic_update_group_t &g = G.g;
     const uint32_t batch = blockIdx.y;
@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(1024)
 void postsynapticUpdateKernel(const PostGroupDev * __restrict__ blocks, StepArgs args, float dt)
 {
     extern __shared__ uint32_t shBits[];
-    postsynapticBody(blocks[blockIdx.x], blockIdx.x, shBits, resolve(args, dt), dt);
+    postsynapticBody(blocks[blockIdx.x], blockIdx.x, shBits, args, dt);
 }
 
 // All synaptic work of a step that can share a launch: the scatter path of every projection, the tile path of those that
@@ -1188,14 +1188,14 @@ void synapseCombinedKernel(const PreGroupDev * __restrict__ pre, uint32_t preBlo
 {
     extern __shared__ float shDynamic[];
     if(blockIdx.x < preBlocks) {
-        presynapticBody(pre[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, resolve(args, dt), dt, eventCounter);
+        presynapticBody(pre[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
     }
     else if(blockIdx.x < preBlocks + tileBlocks) {
         presynapticTileBody(tiles[blockIdx.x - preBlocks], shDynamic, args, dt, eventCounter);
     }
     else {
         const uint32_t b = blockIdx.x - preBlocks - tileBlocks;
-        postsynapticBody(post[b], b, reinterpret_cast<uint32_t*>(shDynamic), resolve(args, dt), dt);
+        postsynapticBody(post[b], b, reinterpret_cast<uint32_t*>(shDynamic), args, dt);
     }
 }
 

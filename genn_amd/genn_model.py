@@ -1009,7 +1009,7 @@ class GeNNModel:
         self.timestep += 1
 
     def run(self, num_steps):
-        """num_steps consecutive step_time() calls replayed from captured HIP graphs."""
+        """num_steps consecutive step_time() calls in one call of the library."""
         nrec = self.num_recording_timesteps or 0
         _abi.check(_abi.load().gennmi_run_steps(self._runner, self.timestep, int(num_steps), nrec))
         self.timestep += int(num_steps)

@@ -409,8 +409,8 @@ int gennmi_step(gennmi_runner *runner, float t, uint32_t recordingTimestep);
 int gennmi_step_time(gennmi_runner *runner, unsigned long long timestep, unsigned long long numRecordingTimesteps);
 /* numSteps consecutive stepTime calls starting at `timestep` without a host round trip per step (no counterpart
  * in the reference, which launches 4-7 kernels per step from the host): one launch that keeps the network resident
- * on the chip where the runner's plan allows it (see gennmi_runner_get_info), else replays of a captured HIP graph
- * of 100 steps.  Either way the arrays are left as numSteps calls of gennmi_step_time would leave them. */
+ * on the chip where the runner's plan allows it (see gennmi_runner_get_info), else the steps launched
+ * one behind another.  Either way the arrays are left as numSteps calls of gennmi_step_time would leave them. */
 int gennmi_run_steps(gennmi_runner *runner, unsigned long long timestep, unsigned long long numSteps,
                      unsigned long long numRecordingTimesteps);
 /* Step queue (no counterpart in the reference).  A caller that advances the model one gennmi_step() at a time -- the
@@ -428,7 +428,7 @@ int gennmi_runner_synchronize(gennmi_runner *runner);
 
 /* Timers: neuronUpdateTime / presynapticUpdateTime / postsynapticUpdateTime of generateRunner.cc:161-174,
  * in seconds, accumulated with HIP events while enabled (backendCUDAHIP.cc:36-76, 1479-1504).  While timing is enabled
- * every step is launched on its own, kernel by kernel (gennmi_run_steps included: no resident launch, no graph replay),
+ * every step is launched on its own, kernel by kernel (gennmi_run_steps included: no resident launch),
  * so that each kernel has an event pair around it.  A single-launch step (see gennmi_runner_get_info) is one kernel that
  * holds the neuron update and the presynaptic update of the previous step's spikes: its duration is reported as
  * neuronUpdateTime and presynapticUpdateTime stays 0 for such a runner. */
