@@ -149,6 +149,7 @@ SYMBOLS = {
     "gennmi_program_get_time": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_double)]),
     "gennmi_program_get_info": (C.c_int, [C.c_void_p, C.POINTER(C.c_ulonglong * 4)]),
     "gennmi_host_malloc": (C.c_int, [C.POINTER(C.c_void_p), C.c_size_t, C.c_int, C.POINTER(C.c_void_p)]),
+    "gennmi_host_acquire": (C.c_int, [C.POINTER(C.c_void_p), C.c_size_t]),
     "gennmi_host_free": (C.c_int, [C.c_void_p]),
     "gennmi_profiler_range_push": (C.c_int, [C.c_char_p]),
     "gennmi_profiler_range_pop": (C.c_int, []),
@@ -169,6 +170,13 @@ SYMBOLS = {
     "gennmi_step_time": (C.c_int, [C.c_void_p, _ULL, _ULL]),
     "gennmi_run_steps": (C.c_int, [C.c_void_p, _ULL, _ULL, _ULL]),
     "gennmi_runner_synchronize": (C.c_int, [C.c_void_p]),
+    "gennmi_runner_push": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]),
+    "gennmi_runner_pull": (C.c_int, [C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "gennmi_runner_pull_spikes": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p, C.c_void_p]),
+    "gennmi_runner_error": (C.c_int, [C.c_void_p]),
+    "gennmi_decode_recording": (C.c_int, [C.c_void_p, C.c_size_t, C.c_size_t, C.c_uint32, C.c_double, C.c_double, C.c_void_p, C.c_void_p,
+                                          C.POINTER(C.c_size_t)]),
+    "gennmi_runner_copy_f32": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]),
     "gennmi_runner_set_timing": (C.c_int, [C.c_void_p, C.c_int]),
     "gennmi_runner_get_times": (C.c_int, [C.c_void_p, C.POINTER(C.c_double), C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "gennmi_runner_kernel_stats": (C.c_int, [C.c_void_p, C.POINTER(C.c_double * 8)]),

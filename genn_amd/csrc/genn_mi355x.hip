@@ -48,6 +48,7 @@
 #include "genn_mi355x_resident_kernels.h"
 #include "genn_mi355x_ordered_kernels.h"
 #include "genn_mi355x_conv_step_kernels.h"
+#include "genn_mi355x_transfer.h"
 
 struct gennmi_runner
 {
@@ -62,6 +63,7 @@ struct gennmi_runner
     uint32_t neuronBlocks = 0, preBlocks = 0, postBlocks = 0;
     unsigned long long *dAgg = nullptr; uint32_t *dError = nullptr; unsigned long long *dEvents = nullptr;
     uint32_t *hError = nullptr;     // the error flag: a pinned host word; dError is the same word's device address
+    uint32_t *hSignal = nullptr; uint32_t signalSeq = 0;     // a pinned host word (a cache line behind it) that gennmi_runner_synchronize has a kernel store to
     unsigned long long epoch = 0;       // completed steps (host mirror)
     bool synapsesDone = false;          // updateSynapses ran for the current step
     bool fusedStep = false;             // zero-delay synapses are delivered by the neuron update; one launch per step
@@ -167,6 +169,13 @@ static void noteDeviceWrite(const void *dev, size_t bytes)
     }
 }
 
+static int runnerError(const gennmi_runner *r)
+{
+    // (host memory the kernels write: read once the stream has drained)
+    if(*r->hError) { return fail(GENNMI_EDEVICE, "a kernel's bounded wait for other work-groups expired (spike offsets or spike exchange); state is undefined"); }
+    return GENNMI_OK;
+}
+
 // Step queue.  A caller that advances the model one gennmi_step() at a time (the reference's Runtime::stepTime does) would
 // pay a launch per step; a runner on the resident plan can do many steps in one launch.  With a queue enabled, gennmi_step()
 // only notes the step; the noted steps run, as one launch where they can, before anything could observe the difference:
@@ -236,15 +245,23 @@ int gennmi_malloc(void **devPtr, size_t bytes)
 int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr)
 {
     if(!hostPtr || (zeroCopy && !devPtr)) { return fail(GENNMI_EINVAL, "host_malloc: null result pointer"); }
-    HIP_TRY(hipHostMalloc(hostPtr, bytes ? bytes : 4, zeroCopy ? hipHostMallocMapped : hipHostMallocPortable));
+    if(zeroCopy) { HIP_TRY(hipHostMalloc(hostPtr, bytes ? bytes : 4, hipHostMallocMapped)); }
+    else { const int rc = pinnedMalloc(hostPtr, bytes); if(rc) { return rc; } }
     std::memset(*hostPtr, 0, bytes);
     if(devPtr) { *devPtr = nullptr; }
     if(zeroCopy) { HIP_TRY(hipHostGetDevicePointer(devPtr, *hostPtr, 0)); }
     return GENNMI_OK;
 }
+int gennmi_host_acquire(void **hostPtr, size_t bytes)
+{
+    if(!hostPtr) { return fail(GENNMI_EINVAL, "host_acquire: null result pointer"); }
+    return pinnedMalloc(hostPtr, bytes);
+}
 int gennmi_host_free(void *hostPtr)
 {
-    if(hostPtr) { HIP_TRY(hipHostFree(hostPtr)); }
+    hipError_t e = hipSuccess;
+    if(hostPtr && !pinnedFree(hostPtr, &e)) { e = hipHostFree(hostPtr); }
+    HIP_TRY(e);
     return GENNMI_OK;
 }
 int gennmi_free(void *devPtr) { FLUSH_QUEUED(); HIP_TRY(hipFree(devPtr)); return GENNMI_OK; }
@@ -483,8 +500,9 @@ int gennmi_runner_create(gennmi_runner **runner, float dt, uint32_t batchSize)
     HIP_TRY(hipStreamCreate(&r->stream));       // blocking stream: ordered against null-stream copies
 
     // the error flag: one pinned host word, which the kernels reach through its device address (raiseErrorFlag)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->hError), sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
-    *r->hError = 0;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->hError), 32 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+    memset(r->hError, 0, 32 * sizeof(uint32_t));
+    r->hSignal = r->hError + 16;
     HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&r->dError), r->hError, 0));
     HIP_TRY(hipMalloc(&r->dEvents, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
     HIP_TRY(hipMemset(r->dEvents, 0, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
@@ -1985,19 +2003,89 @@ int gennmi_runner_synchronize(gennmi_runner *r)
 {
     if(!r) { return fail(GENNMI_EINVAL, "runner_synchronize: null runner"); }
     FLUSH_QUEUED();
-    // (the flag is host memory the kernels write: nothing to copy, it is read below once the stream has drained)
-    // (short waits are polled: a blocking wait wakes up some tens of microseconds after the work has ended; GENNMI_POLL_US=0 blocks at once)
-    static const long pollMicroseconds = [] { const char *e = getenv("GENNMI_POLL_US"); return e ? atol(e) : 500l; }();
-    if(pollMicroseconds > 0) {
-        const auto begin = std::chrono::steady_clock::now();
-        hipError_t state = hipStreamQuery(r->stream);
-        while(state == hipErrorNotReady && std::chrono::steady_clock::now() - begin < std::chrono::microseconds(pollMicroseconds)) { state = hipStreamQuery(r->stream); }
-        (void)hipGetLastError();    // "not ready" is an answer, not a failure to keep
-        if(state != hipSuccess && state != hipErrorNotReady) { HIP_TRY(state); }
+    // A kernel behind everything that is queued stores a number the host spins on: 20 queued launches and this wait take
+    // 58 us, with hipStreamSynchronize 74, with a loop around hipStreamQuery 75 (one launch: 9.3, 11.9 and 22.9 us).
+    r->signalSeq++;
+    signalKernel<<<dim3(1), dim3(1), 0, r->stream>>>(r->hSignal, r->signalSeq);
+    HIP_TRY(hipGetLastError());
+    { const int rc = waitForFlag(r->hSignal, r->signalSeq, r->stream); if(rc) { return rc; } }
+    return runnerError(r);
+}
+
+// Copies in the order of a runner's steps (genn_mi355x_transfer.h).  Until the runner is finalised its arrays are being made
+// by null-stream work, and copies join that.
+static hipStream_t transferStream(const gennmi_runner *r) { return r->finalised ? r->stream : nullptr; }
+
+int gennmi_runner_push(gennmi_runner *r, void *dev, const void *host, size_t bytes)
+{
+    if(!r || (bytes && (!dev || !host))) { return fail(GENNMI_EINVAL, "runner_push: null argument"); }
+    FLUSH_QUEUED();
+    const TransferPart part{static_cast<uint8_t*>(const_cast<void*>(host)), static_cast<uint8_t*>(dev), bytes};
+    { const int rc = pushArray(part, transferStream(r), r->finalised); if(rc) { return rc; } }
+    noteDeviceWrite(dev, bytes);
+    return GENNMI_OK;
+}
+
+int gennmi_runner_pull(gennmi_runner *r, uint32_t count, void *const *hosts, const void *const *devs, const size_t *bytes)
+{
+    if(!r || (count && (!hosts || !devs || !bytes))) { return fail(GENNMI_EINVAL, "runner_pull: null argument"); }
+    FLUSH_QUEUED();
+    std::vector<TransferPart> parts(count);
+    for(uint32_t k = 0; k < count; k++) {
+        if(bytes[k] && (!hosts[k] || !devs[k])) { return fail(GENNMI_EINVAL, "runner_pull: null array"); }
+        parts[k] = {static_cast<uint8_t*>(hosts[k]), static_cast<uint8_t*>(const_cast<void*>(devs[k])), bytes[k]};
     }
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    const uint32_t err = *r->hError;
-    if(err) { return fail(GENNMI_EDEVICE, "a kernel's bounded wait for other work-groups expired (spike offsets or spike exchange); state is undefined"); }
+    return pullParts(parts.data(), count, transferStream(r));
+}
+
+int gennmi_runner_error(const gennmi_runner *r)
+{
+    if(!r) { return fail(GENNMI_EINVAL, "runner_error: null runner"); }
+    return runnerError(r);
+}
+
+int gennmi_runner_pull_spikes(gennmi_runner *r, const uint32_t *spkCnt, const uint32_t *spk, uint32_t numNeurons, uint32_t slots, uint32_t slot,
+                              uint32_t *counts, uint32_t *ids)
+{
+    if(!r || !spkCnt || !spk || !counts || !ids || numNeurons == 0 || slot >= slots) { return fail(GENNMI_EINVAL, "runner_pull_spikes: bad arguments"); }
+    FLUSH_QUEUED();
+    return pullSpikes(spkCnt, spk, numNeurons, slots, slot, r->batch, counts, ids, transferStream(r));
+}
+
+int gennmi_runner_copy_f32(gennmi_runner *r, float *dst, const float *src, size_t count)
+{
+    if(!r || (count && (!dst || !src))) { return fail(GENNMI_EINVAL, "runner_copy_f32: null argument"); }
+    FLUSH_QUEUED();
+    if(count) {
+        { const int rc = copyOnDevice(dst, src, count, transferStream(r)); if(rc) { return rc; } }
+        noteDeviceWrite(dst, count * sizeof(float));
+    }
+    return GENNMI_OK;
+}
+
+// Bits of a recording buffer to (time, neuron) pairs: the host half of getRecordedSpikes (runtime.cc:855-913), rows in time order and
+// neurons ascending within a row.  One pass over the words counts, a second writes; a word without spikes costs a comparison.
+int gennmi_decode_recording(const uint32_t *record, size_t numSteps, size_t rowStride, uint32_t numNeurons, double firstStep, double dt,
+                            double *times, uint32_t *ids, size_t *count)
+{
+    if(!record || !count || (times == nullptr) != (ids == nullptr)) { return fail(GENNMI_EINVAL, "decode_recording: null argument"); }
+    const size_t words = (numNeurons + 31) / 32;
+    const uint32_t lastMask = (numNeurons % 32) ? ((1u << (numNeurons % 32)) - 1u) : 0xFFFFFFFFu;
+    size_t n = 0;
+    for(size_t step = 0; step < numSteps; step++) {
+        const uint32_t *row = record + step * rowStride;
+        const double time = (firstStep + (double)step) * dt;
+        for(size_t w = 0; w < words; w++) {
+            uint32_t bits = (w + 1 == words) ? (row[w] & lastMask) : row[w];
+            if(!times) { n += (size_t)__builtin_popcount(bits); continue; }
+            for(; bits; bits &= bits - 1) {
+                if(n == *count) { return fail(GENNMI_EINVAL, "decode_recording: the arrays hold fewer spikes than the buffer"); }
+                times[n] = time;
+                ids[n++] = (uint32_t)(w * 32) + (uint32_t)__builtin_ctz(bits);
+            }
+        }
+    }
+    *count = n;
     return GENNMI_OK;
 }
 

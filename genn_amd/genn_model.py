@@ -163,22 +163,56 @@ def init_var(snippet, params=None):
 # --------------------------------------------------------------------------------------------
 # device arrays (the reference's Array objects, src/genn/backends/hip/backend.cc:61-236)
 # --------------------------------------------------------------------------------------------
+class _Pinned:
+    """Pinned host memory (not cleared) as numpy's array interface presents it; given back with the last array that shows it."""
+
+    def __init__(self, count, dtype):
+        self._free = _abi.load().gennmi_host_free
+        self._ptr = C.c_void_p()
+        _abi.check(_abi.load().gennmi_host_acquire(C.byref(self._ptr), count * dtype.itemsize))
+        self.__array_interface__ = {"version": 3, "shape": (count,), "typestr": dtype.str, "data": (self._ptr.value, False)}
+
+    def __del__(self):
+        if self._ptr:
+            self._free(self._ptr)
+
+
+PINNED_MOST = 64 << 20      # bytes of an array's host side up to which it is pinned where that is asked for
+
+
 class Array:
-    def __init__(self, count, dtype, fill=None, device_only=False):
-        """``device_only`` arrays (those a device kernel initialises) get their host copy on the first pull."""
+    def __init__(self, count, dtype, fill=None, device_only=False, model=None, pinned=False):
+        """``device_only``: the device array's first value is somebody else's to write.  Copies of an array
+        of a ``model`` run in the order of its steps.  ``pinned``: the host side of an array that is copied again and again."""
         self.dtype = np.dtype(dtype)
         self.count = int(count)
+        self._model, self._pinned = model, pinned
         self._dev = C.c_void_p()
         _abi.check(_abi.load().gennmi_malloc(C.byref(self._dev), self.count * self.dtype.itemsize))
         self._view = None
-        if not device_only:
-            self._view = np.zeros(self.count, dtype=self.dtype) if fill is None else np.full(self.count, fill, dtype=self.dtype)
+        self._fill = fill
+        # (the first value is written on the device; the host copy is made when somebody asks for it)
+        if device_only or not self.count:
+            pass
+        elif fill is None:
+            _abi.check(_abi.load().gennmi_memset(self._dev, 0, self.count * self.dtype.itemsize))
+        elif self.dtype == np.float32:
+            _abi.check(_abi.load().gennmi_init_var(self._dev, _abi.ELEMENT_TYPES["float32"], self.count, _abi.INIT_SNIPPETS["Constant"],
+                                                   C.byref((C.c_double * 4)(fill)), 0, 0))
+        else:
             self.push_to_device()
 
     @property
     def view(self):
         if self._view is None:
-            self._view = np.zeros(self.count, dtype=self.dtype)
+            self._make_view().fill(0 if self._fill is None else self._fill)
+        return self._view
+
+    def _make_view(self):
+        """The host side, its contents left to the caller."""
+        if self._view is None:
+            pinned = self._pinned and 0 < self.count * self.dtype.itemsize <= PINNED_MOST
+            self._view = np.asarray(_Pinned(self.count, self.dtype)) if pinned else np.empty(self.count, dtype=self.dtype)
         return self._view
 
     @property
@@ -189,13 +223,22 @@ class Array:
     def values(self):
         return self.view
 
+    @property
+    def _runner(self):
+        """The runner whose steps copies of this array follow, or None: an array of its own, or of a model that is not loaded."""
+        return self._model._runner if self._model is not None and self._model._runner else None
+
     def push_to_device(self):
-        if self.view.nbytes:
-            _abi.check(_abi.load().gennmi_memcpy_to_device(self._dev, self.view.ctypes.data_as(C.c_void_p), self.view.nbytes))
+        view = self.view
+        if view.nbytes:
+            runner = self._runner
+            if runner is not None:
+                _abi.check(_abi.load().gennmi_runner_push(runner, self._dev, view.ctypes.data, view.nbytes))
+            else:
+                _abi.check(_abi.load().gennmi_memcpy_to_device(self._dev, view.ctypes.data, view.nbytes))
 
     def pull_from_device(self):
-        if self.view.nbytes:
-            _abi.check(_abi.load().gennmi_memcpy_from_device(self.view.ctypes.data_as(C.c_void_p), self._dev, self.view.nbytes))
+        pull_arrays(self._runner, [self])
         return self.view
 
     def pull_slice(self, first, count):
@@ -205,7 +248,7 @@ class Array:
             raise IndexError("slice outside the array")
         out = np.empty(count, dtype=self.dtype)
         if count:
-            _abi.check(_abi.load().gennmi_memcpy_from_device(out.ctypes.data_as(C.c_void_p), C.c_void_p(self._dev.value + first * self.dtype.itemsize), out.nbytes))
+            _abi.check(_abi.load().gennmi_memcpy_from_device(out.ctypes.data, self._dev.value + first * self.dtype.itemsize, out.nbytes))
         return out
 
     def init_on_device(self, init, seed, stream, dt):
@@ -218,12 +261,29 @@ class Array:
         """Device-to-device copy of another fp32 Array of the same length (host views are left alone)."""
         if self.dtype != np.float32 or src.dtype != np.float32 or src.count != self.count:
             raise ValueError("copy_on_device needs two float32 arrays of equal length")
-        _abi.check(_abi.load().gennmi_copy_f32(self._dev, src._dev, self.count))
+        runner = self._runner
+        if runner is not None:
+            _abi.check(_abi.load().gennmi_runner_copy_f32(runner, self._dev, src._dev, self.count))
+        else:
+            _abi.check(_abi.load().gennmi_copy_f32(self._dev, src._dev, self.count))
 
     def free(self):
         if self._dev:
             _abi.load().gennmi_free(self._dev)
             self._dev = C.c_void_p()
+
+
+def pull_arrays(runner, arrays):
+    """Device to host copies of several arrays: behind the runner's steps, with one wait for all of them."""
+    arrays = [a for a in arrays if a._make_view().nbytes]
+    lib = _abi.load()
+    if runner is None:
+        for a in arrays:
+            _abi.check(lib.gennmi_memcpy_from_device(a.view.ctypes.data, a._dev, a.view.nbytes))
+    elif arrays:
+        n = len(arrays)
+        hosts, devs = (C.c_void_p * n)(*(a.view.ctypes.data for a in arrays)), (C.c_void_p * n)(*(a._dev.value for a in arrays))
+        _abi.check(lib.gennmi_runner_pull(runner, n, hosts, devs, (C.c_size_t * n)(*(a.view.nbytes for a in arrays))))
 
 
 class NeuronGroup:
@@ -247,6 +307,7 @@ class NeuronGroup:
         self.needs_spike_time = False
         self.num_delay_slots = 1     # longest axonal delay of the outgoing projections + 1, set by build()
         self.pre_output_syn = []     # outgoing projections whose code calls addToPre
+        self._queue_copy = None      # where current_spikes copies the queue to
         self.event_thresholds = []   # one spike-like event queue per distinct threshold of the outgoing graded projections
 
     @property
@@ -266,11 +327,15 @@ class NeuronGroup:
         """Spike queue written by the last step: ids in ascending order (per batch)."""
         # with axonal delay the queue is a ring of slots; the last step wrote slot timestep % slots (pygenn's current_spikes
         # reads spkQuePtr the same way, genn_groups.py)
-        slots, B = self.num_delay_slots, self._model.batch_size
-        slot = self._model.timestep % slots
-        cnt = self.vars["spkCnt"].pull_from_device().reshape(B, slots)[:, slot].copy()
-        spk = self.vars["spk"].pull_from_device().reshape(B, slots, self.num_neurons)[:, slot]
-        return [spk[b, :cnt[b]].copy() for b in range(B)]
+        model, slots, n = self._model, self.num_delay_slots, self.num_neurons
+        B = model.batch_size
+        if self._queue_copy is None:
+            ids, counts = np.empty((B, n), np.uint32), np.empty(B, np.uint32)
+            self._queue_copy = ids, counts, ids.ctypes.data, counts.ctypes.data
+        ids, counts, ids_address, counts_address = self._queue_copy
+        _abi.check(_abi.load().gennmi_runner_pull_spikes(model._runner, self.vars["spkCnt"]._dev, self.vars["spk"]._dev, n, slots,
+                                                         model.timestep % slots, counts_address, ids_address))
+        return [ids[b, :counts[b]].copy() for b in range(B)]
 
 
 class CurrentSource:
@@ -403,6 +468,7 @@ class GeNNModel:
         self.current_sources = {}
         self.timestep = 0
         self._runner = C.c_void_p()
+        self._gennmi_step_time = lambda *args: _abi.load().gennmi_step_time(*args)      # (the function itself once the model is loaded)
         self._built = False
         self._loaded = False
         self._device = device
@@ -512,13 +578,13 @@ class GeNNModel:
     def _den_delay(s):
         return s.max_dendritic_delay_timesteps if s.wu.snippet == "StaticPulseDendriticDelay" else 0
 
-    def _alloc(self, count, dtype, fill=None, device_only=False):
-        a = Array(count, dtype, fill, device_only)
+    def _alloc(self, count, dtype, fill=None, device_only=False, pinned=False):
+        a = Array(count, dtype, fill, device_only, model=self, pinned=pinned)
         self._arrays.append(a)
         return a
 
-    def _alloc_device_init(self, count, dtype, init, stream=None):
-        a = self._alloc(count, dtype, device_only=True)
+    def _alloc_device_init(self, count, dtype, init, stream=None, pinned=False):
+        a = self._alloc(count, dtype, device_only=True, pinned=pinned)
         a.init_on_device(init, self.seed, self._next_stream() if stream is None else stream, self.dt)
         return a
 
@@ -531,6 +597,7 @@ class GeNNModel:
         if not self._built:
             raise RuntimeError("build() must be called before load()")
         lib = _abi.load()
+        self._gennmi_step_time = lib.gennmi_step_time
         _abi.check(lib.gennmi_init(self._device))
         load_start = time.perf_counter()
         B = self.batch_size
@@ -543,13 +610,13 @@ class GeNNModel:
             N = n.num_neurons
             if n.neuron == "SpikeSourceArray":
                 for v in ("startSpike", "endSpike"):
-                    a = self._alloc(B * N, np.uint32)
+                    a = self._alloc(B * N, np.uint32, pinned=True, device_only=True)
                     a.view[:] = np.broadcast_to(np.asarray(n.var_init[v], dtype=np.uint32), (B, N)).reshape(-1) \
                         if np.ndim(n.var_init[v]) < 2 else np.asarray(n.var_init[v], dtype=np.uint32).reshape(-1)
                     a.push_to_device()
                     n.vars[v] = a
                 st = np.ascontiguousarray(n.extra_global_params["spikeTimes"], dtype=np.float32)
-                a = self._alloc(max(1, st.size), np.float32)
+                a = self._alloc(max(1, st.size), np.float32, pinned=True, device_only=True)
                 a.view[:st.size] = st
                 a.push_to_device()
                 n.vars["spikeTimes"] = a
@@ -557,44 +624,44 @@ class GeNNModel:
                 names = ("V", "RefracTime") if n.neuron == "LIF" else ("V", "U")
                 for v in names:
                     if isinstance(n.var_init[v], VarInit):
-                        n.vars[v] = self._alloc_device_init(B * N, np.float32, n.var_init[v])
+                        n.vars[v] = self._alloc_device_init(B * N, np.float32, n.var_init[v], pinned=True)
                         continue
-                    a = self._alloc(B * N, np.float32)
+                    a = self._alloc(B * N, np.float32, pinned=True, device_only=True)
                     init = np.asarray(n.var_init[v], dtype=np.float32)
                     a.view[:] = np.broadcast_to(init, (B, N)).reshape(-1) if init.ndim < 2 else init.reshape(-1)
                     a.push_to_device()
                     n.vars[v] = a
-            n.vars["spkCnt"] = self._alloc(B * n.num_delay_slots, np.uint32)
-            n.vars["spk"] = self._alloc(B * n.num_delay_slots * N, np.uint32)
+            n.vars["spkCnt"] = self._alloc(B * n.num_delay_slots, np.uint32, pinned=True)
+            n.vars["spk"] = self._alloc(B * n.num_delay_slots * N, np.uint32, pinned=True)
             for s in n.pre_output_syn:
-                s.vars["outPre"] = self._alloc(B * N, np.float32)
+                s.vars["outPre"] = self._alloc(B * N, np.float32, pinned=True)
             for e in range(len(n.event_thresholds)):
-                n.vars[f"spkCntEvent{e}"] = self._alloc(B, np.uint32)
-                n.vars[f"spkEvent{e}"] = self._alloc(B * N, np.uint32)
+                n.vars[f"spkCntEvent{e}"] = self._alloc(B, np.uint32, pinned=True)
+                n.vars[f"spkEvent{e}"] = self._alloc(B * N, np.uint32, pinned=True)
                 if n.spike_event_recording_enabled:
                     if not num_recording_timesteps:
                         raise RuntimeError("Cannot use recording system without specifying number of recording timesteps")
-                    n.vars[f"recordSpkEvent{e}"] = self._alloc(((N + 31) // 32) * B * num_recording_timesteps, np.uint32)
+                    n.vars[f"recordSpkEvent{e}"] = self._alloc(((N + 31) // 32) * B * num_recording_timesteps, np.uint32, pinned=True)
             if n.spike_recording_enabled:
                 if not num_recording_timesteps:
                     raise RuntimeError("Cannot use recording system without specifying number of recording timesteps")
-                n.vars["recordSpk"] = self._alloc(((N + 31) // 32) * B * num_recording_timesteps, np.uint32)
+                n.vars["recordSpk"] = self._alloc(((N + 31) // 32) * B * num_recording_timesteps, np.uint32, pinned=True)
             if n.needs_spike_time:
-                n.vars["sT"] = self._alloc(B * N, np.float32, fill=-FLT_MAX)      # -TIME_MAX, as the reference's initialize()
+                n.vars["sT"] = self._alloc(B * N, np.float32, fill=-FLT_MAX, pinned=True)      # -TIME_MAX, as the reference's initialize()
             for grp in n.fused_psm:
                 owner = grp[0]
-                owner.vars["outPost"] = self._alloc(B * N, np.float32)
+                owner.vars["outPost"] = self._alloc(B * N, np.float32, pinned=True)
                 D = self._den_delay(owner)
                 if D:
                     owner.vars["denDelay"] = self._alloc(B * D * N, np.float32)
-                    owner.vars["denDelayPtr"] = self._alloc(1, np.uint32)
+                    owner.vars["denDelayPtr"] = self._alloc(1, np.uint32, pinned=True)
             if n.pre_trace_owner is not None:
-                n.pre_trace_owner.vars["preTrace"] = self._alloc(B * N, np.float32, fill=n.pre_trace_owner.wu.pre_vars.get("preTrace", 0.0))
+                n.pre_trace_owner.vars["preTrace"] = self._alloc(B * N, np.float32, fill=n.pre_trace_owner.wu.pre_vars.get("preTrace", 0.0), pinned=True)
             if n.post_trace_owner is not None:
-                n.post_trace_owner.vars["postTrace"] = self._alloc(B * N, np.float32, fill=n.post_trace_owner.wu.post_vars.get("postTrace", 0.0))
+                n.post_trace_owner.vars["postTrace"] = self._alloc(B * N, np.float32, fill=n.post_trace_owner.wu.post_vars.get("postTrace", 0.0), pinned=True)
             for cs in n.current_sources:
                 if cs.kind == "PoissonExp":
-                    cs.vars["current"] = self._alloc(B * N, np.float32)
+                    cs.vars["current"] = self._alloc(B * N, np.float32, pinned=True)
                     if cs.stream is None:
                         # by place in the name-ordered list of the model's current sources, as the backend adapter numbers them
                         cs.stream = 1000 + sorted(self.current_sources).index(cs.name)
@@ -602,7 +669,7 @@ class GeNNModel:
                     noise = np.ascontiguousarray(cs.extra_global_params["noise"], dtype=np.float32)
                     if noise.size % N:
                         raise ValueError(f"{cs.name}: noise array is not a multiple of the population size")
-                    a = self._alloc(noise.size, np.float32)
+                    a = self._alloc(noise.size, np.float32, device_only=True)
                     a.view[:] = noise.reshape(-1)
                     a.push_to_device()
                     cs.vars["noise"] = a
@@ -617,7 +684,7 @@ class GeNNModel:
                     raise RuntimeError(f"{s.name}: sparse connectivity has not been set")
                 else:
                     for name, host, dtype in (("rowLength", s.row_length_host, np.uint32), ("ind", s.ind_host, np.uint32)):
-                        a = self._alloc(host.size, dtype)
+                        a = self._alloc(host.size, dtype, device_only=True)
                         a.view[:] = host.reshape(-1)
                         a.push_to_device()
                         s.vars[name] = a
@@ -638,7 +705,7 @@ class GeNNModel:
                         streams = getattr(s, "init_streams", None)
                         s.vars[name] = self._alloc_device_init(n_pre * s.row_stride, dtype, s.wu.vars[name], streams[1] if streams and name == "g" else None)
                         continue
-                    a = self._alloc(copies * n_pre * s.row_stride, dtype)
+                    a = self._alloc(copies * n_pre * s.row_stride, dtype, device_only=True)
                     if name in s.var_host:
                         a.view[:] = np.tile(np.asarray(s.var_host[name], dtype=dtype).reshape(-1), copies)
                     else:
@@ -659,7 +726,7 @@ class GeNNModel:
                     if isinstance(init, VarInit):
                         s.vars["g"] = self._alloc_device_init(count, np.float32, init)
                     else:
-                        a = self._alloc(count, np.float32)
+                        a = self._alloc(count, np.float32, device_only=True)
                         a.view[:] = np.broadcast_to(np.asarray(init, dtype=np.float32).reshape(-1), (count,)) if np.size(init) in (1, count) \
                             else np.asarray(init, dtype=np.float32).reshape(-1)
                         a.push_to_device()
@@ -667,13 +734,13 @@ class GeNNModel:
             elif s.matrix_type == "BITMASK":
                 if s.gp_host is None:
                     raise RuntimeError(f"{s.name}: bitmask connectivity has not been set")
-                a = self._alloc(s.gp_host.size, np.uint32)
+                a = self._alloc(s.gp_host.size, np.uint32, device_only=True)
                 a.view[:] = s.gp_host
                 a.push_to_device()
                 s.vars["gp"] = a
             else:
                 kern = np.ascontiguousarray(s.var_host.get("g", s.wu.vars.get("g")), dtype=np.float32)
-                a = self._alloc(kern.size, np.float32)
+                a = self._alloc(kern.size, np.float32, device_only=True)
                 a.view[:] = kern.reshape(-1)
                 a.push_to_device()
                 s.vars["g"] = a
@@ -726,7 +793,7 @@ class GeNNModel:
                 values = np.ascontiguousarray(init.params["kernel"], dtype=np.float32).reshape(-1)
                 if values.size != conv[0] * conv[1] * conv[8] * conv[11]:
                     raise ValueError(f"{s.name}: the kernel must hold conv_kh * conv_kw * conv_ic * conv_oc values")
-                k = self._alloc(values.size, np.float32)
+                k = self._alloc(values.size, np.float32, device_only=True)
                 k.view[:] = values
                 k.push_to_device()
                 s.vars["kernel"] = k
@@ -993,8 +1060,9 @@ class GeNNModel:
         return float(np.float32(self.timestep) * lit32(self.dt))
 
     def step_time(self):
-        nrec = self.num_recording_timesteps or 0
-        _abi.check(_abi.load().gennmi_step_time(self._runner, self.timestep, nrec))
+        rc = self._gennmi_step_time(self._runner, self.timestep, self.num_recording_timesteps or 0)
+        if rc:
+            _abi.check(rc)
         self.timestep += 1
 
     def update_synapses(self):
@@ -1018,21 +1086,22 @@ class GeNNModel:
         _abi.check(_abi.load().gennmi_runner_synchronize(self._runner))
 
     def pull_recording_buffers_from_device(self):
-        self.synchronize()
-        for n in self.neuron_populations.values():
-            for name, a in n.vars.items():
-                if name.startswith("recordSpk"):
-                    a.pull_from_device()
+        pull_arrays(self._runner, [a for n in self.neuron_populations.values() for name, a in n.vars.items() if name.startswith("recordSpk")])
+        _abi.check(_abi.load().gennmi_runner_error(self._runner))
 
     def _decode_recording(self, n, var="recordSpk"):
         words = (n.num_neurons + 31) // 32
-        rec = n.vars[var].view.reshape(self.num_recording_timesteps, self.batch_size, words)
-        bits = np.unpackbits(rec.view(np.uint8), axis=2, bitorder="little")[:, :, :n.num_neurons]
+        rec = n.vars[var].view
+        decode, rows = _abi.load().gennmi_decode_recording, self.num_recording_timesteps
         start = self.timestep - self.num_recording_timesteps if self.timestep >= self.num_recording_timesteps else 0
         out = []
         for b in range(self.batch_size):
-            steps, ids = np.nonzero(bits[:, b, :])
-            out.append(((start + steps).astype(np.float64) * self.dt, ids.astype(np.uint32)))
+            first, count = rec.ctypes.data + b * words * 4, C.c_size_t()
+            args = (first, rows, self.batch_size * words, n.num_neurons, float(start), self.dt)
+            _abi.check(decode(*args, None, None, C.byref(count)))
+            times, ids = np.empty(count.value, np.float64), np.empty(count.value, np.uint32)
+            _abi.check(decode(*args, times.ctypes.data, ids.ctypes.data, C.byref(count)))
+            out.append((times, ids))
         return out
 
     @property

@@ -84,6 +84,9 @@ int gennmi_malloc(void **devPtr, size_t bytes);                 /* Array::alloca
  * copies.  Without it devPtr may be NULL.  gennmi_host_free releases the memory. */
 int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr);
 int gennmi_host_free(void *hostPtr);
+/* The same memory, not cleared, for a host side that is about to be written whole.  Pinned memory without zeroCopy is kept for
+ * reuse when it is freed (up to 256 MiB of it). */
+int gennmi_host_acquire(void **hostPtr, size_t bytes);
 int gennmi_free(void *devPtr);                                  /* Array::free      hip/backend.cc:110-128 */
 int gennmi_memcpy_to_device(void *dev, const void *host, size_t bytes);    /* pushToDevice / pushSlice1DToDevice   :130-176 */
 int gennmi_memcpy_from_device(void *host, const void *dev, size_t bytes);  /* pullFromDevice / pullSlice1DFromDevice :142-198 */
@@ -425,6 +428,25 @@ int gennmi_runner_set_step_queue(gennmi_runner *runner, uint32_t maxSteps);
 /* stepTimeFinalise: blocks until everything queued has finished and reports device-side
  * failures (backendCUDAHIP.cc:1400-1411). */
 int gennmi_runner_synchronize(gennmi_runner *runner);
+/* Copies in the order of a runner's steps: behind everything its steps so far (and null-stream work) have to do, complete
+ * when the call returns.  They do what gennmi_memcpy_to_device / _from_device / gennmi_copy_f32 do for arrays that only this
+ * runner and null-stream work touch, without making the runner's stream and the null stream wait for each other.  Before
+ * gennmi_runner_finalise they are null-stream work themselves, and gennmi_runner_push returns when the host array may be
+ * changed.  gennmi_runner_pull copies several arrays with one wait.  gennmi_runner_pull_spikes reads one slot of a spike queue
+ * (pushToDevice / pullFromDevice of Array, hip/backend.cc:130-198; pullCurrentSpikesFromDevice): the counts of all batches,
+ * and the first counts[b] entries of batch b to ids + b * numNeurons. */
+int gennmi_runner_push(gennmi_runner *runner, void *dev, const void *host, size_t bytes);
+int gennmi_runner_pull(gennmi_runner *runner, uint32_t count, void *const *hosts, const void *const *devs, const size_t *bytes);
+int gennmi_runner_pull_spikes(gennmi_runner *runner, const uint32_t *spkCnt, const uint32_t *spk, uint32_t numNeurons, uint32_t slots, uint32_t slot,
+                              uint32_t *counts, uint32_t *ids);
+int gennmi_runner_copy_f32(gennmi_runner *runner, float *dst, const float *src, size_t count);
+/* What gennmi_runner_synchronize would report of the work that has already finished, without waiting. */
+int gennmi_runner_error(const gennmi_runner *runner);
+/* Host-side decoding of a pulled recording buffer (Runtime::getRecordedSpikes, runtime.cc:855-913): numSteps rows of bits, rowStride words
+ * apart.  With times == ids == NULL only *count is written; else *count says how many pairs the arrays hold, time (firstStep + row) * dt
+ * each, neurons ascending within a row. */
+int gennmi_decode_recording(const uint32_t *record, size_t numSteps, size_t rowStride, uint32_t numNeurons, double firstStep, double dt,
+                            double *times, uint32_t *ids, size_t *count);
 
 /* Timers: neuronUpdateTime / presynapticUpdateTime / postsynapticUpdateTime of generateRunner.cc:161-174,
  * in seconds, accumulated with HIP events while enabled (backendCUDAHIP.cc:36-76, 1479-1504).  While timing is enabled
