@@ -49,6 +49,7 @@
 #include "genn_mi355x_ordered_kernels.h"
 #include "genn_mi355x_conv_step_kernels.h"
 #include "genn_mi355x_transfer.h"
+#include "genn_mi355x_pool.h"
 
 struct gennmi_runner
 {
@@ -239,7 +240,7 @@ int gennmi_device_name(char *buf, size_t len)
 
 int gennmi_malloc(void **devPtr, size_t bytes)
 {
-    HIP_TRY(hipMalloc(devPtr, bytes ? bytes : 4));
+    HIP_TRY(poolMalloc(devPtr, bytes ? bytes : 4));
     return GENNMI_OK;
 }
 int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr)
@@ -264,7 +265,7 @@ int gennmi_host_free(void *hostPtr)
     HIP_TRY(e);
     return GENNMI_OK;
 }
-int gennmi_free(void *devPtr) { FLUSH_QUEUED(); HIP_TRY(hipFree(devPtr)); return GENNMI_OK; }
+int gennmi_free(void *devPtr) { FLUSH_QUEUED(); HIP_TRY(poolFree(devPtr)); return GENNMI_OK; }
 int gennmi_memcpy_to_device(void *dev, const void *host, size_t bytes)
 {
     FLUSH_QUEUED();
@@ -479,8 +480,18 @@ int gennmi_profiler_range_pop(void)
 }
 int gennmi_free_device_memory_bytes(size_t *bytes)
 {
-    size_t total = 0;
-    HIP_TRY(hipMemGetInfo(bytes, &total));
+    HIP_TRY(poolFreeBytes(bytes));
+    return GENNMI_OK;
+}
+int gennmi_release_cached_memory(void)
+{
+    FLUSH_QUEUED();
+    {
+        std::lock_guard<std::mutex> lock(g_pool.mutex);
+        HIP_TRY(g_pool.releaseAll());
+    }
+    std::lock_guard<std::mutex> lock(g_pinnedMutex);
+    HIP_TRY(releaseIdlePinned());
     return GENNMI_OK;
 }
 
@@ -500,11 +511,11 @@ int gennmi_runner_create(gennmi_runner **runner, float dt, uint32_t batchSize)
     HIP_TRY(hipStreamCreate(&r->stream));       // blocking stream: ordered against null-stream copies
 
     // the error flag: one pinned host word, which the kernels reach through its device address (raiseErrorFlag)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->hError), 32 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+    { const int rc = pinnedMalloc(reinterpret_cast<void**>(&r->hError), 32 * sizeof(uint32_t)); if(rc) { return rc; } }
     memset(r->hError, 0, 32 * sizeof(uint32_t));
     r->hSignal = r->hError + 16;
     HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&r->dError), r->hError, 0));
-    HIP_TRY(hipMalloc(&r->dEvents, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
+    HIP_TRY(poolMalloc(&r->dEvents, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
     HIP_TRY(hipMemset(r->dEvents, 0, sizeof(unsigned long long) * EVENT_SLOTS * EVENT_SLOT_STRIDE));
     {
         std::lock_guard<std::mutex> lock(g_runnersMutex);
@@ -525,12 +536,12 @@ int gennmi_runner_destroy(gennmi_runner *r)
     hipStreamSynchronize(r->stream);
     for(hipEvent_t e : r->eventPool) { hipEventDestroy(e); }
     for(hipEvent_t e : r->marks) { if(e) { hipEventDestroy(e); } }
-    for(void *q : r->owned) { hipFree(q); }
-    for(void *q : r->zeroOwned) { hipFree(q); }
-    for(void *q : r->orderedOwned) { hipFree(q); }
-    hipFree(r->dOrderedSources); hipFree(r->dOrderedBitmaps);
-    hipFree(r->dTile); hipFree(r->dConvTile);
-    hipFree(r->dNeuron); hipFree(r->dPre); hipFree(r->dPost); hipFree(r->dDense); hipFree(r->dProc); hipFree(r->dAgg); if(r->hError) { hipHostFree(r->hError); } hipFree(r->dEvents);
+    for(void *q : r->owned) { poolFree(q); }
+    for(void *q : r->zeroOwned) { poolFree(q); }
+    for(void *q : r->orderedOwned) { poolFree(q); }
+    poolFree(r->dOrderedSources); poolFree(r->dOrderedBitmaps);
+    poolFree(r->dTile); poolFree(r->dConvTile);
+    poolFree(r->dNeuron); poolFree(r->dPre); poolFree(r->dPost); poolFree(r->dDense); poolFree(r->dProc); poolFree(r->dAgg); if(r->hError) { hipError_t e; pinnedFree(r->hError, &e); } poolFree(r->dEvents);
     hipStreamDestroy(r->stream);
     delete r;
     return GENNMI_OK;
@@ -791,7 +802,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         if(incoming > RES_MAX_PROJ) { return GENNMI_OK; }
     }
     uint32_t *dFlag = nullptr;
-    HIP_TRY(hipMalloc(&dFlag, sizeof(uint32_t)));
+    HIP_TRY(poolMalloc(&dFlag, sizeof(uint32_t)));
     HIP_TRY(hipMemset(dFlag, 0, sizeof(uint32_t)));
     for(const auto &p : r->pre) {
         const size_t entries = (size_t)p.g.numSrcNeurons * p.g.rowStride;
@@ -800,7 +811,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     HIP_TRY(hipGetLastError());
     uint32_t unsorted = 0;
     HIP_TRY(hipMemcpy(&unsorted, dFlag, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipFree(dFlag));
+    HIP_TRY(poolFree(dFlag));
     if(unsorted) { return GENNMI_OK; }
     for(size_t k = 0; k < r->pre.size(); k++) {
         const auto &q = r->pre[k].g;
@@ -809,7 +820,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         const size_t entries = (size_t)q.numSrcNeurons * tilesInGroup;
         if(q.rowStride > 0xFFFFu) { return GENNMI_OK; }         // a segment's length is a 16-bit field (device allocations made so far stay owned)
         u32x4 *dSeg = nullptr;
-        HIP_TRY(hipMalloc(&dSeg, entries * 2 * sizeof(u32x4)));
+        HIP_TRY(poolMalloc(&dSeg, entries * 2 * sizeof(u32x4)));
         r->owned.push_back(dSeg);
         const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d,
@@ -819,7 +830,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         HIP_TRY(hipGetLastError());
         const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
         u32x2 *dPacked = nullptr;
-        if(hipMalloc(&dPacked, std::max<size_t>(padded, 1) * sizeof(u32x2)) != hipSuccess) {
+        if(poolMalloc(&dPacked, std::max<size_t>(padded, 1) * sizeof(u32x2)) != hipSuccess) {
             (void)hipGetLastError();            // no room for the second copy of the synapses: the network steps with the other plans
             return GENNMI_OK;
         }
@@ -840,7 +851,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         }
     }
     auto upload = [r](void **dst, const void *src, size_t bytes) -> hipError_t {
-        hipError_t e = hipMalloc(dst, bytes);
+        hipError_t e = poolMalloc(dst, bytes);
         if(e != hipSuccess) { return e; }
         r->owned.push_back(*dst);
         return hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
@@ -850,12 +861,12 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     HIP_TRY(upload((void**)&r->dResGroups, groups.data(), groups.size() * sizeof(NeuronGroupDev)));
     HIP_TRY(upload((void**)&r->dResTileGroup, tileGroup.data(), tileGroup.size()));
     r->resReplicaStride = (uint32_t)((2 * tiles.size() + 511) / 512 * 512);          // in words: copies start 4 KiB-aligned
-    HIP_TRY(hipMalloc(&r->dResTags, (size_t)RES_REPLICAS * r->resReplicaStride * sizeof(unsigned long long)));
+    HIP_TRY(poolMalloc(&r->dResTags, (size_t)RES_REPLICAS * r->resReplicaStride * sizeof(unsigned long long)));
     r->owned.push_back(r->dResTags);
     // cleared once: sequence number 0 is the one no work-group ever waits for before it has come round again
     HIP_TRY(hipMemset(r->dResTags, 0, (size_t)RES_REPLICAS * r->resReplicaStride * sizeof(unsigned long long)));
     r->resSeq = 0;
-    HIP_TRY(hipMalloc(&r->dResSide, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
+    HIP_TRY(poolMalloc(&r->dResSide, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
     r->owned.push_back(r->dResSide);
     // (cleared once as well: its entries name their exchange by the unwrapped sequence number, which starts at 1)
     HIP_TRY(hipMemset(r->dResSide, 0, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
@@ -914,10 +925,10 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
 // connectivity has been rewritten; the caller then uploads the descriptor tables.
 static int buildZeroDelayLists(gennmi_runner *r)
 {
-    for(void *q : r->zeroOwned) { hipFree(q); }
+    for(void *q : r->zeroOwned) { poolFree(q); }
     r->zeroOwned.clear();
     auto devAlloc = [](std::vector<void*> &owner, void **q, size_t bytes) -> hipError_t {
-        hipError_t e = hipMalloc(q, bytes ? bytes : 4);
+        hipError_t e = poolMalloc(q, bytes ? bytes : 4);
         if(e == hipSuccess) { owner.push_back(*q); e = hipMemset(*q, 0, bytes ? bytes : 4); }
         return e;
     };
@@ -1001,17 +1012,25 @@ static int pendingZeroDelay(gennmi_runner *r, std::map<std::pair<const float*, u
     return GENNMI_OK;
 }
 
-// Segment boundaries of the tile path for one projection; rows that are not sorted by target are reported through *unsorted
-static int buildTileOffsets(const gennmi_presynaptic_update_group_t &g, uint16_t *dOff, uint32_t tileSize, uint32_t numTiles, uint32_t *unsorted)
+// Segment boundaries of the tile path for some projections; one word each says whether rows are not sorted by target
+struct TileOffsetsOf { const gennmi_presynaptic_update_group_t *g; uint16_t *off; uint32_t tileSize, numTiles; };
+static int buildTileOffsets(const std::vector<TileOffsetsOf> &projections, std::vector<uint32_t> &unsorted)
 {
-    uint32_t *dFlag = nullptr;
-    HIP_TRY(hipMalloc(&dFlag, sizeof(uint32_t)));
-    HIP_TRY(hipMemset(dFlag, 0, sizeof(uint32_t)));
-    tileOffsetKernel<<<dim3((g.numSrcNeurons + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, 0>>>(
-        g.numSrcNeurons, g.rowStride, g.rowLength, g.ind, tileSize, numTiles, dOff, dFlag);
+    unsorted.assign(projections.size(), 0u);
+    if(projections.empty()) { return GENNMI_OK; }
+    uint32_t *dFlags = nullptr;
+    HIP_TRY(poolMalloc(&dFlags, projections.size() * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(dFlags, 0, projections.size() * sizeof(uint32_t)));
+    for(size_t k = 0; k < projections.size(); k++) {
+        const auto &p = projections[k];
+        const uint32_t shift = ((p.tileSize & (p.tileSize - 1)) == 0) ? (uint32_t)__builtin_ctz(p.tileSize) : 32u;
+        tileOffsetKernel<<<dim3((p.g->numSrcNeurons + BLOCK / WAVE - 1) / (BLOCK / WAVE)), dim3(BLOCK), 0, 0>>>(
+            p.g->numSrcNeurons, p.g->rowStride, p.g->rowLength, p.g->ind, p.tileSize, shift, p.numTiles, p.off, dFlags + k);
+    }
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpy(unsorted, dFlag, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipFree(dFlag));
+    const TransferPart part{reinterpret_cast<uint8_t*>(unsorted.data()), reinterpret_cast<uint8_t*>(dFlags), projections.size() * sizeof(uint32_t)};
+    { const int rc = pullParts(&part, 1, nullptr); if(rc) { return rc; } }
+    HIP_TRY(poolFree(dFlags));
     return GENNMI_OK;
 }
 
@@ -1020,11 +1039,11 @@ static int buildTileOffsets(const gennmi_presynaptic_update_group_t &g, uint16_t
 // whenever the connectivity has been rewritten.
 static int buildOrderedViews(gennmi_runner *r)
 {
-    for(void *q : r->orderedOwned) { hipFree(q); }
+    for(void *q : r->orderedOwned) { poolFree(q); }
     r->orderedOwned.clear();
     r->orderedGroups.clear(); r->orderedPre.clear(); r->orderedSources.clear();
-    if(r->dOrderedSources) { HIP_TRY(hipFree(r->dOrderedSources)); r->dOrderedSources = nullptr; }
-    if(r->dOrderedBitmaps) { HIP_TRY(hipFree(r->dOrderedBitmaps)); r->dOrderedBitmaps = nullptr; }
+    if(r->dOrderedSources) { HIP_TRY(poolFree(r->dOrderedSources)); r->dOrderedSources = nullptr; }
+    if(r->dOrderedBitmaps) { HIP_TRY(poolFree(r->dOrderedBitmaps)); r->dOrderedBitmaps = nullptr; }
     std::vector<size_t> bitmapOffset;       // of every source, in words
     size_t words = 0;
     for(size_t k = 0; k < r->pre.size(); k++) {
@@ -1042,9 +1061,9 @@ static int buildOrderedViews(gennmi_runner *r)
         o.g = g;
         o.colStride = std::max(1u, maxLen);
         uint32_t *colLength = nullptr, *remap = nullptr;
-        HIP_TRY(hipMalloc(&colLength, (size_t)g.numTrgNeurons * sizeof(uint32_t)));
+        HIP_TRY(poolMalloc(&colLength, (size_t)g.numTrgNeurons * sizeof(uint32_t)));
         r->orderedOwned.push_back(colLength);
-        HIP_TRY(hipMalloc(&remap, (size_t)g.numTrgNeurons * o.colStride * sizeof(uint32_t)));
+        HIP_TRY(poolMalloc(&remap, (size_t)g.numTrgNeurons * o.colStride * sizeof(uint32_t)));
         r->orderedOwned.push_back(remap);
         { const int rc = gennmi_build_remap(g.numSrcNeurons, g.numTrgNeurons, g.rowStride, o.colStride, g.rowLength, g.ind, colLength, remap); if(rc) { return rc; } }
         o.colLength = colLength; o.remap = remap;
@@ -1071,7 +1090,7 @@ static int buildOrderedViews(gennmi_runner *r)
     r->scatterNeeded = false;
     for(const auto &p : r->pre) { r->scatterNeeded = r->scatterNeeded || !p.ordered; }
     if(r->orderedGroups.empty()) { return GENNMI_OK; }
-    HIP_TRY(hipMalloc(&r->dOrderedBitmaps, words * sizeof(uint32_t)));
+    HIP_TRY(poolMalloc(&r->dOrderedBitmaps, words * sizeof(uint32_t)));
     HIP_TRY(hipMemset(r->dOrderedBitmaps, 0, words * sizeof(uint32_t)));
     r->orderedBitmapWords = words;
     for(auto &o : r->orderedGroups) { o.bitmap = r->dOrderedBitmaps + reinterpret_cast<uintptr_t>(o.bitmap); }
@@ -1085,7 +1104,7 @@ static int buildOrderedViews(gennmi_runner *r)
         for(uint32_t b = 0; b < c.numBlocks; b++) { table.push_back(c); }
     }
     r->orderedSourceBlocks = block;
-    HIP_TRY(hipMalloc(&r->dOrderedSources, table.size() * sizeof(OrderedSourceDev)));
+    HIP_TRY(poolMalloc(&r->dOrderedSources, table.size() * sizeof(OrderedSourceDev)));
     HIP_TRY(hipMemcpy(r->dOrderedSources, table.data(), table.size() * sizeof(OrderedSourceDev), hipMemcpyHostToDevice));
     return GENNMI_OK;
 }
@@ -1119,9 +1138,11 @@ static int refreshTables(gennmi_runner *r)
         for(const auto &t : r->recordTables) { const int rc = buildTileRecords(r, t); if(rc) { return rc; } }
         return GENNMI_OK;
     }
-    for(const auto &t : r->tileTables) {
-        uint32_t unsorted = 0;
-        { const int rc = buildTileOffsets(r->pre[t.pre].g, t.off, t.tileSize, t.numTiles, &unsorted); if(rc) { return rc; } }
+    std::vector<TileOffsetsOf> offsets;
+    std::vector<uint32_t> unsortedFlags;
+    for(const auto &t : r->tileTables) { offsets.push_back({&r->pre[t.pre].g, t.off, t.tileSize, t.numTiles}); }
+    { const int rc = buildTileOffsets(offsets, unsortedFlags); if(rc) { return rc; } }
+    for(const uint32_t unsorted : unsortedFlags) {
         if(unsorted) {
             return fail(GENNMI_ESTATE, "connectivity written after load leaves the rows of a projection no longer sorted by target, which its launch plan relies on; "
                                        "sort the rows or set GENNMI_TILE_FLOATS=0 before the runner is finalised");
@@ -1143,12 +1164,12 @@ static int refreshTables(gennmi_runner *r)
         for(const auto &e : before) { if(!after.count(e.first)) { fix.push_back({e.second, e.first.first, -1.0f, 0u}); } }
         if(!fix.empty()) {
             ZeroDelayCorrection *dFix = nullptr;
-            HIP_TRY(hipMalloc(&dFix, fix.size() * sizeof(ZeroDelayCorrection)));
+            HIP_TRY(poolMalloc(&dFix, fix.size() * sizeof(ZeroDelayCorrection)));
             HIP_TRY(hipMemcpy(dFix, fix.data(), fix.size() * sizeof(ZeroDelayCorrection), hipMemcpyHostToDevice));
             zeroDelayCorrectionKernel<<<dim3((unsigned int)((fix.size() + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(dFix, (uint32_t)fix.size());
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipDeviceSynchronize());
-            HIP_TRY(hipFree(dFix));
+            HIP_TRY(poolFree(dFix));
         }
         // the per-block descriptor tables carry the lists' addresses: same layout, new contents
         std::vector<NeuronGroupDev> neuronTable;
@@ -1212,7 +1233,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
         {
             if(n->spikeBitmap) { return hipSuccess; }
             const size_t bytes = (size_t)r->batch * ((n->g.numNeurons + 31) / 32) * sizeof(uint32_t);
-            hipError_t e = hipMalloc((void**)&n->spikeBitmap, bytes);
+            hipError_t e = poolMalloc((void**)&n->spikeBitmap, bytes);
             if(e != hipSuccess) { return e; }
             r->owned.push_back(n->spikeBitmap);
             return hipMemset(n->spikeBitmap, 0, bytes);
@@ -1293,18 +1314,23 @@ int gennmi_runner_finalise(gennmi_runner *r)
     }
     r->procBlocks = block;
 
+    // (null-stream work like everything else here: the call ends with a wait for all of it)
+    auto upload = [](void *dev, const void *host, size_t bytes) -> hipError_t {
+        const TransferPart part{static_cast<uint8_t*>(const_cast<void*>(host)), static_cast<uint8_t*>(dev), bytes};
+        return pushArray(part, nullptr, false) ? hipErrorUnknown : hipSuccess;
+    };
     // One descriptor copy per block, indexed by blockIdx.x: a block finds everything it needs with a
     // single round of scalar loads (the reference bisects a start-ID table and then loads the merged
     // struct, backendSIMT.h:244-323 — two to four dependent loads before any work starts).
-    auto uploadPerBlock = [](const auto &groups, uint32_t totalBlocks, auto **dTable) -> hipError_t {
+    auto uploadPerBlock = [&](const auto &groups, uint32_t totalBlocks, auto **dTable) -> hipError_t {
         using T = typename std::remove_reference<decltype(groups[0])>::type;
         std::vector<typename std::remove_const<T>::type> table;
         table.reserve(totalBlocks);
         for(const auto &g : groups) { for(uint32_t b = 0; b < g.numBlocks; b++) { table.push_back(g); } }
         if(table.empty()) { *dTable = nullptr; return hipSuccess; }
-        hipError_t e = hipMalloc(dTable, table.size() * sizeof(table[0]));
+        hipError_t e = poolMalloc(dTable, table.size() * sizeof(table[0]));
         if(e != hipSuccess) { return e; }
-        return hipMemcpy(*dTable, table.data(), table.size() * sizeof(table[0]), hipMemcpyHostToDevice);
+        return upload(*dTable, table.data(), table.size() * sizeof(table[0]));
     };
     // ---- tile path for delay-free SPARSE projections (static or trace-STDP weights) whose rows are sorted by target
     {
@@ -1315,6 +1341,23 @@ int gennmi_runner_finalise(gennmi_runner *r)
         r->tileThreads = envThreads ? (uint32_t)std::min(1024, std::max(64, atoi(envThreads))) : (tileFloats > 16384 ? 1024u : (tileFloats > 8192 ? 512u : (uint32_t)BLOCK));
         std::vector<TileGroupDev> tiles, tileGroups;
         std::vector<ConvTileDev> convTiles;
+        // segment boundaries of every projection that could take the tile path, built together
+        auto tileCandidate = [&](const PreGroupDev &p) {
+            return tileFloats != 0 && p.g.numSrcDelaySlots <= 1 && p.g.matrix == GENNMI_MATRIX_SPARSE && p.g.rowStride <= 65535
+                   && (p.g.wum == GENNMI_WUM_STATIC_PULSE || p.g.wum == GENNMI_WUM_STDP_TRACE || p.g.wum == GENNMI_WUM_STDP);
+        };
+        std::vector<TileOffsetsOf> offsets;
+        std::vector<uint32_t> unsortedFlags;
+        for(const auto &p : r->pre) {
+            if(!tileCandidate(p)) { continue; }
+            const uint32_t tileSize = std::min(tileFloats, p.g.numTrgNeurons), numTiles = (p.g.numTrgNeurons + tileSize - 1) / tileSize;
+            uint16_t *dOff = nullptr;
+            HIP_TRY(poolMalloc(&dOff, (size_t)p.g.numSrcNeurons * (numTiles + 1) * sizeof(uint16_t)));
+            r->owned.push_back(dOff);
+            offsets.push_back({&p.g, dOff, tileSize, numTiles});
+        }
+        { const int rc = buildTileOffsets(offsets, unsortedFlags); if(rc) { return rc; } }
+        size_t candidate = 0;
         for(auto &p : r->pre) {
             p.workPerSpike = (p.g.matrix == GENNMI_MATRIX_SPARSE) ? p.g.rowStride : (uint32_t)(p.g.conv[0] * p.g.conv[1] * p.g.conv[7]);
             if(p.g.numSrcDelaySlots > 1) { continue; }       // the tile kernels read the queue without delay slots
@@ -1349,7 +1392,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
                         if(bytes <= 64 * 1024) {
                             if(!src->spikeBitmap) {
                                 const size_t bitmapBytes = (size_t)r->batch * ((src->g.numNeurons + 31) / 32) * sizeof(uint32_t);
-                                HIP_TRY(hipMalloc((void**)&src->spikeBitmap, bitmapBytes));
+                                HIP_TRY(poolMalloc((void**)&src->spikeBitmap, bitmapBytes));
                                 r->owned.push_back(src->spikeBitmap);
                                 HIP_TRY(hipMemset(src->spikeBitmap, 0, bitmapBytes));
                                 r->bitmapsStale = true;          // the queue may already hold spikes
@@ -1361,8 +1404,8 @@ int gennmi_runner_finalise(gennmi_runner *r)
                             p.tileThreshold = std::max(1u, p.g.numTrgNeurons / 4);
                             m.threshold = p.tileThreshold;
                             r->convMfma = m;
-                            HIP_TRY(hipMalloc(&r->dConvMfma, sizeof(ConvMfmaDev)));
-                            HIP_TRY(hipMemcpy(r->dConvMfma, &m, sizeof(ConvMfmaDev), hipMemcpyHostToDevice));
+                            HIP_TRY(poolMalloc(&r->dConvMfma, sizeof(ConvMfmaDev)));
+                            HIP_TRY(upload(r->dConvMfma, &m, sizeof(ConvMfmaDev)));
                             r->owned.push_back(r->dConvMfma);
                             r->convMfmaBlocks = ((uint32_t)c[5] + rowsPerBlock - 1) / rowsPerBlock;
                             r->convMfmaBytes = bytes;
@@ -1395,15 +1438,9 @@ int gennmi_runner_finalise(gennmi_runner *r)
                 }
                 continue;
             }
-            if(tileFloats == 0 || p.g.matrix != GENNMI_MATRIX_SPARSE || p.g.rowStride > 65535
-               || (p.g.wum != GENNMI_WUM_STATIC_PULSE && p.g.wum != GENNMI_WUM_STDP_TRACE && p.g.wum != GENNMI_WUM_STDP)) { continue; }
-            const uint32_t tileSize = std::min(tileFloats, p.g.numTrgNeurons);
-            const uint32_t numTiles = (p.g.numTrgNeurons + tileSize - 1) / tileSize;
-            uint16_t *dOff = nullptr;
-            HIP_TRY(hipMalloc(&dOff, (size_t)p.g.numSrcNeurons * (numTiles + 1) * sizeof(uint16_t)));
-            r->owned.push_back(dOff);
-            uint32_t unsorted = 0;
-            { const int rc = buildTileOffsets(p.g, dOff, tileSize, numTiles, &unsorted); if(rc) { return rc; } }
+            if(!tileCandidate(p)) { continue; }
+            const uint32_t tileSize = offsets[candidate].tileSize, numTiles = offsets[candidate].numTiles, unsorted = unsortedFlags[candidate];
+            uint16_t *dOff = offsets[candidate++].off;
             if(unsorted) { continue; }          // rows not sorted by target: the scatter kernel handles every step
             p.tileThreshold = std::max(1u, p.g.numTrgNeurons);
             r->tileTables.push_back({(size_t)(&p - r->pre.data()), dOff, tileSize, numTiles});
@@ -1421,18 +1458,18 @@ int gennmi_runner_finalise(gennmi_runner *r)
             if(!(envRecords && atoi(envRecords) == 0) && p.g.wum == GENNMI_WUM_STATIC_PULSE && segLen >= 6 && segLen <= 34 && tileSize <= 65536) {
                 const uint32_t lanes = (segLen <= 17) ? 5u : 10u;
                 const size_t bytes = (size_t)numTiles * p.g.numSrcNeurons * recordBytes(lanes);
-                size_t freeBytes = 0, totalBytes = 0;
-                HIP_TRY(hipMemGetInfo(&freeBytes, &totalBytes));
+                size_t freeBytes = 0;
+                HIP_TRY(poolFreeBytes(&freeBytes));
                 if(bytes + (size_t(2) << 30) < freeBytes) {
                     uint8_t *records = nullptr;
-                    HIP_TRY(hipMalloc(&records, bytes));
+                    HIP_TRY(poolMalloc(&records, bytes));
                     r->owned.push_back(records);
                     // overflow records where memory allows: segments are Poisson-like around rowStride / numTiles, so a
                     // sixth or so of them exceed a record sized for the mean
                     uint8_t *overflow = nullptr;
                     const size_t overflowBytes = (size_t)numTiles * p.g.numSrcNeurons * 64;
                     if(bytes + overflowBytes + (size_t(2) << 30) < freeBytes) {
-                        HIP_TRY(hipMalloc(&overflow, overflowBytes));
+                        HIP_TRY(poolMalloc(&overflow, overflowBytes));
                         r->owned.push_back(overflow);
                     }
                     const gennmi_runner::RecordTable table{(size_t)(&p - r->pre.data()), records, overflow, dOff, lanes, tileSize, numTiles};
@@ -1469,7 +1506,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
             }
         }
         if(!convTiles.empty()) {
-            HIP_TRY(hipMalloc(&r->dConvTile, convTiles.size() * sizeof(ConvTileDev)));
+            HIP_TRY(poolMalloc(&r->dConvTile, convTiles.size() * sizeof(ConvTileDev)));
             HIP_TRY(hipMemcpy(r->dConvTile, convTiles.data(), convTiles.size() * sizeof(ConvTileDev), hipMemcpyHostToDevice));
             r->convTileBlocks = (uint32_t)convTiles.size();
             if(r->convTileBytes > 48 * 1024) {
@@ -1478,8 +1515,8 @@ int gennmi_runner_finalise(gennmi_runner *r)
             }
         }
         if(!tiles.empty()) {
-            HIP_TRY(hipMalloc(&r->dTile, tiles.size() * sizeof(TileGroupDev)));
-            HIP_TRY(hipMemcpy(r->dTile, tiles.data(), tiles.size() * sizeof(TileGroupDev), hipMemcpyHostToDevice));
+            HIP_TRY(poolMalloc(&r->dTile, tiles.size() * sizeof(TileGroupDev)));
+            HIP_TRY(upload(r->dTile, tiles.data(), tiles.size() * sizeof(TileGroupDev)));
             r->tileBlocks = (uint32_t)tiles.size();
             if((size_t)r->tileFloats * sizeof(float) > 48 * 1024) {
                 HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(presynapticTileKernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1573,7 +1610,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
             for(uint32_t q = 0; q < n.g.numExtraSpk; q++) { feeds = feeds || (n.g.extraSpk[q] == p.g.trgSpk); }
             if(!feeds || n.g.numNeurons != p.g.numTrgNeurons) { continue; }
             if(!n.spikeBitmap) {
-                HIP_TRY(hipMalloc((void**)&n.spikeBitmap, (size_t)r->batch * words * sizeof(uint32_t)));
+                HIP_TRY(poolMalloc((void**)&n.spikeBitmap, (size_t)r->batch * words * sizeof(uint32_t)));
                 HIP_TRY(hipMemset(n.spikeBitmap, 0, (size_t)r->batch * words * sizeof(uint32_t)));
                 r->owned.push_back(n.spikeBitmap);
             }
@@ -1604,7 +1641,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
         hipDeviceptr_t base = nullptr; size_t size = 0;
         HIP_TRY(hipMemGetAddressRange(&base, &size, const_cast<float*>(n.g.spikeTimes)));
         n.spikeTimesBytes = (reinterpret_cast<uintptr_t>(base) + size) - reinterpret_cast<uintptr_t>(n.g.spikeTimes);
-        HIP_TRY(hipMalloc(&n.nextSpikeTime, (size_t)r->batch * n.g.numNeurons * sizeof(float)));
+        HIP_TRY(poolMalloc(&n.nextSpikeTime, (size_t)r->batch * n.g.numNeurons * sizeof(float)));
         r->owned.push_back(n.nextSpikeTime);
         r->sourcesStale = true;
     }
@@ -1612,7 +1649,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
     if(anyEvents) {
         const size_t count = (size_t)GENNMI_MAX_SPK_EVENT * 2 * r->neuronBlocks * r->batch;
         unsigned long long *area = nullptr;
-        HIP_TRY(hipMalloc(&area, count * sizeof(unsigned long long)));
+        HIP_TRY(poolMalloc(&area, count * sizeof(unsigned long long)));
         r->owned.push_back(area);
         HIP_TRY(hipMemset(area, 0, count * sizeof(unsigned long long)));
         for(auto &n : r->neuron) { n.aggEvent = area; }
@@ -1643,7 +1680,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
             // the source's spike bitmap twice: the layer reads last step's copy while the source's blocks of the same launch write this step's
             const size_t words = (size_t)r->batch * ((src->g.numNeurons + 31) / 32);
             uint32_t *both = nullptr;
-            HIP_TRY(hipMalloc((void**)&both, 2 * words * sizeof(uint32_t)));
+            HIP_TRY(poolMalloc((void**)&both, 2 * words * sizeof(uint32_t)));
             r->owned.push_back(both);
             HIP_TRY(hipMemset(both, 0, 2 * words * sizeof(uint32_t)));
             src->spikeBitmap = both; src->bitmapStride = words;
@@ -1661,14 +1698,14 @@ int gennmi_runner_finalise(gennmi_runner *r)
             }
             r->convRestBlocks = block;
             m.restBlocks = block; m.restNeuronsPerLane = r->neuronsPerLane;
-            HIP_TRY(hipMemcpy(r->dConvMfma, &m, sizeof(ConvMfmaDev), hipMemcpyHostToDevice));
+            HIP_TRY(upload(r->dConvMfma, &m, sizeof(ConvMfmaDev)));
             HIP_TRY(uploadPerBlock(rest, r->convRestBlocks, &r->dConvRest));
-            HIP_TRY(hipMalloc(&r->dConvTarget, sizeof(NeuronGroupDev)));
-            HIP_TRY(hipMemcpy(r->dConvTarget, target, sizeof(NeuronGroupDev), hipMemcpyHostToDevice));
+            HIP_TRY(poolMalloc(&r->dConvTarget, sizeof(NeuronGroupDev)));
+            HIP_TRY(upload(r->dConvTarget, target, sizeof(NeuronGroupDev)));
             const size_t aggCount = 2 * (size_t)r->convMfmaBlocks * r->batch, restCount = 2 * (size_t)std::max(1u, r->convRestBlocks) * r->batch;
-            HIP_TRY(hipMalloc(&r->dConvAgg, aggCount * sizeof(unsigned long long)));
+            HIP_TRY(poolMalloc(&r->dConvAgg, aggCount * sizeof(unsigned long long)));
             HIP_TRY(hipMemset(r->dConvAgg, 0, aggCount * sizeof(unsigned long long)));
-            HIP_TRY(hipMalloc(&r->dConvRestAgg, restCount * sizeof(unsigned long long)));
+            HIP_TRY(poolMalloc(&r->dConvRestAgg, restCount * sizeof(unsigned long long)));
             HIP_TRY(hipMemset(r->dConvRestAgg, 0, restCount * sizeof(unsigned long long)));
             for(void *q : {(void*)r->dConvRest, (void*)r->dConvTarget, (void*)r->dConvAgg, (void*)r->dConvRestAgg}) { if(q) { r->owned.push_back(q); } }
             r->convStepBytes = bytes;
@@ -1684,16 +1721,20 @@ int gennmi_runner_finalise(gennmi_runner *r)
     HIP_TRY(uploadPerBlock(r->dense, r->denseBlocks, &r->dDense));
     HIP_TRY(uploadPerBlock(r->proc, r->procBlocks, &r->dProc));
     const size_t aggCount = 2 * (size_t)r->neuronBlocks * r->batch;       // per-block counts, then per-group totals
-    HIP_TRY(hipMalloc(&r->dAgg, aggCount * sizeof(unsigned long long)));
+    HIP_TRY(poolMalloc(&r->dAgg, aggCount * sizeof(unsigned long long)));
     HIP_TRY(hipMemset(r->dAgg, 0, aggCount * sizeof(unsigned long long)));
     if(!r->ordered) { const int rc = setupResident(r, numCU); if(rc) { return rc; } }
-    if(const char *envSpin = getenv("GENNMI_SPIN_LIMIT")) {
-        const uint32_t limit = (uint32_t)std::max(0ll, atoll(envSpin));
-        HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_spinLimit), &limit, sizeof(limit)));
-    }
-    else {
-        const uint32_t limit = SPIN_LIMIT;
-        HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_spinLimit), &limit, sizeof(limit)));
+    {
+        const char *envSpin = getenv("GENNMI_SPIN_LIMIT");
+        const uint32_t limit = envSpin ? (uint32_t)std::max(0ll, atoll(envSpin)) : SPIN_LIMIT;
+        static std::mutex spinMutex;
+        static std::map<int, uint32_t> spinLimits;      // what each device's copy holds, where it is not the default it is built with
+        std::lock_guard<std::mutex> lock(spinMutex);
+        const auto held = spinLimits.find(device);
+        if(limit != (held == spinLimits.end() ? SPIN_LIMIT : held->second)) {
+            HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(c_spinLimit), &limit, sizeof(limit)));
+            spinLimits[device] = limit;
+        }
     }
     HIP_TRY(hipDeviceSynchronize());
     r->finalised = true;
@@ -2170,14 +2211,14 @@ int gennmi_max_col_length(uint32_t numSrc, uint32_t numTrg, uint32_t rowStride, 
     if(!rowLength || !ind || !maxColLength || rowStride == 0) { return fail(GENNMI_EINVAL, "max_col_length: bad arguments"); }
     FLUSH_QUEUED();
     uint32_t *dCount = nullptr;
-    HIP_TRY(hipMalloc(&dCount, (size_t)numTrg * sizeof(uint32_t)));
+    HIP_TRY(poolMalloc(&dCount, (size_t)numTrg * sizeof(uint32_t)));
     HIP_TRY(hipMemset(dCount, 0, (size_t)numTrg * sizeof(uint32_t)));
     const size_t total = (size_t)numSrc * rowStride;
     remapCountKernel<<<dim3((unsigned int)((total + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(numSrc, rowStride, rowLength, ind, 0, dCount, nullptr, nullptr);
     HIP_TRY(hipGetLastError());
     std::vector<uint32_t> h(numTrg);
     HIP_TRY(hipMemcpy(h.data(), dCount, (size_t)numTrg * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipFree(dCount));
+    HIP_TRY(poolFree(dCount));
     uint32_t m = 0;
     for(uint32_t v : h) { m = std::max(m, v); }
     *maxColLength = m;
@@ -2267,7 +2308,7 @@ int gennmi_build_remap(uint32_t numSrc, uint32_t numTrg, uint32_t rowStride, uin
     if(!rowLength || !ind || !colLength || !remap || rowStride == 0 || colStride == 0) { return fail(GENNMI_EINVAL, "build_remap: bad arguments"); }
     FLUSH_QUEUED();
     uint32_t *dOverflow = nullptr;
-    HIP_TRY(hipMalloc(&dOverflow, sizeof(uint32_t)));
+    HIP_TRY(poolMalloc(&dOverflow, sizeof(uint32_t)));
     HIP_TRY(hipMemset(dOverflow, 0, sizeof(uint32_t)));
     HIP_TRY(hipMemset(colLength, 0, (size_t)numTrg * sizeof(uint32_t)));
     const size_t total = (size_t)numSrc * rowStride;
@@ -2275,7 +2316,7 @@ int gennmi_build_remap(uint32_t numSrc, uint32_t numTrg, uint32_t rowStride, uin
     HIP_TRY(hipGetLastError());
     uint32_t overflow = 0;
     HIP_TRY(hipMemcpy(&overflow, dOverflow, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipFree(dOverflow));
+    HIP_TRY(poolFree(dOverflow));
     if(overflow) { return fail(GENNMI_EINVAL, "build_remap: a column holds " + std::to_string(overflow) + " synapses, more than colStride"); }
     const size_t lds = (size_t)pow2Ceil(std::min(colStride, REMAP_SORT_MAX)) * sizeof(uint32_t);
     if(lds > 48 * 1024) {

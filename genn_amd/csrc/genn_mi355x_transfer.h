@@ -318,7 +318,7 @@ int pullParts(const TransferPart *parts, uint32_t count, hipStream_t stream)
 int pushArray(const TransferPart &part, hipStream_t stream, bool wait)
 {
     if(part.bytes == 0) { return GENNMI_OK; }
-    if(part.bytes > PUSH_RING_BYTES && !isPinned(part.host, part.bytes)) {
+    if(part.bytes > (wait ? PUSH_RING_BYTES : 2 * TRANSFER_CHUNK) && !isPinned(part.host, part.bytes)) {
         HIP_TRY(hipMemcpyAsync(part.dev, part.host, part.bytes, hipMemcpyHostToDevice, stream));
         HIP_TRY(hipStreamSynchronize(stream));
         return GENNMI_OK;

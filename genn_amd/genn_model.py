@@ -9,6 +9,7 @@ All device work goes through the C ABI in include/genn_mi355x.h; nothing here co
 simulation on the host.
 """
 import ctypes as C
+import functools
 import math
 import time
 from fractions import Fraction
@@ -23,6 +24,7 @@ FLT_MAX = np.float32(3.402823466e+38)
 # --------------------------------------------------------------------------------------------
 # numeric literal handling
 # --------------------------------------------------------------------------------------------
+@functools.lru_cache(maxsize=4096)
 def lit32(x):
     """fp32 value of a parameter the reference bakes into generated code as a literal:
     double -> ``%.9e`` text -> correctly rounded float (src/genn/genn/type.cc:329-350)."""
@@ -190,7 +192,7 @@ class Array:
         self._dev = C.c_void_p()
         _abi.check(_abi.load().gennmi_malloc(C.byref(self._dev), self.count * self.dtype.itemsize))
         self._view = None
-        self._fill = fill
+        self._fill, self._given = fill, False
         # (the first value is written on the device; the host copy is made when somebody asks for it)
         if device_only or not self.count:
             pass
@@ -205,7 +207,10 @@ class Array:
     @property
     def view(self):
         if self._view is None:
-            self._make_view().fill(0 if self._fill is None else self._fill)
+            if self._given:
+                self.pull_from_device()
+            else:
+                self._make_view().fill(0 if self._fill is None else self._fill)
         return self._view
 
     def _make_view(self):
@@ -239,7 +244,7 @@ class Array:
 
     def pull_from_device(self):
         pull_arrays(self._runner, [self])
-        return self.view
+        return self._view
 
     def pull_slice(self, first, count):
         """Elements first .. first + count - 1 from the device, as a new array (for arrays too large to mirror on the host)."""
@@ -279,11 +284,11 @@ def pull_arrays(runner, arrays):
     lib = _abi.load()
     if runner is None:
         for a in arrays:
-            _abi.check(lib.gennmi_memcpy_from_device(a.view.ctypes.data, a._dev, a.view.nbytes))
+            _abi.check(lib.gennmi_memcpy_from_device(a._view.ctypes.data, a._dev, a._view.nbytes))
     elif arrays:
         n = len(arrays)
-        hosts, devs = (C.c_void_p * n)(*(a.view.ctypes.data for a in arrays)), (C.c_void_p * n)(*(a._dev.value for a in arrays))
-        _abi.check(lib.gennmi_runner_pull(runner, n, hosts, devs, (C.c_size_t * n)(*(a.view.nbytes for a in arrays))))
+        hosts, devs = (C.c_void_p * n)(*(a._view.ctypes.data for a in arrays)), (C.c_void_p * n)(*(a._dev.value for a in arrays))
+        _abi.check(lib.gennmi_runner_pull(runner, n, hosts, devs, (C.c_size_t * n)(*(a._view.nbytes for a in arrays))))
 
 
 class NeuronGroup:
@@ -588,6 +593,14 @@ class GeNNModel:
         a.init_on_device(init, self.seed, self._next_stream() if stream is None else stream, self.dt)
         return a
 
+    def _alloc_given(self, values):
+        """An array the device only reads, from the user's values; its own host copy is pulled when somebody asks for it."""
+        a = self._alloc(values.size, values.dtype, device_only=True)
+        a._given = True
+        if values.nbytes:
+            _abi.check(_abi.load().gennmi_runner_push(self._runner, a._dev, values.ctypes.data, values.nbytes))
+        return a
+
     def _next_stream(self):
         self._init_streams += 1
         return self._init_streams
@@ -625,6 +638,9 @@ class GeNNModel:
                 for v in names:
                     if isinstance(n.var_init[v], VarInit):
                         n.vars[v] = self._alloc_device_init(B * N, np.float32, n.var_init[v], pinned=True)
+                        continue
+                    if np.ndim(n.var_init[v]) == 0:
+                        n.vars[v] = self._alloc(B * N, np.float32, fill=np.float32(n.var_init[v]), pinned=True)
                         continue
                     a = self._alloc(B * N, np.float32, pinned=True, device_only=True)
                     init = np.asarray(n.var_init[v], dtype=np.float32)
@@ -669,10 +685,7 @@ class GeNNModel:
                     noise = np.ascontiguousarray(cs.extra_global_params["noise"], dtype=np.float32)
                     if noise.size % N:
                         raise ValueError(f"{cs.name}: noise array is not a multiple of the population size")
-                    a = self._alloc(noise.size, np.float32, device_only=True)
-                    a.view[:] = noise.reshape(-1)
-                    a.push_to_device()
-                    cs.vars["noise"] = a
+                    cs.vars["noise"] = self._alloc_given(noise)
 
         # ---- synapse-group arrays (runtime.cc:330-402)
         for s in self.synapse_populations.values():

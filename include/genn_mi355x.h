@@ -138,6 +138,10 @@ int gennmi_register_device_array(const void *host, void *dev, size_t bytes);
 int gennmi_mirrors_begin_initialisation(void);
 int gennmi_mirror_device_initialised(const void *host);
 int gennmi_mirror_ensure_host(const void *host);
+/* Blocks of device memory that were freed are kept for the next allocation of their size: at most 1/32 of the card's memory in all,
+ * each for at most ten seconds of idleness; the bytes reported free include them.  This gives all of them back to the
+ * system, and the idle pinned memory with them. */
+int gennmi_release_cached_memory(void);
 int gennmi_free_device_memory_bytes(size_t *bytes);
 /* Named ranges for profilers around stepTime / updateSynapses / updateNeurons (BackendBase::genPushProfilerRange /
  * genPopProfilerRange, backendBase.h:345-349; nvtxRangePushA / nvtxRangePop in cuda/backend.cc:741-752): roctxRangePushA /

@@ -1,0 +1,107 @@
+"""Device memory kept between models, and the segment boundaries built with the tables of a new one."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+from genn_amd import _abi, configs
+from genn_amd.genn_model import Array, GeNNModel, init_postsynaptic, init_weight_update, model_from_net
+
+pytestmark = pytest.mark.gpu
+MIB = 1 << 20
+
+
+def _malloc(lib, nbytes):
+    p = C.c_void_p()
+    _abi.check(lib.gennmi_malloc(C.byref(p), nbytes))
+    return p
+
+
+def test_blocks_are_kept_by_size_and_given_back():
+    lib = _abi.load()
+    _abi.check(lib.gennmi_init(0))
+    _abi.check(lib.gennmi_release_cached_memory())
+    a, b = _malloc(lib, 40 * MIB), _malloc(lib, 41 * MIB)
+    assert a.value != b.value
+    for p in (a, b):
+        _abi.check(lib.gennmi_free(p))
+    c = _malloc(lib, 41 * MIB)          # (the smallest kept block it fits)
+    d = _malloc(lib, 38 * MIB)          # (within an eighth of the block's size)
+    e = _malloc(lib, 38 * MIB)          # (none left)
+    assert (c.value, d.value) == (b.value, a.value) and e.value not in (a.value, b.value)
+    for p in (c, d, e):
+        _abi.check(lib.gennmi_free(p))
+    kept, left = C.c_size_t(), C.c_size_t()
+    _abi.check(lib.gennmi_free_device_memory_bytes(C.byref(kept)))
+    _abi.check(lib.gennmi_release_cached_memory())
+    _abi.check(lib.gennmi_free_device_memory_bytes(C.byref(left)))
+    assert abs(kept.value - left.value) <= 64 * MIB
+
+
+def test_kept_blocks_under_threads():
+    """Every thread sees its own bytes: a block in use is never handed out twice."""
+    lib = _abi.load()
+    _abi.check(lib.gennmi_init(0))
+    failures = []
+
+    def work(k):
+        rng = np.random.default_rng(k)
+        for _ in range(8):
+            count = int(rng.integers(600_000, 700_000))
+            a = Array(count, np.float32, fill=float(k))
+            got = a.pull_slice(count - 1000, 1000)
+            if not np.all(got == k):
+                failures.append((k, got))
+            a.free()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
+
+
+def test_models_one_after_another_are_the_same():
+    """A model built from kept blocks (full of the last one's values) runs as the first one did."""
+    net = configs.plastic_stdp(n=5000, n_src=50, steps=60, fan=400, src_fan=100)
+    runs = []
+    for _ in range(3):
+        m = model_from_net(net)
+        m.load(num_recording_timesteps=60)
+        m.run(60)
+        m.pull_recording_buffers_from_device()
+        runs.append([p.vars["recordSpk"].view.copy() for p in m.neuron_populations.values()])
+        m.unload()
+    assert sum(int(a.sum() != 0) for a in runs[0]) > 0
+    for r in runs[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(runs[0], r))
+
+
+@pytest.mark.parametrize("n_trg, tile_floats", [(1, 16), (63, 16), (64, 16), (100, 7), (4097, 1024), (3000, 1000)])
+@pytest.mark.parametrize("row_len", [0, 1, 63, 64, 65, 130])
+def test_tile_path_sums_at_row_and_tile_edges(n_trg, tile_floats, row_len, monkeypatch):
+    """Rows around a wavefront's 64 synapses, targets around tile boundaries (power of two and not): integer weights, exact sums."""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", str(tile_floats))
+    n_src, rng = 70, np.random.default_rng(n_trg * 131 + row_len)
+    rows = [np.sort(rng.integers(0, n_trg, row_len if r else n_trg if n_trg < 200 else 200)) for r in range(n_src)]
+    pre = np.concatenate([np.full(len(r), k) for k, r in enumerate(rows)])
+    post = np.concatenate(rows)
+    m = GeNNModel("float", "edges", dt=1.0)
+    src = m.add_neuron_population("S", n_src, "SpikeSourceArray", {}, {"startSpike": np.arange(n_src), "endSpike": np.arange(n_src) + 1})
+    src.set_extra_global_param("spikeTimes", np.zeros(n_src, np.float32))
+    trg = m.add_neuron_population("T", n_trg, "LIF", dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=1e9, Ioffset=0.0, TauRefrac=5.0),
+                                  {"V": -60.0, "RefracTime": 0.0})
+    s = m.add_synapse_population("ST", "SPARSE", src, trg, init_weight_update("StaticPulse", {}, {"g": 0.0}), init_postsynaptic("DeltaCurr"))
+    s.set_sparse_connections(pre, post)
+    weights = rng.integers(-8, 9, len(pre)).astype(np.float32)
+    s.set_var_coo("g", weights)
+    m.build()
+    m.load()
+    m.step_time()               # every source fires in the first step
+    m.update_synapses()
+    want = np.zeros(n_trg, np.float32)
+    np.add.at(want, post, weights)
+    assert np.array_equal(s.vars["outPost"].pull_from_device(), want)
+    m.unload()
