@@ -116,8 +116,10 @@ void initVarKernel(T *out, unsigned long long count, VarInit v, Stream s)
     for(unsigned long long g = (unsigned long long)blockIdx.x * BLOCK + threadIdx.x; g < groups; g += (unsigned long long)gridDim.x * BLOCK) {
         T value[4];
         if(v.snippet == GENNMI_INIT_GAMMA || v.snippet == GENNMI_INIT_BINOMIAL) {
+            #pragma unroll
             for(int k = 0; k < 4; k++) {
                 const unsigned long long e = g * 4 + k;
+                value[k] = (T)0;
                 if(e < count) {
                     value[k] = (v.snippet == GENNMI_INIT_GAMMA) ? (T)(v.p[1] * gammaDraw(s, e, v.p[0]))
                                                                : (T)binomialDraw(s, e, (uint32_t)v.p64[0], v.p64[1]);
@@ -125,13 +127,10 @@ void initVarKernel(T *out, unsigned long long count, VarInit v, Stream s)
             }
         }
         else {
-            const Words r = s.at(g, 0);
-            float n[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if(v.snippet == GENNMI_INIT_NORMAL || v.snippet == GENNMI_INIT_NORMAL_CLIPPED || v.snippet == GENNMI_INIT_NORMAL_CLIPPED_DELAY) {
-                normals(r, n);
-            }
+            float x[4];
+            valuesAt4(v, s, g * 4, x);
             #pragma unroll
-            for(int k = 0; k < 4; k++) { value[k] = (T)drawValue(v, s, g, k, r, n); }
+            for(int k = 0; k < 4; k++) { value[k] = (T)x[k]; }
         }
         if(g * 4 + 3 < count) {
             Q q;
@@ -139,7 +138,8 @@ void initVarKernel(T *out, unsigned long long count, VarInit v, Stream s)
             *reinterpret_cast<Q*>(out + g * 4) = q;
         }
         else {
-            for(int k = 0; k < 4 && g * 4 + k < count; k++) { out[g * 4 + k] = value[k]; }
+            #pragma unroll
+            for(int k = 0; k < 4; k++) { if(g * 4 + k < count) { out[g * 4 + k] = value[k]; } }
         }
     }
 }
@@ -194,7 +194,8 @@ void fixedNumberPostKernel(uint32_t numPre, uint32_t numPost, uint32_t rowStride
             *reinterpret_cast<uint4*>(rowInd + k) = make_uint4(post[0], post[1], post[2], post[3]);
         }
         else {
-            for(int i = 0; i < 4 && k + i < n; i++) { rowInd[k + i] = post[i]; }
+            #pragma unroll
+            for(int i = 0; i < 4; i++) { if(k + i < n) { rowInd[k + i] = post[i]; } }
         }
     });
     if(lane == 0) { rowLength[row] = n; }

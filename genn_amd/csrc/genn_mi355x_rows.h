@@ -36,6 +36,12 @@ __host__ __device__ inline Words philox4x32(uint32_t c0, uint32_t c1, uint32_t c
     return Words{{c0, c1, c2, c3}};
 }
 
+// One of four values by an index the compiler does not know.  Indexing an array does the same through memory: the compiler puts the
+// array into scratch or, where it can, into 16 KB of LDS, and every access waits for it.
+template<typename T>
+__host__ __device__ inline T pickOf4(T v0, T v1, T v2, T v3, uint32_t k) { return (k & 2u) ? ((k & 1u) ? v3 : v2) : ((k & 1u) ? v1 : v0); }
+__host__ __device__ inline uint32_t wordOf(const Words &r, uint32_t k) { return pickOf4(r.w[0], r.w[1], r.w[2], r.w[3], k); }
+
 // A stream of draws: key = the 64-bit seed, counter = (index low, index high, sub-counter, stream number).
 struct Stream
 {
@@ -92,22 +98,22 @@ __device__ __forceinline__ float drawValue(const VarInit &v, const Stream &s, un
         return v.p[0];
     case GENNMI_INIT_UNIFORM: {
         const float scale = v.p[1] - v.p[0];
-        return v.p[0] + (uniformHalfOpen(r.w[slot]) * scale);
+        return v.p[0] + (uniformHalfOpen(wordOf(r, slot)) * scale);
     }
     case GENNMI_INIT_NORMAL:
-        return v.p[0] + (n[slot] * v.p[1]);
+        return v.p[0] + (pickOf4(n[0], n[1], n[2], n[3], (uint32_t)slot) * v.p[1]);
     case GENNMI_INIT_NORMAL_CLIPPED:
     case GENNMI_INIT_NORMAL_CLIPPED_DELAY: {
-        float value = v.p[0] + (n[slot] * v.p[1]);
+        float value = v.p[0] + (pickOf4(n[0], n[1], n[2], n[3], (uint32_t)slot) * v.p[1]);
         for(uint32_t attempt = 1; value > v.p[3] || value < v.p[2]; attempt++) {
             float retry[4];
             normals(s.at(group, attempt), retry);
-            value = v.p[0] + (retry[slot] * v.p[1]);
+            value = v.p[0] + (pickOf4(retry[0], retry[1], retry[2], retry[3], (uint32_t)slot) * v.p[1]);
         }
         return (v.snippet == GENNMI_INIT_NORMAL_CLIPPED_DELAY) ? rintf(value) : value;
     }
     case GENNMI_INIT_EXPONENTIAL:
-        return v.p[0] * -logf(uniformOpen(r.w[slot]));
+        return v.p[0] * -logf(uniformOpen(wordOf(r, slot)));
     default:
         return 0.0f;
     }
@@ -126,16 +132,33 @@ __device__ __forceinline__ float valueAt(const VarInit &v, const Stream &s, unsi
     return drawValue(v, s, group, (int)(e & 3), r, n);
 }
 
-// elements e0..e0+3 at once (e0 a multiple of four): the four share one generator call
+// elements e0..e0+3 at once (e0 a multiple of four): the four share one generator call — and, where clipped draws are repeated,
+// the call of each attempt (the value of an element is that of drawValue)
 __device__ __forceinline__ void valuesAt4(const VarInit &v, const Stream &s, unsigned long long e0, float out[4])
 {
     if(v.snippet == GENNMI_INIT_CONSTANT) { out[0] = out[1] = out[2] = out[3] = v.p[0]; return; }
     const unsigned long long group = e0 >> 2;
     const Words r = s.at(group, 0);
-    float n[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if(v.snippet == GENNMI_INIT_NORMAL || v.snippet == GENNMI_INIT_NORMAL_CLIPPED || v.snippet == GENNMI_INIT_NORMAL_CLIPPED_DELAY) { normals(r, n); }
+    if(v.snippet == GENNMI_INIT_UNIFORM || v.snippet == GENNMI_INIT_EXPONENTIAL) {
+        #pragma unroll
+        for(int i = 0; i < 4; i++) { out[i] = drawValue(v, s, group, i, r, nullptr); }
+        return;
+    }
+    float n[4];
+    normals(r, n);
     #pragma unroll
-    for(int i = 0; i < 4; i++) { out[i] = drawValue(v, s, group, i, r, n); }
+    for(int i = 0; i < 4; i++) { out[i] = v.p[0] + (n[i] * v.p[1]); }
+    if(v.snippet == GENNMI_INIT_NORMAL) { return; }
+    auto outside = [&](float x) { return x > v.p[3] || x < v.p[2]; };
+    for(uint32_t attempt = 1; outside(out[0]) || outside(out[1]) || outside(out[2]) || outside(out[3]); attempt++) {
+        normals(s.at(group, attempt), n);
+        #pragma unroll
+        for(int i = 0; i < 4; i++) { if(outside(out[i])) { out[i] = v.p[0] + (n[i] * v.p[1]); } }
+    }
+    if(v.snippet == GENNMI_INIT_NORMAL_CLIPPED_DELAY) {
+        #pragma unroll
+        for(int i = 0; i < 4; i++) { out[i] = rintf(out[i]); }
+    }
 }
 
 // FixedProbability / FixedProbabilityNoAutapse (include/genn/genn/initSparseConnectivitySnippet.h:170-187, 208-230), one row
@@ -156,7 +179,7 @@ __device__ __forceinline__ uint32_t fixedProbabilityRow(uint32_t row, uint32_t n
         Words r;
         while(true) {
             if((draw & 3u) == 0) { r = s.at(((unsigned long long)row << 32) | (draw >> 2), lane); }
-            const float skip = logf(uniformOpen(r.w[draw & 3u])) * probLogRecip;
+            const float skip = logf(uniformOpen(wordOf(r, draw & 3u))) * probLogRecip;
             draw++;
             if(skip >= (float)(end - begin)) { break; }
             j += 1 + (int)skip;

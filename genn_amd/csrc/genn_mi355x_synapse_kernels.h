@@ -322,6 +322,9 @@ void presynapticDenseKernel(const DenseGroupDev * __restrict__ blocks, unsigned 
 // neuron with exactly the code and draws the initialisation kernels use (genn_mi355x_rows.h), so a procedural projection
 // behaves synapse for synapse like the stored matrix the same seed would have produced — without reading a byte of
 // connectivity: the only memory traffic of an event is its atomic.
+// What bounds it is the chain of arithmetic that makes a row (generator, logarithms, scan, division).  Nothing in it may index a
+// private array by a run-time number: the compiler then keeps such arrays in LDS (16 KB of a work-group's, and an access on
+// the chain each time); without that a step of 41 spikes x 1000 targets takes 9.4 us instead of 20.3.
 // ------------------------------------------------------------------------------------------------
 struct ProcGroupDev
 {
@@ -355,10 +358,18 @@ void presynapticProceduralKernel(const ProcGroupDev * __restrict__ blocks, unsig
         // a group of four synapses shares one generator call for its weights when the row starts on a multiple of four
         const bool aligned = (rowStride & 3u) == 0;
         auto deliver = [&](unsigned long long firstElement, uint32_t k, const uint32_t post[4]) {
-            float w[4];
-            if(aligned) { valuesAt4(G.weightInit, G.weight, firstElement + k, w); }
-            else { for(int i = 0; i < 4; i++) { w[i] = valueAt(G.weightInit, G.weight, firstElement + k + i); } }
-            for(int i = 0; i < 4 && k + i < n; i++) { atomicAddF32(&outPost[post[i]], w[i]); }
+            if(aligned) {
+                float w[4];
+                valuesAt4(G.weightInit, G.weight, firstElement + k, w);
+                #pragma unroll
+                for(int i = 0; i < 4; i++) { if(k + i < n) { atomicAddF32(&outPost[post[i]], w[i]); } }
+            }
+            else {
+                #pragma unroll 1
+                for(uint32_t i = 0; i < 4 && k + i < n; i++) {
+                    atomicAddF32(&outPost[pickOf4(post[0], post[1], post[2], post[3], i)], valueAt(G.weightInit, G.weight, firstElement + k + i));
+                }
+            }
         };
         if(n / (4 * WAVE) + 1 > 1 && n / (4 * WAVE) + 1 <= MAX_ROUNDS) {
             // long rows: one spike per block, the block's waves share the row's rounds of 256 draws
@@ -772,17 +783,23 @@ void tileOffsetKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLe
     auto tileOf = [&](uint32_t p) { return (shift < 32u) ? (p >> shift) : (p / tileSize); };
     // boundary t is the position of the first synapse whose target's tile is >= t
     uint32_t before = 0, next = 0;      // target of the last synapse of the pass before; first boundary not yet written
-    for(uint32_t j0 = 0; j0 < len; j0 += WAVE) {
-        const uint32_t j = j0 + lane;
-        const uint32_t p = r[min(j, len - 1)];
-        const uint32_t left = (uint32_t)__shfl_up((int)p, 1, WAVE), prev = (lane == 0) ? before : left;
-        if(j < len) {
-            if(p < prev) { atomicOr(unsorted, 1u); }
-            const uint32_t first = (j == 0) ? 0u : tileOf(prev) + 1u;
-            for(uint32_t t = first; t <= min(tileOf(p), numTiles); t++) { o[t] = (uint16_t)j; }
+    constexpr uint32_t AHEAD = 8;       // passes whose entries are asked for together
+    for(uint32_t j0 = 0; j0 < len; j0 += AHEAD * WAVE) {
+        uint32_t entry[AHEAD];
+        #pragma unroll
+        for(uint32_t u = 0; u < AHEAD; u++) { entry[u] = r[min(j0 + u * WAVE + lane, len - 1)]; }
+        #pragma unroll
+        for(uint32_t u = 0; u < AHEAD; u++) {
+            const uint32_t j = j0 + u * WAVE + lane, p = entry[u];
+            const uint32_t left = (uint32_t)__shfl_up((int)p, 1, WAVE), prev = (lane == 0) ? before : left;
+            if(j < len) {
+                if(p < prev) { atomicOr(unsorted, 1u); }
+                const uint32_t first = (j == 0) ? 0u : tileOf(prev) + 1u;
+                for(uint32_t t = first; t <= min(tileOf(p), numTiles); t++) { o[t] = (uint16_t)j; }
+            }
+            before = (uint32_t)__shfl((int)p, WAVE - 1, WAVE);
+            next = tileOf(before) + 1u;
         }
-        before = (uint32_t)__shfl((int)p, WAVE - 1, WAVE);
-        next = tileOf(before) + 1u;
     }
     for(uint32_t t = next + lane; t <= numTiles; t += WAVE) { o[t] = (uint16_t)len; }
 }
