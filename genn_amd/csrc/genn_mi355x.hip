@@ -48,6 +48,7 @@
 #include "genn_mi355x_resident_kernels.h"
 #include "genn_mi355x_ordered_kernels.h"
 #include "genn_mi355x_conv_step_kernels.h"
+#include "genn_mi355x_ahead_kernels.h"
 #include "genn_mi355x_transfer.h"
 #include "genn_mi355x_pool.h"
 
@@ -79,6 +80,11 @@ struct gennmi_runner
     bool convStep = false;
     NeuronGroupDev *dConvTarget = nullptr, *dConvRest = nullptr; uint32_t convRestBlocks = 0; size_t convStepBytes = 0;
     unsigned long long *dConvAgg = nullptr, *dConvRestAgg = nullptr;
+    // a feed-forward layer, many steps per launch (genn_mi355x_ahead_kernels.h): its source population, its target population and the layer
+    bool ahead = false;
+    gennmi_presynaptic_update_group_t aheadLayer{}; AheadConv aheadConv{}; size_t aheadConvBytes = 0; uint32_t aheadCU = 1, aheadMinSteps = 0;
+    NeuronGroupDev *dAhead = nullptr; uint32_t aheadSource = 0, aheadTarget = 0;     // descriptors of source and target; their indices in `neuron`
+    uint8_t *aheadSpace = nullptr; size_t aheadSpaceBytes = 0;                          // workspace, made by the first run that needs it
     bool bitmapsStale = false;          // a spike queue was written by the caller: the bitmaps kept beside the queues are rebuilt before the next step
     std::vector<void*> owned;           // engine-private device allocations (shadow queues, zero-delay lists)
     // resident plan (many steps per launch)
@@ -539,6 +545,7 @@ int gennmi_runner_destroy(gennmi_runner *r)
     for(void *q : r->owned) { poolFree(q); }
     for(void *q : r->zeroOwned) { poolFree(q); }
     for(void *q : r->orderedOwned) { poolFree(q); }
+    poolFree(r->aheadSpace);
     poolFree(r->dOrderedSources); poolFree(r->dOrderedBitmaps);
     poolFree(r->dTile); poolFree(r->dConvTile);
     poolFree(r->dNeuron); poolFree(r->dPre); poolFree(r->dPost); poolFree(r->dDense); poolFree(r->dProc); poolFree(r->dAgg); if(r->hError) { hipError_t e; pinnedFree(r->hError, &e); } poolFree(r->dEvents);
@@ -1186,6 +1193,133 @@ static int refreshTables(gennmi_runner *r)
     return GENNMI_OK;
 }
 
+// Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
+// plain population it feeds, so that no spike ever comes back.
+constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input over the steps of a launch
+constexpr size_t AHEAD_MAX_LDS = 64 * 1024;
+// Runs (and remainders of runs) shorter than this are stepped one by one.  A launch costs as much as 32 steps whatever it is given, so what
+// decides is the product it computes for them.  Steps: us at once / one by one.  Up to 5 GFLOP: DENSE 8192 x 8192 (4.3) 2: 31 / 26,
+// 4: 36 / 46, 8: 47 / 86; 2048 x 2048, batch 16 (4.3) 8: 58 / 144; Conv2D 16x16x1 -> 4 4: 26 / 69.  More: DENSE 8192 x 8192, batch 4
+// (17) 8: 150 / 148, 16: 176 / 291; batch 16 (69) 8: 492 / 344, 16: 580 / 684; Conv2D 64x64x16 -> 32 3x3, batch 16 (19) 8: 246 / 253,
+// 16: 261 / 499.  (5 % and 2.5 % activity; at a fifth and a twenty-fifth of that, at once gains more on one by one.)
+constexpr uint32_t AHEAD_MIN_STEPS_LIGHT = 4, AHEAD_MIN_STEPS_HEAVY = 16;
+constexpr double AHEAD_LIGHT_FLOP = 5e9;
+static int setupAhead(gennmi_runner *r, uint32_t numCU)
+{
+    const char *env = getenv("GENNMI_AHEAD");
+    if((env && atoi(env) == 0) || r->ordered || !r->plainGroups || r->neuron.size() != 2 || !r->proc.empty() || !r->post.empty() || r->dense.size() + r->pre.size() != 1) { return GENNMI_OK; }
+    const gennmi_presynaptic_update_group_t &p = r->dense.empty() ? r->pre[0].g : r->dense[0].g;
+    const bool conv = (p.matrix == GENNMI_MATRIX_TOEPLITZ_CONV2D);
+    if((!conv && p.matrix != GENNMI_MATRIX_DENSE) || p.wum != GENNMI_WUM_STATIC_PULSE || !p.g || p.maxDenDelay || p.numSrcDelaySlots > 1 || p.axonalDelaySteps) { return GENNMI_OK; }
+    const uint32_t s = (r->neuron[0].g.spk == p.srcSpk) ? 0 : 1, t = 1 - s;
+    NeuronGroupDev &src = r->neuron[s];
+    const gennmi_neuron_update_group_t &g = r->neuron[t].g;
+    if(src.g.spk != p.srcSpk || src.g.spkCnt != p.srcSpkCnt || src.g.numNeurons != p.numSrcNeurons || src.g.model != GENNMI_NEURON_SPIKE_SOURCE_ARRAY || src.g.numPSM || src.g.numCS || src.shadowSpk) { return GENNMI_OK; }
+    if((g.model != GENNMI_NEURON_LIF && g.model != GENNMI_NEURON_IZHIKEVICH) || g.numNeurons != p.numTrgNeurons || g.numPSM != 1 || g.psm[0].outPost != p.outPost || g.psm[0].maxDenDelay
+       || (g.psm[0].kind != GENNMI_PSM_EXPCURR && g.psm[0].kind != GENNMI_PSM_DELTACURR) || g.numCS > 1 || (g.numCS == 1 && g.cs[0].kind != GENNMI_CS_DC)
+       || r->neuron[t].spikeBitmap || r->neuron[t].shadowSpk || !(r->dt > 0.0f) || r->batch > 65535) { return GENNMI_OK; }
+    if(conv) {
+        const int32_t *c = p.conv;
+        AheadConv &C = r->aheadConv;
+        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 0u, 1u};
+        C.rowPitch = (uint32_t)(c[6] - 1 + c[1]) * (uint32_t)c[4] + 1;      // (an odd number of taps is read as pairs: one word beyond)
+        C.pairsPerRow = ((uint32_t)(c[1] * c[4]) + 1) / 2;
+        // as many output rows per work-group as leave four work-groups to a compute unit
+        const uint64_t rowsInAll = (uint64_t)c[5] * r->batch * (((uint32_t)c[7] + 31) / 32);
+        C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (4 * numCU)));
+        for(;; C.rowsPerBlock--) {
+            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)c[0] * 2 * C.pairsPerRow * 32) * sizeof(uint32_t);
+            if(r->aheadConvBytes <= AHEAD_MAX_LDS || C.rowsPerBlock == 1) { break; }
+        }
+        if(r->aheadConvBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
+    }
+    else if((size_t)r->batch * AHEAD_WORD * p.numTrgNeurons * sizeof(float) > AHEAD_MAX_SPACE || (uint64_t)r->batch * (AHEAD_MAX_STEPS / AHEAD_WORD) > 65535) { return GENNMI_OK; }
+    if(!src.spikeBitmap) {
+        const size_t bytes = (size_t)r->batch * ((src.g.numNeurons + 31) / 32) * sizeof(uint32_t);
+        HIP_TRY(poolMalloc((void**)&src.spikeBitmap, bytes));
+        r->owned.push_back(src.spikeBitmap);
+        HIP_TRY(hipMemset(src.spikeBitmap, 0, bytes));
+        r->bitmapsStale = true;          // the queue may already hold spikes
+    }
+    HIP_TRY(poolMalloc((void**)&r->dAhead, 2 * sizeof(NeuronGroupDev)));
+    r->owned.push_back(r->dAhead);
+    const double flop = conv ? 2.0 * AHEAD_WORD * r->batch * p.conv[5] * p.conv[6] * p.conv[0] * (2.0 * r->aheadConv.pairsPerRow) * (((uint32_t)p.conv[7] + 31) / 32 * 32)
+                             : 2.0 * AHEAD_WORD * r->batch * p.numSrcNeurons * p.numTrgNeurons;
+    r->aheadMinSteps = (flop <= AHEAD_LIGHT_FLOP) ? AHEAD_MIN_STEPS_LIGHT : AHEAD_MIN_STEPS_HEAVY;
+    r->aheadLayer = p; r->aheadSource = s; r->aheadTarget = t; r->aheadCU = numCU;
+    r->ahead = true;
+    return GENNMI_OK;
+}
+
+// the next numSteps (up to AHEAD_MAX_STEPS) steps; `done` receives how many it took
+static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned long long numSteps, unsigned long long numRecordingTimesteps, uint32_t *done)
+{
+    const gennmi_presynaptic_update_group_t &p = r->aheadLayer;
+    const bool conv = r->aheadConv.isConv != 0;
+    const uint32_t numSrc = p.numSrcNeurons, numTrg = p.numTrgNeurons, B = r->batch, targetWords = (numTrg + 31) / 32;
+    uint32_t steps = (uint32_t)std::min<unsigned long long>(numSteps, AHEAD_MAX_STEPS), blocks = 0, slices = 1, mt = 1, mGroups = 1, perSlice = numSrc;
+    size_t inputBytes = 0;
+    for(;; steps = (blocks - 1) * AHEAD_WORD) {
+        blocks = (steps + AHEAD_WORD - 1) / AHEAD_WORD;
+        if(conv) { inputBytes = (size_t)B * numTrg * sizeof(uint32_t); break; }
+        // up to four words of rows per work-group; the source is cut into slices until there are two work-groups per compute unit,
+        // none smaller than a chunk for every wavefront
+        const uint32_t tiles = blocks * B, columns = (numTrg + 31) / 32;
+        mt = (tiles >= 3) ? 4u : tiles;
+        mGroups = (tiles + mt - 1) / mt;
+        slices = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((numSrc + AHEAD_DENSE_THREADS - 1) / AHEAD_DENSE_THREADS, 2ull * r->aheadCU / ((uint64_t)columns * mGroups)));
+        perSlice = ((numSrc + slices - 1) / slices + WAVE - 1) / WAVE * WAVE;
+        inputBytes = (size_t)slices * tiles * AHEAD_WORD * numTrg * sizeof(float);
+        if(inputBytes <= AHEAD_MAX_SPACE || blocks == 1) { break; }
+    }
+    auto aligned = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t wordBytes = aligned((size_t)blocks * B * numSrc * sizeof(uint32_t)), bitBytes = aligned((size_t)B * targetWords * sizeof(uint32_t));
+    const size_t need = wordBytes + bitBytes + inputBytes;
+    if(need > r->aheadSpaceBytes) {
+        HIP_TRY(hipStreamSynchronize(r->stream));
+        HIP_TRY(poolFree(r->aheadSpace));
+        r->aheadSpace = nullptr; r->aheadSpaceBytes = 0;
+        HIP_TRY(poolMalloc((void**)&r->aheadSpace, need));
+        r->aheadSpaceBytes = need;
+    }
+    uint32_t *words = reinterpret_cast<uint32_t*>(r->aheadSpace), *targetBits = reinterpret_cast<uint32_t*>(r->aheadSpace + wordBytes);
+    uint8_t *input = r->aheadSpace + wordBytes + bitBytes;
+    const NeuronGroupDev *target = r->dAhead + 1, &src = r->neuron[r->aheadSource];
+    const AheadArgs a{timestep, r->epoch, steps, B, (uint32_t)std::max<unsigned long long>(1, std::min<unsigned long long>(numRecordingTimesteps, 0xFFFFFFFFull)), r->dt};
+    // (the kernels of the target's neuron model and postsynaptic model)
+    const gennmi_neuron_update_group_t &g = r->neuron[r->aheadTarget].g;
+    const bool lif = (g.model == GENNMI_NEURON_LIF), exponential = (g.psm[0].kind == GENNMI_PSM_EXPCURR);
+    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
+    const auto convKernel = lif ? (exponential ? aheadConvKernel<LIF, EXP> : aheadConvKernel<LIF, DELTA>) : (exponential ? aheadConvKernel<IZH, EXP> : aheadConvKernel<IZH, DELTA>);
+    const auto neuronKernel = lif ? (exponential ? aheadNeuronKernel<LIF, EXP> : aheadNeuronKernel<LIF, DELTA>) : (exponential ? aheadNeuronKernel<IZH, EXP> : aheadNeuronKernel<IZH, DELTA>);
+    aheadSourceKernel<<<dim3((numSrc + BLOCK - 1) / BLOCK, B), dim3(BLOCK), 0, r->stream>>>(r->dAhead, a, r->aheadConv, numTrg, words, r->dEvents);
+    if(conv) {
+        const AheadConv &C = r->aheadConv;
+        uint32_t *spikes = reinterpret_cast<uint32_t*>(input);
+        for(uint32_t k = 0; k < blocks; k++) {
+            convKernel<<<dim3(((uint32_t)C.oh + C.rowsPerBlock - 1) / C.rowsPerBlock, B, ((uint32_t)C.oc + 31) / 32), dim3(BLOCK), r->aheadConvBytes, r->stream>>>(
+                target, a, C, k, words, p.g, spikes);
+            if(g.recordSpk || k + 1 == blocks) {
+                aheadTransposeKernel<<<dim3((numTrg + 1023) / 1024, B), dim3(BLOCK), 0, r->stream>>>(target, a, k, spikes, targetBits);
+            }
+        }
+    }
+    else {
+        float *partial = reinterpret_cast<float*>(input);
+        const uint32_t tiles = blocks * B;
+        const dim3 grid((numTrg + 31) / 32, mGroups * slices);
+        if(mt == 1) { aheadDenseKernel<1><<<grid, dim3(AHEAD_DENSE_THREADS), 0, r->stream>>>(words, tiles, mGroups, p.g, numSrc, numTrg, perSlice, partial); }
+        else if(mt == 2) { aheadDenseKernel<2><<<grid, dim3(AHEAD_DENSE_THREADS), 0, r->stream>>>(words, tiles, mGroups, p.g, numSrc, numTrg, perSlice, partial); }
+        else { aheadDenseKernel<4><<<grid, dim3(AHEAD_DENSE_THREADS), 0, r->stream>>>(words, tiles, mGroups, p.g, numSrc, numTrg, perSlice, partial); }
+        neuronKernel<<<dim3((numTrg + WAVE - 1) / WAVE, B), dim3(WAVE), 0, r->stream>>>(target, a, partial, slices, tiles, targetBits);
+    }
+    aheadQueueKernel<<<dim3(2, B), dim3(AHEAD_QUEUE_THREADS), 0, r->stream>>>(r->dAhead, src.spikeBitmap + ((r->epoch + steps) & 1) * src.bitmapStride, targetBits);
+    HIP_TRY(hipGetLastError());
+    r->epoch += steps;
+    *done = steps;
+    return GENNMI_OK;
+}
+
 int gennmi_runner_set_ordered(gennmi_runner *r, int enabled)
 {
     if(!r) { return fail(GENNMI_EINVAL, "runner_set_ordered: null runner"); }
@@ -1715,6 +1849,11 @@ int gennmi_runner_finalise(gennmi_runner *r)
             r->convStep = true;
         }
     }
+    { const int rc = setupAhead(r, numCU); if(rc) { return rc; } }
+    if(r->ahead) {
+        const NeuronGroupDev both[2] = {r->neuron[r->aheadSource], r->neuron[r->aheadTarget]};
+        HIP_TRY(upload(r->dAhead, both, sizeof(both)));
+    }
     HIP_TRY(uploadPerBlock(r->neuron, r->neuronBlocks, &r->dNeuron));
     HIP_TRY(uploadPerBlock(r->pre, r->preBlocks, &r->dPre));
     HIP_TRY(uploadPerBlock(r->post, r->postBlocks, &r->dPost));
@@ -2028,11 +2167,18 @@ int gennmi_run_steps(gennmi_runner *r, unsigned long long timestep, unsigned lon
     { const int rc = refreshSpikeSources(r); if(rc) { return rc; } }
     { const int rc = refreshTables(r); if(rc) { return rc; } }
     if(r->resident && !r->timing && numSteps >= 4) { return launchResident(r, timestep, numSteps, numRecordingTimesteps); }
-    // Every step is launched as gennmi_step_time() launches it: time, epoch and recording row are kernel arguments.  (Measured
+    unsigned long long done = 0;
+    while(r->ahead && !r->timing && numSteps - done >= r->aheadMinSteps) {
+        uint32_t taken = 0;
+        const int rc = launchAhead(r, timestep + done, numSteps - done, numRecordingTimesteps, &taken);
+        if(rc) { return rc; }
+        done += taken;
+    }
+    // Every (other) step is launched as gennmi_step_time() launches it: time, epoch and recording row are kernel arguments.  (Measured
     // against replaying captured graphs of 100 steps whose kernels read them from a device-resident state: a launch costs the
     // host 2.5 us, less than any step's kernels take, while the graph cost every kernel a dependent load of that state before its
     // first useful access, runs a copy and a wait for it, and steps beyond a multiple of 100 a launch that advanced it.)
-    for(unsigned long long done = 0; done < numSteps; done++) {
+    for(; done < numSteps; done++) {
         const unsigned long long ts = timestep + done;
         const int rc = stepNow(r, (float)ts * r->dt, numRecordingTimesteps ? (uint32_t)(ts % numRecordingTimesteps) : 0u);
         if(rc) { return rc; }
@@ -2188,7 +2334,7 @@ int gennmi_runner_get_info(gennmi_runner *r, uint32_t info[4])
     if(!r || !info) { return fail(GENNMI_EINVAL, "runner_get_info: null argument"); }
     if(!r->finalised) { return fail(GENNMI_ESTATE, "runner_get_info: runner not finalised"); }
     info[0] = (r->fusedStep ? 1u : 0u) | (r->resident ? 2u : 0u) | (r->neuronsPerLane > 1 ? 4u : 0u) | (r->ordered ? 8u : 0u)
-              | (r->combineSynapses ? 16u : 0u) | ((r->combineSynapses && r->combinePost) ? 32u : 0u) | (r->convMfmaBlocks ? 64u : 0u) | (r->convStep ? 128u : 0u); info[1] = r->neuronBlocks; info[2] = r->preBlocks; info[3] = r->postBlocks;
+              | (r->combineSynapses ? 16u : 0u) | ((r->combineSynapses && r->combinePost) ? 32u : 0u) | (r->convMfmaBlocks ? 64u : 0u) | (r->convStep ? 128u : 0u) | (r->ahead ? 256u : 0u); info[1] = r->neuronBlocks; info[2] = r->preBlocks; info[3] = r->postBlocks;
     return GENNMI_OK;
 }
 

@@ -1,0 +1,531 @@
+// Many timesteps of a feed-forward layer per launch (included by genn_mi355x.hip after the synapse and neuron kernels).
+//
+// A spike source array's spikes depend on nothing but its spike times, and a layer fed by one source alone depends on nothing but
+// those spikes: no step of such a network has to wait for the one before it anywhere else than inside a neuron.  The
+// reference launches updatePresynapticKernel and updateNeuronsKernel for every step all the same (presynapticUpdateStrategySIMT.cc:
+// 57-389, 750-934; backendSIMT.cc:405-662), and so do the step kernels here: each step then pays its launches, the ordered
+// spike queue's look-back and a trip of the layer's state through memory.  Here run() takes up to 128 steps at once:
+//   1. aheadSourceKernel: a lane walks one source neuron's spikes of all these steps.  Its input to the layer is one 32-bit word per
+//      32 steps (bit j: the layer receives a spike from it in step j).
+//   2. the layer's input of 32 steps is a matrix product whose left operand is those bits: rows are timesteps, the inner
+//      dimension the source neurons (DENSE) or an output pixel's taps (Conv2D), columns the target neurons.  A bit becomes the
+//      operand of v_mfma_f32_32x32x2_f32 by a shift, a mask and a conversion; 0 / 1 times an fp32 weight is exact and sums are fp32.
+//   3. the neurons: a lane takes one neuron through the steps with its state in registers.
+//   4. aheadQueueKernel: the spike queues as the last step leaves them, in ascending neuron index.
+// What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
+//
+// Measured with the kernels' launches, copies and waits (run() and its copies; before -> after): DENSE 8192 -> 8192 at 5 % activity,
+// 100 steps; Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: see the kernels.
+#pragma once
+
+namespace
+{
+constexpr uint32_t AHEAD_MAX_STEPS = 128, AHEAD_WORD = 32;      // steps per pass over the source; steps per word (rows of a product)
+constexpr uint32_t AHEAD_DENSE_THREADS = 512, AHEAD_DENSE_WAVES = AHEAD_DENSE_THREADS / WAVE, AHEAD_TILE_COPIES = 4;
+
+struct AheadArgs
+{
+    unsigned long long timestep, epoch;     // of the first step
+    uint32_t steps, batch;
+    uint32_t recordingRows;                 // rows of the recording buffers (1: every step writes row 0)
+    float dt;
+};
+struct AheadConv
+{
+    int32_t kh, kw, ih, iw, ic, oh, ow, oc, PH, PW;
+    uint32_t rowsPerBlock, rowPitch, pairsPerRow;       // patch row in words; (tap, channel) pairs of one kernel row
+    uint32_t isConv;
+};
+
+__device__ __forceinline__ size_t aheadRecordingRow(const AheadArgs &A, uint32_t step) { return (size_t)((A.timestep + step) % A.recordingRows); }
+
+// time of a step as the step-by-step path computes it, (float)timestep * dt (a conversion from 64 bits is a dozen instructions; one
+// from 32 rounds to the same number)
+__device__ __forceinline__ float aheadTime(const AheadArgs &A, uint32_t step)
+{
+    const unsigned long long ts = A.timestep + step;
+    return ((ts >> 32) ? (float)ts : (float)(uint32_t)ts) * A.dt;
+}
+
+// ---- 1. the source.  Bound by the chain of spike-time loads of a lane (one per spike).
+__global__ __launch_bounds__(BLOCK)
+void aheadSourceKernel(const NeuronGroupDev * __restrict__ source, AheadArgs A, AheadConv C, uint32_t numTrg, uint32_t *words,
+                       unsigned long long *eventCounter)
+{
+    const gennmi_neuron_update_group_t &g = source->g;
+    const uint32_t n = g.numNeurons, batch = blockIdx.y, i = blockIdx.x * BLOCK + threadIdx.x, lane = threadIdx.x & (WAVE - 1);
+    const size_t bi = (size_t)batch * n + i;
+    const uint32_t bitmapWords = (n + 31) / 32;
+    uint32_t *recordSpk = g.recordSpk;
+    unsigned long long emitted[2] = {0, 0};        // bit k: a spike in the update of step k
+    uint32_t queued = 0;                            // ... and in the update before the first
+    if(i < n) {
+        queued = (asGlobal(source->spikeBitmap)[(A.epoch & 1) * source->bitmapStride + (size_t)batch * bitmapWords + (i >> 5)] >> (i & 31)) & 1u;
+        uint32_t start = asGlobal(g.startSpike)[bi];
+        const uint32_t end = asGlobal(g.endSpike)[bi], startBefore = start;
+        float next = asGlobal(source->nextSpikeTime)[bi];
+        // the first step from `from` on whose time has reached the next spike (times ascend; a NaN is never reached)
+        for(uint32_t from = 0; from < A.steps; ) {
+            uint32_t lo = from, hi = A.steps;
+            while(lo < hi) {
+                const uint32_t mid = (lo + hi) / 2;
+                if(aheadTime(A, mid) >= next) { hi = mid; } else { lo = mid + 1; }
+            }
+            if(lo >= A.steps) { break; }
+            if(lo < 64) { emitted[0] |= 1ull << lo; } else { emitted[1] |= 1ull << (lo - 64); }
+            start++;
+            next = (start != end) ? asGlobal(g.spikeTimes)[start] : INFINITY;
+            from = lo + 1;
+        }
+        if(start != startBefore) { g.startSpike[bi] = start; source->nextSpikeTime[bi] = next; }
+    }
+    // the layer's input in step j is what was emitted in the update of step j - 1
+    uint32_t received = 0, carry = queued;
+    size_t recordingRow = aheadRecordingRow(A, 0);
+    #pragma unroll
+    for(uint32_t sb = 0; sb < AHEAD_MAX_STEPS / AHEAD_WORD; sb++) {
+        if(sb * AHEAD_WORD < A.steps) {
+            const uint32_t e = (uint32_t)(emitted[sb / 2] >> (32 * (sb & 1)));
+            const uint32_t valid = min(A.steps - sb * AHEAD_WORD, AHEAD_WORD);
+            const uint32_t in = ((e << 1) | carry) & (valid == 32 ? 0xFFFFFFFFu : (1u << valid) - 1u);
+            carry = e >> 31;
+            received += __popc(in);
+            if(i < n) { words[((size_t)sb * A.batch + batch) * n + i] = in; }
+            // recording rows and the last update's spikes: the wavefront's votes
+            if(recordSpk || (sb + 1) * AHEAD_WORD >= A.steps) {
+                for(uint32_t j = recordSpk ? 0 : valid - 1; j < valid; j++) {
+                    const uint32_t step = sb * AHEAD_WORD + j;
+                    const bool last = (step + 1 == A.steps);
+                    const unsigned long long ballot = __ballot((e >> j) & 1u);
+                    if((lane & 31) == 0 && i < n) {
+                        const uint32_t bits = (uint32_t)(ballot >> (lane & 32));
+                        if(recordSpk) { recordSpk[(recordingRow * A.batch + batch) * bitmapWords + (i >> 5)] = bits; }
+                        // (behind this wavefront's read of the same words; nobody else reads or writes them)
+                        if(last) { source->spikeBitmap[((A.epoch + A.steps) & 1) * source->bitmapStride + (size_t)batch * bitmapWords + (i >> 5)] = bits; }
+                    }
+                    recordingRow = (recordingRow + 1 == A.recordingRows) ? 0 : recordingRow + 1;
+                }
+            }
+        }
+    }
+    // synaptic events: a dense row has one synapse per target, a pixel of a convolution as many taps as stay inside the output
+    unsigned long long events = 0;
+    if(received) {
+        if(C.isConv) {
+            const int pixel = (int)(i / (uint32_t)C.ic), row = pixel / C.iw, col = pixel % C.iw;
+            const int firstRow = row - (C.kh - 1 - C.PH), firstCol = col - (C.kw - 1 - C.PW);
+            const int rowTaps = min(firstRow + C.kh, C.oh) - max(firstRow, 0), colTaps = min(firstCol + C.kw, C.ow) - max(firstCol, 0);
+            events = (unsigned long long)received * (uint32_t)(max(rowTaps, 0) * max(colTaps, 0)) * (uint32_t)C.oc;
+        }
+        else { events = (unsigned long long)received * numTrg; }
+    }
+    for(int off = WAVE / 2; off > 0; off >>= 1) { events += __shfl_down(events, off, WAVE); }
+    if(lane == 0 && events) { addEvents(eventCounter, events); }
+}
+
+__device__ __forceinline__ float aheadBit(uint32_t word, uint32_t row) { return (float)((word >> row) & 1u); }
+__device__ __forceinline__ bool aheadFinite(float w) { return (__float_as_uint(w) & 0x7F800000u) != 0x7F800000u; }
+// the accumulator's element v of a lane in the given half is timestep ...
+__device__ __forceinline__ uint32_t aheadRow(uint32_t v, uint32_t half) { return 8 * (v / 4) + 4 * half + (v % 4); }
+
+// ---- 2a. DENSE.  A work-group owns 32 target neurons (columns), up to MT words of (32 steps, batch) as rows and a slice of the
+// source; its wavefronts deal the slice's chunks of 64 source neurons among themselves and add their tiles up in LDS in a fixed order.
+// Source neurons that are silent in all of the group's steps are dropped first (a ballot packs the others), so what is
+// read and multiplied follows the activity: at 5 % and 128 steps all rows remain, at 0.1 % one in eight.  Bound by the fp32 matrix
+// rate for long runs (8192 x 8192 x 128 rows: 17.2 GFLOP) and by reading the weights for short ones.  A weight that is not finite
+// would reach the steps without its spike as 0 * inf: the loop multiplies 0 in its place and such weights are added, step
+// by step, in a pass of their own.
+template<int MT>
+__global__ __launch_bounds__(AHEAD_DENSE_THREADS)
+void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint32_t mGroups, const float * __restrict__ weights, uint32_t numSrc, uint32_t numTrg,
+                      uint32_t sourcesPerSlice, float * __restrict__ partial)
+{
+    constexpr uint32_t LIST_WORDS = WAVE * (MT + 1), TILE = MT * 32 * 32;
+    __shared__ uint32_t lds[(AHEAD_DENSE_WAVES * LIST_WORDS > AHEAD_TILE_COPIES * TILE) ? AHEAD_DENSE_WAVES * LIST_WORDS : AHEAD_TILE_COPIES * TILE];
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
+    const uint32_t mGroup = blockIdx.y % mGroups, slice = blockIdx.y / mGroups;
+    const uint32_t firstTile = mGroup * MT;
+    const uint32_t column = blockIdx.x * 32 + col, readColumn = min(column, numTrg - 1);
+    const uint32_t sliceBegin = slice * sourcesPerSlice, sliceEnd = min(numSrc, sliceBegin + sourcesPerSlice);
+    GLOBAL_AS const uint32_t *in = asGlobal(words);
+    GLOBAL_AS const float *w = asGlobal(weights) + readColumn;
+    uint32_t *list = lds + wave * LIST_WORDS;           // [64] source neurons, then [MT][64] their words
+    f32x16 acc[MT];
+    #pragma unroll
+    for(int q = 0; q < MT; q++) { acc[q] = f32x16{}; }
+    // the active ones of 64 source neurons, packed; returns how many (an odd number is followed by an entry without spikes)
+    auto pack = [&](uint32_t base) -> uint32_t {
+        const uint32_t i = base + lane;
+        uint32_t mine[MT], any = 0;
+        #pragma unroll
+        for(int q = 0; q < MT; q++) {
+            mine[q] = (i < sliceEnd && firstTile + q < mTiles) ? in[(size_t)(firstTile + q) * numSrc + i] : 0u;
+            any |= mine[q];
+        }
+        const unsigned long long active = __ballot(any != 0);
+        const uint32_t count = __popcll(active), at = __popcll(active & ((1ull << lane) - 1ull));
+        __builtin_amdgcn_wave_barrier();
+        if(any) {
+            list[at] = i;
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { list[WAVE * (q + 1) + at] = mine[q]; }
+        }
+        if((count & 1) && lane == 0) {
+            list[count] = base;                         // (count < 64; base < sliceEnd)
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { list[WAVE * (q + 1) + count] = 0u; }
+        }
+        __builtin_amdgcn_wave_barrier();
+        return count;
+    };
+    bool nonFinite = false;
+    for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
+        const uint32_t pairs = (pack(base) + 1) / 2;
+        for(uint32_t p = 0; p < pairs; p += 8) {
+            float b[8];
+            #pragma unroll
+            for(uint32_t u = 0; u < 8; u++) { b[u] = w[(size_t)list[2 * min(p + u, pairs - 1) + half] * numTrg]; }
+            #pragma unroll
+            for(uint32_t u = 0; u < 8; u++) {
+                if(p + u < pairs) {
+                    const bool finite = aheadFinite(b[u]);
+                    nonFinite = nonFinite || !finite;
+                    const float weight = finite ? b[u] : 0.0f;
+                    #pragma unroll
+                    for(int q = 0; q < MT; q++) {
+                        const uint32_t bits = list[WAVE * (q + 1) + 2 * (p + u) + half];
+                        // (two sources silent in all 32 steps: frequent at low activity and in the last, short word of a run)
+                        if(__ballot(bits != 0)) { acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits, col), weight, acc[q], 0, 0, 0); }
+                    }
+                }
+            }
+        }
+    }
+    if(__ballot(nonFinite)) {
+        for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
+            const uint32_t count = pack(base);
+            for(uint32_t k = 0; k < count; k++) {
+                const float b = w[(size_t)list[k] * numTrg];
+                if(aheadFinite(b)) { continue; }
+                #pragma unroll
+                for(int q = 0; q < MT; q++) {
+                    const uint32_t bits = list[WAVE * (q + 1) + k];
+                    #pragma unroll
+                    for(uint32_t v = 0; v < 16; v++) { acc[q][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                }
+            }
+        }
+    }
+    // ---- the wavefronts' tiles: four copies in LDS, two rounds, then the sum of the copies
+    float *tiles = reinterpret_cast<float*>(lds);
+    float *copy = tiles + (wave % AHEAD_TILE_COPIES) * TILE;
+    #pragma unroll
+    for(uint32_t round = 0; round < AHEAD_DENSE_WAVES / AHEAD_TILE_COPIES; round++) {
+        __syncthreads();
+        if(wave / AHEAD_TILE_COPIES == round) {
+            #pragma unroll
+            for(int q = 0; q < MT; q++) {
+                #pragma unroll
+                for(uint32_t v = 0; v < 16; v++) {
+                    float *e = &copy[(q * 32 + aheadRow(v, half)) * 32 + col];
+                    *e = round ? *e + acc[q][v] : acc[q][v];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for(uint32_t e = threadIdx.x; e < TILE; e += AHEAD_DENSE_THREADS) {
+        const uint32_t tile = firstTile + e / 1024, row = (e / 32) % 32, j = blockIdx.x * 32 + e % 32;
+        if(tile < mTiles && j < numTrg) {
+            partial[(((size_t)slice * mTiles + tile) * 32 + row) * numTrg + j] = (tiles[e] + tiles[TILE + e]) + (tiles[2 * TILE + e] + tiles[3 * TILE + e]);
+        }
+    }
+}
+
+// What a target neuron needs of its group, and one of its steps: postsynaptic model on outPost plus the step's input, current
+// source, neuron model (operations and order of neuronBulkBody).  Neuron and postsynaptic model are known when the kernel is compiled:
+// the steps are unrolled, and a branch on either would be taken in each of them.
+template<uint32_t MODEL, uint32_t PSM>
+struct AheadNeuron
+{
+    PlainNeuron constants;
+    float psmInit, psmDecay, inject, dt;
+    __device__ __forceinline__ explicit AheadNeuron(const gennmi_neuron_update_group_t &g, float timestep)
+        : constants(plainNeuronOf(g)), psmInit(g.psm[0].init), psmDecay(g.psm[0].expDecay), inject(g.numCS ? g.cs[0].amp : 0.0f), dt(timestep)
+    {
+        constants.model = MODEL;
+    }
+    __device__ __forceinline__ bool step(float input, float &linSyn, float &v0, float &v1) const
+    {
+        float Isyn = 0;
+        linSyn += input;
+        if(PSM == GENNMI_PSM_EXPCURR) {
+            Isyn += psmInit * linSyn;
+            linSyn *= psmDecay;
+        }
+        else {
+            Isyn += linSyn;
+            linSyn = 0.0f;
+        }
+        Isyn += inject;         // (a sum that starts at +0 is never -0: adding +0 where there is no source changes nothing)
+        return plainNeuronStep(constants, Isyn, dt, v0, v1);
+    }
+};
+
+// ---- 3a. the neurons behind a DENSE projection: one lane each, 16 steps' inputs asked for while the 16 before are worked off (a
+// population of 8192 is 128 wavefronts: the chain of steps bounds it, so work-groups are single wavefronts, spread over the chip)
+template<uint32_t MODEL, uint32_t PSM>
+__global__ __launch_bounds__(WAVE)
+void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, const float * __restrict__ partial, uint32_t slices, uint32_t mTiles, uint32_t *lastBits)
+{
+    const gennmi_neuron_update_group_t &g = target->g;
+    const uint32_t n = g.numNeurons, batch = blockIdx.y, lane = threadIdx.x, i = blockIdx.x * WAVE + lane;
+    const uint32_t bitmapWords = (n + 31) / 32;
+    const AheadNeuron<MODEL, PSM> neuron(g, A.dt);
+    const size_t bi = (size_t)batch * n + min(i, n - 1);
+    uint32_t *recordSpk = g.recordSpk;
+    size_t recordingRow = aheadRecordingRow(A, 0);
+    constexpr uint32_t GROUP = 16;
+    GLOBAL_AS float *var0 = asGlobal(g.var0), *var1 = asGlobal(g.var1), *outPost = asGlobal(g.psm[0].outPost);
+    float v0 = var0[bi], v1 = var1[bi], lin = outPost[bi];
+    GLOBAL_AS const float *input = asGlobal(partial) + min(i, n - 1);
+    auto load = [&](uint32_t first, float x[GROUP]) {
+        #pragma unroll
+        for(uint32_t u = 0; u < GROUP; u++) { x[u] = 0.0f; }
+        #pragma unroll 2
+        for(uint32_t k = 0; k < slices; k++) {
+            const size_t row = (((size_t)k * mTiles + (size_t)(first / 32) * A.batch + batch) * 32 + first % 32) * n;
+            #pragma unroll
+            for(uint32_t u = 0; u < GROUP; u++) { x[u] += input[row + (size_t)u * n]; }
+        }
+    };
+    float now[GROUP], next[GROUP];
+    load(0, now);
+    for(uint32_t first = 0; first < A.steps; first += GROUP) {
+        if(first + GROUP < A.steps) { load(first + GROUP, next); }
+        #pragma unroll
+        for(uint32_t u = 0; u < GROUP; u++) {
+            const uint32_t step = first + u;
+            if(step < A.steps) {
+                const bool spiked = neuron.step(now[u], lin, v0, v1);
+                const unsigned long long ballot = __ballot(spiked && i < n);
+                if((lane & 31) == 0 && i < n) {
+                    const uint32_t bits = (uint32_t)(ballot >> lane);
+                    if(recordSpk) { recordSpk[(recordingRow * A.batch + batch) * bitmapWords + (i >> 5)] = bits; }
+                    if(step + 1 == A.steps) { lastBits[(size_t)batch * bitmapWords + (i >> 5)] = bits; }
+                }
+                recordingRow = (recordingRow + 1 == A.recordingRows) ? 0 : recordingRow + 1;
+            }
+        }
+        #pragma unroll
+        for(uint32_t u = 0; u < GROUP; u++) { now[u] = next[u]; }
+    }
+    if(i < n) { var0[bi] = v0; var1[bi] = v1; outPost[bi] = lin; }
+}
+
+// ---- 2b, 3b. Conv2D and its neurons, up to 32 steps.  A work-group owns some output rows of one batch and 32 output channels: the
+// words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes four output pixels at a
+// time: the rows of its four products are timesteps, the inner dimension the (tap, channel) pairs — consecutive words of the patch
+// for one kernel row — and a kernel weight read once serves all four.  The products stay in registers; one swap of half-wavefronts
+// per register pair puts a neuron's 32 inputs into one lane, which takes the neuron through the steps and leaves its spikes as one word.
+// Bound by the fp32 matrix rate: 2 * 32 * 32 FLOP per (pixel, 32 steps, tap, channel).
+template<uint32_t MODEL, uint32_t PSM>
+__global__ __launch_bounds__(BLOCK, 4)
+void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
+                     const float * __restrict__ kernel, uint32_t *spikeWords)
+{
+    extern __shared__ uint32_t shAhead[];
+    const gennmi_neuron_update_group_t &g = target->g;
+    const uint32_t n = g.numNeurons, batch = blockIdx.y, oc = (uint32_t)C.oc, ow = (uint32_t)C.ow;
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
+    const uint32_t y0 = blockIdx.x * C.rowsPerBlock, rows = min(C.rowsPerBlock, (uint32_t)C.oh - y0), pixels = rows * ow;
+    const uint32_t o = blockIdx.z * 32 + col;
+    const uint32_t steps = min(A.steps - wordBlock * AHEAD_WORD, AHEAD_WORD);
+    const AheadNeuron<MODEL, PSM> neuron(g, A.dt);
+    const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), pairs = C.pairsPerRow;
+    uint32_t *patch = shAhead;
+    float *kern = reinterpret_cast<float*>(shAhead + (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch);        // [kh][2 * pairs][32]
+    // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
+    GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
+    const int inRowWords = C.iw * C.ic;
+    for(uint32_t r = 0; r < rows + (uint32_t)C.kh - 1; r++) {
+        const int y = (int)(y0 + r) - C.PH;
+        for(uint32_t e = threadIdx.x; e < rowPitch; e += BLOCK) {
+            const int x = (int)e - C.PW * C.ic;
+            patch[r * rowPitch + e] = (y >= 0 && y < C.ih && x >= 0 && x < inRowWords) ? in[(size_t)y * inRowWords + x] : 0u;
+        }
+    }
+    bool nonFinite = false;
+    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * 2 * pairs * 32; e += BLOCK) {
+        const uint32_t k = e / 32, a = k / (2 * pairs), c = k - a * 2 * pairs, oo = blockIdx.z * 32 + (e & 31);
+        float weight = (c < rowWords && oo < oc) ? asGlobal(kernel)[((size_t)a * rowWords + c) * oc + oo] : 0.0f;
+        if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
+        kern[e] = weight;
+    }
+    nonFinite = __syncthreads_or(nonFinite);
+
+    GLOBAL_AS float *var0 = asGlobal(g.var0) + (size_t)batch * n, *var1 = asGlobal(g.var1) + (size_t)batch * n, *outPost = asGlobal(g.psm[0].outPost) + (size_t)batch * n;
+    GLOBAL_AS uint32_t *spikes = asGlobal(spikeWords) + (size_t)batch * n;
+    for(uint32_t first = wave * 4; first < pixels; first += (BLOCK / WAVE) * 4) {
+        uint32_t base[4];
+        #pragma unroll
+        for(uint32_t j = 0; j < 4; j++) {
+            const uint32_t p = min(first + j, pixels - 1), r = p / ow;
+            base[j] = r * rowPitch + (p - r * ow) * (uint32_t)C.ic + half;
+        }
+        // state of the lane's two neurons (pixels first + half and first + 2 + half, channel o), asked for before the products
+        bool valid[2]; size_t at[2]; float v0[2], v1[2], lin[2];
+        #pragma unroll
+        for(uint32_t m = 0; m < 2; m++) {
+            const uint32_t p = first + 2 * m + half;
+            valid[m] = (p < pixels && o < oc);
+            at[m] = valid[m] ? ((size_t)y0 * ow + p) * oc + o : 0;
+            v0[m] = var0[at[m]]; v1[m] = var1[at[m]]; lin[m] = outPost[at[m]];
+        }
+        f32x16 acc[4];
+        #pragma unroll
+        for(int j = 0; j < 4; j++) { acc[j] = f32x16{}; }
+        const float *weight = kern + half * 32 + col;
+        for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
+            // four pairs a round: their reads from LDS are issued together, ahead of the sixteen products
+            uint32_t c = 0;
+            for(; c + 4 <= pairs; c += 4) {
+                float b[4]; uint32_t bits[4][4];
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) {
+                    b[u] = weight[(c + u) * 64];
+                    #pragma unroll
+                    for(int j = 0; j < 4; j++) { bits[u][j] = patch[base[j] + 2 * (c + u)]; }
+                }
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) {
+                    #pragma unroll
+                    for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits[u][j], col), b[u], acc[j], 0, 0, 0); }
+                }
+            }
+            for(; c < pairs; c++) {
+                const float b = weight[c * 64];
+                #pragma unroll
+                for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(patch[base[j] + 2 * c], col), b, acc[j], 0, 0, 0); }
+            }
+            weight += pairs * 64;
+            #pragma unroll
+            for(int j = 0; j < 4; j++) { base[j] += rowPitch; }
+        }
+        if(nonFinite) {
+            // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
+            for(uint32_t k = 0; k < (uint32_t)C.kh * rowWords; k++) {
+                const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
+                if(aheadFinite(b)) { continue; }
+                const uint32_t a = k / rowWords;
+                #pragma unroll
+                for(int j = 0; j < 4; j++) {
+                    const uint32_t bits = patch[base[j] - half - ((uint32_t)C.kh - a) * rowPitch + (k - a * rowWords)];
+                    #pragma unroll
+                    for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                }
+            }
+        }
+        #pragma unroll
+        for(int m = 0; m < 2; m++) {
+            // lower half: all steps of the first pixel of the pair, upper half: of the second
+            float x[16], y[16];
+            #pragma unroll
+            for(int v = 0; v < 16; v++) {
+                const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[2 * m][v]), __float_as_uint(acc[2 * m + 1][v]), false, false);
+                x[v] = __uint_as_float(swapped[0]); y[v] = __uint_as_float(swapped[1]);
+            }
+            uint32_t fired = 0;
+            #pragma unroll
+            for(uint32_t t = 0; t < AHEAD_WORD; t++) {
+                // (kept a comparison and a branch: computed ahead for all steps, the conditions are 32 masks, spilled)
+                uint32_t end = steps;
+                asm volatile("" : "+s"(end));
+                if(t < end) {
+                    asm volatile("" : "+v"(lin[m]));
+                    const float input = (t & 4) ? y[4 * (t / 8) + (t & 3)] : x[4 * (t / 8) + (t & 3)];
+                    fired |= neuron.step(input, lin[m], v0[m], v1[m]) ? 1u << t : 0u;
+                }
+            }
+            if(valid[m]) { var0[at[m]] = v0[m]; var1[at[m]] = v1[m]; outPost[at[m]] = lin[m]; spikes[at[m]] = fired; }
+        }
+    }
+}
+
+// The layer's spikes turned from one word per neuron (32 steps) into one word per step (32 neurons): the recording rows and the bitmap of
+// the last step.  A work-group takes 1024 neurons so that a step's words leave as 128 consecutive bytes.
+__global__ __launch_bounds__(BLOCK)
+void aheadTransposeKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, uint32_t wordBlock, const uint32_t * __restrict__ spikeWords, uint32_t *lastBits)
+{
+    __shared__ uint32_t rows[AHEAD_WORD][33];
+    const gennmi_neuron_update_group_t &g = target->g;
+    const uint32_t n = g.numNeurons, batch = blockIdx.y, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const uint32_t steps = min(A.steps - wordBlock * AHEAD_WORD, AHEAD_WORD), bitmapWords = (n + 31) / 32;
+    uint32_t mine[4];
+    #pragma unroll
+    for(uint32_t q = 0; q < 4; q++) {
+        const uint32_t i = blockIdx.x * 1024 + (wave * 4 + q) * WAVE + lane;
+        mine[q] = (i < n) ? asGlobal(spikeWords)[(size_t)batch * n + i] : 0u;
+    }
+    // (low: the bits b with b & j == 0)
+    auto exchange = [&](uint32_t &x, uint32_t j, uint32_t low) {
+        const uint32_t other = (uint32_t)__shfl_xor((int)x, (int)j, WAVE);
+        x = (lane & j) ? ((x & ~low) | ((other & ~low) >> j)) : ((x & low) | ((other & low) << j));
+    };
+    #pragma unroll
+    for(uint32_t q = 0; q < 4; q++) {
+        // 32 x 32 bits per half-wave, transposed by exchanging ever smaller blocks across the diagonal (32 ballots and selects: 18 us
+        // for 2.1 x 10^6 neurons)
+        uint32_t x = mine[q];
+        exchange(x, 16, 0x0000FFFFu);
+        exchange(x, 8, 0x00FF00FFu);
+        exchange(x, 4, 0x0F0F0F0Fu);
+        exchange(x, 2, 0x33333333u);
+        exchange(x, 1, 0x55555555u);
+        rows[lane & 31][(wave * 4 + q) * 2 + (lane >> 5)] = x;
+    }
+    __syncthreads();
+    for(uint32_t e = threadIdx.x; e < AHEAD_WORD * 32; e += BLOCK) {
+        const uint32_t t = e / 32, word = blockIdx.x * 32 + e % 32, step = wordBlock * AHEAD_WORD + t;
+        if(t >= steps || word >= bitmapWords) { continue; }
+        // (of the steps of this launch that share a recording row only the last writes it)
+        if(g.recordSpk && t + A.recordingRows >= steps) { g.recordSpk[(aheadRecordingRow(A, step) * A.batch + batch) * bitmapWords + word] = rows[t][e % 32]; }
+        if(step + 1 == A.steps) { lastBits[(size_t)batch * bitmapWords + word] = rows[t][e % 32]; }
+    }
+}
+
+// ---- 4. the queues of both populations from the bitmaps of the last step: a work-group per population and batch, its threads
+// own consecutive words, so a scan of their counts is the ascending order
+constexpr uint32_t AHEAD_QUEUE_THREADS = 1024;
+__global__ __launch_bounds__(AHEAD_QUEUE_THREADS)
+void aheadQueueKernel(const NeuronGroupDev * __restrict__ populations, const uint32_t *sourceBits, const uint32_t *targetBits)
+{
+    __shared__ uint32_t waveTotal[AHEAD_QUEUE_THREADS / WAVE];
+    const gennmi_neuron_update_group_t &g = populations[blockIdx.x].g;
+    const uint32_t n = g.numNeurons, words = (n + 31) / 32, batch = blockIdx.y, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    GLOBAL_AS const uint32_t *bits = asGlobal(blockIdx.x ? targetBits : sourceBits) + (size_t)batch * words;
+    GLOBAL_AS uint32_t *queue = asGlobal(g.spk) + (size_t)batch * n;
+    const uint32_t per = (words + AHEAD_QUEUE_THREADS - 1) / AHEAD_QUEUE_THREADS;
+    const uint32_t begin = min(threadIdx.x * per, words), end = min(begin + per, words);
+    uint32_t mine = 0;
+    for(uint32_t w = begin; w < end; w++) { mine += __popc(bits[w]); }
+    uint32_t scan = mine;
+    for(int off = 1; off < WAVE; off <<= 1) { const uint32_t up = __shfl_up(scan, off, WAVE); if(lane >= (uint32_t)off) { scan += up; } }
+    if(lane == WAVE - 1) { waveTotal[wave] = scan; }
+    __syncthreads();
+    uint32_t position = scan - mine, total = 0;
+    for(uint32_t w = 0; w < AHEAD_QUEUE_THREADS / WAVE; w++) {
+        if(w < wave) { position += waveTotal[w]; }
+        total += waveTotal[w];
+    }
+    for(uint32_t w = begin; w < end; w++) {
+        uint32_t word = bits[w];
+        while(word) {
+            const uint32_t bit = __ffs(word) - 1;
+            word &= word - 1;
+            queue[position++] = w * 32 + bit;
+        }
+    }
+    if(threadIdx.x == 0) { g.spkCnt[batch] = total; }
+}
+}   // namespace

@@ -1,0 +1,162 @@
+"""run() on feed-forward layers: up to 128 steps at once, the layer's input over the steps as a matrix product on the matrix
+cores.  Weights are multiples of 2^-8 and the postsynaptic model keeps nothing between steps (unless said otherwise), so every
+fp32 sum is exact in any order and queues, rasters, state and event counts must be those of the CPU oracle bit for bit."""
+import copy
+
+import numpy as np
+import pytest
+
+from genn_amd import configs
+from genn_amd.genn_model import model_from_net
+from oracle.genn_cpu import OracleNet
+from parity import compare_state
+
+pytestmark = pytest.mark.gpu
+
+
+def _net(kind, shape, steps, psm="deltacurr", batch_index=0):
+    if kind == "dense":
+        n_in, n_out = shape
+        net = configs.dense_layer(n_in=n_in, n_out=n_out, rate_hz=120.0, steps=steps, w_sd=6.0 / np.sqrt(n_in))
+        if batch_index:
+            source = net.pop("In")
+            source.vars["startSpike"], source.vars["endSpike"], source.spike_times = configs.poisson_spike_source(17, 50 + batch_index, n_in, 120.0, steps, 1.0)
+    else:
+        h, w, ic, oc, k = shape
+        net = configs.conv_toeplitz(h=h, w=w, ic=ic, oc=oc, k=k, steps=steps, w_sd=3.0 / k, max_rate=200.0, ioffset=0.3, batch_index=batch_index)
+    syn = net.syns[0]
+    syn.g = (np.rint(syn.g * 256.0) / 256.0).astype(np.float32)
+    syn.psm = psm
+    return net
+
+
+def _same_rasters(net, model, oracle, steps):
+    model.pull_recording_buffers_from_device()
+    for p in net.pops:
+        words = (p.n + 31) // 32
+        assert np.array_equal(model.neuron_populations[p.name].vars["recordSpk"].view.reshape(steps, words), oracle.record(p.name, steps).reshape(steps, words)), p.name
+        assert np.array_equal(model.neuron_populations[p.name].current_spikes[0], oracle.spikes(p.name)), p.name
+
+
+# sizes around a product's 32 columns, a chunk of 64 sources, a work-group's 512; output pixels around the four of a wavefront, channel
+# counts that make an odd number of taps, more than 32 output channels, an even kernel
+SHAPES = [("dense", (1, 1)), ("dense", (63, 31)), ("dense", (65, 33)), ("dense", (512, 64)), ("dense", (1300, 70)), ("dense", (300, 1000)),
+          ("conv", (1, 1, 1, 1, 3)), ("conv", (5, 7, 3, 4, 3)), ("conv", (9, 6, 1, 33, 5)), ("conv", (8, 8, 16, 32, 3)), ("conv", (6, 5, 2, 40, 1))]
+
+
+@pytest.mark.parametrize("kind,shape", SHAPES, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_runs_of_every_length_mixed_with_single_steps(kind, shape):
+    """Runs on either side of the shortest that is taken at once, of a word of 32 steps and of the longest launch of 128."""
+    chunks = [1, 3, 4, 1, 31, 32, 33, 2, 137, 0, 64]
+    steps = sum(chunks)
+    net = _net(kind, shape, steps)
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=steps)
+    assert model.runner_info()["feed_forward_ahead"]
+    oracle = OracleNet(net, num_recording_timesteps=steps)
+    for chunk in chunks:
+        if chunk == 1:
+            model.step_time()
+        else:
+            model.run(chunk)
+        oracle.run(chunk)
+        compare_state(net, model, oracle, f"after {chunk} more steps", exact=True)
+    _same_rasters(net, model, oracle, steps)
+    assert model.synaptic_event_count == oracle.events()
+    assert int(np.unpackbits(oracle.record("In", steps).view(np.uint8)).sum()) > 0
+    model.unload()
+
+
+@pytest.mark.parametrize("kind,shape,model_name", [("dense", (700, 130), "izh"), ("dense", (700, 130), "lif"), ("conv", (9, 10, 3, 8, 3), "izh"), ("conv", (9, 10, 3, 8, 3), "lif")])
+def test_exponential_synapses_and_both_neuron_models(kind, shape, model_name):
+    """outPost carries over from step to step: the layer's sum is added to it at once instead of weight by weight.  LIF neurons contract
+    such a difference: 1e-5.  The half steps of an Izhikevich neuron multiply one of V by 1 + (0.04 V + 2.5): 1.9^2 a step at -40 mV,
+    2.5^2 at -25, 3.9^2 at +10, about 300 over the upstroke of a spike, and U keeps a share of it: 300 times three roundings of 2^-24
+    is 5e-5 a spike, and the neurons fire fewer than ten times: 5e-4.  The rasters have to be identical."""
+    steps = 100
+    net = _net(kind, shape, steps, psm="expcurr")
+    if model_name == "izh":
+        out = net.pop("Out")
+        out.model, out.params = "izh", dict(a=0.02, b=0.2, c=-65.0, d=8.0)
+        out.vars = {"V": np.full(out.n, -65.0, np.float32), "U": np.full(out.n, -13.0, np.float32)}
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=steps)
+    assert model.runner_info()["feed_forward_ahead"]
+    oracle = OracleNet(net, num_recording_timesteps=steps)
+    model.run(steps)
+    oracle.run(steps)
+    if model_name == "lif":
+        compare_state(net, model, oracle, "after the run", exact=False)
+    else:
+        for k, name in enumerate(("V", "U")):
+            want = oracle.var("Out", k)
+            assert np.abs(model.neuron_populations["Out"].vars[name].pull_from_device() - want).max() <= 5e-4 * np.abs(want).max(), name
+    _same_rasters(net, model, oracle, steps)
+    model.unload()
+
+
+@pytest.mark.parametrize("kind,shape,batch", [("dense", (150, 70), 3), ("dense", (150, 70), 9), ("conv", (7, 6, 2, 5, 3), 3)])
+def test_batches_recording_rows_reused_and_source_rewritten(kind, shape, batch, monkeypatch):
+    """Batches are independent; a recording buffer of fewer rows than the run keeps the last step of each row; spike times and a queue
+    written between runs count.  Against the same network stepped launch by launch."""
+    steps, rows = 70, 6
+    nets = [_net(kind, shape, steps, batch_index=b) for b in range(batch)]
+    times = np.concatenate([n.pop("In").spike_times for n in nets])
+    offs = np.cumsum([0] + [len(n.pop("In").spike_times) for n in nets])
+    net = copy.deepcopy(nets[0])
+    net.pop("In").vars = {v: np.stack([n.pop("In").vars[v] + offs[b] for b, n in enumerate(nets)]).astype(np.uint32) for v in ("startSpike", "endSpike")}
+    net.pop("In").spike_times = times
+    models = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        model = model_from_net(net, batch_size=batch)
+        model.load(num_recording_timesteps=rows)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        models.append(model)
+    start = models[0].neuron_populations["In"].vars["startSpike"].view.copy()
+    for turn in range(2):
+        for model in models:
+            model.run(steps)
+            model.pull_recording_buffers_from_device()
+        for p in net.pops:
+            a, b = (m.neuron_populations[p.name] for m in models)
+            assert np.array_equal(a.vars["recordSpk"].view, b.vars["recordSpk"].view), p.name
+            for name in ("V", "RefracTime", "startSpike"):
+                if name in a.vars:
+                    assert np.array_equal(a.vars[name].pull_from_device(), b.vars[name].pull_from_device()), name
+            for k in range(batch):
+                assert np.array_equal(a.current_spikes[k], b.current_spikes[k])
+        assert models[0].synaptic_event_count == models[1].synaptic_event_count > 0
+        for model in models:
+            # the trains once more, 70 steps later, behind a queue of two spikes
+            source = model.neuron_populations["In"]
+            source.vars["spikeTimes"].view[:len(times)] = times + steps
+            source.vars["startSpike"].view[:] = start
+            source.vars["spkCnt"].view[:] = 2
+            source.vars["spk"].view.reshape(batch, -1)[:, :2] = [3, 11]
+            for v in ("spikeTimes", "startSpike", "spkCnt", "spk"):
+                source.vars[v].push_to_device()
+    for model in models:
+        model.unload()
+
+
+@pytest.mark.parametrize("kind,shape", [("dense", (200, 40)), ("conv", (6, 7, 2, 5, 3))])
+def test_weights_that_are_not_finite_reach_their_own_spikes_only(kind, shape, monkeypatch):
+    """0 * inf is NaN: an infinite weight of a source that is silent in a step must not touch that step."""
+    steps = 40
+    net = _net(kind, shape, steps)
+    g = net.syns[0].g.reshape(-1)
+    g[[5, 17]] = [np.inf, -np.inf]
+    vs = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        monkeypatch.setenv("GENNMI_CONV_MFMA", ahead)       # (compared with the event-driven kernels: spike by spike)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        model.run(steps)
+        model.pull_recording_buffers_from_device()
+        vs.append((model.neuron_populations["Out"].vars["V"].pull_from_device().copy(), model.neuron_populations["Out"].vars["recordSpk"].view.copy()))
+        model.unload()
+    assert np.array_equal(vs[0][0], vs[1][0], equal_nan=True) and np.array_equal(vs[0][1], vs[1][1])
+    assert np.isfinite(vs[0][0]).any()
