@@ -8,14 +8,13 @@
 //   1. aheadSourceKernel: a lane walks one source neuron's spikes of all these steps.  Its input to the layer is one 32-bit word per
 //      32 steps (bit j: the layer receives a spike from it in step j).
 //   2. the layer's input of 32 steps is a matrix product whose left operand is those bits: rows are timesteps, the inner
-//      dimension the source neurons (DENSE) or an output pixel's taps (Conv2D), columns the target neurons.  A bit becomes the
-//      operand of v_mfma_f32_32x32x2_f32 by a shift, a mask and a conversion; 0 / 1 times an fp32 weight is exact and sums are fp32.
+//      dimension the source neurons (DENSE) or an output pixel's taps (Conv2D), columns the target neurons.  See aheadProduct.
 //   3. the neurons: a lane takes one neuron through the steps with its state in registers.
 //   4. aheadQueueKernel: the spike queues as the last step leaves them, in ascending neuron index.
 // What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
 //
-// Measured with the kernels' launches, copies and waits (run() and its copies; before -> after): DENSE 8192 -> 8192 at 5 % activity,
-// 100 steps; Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: see the kernels.
+// run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 205 us;
+// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 850 us, of which 500 move 26 MB between host and device.
 #pragma once
 
 namespace
@@ -33,7 +32,9 @@ struct AheadArgs
 struct AheadConv
 {
     int32_t kh, kw, ih, iw, ic, oh, ow, oc, PH, PW;
-    uint32_t rowsPerBlock, rowPitch, pairsPerRow;       // patch row in words; (tap, channel) pairs of one kernel row
+    uint32_t rowsPerBlock;
+    uint32_t channels;                  // input channels, made even
+    uint32_t rowPitch, rowTaps;         // patch row and (tap, channel) pairs of one kernel row, the latter filled up to whole products of 16
     uint32_t isConv;
 };
 
@@ -123,25 +124,46 @@ void aheadSourceKernel(const NeuronGroupDev * __restrict__ source, AheadArgs A, 
     if(lane == 0 && events) { addEvents(eventCounter, events); }
 }
 
-__device__ __forceinline__ float aheadBit(uint32_t word, uint32_t row) { return (float)((word >> row) & 1u); }
-__device__ __forceinline__ bool aheadFinite(float w) { return (__float_as_uint(w) & 0x7F800000u) != 0x7F800000u; }
+// The product of 32 steps' bits and 32 columns of weights for 16 sources (or taps): v_mfma_f32_32x32x16_bf16 three times.  A bit is 0 or 1, and an
+// fp32 weight is exactly the sum of three bfloat16 numbers of 8 significant bits each, so every product is exact, as it is with the fp32
+// instruction (v_mfma_f32_32x32x2_f32), which takes eight times 64 clocks for what these three do in 32 each; sums are fp32 either way
+// and are rounded less often.  That split needs the lowest of the three to be a normal number and the weight to be finite: weights that are
+// not (infinities, NaN, below 2^-90) are multiplied as 0 and added afterwards to the steps that have their spike.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ bool aheadOrdinary(float w)
+{
+    const uint32_t bits = __float_as_uint(w);
+    return ((bits & 0x7F800000u) - (37u << 23)) < ((255u - 37u) << 23) || (bits << 1) == 0u;
+}
+// top 16 bits of two words, packed; what the top 16 bits leave of a float (exact)
+__device__ __forceinline__ uint32_t aheadTop(float lower, float upper) { return __builtin_amdgcn_perm(__float_as_uint(upper), __float_as_uint(lower), 0x07060302u); }
+__device__ __forceinline__ float aheadRest(float w) { return w - __uint_as_float(__float_as_uint(w) & 0xFFFF0000u); }
+// a lane's operand of 8 sources: bit `row` (0..15) of each half of four words as bfloat16 0 or 1
+__device__ __forceinline__ bf16x8 aheadBits(u32x4 words, uint32_t row)
+{
+    u32x4 operand;
+    #pragma unroll
+    for(int k = 0; k < 4; k++) { operand[k] = ((words[k] >> row) & 0x00010001u) * 0x3F80u; }
+    return __builtin_bit_cast(bf16x8, operand);
+}
+__device__ __forceinline__ f32x16 aheadProduct(bf16x8 bits, bf16x8 weights, f32x16 sum) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(bits, weights, sum, 0, 0, 0); }
 // the accumulator's element v of a lane in the given half is timestep ...
 __device__ __forceinline__ uint32_t aheadRow(uint32_t v, uint32_t half) { return 8 * (v / 4) + 4 * half + (v % 4); }
 
 // ---- 2a. DENSE.  A work-group owns 32 target neurons (columns), up to MT words of (32 steps, batch) as rows and a slice of the
 // source; its wavefronts deal the slice's chunks of 64 source neurons among themselves and add their tiles up in LDS in a fixed order.
 // Source neurons that are silent in all of the group's steps are dropped first (a ballot packs the others), so what is
-// read and multiplied follows the activity: at 5 % and 128 steps all rows remain, at 0.1 % one in eight.  Bound by the fp32 matrix
-// rate for long runs (8192 x 8192 x 128 rows: 17.2 GFLOP) and by reading the weights for short ones.  A weight that is not finite
-// would reach the steps without its spike as 0 * inf: the loop multiplies 0 in its place and such weights are added, step
-// by step, in a pass of their own.
+// read and multiplied follows the activity: at 5 % and 128 steps all rows remain, at 0.1 % one in eight.  Bound by reading the weights:
+// 8192 x 8192 for 100 steps takes 75 us, 3.6 TB/s (152 us with v_mfma_f32_32x32x2_f32, bound by the matrix rate).  Error of outPost after
+// 100 steps against 64 bits, one by one -> here (2-norm, relative): 8192 sources 2.0e-7 -> 1.4e-7, 300 sources 1.6e-7 -> 0.8e-7, weights of
+// one sign 1.4e-7 -> 0.7e-7.
 template<int MT>
 __global__ __launch_bounds__(AHEAD_DENSE_THREADS)
 void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint32_t mGroups, const float * __restrict__ weights, uint32_t numSrc, uint32_t numTrg,
                       uint32_t sourcesPerSlice, float * __restrict__ partial)
 {
     constexpr uint32_t LIST_WORDS = WAVE * (MT + 1), TILE = MT * 32 * 32;
-    __shared__ uint32_t lds[(AHEAD_DENSE_WAVES * LIST_WORDS > AHEAD_TILE_COPIES * TILE) ? AHEAD_DENSE_WAVES * LIST_WORDS : AHEAD_TILE_COPIES * TILE];
+    __shared__ __align__(16) uint32_t lds[(AHEAD_DENSE_WAVES * LIST_WORDS > AHEAD_TILE_COPIES * TILE) ? AHEAD_DENSE_WAVES * LIST_WORDS : AHEAD_TILE_COPIES * TILE];
     const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
     const uint32_t mGroup = blockIdx.y % mGroups, slice = blockIdx.y / mGroups;
     const uint32_t firstTile = mGroup * MT;
@@ -149,11 +171,13 @@ void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint
     const uint32_t sliceBegin = slice * sourcesPerSlice, sliceEnd = min(numSrc, sliceBegin + sourcesPerSlice);
     GLOBAL_AS const uint32_t *in = asGlobal(words);
     GLOBAL_AS const float *w = asGlobal(weights) + readColumn;
-    uint32_t *list = lds + wave * LIST_WORDS;           // [64] source neurons, then [MT][64] their words
+    // [64] source neurons, then per tile [64] lower and [64] upper halves of their words, 16 bits each
+    uint32_t *list = lds + wave * LIST_WORDS;
+    uint16_t *halves = reinterpret_cast<uint16_t*>(list + WAVE);
     f32x16 acc[MT];
     #pragma unroll
     for(int q = 0; q < MT; q++) { acc[q] = f32x16{}; }
-    // the active ones of 64 source neurons, packed; returns how many (an odd number is followed by an entry without spikes)
+    // the active ones of 64 source neurons, packed and filled up to a multiple of 16 with entries without spikes; returns how many
     auto pack = [&](uint32_t base) -> uint32_t {
         const uint32_t i = base + lane;
         uint32_t mine[MT], any = 0;
@@ -163,55 +187,74 @@ void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint
             any |= mine[q];
         }
         const unsigned long long active = __ballot(any != 0);
-        const uint32_t count = __popcll(active), at = __popcll(active & ((1ull << lane) - 1ull));
-        __builtin_amdgcn_wave_barrier();
-        if(any) {
-            list[at] = i;
+        const uint32_t count = __popcll(active), filled = (count + 15) / 16 * 16;
+        // (a silent one, any of them, fills: it has no bits)
+        const uint32_t at = any ? __popcll(active & ((1ull << lane) - 1ull)) : count + __popcll(~active & ((1ull << lane) - 1ull));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");      // (16-bit stores, 128-bit loads: the compiler must not move either across)
+        if(at < filled) {
+            list[at] = min(i, sliceEnd - 1);
             #pragma unroll
-            for(int q = 0; q < MT; q++) { list[WAVE * (q + 1) + at] = mine[q]; }
-        }
-        if((count & 1) && lane == 0) {
-            list[count] = base;                         // (count < 64; base < sliceEnd)
-            #pragma unroll
-            for(int q = 0; q < MT; q++) { list[WAVE * (q + 1) + count] = 0u; }
-        }
-        __builtin_amdgcn_wave_barrier();
-        return count;
-    };
-    bool nonFinite = false;
-    for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
-        const uint32_t pairs = (pack(base) + 1) / 2;
-        for(uint32_t p = 0; p < pairs; p += 8) {
-            float b[8];
-            #pragma unroll
-            for(uint32_t u = 0; u < 8; u++) { b[u] = w[(size_t)list[2 * min(p + u, pairs - 1) + half] * numTrg]; }
-            #pragma unroll
-            for(uint32_t u = 0; u < 8; u++) {
-                if(p + u < pairs) {
-                    const bool finite = aheadFinite(b[u]);
-                    nonFinite = nonFinite || !finite;
-                    const float weight = finite ? b[u] : 0.0f;
-                    #pragma unroll
-                    for(int q = 0; q < MT; q++) {
-                        const uint32_t bits = list[WAVE * (q + 1) + 2 * (p + u) + half];
-                        // (two sources silent in all 32 steps: frequent at low activity and in the last, short word of a run)
-                        if(__ballot(bits != 0)) { acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits, col), weight, acc[q], 0, 0, 0); }
-                    }
-                }
+            for(int q = 0; q < MT; q++) {
+                halves[(2 * q) * WAVE + at] = (uint16_t)mine[q];
+                halves[(2 * q + 1) * WAVE + at] = (uint16_t)(mine[q] >> 16);
             }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        return filled;
+    };
+    // a lane's rows are the steps of its column number: the lower or the upper halves
+    const u32x4 *bits = reinterpret_cast<const u32x4*>(list + WAVE + (col >> 4) * (WAVE / 2)) + half;
+    const u32x4 *sources = reinterpret_cast<const u32x4*>(list) + 2 * half;
+    bool special = false;
+    for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
+        const uint32_t groups = pack(base) / 16;
+        float b[8], bNext[8];
+        auto load = [&](uint32_t g, float x[8]) {
+            const u32x4 first = sources[4 * g], second = sources[4 * g + 1];
+            #pragma unroll
+            for(int k = 0; k < 4; k++) { x[k] = w[(size_t)first[k] * numTrg]; x[4 + k] = w[(size_t)second[k] * numTrg]; }
+        };
+        if(groups) { load(0, b); }
+        for(uint32_t g = 0; g < groups; g++) {
+            if(g + 1 < groups) { load(g + 1, bNext); }
+            u32x4 top, middle, low;
+            #pragma unroll
+            for(int k = 0; k < 8; k++) {
+                const bool ordinary = aheadOrdinary(b[k]);
+                special = special || !ordinary;
+                b[k] = ordinary ? b[k] : 0.0f;
+            }
+            #pragma unroll
+            for(int k = 0; k < 4; k++) {
+                const float r0 = aheadRest(b[2 * k]), r1 = aheadRest(b[2 * k + 1]);
+                top[k] = aheadTop(b[2 * k], b[2 * k + 1]);
+                middle[k] = aheadTop(r0, r1);
+                low[k] = aheadTop(aheadRest(r0), aheadRest(r1));
+            }
+            bf16x8 a[MT];
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { a[q] = aheadBits(bits[q * (WAVE / 4) + 2 * g], col & 15); }
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, low), acc[q]); }
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, middle), acc[q]); }
+            #pragma unroll
+            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, top), acc[q]); }
+            #pragma unroll
+            for(int k = 0; k < 8; k++) { b[k] = bNext[k]; }
+        }
     }
-    if(__ballot(nonFinite)) {
+    if(__ballot(special)) {
         for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
             const uint32_t count = pack(base);
             for(uint32_t k = 0; k < count; k++) {
-                const float b = w[(size_t)list[k] * numTrg];
-                if(aheadFinite(b)) { continue; }
+                const float x = w[(size_t)list[k] * numTrg];
+                if(aheadOrdinary(x)) { continue; }
                 #pragma unroll
                 for(int q = 0; q < MT; q++) {
-                    const uint32_t bits = list[WAVE * (q + 1) + k];
+                    const uint32_t word = halves[(2 * q) * WAVE + k] | ((uint32_t)halves[(2 * q + 1) * WAVE + k] << 16);
                     #pragma unroll
-                    for(uint32_t v = 0; v < 16; v++) { acc[q][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                    for(uint32_t v = 0; v < 16; v++) { acc[q][v] += ((word >> aheadRow(v, half)) & 1u) ? x : 0.0f; }
                 }
             }
         }
@@ -324,17 +367,20 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
 }
 
 // ---- 2b, 3b. Conv2D and its neurons, up to 32 steps.  A work-group owns some output rows of one batch and 32 output channels: the
-// words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes four output pixels at a
+// words of the input pixels they reach (zero outside the input) and the kernel, split, wait in LDS.  A wavefront takes four output pixels at a
 // time: the rows of its four products are timesteps, the inner dimension the (tap, channel) pairs — consecutive words of the patch
-// for one kernel row — and a kernel weight read once serves all four.  The products stay in registers; one swap of half-wavefronts
-// per register pair puts a neuron's 32 inputs into one lane, which takes the neuron through the steps and leaves its spikes as one word.
-// Bound by the fp32 matrix rate: 2 * 32 * 32 FLOP per (pixel, 32 steps, tap, channel).
+// for one kernel row, filled up to whole products of 16 with zero weights — and a kernel weight read once serves all four.  The products
+// stay in registers; one swap of half-wavefronts per register pair puts a neuron's 32 inputs into one lane, which takes the neuron
+// through the steps and leaves its spikes as one word.  Bound by instruction issue: 64x64x16 -> 64x64x32 3x3, batch 16 takes 94 us for
+// 32 steps, of which the products are 23 at the matrix rate, and 74 for 18 steps (229 and 201 with v_mfma_f32_32x32x2_f32, the matrix rate's
+// 123 bounding it).
+constexpr uint32_t AHEAD_CONV_THREADS = 512;
 template<uint32_t MODEL, uint32_t PSM>
-__global__ __launch_bounds__(BLOCK, 4)
+__global__ __launch_bounds__(AHEAD_CONV_THREADS, 4)
 void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
                      const float * __restrict__ kernel, uint32_t *spikeWords)
 {
-    extern __shared__ uint32_t shAhead[];
+    extern __shared__ __align__(16) uint32_t shAhead[];
     const gennmi_neuron_update_group_t &g = target->g;
     const uint32_t n = g.numNeurons, batch = blockIdx.y, oc = (uint32_t)C.oc, ow = (uint32_t)C.ow;
     const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
@@ -342,36 +388,57 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     const uint32_t o = blockIdx.z * 32 + col;
     const uint32_t steps = min(A.steps - wordBlock * AHEAD_WORD, AHEAD_WORD);
     const AheadNeuron<MODEL, PSM> neuron(g, A.dt);
-    const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), pairs = C.pairsPerRow;
-    uint32_t *patch = shAhead;
-    float *kern = reinterpret_cast<float*>(shAhead + (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch);        // [kh][2 * pairs][32]
-    // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
+    const uint32_t rowPitch = C.rowPitch, taps = (uint32_t)C.kw * C.channels, products = C.rowTaps / 16;
+    // the kernel: [kh][products][piece][half][32 columns] of 8 bfloat16 each (16 bytes a lane, lane-consecutive)
+    u32x4 *kern = reinterpret_cast<u32x4*>(shAhead);
+    // the patch: lower halves of the words, then upper halves, [rows + kh - 1][rowPitch] of 16 bits each
+    const uint32_t plane = (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch;
+    uint16_t *patch = reinterpret_cast<uint16_t*>(kern + (size_t)C.kh * products * 3 * WAVE);
     GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
-    const int inRowWords = C.iw * C.ic;
     for(uint32_t r = 0; r < rows + (uint32_t)C.kh - 1; r++) {
         const int y = (int)(y0 + r) - C.PH;
-        for(uint32_t e = threadIdx.x; e < rowPitch; e += BLOCK) {
-            const int x = (int)e - C.PW * C.ic;
-            patch[r * rowPitch + e] = (y >= 0 && y < C.ih && x >= 0 && x < inRowWords) ? in[(size_t)y * inRowWords + x] : 0u;
+        for(uint32_t e = threadIdx.x; e < rowPitch; e += AHEAD_CONV_THREADS) {
+            const uint32_t column = e / C.channels, channel = e - column * C.channels;
+            const int x = (int)column - C.PW;
+            const uint32_t word = (y >= 0 && y < C.ih && x >= 0 && x < C.iw && channel < (uint32_t)C.ic) ? in[((size_t)y * C.iw + x) * C.ic + channel] : 0u;
+            patch[r * rowPitch + e] = (uint16_t)word;
+            patch[plane + r * rowPitch + e] = (uint16_t)(word >> 16);
         }
     }
-    bool nonFinite = false;
-    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * 2 * pairs * 32; e += BLOCK) {
-        const uint32_t k = e / 32, a = k / (2 * pairs), c = k - a * 2 * pairs, oo = blockIdx.z * 32 + (e & 31);
-        float weight = (c < rowWords && oo < oc) ? asGlobal(kernel)[((size_t)a * rowWords + c) * oc + oo] : 0.0f;
-        if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
-        kern[e] = weight;
+    // weight of row a, tap-and-channel c (0 beyond the kernel) and this work-group's output channel `oo`
+    auto weightOf = [&](uint32_t a, uint32_t c, uint32_t oo) -> float {
+        const uint32_t tap = c / C.channels, channel = c - tap * C.channels;
+        return (c < taps && channel < (uint32_t)C.ic && oo < oc) ? asGlobal(kernel)[((size_t)(a * (uint32_t)C.kw + tap) * C.ic + channel) * oc + oo] : 0.0f;
+    };
+    bool special = false;
+    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * products * WAVE; e += AHEAD_CONV_THREADS) {
+        const uint32_t ap = e / WAVE, a = ap / products, first = (ap - a * products) * 16 + ((e & 32) ? 8 : 0), oo = blockIdx.z * 32 + (e & 31);
+        u32x4 top, middle, low;
+        #pragma unroll
+        for(uint32_t k = 0; k < 4; k++) {
+            float w0 = weightOf(a, first + 2 * k, oo), w1 = weightOf(a, first + 2 * k + 1, oo);
+            if(!aheadOrdinary(w0)) { special = true; w0 = 0.0f; }
+            if(!aheadOrdinary(w1)) { special = true; w1 = 0.0f; }
+            const float r0 = aheadRest(w0), r1 = aheadRest(w1);
+            top[k] = aheadTop(w0, w1);
+            middle[k] = aheadTop(r0, r1);
+            low[k] = aheadTop(aheadRest(r0), aheadRest(r1));
+        }
+        u32x4 *at = kern + (size_t)ap * 3 * WAVE + (e & (WAVE - 1));
+        at[0] = low; at[WAVE] = middle; at[2 * WAVE] = top;
     }
-    nonFinite = __syncthreads_or(nonFinite);
+    special = __syncthreads_or(special);
 
     GLOBAL_AS float *var0 = asGlobal(g.var0) + (size_t)batch * n, *var1 = asGlobal(g.var1) + (size_t)batch * n, *outPost = asGlobal(g.psm[0].outPost) + (size_t)batch * n;
     GLOBAL_AS uint32_t *spikes = asGlobal(spikeWords) + (size_t)batch * n;
-    for(uint32_t first = wave * 4; first < pixels; first += (BLOCK / WAVE) * 4) {
+    // (pairs of 16 bits; a row's entries start on a pair because the channels are even)
+    const uint32_t *pairs = reinterpret_cast<const uint32_t*>(patch + ((col & 16) ? plane : 0u));
+    for(uint32_t first = wave * 4; first < pixels; first += (AHEAD_CONV_THREADS / WAVE) * 4) {
         uint32_t base[4];
         #pragma unroll
         for(uint32_t j = 0; j < 4; j++) {
             const uint32_t p = min(first + j, pixels - 1), r = p / ow;
-            base[j] = r * rowPitch + (p - r * ow) * (uint32_t)C.ic + half;
+            base[j] = (r * rowPitch + (p - r * ow) * C.channels) / 2 + 4 * half;
         }
         // state of the lane's two neurons (pixels first + half and first + 2 + half, channel o), asked for before the products
         bool valid[2]; size_t at[2]; float v0[2], v1[2], lin[2];
@@ -385,44 +452,39 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
         f32x16 acc[4];
         #pragma unroll
         for(int j = 0; j < 4; j++) { acc[j] = f32x16{}; }
-        const float *weight = kern + half * 32 + col;
+        const u32x4 *weights = kern + lane;
         for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
-            // four pairs a round: their reads from LDS are issued together, ahead of the sixteen products
-            uint32_t c = 0;
-            for(; c + 4 <= pairs; c += 4) {
-                float b[4]; uint32_t bits[4][4];
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) {
-                    b[u] = weight[(c + u) * 64];
-                    #pragma unroll
-                    for(int j = 0; j < 4; j++) { bits[u][j] = patch[base[j] + 2 * (c + u)]; }
-                }
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) {
-                    #pragma unroll
-                    for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits[u][j], col), b[u], acc[j], 0, 0, 0); }
-                }
-            }
-            for(; c < pairs; c++) {
-                const float b = weight[c * 64];
-                #pragma unroll
-                for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(patch[base[j] + 2 * c], col), b, acc[j], 0, 0, 0); }
-            }
-            weight += pairs * 64;
-            #pragma unroll
-            for(int j = 0; j < 4; j++) { base[j] += rowPitch; }
-        }
-        if(nonFinite) {
-            // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
-            for(uint32_t k = 0; k < (uint32_t)C.kh * rowWords; k++) {
-                const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
-                if(aheadFinite(b)) { continue; }
-                const uint32_t a = k / rowWords;
+            for(uint32_t p = 0; p < products; p++) {
+                const bf16x8 low = __builtin_bit_cast(bf16x8, weights[0]), middle = __builtin_bit_cast(bf16x8, weights[WAVE]), top = __builtin_bit_cast(bf16x8, weights[2 * WAVE]);
+                weights += 3 * WAVE;
+                bf16x8 bits[4];
                 #pragma unroll
                 for(int j = 0; j < 4; j++) {
-                    const uint32_t bits = patch[base[j] - half - ((uint32_t)C.kh - a) * rowPitch + (k - a * rowWords)];
+                    const uint32_t *q = pairs + base[j] + 8 * p;
+                    bits[j] = aheadBits(u32x4{q[0], q[1], q[2], q[3]}, col & 15);
+                }
+                #pragma unroll
+                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], low, acc[j]); }
+                #pragma unroll
+                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], middle, acc[j]); }
+                #pragma unroll
+                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], top, acc[j]); }
+            }
+            #pragma unroll
+            for(int j = 0; j < 4; j++) { base[j] += rowPitch / 2; }
+        }
+        if(special) {
+            for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
+                for(uint32_t c = 0; c < taps; c++) {
+                    const float x = weightOf(a, c, o);
+                    if(aheadOrdinary(x)) { continue; }
                     #pragma unroll
-                    for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                    for(int j = 0; j < 4; j++) {
+                        const uint32_t e = 2 * (base[j] - 4 * half) - ((uint32_t)C.kh - a) * rowPitch + c;
+                        const uint32_t word = patch[e] | ((uint32_t)patch[plane + e] << 16);
+                        #pragma unroll
+                        for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((word >> aheadRow(v, half)) & 1u) ? x : 0.0f; }
+                    }
                 }
             }
         }

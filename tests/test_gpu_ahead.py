@@ -47,7 +47,7 @@ SHAPES = [("dense", (1, 1)), ("dense", (63, 31)), ("dense", (65, 33)), ("dense",
 @pytest.mark.parametrize("kind,shape", SHAPES, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
 def test_runs_of_every_length_mixed_with_single_steps(kind, shape):
     """Runs on either side of the shortest that is taken at once, of a word of 32 steps and of the longest launch of 128."""
-    chunks = [1, 3, 4, 1, 31, 32, 33, 2, 137, 0, 64]
+    chunks = [1, 4, 5, 1, 31, 32, 33, 2, 137, 0, 64]
     steps = sum(chunks)
     net = _net(kind, shape, steps)
     model = model_from_net(net)
@@ -160,3 +160,26 @@ def test_weights_that_are_not_finite_reach_their_own_spikes_only(kind, shape, mo
         model.unload()
     assert np.array_equal(vs[0][0], vs[1][0], equal_nan=True) and np.array_equal(vs[0][1], vs[1][1])
     assert np.isfinite(vs[0][0]).any()
+
+
+@pytest.mark.parametrize("kind,shape", [("dense", (200, 40)), ("conv", (6, 7, 2, 5, 3))])
+def test_weights_too_small_to_split(kind, shape, monkeypatch):
+    """Weights are split into three numbers of 8 bits for the matrix cores; below 2^-90 the lowest would underflow.  All weights are multiples
+    of 2^-107 here: a step's sum is exact, and outPost differs by its rounding in each of forty steps, of a sum of at most four times the
+    largest value left."""
+    steps = 40
+    net = _net(kind, shape, steps, psm="expcurr")
+    syn = net.syns[0]
+    syn.g = (syn.g * np.float32(2.0 ** -99)).astype(np.float32)
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        monkeypatch.setenv("GENNMI_CONV_MFMA", ahead)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        model.run(steps)
+        got.append(model.synapse_populations[syn.name].vars["outPost"].pull_from_device().astype(np.float64).copy())
+        model.unload()
+    assert np.abs(got[1]).max() > 0.0
+    assert np.abs(got[0] - got[1]).max() <= steps * 2.0 ** -24 * 4.0 * np.abs(got[1]).max()
