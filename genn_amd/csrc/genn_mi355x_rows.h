@@ -197,6 +197,47 @@ __device__ __forceinline__ uint32_t fixedProbabilityRow(uint32_t row, uint32_t n
     return total;
 }
 
+// A row of several rounds of 256 draws (see fixedNumberPostRow) whose spacings stay in registers between the total and the targets: the same
+// additions in the same order, so every bit of the result, without making each draw twice.  n < 256 * ROUNDS.
+template<int ROUNDS, typename Sink>
+__device__ __forceinline__ void fixedNumberPostRowKept(uint32_t row, uint32_t numPost, uint32_t n, const Stream &s, uint32_t lane, Sink sink)
+{
+    float spacing[ROUNDS][4];
+    double before[ROUNDS];
+    double carry = 0.0;
+    #pragma unroll
+    for(int round = 0; round < ROUNDS; round++) {
+        const uint32_t base = (uint32_t)round * 4 * WAVE, k = base + 4 * lane;
+        if(base <= n) {
+            const Words r = s.at(((unsigned long long)row << 32) | (k >> 2), 0);
+            double sum = 0.0;
+            #pragma unroll
+            for(int i = 0; i < 4; i++) {
+                spacing[round][i] = (k + i <= n) ? -logf(uniformOpen(r.w[i])) : 0.0f;
+                sum += (double)spacing[round][i];
+            }
+            const double inclusive = waveInclusiveScan(sum, (int)lane);
+            before[round] = carry + (inclusive - sum);
+            carry += __shfl(inclusive, WAVE - 1, WAVE);
+        }
+    }
+    const double scale = (double)numPost / carry;
+    #pragma unroll
+    for(int round = 0; round < ROUNDS; round++) {
+        const uint32_t k = (uint32_t)round * 4 * WAVE + 4 * lane;
+        if(k < n) {
+            uint32_t post[4];
+            double prefix = 0.0;
+            #pragma unroll
+            for(int i = 0; i < 4; i++) {
+                prefix += (double)spacing[round][i];
+                post[i] = min((uint32_t)((before[round] + prefix) * scale), numPost - 1);
+            }
+            sink(k, post);
+        }
+    }
+}
+
 // FixedNumberPostWithReplacement / FixedNumberTotalWithReplacement (:242-276, 292-370), one row of n targets by one wave64.
 // The snippet's loop `x += (1 - x) * (1 - pow(u, 1/c))` for c = n..1 draws the n order statistics of n uniforms in ascending
 // order.  The same joint law is S_k / S_{n+1} with S the prefix sums of n+1 unit exponentials, which a wave computes 256 draws at a

@@ -386,3 +386,19 @@ def test_network_initialised_on_the_device_runs():
     delivered = int((times < (steps - 1) * model.dt - 1e-6).sum()) * fan_out
     assert model.synaptic_event_count == delivered
     model.unload()
+
+
+@pytest.mark.parametrize("num", [1, 200, 255, 256, 511, 512, 1000, 1023, 1024, 2047])
+def test_fixed_number_post_draws_kept_or_made_twice_are_the_same(num):
+    """A row's targets depend on seed, stream and row alone: matrices whose longest row lets the kernel keep a row's draws in registers (1, 2, 4
+    or 8 rounds of 256) hold the same targets, bit for bit, as the same rows in a matrix too wide for that."""
+    lib = _abi.load()
+    _abi.check(lib.gennmi_init(0))
+    rows, num_post, got = 37, 123457, []
+    for stride in (num, 2048):
+        row_length, ind = _device_array(rows, np.uint32), _device_array(rows * stride, np.uint32)
+        _abi.check(lib.gennmi_init_sparse_fixed_number_post(rows, num_post, stride, num, None, 77, 5, row_length.ptr, ind.ptr, None))
+        assert np.all(row_length.pull_from_device() == num)
+        got.append(ind.pull_from_device().reshape(rows, stride)[:, :num].copy())
+        row_length.free(); ind.free()
+    assert np.array_equal(got[0], got[1]) and np.all(np.diff(got[0].astype(np.int64), axis=1) >= 0)
