@@ -91,9 +91,11 @@ struct gennmi_runner
     bool resident = false;
     ResTile *dResTiles = nullptr; NeuronGroupDev *dResGroups = nullptr; uint8_t *dResTileGroup = nullptr;
     unsigned long long *dResTags = nullptr, *dResSide = nullptr;
-    uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0; bool resPoisson = false;
+    uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0;
+    decltype(&residentKernel<false, false>) resKernel = nullptr;     // the instantiation its sources and segment entries need
     std::vector<u32x4*> resSegs;        // segment table of each presynaptic group, in push order
     std::vector<uint32_t> resSegTiles;  // tiles of its target population
+    std::vector<uint32_t> resSegWide;   // its entries are wide ones
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
@@ -772,13 +774,22 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     for(const auto &n : r->neuron) {
         for(uint32_t c = 0; c < n.g.numCS; c++) { poisson = poisson || n.g.cs[c].kind == GENNMI_CS_POISSON_EXP; }
     }
-    const void *kernel = poisson ? reinterpret_cast<const void*>(residentKernel<true>) : reinterpret_cast<const void*>(residentKernel<false>);
+    // Wide segment entries where a projection without a ring leaves a tile up to RES_WIDE_MEAN synapses of a row (rowStride is a little more than
+    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them.
+    constexpr uint32_t RES_WIDE_MEAN = 16;
+    auto wideEntries = [](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
+        const uint64_t mean = ((uint64_t)q.rowStride * RES_T + q.numTrgNeurons - 1) / q.numTrgNeurons;
+        return q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
+    };
+    bool anyWide = false;
+    for(const auto &p : r->pre) { anyWide = anyWide || wideEntries(p.g, (p.g.numTrgNeurons + RES_T - 1) / RES_T); }
+    const auto residentInstance = poisson ? (anyWide ? residentKernel<true, true> : residentKernel<true, false>) : (anyWide ? residentKernel<false, true> : residentKernel<false, false>);
+    const void *kernel = reinterpret_cast<const void*>(residentInstance);
     if(ldsBytes > 32 * 1024) {
         HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
     }
     int perCU = 0;
-    if(poisson) { HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentKernel<true>, BLOCK, ldsBytes)); }
-    else { HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentKernel<false>, BLOCK, ldsBytes)); }
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, BLOCK, ldsBytes));
     if((size_t)perCU * numCU < tiles.size()) { return GENNMI_OK; }
 
     // projections: source group, target group and postsynaptic model, segment table
@@ -827,12 +838,14 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         const size_t entries = (size_t)q.numSrcNeurons * tilesInGroup;
         if(q.rowStride > 0xFFFFu) { return GENNMI_OK; }         // a segment's length is a 16-bit field (device allocations made so far stay owned)
         u32x4 *dSeg = nullptr;
-        HIP_TRY(poolMalloc(&dSeg, entries * 2 * sizeof(u32x4)));
+        const uint32_t wide = wideEntries(q, tilesInGroup) ? 1u : 0u;
+        HIP_TRY(poolMalloc(&dSeg, entries * (wide ? RES_WIDE_QUADS : 2u) * sizeof(u32x4)));
         r->owned.push_back(dSeg);
         const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d,
-                                                                                                     depth, tilesInGroup, dSeg);
+                                                                                                     depth, tilesInGroup, wide, dSeg);
         r->resSegs.push_back(dSeg);
+        r->resSegWide.push_back(wide);
         r->resSegTiles.push_back(tilesInGroup);
         HIP_TRY(hipGetLastError());
         const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
@@ -848,7 +861,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         }
         r->resPacked.push_back(dPacked);
         ResProj proj{};
-        proj.packed = dPacked; proj.seg = dSeg;
+        proj.packed = dPacked; proj.seg = dSeg; proj.wide = wide;
         proj.D = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         proj.magic = proj.D ? (uint32_t)(0x100000000ull / proj.D) + 1u : 0u;
         proj.srcGroup = (uint32_t)l.src;
@@ -879,7 +892,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     HIP_TRY(hipMemset(r->dResSide, 0, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
     r->resTiles = (uint32_t)tiles.size();
     r->resLdsBytes = ldsBytes;
-    r->resPoisson = poisson;
+    r->resKernel = residentInstance;
     r->resident = true;
     return GENNMI_OK;
 }
@@ -905,7 +918,7 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
             const size_t entries = (size_t)q.numSrcNeurons * r->resSegTiles[k];
             const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
             residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(
-                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resSegTiles[k], r->resSegs[k]);
+                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resSegTiles[k], r->resSegWide[k], r->resSegs[k]);
             const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
             if(padded) {
                 residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(padded, q.ind, q.g, depth ? q.d : nullptr, r->resPacked[k]);
@@ -915,7 +928,7 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
     }
     for(unsigned long long done = 0; done < numSteps; ) {
         const uint32_t chunk = (uint32_t)std::min(MAX_STEPS, numSteps - done);
-        auto launch = r->resPoisson ? residentKernel<true> : residentKernel<false>;
+        const auto launch = r->resKernel;
         launch<<<dim3(r->resTiles), dim3(BLOCK), r->resLdsBytes, r->stream>>>(
             r->dResTiles, r->resTiles, r->dResGroups, r->dResTileGroup, r->dResTags, r->dResSide, timestep + done, r->epoch, numRecordingTimesteps,
             chunk, r->dt, r->fusedStep ? 1u : 0u, r->dError, r->dEvents, r->resReplicaStride, r->resSeq);

@@ -320,3 +320,38 @@ def test_expired_wait_is_reported_not_hung(resident, monkeypatch):
     model.run(100)
     model.synchronize()
     model.unload()
+
+
+@pytest.mark.parametrize("stride,crowded", [(2, 0.0), (5, 0.0), (14, 0.0), (30, 0.5), (30, 1.0), (90, 0.0)])
+def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypatch):
+    """Projections without a ring: a row's part in a tile is up to four synapses in an ordinary entry (stride 2), up to 24 in a wide one (5, 14),
+    longer than that (30 targets crowded into one tile, in some or in all rows) or walked as before (90).  Weights are pushed between
+    launches, so that the entries' copies of them are rebuilt.  (The tile path adds a step's sums, not its weights one by one: the single
+    steps in between go without it.)"""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
+    n_a, n_b = 700, 600
+    net = Net(name="resident_inline", dt=1.0, steps=0)
+    net.pops.append(_pop("A", n_a, 0.62, -60.0 + 9.5 * rng.uniform(5, 1, 0, n_a)))
+    net.pops.append(_pop("B", n_b, 0.45, -60.0 + 9.5 * rng.uniform(5, 2, 0, n_b)))
+    ab = _projection("AB", "A", "B", n_a, n_b, stride, 3.0 / stride, 21)
+    rows = rng.uniform(5, 3, 0, n_a) < crowded
+    ab.ind[rows] = np.sort(ab.ind[rows] % 250, axis=1)
+    ab.row_length[::7] = stride // 2                     # (some rows shorter, one in 49 empty)
+    ab.row_length[::49] = 0
+    net.syns.append(ab)
+    net.syns.append(_projection("BA", "B", "A", n_b, n_a, stride, -2.0 / stride, 22))
+    net.steps = 260
+    pushed = []
+
+    def check(model, oracle):
+        compare_state(net, model, oracle, "after a chunk", exact=True)
+        if not pushed:
+            pushed.append(True)
+            for s in net.syns:
+                g = model.synapse_populations[s.name].vars["g"]
+                g.view[:] = g.view * np.float32(0.5)
+                g.push_to_device()
+                oracle.syn_g(s.name)[:] *= np.float32(0.5)
+    model, oracle, spikes = _run_chunks(net, [100, -3, 97, 60], check)
+    assert spikes > 2000
+    model.unload()
