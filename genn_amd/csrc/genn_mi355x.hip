@@ -1495,11 +1495,24 @@ int gennmi_runner_finalise(gennmi_runner *r)
             return tileFloats != 0 && p.g.numSrcDelaySlots <= 1 && p.g.matrix == GENNMI_MATRIX_SPARSE && p.g.rowStride <= 65535
                    && (p.g.wum == GENNMI_WUM_STATIC_PULSE || p.g.wum == GENNMI_WUM_STDP_TRACE || p.g.wum == GENNMI_WUM_STDP);
         };
+        // Plastic projections keep, behind the tile, what the presynaptic-spike rule takes off a synapse of each of its targets and a bit per
+        // target (GENNMI_TILE_FACTORS = 0: never, 2: in every step): half the tile in the same LDS
+        const char *envFactors = getenv("GENNMI_TILE_FACTORS");
+        const uint32_t factorMode = envFactors ? (uint32_t)std::max(0, atoi(envFactors)) : 1u;
+        const uint32_t factorTile = (uint32_t)((uint64_t)tileFloats * 32 / 65) / 32 * 32;
+        // Only where there is more than one tile anyway and rows leave the smaller ones two dozen synapses: us a step without / with, neurons and
+        // targets a row of the plastic network: 100,000 x 500 22.2 / 21.0, 60,000 x 500 18.1 / 17.3, 40,000 x 300 14.7 / 14.2, 40,000 x 100
+        // 25.1 / 20.5; but 100,000 x 100, whose rows leave them ten, 30.0 / 32.4, and one tile cut in two (17,000 neurons) 11.5 / 11.8.
+        constexpr uint32_t FACTOR_SEGMENT = 24;
+        auto withFactors = [&](const PreGroupDev &p) {
+            if(factorMode == 0 || factorTile == 0 || p.g.wum == GENNMI_WUM_STATIC_PULSE) { return false; }
+            return factorMode == 2 || (p.g.numTrgNeurons > tileFloats && p.g.rowStride >= FACTOR_SEGMENT * ((p.g.numTrgNeurons + factorTile - 1) / factorTile));
+        };
         std::vector<TileOffsetsOf> offsets;
         std::vector<uint32_t> unsortedFlags;
         for(const auto &p : r->pre) {
             if(!tileCandidate(p)) { continue; }
-            const uint32_t tileSize = std::min(tileFloats, p.g.numTrgNeurons), numTiles = (p.g.numTrgNeurons + tileSize - 1) / tileSize;
+            const uint32_t tileSize = std::min(withFactors(p) ? factorTile : tileFloats, p.g.numTrgNeurons), numTiles = (p.g.numTrgNeurons + tileSize - 1) / tileSize;
             uint16_t *dOff = nullptr;
             HIP_TRY(poolMalloc(&dOff, (size_t)p.g.numSrcNeurons * (numTiles + 1) * sizeof(uint16_t)));
             r->owned.push_back(dOff);
@@ -1627,8 +1640,10 @@ int gennmi_runner_finalise(gennmi_runner *r)
                     t.records = records; t.recLanes = lanes; t.overflow = overflow;
                 }
             }
+            t.segLength = avgSeg;
+            t.factorEvents = withFactors(p) ? 1ull : 0ull;       // (the rule needs the number of splits: below)
             tileGroups.push_back(t);
-            r->tileFloats = std::max(r->tileFloats, tileSize);
+            r->tileFloats = std::max(r->tileFloats, withFactors(p) ? 2 * tileSize + (tileSize + 31) / 32 : tileSize);
         }
         if(!tileGroups.empty()) {
             // Every group gets a whole resident round of the chip (GENNMI_TILE_BLOCKS_PER_CU x 256 threads per compute
@@ -1649,6 +1664,8 @@ int gennmi_runner_finalise(gennmi_runner *r)
                 const uint32_t numSplits = std::max(1u, std::min(256u, groupBudget / t.numTiles));
                 t.numSplits = numSplits;
                 t.spikesPerSplit = spikesPerSplit;
+                // (worth it from one event per two targets of a block's tile)
+                if(t.factorEvents && factorMode == 1) { t.factorEvents = std::max(1ull, (unsigned long long)numSplits * t.tileSize / 2); }
                 for(uint32_t tile = 0; tile < t.numTiles; tile++) {
                     for(uint32_t split = 0; split < numSplits; split++) { t.tile = tile; t.split = split; tiles.push_back(t); }
                 }

@@ -118,6 +118,8 @@ struct TileGroupDev
     uint32_t lanes;                     // lanes per (spike, tile) segment, power of two
     uint32_t threshold;
     uint32_t spikesPerSplit;            // a step's spikes are shared between max(2, numSpikes / spikesPerSplit) of a tile's blocks (record path)
+    uint32_t segLength;                 // rowStride / numTiles
+    unsigned long long factorEvents;    // plastic: != 0: LDS behind the tile holds its targets' share of the rule in steps with numSpikes * segLength >= this
     uint32_t recLanes;                  // != 0: the projection has segment records (below), read by this many lanes each (5 or 10)
     const uint8_t *records;             // [numTiles][numSrc] records of 24 * recLanes + 8 bytes (128 or 256), or NULL
     const uint8_t *overflow;            // [numTiles][numSrc] 64-byte records of the 8 synapses that follow a full record, or NULL

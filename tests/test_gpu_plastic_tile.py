@@ -1,0 +1,51 @@
+"""The tile path of plastic projections with the presynaptic-spike rule's share worked out once per target in LDS
+(GENNMI_TILE_FACTORS: 0 never, 1 by the rule, 2 in every step that takes the tile path): the same operations on the same numbers, so
+weights must be the same bit for bit wherever the spikes are, and spikes those of the CPU oracle."""
+import numpy as np
+import pytest
+
+from genn_amd import configs
+from genn_amd.genn_model import model_from_net
+from oracle.genn_cpu import OracleNet
+
+pytestmark = pytest.mark.gpu
+
+
+# tiles: all targets in one; 9 of them with a remainder; one of 32 targets, the smallest with room for its bits
+@pytest.mark.parametrize("rule", ["stdp_trace", "stdp_additive"])
+@pytest.mark.parametrize("tile_floats,n", [("16384", 2500), ("512", 2501), ("66", 300)])
+def test_weights_are_the_same_with_and_without(rule, tile_floats, n, monkeypatch):
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", tile_floats)
+    monkeypatch.setenv("GENNMI_TILE_THREADS", "512")
+    steps = 60
+    # strong drive: bursts in which sources and targets of a synapse fire together, so both rules meet on it
+    net = configs.plastic_stdp(n=n, n_src=100, steps=steps, fan=n // 10, src_fan=50, src_w=6.0, ioffset=0.6, rule=rule)
+    ee = next(s for s in net.syns if s.name == "EE")
+    ee.g = np.array(ee.g)
+    ee.g[::5] = 1.75             # beyond wMax: a synapse that neither rule touches keeps it, one that is touched is clipped
+    got = []
+    for factors in ("0", "1", "2"):
+        monkeypatch.setenv("GENNMI_TILE_FACTORS", factors)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        for _ in range(steps):
+            model.step_time()
+        model.pull_recording_buffers_from_device()
+        got.append((model.synapse_populations["EE"].vars["g"].pull_from_device().copy(), {p.name: model.neuron_populations[p.name].vars["recordSpk"].view.copy() for p in net.pops}))
+        col_stride = model.synapse_populations["EE"].col_stride
+        model.unload()
+    oracle = OracleNet(net, num_recording_timesteps=steps, col_stride={"EE": col_stride})
+    oracle.run(steps)
+    spikes = 0
+    for p in net.pops:
+        want = oracle.record(p.name, steps)
+        for g, raster in got:
+            assert np.array_equal(raster[p.name].reshape(-1), want.reshape(-1)), p.name
+        spikes += int(np.unpackbits(want.view(np.uint8)).sum())
+    assert spikes > 2 * n
+    valid = (np.arange(ee.ind.shape[1])[None, :] < np.asarray(ee.row_length)[:, None]).reshape(-1)
+    want = oracle.syn_g("EE").reshape(-1)[valid]
+    for g, raster in got:
+        assert np.array_equal(g.reshape(-1)[valid], got[0][0].reshape(-1)[valid])
+        assert np.abs(g.reshape(-1)[valid] - want).max() <= 1e-5
+    assert (np.abs(want - np.asarray(ee.g).reshape(-1)[valid]) > 1e-3).mean() > 0.5
