@@ -1266,7 +1266,7 @@ static int setupAhead(gennmi_runner *r, uint32_t numCU)
     return GENNMI_OK;
 }
 
-// the next numSteps (up to AHEAD_MAX_STEPS) steps; `done` receives how many it took
+// the next numSteps (up to AHEAD_MAX_STEPS) steps; `done` receives how many it took: none when there is no memory for its workspace
 static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned long long numSteps, unsigned long long numRecordingTimesteps, uint32_t *done)
 {
     const gennmi_presynaptic_update_group_t &p = r->aheadLayer;
@@ -1294,13 +1294,18 @@ static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned l
         HIP_TRY(hipStreamSynchronize(r->stream));
         HIP_TRY(poolFree(r->aheadSpace));
         r->aheadSpace = nullptr; r->aheadSpaceBytes = 0;
-        HIP_TRY(poolMalloc((void**)&r->aheadSpace, need));
+        *done = 0;
+        if(poolMalloc((void**)&r->aheadSpace, need) != hipSuccess) {
+            (void)hipGetLastError();
+            r->aheadSpace = nullptr;
+            return GENNMI_OK;
+        }
         r->aheadSpaceBytes = need;
     }
     uint32_t *words = reinterpret_cast<uint32_t*>(r->aheadSpace), *targetBits = reinterpret_cast<uint32_t*>(r->aheadSpace + wordBytes);
     uint8_t *input = r->aheadSpace + wordBytes + bitBytes;
     const NeuronGroupDev *target = r->dAhead + 1, &src = r->neuron[r->aheadSource];
-    const AheadArgs a{timestep, r->epoch, steps, B, (uint32_t)std::max<unsigned long long>(1, std::min<unsigned long long>(numRecordingTimesteps, 0xFFFFFFFFull)), r->dt};
+    const AheadArgs a{timestep, r->epoch, steps, B, (uint32_t)std::max<unsigned long long>(1, numRecordingTimesteps), r->dt};
     // (the kernels of the target's neuron model and postsynaptic model)
     const gennmi_neuron_update_group_t &g = r->neuron[r->aheadTarget].g;
     const bool lif = (g.model == GENNMI_NEURON_LIF), exponential = (g.psm[0].kind == GENNMI_PSM_EXPCURR);
@@ -2200,10 +2205,11 @@ int gennmi_run_steps(gennmi_runner *r, unsigned long long timestep, unsigned lon
     { const int rc = refreshTables(r); if(rc) { return rc; } }
     if(r->resident && !r->timing && numSteps >= 4) { return launchResident(r, timestep, numSteps, numRecordingTimesteps); }
     unsigned long long done = 0;
-    while(r->ahead && !r->timing && numSteps - done >= AHEAD_MIN_STEPS) {
+    while(r->ahead && !r->timing && numSteps - done >= AHEAD_MIN_STEPS && numRecordingTimesteps <= 0xFFFFFFFFull) {
         uint32_t taken = 0;
         const int rc = launchAhead(r, timestep + done, numSteps - done, numRecordingTimesteps, &taken);
         if(rc) { return rc; }
+        if(!taken) { break; }
         done += taken;
     }
     // Every (other) step is launched as gennmi_step_time() launches it: time, epoch and recording row are kernel arguments.  (Measured
