@@ -85,6 +85,7 @@ struct gennmi_runner
     gennmi_presynaptic_update_group_t aheadLayer{}; AheadConv aheadConv{}; size_t aheadConvBytes = 0; uint32_t aheadCU = 1;
     NeuronGroupDev *dAhead = nullptr; uint32_t aheadSource = 0, aheadTarget = 0;     // descriptors of source and target; their indices in `neuron`
     uint8_t *aheadSpace = nullptr; size_t aheadSpaceBytes = 0;                          // workspace, made by the first run that needs it
+    bool queueWritten = false;          // ... its neuron indices, since the last run()
     bool bitmapsStale = false;          // a spike queue was written by the caller: the bitmaps kept beside the queues are rebuilt before the next step
     std::vector<void*> owned;           // engine-private device allocations (shadow queues, zero-delay lists)
     // resident plan (many steps per launch)
@@ -145,10 +146,12 @@ static void noteDeviceWrite(const void *dev, size_t bytes)
     const uintptr_t a = reinterpret_cast<uintptr_t>(dev), b = a + bytes;
     for(gennmi_runner *r : g_runners) {
         for(const auto &n : r->neuron) {
-            if(n.spikeBitmap && !r->bitmapsStale) {
+            if(n.spikeBitmap && !(r->bitmapsStale && r->queueWritten)) {
                 const uintptr_t q = reinterpret_cast<uintptr_t>(n.g.spk), c = reinterpret_cast<uintptr_t>(n.g.spkCnt);
                 const size_t slots = std::max(1u, n.g.numDelaySlots);
-                if((a < q + (size_t)r->batch * slots * n.g.numNeurons * sizeof(uint32_t) && q < b) || (a < c + (size_t)r->batch * slots * sizeof(uint32_t) && c < b)) { r->bitmapsStale = true; }
+                const bool ids = a < q + (size_t)r->batch * slots * n.g.numNeurons * sizeof(uint32_t) && q < b;
+                if(ids || (a < c + (size_t)r->batch * slots * sizeof(uint32_t) && c < b)) { r->bitmapsStale = true; }
+                if(ids) { r->queueWritten = true; }
             }
             if(n.g.model != GENNMI_NEURON_SPIKE_SOURCE_ARRAY || r->sourcesStale) { continue; }
             const size_t perNeuron = (size_t)r->batch * n.g.numNeurons * sizeof(uint32_t);
@@ -1209,12 +1212,12 @@ static int refreshTables(gennmi_runner *r)
 // Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
 // plain population it feeds, so that no spike ever comes back.
 constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input over the steps of a launch
-constexpr size_t AHEAD_MAX_LDS = 156 * 1024;           // of a compute unit's 160 KB; two work-groups share it where they can
-// Runs (and remainders of runs) shorter than this are stepped one by one: a pass costs nearly as much for 2 steps as for 32.  us at once / one
-// by one for 4 and for 8 steps (5 % activity; a twenty-fifth of it in brackets): DENSE 8192 x 8192 35 / 45, 43 / 85 [28 / 44, 31 / 84], the same
-// with batch 16 195 / 175, 231 / 346 [104 / 167, 109 / 330], 8192 x 10 23 / 40, 25 / 74; Conv2D 64x64x16 -> 64x64x32 3x3, batch 16 94 / 132,
-// 100 / 257, 16x16x1 -> 16x16x4 24 / 68, 24 / 130.
-constexpr uint32_t AHEAD_MIN_STEPS = 5;
+constexpr size_t AHEAD_MAX_LDS = 64 * 1024;
+// Runs (and remainders of runs) shorter than this are stepped one by one: a pass costs a good part of a pass of 32 steps however few it is given.  us
+// at once / one by one for 5 and for 8 steps: Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, at 20 %, 2.5 % and 0.25 % activity 239 / 174 and
+// 259 / 273, 125 / 152 and 144 / 238, 93 / 146 and 98 / 228; 40x40x16 -> 40x40x4 5x5, batch 16, at 0.25 % 185 / 131 and 189 / 204; DENSE 8192 x 8192
+// (5 %; 4 and 8 steps) 35 / 45 and 43 / 85, the same with batch 16 195 / 175 and 231 / 346.
+constexpr uint32_t AHEAD_MIN_STEPS = 8;
 static int setupAhead(gennmi_runner *r, uint32_t numCU)
 {
     const char *env = getenv("GENNMI_AHEAD");
@@ -1232,24 +1235,17 @@ static int setupAhead(gennmi_runner *r, uint32_t numCU)
     if(conv) {
         const int32_t *c = p.conv;
         AheadConv &C = r->aheadConv;
-        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 0u, 0u, 1u};
-        C.channels = ((uint32_t)c[4] + 1) / 2 * 2;
-        C.rowTaps = ((uint32_t)c[1] * C.channels + 15) / 16 * 16;
-        C.rowPitch = (uint32_t)(c[6] - 1) * C.channels + C.rowTaps;
-        // as many output rows per work-group as leave two work-groups to a compute unit
+        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 0u, 1u};
+        C.rowPitch = (uint32_t)(c[6] - 1 + c[1]) * (uint32_t)c[4] + 1;      // (an odd number of taps is read as pairs: one word beyond)
+        C.pairsPerRow = ((uint32_t)(c[1] * c[4]) + 1) / 2;
+        // as many output rows per work-group as leave four work-groups to a compute unit
         const uint64_t rowsInAll = (uint64_t)c[5] * r->batch * (((uint32_t)c[7] + 31) / 32);
-        C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (2 * numCU)));
+        C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (4 * numCU)));
         for(;; C.rowsPerBlock--) {
-            r->aheadConvBytes = (size_t)c[0] * (C.rowTaps / 16) * 3 * WAVE * sizeof(u32x4) + (size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch * 2 * sizeof(uint16_t);
-            if(r->aheadConvBytes <= AHEAD_MAX_LDS / 2 || C.rowsPerBlock == 1) { break; }
+            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)c[0] * 2 * C.pairsPerRow * 32) * sizeof(uint32_t);
+            if(r->aheadConvBytes <= AHEAD_MAX_LDS || C.rowsPerBlock == 1) { break; }
         }
         if(r->aheadConvBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
-        if(r->aheadConvBytes > 48 * 1024) {
-            for(const void *k : {(const void*)aheadConvKernel<GENNMI_NEURON_LIF, GENNMI_PSM_EXPCURR>, (const void*)aheadConvKernel<GENNMI_NEURON_LIF, GENNMI_PSM_DELTACURR>,
-                                 (const void*)aheadConvKernel<GENNMI_NEURON_IZHIKEVICH, GENNMI_PSM_EXPCURR>, (const void*)aheadConvKernel<GENNMI_NEURON_IZHIKEVICH, GENNMI_PSM_DELTACURR>}) {
-                HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)AHEAD_MAX_LDS));
-            }
-        }
     }
     else if((size_t)r->batch * AHEAD_WORD * p.numTrgNeurons * sizeof(float) > AHEAD_MAX_SPACE || (uint64_t)r->batch * (AHEAD_MAX_STEPS / AHEAD_WORD) > 65535) { return GENNMI_OK; }
     if(!src.spikeBitmap) {
@@ -1317,7 +1313,7 @@ static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned l
         const AheadConv &C = r->aheadConv;
         uint32_t *spikes = reinterpret_cast<uint32_t*>(input);
         for(uint32_t k = 0; k < blocks; k++) {
-            convKernel<<<dim3(((uint32_t)C.oh + C.rowsPerBlock - 1) / C.rowsPerBlock, B, ((uint32_t)C.oc + 31) / 32), dim3(AHEAD_CONV_THREADS), r->aheadConvBytes, r->stream>>>(
+            convKernel<<<dim3(((uint32_t)C.oh + C.rowsPerBlock - 1) / C.rowsPerBlock, B, ((uint32_t)C.oc + 31) / 32), dim3(BLOCK), r->aheadConvBytes, r->stream>>>(
                 target, a, C, k, words, p.g, spikes);
             if(g.recordSpk || k + 1 == blocks) {
                 aheadTransposeKernel<<<dim3((numTrg + 1023) / 1024, B), dim3(BLOCK), 0, r->stream>>>(target, a, k, spikes, targetBits);
@@ -2205,6 +2201,18 @@ int gennmi_run_steps(gennmi_runner *r, unsigned long long timestep, unsigned lon
     { const int rc = refreshTables(r); if(rc) { return rc; } }
     if(r->resident && !r->timing && numSteps >= 4) { return launchResident(r, timestep, numSteps, numRecordingTimesteps); }
     unsigned long long done = 0;
+    bool queueWritten;
+    {
+        std::lock_guard<std::mutex> lock(g_runnersMutex);
+        queueWritten = r->queueWritten;
+        r->queueWritten = false;
+    }
+    if(r->ahead && queueWritten && numSteps) {
+        // (a queue the caller wrote may name a neuron twice, which the step's kernels deliver twice and a bit cannot say)
+        const int rc = stepNow(r, (float)timestep * r->dt, numRecordingTimesteps ? (uint32_t)(timestep % numRecordingTimesteps) : 0u);
+        if(rc) { return rc; }
+        done = 1;
+    }
     while(r->ahead && !r->timing && numSteps - done >= AHEAD_MIN_STEPS && numRecordingTimesteps <= 0xFFFFFFFFull) {
         uint32_t taken = 0;
         const int rc = launchAhead(r, timestep + done, numSteps - done, numRecordingTimesteps, &taken);

@@ -8,13 +8,13 @@
 //   1. aheadSourceKernel: a lane walks one source neuron's spikes of all these steps.  Its input to the layer is one 32-bit word per
 //      32 steps (bit j: the layer receives a spike from it in step j).
 //   2. the layer's input of 32 steps is a matrix product whose left operand is those bits: rows are timesteps, the inner
-//      dimension the source neurons (DENSE) or an output pixel's taps (Conv2D), columns the target neurons.  See aheadProduct.
+//      dimension the source neurons (DENSE) or an output pixel's taps (Conv2D), columns the target neurons.
 //   3. the neurons: a lane takes one neuron through the steps with its state in registers.
 //   4. aheadQueueKernel: the spike queues as the last step leaves them, in ascending neuron index.
 // What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
 //
 // run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 205 us;
-// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 850 us, of which 500 move 26 MB between host and device.
+// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 1040 us, of which 500 move 26 MB between host and device.
 #pragma once
 
 namespace
@@ -32,9 +32,7 @@ struct AheadArgs
 struct AheadConv
 {
     int32_t kh, kw, ih, iw, ic, oh, ow, oc, PH, PW;
-    uint32_t rowsPerBlock;
-    uint32_t channels;                  // input channels, made even
-    uint32_t rowPitch, rowTaps;         // patch row and (tap, channel) pairs of one kernel row, the latter filled up to whole products of 16
+    uint32_t rowsPerBlock, rowPitch, pairsPerRow;       // patch row in words; (tap, channel) pairs of one kernel row
     uint32_t isConv;
 };
 
@@ -124,7 +122,7 @@ void aheadSourceKernel(const NeuronGroupDev * __restrict__ source, AheadArgs A, 
     if(lane == 0 && events) { addEvents(eventCounter, events); }
 }
 
-// The product of 32 steps' bits and 32 columns of weights for 16 sources (or taps): v_mfma_f32_32x32x16_bf16 three times.  A bit is 0 or 1, and an
+// DENSE: the product of 32 steps' bits and 32 columns of weights for 16 sources: v_mfma_f32_32x32x16_bf16 three times.  A bit is 0 or 1, and an
 // fp32 weight is exactly the sum of three bfloat16 numbers of 8 significant bits each, so every product is exact, as it is with the fp32
 // instruction (v_mfma_f32_32x32x2_f32), which takes eight times 64 clocks for what these three do in 32 each; sums are fp32 either way
 // and are rounded less often.  That split needs the lowest of the three to be a normal number and the weight to be finite: weights that are
@@ -147,6 +145,8 @@ __device__ __forceinline__ bf16x8 aheadBits(u32x4 words, uint32_t row)
     return __builtin_bit_cast(bf16x8, operand);
 }
 __device__ __forceinline__ f32x16 aheadProduct(bf16x8 bits, bf16x8 weights, f32x16 sum) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(bits, weights, sum, 0, 0, 0); }
+__device__ __forceinline__ float aheadBit(uint32_t word, uint32_t row) { return (float)((word >> row) & 1u); }
+__device__ __forceinline__ bool aheadFinite(float w) { return (__float_as_uint(w) & 0x7F800000u) != 0x7F800000u; }
 // the accumulator's element v of a lane in the given half is timestep ...
 __device__ __forceinline__ uint32_t aheadRow(uint32_t v, uint32_t half) { return 8 * (v / 4) + 4 * half + (v % 4); }
 
@@ -367,80 +367,108 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
 }
 
 // ---- 2b, 3b. Conv2D and its neurons, up to 32 steps.  A work-group owns some output rows of one batch and 32 output channels: the
-// words of the input pixels they reach (zero outside the input) and the kernel, split, wait in LDS.  A wavefront takes four output pixels at a
+// words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes four output pixels at a
 // time: the rows of its four products are timesteps, the inner dimension the (tap, channel) pairs — consecutive words of the patch
-// for one kernel row, filled up to whole products of 16 with zero weights — and a kernel weight read once serves all four.  The products
-// stay in registers; one swap of half-wavefronts per register pair puts a neuron's 32 inputs into one lane, which takes the neuron
-// through the steps and leaves its spikes as one word.  Bound by instruction issue: 64x64x16 -> 64x64x32 3x3, batch 16 takes 94 us for
-// 32 steps, of which the products are 23 at the matrix rate, and 74 for 18 steps (229 and 201 with v_mfma_f32_32x32x2_f32, the matrix rate's
-// 123 bounding it).
-constexpr uint32_t AHEAD_CONV_THREADS = 512;
+// for one kernel row — and a kernel weight read once serves all four.  The products stay in registers; one swap of half-wavefronts
+// per register pair puts a neuron's 32 inputs into one lane, which takes the neuron through the steps and leaves its spikes as one word.
+// The products are those of the step kernel, v_mfma_f32_32x32x2_f32 over taps and channels in the same order, so that a layer's sums are the
+// same bits whether its steps are taken at once or one by one (with weights in three bfloat16 parts, as in aheadDenseKernel, the kernel
+// takes 88 us instead of 204 and one spike in 10^6 moves by a step).  Bound by the fp32 matrix rate: 64x64x16 -> 64x64x32 3x3, batch 16 takes
+// 204 us for 32 steps and 154 for 18; at that rate the products take 123 without the silent pairs left out.
 template<uint32_t MODEL, uint32_t PSM>
-__global__ __launch_bounds__(AHEAD_CONV_THREADS, 4)
+__global__ __launch_bounds__(BLOCK, 4)
 void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
                      const float * __restrict__ kernel, uint32_t *spikeWords)
 {
-    extern __shared__ __align__(16) uint32_t shAhead[];
+    extern __shared__ uint32_t shAhead[];
     const gennmi_neuron_update_group_t &g = target->g;
     const uint32_t n = g.numNeurons, batch = blockIdx.y, oc = (uint32_t)C.oc, ow = (uint32_t)C.ow;
-    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), half = lane >> 5, col = lane & 31;
     const uint32_t y0 = blockIdx.x * C.rowsPerBlock, rows = min(C.rowsPerBlock, (uint32_t)C.oh - y0), pixels = rows * ow;
     const uint32_t o = blockIdx.z * 32 + col;
     const uint32_t steps = min(A.steps - wordBlock * AHEAD_WORD, AHEAD_WORD);
     const AheadNeuron<MODEL, PSM> neuron(g, A.dt);
-    const uint32_t rowPitch = C.rowPitch, taps = (uint32_t)C.kw * C.channels, products = C.rowTaps / 16;
-    // the kernel: [kh][products][piece][half][32 columns] of 8 bfloat16 each (16 bytes a lane, lane-consecutive)
-    u32x4 *kern = reinterpret_cast<u32x4*>(shAhead);
-    // the patch: lower halves of the words, then upper halves, [rows + kh - 1][rowPitch] of 16 bits each
-    const uint32_t plane = (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch;
-    uint16_t *patch = reinterpret_cast<uint16_t*>(kern + (size_t)C.kh * products * 3 * WAVE);
+    const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), pairs = C.pairsPerRow;
+    uint32_t *patch = shAhead;
+    float *kern = reinterpret_cast<float*>(shAhead + (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch);        // [kh][2 * pairs][32]
+    // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
     GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
+    const int inRowWords = C.iw * C.ic;
     for(uint32_t r = 0; r < rows + (uint32_t)C.kh - 1; r++) {
         const int y = (int)(y0 + r) - C.PH;
-        for(uint32_t e = threadIdx.x; e < rowPitch; e += AHEAD_CONV_THREADS) {
-            const uint32_t column = e / C.channels, channel = e - column * C.channels;
-            const int x = (int)column - C.PW;
-            const uint32_t word = (y >= 0 && y < C.ih && x >= 0 && x < C.iw && channel < (uint32_t)C.ic) ? in[((size_t)y * C.iw + x) * C.ic + channel] : 0u;
-            patch[r * rowPitch + e] = (uint16_t)word;
-            patch[plane + r * rowPitch + e] = (uint16_t)(word >> 16);
+        for(uint32_t e = threadIdx.x; e < rowPitch; e += BLOCK) {
+            const int x = (int)e - C.PW * C.ic;
+            patch[r * rowPitch + e] = (y >= 0 && y < C.ih && x >= 0 && x < inRowWords) ? in[(size_t)y * inRowWords + x] : 0u;
         }
     }
-    // weight of row a, tap-and-channel c (0 beyond the kernel) and this work-group's output channel `oo`
-    auto weightOf = [&](uint32_t a, uint32_t c, uint32_t oo) -> float {
-        const uint32_t tap = c / C.channels, channel = c - tap * C.channels;
-        return (c < taps && channel < (uint32_t)C.ic && oo < oc) ? asGlobal(kernel)[((size_t)(a * (uint32_t)C.kw + tap) * C.ic + channel) * oc + oo] : 0.0f;
-    };
-    bool special = false;
-    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * products * WAVE; e += AHEAD_CONV_THREADS) {
-        const uint32_t ap = e / WAVE, a = ap / products, first = (ap - a * products) * 16 + ((e & 32) ? 8 : 0), oo = blockIdx.z * 32 + (e & 31);
-        u32x4 top, middle, low;
-        #pragma unroll
-        for(uint32_t k = 0; k < 4; k++) {
-            float w0 = weightOf(a, first + 2 * k, oo), w1 = weightOf(a, first + 2 * k + 1, oo);
-            if(!aheadOrdinary(w0)) { special = true; w0 = 0.0f; }
-            if(!aheadOrdinary(w1)) { special = true; w1 = 0.0f; }
-            const float r0 = aheadRest(w0), r1 = aheadRest(w1);
-            top[k] = aheadTop(w0, w1);
-            middle[k] = aheadTop(r0, r1);
-            low[k] = aheadTop(aheadRest(r0), aheadRest(r1));
-        }
-        u32x4 *at = kern + (size_t)ap * 3 * WAVE + (e & (WAVE - 1));
-        at[0] = low; at[WAVE] = middle; at[2 * WAVE] = top;
+    bool nonFinite = false;
+    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * 2 * pairs * 32; e += BLOCK) {
+        const uint32_t k = e / 32, a = k / (2 * pairs), c = k - a * 2 * pairs, oo = blockIdx.z * 32 + (e & 31);
+        float weight = (c < rowWords && oo < oc) ? asGlobal(kernel)[((size_t)a * rowWords + c) * oc + oo] : 0.0f;
+        if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
+        kern[e] = weight;
     }
-    special = __syncthreads_or(special);
+    nonFinite = __syncthreads_or(nonFinite);
+    const uint32_t *patchOfHalf = patch + half;
 
     GLOBAL_AS float *var0 = asGlobal(g.var0) + (size_t)batch * n, *var1 = asGlobal(g.var1) + (size_t)batch * n, *outPost = asGlobal(g.psm[0].outPost) + (size_t)batch * n;
     GLOBAL_AS uint32_t *spikes = asGlobal(spikeWords) + (size_t)batch * n;
-    // (pairs of 16 bits; a row's entries start on a pair because the channels are even)
-    const uint32_t *pairs = reinterpret_cast<const uint32_t*>(patch + ((col & 16) ? plane : 0u));
-    for(uint32_t first = wave * 4; first < pixels; first += (AHEAD_CONV_THREADS / WAVE) * 4) {
+    for(uint32_t first = wave * 4; first < pixels; first += (BLOCK / WAVE) * 4) {
         uint32_t base[4];
         #pragma unroll
         for(uint32_t j = 0; j < 4; j++) {
             const uint32_t p = min(first + j, pixels - 1), r = p / ow;
-            base[j] = (r * rowPitch + (p - r * ow) * C.channels) / 2 + 4 * half;
+            base[j] = r * rowPitch + (p - r * ow) * (uint32_t)C.ic;
         }
-        // state of the lane's two neurons (pixels first + half and first + 2 + half, channel o), asked for before the products
+        f32x16 acc[4];
+        #pragma unroll
+        for(int j = 0; j < 4; j++) { acc[j] = f32x16{}; }
+        const float *weight = kern + half * 32 + col;
+        for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
+            // four pairs a round: their reads from LDS are issued together, ahead of the sixteen products
+            uint32_t c = 0;
+            for(; c + 4 <= pairs; c += 4) {
+                float b[4]; uint32_t bits[4][4];
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) {
+                    b[u] = weight[(c + u) * 64];
+                    #pragma unroll
+                    for(int j = 0; j < 4; j++) { bits[u][j] = patchOfHalf[base[j] + 2 * (c + u)]; }
+                }
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) {
+                    #pragma unroll
+                    for(int j = 0; j < 4; j++) {
+                        // (two inputs silent in all steps add nothing: a fifth of the pairs at 2.5 % and 32 steps, two fifths at 18)
+                        if(__ballot(bits[u][j] != 0)) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits[u][j], col), b[u], acc[j], 0, 0, 0); }
+                    }
+                }
+            }
+            for(; c < pairs; c++) {
+                const float b = weight[c * 64];
+                #pragma unroll
+                for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(patchOfHalf[base[j] + 2 * c], col), b, acc[j], 0, 0, 0); }
+            }
+            weight += pairs * 64;
+            #pragma unroll
+            for(int j = 0; j < 4; j++) { base[j] += rowPitch; }
+        }
+        if(nonFinite) {
+            // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
+            for(uint32_t k = 0; k < (uint32_t)C.kh * rowWords; k++) {
+                const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
+                if(aheadFinite(b)) { continue; }
+                const uint32_t a = k / rowWords;
+                #pragma unroll
+                for(int j = 0; j < 4; j++) {
+                    const uint32_t bits = patch[base[j] - ((uint32_t)C.kh - a) * rowPitch + (k - a * rowWords)];
+                    #pragma unroll
+                    for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                }
+            }
+        }
+        // state of the lane's two neurons (pixels first + half and first + 2 + half, channel o), asked for behind the products: held across them, it and its addresses do not fit
+        // the registers
         bool valid[2]; size_t at[2]; float v0[2], v1[2], lin[2];
         #pragma unroll
         for(uint32_t m = 0; m < 2; m++) {
@@ -448,45 +476,6 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
             valid[m] = (p < pixels && o < oc);
             at[m] = valid[m] ? ((size_t)y0 * ow + p) * oc + o : 0;
             v0[m] = var0[at[m]]; v1[m] = var1[at[m]]; lin[m] = outPost[at[m]];
-        }
-        f32x16 acc[4];
-        #pragma unroll
-        for(int j = 0; j < 4; j++) { acc[j] = f32x16{}; }
-        const u32x4 *weights = kern + lane;
-        for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
-            for(uint32_t p = 0; p < products; p++) {
-                const bf16x8 low = __builtin_bit_cast(bf16x8, weights[0]), middle = __builtin_bit_cast(bf16x8, weights[WAVE]), top = __builtin_bit_cast(bf16x8, weights[2 * WAVE]);
-                weights += 3 * WAVE;
-                bf16x8 bits[4];
-                #pragma unroll
-                for(int j = 0; j < 4; j++) {
-                    const uint32_t *q = pairs + base[j] + 8 * p;
-                    bits[j] = aheadBits(u32x4{q[0], q[1], q[2], q[3]}, col & 15);
-                }
-                #pragma unroll
-                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], low, acc[j]); }
-                #pragma unroll
-                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], middle, acc[j]); }
-                #pragma unroll
-                for(int j = 0; j < 4; j++) { acc[j] = aheadProduct(bits[j], top, acc[j]); }
-            }
-            #pragma unroll
-            for(int j = 0; j < 4; j++) { base[j] += rowPitch / 2; }
-        }
-        if(special) {
-            for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
-                for(uint32_t c = 0; c < taps; c++) {
-                    const float x = weightOf(a, c, o);
-                    if(aheadOrdinary(x)) { continue; }
-                    #pragma unroll
-                    for(int j = 0; j < 4; j++) {
-                        const uint32_t e = 2 * (base[j] - 4 * half) - ((uint32_t)C.kh - a) * rowPitch + c;
-                        const uint32_t word = patch[e] | ((uint32_t)patch[plane + e] << 16);
-                        #pragma unroll
-                        for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((word >> aheadRow(v, half)) & 1u) ? x : 0.0f; }
-                    }
-                }
-            }
         }
         #pragma unroll
         for(int m = 0; m < 2; m++) {

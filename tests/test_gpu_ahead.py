@@ -47,7 +47,7 @@ SHAPES = [("dense", (1, 1)), ("dense", (63, 31)), ("dense", (65, 33)), ("dense",
 @pytest.mark.parametrize("kind,shape", SHAPES, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
 def test_runs_of_every_length_mixed_with_single_steps(kind, shape):
     """Runs on either side of the shortest that is taken at once, of a word of 32 steps and of the longest launch of 128."""
-    chunks = [1, 4, 5, 1, 31, 32, 33, 2, 137, 0, 64]
+    chunks = [1, 7, 8, 1, 31, 32, 33, 2, 137, 0, 64]
     steps = sum(chunks)
     net = _net(kind, shape, steps)
     model = model_from_net(net)
@@ -183,3 +183,23 @@ def test_weights_too_small_to_split(kind, shape, monkeypatch):
         model.unload()
     assert np.abs(got[1]).max() > 0.0
     assert np.abs(got[0] - got[1]).max() <= steps * 2.0 ** -24 * 4.0 * np.abs(got[1]).max()
+
+
+def test_a_written_queue_that_names_a_neuron_twice(monkeypatch):
+    """The DENSE kernel of a single step walks the queue as it is: so does the first step of a run."""
+    steps = 20
+    net = _net("dense", (90, 40), steps)
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        source = model.neuron_populations["In"]
+        source.vars["spk"].view[:3] = [7, 7, 60]
+        source.vars["spkCnt"].view[:] = 3
+        for v in ("spk", "spkCnt"):
+            source.vars[v].push_to_device()
+        model.run(steps)
+        got.append((model.neuron_populations["Out"].vars["V"].pull_from_device().copy(), model.synaptic_event_count))
+        model.unload()
+    assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
