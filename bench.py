@@ -38,9 +38,9 @@ BYTES_PER_EVENT = {"dense": 4,          # one weight read per (spike, target); o
 # its seed and therefore its activity are then identical); any other run reports null.
 # The kernel's source is named with a digest: a figure measured on another version of the kernel is not attached.
 MEASURED_TRAFFIC_BYTES = {
-    ("potjans", 20, 5): {"plan": "resident", "bytes_per_launch": 155216672,
-                         "kernel_source": ("genn_amd/csrc/genn_mi355x_resident_kernels.h", "861e3def22045d8a"),
-                         "source": "rocprofv3 --pmc FETCH_SIZE (67692.56 x 2 KiB) + WRITE_SIZE (16193.66 x 1 KiB) of the timed 20-step "
+    ("potjans", 20, 5): {"plan": "resident", "bytes_per_launch": 155122848,
+                         "kernel_source": ("genn_amd/csrc/genn_mi355x_resident_kernels.h", "145083ece8edb10b"),
+                         "source": "rocprofv3 --pmc FETCH_SIZE (67646.50 x 2 KiB) + WRITE_SIZE (16194.16 x 1 KiB) of the timed 20-step "
                                    "launch, profiles/residentKernel_potjans_full.md"},
     ("conv", 1000, 100): {"plan": "stepped", "requires": "conv_step_in_one_launch", "bytes_per_launch": 66118287,
                           "kernel_source": ("genn_amd/csrc/genn_mi355x_conv_step_kernels.h", "b33aec4cfae473d9"),
@@ -296,13 +296,16 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
         elif info["conv_step_in_one_launch"]:
             # the timed region consists of this kernel only (the layer on the matrix cores, the postsynaptic and neuron model on its
             # accumulators, the source population's update in blocks of the same launch), so HIP events around the region give
-            # its average duration; bytes by the event accounting (8 B per event: the target's read-modify-write) plus the state
-            avg_s = region_s / steps
-            ev_per_launch = events / steps
+            # its average duration; bytes by the event accounting (8 B per event: the target's read-modify-write) plus the state.
+            # Where the region took many steps at once instead, the kernel is that of the timed pass, a launch and an event pair per step.
+            ahead = info["feed_forward_ahead"]
+            avg_s = st["step_seconds"] / max(1, st["step_launches"]) if ahead else region_s / steps
+            ev_per_launch = evp / max(1, st["step_launches"]) if ahead else events / steps
             achieved = (ev_per_launch * bpe + neuron_bytes) / avg_s / 1e9
             c = [s_ for s_ in net.syns if s_.matrix == "conv2d"][0].conv
             flops = 2.0 * batch * c["conv_oh"] * c["conv_ow"] * c["conv_kh"] * c["conv_kw"] * c["conv_ic"] * c["conv_oc"]
-            roofline = {"bound": "hbm", "kernel": "convStepKernel (Conv2D on the matrix cores + neuron update of one timestep)",
+            roofline = {"bound": "hbm", "kernel": "convStepKernel (Conv2D on the matrix cores + neuron update of one timestep)"
+                                                  + (", launched step by step in this timed pass; the untimed region takes up to 128 steps at once (aheadConvKernel)" if ahead else ""),
                         "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 6),
                         "traffic": None, "bytes_per_event": bpe, "events_per_launch": round(ev_per_launch, 1),
                         "neuron_bytes_per_launch": neuron_bytes, "avg_launch_us": round(avg_s * 1e6, 3),
@@ -318,6 +321,8 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
             # synaptic kernels of a step into one launch where the runner's plan says so)
             if kinds == {"dense"}:
                 kernel = "presynapticDenseKernel"
+                if info["feed_forward_ahead"]:
+                    kernel += ", launched step by step in this timed pass; the untimed region takes up to 128 steps at once (aheadDenseKernel)"
             elif info["conv_on_matrix_cores"]:
                 kernel = "presynapticConvMfmaKernel (busy steps) + presynapticUpdateKernel (quiet steps)"
             elif info["combined_synapse_launch"]:
