@@ -184,23 +184,25 @@ PINNED_MOST = 64 << 20      # bytes of an array's host side up to which it is pi
 
 class Array:
     def __init__(self, count, dtype, fill=None, device_only=False, model=None, pinned=False):
-        """``device_only``: the device array's first value is somebody else's to write.  Copies of an array
-        of a ``model`` run in the order of its steps.  ``pinned``: the host side of an array that is copied again and again."""
+        """``fill``: the first value, one of all elements or one each.  ``device_only``: the device array's first value is somebody else's
+        to write.  Copies of an array of a ``model`` run in the order of its steps.  ``pinned``: the host side of an array that is
+        copied again and again."""
         self.dtype = np.dtype(dtype)
         self.count = int(count)
         self._model, self._pinned = model, pinned
         self._dev = C.c_void_p()
         _abi.check(_abi.load().gennmi_malloc(C.byref(self._dev), self.count * self.dtype.itemsize))
         self._view = None
+        fill = None if fill is None else np.asarray(fill, dtype=self.dtype)
         self._fill, self._given = fill, False
-        # (the first value is written on the device; the host copy is made when somebody asks for it)
+        # (one first value of all elements is written on the device; the host copy is made when somebody asks for it)
         if device_only or not self.count:
             pass
         elif fill is None:
             _abi.check(_abi.load().gennmi_memset(self._dev, 0, self.count * self.dtype.itemsize))
-        elif self.dtype == np.float32:
+        elif self.dtype == np.float32 and fill.ndim == 0:
             _abi.check(_abi.load().gennmi_init_var(self._dev, _abi.ELEMENT_TYPES["float32"], self.count, _abi.INIT_SNIPPETS["Constant"],
-                                                   C.byref((C.c_double * 4)(fill)), 0, 0))
+                                                   C.byref((C.c_double * 4)(float(fill))), 0, 0))
         else:
             self.push_to_device()
 
@@ -210,7 +212,7 @@ class Array:
             if self._given:
                 self.pull_from_device()
             else:
-                self._make_view().fill(0 if self._fill is None else self._fill)
+                self._make_view()[:] = 0 if self._fill is None else self._fill
         return self._view
 
     def _make_view(self):
