@@ -24,13 +24,18 @@ FLT_MAX = np.float32(3.402823466e+38)
 # --------------------------------------------------------------------------------------------
 # numeric literal handling
 # --------------------------------------------------------------------------------------------
-@functools.lru_cache(maxsize=4096)
 def lit32(x):
     """fp32 value of a parameter the reference bakes into generated code as a literal:
     double -> ``%.9e`` text -> correctly rounded float (src/genn/genn/type.cc:329-350)."""
     x = float(x)
     if x == 0.0 or math.isinf(x) or math.isnan(x):
         return np.float32(x)
+    return _lit32(x)
+
+
+# (kept by value: a float, never the object it came from, and no zero, whose two signs compare equal)
+@functools.lru_cache(maxsize=4096)
+def _lit32(x):
     text = "%.9e" % x
     exact = Fraction(text)
     c = np.float32(float(text))

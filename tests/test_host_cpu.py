@@ -6,6 +6,7 @@ import re
 
 import numpy as np
 import pytest
+import torch
 
 from genn_amd import _abi, configs, netgen, rng
 from genn_amd.genn_model import GeNNModel, init_postsynaptic, init_weight_update, lit32, field32, model_from_net
@@ -46,6 +47,18 @@ def test_literal_and_field_rounding():
     assert lit32(x) == np.float32(float("%.9e" % x))
     assert lit32(math.exp(-0.1 / 20.0)) == np.float32("9.950124792e-01")
     assert lit32(0.0) == 0.0 and lit32(-65.0) == np.float32(-65.0)
+
+
+def test_literals_are_of_values_not_of_objects():
+    """An array of one value is a value, one that is written again is another, and zero has two signs."""
+    for x in (np.array(0.1), np.array([0.1]), np.float32(0.1), 0.1):
+        assert lit32(x) == np.float32(float("%.9e" % float(np.asarray(x).reshape(-1)[0])))
+    held = torch.tensor(1.5, dtype=torch.float64)
+    assert lit32(held) == np.float32(1.5)
+    held.fill_(2.5)
+    assert lit32(held) == np.float32(2.5)
+    assert [np.signbit(lit32(z)) for z in (0.0, -0.0, 0.0)] == [False, True, False]
+    assert np.isnan(lit32(float("nan"))) and lit32(-np.inf) == -np.inf
 
 
 def test_generators_agree_and_shapes_hold():
