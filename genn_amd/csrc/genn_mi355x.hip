@@ -1047,7 +1047,8 @@ static int buildTileOffsets(const std::vector<TileOffsetsOf> &projections, std::
     for(size_t k = 0; k < projections.size(); k++) {
         const auto &p = projections[k];
         const uint32_t shift = ((p.tileSize & (p.tileSize - 1)) == 0) ? (uint32_t)__builtin_ctz(p.tileSize) : 32u;
-        tileOffsetKernel<<<dim3((p.g->numSrcNeurons + BLOCK / WAVE - 1) / (BLOCK / WAVE)), dim3(BLOCK), 0, 0>>>(
+        const uint32_t blocks = std::min(TILE_OFFSET_BLOCKS, (uint32_t)(((size_t)p.g->numSrcNeurons + BLOCK / WAVE - 1) / (BLOCK / WAVE)));
+        tileOffsetKernel<<<dim3(blocks), dim3(BLOCK), 0, 0>>>(
             p.g->numSrcNeurons, p.g->rowStride, p.g->rowLength, p.g->ind, p.tileSize, shift, p.numTiles, p.off, dFlags + k);
     }
     HIP_TRY(hipGetLastError());

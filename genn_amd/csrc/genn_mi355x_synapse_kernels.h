@@ -806,38 +806,41 @@ void presynapticConvTileKernel(const ConvTileDev * __restrict__ blocks, unsigned
 // Segment boundaries of every row for the tile kernel; also verifies that rows are sorted by target.  A wavefront takes a row,
 // 64 consecutive synapses at a time (one lane per row read every row's entries one dependent access after another: 0.16 ms for
 // 2 x 10^7 synapses, now 0.03).  The lane whose synapse is the first one at or beyond a boundary writes it.  `shift`: log2 of the tile
-// size, or 32 if it is no power of two.
+// size, or 32 if it is no power of two.  Rows beyond the grid's wavefronts come in further rounds: a launch holds fewer than 2^32
+// threads, which a wavefront a row would exceed from 2^26 rows on.
+constexpr uint32_t TILE_OFFSET_BLOCKS = 1u << 20;
 __global__ __launch_bounds__(BLOCK)
 void tileOffsetKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLength, const uint32_t *ind,
                       uint32_t tileSize, uint32_t shift, uint32_t numTiles, uint16_t *off, uint32_t *unsorted)
 {
-    const uint32_t row = (blockIdx.x * BLOCK + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    if(row >= numSrc) { return; }
-    const uint32_t len = rowLength[row];
-    const uint32_t *r = ind + (size_t)row * rowStride;
-    uint16_t *o = off + (size_t)row * (numTiles + 1);
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
     auto tileOf = [&](uint32_t p) { return (shift < 32u) ? (p >> shift) : (p / tileSize); };
-    // boundary t is the position of the first synapse whose target's tile is >= t
-    uint32_t before = 0, next = 0;      // target of the last synapse of the pass before; first boundary not yet written
-    constexpr uint32_t AHEAD = 8;       // passes whose entries are asked for together
-    for(uint32_t j0 = 0; j0 < len; j0 += AHEAD * WAVE) {
-        uint32_t entry[AHEAD];
-        #pragma unroll
-        for(uint32_t u = 0; u < AHEAD; u++) { entry[u] = r[min(j0 + u * WAVE + lane, len - 1)]; }
-        #pragma unroll
-        for(uint32_t u = 0; u < AHEAD; u++) {
-            const uint32_t j = j0 + u * WAVE + lane, p = entry[u];
-            const uint32_t left = (uint32_t)__shfl_up((int)p, 1, WAVE), prev = (lane == 0) ? before : left;
-            if(j < len) {
-                if(p < prev) { atomicOr(unsorted, 1u); }
-                const uint32_t first = (j == 0) ? 0u : tileOf(prev) + 1u;
-                for(uint32_t t = first; t <= min(tileOf(p), numTiles); t++) { o[t] = (uint16_t)j; }
+    for(size_t row = (size_t)blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE; row < numSrc; row += (size_t)gridDim.x * (BLOCK / WAVE)) {
+        const uint32_t len = rowLength[row];
+        const uint32_t *r = ind + row * rowStride;
+        uint16_t *o = off + row * (numTiles + 1);
+        // boundary t is the position of the first synapse whose target's tile is >= t
+        uint32_t before = 0, next = 0;      // target of the last synapse of the pass before; first boundary not yet written
+        constexpr uint32_t AHEAD = 8;       // passes whose entries are asked for together
+        for(uint32_t j0 = 0; j0 < len; j0 += AHEAD * WAVE) {
+            uint32_t entry[AHEAD];
+            #pragma unroll
+            for(uint32_t u = 0; u < AHEAD; u++) { entry[u] = r[min(j0 + u * WAVE + lane, len - 1)]; }
+            #pragma unroll
+            for(uint32_t u = 0; u < AHEAD; u++) {
+                const uint32_t j = j0 + u * WAVE + lane, p = entry[u];
+                const uint32_t left = (uint32_t)__shfl_up((int)p, 1, WAVE), prev = (lane == 0) ? before : left;
+                if(j < len) {
+                    if(p < prev) { atomicOr(unsorted, 1u); }
+                    const uint32_t first = (j == 0) ? 0u : tileOf(prev) + 1u;
+                    for(uint32_t t = first; t <= min(tileOf(p), numTiles); t++) { o[t] = (uint16_t)j; }
+                }
+                before = (uint32_t)__shfl((int)p, WAVE - 1, WAVE);
+                next = tileOf(before) + 1u;
             }
-            before = (uint32_t)__shfl((int)p, WAVE - 1, WAVE);
-            next = tileOf(before) + 1u;
         }
+        for(uint32_t t = next + lane; t <= numTiles; t += WAVE) { o[t] = (uint16_t)len; }
     }
-    for(uint32_t t = next + lane; t <= numTiles; t += WAVE) { o[t] = (uint16_t)len; }
 }
 
 // Builds the segment records of one projection from its rows and the segment boundaries: one thread per (tile, row).

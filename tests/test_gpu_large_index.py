@@ -75,3 +75,38 @@ def test_rows_beyond_32_bit_synapse_ids_are_delivered():
         assert model.synaptic_event_count == total_events
         model.update_neurons()
     model.unload()
+
+
+def test_rows_beyond_a_launch_of_a_wavefront_each():
+    """2^26 rows and a few: a wavefront per row would be more threads than a launch may have.  The source's queue is written by hand,
+    so that both presynaptic paths (some spikes, then enough for the tile kernel) are seen at rows on either side; integer weights."""
+    n_src, n_trg, rng = (1 << 26) + 70, 100, np.random.default_rng(4)
+    rows = np.unique(np.concatenate([[0, 1, (1 << 22) - 1, 1 << 22, (1 << 26) - 1, 1 << 26, n_src - 1], rng.integers(0, n_src, 200), rng.integers(1 << 26, n_src, 30)]))
+    row_length, ind, g = np.zeros(n_src, np.uint32), np.zeros((n_src, 2), np.uint32), np.zeros((n_src, 2), np.float32)
+    row_length[rows] = rng.integers(0, 3, len(rows))
+    row_length[rows[-3:]] = 2
+    ind[rows] = np.sort(rng.integers(0, n_trg, (len(rows), 2)), axis=1)
+    g[rows] = rng.integers(1, 9, (len(rows), 2))
+
+    model = GeNNModel("float", "many_rows", dt=1.0)
+    src = model.add_neuron_population("S", n_src, "SpikeSourceArray", {}, {"startSpike": np.zeros(1), "endSpike": np.zeros(1)})
+    src.set_extra_global_param("spikeTimes", np.zeros(1, np.float32))
+    trg = model.add_neuron_population("T", n_trg, "LIF", LIF_SILENT, {"V": -60.0, "RefracTime": 0.0})
+    s = model.add_synapse_population("ST", "SPARSE", src, trg, init_weight_update("StaticPulse", {}, {"g": 0.0}), init_postsynaptic("DeltaCurr"))
+    s.set_ragged(row_length, ind)
+    s.set_var_ragged("g", g)
+    model.build()
+    model.load()
+    want = np.zeros(n_trg)
+    for spikes in (rows[-3:], rows):
+        src.vars["spkCnt"].view[:] = len(spikes)
+        src.vars["spk"].view[:len(spikes)] = spikes
+        for name in ("spkCnt", "spk"):
+            src.vars[name].push_to_device()
+        model.update_synapses()
+        for k in range(2):
+            there = spikes[row_length[spikes] > k]
+            np.add.at(want, ind[there, k], g[there, k])
+        assert np.array_equal(s.vars["outPost"].pull_from_device(), want.astype(np.float32)), f"{len(spikes)} spikes"
+    assert 3 * 2 < n_trg <= 2 * len(rows)       # (the tile kernel takes a step of as many possible events as targets)
+    model.unload()
