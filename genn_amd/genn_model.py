@@ -225,7 +225,15 @@ class Array:
         if self._view is None:
             pinned = self._pinned and 0 < self.count * self.dtype.itemsize <= PINNED_MOST
             self._view = np.asarray(_Pinned(self.count, self.dtype)) if pinned else np.empty(self.count, dtype=self.dtype)
+            self._host_address = self._view.ctypes.data
         return self._view
+
+    @property
+    def host_address(self):
+        """Where the host side lies (asked of numpy once: a microsecond each time)."""
+        if self._view is None:
+            self.view
+        return self._host_address
 
     @property
     def ptr(self):
@@ -319,7 +327,6 @@ class NeuronGroup:
         self.needs_spike_time = False
         self.num_delay_slots = 1     # longest axonal delay of the outgoing projections + 1, set by build()
         self.pre_output_syn = []     # outgoing projections whose code calls addToPre
-        self._queue_copy = None      # where current_spikes copies the queue to
         self.event_thresholds = []   # one spike-like event queue per distinct threshold of the outgoing graded projections
 
     @property
@@ -336,18 +343,19 @@ class NeuronGroup:
 
     @property
     def current_spikes(self):
-        """Spike queue written by the last step: ids in ascending order (per batch)."""
+        """Spike queue written by the last step: ids in ascending order (per batch).  The host sides of `spkCnt` and `spk` hold it as well."""
         # with axonal delay the queue is a ring of slots; the last step wrote slot timestep % slots (pygenn's current_spikes
         # reads spkQuePtr the same way, genn_groups.py)
         model, slots, n = self._model, self.num_delay_slots, self.num_neurons
-        B = model.batch_size
-        if self._queue_copy is None:
-            ids, counts = np.empty((B, n), np.uint32), np.empty(B, np.uint32)
-            self._queue_copy = ids, counts, ids.ctypes.data, counts.ctypes.data
-        ids, counts, ids_address, counts_address = self._queue_copy
-        _abi.check(_abi.load().gennmi_runner_pull_spikes(model._runner, self.vars["spkCnt"]._dev, self.vars["spk"]._dev, n, slots,
-                                                         model.timestep % slots, counts_address, ids_address))
-        return [ids[b, :counts[b]].copy() for b in range(B)]
+        count, spk = self.vars["spkCnt"], self.vars["spk"]
+        if slots > 1:
+            pull_arrays(model._runner, [count, spk])
+        else:
+            # (the counts and each batch's valid entries, which lie in these arrays as the call writes them)
+            _abi.check(_abi.load().gennmi_runner_pull_spikes(model._runner, count._dev, spk._dev, n, 1, 0, count.host_address, spk.host_address))
+        counts, ids = count.view.reshape(-1, slots), spk.view.reshape(-1, slots, n)
+        slot = model.timestep % slots
+        return [ids[b, slot, :counts[b, slot]].copy() for b in range(model.batch_size)]
 
 
 class CurrentSource:

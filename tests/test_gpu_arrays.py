@@ -48,3 +48,39 @@ def test_an_arrays_first_value_is_one_of_all_or_one_each(fill):
     assert np.array_equal(a.pull_slice(0, 5), want)
     assert np.array_equal(a.view, want) and np.array_equal(a.pull_from_device(), want)
     a.free()
+
+
+@pytest.mark.parametrize("batch, delay", [(1, 0), (3, 0), (1, 3), (2, 2)])
+def test_current_spikes_leaves_the_queue_on_the_host_side(make_model, batch, delay):
+    """After current_spikes the host sides of `spkCnt` and `spk` show what the device's hold, in arrays a program may have kept."""
+    n, steps, rng = 300, 8, np.random.default_rng(11)
+    fire = rng.random((batch, n, steps)) < 0.2
+    fire[:, :, 3] = False
+    fire[:, :, 5] = True
+    count = fire.sum(axis=2).reshape(-1)
+    end = np.cumsum(count).reshape(batch, n)
+    m = make_model("float", "queues", dt=1.0, batch_size=batch)
+    src = m.add_neuron_population("S", n, "SpikeSourceArray", {}, {"startSpike": end - count.reshape(batch, n), "endSpike": end})
+    src.set_extra_global_param("spikeTimes", np.nonzero(fire.reshape(batch * n, steps))[1].astype(np.float32))
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=1e9, Ioffset=0.0, TauRefrac=5.0)
+    trg = m.add_neuron_population("T", 5, "LIF", lif, {"V": -60.0, "RefracTime": 0.0})
+    s = m.add_synapse_population("ST", "SPARSE", src, trg, init_weight_update("StaticPulse", {}, {"g": 1.0}), init_postsynaptic("DeltaCurr"))
+    s.set_sparse_connections([0, 1], [0, 1])
+    s.axonal_delay_steps = delay
+    m.build()
+    m.load()
+    slots = src.num_delay_slots
+    assert slots == (delay + 1 if delay else 1)
+    kept = src.vars["spkCnt"].view, src.vars["spk"].view
+    for step in range(steps):
+        m.step_time()
+        spikes = src.current_spikes
+        counts, ids = src.vars["spkCnt"].view, src.vars["spk"].view
+        assert counts is kept[0] and ids is kept[1]
+        assert np.array_equal(counts, src.vars["spkCnt"].pull_slice(0, batch * slots))
+        device = src.vars["spk"].pull_slice(0, batch * slots * n).reshape(-1, n)
+        for q, c in enumerate(counts):
+            assert np.array_equal(ids.reshape(-1, n)[q, :c], device[q, :c])
+        for b in range(batch):
+            assert np.array_equal(spikes[b], np.nonzero(fire[b, :, step])[0])
+            assert not np.shares_memory(spikes[b], ids)
