@@ -267,6 +267,7 @@ int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr
 int gennmi_host_acquire(void **hostPtr, size_t bytes)
 {
     if(!hostPtr) { return fail(GENNMI_EINVAL, "host_acquire: null result pointer"); }
+    if(!pinnedCopies()) { return fail(GENNMI_EUNSUPPORTED, "host_acquire: GENNMI_PINNED_COPIES=0"); }
     return pinnedMalloc(hostPtr, bytes);
 }
 int gennmi_host_free(void *hostPtr)
@@ -501,6 +502,7 @@ int gennmi_release_cached_memory(void)
         std::lock_guard<std::mutex> lock(g_pool.mutex);
         HIP_TRY(g_pool.releaseAll());
     }
+    { const int rc = releaseIdleRings(); if(rc) { return rc; } }
     std::lock_guard<std::mutex> lock(g_pinnedMutex);
     HIP_TRY(releaseIdlePinned());
     return GENNMI_OK;

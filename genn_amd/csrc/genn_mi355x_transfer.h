@@ -12,6 +12,7 @@
 // back: touching it for the first time costs 0.4 ms per MiB.  Other host memory goes through a small ring of pinned chunks
 // on its way from the device — while the device moves one chunk, the host copies the one before it: 13 MB in 0.5 ms, by
 // hipMemcpy 0.8 ms — and by the runtime's own copy on its way there (it reads pageable memory in place: 13 MB in 0.4 ms).
+// Where no pinned memory is to be had (GENNMI_PINNED_COPIES=0 asks for none), all of it goes by the runtime's copies.
 #ifndef GENN_MI355X_TRANSFER_H
 #define GENN_MI355X_TRANSFER_H
 
@@ -156,6 +157,7 @@ int pinnedMalloc(void **ptr, size_t bytes)
         HIP_TRY(releaseIdlePinned());
         e = hipHostMalloc(ptr, bytes, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
     }
+    if(e != hipSuccess) { (void)hipGetLastError(); }        // (reported here, and not by the next launch of a caller that does without)
     HIP_TRY(e);
     g_pinned[reinterpret_cast<uintptr_t>(*ptr)] = bytes;
     return GENNMI_OK;
@@ -203,11 +205,20 @@ struct TransferRing
 };
 
 std::mutex g_ringMutex;
-std::vector<TransferRing*> g_rings;     // idle ones; as many exist as transfers have ever run at once
+std::vector<TransferRing*> g_rings;     // idle ones; as many exist as transfers have run at once
 
+// copies may take pinned memory of their own (looked at where memory is taken: rings and host sides that exist are used on)
+bool pinnedCopies()
+{
+    const char *e = getenv("GENNMI_PINNED_COPIES");
+    return !(e && atoi(e) == 0);
+}
+
+// *out: null where there is no memory for a ring
 int borrowRing(TransferRing **out)
 {
     int device = 0;
+    *out = nullptr;
     HIP_TRY(hipGetDevice(&device));
     {
         std::lock_guard<std::mutex> lock(g_ringMutex);
@@ -215,6 +226,7 @@ int borrowRing(TransferRing **out)
             if(g_rings[k]->device == device) { *out = g_rings[k]; g_rings.erase(g_rings.begin() + k); return GENNMI_OK; }
         }
     }
+    if(!pinnedCopies()) { return GENNMI_OK; }
     TransferRing *ring = new TransferRing;
     ring->device = device;
     const size_t flagBytes = TRANSFER_SLOTS * 16 * sizeof(uint32_t);
@@ -232,7 +244,8 @@ int borrowRing(TransferRing **out)
         if(ring->counters) { (void)hipFree(ring->counters); }
         if(host) { (void)hipHostFree(host); }
         delete ring;
-        return fail(GENNMI_EHIP, std::string("transfer ring: ") + hipGetErrorString(e));
+        (void)hipGetLastError();
+        return GENNMI_OK;           // (an error that is not of this memory comes back from the runtime's copy)
     }
     *out = ring;
     return GENNMI_OK;
@@ -241,10 +254,11 @@ int borrowRing(TransferRing **out)
 struct RingLease
 {
     TransferRing *ring = nullptr;
-    ~RingLease()
+    void end()
     {
-        if(ring) { std::lock_guard<std::mutex> lock(g_ringMutex); g_rings.push_back(ring); }
+        if(ring) { std::lock_guard<std::mutex> lock(g_ringMutex); g_rings.push_back(ring); ring = nullptr; }
     }
+    ~RingLease() { end(); }
 };
 
 // the ring's next slot, once the device is done with what it held
@@ -253,6 +267,25 @@ int nextSlot(TransferRing *ring, hipStream_t stream, uint32_t *slot)
     *slot = ring->next;
     ring->next = (ring->next + 1) % TRANSFER_SLOTS;
     return waitForFlag(ring->flag(*slot), ring->seq[*slot], stream);
+}
+
+// Gives the idle rings back, once the device is done with them
+int releaseIdleRings()
+{
+    std::vector<TransferRing*> rings;
+    { std::lock_guard<std::mutex> lock(g_ringMutex); rings.swap(g_rings); }
+    int rc = GENNMI_OK, device = 0;
+    if(!rings.empty()) { HIP_TRY(hipGetDevice(&device)); }
+    for(TransferRing *ring : rings) {
+        hipError_t e = hipSetDevice(ring->device);
+        if(e == hipSuccess) { e = hipDeviceSynchronize(); }
+        if(e == hipSuccess) { e = hipFree(ring->counters); }
+        if(e == hipSuccess) { e = hipHostFree(ring->flags); }           // (the chunks lie behind the flags)
+        if(e != hipSuccess) { rc = fail(GENNMI_EHIP, std::string("transfer ring: ") + hipGetErrorString(e)); }
+        delete ring;
+    }
+    if(!rings.empty()) { HIP_TRY(hipSetDevice(device)); }
+    return rc;
 }
 
 struct TransferPart { uint8_t *host; uint8_t *dev; size_t bytes; };
@@ -289,6 +322,13 @@ int pullParts(const TransferPart *parts, uint32_t count, hipStream_t stream)
     RingLease lease;
     { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
     TransferRing *ring = lease.ring;
+    if(!ring) {
+        for(uint32_t p = 0; p < count; p++) {
+            if(parts[p].bytes) { HIP_TRY(hipMemcpyAsync(parts[p].host, parts[p].dev, parts[p].bytes, hipMemcpyDeviceToHost, stream)); }
+        }
+        HIP_TRY(hipStreamSynchronize(stream));
+        return GENNMI_OK;
+    }
     struct Pending { uint8_t *host; const uint8_t *chunk; uint32_t bytes, slot, seq; };
     Pending pending[TRANSFER_SLOTS];
     uint32_t first = 0, waiting = 0;
@@ -318,14 +358,14 @@ int pullParts(const TransferPart *parts, uint32_t count, hipStream_t stream)
 int pushArray(const TransferPart &part, hipStream_t stream, bool wait)
 {
     if(part.bytes == 0) { return GENNMI_OK; }
-    if(part.bytes > (wait ? PUSH_RING_BYTES : 2 * TRANSFER_CHUNK) && !isPinned(part.host, part.bytes)) {
+    RingLease lease;
+    if(part.bytes <= (wait ? PUSH_RING_BYTES : 2 * TRANSFER_CHUNK) || isPinned(part.host, part.bytes)) { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
+    TransferRing *ring = lease.ring;
+    if(!ring) {
         HIP_TRY(hipMemcpyAsync(part.dev, part.host, part.bytes, hipMemcpyHostToDevice, stream));
         HIP_TRY(hipStreamSynchronize(stream));
         return GENNMI_OK;
     }
-    RingLease lease;
-    { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
-    TransferRing *ring = lease.ring;
     uint32_t last = 0;
     const int rc = forEachChunk(&part, 1, [&](uint8_t *host, uint8_t *dev, uint32_t bytes, bool direct) -> int {
         uint32_t slot;
@@ -344,6 +384,11 @@ int copyOnDevice(float *dst, const float *src, size_t count, hipStream_t stream)
 {
     RingLease lease;
     { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
+    if(!lease.ring) {
+        HIP_TRY(hipMemcpyAsync(dst, src, count * sizeof(float), hipMemcpyDeviceToDevice, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        return GENNMI_OK;
+    }
     uint32_t slot;
     { const int rc = nextSlot(lease.ring, stream, &slot); if(rc) { return rc; } }
     const uint32_t blocks = (uint32_t)std::min<size_t>(2048, std::max<size_t>(1, (count + 4 * BLOCK - 1) / (4 * BLOCK)));
@@ -359,30 +404,40 @@ int pullSpikes(const uint32_t *spkCnt, const uint32_t *spk, uint32_t numNeurons,
 {
     const size_t words = TRANSFER_CHUNK / sizeof(uint32_t);
     if(batch > words) { return fail(GENNMI_EINVAL, "pull_spikes: too many batches"); }
-    const uint32_t capacity = (uint32_t)std::min<size_t>(numNeurons, (words - batch) / batch);
-    std::vector<TransferPart> rest;         // queues of more spikes than the chunk holds
+    auto part = [](uint32_t *host, const uint32_t *dev, size_t count)
     {
-        RingLease lease;
-        { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
-        TransferRing *ring = lease.ring;
-        uint32_t s;
-        { const int rc = nextSlot(ring, stream, &s); if(rc) { return rc; } }
-        uint32_t *out = reinterpret_cast<uint32_t*>(ring->chunk(s));
-        pullSpikesKernel<<<dim3(std::min(batch, TRANSFER_BLOCKS)), dim3(BLOCK), 0, stream>>>(spkCnt, spk, numNeurons, slots, slot, batch, capacity, out,
-                                                                                           ring->counters + s, ring->flag(s), ring->seq[s] + 1);
-        HIP_TRY(hipGetLastError());
-        ring->seq[s]++;
-        { const int rc = waitForFlag(ring->flag(s), ring->seq[s], stream); if(rc) { return rc; } }
-        memcpy(counts, out, batch * sizeof(uint32_t));
+        return TransferPart{reinterpret_cast<uint8_t*>(host), reinterpret_cast<uint8_t*>(const_cast<uint32_t*>(dev)), count * sizeof(uint32_t)};
+    };
+    std::vector<TransferPart> rest;         // queues of more spikes than the chunk holds
+    RingLease lease;
+    { const int rc = borrowRing(&lease.ring); if(rc) { return rc; } }
+    TransferRing *ring = lease.ring;
+    if(!ring) {
+        for(uint32_t b = 0; b < batch; b++) { rest.push_back(part(counts + b, spkCnt + (size_t)b * slots + slot, 1)); }
+        { const int rc = pullParts(rest.data(), batch, stream); if(rc) { return rc; } }
+        rest.clear();
         for(uint32_t b = 0; b < batch; b++) {
-            const uint32_t fit = std::min(counts[b], capacity);
-            memcpy(ids + (size_t)b * numNeurons, out + batch + (size_t)b * capacity, (size_t)fit * sizeof(uint32_t));
-            if(counts[b] > fit) {
-                rest.push_back({reinterpret_cast<uint8_t*>(ids + (size_t)b * numNeurons + fit),
-                                reinterpret_cast<uint8_t*>(const_cast<uint32_t*>(spk + ((size_t)b * slots + slot) * numNeurons + fit)), (size_t)(counts[b] - fit) * sizeof(uint32_t)});
-            }
+            counts[b] = std::min(counts[b], numNeurons);
+            if(counts[b]) { rest.push_back(part(ids + (size_t)b * numNeurons, spk + ((size_t)b * slots + slot) * numNeurons, counts[b])); }
         }
+        return pullParts(rest.data(), (uint32_t)rest.size(), stream);
     }
+    const uint32_t capacity = (uint32_t)std::min<size_t>(numNeurons, (words - batch) / batch);
+    uint32_t s;
+    { const int rc = nextSlot(ring, stream, &s); if(rc) { return rc; } }
+    uint32_t *out = reinterpret_cast<uint32_t*>(ring->chunk(s));
+    pullSpikesKernel<<<dim3(std::min(batch, TRANSFER_BLOCKS)), dim3(BLOCK), 0, stream>>>(spkCnt, spk, numNeurons, slots, slot, batch, capacity, out,
+                                                                                       ring->counters + s, ring->flag(s), ring->seq[s] + 1);
+    HIP_TRY(hipGetLastError());
+    ring->seq[s]++;
+    { const int rc = waitForFlag(ring->flag(s), ring->seq[s], stream); if(rc) { return rc; } }
+    memcpy(counts, out, batch * sizeof(uint32_t));
+    for(uint32_t b = 0; b < batch; b++) {
+        const uint32_t fit = std::min(counts[b], capacity);
+        memcpy(ids + (size_t)b * numNeurons, out + batch + (size_t)b * capacity, (size_t)fit * sizeof(uint32_t));
+        if(counts[b] > fit) { rest.push_back(part(ids + (size_t)b * numNeurons + fit, spk + ((size_t)b * slots + slot) * numNeurons + fit, counts[b] - fit)); }
+    }
+    lease.end();
     return rest.empty() ? GENNMI_OK : pullParts(rest.data(), (uint32_t)rest.size(), stream);
 }
 }   // namespace

@@ -223,8 +223,13 @@ class Array:
     def _make_view(self):
         """The host side, its contents left to the caller."""
         if self._view is None:
-            pinned = self._pinned and 0 < self.count * self.dtype.itemsize <= PINNED_MOST
-            self._view = np.asarray(_Pinned(self.count, self.dtype)) if pinned else np.empty(self.count, dtype=self.dtype)
+            if self._pinned and 0 < self.count * self.dtype.itemsize <= PINNED_MOST:
+                try:
+                    self._view = np.asarray(_Pinned(self.count, self.dtype))
+                except _abi.GennmiError:
+                    pass        # (no pinned memory to be had: ordinary memory is copied more slowly)
+            if self._view is None:
+                self._view = np.empty(self.count, dtype=self.dtype)
             self._host_address = self._view.ctypes.data
         return self._view
 

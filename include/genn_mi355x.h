@@ -84,8 +84,8 @@ int gennmi_malloc(void **devPtr, size_t bytes);                 /* Array::alloca
  * copies.  Without it devPtr may be NULL.  gennmi_host_free releases the memory. */
 int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr);
 int gennmi_host_free(void *hostPtr);
-/* The same memory, not cleared, for a host side that is about to be written whole.  Pinned memory without zeroCopy is kept for
- * reuse when it is freed (up to 256 MiB of it). */
+/* The same memory, not cleared, for a host side that is about to be written whole; a caller that is refused it does as well with
+ * memory of its own, which every copy takes.  Pinned memory without zeroCopy is kept for reuse when it is freed (up to 256 MiB of it). */
 int gennmi_host_acquire(void **hostPtr, size_t bytes);
 int gennmi_free(void *devPtr);                                  /* Array::free      hip/backend.cc:110-128 */
 int gennmi_memcpy_to_device(void *dev, const void *host, size_t bytes);    /* pushToDevice / pushSlice1DToDevice   :130-176 */
@@ -140,7 +140,7 @@ int gennmi_mirror_device_initialised(const void *host);
 int gennmi_mirror_ensure_host(const void *host);
 /* Blocks of device memory that were freed are kept for the next allocation of their size: at most 1/32 of the card's memory in all,
  * each for at most ten seconds of idleness; the bytes reported free include them.  This gives all of them back to the
- * system, and the idle pinned memory with them. */
+ * system, and the idle pinned memory (freed host sides, staging of copies) with them. */
 int gennmi_release_cached_memory(void);
 int gennmi_free_device_memory_bytes(size_t *bytes);
 /* Named ranges for profilers around stepTime / updateSynapses / updateNeurons (BackendBase::genPushProfilerRange /

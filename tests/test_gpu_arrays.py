@@ -2,7 +2,8 @@
 import numpy as np
 import pytest
 
-from genn_amd.genn_model import init_postsynaptic, init_weight_update
+from genn_amd import _abi, configs, genn_model
+from genn_amd.genn_model import init_postsynaptic, init_weight_update, model_from_net
 
 pytestmark = pytest.mark.gpu
 
@@ -40,10 +41,8 @@ def test_initial_traces_may_be_one_a_neuron(make_model, fires, batch):
 
 @pytest.mark.parametrize("fill", [2.5, np.float32(2.5), np.array(2.5), [2.5], np.arange(5.0), [1, 2, 3, 4, 5]])
 def test_an_arrays_first_value_is_one_of_all_or_one_each(fill):
-    from genn_amd import _abi
-    from genn_amd.genn_model import Array
     _abi.check(_abi.load().gennmi_init(0))
-    a = Array(5, np.float32, fill=fill)
+    a = genn_model.Array(5, np.float32, fill=fill)
     want = np.full(5, fill, dtype=np.float32)
     assert np.array_equal(a.pull_slice(0, 5), want)
     assert np.array_equal(a.view, want) and np.array_equal(a.pull_from_device(), want)
@@ -84,3 +83,54 @@ def test_current_spikes_leaves_the_queue_on_the_host_side(make_model, batch, del
         for b in range(batch):
             assert np.array_equal(spikes[b], np.nonzero(fire[b, :, step])[0])
             assert not np.shares_memory(spikes[b], ids)
+
+
+def _run_of_a_small_network():
+    """Everything that is copied: pushes and pulls of small and large arrays, queues of one slot and of several, recordings, a copy on the device."""
+    m = model_from_net(configs.vogels_abbott(n=2000, steps=40, p=0.05, axonal_delays={"EI": 3}), ordered=True)     # (sums in a fixed order)
+    batched = model_from_net(configs.conv_toeplitz(h=16, w=16, ic=4, oc=8, steps=10, max_rate=300.0), batch_size=2)
+    out = []
+    for model, steps in ((m, 40), (batched, 10)):
+        model.load(num_recording_timesteps=steps)
+        for _ in range(steps):
+            model.step_time()
+            out += [ids for p in model.neuron_populations.values() for ids in p.current_spikes]
+        model.pull_recording_buffers_from_device()
+        out += [p.vars["recordSpk"].view.copy() for p in model.neuron_populations.values()]
+    a, b = m._alloc(1_300_001, np.float32), m._alloc(1_300_001, np.float32)
+    a.view[:] = np.arange(a.count)
+    a.push_to_device()
+    b.copy_on_device(a)
+    out += [b.pull_from_device().copy()] + [p.vars["V"].pull_from_device().copy() for p in m.neuron_populations.values()]
+    for model in (m, batched):
+        model.unload()
+    return out
+
+
+def test_copies_without_pinned_memory(monkeypatch):
+    """Where none is to be had the host sides are ordinary memory and the runtime's copies move everything: the same bytes."""
+    _abi.check(_abi.load().gennmi_init(0))
+    want = _run_of_a_small_network()
+    monkeypatch.setenv("GENNMI_PINNED_COPIES", "0")
+    _abi.check(_abi.load().gennmi_release_cached_memory())      # (also the staging memory of earlier copies)
+    a = genn_model.Array(10, np.float32, pinned=True)
+    assert a.view.base is None          # (its own memory, nothing of the library's)
+    a.free()
+    got = _run_of_a_small_network()
+    monkeypatch.delenv("GENNMI_PINNED_COPIES")
+    assert len(want) == len(got) and sum(int(np.any(w)) for w in want) > 20
+    assert all(np.array_equal(w, g) for w, g in zip(want, got))
+    again = _run_of_a_small_network()
+    assert all(np.array_equal(w, g) for w, g in zip(want, again))
+
+
+def test_a_refused_host_side_is_ordinary_memory(make_model, monkeypatch):
+    lib = _abi.load()
+    _abi.check(lib.gennmi_init(0))
+    monkeypatch.setattr(genn_model, "_Pinned", lambda count, dtype: _abi.check(2))
+    a = genn_model.Array(1000, np.float32, fill=3.0, pinned=True)
+    assert np.array_equal(a.pull_from_device(), np.full(1000, 3.0, np.float32))
+    a.view[:] = 4.0
+    a.push_to_device()
+    assert np.array_equal(a.pull_slice(0, 1000), a.view)
+    a.free()
