@@ -49,6 +49,7 @@
 #include "genn_mi355x_ordered_kernels.h"
 #include "genn_mi355x_conv_step_kernels.h"
 #include "genn_mi355x_ahead_kernels.h"
+#include "genn_mi355x_idle.h"
 #include "genn_mi355x_transfer.h"
 #include "genn_mi355x_pool.h"
 

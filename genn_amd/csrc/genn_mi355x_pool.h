@@ -5,21 +5,21 @@
 // model after model (a parameter scan, a session) paid that for every one of them; 10^5 neurons with 10^8 synapses take 22 ms
 // to build that way and 2 ms from kept blocks.
 //
-// Blocks of POOL_SMALLEST bytes and more are kept, at most a thirty-second of the card's memory in all, and each for at most
-// POOL_SECONDS of idleness (seen when memory is next asked for or given back); an allocation that fails gives all of them back
-// first, and gennmi_release_cached_memory does at any time.  A kept block is handed out again only after everything that
-// the device had been given when the block was freed has finished, on whatever stream and from whatever thread.
+// Blocks of POOL_SMALLEST bytes and more are kept, at most a thirty-second of the card's memory in all, and each for ten seconds
+// (GENNMI_POOL_SECONDS; 0: none is kept), after which a thread of the library's gives it back, also in a process that does
+// nothing any more; an allocation that fails gives all of them back first, and gennmi_release_cached_memory does at any time.
+// A kept block is handed out again only after everything that the device had been given when the block was freed has
+// finished, on whatever stream and from whatever thread.
 #ifndef GENN_MI355X_POOL_H
 #define GENN_MI355X_POOL_H
 
 namespace
 {
 constexpr size_t POOL_SMALLEST = size_t(2) << 20;           // (smaller ones the runtime hands out in less than a microsecond)
-constexpr int POOL_SECONDS = 10;
 
 struct DevicePool
 {
-    struct Idle { void *ptr; size_t bytes; int device; bool finished; std::chrono::steady_clock::time_point since; };
+    struct Idle { void *ptr; size_t bytes; int device; bool finished; IdleTime until; };
     struct Used { size_t bytes; int device; };
     std::mutex mutex;
     std::map<void*, Used> used;
@@ -42,15 +42,30 @@ struct DevicePool
     }
     hipError_t releaseOld()
     {
-        const auto now = std::chrono::steady_clock::now();
-        while(!idle.empty() && (idleBytes > limit || now - idle.front().since > std::chrono::seconds(POOL_SECONDS))) {
-            const hipError_t e = release(0);
+        const IdleTime now = IdleClock::now();
+        for(size_t k = 0; k < idle.size(); ) {
+            if(idleBytes <= limit && idle[k].until > now) { k++; continue; }
+            const hipError_t e = release(k);
             if(e != hipSuccess) { return e; }
         }
         return hipSuccess;
     }
 };
 DevicePool g_pool;
+
+// (called by the library's thread) gives back what has been idle long enough; when to look again
+IdleTime poolReleaseOld()
+{
+    std::lock_guard<std::mutex> lock(g_pool.mutex);
+    const IdleTime now = IdleClock::now();
+    IdleTime next = IdleTime::max();
+    for(size_t k = 0; k < g_pool.idle.size(); ) {
+        if(g_pool.idle[k].until > now) { next = std::min(next, g_pool.idle[k++].until); continue; }
+        if(hipSetDevice(g_pool.idle[k].device) != hipSuccess) { (void)hipGetLastError(); k++; continue; }
+        if(g_pool.release(k) != hipSuccess) { (void)hipGetLastError(); }
+    }
+    return next;
+}
 
 hipError_t poolMalloc(void **ptr, size_t bytes)
 {
@@ -103,10 +118,13 @@ hipError_t poolFree(void *ptr)
                 if(e != hipSuccess) { return e; }
                 g_pool.limit = total / 32;
             }
-            g_pool.idle.push_back({ptr, block->second.bytes, block->second.device, false, std::chrono::steady_clock::now()});
+            const IdleTime until = idleUntil();
+            g_pool.idle.push_back({ptr, block->second.bytes, block->second.device, false, until});
             g_pool.idleBytes += block->second.bytes;
             g_pool.used.erase(block);
-            return g_pool.releaseOld();
+            const hipError_t e = g_pool.releaseOld();
+            if(!g_pool.idle.empty()) { releaseIdleAt(until); }
+            return e;
         }
     }
     return hipFree(ptr);

@@ -119,25 +119,40 @@ int waitForFlag(const uint32_t *flag, uint32_t seq, hipStream_t stream)
     return GENNMI_OK;
 }
 
-// ---- pinned host memory, kept for reuse.  At most PINNED_KEPT bytes lie idle; what exceeds that is given back to the system at once,
-// and everything idle is when an allocation fails.
+// ---- pinned host memory, kept for reuse.  At most PINNED_KEPT bytes lie idle, each block as long as idle device memory does
+// (genn_mi355x_idle.h); what exceeds that is given back to the system at once, and everything idle is when an allocation fails.
 constexpr size_t PINNED_KEPT = size_t(256) << 20, PINNED_UNIT = 4096;
+struct PinnedIdle { uintptr_t address; IdleTime until; };
 std::mutex g_pinnedMutex;
 std::map<uintptr_t, size_t> g_pinned;                   // every block in use or idle: address, bytes
-std::multimap<size_t, uintptr_t> g_pinnedIdle;          // the idle ones by size
+std::multimap<size_t, PinnedIdle> g_pinnedIdle;         // the idle ones by size
 size_t g_pinnedIdleBytes = 0;
 
-hipError_t releaseIdlePinned()
+// (mutex held) gives the idle blocks that are due at `now` back to the system; when the next one is
+hipError_t releaseIdlePinned(IdleTime now = IdleTime::max(), IdleTime *next = nullptr)
 {
     hipError_t e = hipSuccess;
-    for(const auto &b : g_pinnedIdle) {
-        const hipError_t f = hipHostFree(reinterpret_cast<void*>(b.second));
+    for(auto b = g_pinnedIdle.begin(); b != g_pinnedIdle.end(); ) {
+        if(b->second.until > now) {
+            if(next) { *next = std::min(*next, b->second.until); }
+            ++b;
+            continue;
+        }
+        const hipError_t f = hipHostFree(reinterpret_cast<void*>(b->second.address));
         if(f != hipSuccess) { e = f; }
-        g_pinned.erase(b.second);
+        g_pinned.erase(b->second.address);
+        g_pinnedIdleBytes -= b->first;
+        b = g_pinnedIdle.erase(b);
     }
-    g_pinnedIdle.clear();
-    g_pinnedIdleBytes = 0;
     return e;
+}
+
+IdleTime pinnedReleaseOld()
+{
+    std::lock_guard<std::mutex> lock(g_pinnedMutex);
+    IdleTime next = IdleTime::max();
+    if(releaseIdlePinned(IdleClock::now(), &next) != hipSuccess) { (void)hipGetLastError(); }
+    return next;
 }
 
 int pinnedMalloc(void **ptr, size_t bytes)
@@ -146,7 +161,7 @@ int pinnedMalloc(void **ptr, size_t bytes)
     std::lock_guard<std::mutex> lock(g_pinnedMutex);
     const auto idle = g_pinnedIdle.lower_bound(bytes);
     if(idle != g_pinnedIdle.end() && idle->first <= bytes + bytes / 4) {
-        *ptr = reinterpret_cast<void*>(idle->second);
+        *ptr = reinterpret_cast<void*>(idle->second.address);
         g_pinnedIdleBytes -= idle->first;
         g_pinnedIdle.erase(idle);
         return GENNMI_OK;
@@ -170,13 +185,15 @@ bool pinnedFree(void *ptr, hipError_t *error)
     std::lock_guard<std::mutex> lock(g_pinnedMutex);
     const auto block = g_pinned.find(reinterpret_cast<uintptr_t>(ptr));
     if(block == g_pinned.end()) { return false; }
-    if(g_pinnedIdleBytes + block->second > PINNED_KEPT) {
+    const IdleTime until = idleUntil();
+    if(g_pinnedIdleBytes + block->second > PINNED_KEPT || until <= IdleClock::now()) {
         g_pinned.erase(block);
         *error = hipHostFree(ptr);
         return true;
     }
-    g_pinnedIdle.emplace(block->second, block->first);
+    g_pinnedIdle.emplace(block->second, PinnedIdle{block->first, until});
     g_pinnedIdleBytes += block->second;
+    releaseIdleAt(until);
     return true;
 }
 

@@ -298,6 +298,12 @@ class Array:
             self._dev = C.c_void_p()
 
 
+def release_cached_memory():
+    """Gives the system back what the library keeps of freed arrays for the next model (device memory, pinned host memory).  By itself it
+    does so ten seconds after they were freed (GENNMI_POOL_SECONDS; 0: at once)."""
+    _abi.check(_abi.load().gennmi_release_cached_memory())
+
+
 def pull_arrays(runner, arrays):
     """Device to host copies of several arrays: behind the runner's steps, with one wait for all of them."""
     arrays = [a for a in arrays if a._make_view().nbytes]

@@ -85,7 +85,8 @@ int gennmi_malloc(void **devPtr, size_t bytes);                 /* Array::alloca
 int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr);
 int gennmi_host_free(void *hostPtr);
 /* The same memory, not cleared, for a host side that is about to be written whole; a caller that is refused it does as well with
- * memory of its own, which every copy takes.  Pinned memory without zeroCopy is kept for reuse when it is freed (up to 256 MiB of it). */
+ * memory of its own, which every copy takes.  Pinned memory without zeroCopy is kept for reuse when it is freed (up to 256 MiB of
+ * it, as long as freed device memory is). */
 int gennmi_host_acquire(void **hostPtr, size_t bytes);
 int gennmi_free(void *devPtr);                                  /* Array::free      hip/backend.cc:110-128 */
 int gennmi_memcpy_to_device(void *dev, const void *host, size_t bytes);    /* pushToDevice / pushSlice1DToDevice   :130-176 */
@@ -139,8 +140,8 @@ int gennmi_mirrors_begin_initialisation(void);
 int gennmi_mirror_device_initialised(const void *host);
 int gennmi_mirror_ensure_host(const void *host);
 /* Blocks of device memory that were freed are kept for the next allocation of their size: at most 1/32 of the card's memory in all,
- * each for at most ten seconds of idleness; the bytes reported free include them.  This gives all of them back to the
- * system, and the idle pinned memory (freed host sides, staging of copies) with them. */
+ * each for ten seconds (GENNMI_POOL_SECONDS; 0: none), after which a thread of the library's gives it back; the bytes reported
+ * free include them.  This gives all of them back to the system, and the idle pinned memory (freed host sides, staging of copies) with them. */
 int gennmi_release_cached_memory(void);
 int gennmi_free_device_memory_bytes(size_t *bytes);
 /* Named ranges for profilers around stepTime / updateSynapses / updateNeurons (BackendBase::genPushProfilerRange /

@@ -1,12 +1,14 @@
 """Device memory kept between models, and the segment boundaries built with the tables of a new one."""
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
+import torch
 
 from genn_amd import _abi, configs
-from genn_amd.genn_model import Array, GeNNModel, init_postsynaptic, init_weight_update, model_from_net
+from genn_amd.genn_model import Array, GeNNModel, init_postsynaptic, init_weight_update, model_from_net, release_cached_memory
 
 pytestmark = pytest.mark.gpu
 MIB = 1 << 20
@@ -105,3 +107,45 @@ def test_tile_path_sums_at_row_and_tile_edges(n_trg, tile_floats, row_len, monke
     np.add.at(want, post, weights)
     assert np.array_equal(s.vars["outPost"].pull_from_device(), want)
     m.unload()
+
+
+def _gib_in_use():
+    """Device memory in use, in whole GiB over or under a start: the runtime's own few MiB come and go between two looks."""
+    free, total = torch.cuda.mem_get_info()
+    return (total - free) / 1024.0 ** 3
+
+
+def test_kept_memory_goes_back_by_itself(monkeypatch):
+    """A process that frees and then does nothing gives kept memory back when its time has come; what is asked for before is a kept block."""
+    _abi.check(_abi.load().gennmi_init(0))
+    release_cached_memory()
+    before, size = _gib_in_use(), 1024 * MIB
+    monkeypatch.setenv("GENNMI_POOL_SECONDS", "0.5")
+    lib = _abi.load()
+    kept = _malloc(lib, size)
+    _abi.check(lib.gennmi_free(kept))
+    assert round(_gib_in_use() - before) == 1
+    again = _malloc(lib, size)
+    assert again.value == kept.value
+    time.sleep(0.7)             # (in use: its time does not run)
+    assert round(_gib_in_use() - before) == 1
+    _abi.check(lib.gennmi_free(again))
+    deadline = time.monotonic() + 20.0
+    while round(_gib_in_use() - before) and time.monotonic() < deadline:
+        time.sleep(0.05)
+    assert round(_gib_in_use() - before) == 0
+    monkeypatch.setenv("GENNMI_POOL_SECONDS", "0")
+    _abi.check(lib.gennmi_free(_malloc(lib, size)))
+    assert round(_gib_in_use() - before) == 0
+
+
+def test_release_cached_memory_gives_everything_back():
+    _abi.check(_abi.load().gennmi_init(0))
+    release_cached_memory()
+    before = _gib_in_use()
+    arrays = [Array(64 << 20, np.float32, fill=1.0) for _ in range(4)]
+    for a in arrays:
+        a.free()
+    assert round(_gib_in_use() - before) == 1
+    release_cached_memory()
+    assert round(_gib_in_use() - before) == 0
