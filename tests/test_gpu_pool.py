@@ -8,7 +8,8 @@ import pytest
 import torch
 
 from genn_amd import _abi, configs
-from genn_amd.genn_model import Array, GeNNModel, init_postsynaptic, init_weight_update, model_from_net, release_cached_memory
+from genn_amd.genn_model import (Array, GeNNModel, init_postsynaptic, init_sparse_connectivity, init_var, init_weight_update, model_from_net,
+                                 release_cached_memory)
 
 pytestmark = pytest.mark.gpu
 MIB = 1 << 20
@@ -65,20 +66,51 @@ def test_kept_blocks_under_threads():
     assert not failures
 
 
-def test_models_one_after_another_are_the_same():
-    """A model built from kept blocks (full of the last one's values) runs as the first one did."""
-    net = configs.plastic_stdp(n=5000, n_src=50, steps=60, fan=400, src_fan=100)
-    runs = []
-    for _ in range(3):
-        m = model_from_net(net)
-        m.load(num_recording_timesteps=60)
-        m.run(60)
+def _pooled(m):
+    return {v.ptr for g in (m.neuron_populations, m.synapse_populations) for p in g.values() for v in p.vars.values() if v.count * v.dtype.itemsize >= 2 * MIB}
+
+
+def _plastic(seed):
+    return model_from_net(configs.plastic_stdp(n=5000, n_src=50, steps=60, fan=400, src_fan=100, seed=seed)), 60
+
+
+def _device_made(seed):
+    """Matrices made on the device, rows of different lengths (what lies behind a row's end is nobody's); sums of halves, exact in any order."""
+    m = GeNNModel("float", "made", dt=1.0)
+    m.seed = seed
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.55, TauRefrac=5.0)
+    pops = {k: m.add_neuron_population(k, n, "LIF", lif, {"V": init_var("Uniform", {"min": -60.0, "max": -50.0}), "RefracTime": 0.0})
+            for k, n in (("E", 20000), ("I", 5003))}
+    for src, w in (("E", 0.5), ("I", -2.0)):
+        for trg in "EI":
+            m.add_synapse_population(src + trg, "SPARSE", pops[src], pops[trg], init_weight_update("StaticPulse", {}, {"g": init_var("Constant", {"constant": w})}),
+                                     init_postsynaptic("DeltaCurr"), init_sparse_connectivity("FixedProbability", {"prob": 0.015}))
+    for p in pops.values():
+        p.spike_recording_enabled = True
+    m.build()
+    return m, 60
+
+
+@pytest.mark.parametrize("model", [_plastic, _device_made])
+def test_models_one_after_another_are_the_same(model):
+    """A model built from kept blocks that are full of another one's values (its indices are in range here) runs as the first one did."""
+    release_cached_memory()
+    runs, blocks = [], []
+    for seed in (99, 100, 99, 101, 99):
+        m, steps = model(seed)
+        m.load(num_recording_timesteps=steps)
+        m.run(steps)
         m.pull_recording_buffers_from_device()
         runs.append([p.vars["recordSpk"].view.copy() for p in m.neuron_populations.values()])
+        blocks.append(_pooled(m))
         m.unload()
-    assert sum(int(a.sum() != 0) for a in runs[0]) > 0
-    for r in runs[1:]:
-        assert all(np.array_equal(a, b) for a, b in zip(runs[0], r))
+    first, others = runs[0], (runs[1], runs[3])
+    assert sum(int(a.sum() != 0) for a in first) > 0
+    for r in (runs[2], runs[4]):
+        assert all(np.array_equal(a, b) for a, b in zip(first, r))
+    for r in others:            # (another model indeed, in the same blocks)
+        assert any(not np.array_equal(a, b) for a, b in zip(first, r))
+    assert blocks[0] and all(b & blocks[0] for b in blocks[1:])
 
 
 @pytest.mark.parametrize("n_trg, tile_floats", [(1, 16), (63, 16), (64, 16), (100, 7), (4097, 1024), (3000, 1000)])
