@@ -197,7 +197,7 @@ class Array:
         self._model, self._pinned = model, pinned
         self._dev = C.c_void_p()
         _abi.check(_abi.load().gennmi_malloc(C.byref(self._dev), self.count * self.dtype.itemsize))
-        self._view = None
+        self._view = self._host_address = None
         fill = None if fill is None else np.asarray(fill, dtype=self.dtype)
         self._fill, self._given = fill, False
         # (one first value of all elements is written on the device; the host copy is made when somebody asks for it)
@@ -216,6 +216,8 @@ class Array:
         if self._view is None:
             if self._given:
                 self.pull_from_device()
+            elif self._fill is None and not self._pinned:
+                self._view = np.zeros(self.count, dtype=self.dtype)
             else:
                 self._make_view()[:] = 0 if self._fill is None else self._fill
         return self._view
@@ -230,15 +232,15 @@ class Array:
                     pass        # (no pinned memory to be had: ordinary memory is copied more slowly)
             if self._view is None:
                 self._view = np.empty(self.count, dtype=self.dtype)
-            self._host_address = self._view.ctypes.data
         return self._view
 
     @property
     def host_address(self):
-        """Where the host side lies (asked of numpy once: a microsecond each time)."""
-        if self._view is None:
-            self.view
-        return self._host_address
+        """Where the host side lies (asked of numpy once: it takes a microsecond)."""
+        address = self._host_address
+        if address is None:
+            address = self._host_address = self.view.ctypes.data
+        return address
 
     @property
     def ptr(self):
@@ -363,10 +365,11 @@ class NeuronGroup:
             pull_arrays(model._runner, [count, spk])
         else:
             # (the counts and each batch's valid entries, which lie in these arrays as the call writes them)
-            _abi.check(_abi.load().gennmi_runner_pull_spikes(model._runner, count._dev, spk._dev, n, 1, 0, count.host_address, spk.host_address))
-        counts, ids = count.view.reshape(-1, slots), spk.view.reshape(-1, slots, n)
-        slot = model.timestep % slots
-        return [ids[b, slot, :counts[b, slot]].copy() for b in range(model.batch_size)]
+            rc = _abi.load().gennmi_runner_pull_spikes(model._runner, count._dev, spk._dev, n, 1, 0, count.host_address, spk.host_address)
+            if rc:
+                _abi.check(rc)
+        counts, ids = count._view.tolist(), spk._view
+        return [ids[q * n:q * n + counts[q]].copy() for q in range(model.timestep % slots, len(counts), slots)]
 
 
 class CurrentSource:
@@ -673,8 +676,9 @@ class GeNNModel:
                     a.view[:] = np.broadcast_to(init, (B, N)).reshape(-1) if init.ndim < 2 else init.reshape(-1)
                     a.push_to_device()
                     n.vars[v] = a
-            n.vars["spkCnt"] = self._alloc(B * n.num_delay_slots, np.uint32, pinned=True)
-            n.vars["spk"] = self._alloc(B * n.num_delay_slots * N, np.uint32, pinned=True)
+            # (host sides in ordinary memory: current_spikes copies the few entries that are valid, and pinning takes 70 us and 0.4 ms a MiB)
+            n.vars["spkCnt"] = self._alloc(B * n.num_delay_slots, np.uint32)
+            n.vars["spk"] = self._alloc(B * n.num_delay_slots * N, np.uint32)
             for s in n.pre_output_syn:
                 s.vars["outPre"] = self._alloc(B * N, np.float32, pinned=True)
             for e in range(len(n.event_thresholds)):
