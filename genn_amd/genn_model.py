@@ -199,7 +199,7 @@ class Array:
         _abi.check(_abi.load().gennmi_malloc(C.byref(self._dev), self.count * self.dtype.itemsize))
         self._view = self._host_address = None
         fill = None if fill is None else np.asarray(fill, dtype=self.dtype)
-        self._fill, self._given = fill, False
+        self._fill, self._given = fill, None
         # (one first value of all elements is written on the device; the host copy is made when somebody asks for it)
         if device_only or not self.count:
             pass
@@ -214,8 +214,10 @@ class Array:
     @property
     def view(self):
         if self._view is None:
-            if self._given:
+            if self._given is not None and self._dev:
                 self.pull_from_device()
+            elif self._given is not None:
+                self._make_view()[:] = self._given.reshape(-1)
             elif self._fill is None and not self._pinned:
                 self._view = np.zeros(self.count, dtype=self.dtype)
             else:
@@ -623,9 +625,10 @@ class GeNNModel:
         return a
 
     def _alloc_given(self, values):
-        """An array the device only reads, from the user's values; its own host copy is pulled when somebody asks for it."""
+        """An array the device only reads, from the user's values; its own host copy is pulled when somebody asks for it (or, when the
+        device's is gone, made from those values)."""
         a = self._alloc(values.size, values.dtype, device_only=True)
-        a._given = True
+        a._given = values
         if values.nbytes:
             _abi.check(_abi.load().gennmi_runner_push(self._runner, a._dev, values.ctypes.data, values.nbytes))
         return a

@@ -134,3 +134,18 @@ def test_a_refused_host_side_is_ordinary_memory(make_model, monkeypatch):
     a.push_to_device()
     assert np.array_equal(a.pull_slice(0, 1000), a.view)
     a.free()
+
+
+@pytest.mark.parametrize("looked_at_before", [False, True])
+def test_given_values_are_there_after_unload(looked_at_before):
+    m = genn_model.GeNNModel("float", "noise", dt=1.0)
+    pop = m.add_neuron_population("N", 40, "LIF", dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.0, TauRefrac=5.0), {"V": -60.0, "RefracTime": 0.0})
+    noise = np.random.default_rng(5).random((3, 40)).astype(np.float32)
+    source = m.add_current_source("noise", "ArrayNoise", pop)
+    source.set_extra_global_param("noise", noise)
+    m.build()
+    m.load()
+    if looked_at_before:
+        assert np.array_equal(source.vars["noise"].view, noise.reshape(-1))
+    m.unload()
+    assert np.array_equal(source.vars["noise"].view, noise.reshape(-1))
