@@ -324,7 +324,7 @@ void presynapticDenseKernel(const DenseGroupDev * __restrict__ blocks, unsigned 
 // connectivity: the only memory traffic of an event is its atomic.
 // What bounds it is the chain of arithmetic that makes a row (generator, logarithms, scan, division).  Nothing in it may index a
 // private array by a run-time number: the compiler then keeps such arrays in LDS (16 KB of a work-group's, and an access on
-// the chain each time); without that a step of 41 spikes x 1000 targets takes 9.4 us instead of 20.3.
+// the chain each time); without that a step of 41 spikes x 1000 targets takes 8.8 us instead of 17.8.
 // ------------------------------------------------------------------------------------------------
 struct ProcGroupDev
 {
@@ -589,7 +589,7 @@ __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float
     // What the presynaptic-spike rule takes off a synapse depends on its target alone (times, trace and constants): in a busy step a block works
     // it out once per target of its tile and keeps it in LDS behind the tile, with the targets' bits of the spike bitmap.  Three gathers
     // over the chip's memory per synapse, a cache line each, are what a burst otherwise spends its time on (and, under the
-    // additive rule, an exponential in double).  A burst of 4 x 10^7 events: 424 -> 295 us.
+    // additive rule, an exponential in double).  A burst of 4 x 10^7 events: 403 -> 298 us.
     float *shFactor = shTile + G.tileSize;
     uint32_t *shFired = reinterpret_cast<uint32_t*>(shFactor + G.tileSize);
     const bool factors = stdp && G.factorEvents != 0u && (unsigned long long)numSpikes * G.segLength >= G.factorEvents;
@@ -804,8 +804,8 @@ void presynapticConvTileKernel(const ConvTileDev * __restrict__ blocks, unsigned
 }
 
 // Segment boundaries of every row for the tile kernel; also verifies that rows are sorted by target.  A wavefront takes a row,
-// 64 consecutive synapses at a time (one lane per row read every row's entries one dependent access after another: 0.16 ms for
-// 2 x 10^7 synapses, now 0.03).  The lane whose synapse is the first one at or beyond a boundary writes it.  `shift`: log2 of the tile
+// 64 consecutive synapses at a time (one lane per row read every row's entries one dependent access after another: 0.31 ms for 80,000
+// rows of 800, now 0.09).  The lane whose synapse is the first one at or beyond a boundary writes it.  `shift`: log2 of the tile
 // size, or 32 if it is no power of two.  Rows beyond the grid's wavefronts come in further rounds: a launch holds fewer than 2^32
 // threads, which a wavefront a row would exceed from 2^26 rows on.
 constexpr uint32_t TILE_OFFSET_BLOCKS = 1u << 20;

@@ -3,12 +3,12 @@
 // Copies between host arrays and device arrays in the order of a runner's steps.
 //
 // What a copy costs here is waiting, not bytes.  hipMemcpy runs on the null stream: behind a kernel on another (blocking)
-// stream it took 43 us for 4 bytes (two queues made to wait for each other), a copy command on the kernel's own stream and a
-// wait for it 15 us, and what this file does 10 us: a copy kernel on the runner's stream that moves the bytes to or from
+// stream it takes 41 us for 4 bytes (two queues made to wait for each other), a copy command on the idle stream of its own and a wait
+// for it 23 us, and what this file does 9 us (16 behind a step that takes 15 by itself): a copy kernel on the runner's stream that moves the bytes to or from
 // pinned host memory and then stores a number the host spins on.
 //
-// Host arrays that are copied again and again (state, spike queues, recordings, spike times) are pinned and copied in one
-// launch at the rate of PCIe (16 MB: 302 us either way).  Pinned memory is kept for the next model when a model gives it
+// Host arrays that are copied again and again (state, recordings, spike times) are pinned and copied in one
+// launch at the rate of PCIe (16 MB: 304 us to the host, 310 from it).  Pinned memory is kept for the next model when a model gives it
 // back: touching it for the first time costs 0.4 ms per MiB.  Other host memory goes through a small ring of pinned chunks
 // on its way from the device — while the device moves one chunk, the host copies the one before it: 13 MB in 0.5 ms, by
 // hipMemcpy 0.8 ms — and by the runtime's own copy on its way there (it reads pageable memory in place: 13 MB in 0.4 ms).
@@ -21,7 +21,7 @@ namespace
 constexpr size_t TRANSFER_CHUNK = size_t(1) << 20;      // 18 us of PCIe time: long against a launch, short against a megabyte-sized array
 constexpr uint32_t TRANSFER_SLOTS = 4;
 constexpr uint32_t TRANSFER_BLOCKS = 32;                // (16 MB from the device with 16 / 32 / 64 / 128 work-groups: 303 / 301 / 302 / 302 us, to it 301 / 311 / 304 / 311)
-constexpr size_t PUSH_RING_BYTES = size_t(128) << 10;   // pageable memory up to this size is pushed through the ring (64 KB: 12 against 35 us, 256 KB: 19 against 17)
+constexpr size_t PUSH_RING_BYTES = size_t(128) << 10;   // pageable memory up to this size is pushed through the ring (128 KB: 13 us; the runtime takes 20 from there up to 192, 35 for 64)
 
 // Stores that go through to memory.  Nothing then has to be written back before the host (or a kernel on another stream) may look:
 // waiting for the stores is enough, where a fence of the whole system in every wavefront made 1 MiB cost 25 us instead of 20.

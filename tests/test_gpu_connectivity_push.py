@@ -89,8 +89,8 @@ def test_rewritten_delays(ordered):
     on the single-launch step, where those synapses join the zero-delay lists (delivered by the spiking neuron's own
     wavefront) — the lists must be rebuilt, and the resident plan's segment tables with them; rasters must stay identical to
     the oracle's while reassociated sums allow (checked for 150 steps after the push; this network parts from the oracle
-    near step 343 in every default plan).  Ordered accumulation: the column views are rebuilt and the captured step graph,
-    which holds their addresses, is captured again; there the whole run must be identical bit for bit."""
+    near step 343 in every default plan).  Ordered accumulation: the column views are rebuilt, at other addresses; there the
+    whole run must be identical bit for bit."""
     net = configs.potjans(neuron_scale=0.05, connectivity_scale=1.0, steps=400)
     model = model_from_net(net, ordered=ordered)
     model.load(num_recording_timesteps=400)

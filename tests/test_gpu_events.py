@@ -84,7 +84,7 @@ def test_event_queues_across_many_blocks():
 
 
 def test_graded_synapses_through_run():
-    """The same network stepped by run() (replayed graphs of the separate launches) ends in the same state."""
+    """The same network stepped by run() (one call for all steps) ends in the same state."""
     net = configs.graded(steps=230)
     model = model_from_net(net)
     model.load(num_recording_timesteps=230)

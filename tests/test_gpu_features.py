@@ -220,7 +220,7 @@ def test_spike_source_arrays_rewritten_between_steps(replay):
     """The neuron update keeps the time of each source's next spike beside its state instead of gathering
     spikeTimes[startSpike] every step; that copy must follow the user's arrays.  After 25 steps the host rewinds startSpike
     and shifts spikeTimes by 30 ms (the way new input is fed to a SpikeSourceArray): the same pattern must come out again,
-    30 steps later, through single steps and through replayed graphs."""
+    30 steps later, through single steps and through run()."""
     n, first = 300, 25
     rng = np.random.default_rng(12)
     per = rng.integers(0, 4, n)                                  # 0..3 spikes per source

@@ -1,7 +1,7 @@
 """GPU parity at the full sizes the throughput figures are quoted on.
 
 Each network is generated at its published size, run for (at least) its first 100 ms of simulated time
-through the captured-graph path (`run`) — the path the benchmark times — and compared with the CPU
+through `run` — what the benchmark times — and compared with the CPU
 oracle run over the same steps:
 
 * the recorded spike raster (every neuron, every step) must be identical bit for bit,

@@ -318,14 +318,14 @@ def test_plastic_batches_are_independent(rule, combined, monkeypatch):
 def test_axonal_delays(span):
     """Balanced LIF network with axonal delays of 3, 1, 0 and 5 timesteps: the spike queue of a population is a ring of
     slots (4 for E, 6 for I) and every projection reads the slot its delay selects.  One weight per outPost, so the whole
-    state must be identical to the oracle's, stepped one launch at a time and through graph replay."""
+    state must be identical to the oracle's, stepped one call at a time and through run()."""
     delays = {"EE": 3, "EI": 1, "IE": 0, "II": 5}
     net = configs.vogels_abbott(n=2000, steps=600, p=0.04, axonal_delays=delays)
     model, oracle, counts = run_side_by_side(net, check_every=100, exact=True, span=span)
     assert counts["E"] > 300 and counts["I"] > 50
     info = model.runner_info()
     assert not info["resident_plan"] and not info["single_launch_step"]
-    # the same network through run(): graph replays of the two-launch step
+    # the same network through run(): two launches a step
     replay = model_from_net(net, span=span)
     replay.load(num_recording_timesteps=600)
     replay.run(600)
@@ -397,7 +397,7 @@ def test_dense_projection_batched():
 @pytest.mark.parametrize("resident", ["1", "0"])
 def test_graph_replay_matches_stepping(resident, monkeypatch):
     """run() either keeps the network resident on the chip for the whole chunk (one launch) or, with that plan switched
-    off, replays captured HIP graphs; either way every chunk must leave the state eager stepping leaves.
+    off, launches step by step; either way every chunk must leave the state eager stepping leaves.
     Chunks are interleaved with eager steps and synchronisations."""
     monkeypatch.setenv("GENNMI_RESIDENT", resident)
     net = configs.vogels_abbott(n=2000, steps=730, p=0.04)
@@ -406,7 +406,7 @@ def test_graph_replay_matches_stepping(resident, monkeypatch):
     graph = model_from_net(net)
     graph.load(num_recording_timesteps=net.steps)
     assert graph.runner_info()["resident_plan"] == (resident == "1")
-    for chunk in (250, 3, 200, 77, 200):           # 200/250 -> graph replays (+ remainder), 3/77 -> single steps
+    for chunk in (250, 3, 200, 77, 200):           # (3: fewer than a resident launch takes)
         graph.run(chunk)
         graph.synchronize()
         for _ in range(chunk):
@@ -431,7 +431,7 @@ def test_graph_replay_matches_stepping(resident, monkeypatch):
 
 @pytest.mark.parametrize("resident", ["1", "0"])
 def test_graph_replay_single_launch_step(resident, monkeypatch):
-    """Chunks of steps of a dendritic-delay network — resident plan, or graph replay of the one-launch-per-step plan —
+    """Chunks of steps of a dendritic-delay network — resident plan, or the one-launch-per-step plan —
     against eager stepping (one launch per step, which hands front-slot synapses over one step early) and the oracle:
     rasters identical, membrane potentials within tolerance (weights differ, so the order of additions may differ)."""
     monkeypatch.setenv("GENNMI_RESIDENT", resident)
