@@ -181,3 +181,71 @@ def test_release_cached_memory_gives_everything_back():
     assert round(_gib_in_use() - before) == 1
     release_cached_memory()
     assert round(_gib_in_use() - before) == 0
+
+
+def test_memory_goes_back_while_models_step_and_threads_allocate(monkeypatch):
+    """The thread that gives blocks back runs beside steps, copies and allocations: nobody's values change."""
+    monkeypatch.setenv("GENNMI_POOL_SECONDS", "0.01")
+    m, steps = _device_made(99)
+    m.load(num_recording_timesteps=steps)
+    m.run(steps)
+    m.pull_recording_buffers_from_device()
+    want = [p.vars["recordSpk"].view.copy() for p in m.neuron_populations.values()]
+    m.unload()
+    failures, stop = [], threading.Event()
+
+    def work(k):
+        rng = np.random.default_rng(k)
+        while not stop.is_set():
+            count = int(rng.integers(600_000, 2_000_000))
+            a = Array(count, np.float32, fill=float(k), pinned=True)
+            a.pull_from_device()
+            if not (a.view[0] == a.view[-1] == k):
+                failures.append(k)
+            a.free()
+            time.sleep(float(rng.uniform(0.0, 0.02)))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    try:
+        for _ in range(8):
+            m, _ = _device_made(99)
+            m.load(num_recording_timesteps=steps)
+            for _ in range(steps):
+                m.step_time()
+            m.pull_recording_buffers_from_device()
+            assert all(np.array_equal(p.vars["recordSpk"].view, w) for p, w in zip(m.neuron_populations.values(), want))
+            m.unload()
+    finally:
+        stop.set()
+        for t in threads:
+            t.join()
+    assert not failures
+
+
+def test_memory_goes_back_beside_a_capture(monkeypatch):
+    """Giving a block back waits for the device, which a stream that somebody is capturing must not notice."""
+    _abi.check(_abi.load().gennmi_init(0))
+    release_cached_memory()
+    lib, size = _abi.load(), 1024 * MIB
+    x = torch.arange(1000, dtype=torch.float32, device="cuda")
+    y = x * 2.0                 # (compiled and allocated before the capture)
+    torch.cuda.synchronize()
+    before = _gib_in_use()
+    monkeypatch.setenv("GENNMI_POOL_SECONDS", "0.3")
+    kept = _malloc(lib, size)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _abi.check(lib.gennmi_free(kept))       # (kept, not freed: nothing of the runtime's is called)
+        time.sleep(0.8)
+        y = x * 3.0
+    deadline = time.monotonic() + 20.0
+    while round(_gib_in_use() - before) and time.monotonic() < deadline:
+        time.sleep(0.05)
+    assert round(_gib_in_use() - before) == 0
+    for k in range(3):
+        x.fill_(float(k))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.all(y == 3.0 * k)
