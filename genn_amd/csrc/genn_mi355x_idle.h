@@ -15,11 +15,11 @@ namespace
 using IdleClock = std::chrono::steady_clock;
 using IdleTime = IdleClock::time_point;
 
-// until when memory freed now is kept
-IdleTime idleUntil()
+// until when memory freed now is kept (times as long as device memory is)
+IdleTime idleUntil(double times = 1.0)
 {
     const char *e = getenv("GENNMI_POOL_SECONDS");
-    const double seconds = e ? std::min(1e6, std::max(0.0, atof(e))) : 10.0;
+    const double seconds = times * (e ? std::min(1e6, std::max(0.0, atof(e))) : 10.0);
     return IdleClock::now() + std::chrono::duration_cast<IdleClock::duration>(std::chrono::duration<double>(seconds));
 }
 

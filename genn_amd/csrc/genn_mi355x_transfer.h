@@ -119,9 +119,12 @@ int waitForFlag(const uint32_t *flag, uint32_t seq, hipStream_t stream)
     return GENNMI_OK;
 }
 
-// ---- pinned host memory, kept for reuse.  At most PINNED_KEPT bytes lie idle, each block as long as idle device memory does
-// (genn_mi355x_idle.h); what exceeds that is given back to the system at once, and everything idle is when an allocation fails.
+// ---- pinned host memory, kept for reuse.  At most PINNED_KEPT bytes lie idle, each block six times as long as idle device memory
+// does (genn_mi355x_idle.h): a byte of it takes a thousand times as long to make.  Given back after ten seconds as well, loads
+// that far apart took 0.25 ms longer (2.0 against 1.75 of a small network).  What exceeds PINNED_KEPT is given back to the system at
+// once, and everything idle is when an allocation fails.
 constexpr size_t PINNED_KEPT = size_t(256) << 20, PINNED_UNIT = 4096;
+constexpr double PINNED_TIMES = 6.0;
 struct PinnedIdle { uintptr_t address; IdleTime until; };
 std::mutex g_pinnedMutex;
 std::map<uintptr_t, size_t> g_pinned;                   // every block in use or idle: address, bytes
@@ -185,7 +188,7 @@ bool pinnedFree(void *ptr, hipError_t *error)
     std::lock_guard<std::mutex> lock(g_pinnedMutex);
     const auto block = g_pinned.find(reinterpret_cast<uintptr_t>(ptr));
     if(block == g_pinned.end()) { return false; }
-    const IdleTime until = idleUntil();
+    const IdleTime until = idleUntil(PINNED_TIMES);
     if(g_pinnedIdleBytes + block->second > PINNED_KEPT || until <= IdleClock::now()) {
         g_pinned.erase(block);
         *error = hipHostFree(ptr);

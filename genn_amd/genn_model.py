@@ -304,7 +304,7 @@ class Array:
 
 def release_cached_memory():
     """Gives the system back what the library keeps of freed arrays for the next model (device memory, pinned host memory).  By itself it
-    does so ten seconds after they were freed (GENNMI_POOL_SECONDS; 0: at once)."""
+    does so ten seconds after they were freed (GENNMI_POOL_SECONDS; 0: at once), a minute for the pinned memory."""
     _abi.check(_abi.load().gennmi_release_cached_memory())
 
 

@@ -86,7 +86,7 @@ int gennmi_host_malloc(void **hostPtr, size_t bytes, int zeroCopy, void **devPtr
 int gennmi_host_free(void *hostPtr);
 /* The same memory, not cleared, for a host side that is about to be written whole; a caller that is refused it does as well with
  * memory of its own, which every copy takes.  Pinned memory without zeroCopy is kept for reuse when it is freed (up to 256 MiB of
- * it, as long as freed device memory is). */
+ * it, six times as long as freed device memory is). */
 int gennmi_host_acquire(void **hostPtr, size_t bytes);
 int gennmi_free(void *devPtr);                                  /* Array::free      hip/backend.cc:110-128 */
 int gennmi_memcpy_to_device(void *dev, const void *host, size_t bytes);    /* pushToDevice / pushSlice1DToDevice   :130-176 */
