@@ -83,12 +83,13 @@ def test_izhikevich_full_run():
     This network fires in population bursts, about one spike per neuron each and a dozen per second, and parts from the
     oracle at the first of them (step 66: a threshold crossing flipped by the order of fp32 atomic additions).  Whether the
     window's last burst falls inside it then moves the rate over the configuration's one simulated second by a few
-    per cent from run to run of the very same kernels (three runs: 0.45 %, 2.5 % and 3.1 % from the oracle), and the
-    intervals between bursts vary from run to run as well: over four seconds (some fifty bursts) two runs of the same
-    build were 0.4 % and 2.0 % from the oracle.  A 2 % gate on this configuration would fail every other run for a reason
-    that has nothing to do with the kernels, so the rate over four seconds is held to 5 % and the first second to 8 %
-    (one burst's worth); what pins the arithmetic of this configuration is the lock-step comparison and the bit-identical
-    ordered run of test_gpu_full_size.py."""
+    per cent from run to run of the very same kernels, and the intervals between bursts vary as well: the rates of single
+    seconds are independent and have a standard deviation of 2.2 %.  240 runs of two builds, alike in both: over four
+    seconds +0.9 % from the oracle's one run on average, standard deviation 1.1 %, -1.9 to +4.5 % (and one of +5.5 % seen
+    elsewhere); over the first 0.0 %, 1.8 %, -3.4 to +4.6 %.  A 2 % gate would fail every fifth run for a reason that has
+    nothing to do with the kernels, so both are held to 8 %: the mean and six standard deviations of the one, more than
+    four of the other.  What pins the arithmetic of this configuration is the next test, and the lock-step comparison and
+    the bit-identical ordered run of test_gpu_full_size.py."""
     steps, second = 4000, 1000
     net = configs.izhikevich_fanout(steps=steps, noise_steps=1000)
     n = net.pops[0].n
@@ -105,15 +106,34 @@ def test_izhikevich_full_run():
     report = []
     for name, first, last, count in (("excitatory", 0, n_e // 32, n_e), ("inhibitory", n_e // 32, words, n - n_e)):
         per_step_got, per_step_want = _spikes_per_step(got, steps, words, first, last), _spikes_per_step(want, steps, words, first, last)
-        for label, upto, tol in (("first second", second, 0.08), ("four seconds", steps, 0.05)):
+        for label, upto, tol in (("first second", second, 0.08), ("four seconds", steps, 0.08)):
             rate_got, rate_want = per_step_got[:upto].sum() / count / (upto / 1000.0), per_step_want[:upto].sum() / count / (upto / 1000.0)
             report.append(f"{name} {label}: {rate_got:.3f} / {rate_want:.3f} Hz")
             assert rate_want > 1.0, f"{name} neurons are silent in the oracle"
             assert abs(rate_got - rate_want) <= tol * rate_want, f"{name}, {label}: {rate_got:.3f} Hz vs {rate_want:.3f} Hz"
-    # (every spike of this network is 1000 events: the event total is the rate over the four seconds under another name, and is
-    # held to the same 5 % — a third run of one build was 2.8 % above the oracle where the first two were 0.4 % and 2.0 %)
-    assert abs(model.synaptic_event_count - oracle.events()) <= 0.05 * oracle.events()
+    # (every spike of this network is 1000 events: the event total is the rate over the four seconds under another name)
+    assert abs(model.synaptic_event_count - oracle.events()) <= 0.08 * oracle.events()
     print(f"config 3: rasters identical for the first {identical_until} of {steps} steps; " + "; ".join(report), flush=True)
+    model.unload()
+
+
+def test_izhikevich_full_run_with_exact_sums():
+    """The same network with its weights rounded to multiples of 2^-8: inputs are sums of a thousand of them, below 2^16, and
+    exact in fp32 in any order.  Then nothing separates the default kernels (scatter path, tile path with its records, bulk
+    neuron update) from the oracle over the whole second: rasters, state and events are the same to the last bit."""
+    steps = 1000
+    net = configs.izhikevich_fanout(steps=steps, noise_steps=steps)
+    g = net.syns[0].g
+    np.rint(np.multiply(g, 256.0, out=g), out=g)
+    np.multiply(g, 1.0 / 256.0, out=g)
+    model, oracle = _full_run(net, steps)
+    words = (net.pops[0].n + 31) // 32
+    got, want = (np.ascontiguousarray(r).reshape(steps, words) for r in (model.neuron_populations["N"].vars["recordSpk"].view, oracle.record("N", steps)))
+    diff = np.nonzero((got != want).any(axis=1))[0]
+    assert len(diff) == 0, f"rasters differ from step {diff[0]}"
+    for k, name in enumerate(("V", "U")):
+        assert np.array_equal(model.neuron_populations["N"].vars[name].pull_from_device(), oracle.var("N", k)), name
+    assert model.synaptic_event_count == oracle.events() > 5 * 10 ** 9
     model.unload()
 
 
