@@ -94,7 +94,8 @@ struct gennmi_runner
     ResTile *dResTiles = nullptr; NeuronGroupDev *dResGroups = nullptr; uint8_t *dResTileGroup = nullptr;
     unsigned long long *dResTags = nullptr, *dResSide = nullptr;
     uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0;
-    decltype(&residentKernel<false, false>) resKernel = nullptr;     // the instantiation its sources and segment entries need
+    decltype(&residentKernel<false, false, 2, 1, 0>) resKernel = nullptr;     // the instantiation its sources and segment entries need
+    uint32_t resThreads = BLOCK;        // ... and its work-group
     std::vector<u32x4*> resSegs;        // segment table of each presynaptic group, in push order
     std::vector<uint32_t> resSegTiles;  // tiles of its target population
     std::vector<uint32_t> resSegWide;   // its entries are wide ones
@@ -777,25 +778,43 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     const size_t ldsBytes = std::max<size_t>(ldsFloatsMax, 1) * sizeof(float);
     if(ldsBytes > 96 * 1024) { return GENNMI_OK; }
     bool poisson = false;
+    uint32_t maxPSM = 0;
     for(const auto &n : r->neuron) {
+        maxPSM = std::max(maxPSM, n.g.numPSM);
         for(uint32_t c = 0; c < n.g.numCS; c++) { poisson = poisson || n.g.cs[c].kind == GENNMI_CS_POISSON_EXP; }
     }
     // Wide segment entries where a projection without a ring leaves a tile up to RES_WIDE_MEAN synapses of a row (rowStride is a little more than
-    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them.
+    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them, and not in the networks whose
+    // instances go without them (registers): those with rings, and those of more tiles than two a compute unit.
     constexpr uint32_t RES_WIDE_MEAN = 16;
-    auto wideEntries = [](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
+    bool anyWide = false, anyRing = false, onlyRings = true;
+    for(const auto &p : r->pre) { anyRing = anyRing || p.g.maxDenDelay != 0; onlyRings = onlyRings && p.g.maxDenDelay >= 2; }
+    const bool widePossible = !anyRing && tiles.size() <= 2 * BLOCK;
+    auto wideEntries = [widePossible](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
         const uint64_t mean = ((uint64_t)q.rowStride * RES_T + q.numTrgNeurons - 1) / q.numTrgNeurons;
-        return q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
+        return widePossible && q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
     };
-    bool anyWide = false;
     for(const auto &p : r->pre) { anyWide = anyWide || wideEntries(p.g, (p.g.numTrgNeurons + RES_T - 1) / RES_T); }
-    const auto residentInstance = poisson ? (anyWide ? residentKernel<true, true> : residentKernel<true, false>) : (anyWide ? residentKernel<false, true> : residentKernel<false, false>);
+    // The instantiation for the network's sources, segment entries, postsynaptic models and number of tiles.  Where every projection has
+    // a ring that puts its synapses off for later, wavefronts of their own walk them, as long as two such work-groups a compute unit hold the network.
+    constexpr uint32_t WALK = BLOCK / WAVE, MAX = GENNMI_MAX_PSM;
+    const bool few = tiles.size() <= BLOCK, some = tiles.size() <= 2 * BLOCK, walkers = onlyRings && some && maxPSM <= 2;
+    decltype(r->resKernel) residentInstance;
+    if(maxPSM > 2) { residentInstance = some ? residentKernel<true, true, MAX, 2, 0> : residentKernel<true, false, MAX, 4, 0>; }
+    else if(walkers) {
+        if(few) { residentInstance = poisson ? residentKernel<true, false, 2, 1, WALK> : residentKernel<false, false, 2, 1, WALK>; }
+        else { residentInstance = poisson ? residentKernel<true, false, 2, 2, WALK> : residentKernel<false, false, 2, 2, WALK>; }
+    }
+    else if(few) { residentInstance = poisson ? residentKernel<true, true, 2, 1, 0> : anyWide ? residentKernel<false, true, 2, 1, 0> : residentKernel<false, false, 2, 1, 0>; }
+    else if(some) { residentInstance = poisson ? residentKernel<true, true, 2, 2, 0> : anyWide ? residentKernel<false, true, 2, 2, 0> : residentKernel<false, false, 2, 2, 0>; }
+    else { residentInstance = poisson ? residentKernel<true, false, 2, 4, 0> : residentKernel<false, false, 2, 4, 0>; }
+    const uint32_t residentThreads = walkers ? BLOCK + WALK * WAVE : BLOCK;
     const void *kernel = reinterpret_cast<const void*>(residentInstance);
     if(ldsBytes > 32 * 1024) {
         HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
     }
     int perCU = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, BLOCK, ldsBytes));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, (int)residentThreads, ldsBytes));
     if((size_t)perCU * numCU < tiles.size()) { return GENNMI_OK; }
 
     // projections: source group, target group and postsynaptic model, segment table
@@ -899,6 +918,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     r->resTiles = (uint32_t)tiles.size();
     r->resLdsBytes = ldsBytes;
     r->resKernel = residentInstance;
+    r->resThreads = residentThreads;
     r->resident = true;
     return GENNMI_OK;
 }
@@ -935,7 +955,7 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
     for(unsigned long long done = 0; done < numSteps; ) {
         const uint32_t chunk = (uint32_t)std::min(MAX_STEPS, numSteps - done);
         const auto launch = r->resKernel;
-        launch<<<dim3(r->resTiles), dim3(BLOCK), r->resLdsBytes, r->stream>>>(
+        launch<<<dim3(r->resTiles), dim3(r->resThreads), r->resLdsBytes, r->stream>>>(
             r->dResTiles, r->resTiles, r->dResGroups, r->dResTileGroup, r->dResTags, r->dResSide, timestep + done, r->epoch, numRecordingTimesteps,
             chunk, r->dt, r->fusedStep ? 1u : 0u, r->dError, r->dEvents, r->resReplicaStride, r->resSeq);
         HIP_TRY(hipGetLastError());

@@ -27,7 +27,7 @@ constexpr uint32_t RES_T = BLOCK;            // neurons per tile = threads per w
 constexpr uint32_t RES_MAX_TILES = 1024;
 constexpr uint32_t RES_MAX_PROJ = 16;        // projections into one population
 constexpr uint32_t RES_MAX_GROUPS = 64;      // neuron groups
-constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs staged per pass
+constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs a tile lists per exchange
 constexpr uint32_t RES_FRONT_MAX = 4;        // front-slot synapses held inline in a segment entry
 // Without a ring every synapse of a row part is due at once.  Where the parts are short they go into the entry whole: up to four into 32
 // bytes, up to 24 into a wide entry of 128 — one cache line, read where 32 bytes of it were — and the step is spared the second trip to
@@ -35,7 +35,7 @@ constexpr uint32_t RES_FRONT_MAX = 4;        // front-slot synapses held inline 
 // (ordinary entries); 12,000 x 100 4.19 -> 4.00, 4,000 x 80 3.79 -> 3.62 (wide ones; 4.19 and 3.70 without).
 constexpr uint32_t RES_WIDE_QUADS = 8, RES_WIDE_MAX = 24;
 constexpr uint32_t RES_SEG_OVERFLOW = 1u << 24, RES_SEG_NO_DELAY = 1u << 25;
-constexpr uint32_t RES_PAIR_GROUP = 16;      // pairs a wavefront expands at a time
+constexpr uint32_t RES_SEG_PROJ_SHIFT = 26;  // in the kernel's list of pairs: the projection, above an entry's flags
 constexpr int RES_SEQ_SHIFT = 41;            // word = seq << 41 | count << 32 | up to four tile-local neuron indices, 8 bits each
 constexpr uint32_t RES_SEQ_MASK = (1u << (64 - RES_SEQ_SHIFT)) - 1u;    // sequence numbers run on from launch to launch, modulo 2^23
 constexpr uint32_t RES_WORD_IDS = 4;         // spikes of a tile and step that travel inside its word (more: side buffer)
@@ -150,10 +150,35 @@ __device__ __forceinline__ uint32_t waveInclusiveScanU32(uint32_t v, uint32_t la
     return v;
 }
 
+// Waits for the work-group with its LDS accesses done, and for nothing else: global loads and stores stay in flight.
+__device__ __forceinline__ void ldsBarrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The step is a chain of latencies, and what bounds it is the number of links: words arrive -> segment entries -> update -> word.
+// The thread that sees a tile's word reads the entries of that tile's spikes itself and adds what is due at once, so there
+// is one barrier in a step, between the words and the update (every due synapse is in); the wavefront that finishes the update last
+// publishes the tile's word.  The pairs are listed on the side, and the synapses that are not due are added by WALK wavefronts of
+// their own, between that barrier and the next one: a step lasts as long as the slowest tile takes around its loop, and time stamps
+// showed that tile never waiting for a word, but walking, polling, reading entries and updating one after the other.
+// us a step, with five barriers and the walk behind the word / now: the full microcircuit 6.1 / 4.4, with PoissonExp sources at half size
+// 5.3 / 3.4, balanced networks of 4,000 x 80 3.8 / 2.9, 100,000 x 80 7.2 / 5.9, 250,000 x 200 (four tiles a compute unit) 10.9 / 10.5.
+// (Spikes taken one after another by the thread that watches their word, however many: 180,000 x 100 10.1 -> 15.9.)
+// What consecutive exchanges share exists once for each of them: pair lists twice, counters and ring fronts four times (those of the
+// exchange after the next are prepared behind the barrier, so no thread meets them half prepared).
 // POISSON: some population has a PoissonExp current source (its state then lives in a register per source and neuron);
-// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection has wide entries
-template<bool POISSON, bool WIDE>
-__global__ __launch_bounds__(BLOCK)
+// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries.
+// NPSM: postsynaptic models of any group (their constants are wave-uniform: eight models' worth does not fit the scalar
+// registers, and what does not fit is read back lane by lane every step).  WATCH: source tiles a thread watches (up to WATCH x BLOCK
+// tiles); as many work-groups share a compute unit then, which is what the registers are budgeted for.  WALK: wavefronts beyond those that
+// own the tile's neurons; 0: these walk too, once they have published.  With walkers nothing holds a wavefront back between its
+// update and the next exchange, so every projection must have a ring of two slots or more: what an early wavefront adds then goes to another slot
+// than the one a late one is reading and clearing.  Without, a barrier behind the update keeps them apart, and inSyn itself can be added to.
+template<bool POISSON, bool WIDE, uint32_t NPSM, uint32_t WATCH, uint32_t WALK>
+__global__ __launch_bounds__(BLOCK + WALK * WAVE, WATCH * (1 + WALK * WAVE / BLOCK))
 void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const NeuronGroupDev * __restrict__ groups,
                     const uint8_t * __restrict__ tileGroup, unsigned long long *tags, unsigned long long *side,
                     unsigned long long timestep0, unsigned long long epoch0, unsigned long long numRecordingTimesteps, uint32_t numSteps,
@@ -161,17 +186,18 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                     unsigned long long seqBase)
 {
     extern __shared__ float lds[];                       // inSyn rows and ring slices of this tile
-    __shared__ unsigned long long shTag[RES_MAX_TILES];
-    __shared__ uint2 shPair[RES_PAIR_CAP];               // (presynaptic neuron, projection)
-    __shared__ uint2 shSeg[RES_PAIR_CAP];                // (first idSyn, length | flags) of each staged pair
-    __shared__ uint32_t shFlagged;                       // staged pairs whose row has to be walked before the update
+    __shared__ uint2 shSeg[2][RES_PAIR_CAP];             // (first idSyn, length | flags | projection) of each listed pair
+    // of an exchange: pairs claimed; listed pairs whose row has to be walked before the update; pairs were left over; a wait expired
+    struct Taken { uint32_t pairs, flagged, left, failed; };
+    __shared__ __align__(16) Taken shTaken[4];
+    __shared__ uint32_t shDone[4];                       // of the update an exchange feeds: wavefronts done << 16 | spikes
     __shared__ ResProj shProj[RES_MAX_PROJ];
-    __shared__ uint32_t shProjPtr[RES_MAX_PROJ];         // this step's front slot of each projection's ring
+    __shared__ uint32_t shProjPtr[4][RES_MAX_PROJ];      // front slot of each projection's ring in the step an exchange feeds
     __shared__ uint32_t shProjStart[RES_MAX_GROUPS + 1]; // projections of this tile by source group
     __shared__ uint8_t shProjIdx[RES_MAX_PROJ];
-    __shared__ uint8_t shTileGroup[RES_MAX_TILES];
-    __shared__ uint32_t shOwn[RES_T];                    // this tile's spikes of the last step, ascending
-    __shared__ uint32_t shWave[BLOCK / WAVE];
+    __shared__ uint32_t shOwn[RES_T];                    // this tile's spikes of the last step, in no particular order
+    constexpr uint32_t THREADS = BLOCK + WALK * WAVE, WAVES = THREADS / WAVE, MAIN = BLOCK / WAVE;
+    __shared__ uint32_t shWave[WAVES];
     __shared__ uint32_t shScalar[4];
 
     // every tile publishes its word into all copies of the word array and reads the copy of its own XCD
@@ -183,19 +209,18 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     const gennmi_neuron_update_group_t &g = G.g;
     const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
     const uint32_t n = g.numNeurons;
-    const uint32_t i = T.first + tid;
-    const bool mine = tid < T.count;
+    const uint32_t tileFirst = T.first, tilesInGroup = T.tilesInGroup, tileInGroup = T.tileInGroup;
+    const uint32_t i = tileFirst + tid;
+    const bool mine = tid < T.count, main = (WALK == 0 || wave < MAIN);
     const uint32_t numPSM = g.numPSM, numCS = g.numCS;
 
     // (a runner whose error flag is raised launches nothing more: the host looks at the flag before every launch; the flag
     // is host memory, and reading it here would put a trip over the bus in front of every launch)
-    if(tid == 0) { shScalar[3] = 0u; }
-    __syncthreads();
-
     // ---- tables into LDS
-    for(uint32_t k = tid; k < numTiles; k += BLOCK) { shTileGroup[k] = tileGroup[k]; }
     const uint32_t numProj = T.numProj;
     if(tid < numProj) { shProj[tid] = T.proj[tid]; }
+    if(tid < 4) { shScalar[tid] = 0u; }
+    if(tid < 4) { shTaken[tid] = Taken{0u, 0u, 0u, 0u}; shDone[tid] = 0u; }
     __syncthreads();
     // projections grouped by source group (a counting sort of a handful of entries, read from the LDS copy; every thread
     // finds one entry's place by itself — one thread doing all of it is a chain of a hundred dependent LDS reads, 3 us
@@ -214,9 +239,14 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             before += (q < tid && sq == s) ? 1u : 0u;
         }
         shProjIdx[below + before] = (uint8_t)tid;
+        const uint32_t D = shProj[tid].D;
+        for(uint32_t e = 1; e <= 2; e++) { shProjPtr[(seqBase + e) & 3][tid] = D ? modStep(epoch0 + e, D) : 0u; }
     }
+    // (lane p < numProj of the last wavefront, which prepares what the exchange after the next needs) front slot of projection p's ring then
+    const uint32_t ptrDepth = (wave == WAVES - 1 && lane < numProj) ? max(1u, shProj[lane].D) : 1u;
+    uint32_t ptrNext = modStep(epoch0 + 3, ptrDepth);
 
-    // ---- state: neuron variables in registers, inSyn and ring slices in LDS
+    // ---- state: neuron variables in registers, inSyn in registers (in LDS where synapses add to it) and ring slices in LDS
     float l0 = 0, l1 = 0;
     if(mine) { l0 = asGlobal(g.var0)[i]; l1 = asGlobal(g.var1)[i]; }
     // state of the PoissonExp sources, in registers like the neuron's own
@@ -225,9 +255,30 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
         csState[c] = (POISSON && mine && c < numCS && g.cs[c].kind == GENNMI_CS_POISSON_EXP) ? asGlobal(g.cs[c].current)[i] : 0.0f;
     }
-    for(uint32_t m = 0; m < numPSM; m++) {
-        lds[T.ldsIn[m] + tid] = mine ? asGlobal(g.psm[m].outPost)[i] : 0.0f;
-        const uint32_t D = g.psm[m].maxDenDelay;
+    // What the update reads of its group and tile, once: through the references every step would load it again (the
+    // compiler cannot tell that nobody writes those structures while the kernel runs).
+    float psmInit[NPSM], psmDecay[NPSM], csAmp[GENNMI_MAX_CS], par[8], lin[NPSM];
+    uint32_t psmKind[NPSM], psmDepth[NPSM], psmIn[NPSM], psmRing[NPSM], psmFront[NPSM], csKind[GENNMI_MAX_CS];
+    #pragma unroll
+    for(uint32_t m = 0; m < NPSM; m++) {
+        const bool on = m < numPSM;
+        psmInit[m] = on ? g.psm[m].init : 0.0f; psmDecay[m] = on ? g.psm[m].expDecay : 0.0f;
+        psmKind[m] = on ? g.psm[m].kind : 0u; psmDepth[m] = on ? g.psm[m].maxDenDelay : 0u;
+        psmIn[m] = on ? T.ldsIn[m] : 0u; psmRing[m] = on ? T.ldsRing[m] : 0u;
+        psmFront[m] = psmDepth[m] ? modStep(epoch0 + 1, psmDepth[m]) : 0u;         // the slot the coming step reads
+        lin[m] = (on && mine) ? asGlobal(g.psm[m].outPost)[i] : 0.0f;
+    }
+    #pragma unroll
+    for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) { csAmp[c] = (c < numCS) ? g.cs[c].amp : 0.0f; csKind[c] = (c < numCS) ? g.cs[c].kind : 0u; }
+    #pragma unroll
+    for(uint32_t q = 0; q < 8; q++) { par[q] = g.params[q]; }
+    const uint32_t neuronModel = g.model;
+    GLOBAL_AS uint32_t * const recordSpk = asGlobal(g.recordSpk);
+    #pragma unroll
+    for(uint32_t m = 0; m < NPSM; m++) {
+        if(m >= numPSM) { break; }
+        const uint32_t D = psmDepth[m];
+        if(!D && main) { lds[psmIn[m] + tid] = lin[m]; }
         // (sixteen slots' loads in flight at a time: one at a time, a ring of 43 slots is 43 memory round trips per launch)
         GLOBAL_AS const float *ring = asGlobal(g.psm[m].denDelay) + (mine ? i : 0u);
         for(uint32_t slot0 = 0; slot0 < D; slot0 += 16) {
@@ -235,28 +286,26 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             #pragma unroll
             for(uint32_t u = 0; u < 16; u++) { v[u] = (mine && slot0 + u < D) ? ring[(size_t)min(slot0 + u, D - 1) * n] : 0.0f; }
             #pragma unroll
-            for(uint32_t u = 0; u < 16; u++) { if(slot0 + u < D) { lds[T.ldsRing[m] + (slot0 + u) * RES_T + tid] = v[u]; } }
+            for(uint32_t u = 0; u < 16; u++) { if(main && slot0 + u < D) { lds[psmRing[m] + (slot0 + u) * RES_T + tid] = v[u]; } }
         }
     }
 
     // ---- this tile's spikes of the step before the first one, from the population's (ascending) queue
-    if(tid == 0) { shScalar[0] = 0; shScalar[1] = 0; }
-    __syncthreads();
     {
         const uint32_t cnt = asGlobal(g.spkCnt)[0];
         uint32_t below = 0, inside = 0;
-        for(uint32_t k = tid; k < cnt; k += BLOCK) {
+        for(uint32_t k = tid; k < cnt; k += THREADS) {
             const uint32_t id = asGlobal(g.spk)[k];
-            below += (id < T.first) ? 1u : 0u;
-            inside += (id >= T.first && id < T.first + T.count) ? 1u : 0u;
+            below += (id < tileFirst) ? 1u : 0u;
+            inside += (id >= tileFirst && id < tileFirst + T.count) ? 1u : 0u;
         }
         if(below) { atomicAdd(&shScalar[0], below); }
         if(inside) { atomicAdd(&shScalar[1], inside); }
         __syncthreads();
         const uint32_t lo = shScalar[0];
-        for(uint32_t k = tid; k < cnt; k += BLOCK) {
+        for(uint32_t k = tid; k < cnt; k += THREADS) {
             const uint32_t id = asGlobal(g.spk)[k];
-            if(id >= T.first && id < T.first + T.count) { shOwn[k - lo] = id; }
+            if(id >= tileFirst && id < tileFirst + T.count) { shOwn[k - lo] = id; }
         }
     }
     __syncthreads();
@@ -268,49 +317,69 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // between launches.  A tile's spikes beyond those its word holds go through the side buffer, one 64-bit entry each that
     // says which exchange it belongs to (the unwrapped sequence number, 56 bits, above the tile-local index): entries and
     // word are stored in any order without a fence, and a reader that finds the word first waits for the entries.
+    // (called by one wavefront)
     auto publish = [&](uint32_t step, uint32_t count) {
         const uint32_t seq = (uint32_t)((seqBase + step) & RES_SEQ_MASK);
         const uint32_t parity = seq & 1u;
         if(count > RES_WORD_IDS) {
-            for(uint32_t r = tid; r < count; r += BLOCK) {
-                __hip_atomic_store(&side[((size_t)parity * numTiles + blockIdx.x) * RES_T + r], ((seqBase + step) << 8) | (shOwn[r] - T.first),
+            for(uint32_t r = lane; r < count; r += WAVE) {
+                __hip_atomic_store(&side[((size_t)parity * numTiles + blockIdx.x) * RES_T + r], ((seqBase + step) << 8) | (shOwn[r] - tileFirst),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        if(tid < RES_REPLICAS) {
+        if(lane < RES_REPLICAS) {
             uint32_t locals = 0;
-            for(uint32_t e = 0; e < min(count, RES_WORD_IDS); e++) { locals |= (shOwn[e] - T.first) << (8 * e); }
+            for(uint32_t e = 0; e < min(count, RES_WORD_IDS); e++) { locals |= (shOwn[e] - tileFirst) << (8 * e); }
             const unsigned long long word = ((unsigned long long)seq << RES_SEQ_SHIFT) | ((unsigned long long)count << 32) | locals;
-            __hip_atomic_store(&tags[(size_t)tid * replicaStride + (size_t)parity * numTiles + blockIdx.x], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&tags[(size_t)lane * replicaStride + (size_t)parity * numTiles + blockIdx.x], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
 
-    // source tiles this thread watches (tile tid, tid + 256, ...) and how many of this tile's projections each feeds
-    constexpr uint32_t WATCH = RES_MAX_TILES / BLOCK;
-    uint32_t watchProj0[WATCH], watchNumProj[WATCH], watchFirst[WATCH];
+    // Source tiles this thread watches and, of each, the spikes it takes.  More than 128 tiles: tiles tid, tid + 256, ..., all
+    // their spikes.  Fewer tiles than half the threads: several threads watch the same tile and deal its spikes between them.
+    uint32_t perTile = 1, perShift = 0, watchTile = tid, watchSub = 0;
+    if(WATCH == 1 && numTiles <= BLOCK / 2) {
+        const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u);       // (tiles rounded up to a power of two)
+        perTile = BLOCK >> shift; perShift = 8 - shift;
+        static_assert(BLOCK == 1 << 8, "threads per watched tile");
+        watchTile = tid & ((1u << shift) - 1u); watchSub = tid >> shift;
+    }
+    uint32_t watchProj0[WATCH], watchNumProj[WATCH], watchFirst[WATCH], watchLds[WATCH];
+    GLOBAL_AS const u32x4 *watchSeg[WATCH];              // entry of the tile's first neuron under its group's first projection into this tile
+    uint32_t watchFlags[WATCH];                          // that projection's number << 26
+    const uint32_t narrowStride = 2u * tilesInGroup;     // entries of consecutive rows, in quads
     #pragma unroll
     for(uint32_t q = 0; q < WATCH; q++) {
-        const uint32_t k = tid + q * BLOCK;
+        const uint32_t k = main ? watchTile + q * BLOCK : numTiles;
         watchFirst[q] = (k < numTiles) ? tiles[k].first : 0u;
-        const uint32_t s = (k < numTiles) ? shTileGroup[k] : 0u;
+        const uint32_t s = (k < numTiles) ? tileGroup[k] : 0u;
         watchProj0[q] = shProjStart[s];
-        watchNumProj[q] = (k < numTiles) ? shProjStart[s + 1] - shProjStart[s] : 0u;
+        watchNumProj[q] = (k < numTiles) ? shProjStart[s + 1] - watchProj0[q] : 0u;
+        watchSeg[q] = nullptr; watchFlags[q] = 0; watchLds[q] = 0;
+        if(watchNumProj[q]) {
+            const uint32_t p = shProjIdx[watchProj0[q]];
+            const uint32_t quads = (WIDE && shProj[p].wide) ? RES_WIDE_QUADS : 2u;
+            watchSeg[q] = asGlobal(shProj[p].seg) + quads * ((size_t)watchFirst[q] * tilesInGroup + tileInGroup);
+            watchFlags[q] = p << RES_SEG_PROJ_SHIFT;
+            watchLds[q] = shProj[p].lds;
+        }
     }
 
-    // Waits for every tile's word of sequence number seq (false when the bounded wait expired somewhere) and stages the
-    // (spike, projection) pairs that concern this tile in shPair; shScalar[0] receives their number, which may exceed
-    // RES_PAIR_CAP (then only the claims that fitted were written and the caller takes the chunked path).
-    // Entries e0 .. e0 + 7 (below c) of a tile's side list of the exchange `full`: waits, bounded, until each says so
-    auto sideIds = [&](uint32_t tile, uint32_t e0, uint32_t c, unsigned long long full, uint32_t parity, uint32_t (&local)[8]) -> bool {
+    // spikes of a word whose entries a thread has in flight at a time
+    constexpr uint32_t FLIGHT = (WATCH * (1 + WALK * WAVE / BLOCK) <= 2) ? 4 : (WATCH <= 2) ? 2 : 1;
+    // Entries e0, e0 + stepE, ... (FLIGHT of them, below c) of a tile's side list of the exchange `full`: waits, bounded, until each says so
+    auto sideIds = [&](uint32_t tile, uint32_t e0, uint32_t stepE, uint32_t c, unsigned long long full, uint32_t parity, uint32_t (&local)[FLIGHT]) -> bool {
         const unsigned long long *base = side + ((size_t)parity * numTiles + tile) * RES_T + e0;
         const unsigned long long want = full & 0x00FFFFFFFFFFFFFFull;
-        uint32_t need = (c - e0 >= 8) ? 0xFFu : (1u << (c - e0)) - 1u, spins = 0;
-        unsigned long long v[8];
+        uint32_t need = 0, spins = 0;
+        #pragma unroll
+        for(uint32_t u = 0; u < FLIGHT; u++) { if(e0 + u * stepE < c) { need |= 1u << u; } }
+        unsigned long long v[FLIGHT];
         while(true) {
             #pragma unroll
-            for(uint32_t u = 0; u < 8; u++) { v[u] = 0; if(need & (1u << u)) { v[u] = __hip_atomic_load(base + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); } }
+            for(uint32_t u = 0; u < FLIGHT; u++) { v[u] = 0; if(need & (1u << u)) { v[u] = __hip_atomic_load(base + u * stepE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); } }
             #pragma unroll
-            for(uint32_t u = 0; u < 8; u++) {
+            for(uint32_t u = 0; u < FLIGHT; u++) {
                 if((need & (1u << u)) && (v[u] >> 8) == want) { local[u] = (uint32_t)v[u] & 0xFFu; need &= ~(1u << u); }
             }
             if(!need) { return true; }
@@ -318,22 +387,74 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             __builtin_amdgcn_s_sleep(1);
         }
     };
-    auto poll = [&](uint32_t step, unsigned long long epoch) -> bool {
-        const uint32_t seq = (uint32_t)((seqBase + step) & RES_SEQ_MASK);
-        const uint32_t parity = seq & 1u;
-        bool ok = true;
-        unsigned long long word[WATCH];
-        uint32_t pending = 0;
+
+    unsigned long long events = 0;
+
+    constexpr uint32_t PASS_ALL = 0, PASS_LATER = 1, PASS_DUE = 2, PASS_NONE = 3;      // which synapses a pass adds: see process()
+
+    // What one ordinary segment entry says: lists the pair and — unless `skipInline` — adds the entry's inline synapses to the front slot
+    auto takeNarrow = [&](u32x4 lo4, u32x4 hi4, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
+        shSeg[slot & 1][pos] = make_uint2(lo4.x, lo4.y | flags);
+        if(lo4.y & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
+        if(count) { events += lo4.y & 0xFFFFu; }
+        const uint32_t numFront = skipInline ? 0u : (lo4.y >> 16) & 0xFFu;
+        const uint32_t w[RES_FRONT_MAX] = {lo4.z, lo4.w, hi4.x, hi4.y};
         #pragma unroll
-        for(uint32_t q = 0; q < WATCH; q++) { word[q] = 0; if(tid + q * BLOCK < numTiles) { pending |= 1u << q; } }
-        if(tid == 0) { shScalar[0] = 0; shFlagged = 0; }
+        for(uint32_t f = 0; f < RES_FRONT_MAX; f++) {
+            if(f < numFront) { unsafeAtomicAdd(&lds[frontBase + ((hi4.z >> (8 * f)) & 0xFFu)], __uint_as_float(w[f])); }
+        }
+    };
+    auto takeWide = [&](GLOBAL_AS const u32x4 *entry, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
+        uint32_t e[4 * RES_WIDE_QUADS];
+        #pragma unroll
+        for(uint32_t u = 0; u < RES_WIDE_QUADS; u++) {
+            const u32x4 x = entry[u];
+            e[4 * u] = x.x; e[4 * u + 1] = x.y; e[4 * u + 2] = x.z; e[4 * u + 3] = x.w;
+        }
+        shSeg[slot & 1][pos] = make_uint2(e[0], e[1] | flags);
+        if(e[1] & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
+        if(count) { events += e[1] & 0xFFFFu; }
+        const uint32_t inside = skipInline ? 0u : (e[1] >> 16) & 0xFFu;
+        #pragma unroll
+        for(uint32_t f = 0; f < RES_WIDE_MAX; f++) {
+            if((f & 3) == 0 && !__any(f < inside)) { break; }
+            if(f < inside) { unsafeAtomicAdd(&lds[frontBase + ((e[2 + f / 4] >> (8 * (f & 3))) & 0xFFu)], __uint_as_float(e[8 + f])); }
+        }
+    };
+    // entry of (neuron, projection), read where a pair is not taken by the thread that saw its word
+    auto takeEntry = [&](uint32_t id, uint32_t p, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
+        const ResProj &P = shProj[p];
+        const size_t row = (size_t)id * tilesInGroup + tileInGroup;
+        const uint32_t frontBase = P.lds + shProjPtr[slot][p] * RES_T;
+        if(WIDE && P.wide) { takeWide(asGlobal(P.seg) + RES_WIDE_QUADS * row, p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count); }
+        else {
+            GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + 2 * row;
+            takeNarrow(entry[0], entry[1], p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count);
+        }
+    };
+
+    // Waits for every tile's word of exchange `step` (main threads; shTaken says when the bounded wait expired somewhere) and takes the
+    // (spike, projection) pairs that concern this tile: lists them and — `convention` PASS_ALL or PASS_DUE — adds the due synapses
+    // their entries hold.  Pairs that find no place in the list are left to leftOver() (`left`: this thread's words that have some).
+    unsigned long long word[WATCH];
+    #pragma unroll
+    for(uint32_t q = 0; q < WATCH; q++) { word[q] = 0; }
+    uint32_t left = 0;
+    auto poll = [&](uint32_t step, uint32_t convention) {
+        const uint32_t seq = (uint32_t)((seqBase + step) & RES_SEQ_MASK);
+        const uint32_t parity = seq & 1u, slot = seq & 3u;
+        const bool skipInline = (convention == PASS_LATER), count = (convention != PASS_DUE);
+        bool ok = true;
+        uint32_t pending = 0;
+        left = 0;
+        #pragma unroll
+        for(uint32_t q = 0; q < WATCH; q++) { word[q] = 0; if(watchTile + q * BLOCK < numTiles) { pending |= 1u << q; } }
+        const unsigned long long *mine_ = myTags + (size_t)parity * numTiles + watchTile;
         uint32_t spins = 0;
         while(pending) {
             #pragma unroll
             for(uint32_t q = 0; q < WATCH; q++) {
-                if(pending & (1u << q)) {
-                    word[q] = __hip_atomic_load(&myTags[(size_t)parity * numTiles + tid + q * BLOCK], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
+                if(pending & (1u << q)) { word[q] = __hip_atomic_load(mine_ + q * BLOCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
             }
             #pragma unroll
             for(uint32_t q = 0; q < WATCH; q++) {
@@ -344,95 +465,102 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             if(spins > c_spinLimit || ((spins & 255u) == 0 && __hip_atomic_load(errorFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) { ok = false; break; }
             __builtin_amdgcn_s_sleep(1);
         }
-        #pragma unroll
-        for(uint32_t q = 0; q < WATCH; q++) { if(tid + q * BLOCK < numTiles) { shTag[tid + q * BLOCK] = word[q]; } }
-        if(!ok) { shScalar[3] = 1u; }                  // (zero since the launch began: a launch that finds the error flag raised has left)
-        __syncthreads();
-        if(shScalar[3]) {
-            if(tid == 0) { raiseErrorFlag(errorFlag); }
-            return false;
-        }
-        // front slot of every projection's ring in the step this exchange feeds
-        if(tid < numProj) { shProjPtr[tid] = shProj[tid].D ? modStep(epoch + 1, shProj[tid].D) : 0u; }
-        #pragma unroll
-        for(uint32_t q = 0; q < WATCH; q++) {
-            const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu, np = watchNumProj[q];
-            if(c == 0 || np == 0) { continue; }
-            uint32_t pos = atomicAdd(&shScalar[0], c * np);
-            const bool fits = pos + c * np <= RES_PAIR_CAP;
-            if(c <= RES_WORD_IDS) {
-                for(uint32_t e = 0; fits && e < c; e++) {
-                    const uint32_t id = watchFirst[q] + (((uint32_t)word[q] >> (8 * e)) & 0xFFu);
-                    for(uint32_t j = 0; j < np; j++) { shPair[pos++] = make_uint2(id, shProjIdx[watchProj0[q] + j]); }
-                }
-                continue;
-            }
-            // a longer list: its entries, eight loads at a time (also when the pairs do not fit and the chunked walk will
-            // read the list again: once seen here, an entry is there for every later read of this work-group)
-            for(uint32_t e0 = 0; e0 < c && ok; e0 += 8) {
-                uint32_t local[8];
-                if(!sideIds(tid + q * BLOCK, e0, c, seqBase + step, parity, local)) { ok = false; break; }
-                #pragma unroll
-                for(uint32_t u = 0; u < 8; u++) {
-                    if(!fits || e0 + u >= c) { continue; }
-                    for(uint32_t j = 0; j < np; j++) { shPair[pos++] = make_uint2(watchFirst[q] + local[u], shProjIdx[watchProj0[q] + j]); }
-                }
-            }
-        }
-        if(!ok) { shScalar[3] = 1u; }
-        __syncthreads();
-        if(shScalar[3]) {
-            if(tid == 0) { raiseErrorFlag(errorFlag); }
-            return false;
-        }
-        return true;
-    };
-
-    unsigned long long events = 0;
-
-    constexpr uint32_t PASS_ALL = 0, PASS_LATER = 1, PASS_DUE = 2;      // which synapses a pass adds: see process()
-
-    // First pass over the staged pairs, one lane per pair: reads the pair's segment entry, keeps (start, length, flags)
-    // for the passes that walk the row, and — unless `skipInline` — adds the entry's inline synapses to the front slot.
-    auto readSegments = [&](uint32_t numPairs, bool skipInline, bool count) {
-        for(uint32_t q = tid; q < numPairs; q += BLOCK) {
-            const uint2 pr = shPair[q];
-            const ResProj &P = shProj[pr.y];
-            GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + ((WIDE && P.wide) ? RES_WIDE_QUADS : 2u) * ((size_t)pr.x * T.tilesInGroup + T.tileInGroup);
-            if(WIDE && P.wide) {
-                uint32_t e[4 * RES_WIDE_QUADS];
-                #pragma unroll
-                for(uint32_t u = 0; u < RES_WIDE_QUADS; u++) {
-                    const u32x4 x = entry[u];
-                    e[4 * u] = x.x; e[4 * u + 1] = x.y; e[4 * u + 2] = x.z; e[4 * u + 3] = x.w;
-                }
-                shSeg[q] = make_uint2(e[0], e[1]);
-                if(e[1] & RES_SEG_OVERFLOW) { atomicAdd(&shFlagged, 1u); }
-                if(count) { events += e[1] & 0xFFFFu; }
-                if(skipInline) { continue; }
-                const uint32_t inside = (e[1] >> 16) & 0xFFu;
-                #pragma unroll
-                for(uint32_t f = 0; f < RES_WIDE_MAX; f++) {
-                    if(f < inside) { unsafeAtomicAdd(&lds[P.lds + ((e[2 + f / 4] >> (8 * (f & 3))) & 0xFFu)], __uint_as_float(e[8 + f])); }
-                }
-                continue;
-            }
-            const u32x4 lo4 = entry[0], hi4 = entry[1];
-            shSeg[q] = make_uint2(lo4.x, lo4.y);
-            if(lo4.y & RES_SEG_OVERFLOW) { atomicAdd(&shFlagged, 1u); }
-            if(count) { events += lo4.y & 0xFFFFu; }
-            if(skipInline) { continue; }
-            const uint32_t numFront = (lo4.y >> 16) & 0xFFu;
-            const uint32_t frontBase = P.lds + shProjPtr[pr.y] * RES_T;
-            const uint32_t w[RES_FRONT_MAX] = {lo4.z, lo4.w, hi4.x, hi4.y};
+        if(convention != PASS_NONE) {
+            // this thread's pairs, and the word they come from when it is only one
+            uint32_t total = 0, mineCount[WATCH];
+            bool several = false;
+            unsigned long long busyWord = 0;
+            uint32_t busyFlags = 0, busyLds = 0;
+            GLOBAL_AS const u32x4 *busySeg = nullptr;
             #pragma unroll
-            for(uint32_t f = 0; f < RES_FRONT_MAX; f++) {
-                if(f < numFront) { unsafeAtomicAdd(&lds[frontBase + ((hi4.z >> (8 * f)) & 0xFFu)], __uint_as_float(w[f])); }
+            for(uint32_t q = 0; q < WATCH; q++) {
+                const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu, np = watchNumProj[q];
+                mineCount[q] = (ok && c > watchSub && np != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u;
+                if(mineCount[q]) {
+                    several = total != 0 || c > RES_WORD_IDS || np > 1 || mineCount[q] > FLIGHT;
+                    total += mineCount[q] * np;
+                    busyWord = word[q]; busyFlags = watchFlags[q]; busyLds = watchLds[q]; busySeg = watchSeg[q];
+                }
+            }
+            if(__any(several)) {
+                // Some thread of the wavefront has pairs from several words, or many: the wavefront lists its pairs first and every
+                // lane then takes as many of them as every other, so that their entries are one trip to memory and not one after another.
+                const uint32_t inclusive = waveInclusiveScanU32(total, lane);
+                const uint32_t waveTotal = (uint32_t)__builtin_amdgcn_readlane((int)inclusive, WAVE - 1);
+                uint32_t base = 0;
+                if(lane == 0) { base = atomicAdd(&shTaken[slot].pairs, waveTotal); }
+                base = __builtin_amdgcn_readfirstlane(base);
+                const bool fits = (base + waveTotal <= RES_PAIR_CAP);
+                uint32_t pos = base + inclusive - total;
+                #pragma unroll
+                for(uint32_t q = 0; q < WATCH; q++) {
+                    if(!mineCount[q]) { continue; }
+                    if(!fits) { left |= 1u << q; }
+                    const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu;
+                    for(uint32_t e0 = watchSub; e0 < c && ok; e0 += FLIGHT * perTile) {
+                        uint32_t local[FLIGHT];
+                        #pragma unroll
+                        for(uint32_t u = 0; u < FLIGHT; u++) { local[u] = ((uint32_t)word[q] >> (8 * ((e0 + u * perTile) & 3u))) & 0xFFu; }
+                        // (also when the pairs do not fit and leftOver() will read the list again: once seen here, an entry is there
+                        // for every later read of this thread)
+                        if(c > RES_WORD_IDS && !sideIds(watchTile + q * BLOCK, e0, perTile, c, seqBase + step, parity, local)) { ok = false; }
+                        #pragma unroll
+                        for(uint32_t u = 0; u < FLIGHT; u++) {
+                            if(!fits || e0 + u * perTile >= c) { break; }
+                            for(uint32_t j = 0; j < watchNumProj[q]; j++) { shSeg[slot & 1][pos++] = make_uint2(watchFirst[q] + local[u], shProjIdx[watchProj0[q] + j]); }
+                        }
+                    }
+                }
+                if(!fits) {
+                    // (a claim across the list's end: the places it does not use say "no synapses")
+                    for(uint32_t r = base + lane; r < RES_PAIR_CAP; r += WAVE) { shSeg[slot & 1][r] = make_uint2(0u, 0u); }
+                    if(lane == 0) { shTaken[slot].left = 1u; }
+                }
+                else if(!__any(!ok)) {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                    for(uint32_t x = base + lane; x < base + waveTotal; x += WAVE) {
+                        const uint2 pr = shSeg[slot & 1][x];
+                        takeEntry(pr.x, pr.y, slot, x, skipInline, count);
+                    }
+                }
+            }
+            else if(total) {
+                // up to FLIGHT spikes of one tile under one projection: their entries are asked for before they have their place in the list
+                const bool narrow = !WIDE || !shProj[busyFlags >> RES_SEG_PROJ_SHIFT].wide;
+                uint32_t local[FLIGHT];
+                u32x4 lo4[FLIGHT], hi4[FLIGHT];
+                #pragma unroll
+                for(uint32_t u = 0; u < FLIGHT; u++) {
+                    local[u] = ((uint32_t)busyWord >> (8 * ((watchSub + u * perTile) & 3u))) & 0xFFu;
+                    if(narrow && u < total) {
+                        GLOBAL_AS const u32x4 *entry = busySeg + (size_t)local[u] * narrowStride;
+                        lo4[u] = entry[0]; hi4[u] = entry[1];
+                    }
+                }
+                const uint32_t pos = atomicAdd(&shTaken[slot].pairs, total);
+                if(pos + total <= RES_PAIR_CAP) {
+                    const uint32_t frontBase = busyLds + shProjPtr[slot][busyFlags >> RES_SEG_PROJ_SHIFT] * RES_T;
+                    #pragma unroll
+                    for(uint32_t u = 0; u < FLIGHT; u++) {
+                        if(u >= total) { break; }
+                        if(narrow) { takeNarrow(lo4[u], hi4[u], busyFlags, frontBase, slot, pos + u, skipInline, count); }
+                        else if(WIDE) { takeWide(busySeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), busyFlags, frontBase, slot, pos + u, skipInline, count); }
+                    }
+                }
+                else {
+                    #pragma unroll
+                    for(uint32_t q = 0; q < WATCH; q++) { if(mineCount[q]) { left |= 1u << q; } }
+                    for(uint32_t r = pos; r < RES_PAIR_CAP; r++) { shSeg[slot & 1][r] = make_uint2(0u, 0u); }
+                    shTaken[slot].left = 1u;
+                }
             }
         }
+        if(!ok) { shTaken[slot].failed = 1u; }
     };
 
-    // Walks the row segments of the staged pairs: a group of lanes per pair, a lane taking every n-th synapse of its
+    // Walks the row segments of the listed pairs: a group of lanes per pair, a lane taking every n-th synapse of its
     // pair's segment, eight of them per trip to memory.  Sixteen lanes per pair when the pairs are few (a quiet step: one
     // trip covers 128 synapses of each of a wavefront's four pairs), four when they are many (a synchronous burst).
     // (Segments of a tile are short — a row's share of 256 targets — so lanes idle in the longest segment's last trip
@@ -440,22 +568,23 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // A synapse is "due" when it lands in the slot read this step (delay a multiple of the ring depth, or no ring).
     // PASS_ALL adds every synapse, PASS_LATER those not due, PASS_DUE the due ones; `flaggedOnly` restricts the walk to
     // segments whose due synapses are not all inline in their entry.
-    auto process = [&](uint32_t numPairs, uint32_t pass, bool flaggedOnly) {
+    // (wavefront `first` of the `count` that call)
+    auto process = [&](const uint2 *segs, const uint32_t *fronts, uint32_t numPairs, uint32_t pass, bool flaggedOnly, uint32_t first, uint32_t count) {
         constexpr uint32_t TRIP = 8;
-        const uint32_t shift = (numPairs <= 4 * (BLOCK / WAVE)) ? 4u : (numPairs <= 8 * (BLOCK / WAVE)) ? 3u : 2u;
+        const uint32_t shift = (numPairs <= 4 * count) ? 4u : (numPairs <= 8 * count) ? 3u : 2u;
         const uint32_t lanesPerPair = 1u << shift, pairsPerGroup = WAVE >> shift;
-        for(uint32_t q0 = wave * pairsPerGroup; q0 < numPairs; q0 += (BLOCK / WAVE) * pairsPerGroup) {
+        for(uint32_t q0 = first * pairsPerGroup; q0 < numPairs; q0 += count * pairsPerGroup) {
             const uint32_t q = q0 + (lane >> shift);
             uint32_t len = 0, start = 0, proj = 0;
             if(q < numPairs) {
-                const uint2 sg = shSeg[q];
-                proj = shPair[q].y;
+                const uint2 sg = segs[q];
+                proj = sg.y >> RES_SEG_PROJ_SHIFT;
                 const bool flagged = (sg.y & RES_SEG_OVERFLOW) != 0;
                 const bool skip = (flaggedOnly && !flagged) || (pass == PASS_LATER && (sg.y & RES_SEG_NO_DELAY));
                 start = sg.x; len = skip ? 0u : (sg.y & 0xFFFFu);
             }
             const ResProj &P = shProj[proj];
-            const uint32_t depth = P.D, front = shProjPtr[proj], ldsBase = P.lds, magic = P.magic;
+            const uint32_t depth = P.D, front = fronts[proj], ldsBase = P.lds, magic = P.magic;
             GLOBAL_AS const u32x2 *packed = asGlobal(P.packed) + start;
             for(uint32_t i0 = lane & (lanesPerPair - 1); __any(i0 < len); i0 += TRIP * lanesPerPair) {
                 u32x2 rec[TRIP];
@@ -478,124 +607,133 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
     };
 
-    // the pairs of a step that holds more of them than shPair does: staged and walked RES_PAIR_CAP at a time, in full
-    auto processChunked = [&](uint32_t step, uint32_t total, uint32_t pass, bool count) {
-        const uint32_t parity = (seqBase + step) & 1u;
+    // The pairs of the words that found no place in the list: listed and walked RES_PAIR_CAP at a time, in full, before the
+    // update (in the other parity's list: its pairs were walked before this exchange's words were looked for, and the next
+    // exchange's threads come here first).
+    auto leftOver = [&](uint32_t step, uint32_t pass, bool count) {
+        const uint32_t slot = (uint32_t)(seqBase + step) & 3u, parity = slot & 1u, other = parity ^ 1u;
         uint32_t want = 0;
-        for(uint32_t k = tid; k < numTiles; k += BLOCK) {
-            const uint32_t c = (uint32_t)(shTag[k] >> 32) & 0x1FFu;
-            const uint32_t s = shTileGroup[k];
-            want += c * (shProjStart[s + 1] - shProjStart[s]);
+        #pragma unroll
+        for(uint32_t q = 0; q < WATCH; q++) {
+            const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu;
+            if(left & (1u << q)) { want += ((c - watchSub + perTile - 1) / perTile) * watchNumProj[q]; }
         }
         const uint32_t inclusive = waveInclusiveScanU32(want, lane);
         if(lane == WAVE - 1) { shWave[wave] = inclusive; }
         __syncthreads();
-        uint32_t base = inclusive - want;
+        uint32_t base = inclusive - want, total = 0;
         #pragma unroll
-        for(uint32_t w = 0; w < BLOCK / WAVE; w++) { if(w < wave) { base += shWave[w]; } }
+        for(uint32_t w = 0; w < WAVES; w++) { if(w < wave) { base += shWave[w]; } total += shWave[w]; }
         for(uint32_t chunk0 = 0; chunk0 < total; chunk0 += RES_PAIR_CAP) {
             uint32_t pos = base;
-            for(uint32_t k = tid; k < numTiles; k += BLOCK) {
-                const unsigned long long tag = shTag[k];
-                const uint32_t c = (uint32_t)(tag >> 32) & 0x1FFu;
-                const uint32_t s = shTileGroup[k];
-                const uint32_t p0 = shProjStart[s], np = shProjStart[s + 1] - p0;
-                if(c == 0 || np == 0) { continue; }
-                if(pos + c * np <= chunk0 || pos >= chunk0 + RES_PAIR_CAP) { pos += c * np; continue; }
-                for(uint32_t q = 0; q < c; q++) {
-                    const uint32_t id = (c <= RES_WORD_IDS) ? tiles[k].first + (((uint32_t)tag >> (8 * q)) & 0xFFu)
-                                                            : tiles[k].first + ((uint32_t)__hip_atomic_load(&side[((size_t)parity * numTiles + k) * RES_T + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFFu);
+            #pragma unroll
+            for(uint32_t q = 0; q < WATCH; q++) {
+                if(!(left & (1u << q))) { continue; }
+                const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu, np = watchNumProj[q];
+                const uint32_t mineCount = (c - watchSub + perTile - 1) / perTile;
+                if(pos + mineCount * np <= chunk0 || pos >= chunk0 + RES_PAIR_CAP) { pos += mineCount * np; continue; }
+                for(uint32_t e = watchSub; e < c; e += perTile) {
+                    const uint32_t id = (c <= RES_WORD_IDS) ? watchFirst[q] + (((uint32_t)word[q] >> (8 * e)) & 0xFFu)
+                                                            : watchFirst[q] + ((uint32_t)__hip_atomic_load(&side[((size_t)parity * numTiles + watchTile + q * BLOCK) * RES_T + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFFu);
                     for(uint32_t j = 0; j < np; j++, pos++) {
-                        if(pos >= chunk0 && pos < chunk0 + RES_PAIR_CAP) { shPair[pos - chunk0] = make_uint2(id, shProjIdx[p0 + j]); }
+                        if(pos >= chunk0 && pos < chunk0 + RES_PAIR_CAP) { shSeg[other][pos - chunk0] = make_uint2(id, shProjIdx[watchProj0[q] + j]); }
                     }
                 }
             }
             __syncthreads();
             const uint32_t numPairs = min(RES_PAIR_CAP, total - chunk0);
-            readSegments(numPairs, true, count);
+            for(uint32_t q = tid; q < numPairs; q += THREADS) {
+                const uint2 pr = shSeg[other][q];
+                const ResProj &P = shProj[pr.y];
+                const u32x4 lo4 = (asGlobal(P.seg) + ((WIDE && P.wide) ? RES_WIDE_QUADS : 2u) * ((size_t)pr.x * tilesInGroup + tileInGroup))[0];
+                shSeg[other][q] = make_uint2(lo4.x, (lo4.y & ~(0x3Fu << RES_SEG_PROJ_SHIFT)) | (pr.y << RES_SEG_PROJ_SHIFT));
+                if(count) { events += lo4.y & 0xFFFFu; }
+            }
             __syncthreads();
-            process(numPairs, pass, false);
+            process(shSeg[other], shProjPtr[slot], numPairs, pass, false, wave, WAVES);
             __syncthreads();
         }
     };
 
-    // After a successful poll(seq): what the spikes of that exchange owe this tile NOW — the synapses due this step
-    // (inline in the segment entries; row walks only for segments that say so).  `convention` is PASS_ALL normally,
-    // PASS_LATER when a previous launch has already delivered the due synapses of these spikes, PASS_DUE when only those
-    // are wanted.  Returns the number of staged pairs whose remaining synapses deliverLater() has to add, or 0.
-    auto deliverDue = [&](uint32_t seq, uint32_t convention) -> uint32_t {
-        const uint32_t total = shScalar[0];
-        if(total > RES_PAIR_CAP) {
-            processChunked(seq, total, convention, convention != PASS_DUE);
-            return 0u;
+    // After poll(), by all threads: the barrier, and whatever the listed entries could not deliver at once.  `convention` is PASS_ALL
+    // normally, PASS_LATER when a previous launch has already delivered the due synapses of these spikes, PASS_DUE when only those
+    // are wanted.  False: some wait expired.  `later`: listed pairs whose remaining synapses are to be added before the next update.
+    uint32_t later = 0;
+    auto deliverDue = [&](uint32_t step, uint32_t convention) -> bool {
+        const uint32_t slot = (uint32_t)(seqBase + step) & 3u;
+        ldsBarrier();
+        const Taken taken = shTaken[slot];
+        later = min(taken.pairs, RES_PAIR_CAP);
+        if(taken.flagged | taken.left | taken.failed) {
+            if(taken.failed) {
+                if(tid == 0) { raiseErrorFlag(errorFlag); }
+                return false;
+            }
+            if(convention != PASS_LATER && taken.flagged) { process(shSeg[slot & 1], shProjPtr[slot], later, PASS_DUE, true, wave, WAVES); ldsBarrier(); }
+            if(taken.left) { leftOver(step, convention, convention != PASS_DUE); }
         }
-        readSegments(total, convention == PASS_LATER, convention != PASS_DUE);
-        __syncthreads();
-        if(convention != PASS_LATER && shFlagged) { process(total, PASS_DUE, true); __syncthreads(); }
-        return (convention == PASS_DUE) ? 0u : total;
+        return true;
     };
-    // the rest of those pairs' synapses: none of them is read before the next step
-    auto deliverLater = [&](uint32_t numPairs) {
-        if(numPairs) { process(numPairs, PASS_LATER, false); }
-    };
-
-    // What the update reads of its group and tile, once: through the references every step would load it again (the
-    // compiler cannot tell that nobody writes those structures while the kernel runs).
-    float psmInit[GENNMI_MAX_PSM], psmDecay[GENNMI_MAX_PSM], csAmp[GENNMI_MAX_CS], par[8];
-    uint32_t psmKind[GENNMI_MAX_PSM], psmDepth[GENNMI_MAX_PSM], psmIn[GENNMI_MAX_PSM], psmRing[GENNMI_MAX_PSM], csKind[GENNMI_MAX_CS];
-    #pragma unroll
-    for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) {
-        const bool on = m < numPSM;
-        psmInit[m] = on ? g.psm[m].init : 0.0f; psmDecay[m] = on ? g.psm[m].expDecay : 0.0f;
-        psmKind[m] = on ? g.psm[m].kind : 0u; psmDepth[m] = on ? g.psm[m].maxDenDelay : 0u;
-        psmIn[m] = on ? T.ldsIn[m] : 0u; psmRing[m] = on ? T.ldsRing[m] : 0u;
-    }
-    #pragma unroll
-    for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) { csAmp[c] = (c < numCS) ? g.cs[c].amp : 0.0f; csKind[c] = (c < numCS) ? g.cs[c].kind : 0u; }
-    #pragma unroll
-    for(uint32_t q = 0; q < 8; q++) { par[q] = g.params[q]; }
-    const uint32_t neuronModel = g.model;
-    uint32_t * const recordSpk = g.recordSpk;
 
     bool anyRing = false;
     for(uint32_t q = 0; q < numProj; q++) { anyRing = anyRing || shProj[q].D != 0; }
+    unsigned long long recT = numRecordingTimesteps ? (((timestep0 | numRecordingTimesteps) >> 32) ? timestep0 % numRecordingTimesteps
+                                                                                                    : (uint32_t)timestep0 % (uint32_t)numRecordingTimesteps) : 0ull;
+    const uint32_t recordWords = (n + 31) / 32;
     // ---- exchange the spikes that precede the first step, then step
-    publish(1u, ownCount);
+    if(wave == 0) { publish(1u, ownCount); }
     bool ok = true;
     uint32_t k = 0;
     for(; k < numSteps; k++) {
         const unsigned long long epoch = epoch0 + k;
-        if(!poll(k + 1, epoch)) { ok = false; break; }
-        const uint32_t later = deliverDue(k + 1, (zeroDelaySplit && k == 0) ? PASS_LATER : PASS_ALL);     // (ends with a barrier)
-
+        const uint32_t slot = (uint32_t)(seqBase + k + 1) & 3u, afterNext = (slot + 2) & 3u;
+        const uint32_t convention = (zeroDelaySplit && k == 0) ? PASS_LATER : PASS_ALL;
+        float inject[GENNMI_MAX_CS];
+        if(main) {
+            // (what the sources inject does not depend on the exchange: drawn while the words travel)
+            #pragma unroll
+            for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
+                inject[c] = 0.0f;
+                if(POISSON && c < numCS) { inject[c] = (csKind[c] == GENNMI_CS_DC) ? csAmp[c] : (mine ? poissonExpStep(g.cs[c], csState[c], i, epoch) : 0.0f); }
+            }
+            poll(k + 1, convention);
+        }
+        if(!deliverDue(k + 1, convention)) { ok = false; break; }
+        if(wave == WAVES - 1) {
+            if(lane < numProj) { shProjPtr[afterNext][lane] = ptrNext; }
+            if(lane == 0) { shTaken[afterNext] = Taken{0u, 0u, 0u, 0u}; shDone[afterNext] = 0u; }
+            ptrNext = (ptrNext + 1 >= ptrDepth) ? 0u : ptrNext + 1;
+        }
+        if(main) {
         // neuron update: same operations in the same order as neuronBody
         bool spiked = false;
         if(mine) {
             float Isyn = 0;
             #pragma unroll
-            for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) {
-                if(m < numPSM) {
-                    float linSyn = lds[psmIn[m] + tid];
-                    const uint32_t D = psmDepth[m];
-                    if(D) {
-                        const uint32_t front = psmRing[m] + modStep(epoch + 1, D) * RES_T + tid;
-                        linSyn += lds[front];
-                        lds[front] = 0.0f;
-                    }
-                    if(psmKind[m] == GENNMI_PSM_EXPCURR) {
-                        Isyn += psmInit[m] * linSyn;
-                        linSyn *= psmDecay[m];
-                    }
-                    else {
-                        Isyn += linSyn;
-                        linSyn = 0.0f;
-                    }
-                    lds[psmIn[m] + tid] = linSyn;
+            for(uint32_t m = 0; m < NPSM; m++) {
+                if(m >= numPSM) { break; }
+                float linSyn;
+                if(psmDepth[m]) {
+                    const uint32_t front = psmRing[m] + psmFront[m] * RES_T + tid;
+                    linSyn = lin[m] + lds[front];
+                    lds[front] = 0.0f;
                 }
+                else { linSyn = lds[psmIn[m] + tid]; }
+                if(psmKind[m] == GENNMI_PSM_EXPCURR) {
+                    Isyn += psmInit[m] * linSyn;
+                    linSyn *= psmDecay[m];
+                }
+                else {
+                    Isyn += linSyn;
+                    linSyn = 0.0f;
+                }
+                if(psmDepth[m]) { lin[m] = linSyn; }
+                else { lds[psmIn[m] + tid] = linSyn; }
             }
             #pragma unroll
             for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
-                if(c < numCS) { Isyn += (!POISSON || csKind[c] == GENNMI_CS_DC) ? csAmp[c] : poissonExpStep(g.cs[c], csState[c], i, epoch); }
+                if(c >= numCS) { break; }
+                Isyn += POISSON ? inject[c] : csAmp[c];
             }
             if(neuronModel == GENNMI_NEURON_LIF) {
                 if(l1 <= 0.0f) {
@@ -620,39 +758,52 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                 spiked = (l0 >= 29.99f);
             }
         }
+        // (a wavefront without spikes, which nearly all are, only says that it is done)
         const unsigned long long ballot = __ballot(spiked);
-        const uint32_t laneRank = __popcll(ballot & ((1ull << lane) - 1ull));
-        if(lane == 0) { shWave[wave] = __popcll(ballot); }
-        __syncthreads();
-        uint32_t waveOffset = 0;
-        ownCount = 0;
-        #pragma unroll
-        for(uint32_t w = 0; w < BLOCK / WAVE; w++) {
-            const uint32_t c = shWave[w];
-            if(w < wave) { waveOffset += c; }
-            ownCount += c;
+        if(ballot) {
+            uint32_t base = 0;
+            if(lane == 0) { base = atomicAdd(&shDone[slot], (uint32_t)__popcll(ballot)); }
+            base = __builtin_amdgcn_readfirstlane(base) & 0xFFFFu;
+            if(spiked) { shOwn[base + __popcll(ballot & ((1ull << lane) - 1ull))] = i; }
         }
-        if(spiked) { shOwn[waveOffset + laneRank] = i; }
-        __syncthreads();
-        publish(k + 2, ownCount);
-        // while the words of this step travel: the step's recording words, and the synapses of the previous step's spikes
+        if(WALK) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            uint32_t done = 0;
+            if(lane == 0) { done = atomicAdd(&shDone[slot], 1u << 16); }
+            done = __builtin_amdgcn_readfirstlane(done);
+            if((done >> 16) == MAIN - 1) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                publish(k + 2, done & 0xFFFFu);
+            }
+        }
+        else {
+            ldsBarrier();
+            if(wave == 0) { publish(k + 2, shDone[slot]); }
+        }
+        // while the words of this step travel: the step's recording words, and (next) the synapses of the previous step's spikes
         // that are not due yet
-        if(recordSpk && (lane & 31) == 0 && mine) {
-            const unsigned long long ts = timestep0 + k;
-            const uint32_t recT = numRecordingTimesteps ? (((ts | numRecordingTimesteps) >> 32) ? (uint32_t)(ts % numRecordingTimesteps)
-                                                                                                : ((uint32_t)ts % (uint32_t)numRecordingTimesteps)) : 0u;
-            recordSpk[(size_t)recT * ((n + 31) / 32) + (i >> 5)] = (uint32_t)(ballot >> (lane & 32));
+        if(recordSpk && (lane & 31) == 0 && mine) { recordSpk[(size_t)recT * recordWords + (i >> 5)] = (uint32_t)(ballot >> (lane & 32)); }
+        if(numRecordingTimesteps) { recT = (recT + 1 == numRecordingTimesteps) ? 0ull : recT + 1; }
+        #pragma unroll
+        for(uint32_t m = 0; m < NPSM; m++) {
+            if(m >= numPSM) { break; }
+            psmFront[m] = (psmFront[m] + 1 >= psmDepth[m]) ? 0u : psmFront[m] + 1;
         }
-        if(anyRing) { deliverLater(later); }       // (without a ring nothing is: the next word is looked for at once)
+        }
+        if((WALK == 0 || !main) && anyRing && later) {       // (without a ring nothing is: the next word is looked for at once)
+            process(shSeg[slot & 1], shProjPtr[slot], later, PASS_LATER, false, WALK ? wave - MAIN : wave, WALK ? WALK : MAIN);
+        }
     }
 
     // ---- after the last step: everybody's last spikes give the position of this tile's spikes in the population's
     // queue; a runner that delivers front-slot synapses one step early (single-launch plan) wants them in the ring now
     const unsigned long long epochEnd = epoch0 + numSteps;       // completed steps
-    if(ok && !poll(numSteps + 1, epochEnd)) { ok = false; }
     if(!ok) { return; }
-    if(zeroDelaySplit) { deliverDue(numSteps + 1, PASS_DUE); }
+    const uint32_t lastConvention = zeroDelaySplit ? PASS_DUE : PASS_NONE;
+    if(main) { poll(numSteps + 1, lastConvention); }
+    if(!deliverDue(numSteps + 1, lastConvention)) { return; }
     __syncthreads();
+    ownCount = shDone[(uint32_t)(seqBase + numSteps) & 3u] & 0xFFFFu;       // (the last update's)
 
     if(mine) {
         asGlobal(g.var0)[i] = l0; asGlobal(g.var1)[i] = l1;
@@ -661,28 +812,36 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             if(POISSON && c < numCS && g.cs[c].kind == GENNMI_CS_POISSON_EXP) { asGlobal(g.cs[c].current)[i] = csState[c]; }
         }
     }
-    for(uint32_t m = 0; m < numPSM; m++) {
-        if(mine) { asGlobal(g.psm[m].outPost)[i] = lds[T.ldsIn[m] + tid]; }
-        const uint32_t D = g.psm[m].maxDenDelay;
+    #pragma unroll
+    for(uint32_t m = 0; m < NPSM; m++) {
+        if(m >= numPSM) { break; }
+        const uint32_t D = psmDepth[m];
+        if(mine) { asGlobal(g.psm[m].outPost)[i] = D ? lin[m] : lds[psmIn[m] + tid]; }
         for(uint32_t slot = 0; slot < D; slot++) {
-            if(mine) { asGlobal(g.psm[m].denDelay)[(size_t)slot * n + i] = lds[T.ldsRing[m] + slot * RES_T + tid]; }
+            if(mine) { asGlobal(g.psm[m].denDelay)[(size_t)slot * n + i] = lds[psmRing[m] + slot * RES_T + tid]; }
         }
-        if(T.tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
+        if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
     }
     uint32_t offset = 0;
-    for(uint32_t q = T.firstTileOfGroup + tid; q < T.firstTileOfGroup + T.tileInGroup; q += BLOCK) { offset += (uint32_t)(shTag[q] >> 32) & 0x1FFu; }
+    #pragma unroll
+    for(uint32_t q = 0; q < WATCH; q++) {
+        const uint32_t tile = watchTile + q * BLOCK;
+        if(main && watchSub == 0 && tile >= T.firstTileOfGroup && tile < T.firstTileOfGroup + tileInGroup) { offset += (uint32_t)(word[q] >> 32) & 0x1FFu; }
+    }
     if(tid == 0) { shScalar[2] = 0; }
     __syncthreads();
     if(offset) { atomicAdd(&shScalar[2], offset); }
     __syncthreads();
     offset = shScalar[2];
-    const bool lastTile = (T.tileInGroup == T.tilesInGroup - 1);
+    const bool lastTile = (tileInGroup == tilesInGroup - 1);
     const uint32_t shadowParity = (uint32_t)((epochEnd - 1) & 1);
-    for(uint32_t r = tid; r < ownCount; r += BLOCK) {
+    for(uint32_t r = tid; r < ownCount; r += THREADS) {
         const uint32_t id = shOwn[r];
-        g.spk[offset + r] = id;
-        for(uint32_t q = 0; q < g.numExtraSpk; q++) { g.extraSpk[q][offset + r] = id; }
-        if(G.shadowSpk) { G.shadowSpk[(size_t)shadowParity * n + offset + r] = id; }
+        uint32_t place = offset;                         // (queues ascend)
+        for(uint32_t q = 0; q < ownCount; q++) { place += (shOwn[q] < id) ? 1u : 0u; }
+        g.spk[place] = id;
+        for(uint32_t q = 0; q < g.numExtraSpk; q++) { g.extraSpk[q][place] = id; }
+        if(G.shadowSpk) { G.shadowSpk[(size_t)shadowParity * n + place] = id; }
     }
     if(lastTile && tid == 0) {
         g.spkCnt[0] = offset + ownCount;

@@ -11,7 +11,7 @@ import pytest
 
 from genn_amd import rng
 from genn_amd.genn_model import model_from_net
-from genn_amd.netspec import Net, Pop, Syn
+from genn_amd.netspec import CurrentSource, Net, Pop, Syn
 from oracle.genn_cpu import OracleNet
 from parity import compare_state
 
@@ -354,4 +354,37 @@ def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypat
                 oracle.syn_g(s.name)[:] *= np.float32(0.5)
     model, oracle, spikes = _run_chunks(net, [100, -3, 97, 60], check)
     assert spikes > 2000
+    model.unload()
+
+
+@pytest.mark.parametrize("n_a, n_b, depth, models, poisson", [
+    (256, 1, 0, 1, False), (250, 255, 1, 1, False), (32760, 3, 0, 1, False), (32760, 260, 2, 1, False),            # few tiles, threads share a tile's word
+    (65000, 300, 3, 2, False), (65500, 200, 5, 1, True), (65530, 300, 0, 2, True), (65530, 300, 4, 2, False),      # up to, and one beyond, a tile a thread
+    (130000, 1000, 3, 1, False), (130800, 500, 2, 1, True), (130800, 500, 0, 1, False),                           # two tiles a thread, and more
+    (5000, 700, 0, 3, False), (5000, 700, 6, 3, False), (70000, 700, 3, 3, True), (131000, 600, 0, 3, False)])     # more than two postsynaptic models
+def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
+    """Which of the kernel's instances runs depends on the number of tiles (256 neurons each), rings, postsynaptic models a population and sources;
+    a ring of one slot is a case of its own (everything is due at once).  Every (target, postsynaptic model) has one projection: identical.
+    (The tile path adds a step's sums, not its weights one by one: the single steps in between go without it.)"""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
+    net = Net(name="resident_tiles", dt=1.0, steps=0)
+    net.pops.append(_pop("A", n_a, 0.62, -60.0 + 9.9 * rng.uniform(5, 1, 0, n_a)))
+    net.pops.append(_pop("B", n_b, 0.45, -60.0 + 9.9 * rng.uniform(5, 2, 0, n_b)))
+    if poisson:
+        net.css.append(CurrentSource("A_bg", "poisson_exp", "A", params=dict(weight=0.2, tauSyn=2.0, rate=800.0)))
+    def ring(k):
+        return dict(depth=depth, due_share=0.3) if depth > 1 else dict(depth=0)
+    for k in range(models):
+        net.syns.append(_projection(f"BA{k}", "B", "A", n_b, n_a, 40, 0.21 / (k + 1), 11 + k, tau=5.0 + k, **ring(k)))
+    net.syns.append(_projection("AB", "A", "B", n_a, n_b, 4, 0.002, 31, **ring(0)))
+    if depth == 1:
+        for s in net.syns:
+            s.wum, s.d, s.max_den_delay = "static_delay", np.zeros(s.ind.shape, np.uint8), 1
+    net.steps = 30
+
+    def check(model, oracle):
+        compare_state(net, model, oracle, f"after {model.timestep} steps", exact=True)
+
+    model, oracle, spikes = _run_chunks(net, (14, -2, 14), check)
+    assert spikes > n_a // 16
     model.unload()
