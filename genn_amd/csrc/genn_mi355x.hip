@@ -94,8 +94,8 @@ struct gennmi_runner
     ResTile *dResTiles = nullptr; NeuronGroupDev *dResGroups = nullptr; uint8_t *dResTileGroup = nullptr;
     unsigned long long *dResTags = nullptr, *dResSide = nullptr;
     uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0;
-    decltype(&residentKernel<false, false, 2, 1, 0>) resKernel = nullptr;     // the instantiation its sources and segment entries need
-    uint32_t resThreads = BLOCK;        // ... and its work-group
+    decltype(&residentKernel<false, false, 2, 256, 0>) resKernel = nullptr;      // the instantiation its sources, segment entries and tiles need
+    uint32_t resThreads = BLOCK, resTileSize = BLOCK;     // ... its work-group, and neurons of a tile
     std::vector<u32x4*> resSegs;        // segment table of each presynaptic group, in push order
     std::vector<uint32_t> resSegTiles;  // tiles of its target population
     std::vector<uint32_t> resSegWide;   // its entries are wide ones
@@ -738,7 +738,7 @@ int gennmi_push_postsynaptic_update_group(gennmi_runner *r, const gennmi_postsyn
 
 // Resident plan (residentKernel): chosen when the whole network fits the chip — batch 1, static SPARSE projections
 // (with or without dendritic delay) with ascending rows between LIF / Izhikevich populations driven by DC or PoissonExp sources, every
-// tile of 256 neurons with its ring slices in LDS and all tiles resident at once.  GENNMI_RESIDENT=0 disables it.
+// tile of neurons with its ring slices in LDS and all tiles resident at once.  GENNMI_RESIDENT=0 disables it.
 static int setupResident(gennmi_runner *r, uint32_t numCU)
 {
     const char *env = getenv("GENNMI_RESIDENT");
@@ -749,66 +749,80 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         if((g.model != GENNMI_NEURON_LIF && g.model != GENNMI_NEURON_IZHIKEVICH) || g.preTrace || g.postTrace || g.sT || g.numDelaySlots > 1 || g.numSpkEvent || g.numPreOutput) { return GENNMI_OK; }
         for(uint32_t c = 0; c < g.numCS; c++) { if(g.cs[c].kind == GENNMI_CS_ARRAY) { return GENNMI_OK; } }
     }
-    // tiles and their LDS layout
-    std::vector<ResTile> tiles;
-    std::vector<uint8_t> tileGroup;
-    std::vector<uint32_t> firstTile(r->neuron.size()), numTilesOf(r->neuron.size());
-    size_t ldsFloatsMax = 0;
-    for(size_t gi = 0; gi < r->neuron.size(); gi++) {
-        const auto &g = r->neuron[gi].g;
-        ResTile t{};
-        uint32_t offset = 0;
-        for(uint32_t m = 0; m < g.numPSM; m++) {
-            t.ldsIn[m] = offset; offset += RES_T;
-            if(g.psm[m].maxDenDelay) { t.ldsRing[m] = offset; offset += g.psm[m].maxDenDelay * RES_T; }
-        }
-        t.ldsFloats = offset;
-        ldsFloatsMax = std::max<size_t>(ldsFloatsMax, offset);
-        t.group = (uint32_t)gi;
-        t.tilesInGroup = (g.numNeurons + RES_T - 1) / RES_T;
-        t.firstTileOfGroup = (uint32_t)tiles.size();
-        firstTile[gi] = t.firstTileOfGroup; numTilesOf[gi] = t.tilesInGroup;
-        for(uint32_t k = 0; k < t.tilesInGroup; k++) {
-            t.tileInGroup = k; t.first = k * RES_T; t.count = std::min<uint32_t>(RES_T, g.numNeurons - t.first);
-            tiles.push_back(t);
-            tileGroup.push_back((uint8_t)gi);
-        }
-    }
-    if(tiles.empty() || tiles.size() > RES_MAX_TILES) { return GENNMI_OK; }
-    const size_t ldsBytes = std::max<size_t>(ldsFloatsMax, 1) * sizeof(float);
-    if(ldsBytes > 96 * 1024) { return GENNMI_OK; }
-    bool poisson = false;
+    bool poisson = false, anyRing = false, onlyRings = true;
     uint32_t maxPSM = 0;
     for(const auto &n : r->neuron) {
         maxPSM = std::max(maxPSM, n.g.numPSM);
         for(uint32_t c = 0; c < n.g.numCS; c++) { poisson = poisson || n.g.cs[c].kind == GENNMI_CS_POISSON_EXP; }
     }
-    // Wide segment entries where a projection without a ring leaves a tile up to RES_WIDE_MEAN synapses of a row (rowStride is a little more than
-    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them, and not in the networks whose
-    // instances go without them (registers): those with rings, and those of more tiles than two a compute unit.
-    constexpr uint32_t RES_WIDE_MEAN = 16;
-    bool anyWide = false, anyRing = false, onlyRings = true;
     for(const auto &p : r->pre) { anyRing = anyRing || p.g.maxDenDelay != 0; onlyRings = onlyRings && p.g.maxDenDelay >= 2; }
-    const bool widePossible = !anyRing && tiles.size() <= 2 * BLOCK;
-    auto wideEntries = [widePossible](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
-        const uint64_t mean = ((uint64_t)q.rowStride * RES_T + q.numTrgNeurons - 1) / q.numTrgNeurons;
-        return widePossible && q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
+    // tiles and their LDS layout: the smallest tile with which the network's tiles have a compute unit each
+    std::vector<ResTile> tiles;
+    std::vector<uint8_t> tileGroup;
+    std::vector<uint32_t> firstTile(r->neuron.size()), numTilesOf(r->neuron.size());
+    const char *envTile = getenv("GENNMI_RESIDENT_TILE");
+    uint32_t tileSize = 0, residentThreads = 0;
+    size_t ldsBytes = 0;
+    decltype(r->resKernel) residentInstance = nullptr;
+    bool anyWide = false;
+    // Wide segment entries where a projection without a ring leaves a tile up to RES_WIDE_MEAN synapses of a row (rowStride is a little more than
+    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them.
+    constexpr uint32_t RES_WIDE_MEAN = 16;
+    auto wideEntries = [&](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
+        const uint64_t mean = ((uint64_t)q.rowStride * tileSize + q.numTrgNeurons - 1) / q.numTrgNeurons;
+        return tileSize == 256 && !anyRing && q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN
+               && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
     };
-    for(const auto &p : r->pre) { anyWide = anyWide || wideEntries(p.g, (p.g.numTrgNeurons + RES_T - 1) / RES_T); }
-    // The instantiation for the network's sources, segment entries, postsynaptic models and number of tiles.  Where every projection has
-    // a ring that puts its synapses off for later, wavefronts of their own walk them, as long as two such work-groups a compute unit hold the network.
-    constexpr uint32_t WALK = BLOCK / WAVE, MAX = GENNMI_MAX_PSM;
-    const bool few = tiles.size() <= BLOCK, some = tiles.size() <= 2 * BLOCK, walkers = onlyRings && some && maxPSM <= 2;
-    decltype(r->resKernel) residentInstance;
-    if(maxPSM > 2) { residentInstance = some ? residentKernel<true, true, MAX, 2, 0> : residentKernel<true, false, MAX, 4, 0>; }
-    else if(walkers) {
-        if(few) { residentInstance = poisson ? residentKernel<true, false, 2, 1, WALK> : residentKernel<false, false, 2, 1, WALK>; }
-        else { residentInstance = poisson ? residentKernel<true, false, 2, 2, WALK> : residentKernel<false, false, 2, 2, WALK>; }
+    for(const uint32_t size : RES_TILES) {
+        if(envTile && (uint32_t)atoi(envTile) != size) { continue; }
+        size_t count = 0, ldsFloatsMax = 1;
+        for(const auto &n : r->neuron) {
+            count += (n.g.numNeurons + size - 1) / size;
+            size_t floats = 0;
+            for(uint32_t m = 0; m < n.g.numPSM; m++) { floats += (size_t)size * (1 + n.g.psm[m].maxDenDelay); }
+            ldsFloatsMax = std::max(ldsFloatsMax, floats);
+        }
+        if(count > size || count > numCU || ldsFloatsMax * sizeof(float) > (size == 256 ? 96u : 128u) * 1024) { continue; }
+        tileSize = size;
+        ldsBytes = ldsFloatsMax * sizeof(float);
+        for(const auto &p : r->pre) { anyWide = anyWide || wideEntries(p.g, (p.g.numTrgNeurons + size - 1) / size); }
+        // The instantiation for the network's sources, segment entries and postsynaptic models.  Where every projection has a ring that puts its
+        // synapses off for later, wavefronts of their own walk them, as far as a work-group's registers go.
+        constexpr uint32_t WALK = 4, MAX = GENNMI_MAX_PSM;
+        const bool walkers = onlyRings && maxPSM <= 2 && size <= 512;
+        if(maxPSM > 2) { residentInstance = (size == 256) ? residentKernel<true, true, MAX, 256, 0> : (size <= 512) ? residentKernel<true, false, MAX, 512, 0> : residentKernel<true, false, MAX, 1024, 0>; }
+        else if(walkers) {
+            if(size == 256) { residentInstance = poisson ? residentKernel<true, false, 2, 256, WALK> : residentKernel<false, false, 2, 256, WALK>; }
+            else if(size == 320) { residentInstance = poisson ? residentKernel<true, false, 2, 320, WALK> : residentKernel<false, false, 2, 320, WALK>; }
+            else { residentInstance = poisson ? residentKernel<true, false, 2, 512, WALK> : residentKernel<false, false, 2, 512, WALK>; }
+        }
+        else if(size == 256) { residentInstance = poisson ? residentKernel<true, true, 2, 256, 0> : anyWide ? residentKernel<false, true, 2, 256, 0> : residentKernel<false, false, 2, 256, 0>; }
+        else if(size <= 512) { residentInstance = poisson ? residentKernel<true, false, 2, 512, 0> : residentKernel<false, false, 2, 512, 0>; }
+        else { residentInstance = poisson ? residentKernel<true, false, 2, 1024, 0> : residentKernel<false, false, 2, 1024, 0>; }
+        if(!walkers && size == 320) { residentInstance = nullptr; continue; }          // (made for networks with walkers only)
+        residentThreads = size + (walkers ? WALK * WAVE : 0u);
+        break;
     }
-    else if(few) { residentInstance = poisson ? residentKernel<true, true, 2, 1, 0> : anyWide ? residentKernel<false, true, 2, 1, 0> : residentKernel<false, false, 2, 1, 0>; }
-    else if(some) { residentInstance = poisson ? residentKernel<true, true, 2, 2, 0> : anyWide ? residentKernel<false, true, 2, 2, 0> : residentKernel<false, false, 2, 2, 0>; }
-    else { residentInstance = poisson ? residentKernel<true, false, 2, 4, 0> : residentKernel<false, false, 2, 4, 0>; }
-    const uint32_t residentThreads = walkers ? BLOCK + WALK * WAVE : BLOCK;
+    if(!residentInstance) { return GENNMI_OK; }
+    for(size_t gi = 0; gi < r->neuron.size(); gi++) {
+        const auto &g = r->neuron[gi].g;
+        ResTile t{};
+        uint32_t offset = 0;
+        for(uint32_t m = 0; m < g.numPSM; m++) {
+            t.ldsIn[m] = offset; offset += tileSize;
+            if(g.psm[m].maxDenDelay) { t.ldsRing[m] = offset; offset += g.psm[m].maxDenDelay * tileSize; }
+        }
+        t.ldsFloats = offset;
+        t.group = (uint32_t)gi;
+        t.tilesInGroup = (g.numNeurons + tileSize - 1) / tileSize;
+        t.firstTileOfGroup = (uint32_t)tiles.size();
+        firstTile[gi] = t.firstTileOfGroup; numTilesOf[gi] = t.tilesInGroup;
+        for(uint32_t k = 0; k < t.tilesInGroup; k++) {
+            t.tileInGroup = k; t.first = k * tileSize; t.count = std::min<uint32_t>(tileSize, g.numNeurons - t.first);
+            tiles.push_back(t);
+            tileGroup.push_back((uint8_t)gi);
+        }
+    }
     const void *kernel = reinterpret_cast<const void*>(residentInstance);
     if(ldsBytes > 32 * 1024) {
         HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
@@ -868,7 +882,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         r->owned.push_back(dSeg);
         const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d,
-                                                                                                     depth, tilesInGroup, wide, dSeg);
+                                                                                                     depth, tileSize, tilesInGroup, wide, dSeg);
         r->resSegs.push_back(dSeg);
         r->resSegWide.push_back(wide);
         r->resSegTiles.push_back(tilesInGroup);
@@ -881,14 +895,13 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         }
         r->owned.push_back(dPacked);
         if(padded) {
-            residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(padded, q.ind, q.g, depth ? q.d : nullptr, dPacked);
+            residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(padded, q.ind, q.g, q.d, depth, tileSize, dPacked);
             HIP_TRY(hipGetLastError());
         }
         r->resPacked.push_back(dPacked);
         ResProj proj{};
         proj.packed = dPacked; proj.seg = dSeg; proj.wide = wide;
         proj.D = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
-        proj.magic = proj.D ? (uint32_t)(0x100000000ull / proj.D) + 1u : 0u;
         proj.srcGroup = (uint32_t)l.src;
         for(uint32_t t = firstTile[l.trg]; t < firstTile[l.trg] + tilesInGroup; t++) {
             proj.lds = proj.D ? tiles[t].ldsRing[l.psm] : tiles[t].ldsIn[l.psm];
@@ -911,14 +924,14 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     // cleared once: sequence number 0 is the one no work-group ever waits for before it has come round again
     HIP_TRY(hipMemset(r->dResTags, 0, (size_t)RES_REPLICAS * r->resReplicaStride * sizeof(unsigned long long)));
     r->resSeq = 0;
-    HIP_TRY(poolMalloc(&r->dResSide, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
+    HIP_TRY(poolMalloc(&r->dResSide, 2 * tiles.size() * tileSize * sizeof(unsigned long long)));
     r->owned.push_back(r->dResSide);
     // (cleared once as well: its entries name their exchange by the unwrapped sequence number, which starts at 1)
-    HIP_TRY(hipMemset(r->dResSide, 0, 2 * tiles.size() * RES_T * sizeof(unsigned long long)));
+    HIP_TRY(hipMemset(r->dResSide, 0, 2 * tiles.size() * tileSize * sizeof(unsigned long long)));
     r->resTiles = (uint32_t)tiles.size();
     r->resLdsBytes = ldsBytes;
     r->resKernel = residentInstance;
-    r->resThreads = residentThreads;
+    r->resThreads = residentThreads; r->resTileSize = tileSize;
     r->resident = true;
     return GENNMI_OK;
 }
@@ -944,10 +957,10 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
             const size_t entries = (size_t)q.numSrcNeurons * r->resSegTiles[k];
             const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
             residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(
-                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resSegTiles[k], r->resSegWide[k], r->resSegs[k]);
+                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resTileSize, r->resSegTiles[k], r->resSegWide[k], r->resSegs[k]);
             const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
             if(padded) {
-                residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(padded, q.ind, q.g, depth ? q.d : nullptr, r->resPacked[k]);
+                residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(padded, q.ind, q.g, q.d, depth, r->resTileSize, r->resPacked[k]);
             }
         }
         HIP_TRY(hipGetLastError());
@@ -959,7 +972,7 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
             r->dResTiles, r->resTiles, r->dResGroups, r->dResTileGroup, r->dResTags, r->dResSide, timestep + done, r->epoch, numRecordingTimesteps,
             chunk, r->dt, r->fusedStep ? 1u : 0u, r->dError, r->dEvents, r->resReplicaStride, r->resSeq);
         HIP_TRY(hipGetLastError());
-        r->resSeq += chunk + 1u;                                   // the launch used sequence numbers resSeq + 1 ... resSeq + chunk + 1 (words hold them modulo 2^23)
+        r->resSeq += chunk + 1u;                                   // the launch used sequence numbers resSeq + 1 ... resSeq + chunk + 1 (words hold them modulo 2^21)
         done += chunk;
         r->epoch += chunk;
     }

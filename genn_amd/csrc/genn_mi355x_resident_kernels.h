@@ -10,7 +10,7 @@
 // A timestep of such a network moves a few megabytes — half a microsecond of HBM time — but as a chain of
 // launches it costs ~12 us: ~4 us per kernel boundary (every L2 is written back and invalidated), then step
 // state -> spike count -> spike ids -> rows -> ~10^5 scattered fp32 atomics that retire at ~20 G/s on the memory
-// side.  Here one work-group owns RES_T neurons for a whole run: their state stays in registers, their
+// side.  Here one work-group owns a tile of neurons for a whole run: their state stays in registers, their
 // postsynaptic input (inSyn) and their slice of every dendritic-delay ring stay in LDS, and the only thing
 // work-groups exchange is each step's spikes — one 64-bit word per tile (sequence number, count, and the id
 // itself when a single neuron fired; longer lists go through a side buffer).  Every tile reads the words of
@@ -23,8 +23,13 @@
 // The wait for the other tiles' words is bounded (c_spinLimit polls) and also watches the error flag, so a launch
 // whose work-groups are not all resident ends with an error instead of hanging.
 // ------------------------------------------------------------------------------------------------
-constexpr uint32_t RES_T = BLOCK;            // neurons per tile = threads per work-group
-constexpr uint32_t RES_MAX_TILES = 1024;
+// Neurons of a tile.  A network takes the smallest of these with which its tiles have a compute unit each: work-groups that share one take twice
+// as long around their loop, and every tile waits for the slowest; and with T x T neurons at most each of a tile's T threads has
+// one other tile's word to look for.  us a step with tiles of 256, two and four to a compute unit / with these: the full microcircuit 4.4 / 4.1
+// (320), 100,000 x 80 5.9 / 5.0 (512), 180,000 x 100 9.0 / 5.7 and 250,000 x 200 10.5 / 4.9 (1024).  Larger ones than needed do not pay: 4,000 x 80
+// to 40,000 x 80 within 3 % with 512, up to 20 % more with 1024; the microcircuit at half size 2.8 -> 3.3 with 512.
+constexpr uint32_t RES_TILES[] = {256, 320, 512, 1024};
+constexpr uint32_t RES_MAX_TILE = 1024;
 constexpr uint32_t RES_MAX_PROJ = 16;        // projections into one population
 constexpr uint32_t RES_MAX_GROUPS = 64;      // neuron groups
 constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs a tile lists per exchange
@@ -36,9 +41,11 @@ constexpr uint32_t RES_FRONT_MAX = 4;        // front-slot synapses held inline 
 constexpr uint32_t RES_WIDE_QUADS = 8, RES_WIDE_MAX = 24;
 constexpr uint32_t RES_SEG_OVERFLOW = 1u << 24, RES_SEG_NO_DELAY = 1u << 25;
 constexpr uint32_t RES_SEG_PROJ_SHIFT = 26;  // in the kernel's list of pairs: the projection, above an entry's flags
-constexpr int RES_SEQ_SHIFT = 41;            // word = seq << 41 | count << 32 | up to four tile-local neuron indices, 8 bits each
-constexpr uint32_t RES_SEQ_MASK = (1u << (64 - RES_SEQ_SHIFT)) - 1u;    // sequence numbers run on from launch to launch, modulo 2^23
-constexpr uint32_t RES_WORD_IDS = 4;         // spikes of a tile and step that travel inside its word (more: side buffer)
+// word: upper half sequence number << 11 | count, lower half up to three tile-local neuron indices, 10 bits each
+constexpr uint32_t RES_COUNT_BITS = 11, RES_COUNT_MASK = (1u << RES_COUNT_BITS) - 1u;
+constexpr uint32_t RES_SEQ_MASK = (1u << (32 - RES_COUNT_BITS)) - 1u;    // sequence numbers run on from launch to launch, modulo 2^21
+constexpr uint32_t RES_WORD_IDS = 3;         // spikes of a tile and step that travel inside its word (more: side buffer)
+constexpr uint32_t RES_ID_BITS = 10, RES_ID_MASK = (1u << RES_ID_BITS) - 1u;
 constexpr uint32_t RES_REPLICAS = 8;         // copies of the word array, one per XCD, so that polling spreads over memory channels
 
 struct ResProj
@@ -46,11 +53,10 @@ struct ResProj
     const u32x2 *packed;                // one record per (padded) synapse, see residentPackKernel
     const u32x4 *seg;                   // [numSrc * tilesInGroup][2]: the row's part inside a tile, see residentSegKernel
     uint32_t D;                         // ring depth; 0 = no dendritic delay, events add to inSyn
-    uint32_t lds;                       // float offset of the ring (D x RES_T, slot-major) or inSyn row in the tile's LDS
+    uint32_t lds;                       // float offset of the ring (D x tile size, slot-major) or inSyn row in the tile's LDS
     uint32_t srcGroup;
     uint32_t wide;                      // != 0: entries of RES_WIDE_QUADS x 16 bytes instead of two
-    uint32_t pad_;
-    uint32_t magic;                     // floor(2^32 / D) + 1: x % D for x < 2^16 is x - mulhi(x, magic) * D
+    uint32_t pad_[2];
 };
 
 struct ResTile
@@ -64,14 +70,14 @@ struct ResTile
 };
 
 // One 32-byte entry per (row, tile of the target population): word 0 = first idSyn of the row's part inside the tile,
-// word 1 = its length | number of inline synapses << 16 | flags, words 2-5 = weights and word 6 = the packed tile-local
-// targets of up to four synapses whose delay is a multiple of the ring depth.  Those land in the slot the target reads in
+// word 1 = its length | number of inline synapses << 16 | flags, words 2-5 = weights and words 6 and 7 = the tile-local
+// targets (byte offsets, 16 bits each) of up to four synapses whose delay is a multiple of the ring depth.  Those land in the slot the target reads in
 // the very step that delivers them, so they are the only ones a step has to wait for; carrying them inside the entry
 // saves that step the dependent read of the row.  RES_SEG_OVERFLOW: the segment has more of them than fit (the row part
 // is then read at once); RES_SEG_NO_DELAY: the projection has no ring, every synapse is due at once.  A wide entry has words 0 and 1,
-// the packed targets of up to 24 synapses in words 2-7 and their weights in words 8-31.
+// the targets of up to 24 synapses in words 2-7 (tiles of 256: indices of a byte each) and their weights in words 8-31.
 __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLength, const uint32_t *ind, const float *weight,
-                                  const uint8_t *delay, uint32_t depth, uint32_t tilesInGroup, uint32_t wide, u32x4 *seg)
+                                  const uint8_t *delay, uint32_t depth, uint32_t tileSize, uint32_t tilesInGroup, uint32_t wide, u32x4 *seg)
 {
     const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if(id >= (size_t)numSrc * tilesInGroup) { return; }
@@ -83,7 +89,7 @@ __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uin
         while(lo < hi) { const uint32_t mid = (lo + hi) / 2; if(r[mid] < key) { lo = mid + 1; } else { hi = mid; } }
         return lo;
     };
-    const uint32_t a = lowerBound(tile * RES_T), b = lowerBound((tile + 1) * RES_T);
+    const uint32_t a = lowerBound(tile * tileSize), b = lowerBound((tile + 1) * tileSize);
     const uint32_t start = row * rowStride + a;
     uint32_t flags = depth ? 0u : RES_SEG_NO_DELAY, numFront = 0, locals = 0;
     if(wide) {
@@ -93,7 +99,7 @@ __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uin
         entry[0] = start; entry[1] = min(b - a, 0xFFFFu) | (inside << 16) | flags;
         for(uint32_t f = 0; f < RES_WIDE_MAX; f += 4) {
             for(uint32_t q = f; q < f + 4; q++) {
-                if(q < inside) { locals |= (r[a + q] - tile * RES_T) << (8 * (q - f)); }
+                if(q < inside) { locals |= (r[a + q] - tile * tileSize) << (8 * (q - f)); }
                 entry[8 + q] = (q < inside) ? __float_as_uint(weight[(size_t)row * rowStride + a + q]) : 0u;
             }
             entry[2 + f / 4] = locals;
@@ -101,33 +107,34 @@ __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uin
         }
         return;
     }
-    uint32_t w[RES_FRONT_MAX] = {0, 0, 0, 0};
+    uint32_t w[RES_FRONT_MAX] = {0, 0, 0, 0}, at[2] = {0, 0};
     if(!depth && b - a > RES_FRONT_MAX) { flags |= RES_SEG_OVERFLOW; }
     else {
         for(uint32_t j = a; j < b; j++) {
             if(depth && delay[(size_t)row * rowStride + j] % depth != 0) { continue; }
             if(numFront == RES_FRONT_MAX) { flags |= RES_SEG_OVERFLOW; numFront = 0; break; }    // the row walk adds all of them
             w[numFront] = __float_as_uint(weight[(size_t)row * rowStride + j]);
-            locals |= (r[j] - tile * RES_T) << (8 * numFront);
+            at[numFront / 2] |= 4u * (r[j] - tile * tileSize) << (16 * (numFront & 1));
             numFront++;
         }
     }
     u32x4 lo4, hi4;
     lo4.x = start; lo4.y = min(b - a, 0xFFFFu) | (numFront << 16) | flags; lo4.z = w[0]; lo4.w = w[1];
-    hi4.x = w[2]; hi4.y = w[3]; hi4.z = locals; hi4.w = 0;
+    hi4.x = w[2]; hi4.y = w[3]; hi4.z = at[0]; hi4.w = at[1];
     seg[2 * id] = lo4;
     seg[2 * id + 1] = hi4;
 }
 
-// The synapses as the row walk reads them: target inside its tile | dendritic delay << 8, and the weight's bits — one
-// 8-byte load per synapse instead of three loads from three arrays (three pages, three cache lines per row part).
+// The synapses as the row walk reads them: where in the tile's ring they land, in bytes from its front slot (slots of a float a
+// neuron of the tile; below the first slot's end: due), and the weight's bits — one 8-byte load per synapse instead of three loads from three arrays (three pages, three cache
+// lines per row part), and an addition and a minimum instead of a division by the ring's depth.
 // Same index as the arrays it is made from; padding beyond a row's length is copied as it is and never read.
-__global__ void residentPackKernel(size_t numSynapses, const uint32_t *ind, const float *weight, const uint8_t *delay, u32x2 *packed)
+__global__ void residentPackKernel(size_t numSynapses, const uint32_t *ind, const float *weight, const uint8_t *delay, uint32_t depth, uint32_t tileSize, u32x2 *packed)
 {
     const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if(id >= numSynapses) { return; }
     u32x2 rec;
-    rec.x = (ind[id] & (RES_T - 1)) | (delay ? (uint32_t)delay[id] << 8 : 0u); rec.y = __float_as_uint(weight[id]);
+    rec.x = 4u * (ind[id] % tileSize + (depth ? ((uint32_t)delay[id] % depth) * tileSize : 0u)); rec.y = __float_as_uint(weight[id]);
     packed[id] = rec;
 }
 
@@ -164,21 +171,19 @@ __device__ __forceinline__ void ldsBarrier()
 // publishes the tile's word.  The pairs are listed on the side, and the synapses that are not due are added by WALK wavefronts of
 // their own, between that barrier and the next one: a step lasts as long as the slowest tile takes around its loop, and time stamps
 // showed that tile never waiting for a word, but walking, polling, reading entries and updating one after the other.
-// us a step, with five barriers and the walk behind the word / now: the full microcircuit 6.1 / 4.4, with PoissonExp sources at half size
-// 5.3 / 3.4, balanced networks of 4,000 x 80 3.8 / 2.9, 100,000 x 80 7.2 / 5.9, 250,000 x 200 (four tiles a compute unit) 10.9 / 10.5.
-// (Spikes taken one after another by the thread that watches their word, however many: 180,000 x 100 10.1 -> 15.9.)
+// us a step, with five barriers and the walk behind the word / now: the full microcircuit 6.1 / 4.1, with PoissonExp sources at half size
+// 5.3 / 2.8, balanced networks of 4,000 x 80 3.8 / 2.85, 100,000 x 80 7.2 / 5.0.  (Spikes taken one after another by the thread that
+// watches their word, however many: 180,000 x 100 10.1 -> 15.9.)
 // What consecutive exchanges share exists once for each of them: pair lists twice, counters and ring fronts four times (those of the
 // exchange after the next are prepared behind the barrier, so no thread meets them half prepared).
 // POISSON: some population has a PoissonExp current source (its state then lives in a register per source and neuron);
-// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries.
-// NPSM: postsynaptic models of any group (their constants are wave-uniform: eight models' worth does not fit the scalar
-// registers, and what does not fit is read back lane by lane every step).  WATCH: source tiles a thread watches (up to WATCH x BLOCK
-// tiles); as many work-groups share a compute unit then, which is what the registers are budgeted for.  WALK: wavefronts beyond those that
+// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries (tiles of 256).
+// NPSM: postsynaptic models of any group.  TILE: neurons of a tile, and threads that own one.  WALK: wavefronts beyond those that
 // own the tile's neurons; 0: these walk too, once they have published.  With walkers nothing holds a wavefront back between its
 // update and the next exchange, so every projection must have a ring of two slots or more: what an early wavefront adds then goes to another slot
 // than the one a late one is reading and clearing.  Without, a barrier behind the update keeps them apart, and inSyn itself can be added to.
-template<bool POISSON, bool WIDE, uint32_t NPSM, uint32_t WATCH, uint32_t WALK>
-__global__ __launch_bounds__(BLOCK + WALK * WAVE, WATCH * (1 + WALK * WAVE / BLOCK))
+template<bool POISSON, bool WIDE, uint32_t NPSM, uint32_t TILE, uint32_t WALK>
+__global__ __launch_bounds__(TILE + WALK * WAVE, (TILE + WALK * WAVE + 4 * WAVE - 1) / (4 * WAVE))
 void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const NeuronGroupDev * __restrict__ groups,
                     const uint8_t * __restrict__ tileGroup, unsigned long long *tags, unsigned long long *side,
                     unsigned long long timestep0, unsigned long long epoch0, unsigned long long numRecordingTimesteps, uint32_t numSteps,
@@ -192,11 +197,11 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     __shared__ __align__(16) Taken shTaken[4];
     __shared__ uint32_t shDone[4];                       // of the update an exchange feeds: wavefronts done << 16 | spikes
     __shared__ ResProj shProj[RES_MAX_PROJ];
-    __shared__ uint32_t shProjPtr[4][RES_MAX_PROJ];      // front slot of each projection's ring in the step an exchange feeds
+    __shared__ uint32_t shProjPtr[4][RES_MAX_PROJ];      // front slot of each projection's ring in the step an exchange feeds, as a float offset
     __shared__ uint32_t shProjStart[RES_MAX_GROUPS + 1]; // projections of this tile by source group
     __shared__ uint8_t shProjIdx[RES_MAX_PROJ];
-    __shared__ uint32_t shOwn[RES_T];                    // this tile's spikes of the last step, in no particular order
-    constexpr uint32_t THREADS = BLOCK + WALK * WAVE, WAVES = THREADS / WAVE, MAIN = BLOCK / WAVE;
+    __shared__ uint32_t shOwn[TILE];                    // this tile's spikes of the last step, in no particular order
+    constexpr uint32_t THREADS = TILE + WALK * WAVE, WAVES = THREADS / WAVE, MAIN = TILE / WAVE;
     __shared__ uint32_t shWave[WAVES];
     __shared__ uint32_t shScalar[4];
 
@@ -240,7 +245,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         shProjIdx[below + before] = (uint8_t)tid;
         const uint32_t D = shProj[tid].D;
-        for(uint32_t e = 1; e <= 2; e++) { shProjPtr[(seqBase + e) & 3][tid] = D ? modStep(epoch0 + e, D) : 0u; }
+        for(uint32_t e = 1; e <= 2; e++) { shProjPtr[(seqBase + e) & 3][tid] = D ? modStep(epoch0 + e, D) * TILE : 0u; }
     }
     // (lane p < numProj of the last wavefront, which prepares what the exchange after the next needs) front slot of projection p's ring then
     const uint32_t ptrDepth = (wave == WAVES - 1 && lane < numProj) ? max(1u, shProj[lane].D) : 1u;
@@ -256,29 +261,34 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         csState[c] = (POISSON && mine && c < numCS && g.cs[c].kind == GENNMI_CS_POISSON_EXP) ? asGlobal(g.cs[c].current)[i] : 0.0f;
     }
     // What the update reads of its group and tile, once: through the references every step would load it again (the
-    // compiler cannot tell that nobody writes those structures while the kernel runs).
-    float psmInit[NPSM], psmDecay[NPSM], csAmp[GENNMI_MAX_CS], par[8], lin[NPSM];
-    uint32_t psmKind[NPSM], psmDepth[NPSM], psmIn[NPSM], psmRing[NPSM], psmFront[NPSM], csKind[GENNMI_MAX_CS];
+    // compiler cannot tell that nobody writes those structures while the kernel runs), and in vector registers: left to itself the compiler
+    // keeps such wave-uniform values in scalar registers, of which there are too few, and fetches them back lane by lane every step.
+    auto inVector = [](auto x) { asm volatile("" : "+v"(x)); return x; };
+    float psmInit[NPSM], psmDecay[NPSM], csAmp[GENNMI_MAX_CS], par[7], lin[NPSM];
+    uint32_t psmExp[NPSM], psmRing[NPSM], psmAt[NPSM], psmEnd[NPSM], csKind[GENNMI_MAX_CS];
     #pragma unroll
     for(uint32_t m = 0; m < NPSM; m++) {
-        const bool on = m < numPSM;
-        psmInit[m] = on ? g.psm[m].init : 0.0f; psmDecay[m] = on ? g.psm[m].expDecay : 0.0f;
-        psmKind[m] = on ? g.psm[m].kind : 0u; psmDepth[m] = on ? g.psm[m].maxDenDelay : 0u;
-        psmIn[m] = on ? T.ldsIn[m] : 0u; psmRing[m] = on ? T.ldsRing[m] : 0u;
-        psmFront[m] = psmDepth[m] ? modStep(epoch0 + 1, psmDepth[m]) : 0u;         // the slot the coming step reads
+        const bool on = m < numPSM, exponential = on && g.psm[m].kind == GENNMI_PSM_EXPCURR;
+        const uint32_t D = on ? g.psm[m].maxDenDelay : 0u;
+        psmExp[m] = inVector(exponential ? 1u : 0u); psmRing[m] = inVector(D ? D * TILE : 0u);
+        psmInit[m] = inVector(exponential ? g.psm[m].init : 1.0f); psmDecay[m] = inVector(exponential ? g.psm[m].expDecay : 0.0f);
+        // this neuron's element of the slot the coming step reads, and one beyond the last slot's; without a ring inSyn itself, in LDS
+        psmAt[m] = on ? (D ? T.ldsRing[m] + modStep(epoch0 + 1, D) * TILE : T.ldsIn[m]) + tid : 0u;
+        psmEnd[m] = on ? (D ? T.ldsRing[m] + D * TILE : T.ldsIn[m] + 1u) + tid : 0u;
         lin[m] = (on && mine) ? asGlobal(g.psm[m].outPost)[i] : 0.0f;
     }
     #pragma unroll
     for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) { csAmp[c] = (c < numCS) ? g.cs[c].amp : 0.0f; csKind[c] = (c < numCS) ? g.cs[c].kind : 0u; }
     #pragma unroll
-    for(uint32_t q = 0; q < 8; q++) { par[q] = g.params[q]; }
-    const uint32_t neuronModel = g.model;
+    for(uint32_t q = 0; q < 7; q++) { par[q] = inVector(g.params[q]); }
+    const bool lif = (g.model == GENNMI_NEURON_LIF);
     GLOBAL_AS uint32_t * const recordSpk = asGlobal(g.recordSpk);
     #pragma unroll
     for(uint32_t m = 0; m < NPSM; m++) {
         if(m >= numPSM) { break; }
-        const uint32_t D = psmDepth[m];
-        if(!D && main) { lds[psmIn[m] + tid] = lin[m]; }
+        const uint32_t D = g.psm[m].maxDenDelay, ringBase = T.ldsRing[m] + tid;
+        // (without a ring synapses add to inSyn itself, and what the register holds of it must add nothing: -0 + x is x, zeros included)
+        if(!D) { if(main) { lds[T.ldsIn[m] + tid] = lin[m]; } lin[m] = -0.0f; }
         // (sixteen slots' loads in flight at a time: one at a time, a ring of 43 slots is 43 memory round trips per launch)
         GLOBAL_AS const float *ring = asGlobal(g.psm[m].denDelay) + (mine ? i : 0u);
         for(uint32_t slot0 = 0; slot0 < D; slot0 += 16) {
@@ -286,7 +296,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             #pragma unroll
             for(uint32_t u = 0; u < 16; u++) { v[u] = (mine && slot0 + u < D) ? ring[(size_t)min(slot0 + u, D - 1) * n] : 0.0f; }
             #pragma unroll
-            for(uint32_t u = 0; u < 16; u++) { if(main && slot0 + u < D) { lds[psmRing[m] + (slot0 + u) * RES_T + tid] = v[u]; } }
+            for(uint32_t u = 0; u < 16; u++) { if(main && slot0 + u < D) { lds[ringBase + (slot0 + u) * TILE] = v[u]; } }
         }
     }
 
@@ -315,72 +325,68 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // A word slot is rewritten every second sequence number, and a launch continues the numbering of the one before
     // (seqBase), so a slot never holds the number a reader waits for before its writer has stored it: nothing is cleared
     // between launches.  A tile's spikes beyond those its word holds go through the side buffer, one 64-bit entry each that
-    // says which exchange it belongs to (the unwrapped sequence number, 56 bits, above the tile-local index): entries and
+    // says which exchange it belongs to (the unwrapped sequence number, 54 bits, above the tile-local index): entries and
     // word are stored in any order without a fence, and a reader that finds the word first waits for the entries.
     // (called by one wavefront)
+    GLOBAL_AS unsigned long long *tagOut = asGlobal(tags) + (size_t)(lane & (RES_REPLICAS - 1)) * replicaStride + blockIdx.x;
     auto publish = [&](uint32_t step, uint32_t count) {
-        const uint32_t seq = (uint32_t)((seqBase + step) & RES_SEQ_MASK);
-        const uint32_t parity = seq & 1u;
-        if(count > RES_WORD_IDS) {
-            for(uint32_t r = lane; r < count; r += WAVE) {
-                __hip_atomic_store(&side[((size_t)parity * numTiles + blockIdx.x) * RES_T + r], ((seqBase + step) << 8) | (shOwn[r] - tileFirst),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t seq = (uint32_t)(seqBase + step) & RES_SEQ_MASK, parity = seq & 1u;
+        uint32_t locals = 0;
+        if(count) {
+            if(count > RES_WORD_IDS) {
+                for(uint32_t r = lane; r < count; r += WAVE) {
+                    __hip_atomic_store(&side[((size_t)parity * numTiles + blockIdx.x) * TILE + r], ((seqBase + step) << RES_ID_BITS) | (shOwn[r] - tileFirst),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
+            for(uint32_t e = 0; e < min(count, RES_WORD_IDS); e++) { locals |= (shOwn[e] - tileFirst) << (RES_ID_BITS * e); }
         }
-        if(lane < RES_REPLICAS) {
-            uint32_t locals = 0;
-            for(uint32_t e = 0; e < min(count, RES_WORD_IDS); e++) { locals |= (shOwn[e] - tileFirst) << (8 * e); }
-            const unsigned long long word = ((unsigned long long)seq << RES_SEQ_SHIFT) | ((unsigned long long)count << 32) | locals;
-            __hip_atomic_store(&tags[(size_t)lane * replicaStride + (size_t)parity * numTiles + blockIdx.x], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        const unsigned long long word = ((unsigned long long)((seq << RES_COUNT_BITS) | count) << 32) | locals;
+        if(lane < RES_REPLICAS) { __hip_atomic_store(tagOut + (parity ? numTiles : 0u), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
     };
 
-    // Source tiles this thread watches and, of each, the spikes it takes.  More than 128 tiles: tiles tid, tid + 256, ..., all
-    // their spikes.  Fewer tiles than half the threads: several threads watch the same tile and deal its spikes between them.
+    // The source tile this thread watches and the spikes it takes of it: all of them, or, where there are fewer tiles than half the threads,
+    // those that fall to it among the threads that watch the same one.
     uint32_t perTile = 1, perShift = 0, watchTile = tid, watchSub = 0;
-    if(WATCH == 1 && numTiles <= BLOCK / 2) {
+    if((TILE & (TILE - 1)) == 0 && numTiles <= TILE / 2) {
         const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u);       // (tiles rounded up to a power of two)
-        perTile = BLOCK >> shift; perShift = 8 - shift;
-        static_assert(BLOCK == 1 << 8, "threads per watched tile");
+        perTile = TILE >> shift; perShift = 31u - (uint32_t)__clz(perTile);
         watchTile = tid & ((1u << shift) - 1u); watchSub = tid >> shift;
     }
-    uint32_t watchProj0[WATCH], watchNumProj[WATCH], watchFirst[WATCH], watchLds[WATCH];
-    GLOBAL_AS const u32x4 *watchSeg[WATCH];              // entry of the tile's first neuron under its group's first projection into this tile
-    uint32_t watchFlags[WATCH];                          // that projection's number << 26
+    const bool watching = main && watchTile < numTiles;
     const uint32_t narrowStride = 2u * tilesInGroup;     // entries of consecutive rows, in quads
-    #pragma unroll
-    for(uint32_t q = 0; q < WATCH; q++) {
-        const uint32_t k = main ? watchTile + q * BLOCK : numTiles;
-        watchFirst[q] = (k < numTiles) ? tiles[k].first : 0u;
-        const uint32_t s = (k < numTiles) ? tileGroup[k] : 0u;
-        watchProj0[q] = shProjStart[s];
-        watchNumProj[q] = (k < numTiles) ? shProjStart[s + 1] - watchProj0[q] : 0u;
-        watchSeg[q] = nullptr; watchFlags[q] = 0; watchLds[q] = 0;
-        if(watchNumProj[q]) {
-            const uint32_t p = shProjIdx[watchProj0[q]];
+    const uint32_t watchFirst = watching ? tiles[watchTile].first : 0u;
+    uint32_t watchProj0 = 0, watchNumProj = 0, watchLds = 0, watchFlags = 0;             // (flags: the first projection's number << 26)
+    GLOBAL_AS const u32x4 *watchSeg = nullptr;           // entry of the tile's first neuron under its group's first projection into this tile
+    if(watching) {
+        const uint32_t s = tileGroup[watchTile];
+        watchProj0 = shProjStart[s];
+        watchNumProj = shProjStart[s + 1] - watchProj0;
+        if(watchNumProj) {
+            const uint32_t p = shProjIdx[watchProj0];
             const uint32_t quads = (WIDE && shProj[p].wide) ? RES_WIDE_QUADS : 2u;
-            watchSeg[q] = asGlobal(shProj[p].seg) + quads * ((size_t)watchFirst[q] * tilesInGroup + tileInGroup);
-            watchFlags[q] = p << RES_SEG_PROJ_SHIFT;
-            watchLds[q] = shProj[p].lds;
+            watchSeg = asGlobal(shProj[p].seg) + quads * ((size_t)watchFirst * tilesInGroup + tileInGroup);
+            watchFlags = p << RES_SEG_PROJ_SHIFT;
+            watchLds = shProj[p].lds;
         }
     }
 
     // spikes of a word whose entries a thread has in flight at a time
-    constexpr uint32_t FLIGHT = (WATCH * (1 + WALK * WAVE / BLOCK) <= 2) ? 4 : (WATCH <= 2) ? 2 : 1;
-    // Entries e0, e0 + stepE, ... (FLIGHT of them, below c) of a tile's side list of the exchange `full`: waits, bounded, until each says so
-    auto sideIds = [&](uint32_t tile, uint32_t e0, uint32_t stepE, uint32_t c, unsigned long long full, uint32_t parity, uint32_t (&local)[FLIGHT]) -> bool {
-        const unsigned long long *base = side + ((size_t)parity * numTiles + tile) * RES_T + e0;
-        const unsigned long long want = full & 0x00FFFFFFFFFFFFFFull;
+    constexpr uint32_t FLIGHT = (THREADS <= 512) ? 3 : 1;
+    // Entries e0, e0 + perTile, ... (FLIGHT of them, below c) of the watched tile's side list of the exchange `full`: waits, bounded, until each says so
+    auto sideIds = [&](uint32_t e0, uint32_t c, unsigned long long full, uint32_t parity, uint32_t (&local)[FLIGHT]) -> bool {
+        const unsigned long long *base = side + ((size_t)parity * numTiles + watchTile) * TILE + e0;
+        const unsigned long long want = full & (~0ull >> RES_ID_BITS);
         uint32_t need = 0, spins = 0;
         #pragma unroll
-        for(uint32_t u = 0; u < FLIGHT; u++) { if(e0 + u * stepE < c) { need |= 1u << u; } }
+        for(uint32_t u = 0; u < FLIGHT; u++) { if(e0 + u * perTile < c) { need |= 1u << u; } }
         unsigned long long v[FLIGHT];
         while(true) {
             #pragma unroll
-            for(uint32_t u = 0; u < FLIGHT; u++) { v[u] = 0; if(need & (1u << u)) { v[u] = __hip_atomic_load(base + u * stepE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); } }
+            for(uint32_t u = 0; u < FLIGHT; u++) { v[u] = 0; if(need & (1u << u)) { v[u] = __hip_atomic_load(base + u * perTile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); } }
             #pragma unroll
             for(uint32_t u = 0; u < FLIGHT; u++) {
-                if((need & (1u << u)) && (v[u] >> 8) == want) { local[u] = (uint32_t)v[u] & 0xFFu; need &= ~(1u << u); }
+                if((need & (1u << u)) && (v[u] >> RES_ID_BITS) == want) { local[u] = (uint32_t)v[u] & RES_ID_MASK; need &= ~(1u << u); }
             }
             if(!need) { return true; }
             if(++spins > c_spinLimit) { return false; }
@@ -398,10 +404,11 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         if(lo4.y & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
         if(count) { events += lo4.y & 0xFFFFu; }
         const uint32_t numFront = skipInline ? 0u : (lo4.y >> 16) & 0xFFu;
+        if(!__any(numFront != 0u)) { return; }
         const uint32_t w[RES_FRONT_MAX] = {lo4.z, lo4.w, hi4.x, hi4.y};
         #pragma unroll
         for(uint32_t f = 0; f < RES_FRONT_MAX; f++) {
-            if(f < numFront) { unsafeAtomicAdd(&lds[frontBase + ((hi4.z >> (8 * f)) & 0xFFu)], __uint_as_float(w[f])); }
+            if(f < numFront) { unsafeAtomicAdd(reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + (4u * frontBase + (((f & 2) ? hi4.w : hi4.z) >> (16 * (f & 1)) & 0xFFFFu))), __uint_as_float(w[f])); }
         }
     };
     auto takeWide = [&](GLOBAL_AS const u32x4 *entry, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
@@ -425,7 +432,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     auto takeEntry = [&](uint32_t id, uint32_t p, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
         const ResProj &P = shProj[p];
         const size_t row = (size_t)id * tilesInGroup + tileInGroup;
-        const uint32_t frontBase = P.lds + shProjPtr[slot][p] * RES_T;
+        const uint32_t frontBase = P.lds + shProjPtr[slot][p];
         if(WIDE && P.wide) { takeWide(asGlobal(P.seg) + RES_WIDE_QUADS * row, p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count); }
         else {
             GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + 2 * row;
@@ -435,55 +442,35 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
 
     // Waits for every tile's word of exchange `step` (main threads; shTaken says when the bounded wait expired somewhere) and takes the
     // (spike, projection) pairs that concern this tile: lists them and — `convention` PASS_ALL or PASS_DUE — adds the due synapses
-    // their entries hold.  Pairs that find no place in the list are left to leftOver() (`left`: this thread's words that have some).
-    unsigned long long word[WATCH];
-    #pragma unroll
-    for(uint32_t q = 0; q < WATCH; q++) { word[q] = 0; }
-    uint32_t left = 0;
+    // their entries hold.  Pairs that find no place in the list are left to leftOver() (`left`: this thread's are).
+    unsigned long long word = 0;
+    bool left = false;
+    auto spikesOf = [&]() -> uint32_t { return (uint32_t)(word >> 32) & RES_COUNT_MASK; };
+    auto idOf = [&](uint32_t e) -> uint32_t { return ((uint32_t)word >> (RES_ID_BITS * e)) & RES_ID_MASK; };        // (e < RES_WORD_IDS)
     auto poll = [&](uint32_t step, uint32_t convention) {
-        const uint32_t seq = (uint32_t)((seqBase + step) & RES_SEQ_MASK);
+        const uint32_t seq = (uint32_t)(seqBase + step) & RES_SEQ_MASK;
         const uint32_t parity = seq & 1u, slot = seq & 3u;
         const bool skipInline = (convention == PASS_LATER), count = (convention != PASS_DUE);
         bool ok = true;
-        uint32_t pending = 0;
-        left = 0;
-        #pragma unroll
-        for(uint32_t q = 0; q < WATCH; q++) { word[q] = 0; if(watchTile + q * BLOCK < numTiles) { pending |= 1u << q; } }
-        const unsigned long long *mine_ = myTags + (size_t)parity * numTiles + watchTile;
-        uint32_t spins = 0;
-        while(pending) {
-            #pragma unroll
-            for(uint32_t q = 0; q < WATCH; q++) {
-                if(pending & (1u << q)) { word[q] = __hip_atomic_load(mine_ + q * BLOCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+        left = false;
+        word = 0;
+        if(watching) {
+            const unsigned long long *mine_ = myTags + (parity ? numTiles : 0u) + watchTile;
+            uint32_t spins = 0;
+            while(true) {
+                word = __hip_atomic_load(mine_, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if((uint32_t)(word >> (32 + RES_COUNT_BITS)) == seq) { break; }
+                ++spins;
+                if(spins > c_spinLimit || ((spins & 255u) == 0 && __hip_atomic_load(errorFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) { ok = false; word = 0; break; }
+                __builtin_amdgcn_s_sleep(1);
             }
-            #pragma unroll
-            for(uint32_t q = 0; q < WATCH; q++) {
-                if((pending & (1u << q)) && (uint32_t)(word[q] >> RES_SEQ_SHIFT) == seq) { pending &= ~(1u << q); }
-            }
-            if(!pending) { break; }
-            ++spins;
-            if(spins > c_spinLimit || ((spins & 255u) == 0 && __hip_atomic_load(errorFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) { ok = false; break; }
-            __builtin_amdgcn_s_sleep(1);
         }
-        if(convention != PASS_NONE) {
-            // this thread's pairs, and the word they come from when it is only one
-            uint32_t total = 0, mineCount[WATCH];
-            bool several = false;
-            unsigned long long busyWord = 0;
-            uint32_t busyFlags = 0, busyLds = 0;
-            GLOBAL_AS const u32x4 *busySeg = nullptr;
-            #pragma unroll
-            for(uint32_t q = 0; q < WATCH; q++) {
-                const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu, np = watchNumProj[q];
-                mineCount[q] = (ok && c > watchSub && np != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u;
-                if(mineCount[q]) {
-                    several = total != 0 || c > RES_WORD_IDS || np > 1 || mineCount[q] > FLIGHT;
-                    total += mineCount[q] * np;
-                    busyWord = word[q]; busyFlags = watchFlags[q]; busyLds = watchLds[q]; busySeg = watchSeg[q];
-                }
-            }
-            if(__any(several)) {
-                // Some thread of the wavefront has pairs from several words, or many: the wavefront lists its pairs first and every
+        const uint32_t c = spikesOf();
+        if(convention != PASS_NONE && __any(c != 0u)) {
+            // this thread's pairs
+            const uint32_t mineCount = (c > watchSub && watchNumProj != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u, total = mineCount * watchNumProj;
+            if(__any(total != 0u && (c > RES_WORD_IDS || watchNumProj > 1 || mineCount > FLIGHT))) {
+                // Some thread of the wavefront has many pairs: the wavefront lists its pairs first and every
                 // lane then takes as many of them as every other, so that their entries are one trip to memory and not one after another.
                 const uint32_t inclusive = waveInclusiveScanU32(total, lane);
                 const uint32_t waveTotal = (uint32_t)__builtin_amdgcn_readlane((int)inclusive, WAVE - 1);
@@ -492,23 +479,18 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                 base = __builtin_amdgcn_readfirstlane(base);
                 const bool fits = (base + waveTotal <= RES_PAIR_CAP);
                 uint32_t pos = base + inclusive - total;
-                #pragma unroll
-                for(uint32_t q = 0; q < WATCH; q++) {
-                    if(!mineCount[q]) { continue; }
-                    if(!fits) { left |= 1u << q; }
-                    const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu;
-                    for(uint32_t e0 = watchSub; e0 < c && ok; e0 += FLIGHT * perTile) {
-                        uint32_t local[FLIGHT];
-                        #pragma unroll
-                        for(uint32_t u = 0; u < FLIGHT; u++) { local[u] = ((uint32_t)word[q] >> (8 * ((e0 + u * perTile) & 3u))) & 0xFFu; }
-                        // (also when the pairs do not fit and leftOver() will read the list again: once seen here, an entry is there
-                        // for every later read of this thread)
-                        if(c > RES_WORD_IDS && !sideIds(watchTile + q * BLOCK, e0, perTile, c, seqBase + step, parity, local)) { ok = false; }
-                        #pragma unroll
-                        for(uint32_t u = 0; u < FLIGHT; u++) {
-                            if(!fits || e0 + u * perTile >= c) { break; }
-                            for(uint32_t j = 0; j < watchNumProj[q]; j++) { shSeg[slot & 1][pos++] = make_uint2(watchFirst[q] + local[u], shProjIdx[watchProj0[q] + j]); }
-                        }
+                left = !fits && total != 0;
+                for(uint32_t e0 = watchSub; total != 0 && e0 < c && ok; e0 += FLIGHT * perTile) {
+                    uint32_t local[FLIGHT];
+                    #pragma unroll
+                    for(uint32_t u = 0; u < FLIGHT; u++) { local[u] = (e0 + u * perTile < RES_WORD_IDS) ? idOf(e0 + u * perTile) : 0u; }
+                    // (also when the pairs do not fit and leftOver() will read the list again: once seen here, an entry is there
+                    // for every later read of this thread)
+                    if(c > RES_WORD_IDS && !sideIds(e0, c, seqBase + step, parity, local)) { ok = false; }
+                    #pragma unroll
+                    for(uint32_t u = 0; u < FLIGHT; u++) {
+                        if(!fits || e0 + u * perTile >= c) { break; }
+                        for(uint32_t j = 0; j < watchNumProj; j++) { shSeg[slot & 1][pos++] = make_uint2(watchFirst + local[u], shProjIdx[watchProj0 + j]); }
                     }
                 }
                 if(!fits) {
@@ -527,31 +509,31 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                 }
             }
             else if(total) {
-                // up to FLIGHT spikes of one tile under one projection: their entries are asked for before they have their place in the list
-                const bool narrow = !WIDE || !shProj[busyFlags >> RES_SEG_PROJ_SHIFT].wide;
+                // up to FLIGHT spikes of the tile under one projection: their entries are asked for before they have their place in the list
+                const bool narrow = !WIDE || !shProj[watchFlags >> RES_SEG_PROJ_SHIFT].wide;
                 uint32_t local[FLIGHT];
                 u32x4 lo4[FLIGHT], hi4[FLIGHT];
                 #pragma unroll
                 for(uint32_t u = 0; u < FLIGHT; u++) {
-                    local[u] = ((uint32_t)busyWord >> (8 * ((watchSub + u * perTile) & 3u))) & 0xFFu;
+                    const uint32_t e = watchSub + u * perTile;
+                    local[u] = (e < RES_WORD_IDS) ? idOf(e) : 0u;
                     if(narrow && u < total) {
-                        GLOBAL_AS const u32x4 *entry = busySeg + (size_t)local[u] * narrowStride;
+                        GLOBAL_AS const u32x4 *entry = watchSeg + (size_t)local[u] * narrowStride;
                         lo4[u] = entry[0]; hi4[u] = entry[1];
                     }
                 }
                 const uint32_t pos = atomicAdd(&shTaken[slot].pairs, total);
                 if(pos + total <= RES_PAIR_CAP) {
-                    const uint32_t frontBase = busyLds + shProjPtr[slot][busyFlags >> RES_SEG_PROJ_SHIFT] * RES_T;
+                    const uint32_t frontBase = watchLds + shProjPtr[slot][watchFlags >> RES_SEG_PROJ_SHIFT];
                     #pragma unroll
                     for(uint32_t u = 0; u < FLIGHT; u++) {
                         if(u >= total) { break; }
-                        if(narrow) { takeNarrow(lo4[u], hi4[u], busyFlags, frontBase, slot, pos + u, skipInline, count); }
-                        else if(WIDE) { takeWide(busySeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), busyFlags, frontBase, slot, pos + u, skipInline, count); }
+                        if(narrow) { takeNarrow(lo4[u], hi4[u], watchFlags, frontBase, slot, pos + u, skipInline, count); }
+                        else if(WIDE) { takeWide(watchSeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), watchFlags, frontBase, slot, pos + u, skipInline, count); }
                     }
                 }
                 else {
-                    #pragma unroll
-                    for(uint32_t q = 0; q < WATCH; q++) { if(mineCount[q]) { left |= 1u << q; } }
+                    left = true;
                     for(uint32_t r = pos; r < RES_PAIR_CAP; r++) { shSeg[slot & 1][r] = make_uint2(0u, 0u); }
                     shTaken[slot].left = 1u;
                 }
@@ -570,7 +552,8 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // segments whose due synapses are not all inline in their entry.
     // (wavefront `first` of the `count` that call)
     auto process = [&](const uint2 *segs, const uint32_t *fronts, uint32_t numPairs, uint32_t pass, bool flaggedOnly, uint32_t first, uint32_t count) {
-        constexpr uint32_t TRIP = 8;
+        constexpr uint32_t TRIP = 4, DUE_END = 4 * TILE;
+        const uint32_t from = (pass == PASS_LATER) ? DUE_END : 0u, span = (pass == PASS_DUE) ? DUE_END : 0xFFFFFFFFu - from;      // offsets that are added
         const uint32_t shift = (numPairs <= 4 * count) ? 4u : (numPairs <= 8 * count) ? 3u : 2u;
         const uint32_t lanesPerPair = 1u << shift, pairsPerGroup = WAVE >> shift;
         for(uint32_t q0 = first * pairsPerGroup; q0 < numPairs; q0 += count * pairsPerGroup) {
@@ -581,43 +564,36 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                 proj = sg.y >> RES_SEG_PROJ_SHIFT;
                 const bool flagged = (sg.y & RES_SEG_OVERFLOW) != 0;
                 const bool skip = (flaggedOnly && !flagged) || (pass == PASS_LATER && (sg.y & RES_SEG_NO_DELAY));
-                start = sg.x; len = skip ? 0u : (sg.y & 0xFFFFu);
+                len = skip ? 0u : (sg.y & 0xFFFFu);
+                start = len ? sg.x : 0u;                          // (an empty part may start where the array ends)
             }
             const ResProj &P = shProj[proj];
-            const uint32_t depth = P.D, front = fronts[proj], ldsBase = P.lds, magic = P.magic;
+            const uint32_t front = 4u * fronts[proj], ringBytes = 4u * TILE * P.D, ldsBase = 4u * P.lds;
             GLOBAL_AS const u32x2 *packed = asGlobal(P.packed) + start;
+            const uint32_t last = len ? len - 1u : 0u;
             for(uint32_t i0 = lane & (lanesPerPair - 1); __any(i0 < len); i0 += TRIP * lanesPerPair) {
+                // (a lane beyond the part's end reads its last record again: no branch between the loads)
                 u32x2 rec[TRIP];
                 #pragma unroll
-                for(uint32_t u = 0; u < TRIP; u++) {
-                    const uint32_t i = i0 + u * lanesPerPair;
-                    rec[u].x = 0x80000000u; rec[u].y = 0u;               // (no synapse)
-                    if(i < len) { rec[u] = packed[i]; }
-                }
+                for(uint32_t u = 0; u < TRIP; u++) { rec[u] = packed[min(i0 + u * lanesPerPair, last)]; }
                 #pragma unroll
                 for(uint32_t u = 0; u < TRIP; u++) {
-                    if(rec[u].x >> 31) { continue; }
-                    const uint32_t x = front + (rec[u].x >> 8);              // far below 2^16: the ring fits the LDS, a delay is a byte
-                    const uint32_t slot = depth ? x - __umulhi(x, magic) * depth : 0u;
-                    const bool due = !depth || (slot == front);
-                    if((pass == PASS_LATER && due) || (pass == PASS_DUE && !due)) { continue; }
-                    unsafeAtomicAdd(&lds[ldsBase + slot * RES_T + (rec[u].x & 0xFFu)], __uint_as_float(rec[u].y));
+                    uint32_t at = front + rec[u].x;                          // (a multiple of four below twice the ring's bytes)
+                    at = min(at, at - ringBytes);                             // (at < ringBytes: the difference wraps round)
+                    if(i0 + u * lanesPerPair < len && rec[u].x - from < span) {
+                        unsafeAtomicAdd(reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + (ldsBase + at)), __uint_as_float(rec[u].y));
+                    }
                 }
             }
         }
     };
 
-    // The pairs of the words that found no place in the list: listed and walked RES_PAIR_CAP at a time, in full, before the
+    // The pairs that found no place in the list: listed and walked RES_PAIR_CAP at a time, in full, before the
     // update (in the other parity's list: its pairs were walked before this exchange's words were looked for, and the next
     // exchange's threads come here first).
     auto leftOver = [&](uint32_t step, uint32_t pass, bool count) {
         const uint32_t slot = (uint32_t)(seqBase + step) & 3u, parity = slot & 1u, other = parity ^ 1u;
-        uint32_t want = 0;
-        #pragma unroll
-        for(uint32_t q = 0; q < WATCH; q++) {
-            const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu;
-            if(left & (1u << q)) { want += ((c - watchSub + perTile - 1) / perTile) * watchNumProj[q]; }
-        }
+        const uint32_t c = spikesOf(), want = left ? ((c - watchSub + perTile - 1) >> perShift) * watchNumProj : 0u;
         const uint32_t inclusive = waveInclusiveScanU32(want, lane);
         if(lane == WAVE - 1) { shWave[wave] = inclusive; }
         __syncthreads();
@@ -626,17 +602,12 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         for(uint32_t w = 0; w < WAVES; w++) { if(w < wave) { base += shWave[w]; } total += shWave[w]; }
         for(uint32_t chunk0 = 0; chunk0 < total; chunk0 += RES_PAIR_CAP) {
             uint32_t pos = base;
-            #pragma unroll
-            for(uint32_t q = 0; q < WATCH; q++) {
-                if(!(left & (1u << q))) { continue; }
-                const uint32_t c = (uint32_t)(word[q] >> 32) & 0x1FFu, np = watchNumProj[q];
-                const uint32_t mineCount = (c - watchSub + perTile - 1) / perTile;
-                if(pos + mineCount * np <= chunk0 || pos >= chunk0 + RES_PAIR_CAP) { pos += mineCount * np; continue; }
+            if(left && pos + want > chunk0 && pos < chunk0 + RES_PAIR_CAP) {
                 for(uint32_t e = watchSub; e < c; e += perTile) {
-                    const uint32_t id = (c <= RES_WORD_IDS) ? watchFirst[q] + (((uint32_t)word[q] >> (8 * e)) & 0xFFu)
-                                                            : watchFirst[q] + ((uint32_t)__hip_atomic_load(&side[((size_t)parity * numTiles + watchTile + q * BLOCK) * RES_T + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFFu);
-                    for(uint32_t j = 0; j < np; j++, pos++) {
-                        if(pos >= chunk0 && pos < chunk0 + RES_PAIR_CAP) { shSeg[other][pos - chunk0] = make_uint2(id, shProjIdx[watchProj0[q] + j]); }
+                    const uint32_t id = watchFirst + ((c <= RES_WORD_IDS) ? idOf(e)
+                                                                          : (uint32_t)__hip_atomic_load(&side[((size_t)parity * numTiles + watchTile) * TILE + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & RES_ID_MASK);
+                    for(uint32_t j = 0; j < watchNumProj; j++, pos++) {
+                        if(pos >= chunk0 && pos < chunk0 + RES_PAIR_CAP) { shSeg[other][pos - chunk0] = make_uint2(id, shProjIdx[watchProj0 + j]); }
                     }
                 }
             }
@@ -662,7 +633,9 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     auto deliverDue = [&](uint32_t step, uint32_t convention) -> bool {
         const uint32_t slot = (uint32_t)(seqBase + step) & 3u;
         ldsBarrier();
-        const Taken taken = shTaken[slot];
+        Taken taken = shTaken[slot];
+        taken.pairs = __builtin_amdgcn_readfirstlane(taken.pairs); taken.flagged = __builtin_amdgcn_readfirstlane(taken.flagged);
+        taken.left = __builtin_amdgcn_readfirstlane(taken.left); taken.failed = __builtin_amdgcn_readfirstlane(taken.failed);
         later = min(taken.pairs, RES_PAIR_CAP);
         if(taken.flagged | taken.left | taken.failed) {
             if(taken.failed) {
@@ -677,9 +650,13 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
 
     bool anyRing = false;
     for(uint32_t q = 0; q < numProj; q++) { anyRing = anyRing || shProj[q].D != 0; }
-    unsigned long long recT = numRecordingTimesteps ? (((timestep0 | numRecordingTimesteps) >> 32) ? timestep0 % numRecordingTimesteps
-                                                                                                    : (uint32_t)timestep0 % (uint32_t)numRecordingTimesteps) : 0ull;
-    const uint32_t recordWords = (n + 31) / 32;
+    // where the coming step's recording word of this half wavefront goes, and the steps until the buffer wraps
+    const unsigned long long recT = numRecordingTimesteps ? (((timestep0 | numRecordingTimesteps) >> 32) ? timestep0 % numRecordingTimesteps
+                                                                                                          : (uint32_t)timestep0 % (uint32_t)numRecordingTimesteps) : 0ull;
+    const uint32_t recordWords = numRecordingTimesteps ? (n + 31) / 32 : 0u;
+    const bool recordHere = recordSpk != nullptr && (lane & 31) == 0 && mine;
+    GLOBAL_AS uint32_t *recordAt = recordSpk + (size_t)recT * recordWords + (i >> 5);
+    uint32_t recordLeft = (uint32_t)min(numRecordingTimesteps - recT, 0xFFFFFFFFull);       // (a launch has fewer steps than this can count)
     // ---- exchange the spikes that precede the first step, then step
     if(wave == 0) { publish(1u, ownCount); }
     bool ok = true;
@@ -700,63 +677,45 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         if(!deliverDue(k + 1, convention)) { ok = false; break; }
         if(wave == WAVES - 1) {
-            if(lane < numProj) { shProjPtr[afterNext][lane] = ptrNext; }
+            if(lane < numProj) { shProjPtr[afterNext][lane] = ptrNext * TILE; }
             if(lane == 0) { shTaken[afterNext] = Taken{0u, 0u, 0u, 0u}; shDone[afterNext] = 0u; }
             ptrNext = (ptrNext + 1 >= ptrDepth) ? 0u : ptrNext + 1;
         }
         if(main) {
-        // neuron update: same operations in the same order as neuronBody
+        // neuron update: same operations in the same order as neuronBody, as selections instead of branches
         bool spiked = false;
-        if(mine) {
-            float Isyn = 0;
-            #pragma unroll
-            for(uint32_t m = 0; m < NPSM; m++) {
-                if(m >= numPSM) { break; }
-                float linSyn;
-                if(psmDepth[m]) {
-                    const uint32_t front = psmRing[m] + psmFront[m] * RES_T + tid;
-                    linSyn = lin[m] + lds[front];
-                    lds[front] = 0.0f;
-                }
-                else { linSyn = lds[psmIn[m] + tid]; }
-                if(psmKind[m] == GENNMI_PSM_EXPCURR) {
-                    Isyn += psmInit[m] * linSyn;
-                    linSyn *= psmDecay[m];
-                }
-                else {
-                    Isyn += linSyn;
-                    linSyn = 0.0f;
-                }
-                if(psmDepth[m]) { lin[m] = linSyn; }
-                else { lds[psmIn[m] + tid] = linSyn; }
-            }
-            #pragma unroll
-            for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
-                if(c >= numCS) { break; }
-                Isyn += POISSON ? inject[c] : csAmp[c];
-            }
-            if(neuronModel == GENNMI_NEURON_LIF) {
-                if(l1 <= 0.0f) {
-                    const float alpha = ((Isyn + par[0]) * par[1]) + par[2];
-                    l0 = alpha - (par[3] * (alpha - l0));
-                }
-                else {
-                    l1 -= dt;
-                }
-                spiked = (l1 <= 0.0f && l0 >= par[4]);
-                if(spiked) { l0 = par[5]; l1 = par[6]; }
-            }
-            else {
-                if(l0 >= 30.0f) {
-                    l0 = par[2];
-                    l1 += par[3];
-                }
-                l0 += 0.5f * (0.04f * l0 * l0 + 5.0f * l0 + 140.0f - l1 + Isyn) * dt;
-                l0 += 0.5f * (0.04f * l0 * l0 + 5.0f * l0 + 140.0f - l1 + Isyn) * dt;
-                l1 += par[0] * (par[1] * l0 - l1) * dt;
-                if(l0 > 30.0f) { l0 = 30.0f; }
-                spiked = (l0 >= 29.99f);
-            }
+        float Isyn = 0;
+        #pragma unroll
+        for(uint32_t m = 0; m < NPSM; m++) {
+            if(m >= numPSM) { break; }
+            const bool ring = (psmRing[m] != 0u);
+            const float linSyn = lin[m] + lds[psmAt[m]];
+            const float decayed = psmExp[m] ? linSyn * psmDecay[m] : 0.0f;
+            Isyn += psmInit[m] * linSyn;
+            lds[psmAt[m]] = ring ? 0.0f : decayed;
+            lin[m] = ring ? decayed : -0.0f;
+        }
+        #pragma unroll
+        for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
+            if(c >= numCS) { break; }
+            Isyn += POISSON ? inject[c] : csAmp[c];
+        }
+        if(lif) {
+            const bool active = (l1 <= 0.0f);
+            const float alpha = ((Isyn + par[0]) * par[1]) + par[2];
+            l0 = active ? alpha - (par[3] * (alpha - l0)) : l0;
+            l1 = active ? l1 : l1 - dt;
+            spiked = (mine && l1 <= 0.0f && l0 >= par[4]);
+            l0 = spiked ? par[5] : l0; l1 = spiked ? par[6] : l1;
+        }
+        else {
+            const bool reset = (l0 >= 30.0f);
+            l0 = reset ? par[2] : l0; l1 = reset ? l1 + par[3] : l1;
+            l0 += 0.5f * (0.04f * l0 * l0 + 5.0f * l0 + 140.0f - l1 + Isyn) * dt;
+            l0 += 0.5f * (0.04f * l0 * l0 + 5.0f * l0 + 140.0f - l1 + Isyn) * dt;
+            l1 += par[0] * (par[1] * l0 - l1) * dt;
+            l0 = (l0 > 30.0f) ? 30.0f : l0;
+            spiked = (mine && l0 >= 29.99f);
         }
         // (a wavefront without spikes, which nearly all are, only says that it is done)
         const unsigned long long ballot = __ballot(spiked);
@@ -782,12 +741,14 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         // while the words of this step travel: the step's recording words, and (next) the synapses of the previous step's spikes
         // that are not due yet
-        if(recordSpk && (lane & 31) == 0 && mine) { recordSpk[(size_t)recT * recordWords + (i >> 5)] = (uint32_t)(ballot >> (lane & 32)); }
-        if(numRecordingTimesteps) { recT = (recT + 1 == numRecordingTimesteps) ? 0ull : recT + 1; }
+        if(recordHere) { *recordAt = (lane & 32) ? (uint32_t)(ballot >> 32) : (uint32_t)ballot; }
+        recordAt += recordWords;
+        if(--recordLeft == 0u) { recordAt = recordSpk + (i >> 5); recordLeft = (uint32_t)min(numRecordingTimesteps, 0xFFFFFFFFull); }
         #pragma unroll
         for(uint32_t m = 0; m < NPSM; m++) {
             if(m >= numPSM) { break; }
-            psmFront[m] = (psmFront[m] + 1 >= psmDepth[m]) ? 0u : psmFront[m] + 1;
+            const uint32_t next = psmAt[m] + TILE;
+            psmAt[m] = (next >= psmEnd[m]) ? psmAt[m] + (psmRing[m] ? TILE - psmRing[m] : 0u) : next;
         }
         }
         if((WALK == 0 || !main) && anyRing && later) {       // (without a ring nothing is: the next word is looked for at once)
@@ -815,19 +776,14 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     #pragma unroll
     for(uint32_t m = 0; m < NPSM; m++) {
         if(m >= numPSM) { break; }
-        const uint32_t D = psmDepth[m];
-        if(mine) { asGlobal(g.psm[m].outPost)[i] = D ? lin[m] : lds[psmIn[m] + tid]; }
+        const uint32_t D = g.psm[m].maxDenDelay;
+        if(mine) { asGlobal(g.psm[m].outPost)[i] = D ? lin[m] : lds[T.ldsIn[m] + tid]; }
         for(uint32_t slot = 0; slot < D; slot++) {
-            if(mine) { asGlobal(g.psm[m].denDelay)[(size_t)slot * n + i] = lds[psmRing[m] + slot * RES_T + tid]; }
+            if(mine) { asGlobal(g.psm[m].denDelay)[(size_t)slot * n + i] = lds[T.ldsRing[m] + slot * TILE + tid]; }
         }
         if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
     }
-    uint32_t offset = 0;
-    #pragma unroll
-    for(uint32_t q = 0; q < WATCH; q++) {
-        const uint32_t tile = watchTile + q * BLOCK;
-        if(main && watchSub == 0 && tile >= T.firstTileOfGroup && tile < T.firstTileOfGroup + tileInGroup) { offset += (uint32_t)(word[q] >> 32) & 0x1FFu; }
-    }
+    uint32_t offset = (watching && watchSub == 0 && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
     if(tid == 0) { shScalar[2] = 0; }
     __syncthreads();
     if(offset) { atomicAdd(&shScalar[2], offset); }

@@ -363,8 +363,8 @@ def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypat
     (130000, 1000, 3, 1, False), (130800, 500, 2, 1, True), (130800, 500, 0, 1, False),                           # two tiles a thread, and more
     (5000, 700, 0, 3, False), (5000, 700, 6, 3, False), (70000, 700, 3, 3, True), (131000, 600, 0, 3, False)])     # more than two postsynaptic models
 def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
-    """Which of the kernel's instances runs depends on the number of tiles (256 neurons each), rings, postsynaptic models a population and sources;
-    a ring of one slot is a case of its own (everything is due at once).  Every (target, postsynaptic model) has one projection: identical.
+    """Which of the kernel's instances runs depends on how many neurons a tile needs (256, 320, 512 or 1024 for a tile a compute unit), rings,
+    postsynaptic models a population and sources; a ring of one slot is a case of its own (everything is due at once).  Every (target, postsynaptic model) has one projection: identical.
     (The tile path adds a step's sums, not its weights one by one: the single steps in between go without it.)"""
     monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
     net = Net(name="resident_tiles", dt=1.0, steps=0)
