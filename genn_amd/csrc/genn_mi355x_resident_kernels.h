@@ -35,10 +35,11 @@ constexpr uint32_t RES_MAX_GROUPS = 64;      // neuron groups
 constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs a tile lists per exchange
 constexpr uint32_t RES_FRONT_MAX = 4;        // front-slot synapses held inline in a segment entry
 // Without a ring every synapse of a row part is due at once.  Where the parts are short they go into the entry whole: up to four into 32
-// bytes, up to 24 into a wide entry of 128 — one cache line, read where 32 bytes of it were — and the step is spared the second trip to
+// bytes, up to 22 into a wide entry of 128 — one cache line, read where 32 bytes of it were — and the step is spared the second trip to
 // memory, to the records, and a barrier.  us a step of a balanced network: 100,000 neurons x 80 targets 8.1 -> 6.7, 40,000 x 80 4.7 -> 4.3
-// (ordinary entries); 12,000 x 100 4.19 -> 4.00, 4,000 x 80 3.79 -> 3.62 (wide ones; 4.19 and 3.70 without).
-constexpr uint32_t RES_WIDE_QUADS = 8, RES_WIDE_MAX = 24;
+// (ordinary entries); 12,000 x 100 4.19 -> 4.00, 4,000 x 80 3.79 -> 3.62 (wide ones; 4.19 and 3.70 without), and 2.85 -> 2.47 since
+// eight lanes read a wide entry, a quad each, instead of one lane all of it.
+constexpr uint32_t RES_WIDE_QUADS = 8, RES_WIDE_MAX = 22, RES_WIDE_COUNT = 30;       // (shift of a quad's number of synapses)
 constexpr uint32_t RES_SEG_OVERFLOW = 1u << 24, RES_SEG_NO_DELAY = 1u << 25;
 constexpr uint32_t RES_SEG_PROJ_SHIFT = 26;  // in the kernel's list of pairs: the projection, above an entry's flags
 // word: upper half sequence number << 11 | count, lower half up to three tile-local neuron indices, 10 bits each
@@ -74,8 +75,9 @@ struct ResTile
 // targets (byte offsets, 16 bits each) of up to four synapses whose delay is a multiple of the ring depth.  Those land in the slot the target reads in
 // the very step that delivers them, so they are the only ones a step has to wait for; carrying them inside the entry
 // saves that step the dependent read of the row.  RES_SEG_OVERFLOW: the segment has more of them than fit (the row part
-// is then read at once); RES_SEG_NO_DELAY: the projection has no ring, every synapse is due at once.  A wide entry has words 0 and 1,
-// the targets of up to 24 synapses in words 2-7 (tiles of 256: indices of a byte each) and their weights in words 8-31.
+// is then read at once); RES_SEG_NO_DELAY: the projection has no ring, every synapse is due at once.  A wide entry is eight quads that
+// lanes read one each: the first has words 0 and 1, a weight and what the last word of every quad is, the targets (10 bits each)
+// and the number of the quad's synapses; the others have three weights and such a word.
 __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLength, const uint32_t *ind, const float *weight,
                                   const uint8_t *delay, uint32_t depth, uint32_t tileSize, uint32_t tilesInGroup, uint32_t wide, u32x4 *seg)
 {
@@ -91,19 +93,21 @@ __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uin
     };
     const uint32_t a = lowerBound(tile * tileSize), b = lowerBound((tile + 1) * tileSize);
     const uint32_t start = row * rowStride + a;
-    uint32_t flags = depth ? 0u : RES_SEG_NO_DELAY, numFront = 0, locals = 0;
+    uint32_t flags = depth ? 0u : RES_SEG_NO_DELAY, numFront = 0;
     if(wide) {
-        uint32_t *entry = reinterpret_cast<uint32_t*>(seg + RES_WIDE_QUADS * id);
         const uint32_t inside = (b - a <= RES_WIDE_MAX) ? b - a : 0u;
         if(b - a > RES_WIDE_MAX) { flags |= RES_SEG_OVERFLOW; }
-        entry[0] = start; entry[1] = min(b - a, 0xFFFFu) | (inside << 16) | flags;
-        for(uint32_t f = 0; f < RES_WIDE_MAX; f += 4) {
-            for(uint32_t q = f; q < f + 4; q++) {
-                if(q < inside) { locals |= (r[a + q] - tile * tileSize) << (8 * (q - f)); }
-                entry[8 + q] = (q < inside) ? __float_as_uint(weight[(size_t)row * rowStride + a + q]) : 0u;
+        uint32_t j = 0;
+        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) {
+            uint32_t x[4] = {0u, 0u, 0u, 0u};
+            if(q == 0) { x[0] = start; x[1] = min(b - a, 0xFFFFu) | (inside << 16) | flags; }
+            uint32_t n = 0;
+            for(uint32_t f = q ? 0u : 2u; f < 3 && j < inside; f++, j++, n++) {
+                x[f] = __float_as_uint(weight[(size_t)row * rowStride + a + j]);
+                x[3] |= (r[a + j] - tile * tileSize) << (RES_ID_BITS * n);
             }
-            entry[2 + f / 4] = locals;
-            locals = 0;
+            x[3] |= n << RES_WIDE_COUNT;
+            seg[RES_WIDE_QUADS * id + q] = u32x4{x[0], x[1], x[2], x[3]};
         }
         return;
     }
@@ -177,7 +181,7 @@ __device__ __forceinline__ void ldsBarrier()
 // What consecutive exchanges share exists once for each of them: pair lists twice, counters and ring fronts four times (those of the
 // exchange after the next are prepared behind the barrier, so no thread meets them half prepared).
 // POISSON: some population has a PoissonExp current source (its state then lives in a register per source and neuron);
-// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries (tiles of 256).
+// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries.
 // NPSM: postsynaptic models of any group.  TILE: neurons of a tile, and threads that own one.  WALK: wavefronts beyond those that
 // own the tile's neurons; 0: these walk too, once they have published.  With walkers nothing holds a wavefront back between its
 // update and the next exchange, so every projection must have a ring of two slots or more: what an early wavefront adds then goes to another slot
@@ -348,7 +352,15 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // The source tile this thread watches and the spikes it takes of it: all of them, or, where there are fewer tiles than half the threads,
     // those that fall to it among the threads that watch the same one.
     uint32_t perTile = 1, perShift = 0, watchTile = tid, watchSub = 0;
-    if((TILE & (TILE - 1)) == 0 && numTiles <= TILE / 2) {
+    // (wide entries are read by eight lanes each: with few enough tiles the eight watch the same one, `grouped`)
+    bool grouped = WIDE && numProj != 0 && numTiles <= TILE / RES_WIDE_QUADS;
+    for(uint32_t q = 0; grouped && q < numProj; q++) { grouped = shProj[q].wide != 0; }
+    if(grouped) {
+        const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u), group = tid / RES_WIDE_QUADS;
+        perTile = (TILE / RES_WIDE_QUADS) >> shift;
+        watchTile = group & ((1u << shift) - 1u); watchSub = group >> shift;
+    }
+    else if((TILE & (TILE - 1)) == 0 && numTiles <= TILE / 2) {
         const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u);       // (tiles rounded up to a power of two)
         perTile = TILE >> shift; perShift = 31u - (uint32_t)__clz(perTile);
         watchTile = tid & ((1u << shift) - 1u); watchSub = tid >> shift;
@@ -357,6 +369,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     const uint32_t narrowStride = 2u * tilesInGroup;     // entries of consecutive rows, in quads
     const uint32_t watchFirst = watching ? tiles[watchTile].first : 0u;
     uint32_t watchProj0 = 0, watchNumProj = 0, watchLds = 0, watchFlags = 0;             // (flags: the first projection's number << 26)
+    bool watchWide = false;
     GLOBAL_AS const u32x4 *watchSeg = nullptr;           // entry of the tile's first neuron under its group's first projection into this tile
     if(watching) {
         const uint32_t s = tileGroup[watchTile];
@@ -364,8 +377,8 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         watchNumProj = shProjStart[s + 1] - watchProj0;
         if(watchNumProj) {
             const uint32_t p = shProjIdx[watchProj0];
-            const uint32_t quads = (WIDE && shProj[p].wide) ? RES_WIDE_QUADS : 2u;
-            watchSeg = asGlobal(shProj[p].seg) + quads * ((size_t)watchFirst * tilesInGroup + tileInGroup);
+            watchWide = WIDE && shProj[p].wide;
+            watchSeg = asGlobal(shProj[p].seg) + (watchWide ? RES_WIDE_QUADS : 2u) * ((size_t)watchFirst * tilesInGroup + tileInGroup);
             watchFlags = p << RES_SEG_PROJ_SHIFT;
             watchLds = shProj[p].lds;
         }
@@ -411,21 +424,46 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             if(f < numFront) { unsafeAtomicAdd(reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + (4u * frontBase + (((f & 2) ? hi4.w : hi4.z) >> (16 * (f & 1)) & 0xFFFFu))), __uint_as_float(w[f])); }
         }
     };
-    auto takeWide = [&](GLOBAL_AS const u32x4 *entry, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
-        uint32_t e[4 * RES_WIDE_QUADS];
+    // A wide entry, by eight consecutive lanes with the same arguments: a quad each, and each adds its synapses.  A row part that is longer than
+    // an entry is walked on the spot (without a ring all of it is due).  (Nothing is listed: there is nothing left for later.)
+    auto takeWide = [&](uint32_t id, uint32_t p, bool skipInline, bool count) {
+        const ResProj &P = shProj[p];
+        const uint32_t u = lane & (RES_WIDE_QUADS - 1), base = P.lds;
+        const u32x4 x = (asGlobal(P.seg) + RES_WIDE_QUADS * ((size_t)id * tilesInGroup + tileInGroup))[u];
+        const uint32_t n = skipInline ? 0u : x.w >> RES_WIDE_COUNT;
+        const float w[3] = {__uint_as_float(u ? x.x : x.z), __uint_as_float(x.y), __uint_as_float(x.z)};
         #pragma unroll
-        for(uint32_t u = 0; u < RES_WIDE_QUADS; u++) {
-            const u32x4 x = entry[u];
-            e[4 * u] = x.x; e[4 * u + 1] = x.y; e[4 * u + 2] = x.z; e[4 * u + 3] = x.w;
+        for(uint32_t f = 0; f < 3; f++) {
+            if(f < n) { unsafeAtomicAdd(&lds[base + ((x.w >> (RES_ID_BITS * f)) & RES_ID_MASK)], w[f]); }
         }
-        shSeg[slot & 1][pos] = make_uint2(e[0], e[1] | flags);
-        if(e[1] & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
-        if(count) { events += e[1] & 0xFFFFu; }
-        const uint32_t inside = skipInline ? 0u : (e[1] >> 16) & 0xFFu;
+        if(count && u == 0) { events += x.y & 0xFFFFu; }
+        const uint32_t head = __shfl(x.y, 0, RES_WIDE_QUADS), start = __shfl(x.x, 0, RES_WIDE_QUADS);
+        if((head & RES_SEG_OVERFLOW) && !skipInline) {
+            GLOBAL_AS const u32x2 *packed = asGlobal(P.packed) + start;
+            for(uint32_t r = u; r < (head & 0xFFFFu); r += RES_WIDE_QUADS) {
+                const u32x2 rec = packed[r];
+                unsafeAtomicAdd(&lds[base + rec.x / 4u], __uint_as_float(rec.y));
+            }
+        }
+    };
+    // The same by one lane, where eight cannot watch one tile: all quads' loads together, as far as any lane's entry goes.
+    auto takeWideAlone = [&](GLOBAL_AS const u32x4 *entry, const ResProj &P, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
+        u32x4 x[RES_WIDE_QUADS];
         #pragma unroll
-        for(uint32_t f = 0; f < RES_WIDE_MAX; f++) {
-            if((f & 3) == 0 && !__any(f < inside)) { break; }
-            if(f < inside) { unsafeAtomicAdd(&lds[frontBase + ((e[2 + f / 4] >> (8 * (f & 3))) & 0xFFu)], __uint_as_float(e[8 + f])); }
+        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) { x[q] = entry[q]; }
+        const bool flagged = (x[0].y & RES_SEG_OVERFLOW) != 0;
+        shSeg[slot & 1][pos] = make_uint2(flagged ? x[0].x : 0u, flagged ? x[0].y | ((uint32_t)(&P - shProj) << RES_SEG_PROJ_SHIFT) : 0u);
+        if(flagged) { atomicAdd(&shTaken[slot].flagged, 1u); }
+        if(count) { events += x[0].y & 0xFFFFu; }
+        #pragma unroll
+        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) {
+            const uint32_t n = skipInline ? 0u : x[q].w >> RES_WIDE_COUNT;
+            if(!__any(n != 0u)) { break; }
+            const float w[3] = {__uint_as_float(q ? x[q].x : x[q].z), __uint_as_float(x[q].y), __uint_as_float(x[q].z)};
+            #pragma unroll
+            for(uint32_t f = 0; f < 3; f++) {
+                if(f < n) { unsafeAtomicAdd(&lds[P.lds + ((x[q].w >> (RES_ID_BITS * f)) & RES_ID_MASK)], w[f]); }
+            }
         }
     };
     // entry of (neuron, projection), read where a pair is not taken by the thread that saw its word
@@ -433,11 +471,9 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         const ResProj &P = shProj[p];
         const size_t row = (size_t)id * tilesInGroup + tileInGroup;
         const uint32_t frontBase = P.lds + shProjPtr[slot][p];
-        if(WIDE && P.wide) { takeWide(asGlobal(P.seg) + RES_WIDE_QUADS * row, p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count); }
-        else {
-            GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + 2 * row;
-            takeNarrow(entry[0], entry[1], p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count);
-        }
+        if(WIDE && P.wide) { takeWideAlone(asGlobal(P.seg) + RES_WIDE_QUADS * row, P, slot, pos, skipInline, count); return; }
+        GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + 2 * row;
+        takeNarrow(entry[0], entry[1], p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count);
     };
 
     // Waits for every tile's word of exchange `step` (main threads; shTaken says when the bounded wait expired somewhere) and takes the
@@ -467,6 +503,16 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         const uint32_t c = spikesOf();
         if(convention != PASS_NONE && __any(c != 0u)) {
+            if(grouped) {
+                for(uint32_t e = watchSub; e < c && ok; e += perTile) {
+                    uint32_t local[FLIGHT] = {};
+                    if(c <= RES_WORD_IDS) { local[0] = idOf(e); }
+                    else if(!sideIds(e, min(c, e + 1), seqBase + step, parity, local)) { ok = false; }
+                    for(uint32_t j = 0; ok && j < watchNumProj; j++) { takeWide(watchFirst + local[0], shProjIdx[watchProj0 + j], skipInline, count); }
+                }
+                if(!ok) { shTaken[slot].failed = 1u; }
+                return;
+            }
             // this thread's pairs
             const uint32_t mineCount = (c > watchSub && watchNumProj != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u, total = mineCount * watchNumProj;
             if(__any(total != 0u && (c > RES_WORD_IDS || watchNumProj > 1 || mineCount > FLIGHT))) {
@@ -510,14 +556,13 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             }
             else if(total) {
                 // up to FLIGHT spikes of the tile under one projection: their entries are asked for before they have their place in the list
-                const bool narrow = !WIDE || !shProj[watchFlags >> RES_SEG_PROJ_SHIFT].wide;
                 uint32_t local[FLIGHT];
                 u32x4 lo4[FLIGHT], hi4[FLIGHT];
                 #pragma unroll
                 for(uint32_t u = 0; u < FLIGHT; u++) {
                     const uint32_t e = watchSub + u * perTile;
                     local[u] = (e < RES_WORD_IDS) ? idOf(e) : 0u;
-                    if(narrow && u < total) {
+                    if(!watchWide && u < total) {
                         GLOBAL_AS const u32x4 *entry = watchSeg + (size_t)local[u] * narrowStride;
                         lo4[u] = entry[0]; hi4[u] = entry[1];
                     }
@@ -528,8 +573,8 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
                     #pragma unroll
                     for(uint32_t u = 0; u < FLIGHT; u++) {
                         if(u >= total) { break; }
-                        if(narrow) { takeNarrow(lo4[u], hi4[u], watchFlags, frontBase, slot, pos + u, skipInline, count); }
-                        else if(WIDE) { takeWide(watchSeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), watchFlags, frontBase, slot, pos + u, skipInline, count); }
+                        if(!watchWide) { takeNarrow(lo4[u], hi4[u], watchFlags, frontBase, slot, pos + u, skipInline, count); }
+                        else if(WIDE) { takeWideAlone(watchSeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), shProj[watchFlags >> RES_SEG_PROJ_SHIFT], slot, pos + u, skipInline, count); }
                     }
                 }
                 else {
@@ -783,7 +828,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
     }
-    uint32_t offset = (watching && watchSub == 0 && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
+    uint32_t offset = (watching && watchSub == 0 && !(grouped && (lane & (RES_WIDE_QUADS - 1)) != 0) && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
     if(tid == 0) { shScalar[2] = 0; }
     __syncthreads();
     if(offset) { atomicAdd(&shScalar[2], offset); }

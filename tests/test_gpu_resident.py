@@ -359,8 +359,9 @@ def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypat
 
 @pytest.mark.parametrize("n_a, n_b, depth, models, poisson", [
     (256, 1, 0, 1, False), (250, 255, 1, 1, False), (32760, 3, 0, 1, False), (32760, 260, 2, 1, False),            # few tiles, threads share a tile's word
-    (65000, 300, 3, 2, False), (65500, 200, 5, 1, True), (65530, 300, 0, 2, True), (65530, 300, 4, 2, False),      # up to, and one beyond, a tile a thread
-    (130000, 1000, 3, 1, False), (130800, 500, 2, 1, True), (130800, 500, 0, 1, False),                           # two tiles a thread, and more
+    (65000, 300, 3, 2, False), (65500, 200, 5, 1, True), (65530, 300, 0, 2, True), (65530, 300, 4, 2, False),      # up to, and one beyond, 256 tiles of 256
+    (130000, 1000, 3, 1, False), (130800, 500, 2, 1, True), (130800, 500, 0, 1, False),                           # tiles of 512 and 1024
+    (2000, 300, 0, 1, True), (9000, 300, 0, 1, False), (9000, 300, 0, 1, True), (9000, 300, 0, 2, False),          # wide entries: all, or under one projection
     (5000, 700, 0, 3, False), (5000, 700, 6, 3, False), (70000, 700, 3, 3, True), (131000, 600, 0, 3, False)])     # more than two postsynaptic models
 def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
     """Which of the kernel's instances runs depends on how many neurons a tile needs (256, 320, 512 or 1024 for a tile a compute unit), rings,
