@@ -94,11 +94,11 @@ struct gennmi_runner
     ResTile *dResTiles = nullptr; NeuronGroupDev *dResGroups = nullptr; uint8_t *dResTileGroup = nullptr;
     unsigned long long *dResTags = nullptr, *dResSide = nullptr;
     uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0;
-    decltype(&residentKernel<false, false, 2, 256, 0>) resKernel = nullptr;      // the instantiation its sources, segment entries and tiles need
+    decltype(&residentKernel<false, 2, 2, 256, 0>) resKernel = nullptr;      // the instantiation its sources, segment entries and tiles need
     uint32_t resThreads = BLOCK, resTileSize = BLOCK;     // ... its work-group, and neurons of a tile
     std::vector<u32x4*> resSegs;        // segment table of each presynaptic group, in push order
     std::vector<uint32_t> resSegTiles;  // tiles of its target population
-    std::vector<uint32_t> resSegWide;   // its entries are wide ones
+    uint32_t resQuads = 2;              // 16-byte quads of an entry
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
@@ -761,18 +761,9 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     std::vector<uint8_t> tileGroup;
     std::vector<uint32_t> firstTile(r->neuron.size()), numTilesOf(r->neuron.size());
     const char *envTile = getenv("GENNMI_RESIDENT_TILE");
-    uint32_t tileSize = 0, residentThreads = 0;
+    uint32_t tileSize = 0;
     size_t ldsBytes = 0;
-    decltype(r->resKernel) residentInstance = nullptr;
-    bool anyWide = false;
-    // Wide segment entries where a projection without a ring leaves a tile up to RES_WIDE_MEAN synapses of a row (rowStride is a little more than
-    // a row's mean), but more than the four of an ordinary entry would cover; not beyond 256 MiB of them.
-    constexpr uint32_t RES_WIDE_MEAN = 16;
-    auto wideEntries = [&](const gennmi_presynaptic_update_group_t &q, uint32_t tilesInGroup) {
-        const uint64_t mean = ((uint64_t)q.rowStride * tileSize + q.numTrgNeurons - 1) / q.numTrgNeurons;
-        return tileSize == 256 && !anyRing && q.wum == GENNMI_WUM_STATIC_PULSE && mean > 2 && mean <= RES_WIDE_MEAN
-               && (uint64_t)q.numSrcNeurons * tilesInGroup * RES_WIDE_QUADS * sizeof(u32x4) <= (256ull << 20);
-    };
+    bool walkers = false;
     for(const uint32_t size : RES_TILES) {
         if(envTile && (uint32_t)atoi(envTile) != size) { continue; }
         size_t count = 0, ldsFloatsMax = 1;
@@ -785,25 +776,15 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         if(count > size || count > numCU || ldsFloatsMax * sizeof(float) > (size == 256 ? 96u : 128u) * 1024) { continue; }
         tileSize = size;
         ldsBytes = ldsFloatsMax * sizeof(float);
-        for(const auto &p : r->pre) { anyWide = anyWide || wideEntries(p.g, (p.g.numTrgNeurons + size - 1) / size); }
-        // The instantiation for the network's sources, segment entries and postsynaptic models.  Where every projection has a ring that puts its
-        // synapses off for later, wavefronts of their own walk them, as far as a work-group's registers go.
-        constexpr uint32_t WALK = 4, MAX = GENNMI_MAX_PSM;
-        const bool walkers = onlyRings && maxPSM <= 2 && size <= 512;
-        if(maxPSM > 2) { residentInstance = (size == 256) ? residentKernel<true, true, MAX, 256, 0> : (size <= 512) ? residentKernel<true, false, MAX, 512, 0> : residentKernel<true, false, MAX, 1024, 0>; }
-        else if(walkers) {
-            if(size == 256) { residentInstance = poisson ? residentKernel<true, false, 2, 256, WALK> : residentKernel<false, false, 2, 256, WALK>; }
-            else if(size == 320) { residentInstance = poisson ? residentKernel<true, false, 2, 320, WALK> : residentKernel<false, false, 2, 320, WALK>; }
-            else { residentInstance = poisson ? residentKernel<true, false, 2, 512, WALK> : residentKernel<false, false, 2, 512, WALK>; }
-        }
-        else if(size == 256) { residentInstance = poisson ? residentKernel<true, true, 2, 256, 0> : anyWide ? residentKernel<false, true, 2, 256, 0> : residentKernel<false, false, 2, 256, 0>; }
-        else if(size <= 512) { residentInstance = poisson ? residentKernel<true, false, 2, 512, 0> : residentKernel<false, false, 2, 512, 0>; }
-        else { residentInstance = poisson ? residentKernel<true, false, 2, 1024, 0> : residentKernel<false, false, 2, 1024, 0>; }
-        if(!walkers && size == 320) { residentInstance = nullptr; continue; }          // (made for networks with walkers only)
-        residentThreads = size + (walkers ? WALK * WAVE : 0u);
+        // Where every projection has a ring that puts its synapses off for later, wavefronts of their own walk them, as far as a
+        // work-group's registers go.
+        walkers = onlyRings && maxPSM <= 2 && size <= 512;
+        if(!walkers && size == 320) { tileSize = 0; continue; }          // (made for networks with walkers only)
         break;
     }
-    if(!residentInstance) { return GENNMI_OK; }
+    if(!tileSize) { return GENNMI_OK; }
+    constexpr uint32_t WALK = 4;
+    const uint32_t residentThreads = tileSize + (walkers ? WALK * WAVE : 0u);
     for(size_t gi = 0; gi < r->neuron.size(); gi++) {
         const auto &g = r->neuron[gi].g;
         ResTile t{};
@@ -823,14 +804,6 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
             tileGroup.push_back((uint8_t)gi);
         }
     }
-    const void *kernel = reinterpret_cast<const void*>(residentInstance);
-    if(ldsBytes > 32 * 1024) {
-        HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
-    }
-    int perCU = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, (int)residentThreads, ldsBytes));
-    if((size_t)perCU * numCU < tiles.size()) { return GENNMI_OK; }
-
     // projections: source group, target group and postsynaptic model, segment table
     struct Link { size_t src, trg; uint32_t psm; };
     std::vector<Link> links;
@@ -858,18 +831,64 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         for(const auto &l : links) { incoming += (l.trg == gi) ? 1 : 0; }
         if(incoming > RES_MAX_PROJ) { return GENNMI_OK; }
     }
-    uint32_t *dFlag = nullptr;
-    HIP_TRY(poolMalloc(&dFlag, sizeof(uint32_t)));
-    HIP_TRY(hipMemset(dFlag, 0, sizeof(uint32_t)));
-    for(const auto &p : r->pre) {
-        const size_t entries = (size_t)p.g.numSrcNeurons * p.g.rowStride;
-        residentSortedKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(p.g.numSrcNeurons, p.g.rowStride, p.g.rowLength, p.g.ind, dFlag);
+    // are rows sorted by target, and how many of a sample of each projection's synapses are due (words 1 + 2 k: of 2 + 2 k)
+    uint32_t *dSeen = nullptr;
+    std::vector<uint32_t> seen(1 + 2 * r->pre.size(), 0u);
+    HIP_TRY(poolMalloc(&dSeen, seen.size() * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(dSeen, 0, seen.size() * sizeof(uint32_t)));
+    for(size_t k = 0; k < r->pre.size(); k++) {
+        const auto &q = r->pre[k].g;
+        const size_t entries = (size_t)q.numSrcNeurons * q.rowStride;
+        residentSortedKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, dSeen);
+        if(q.maxDenDelay) { residentDueKernel<<<dim3(std::min(64u, q.numSrcNeurons)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.d, q.maxDenDelay, dSeen + 1 + 2 * k); }
     }
     HIP_TRY(hipGetLastError());
-    uint32_t unsorted = 0;
-    HIP_TRY(hipMemcpy(&unsorted, dFlag, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(poolFree(dFlag));
-    if(unsorted) { return GENNMI_OK; }
+    HIP_TRY(hipMemcpy(seen.data(), dSeen, seen.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    HIP_TRY(poolFree(dSeen));
+    if(seen[0]) { return GENNMI_OK; }
+    // Quads of a segment entry, by the largest mean number of synapses of a row part that are due (rowStride is a little more than a row's
+    // mean): an entry should hold what all but one part in thousands has.  Where eight lanes can watch a tile, one of eight costs what
+    // a smaller one does; nowhere more than 4 GiB of them, and not where the parts are too long for any.
+    double due = 0.0;
+    uint64_t entriesInAll = 0;
+    for(size_t k = 0; k < r->pre.size(); k++) {
+        const auto &q = r->pre[k].g;
+        const double share = q.maxDenDelay ? (double)seen[1 + 2 * k] / std::max(1u, seen[2 + 2 * k]) : 1.0;
+        due = std::max(due, share * q.rowStride * tileSize / q.numTrgNeurons);
+        entriesInAll += (uint64_t)q.numSrcNeurons * numTilesOf[links[k].trg];
+    }
+    uint32_t wanted = (due <= 1.0 || due > 16.0) ? 2u : (due <= 5.0 && (anyRing || tiles.size() > tileSize / RES_MAX_QUADS)) ? 4u : 8u;
+    if(const char *envQuads = getenv("GENNMI_RESIDENT_QUADS")) { wanted = (uint32_t)atoi(envQuads); }
+    while(wanted > 2 && entriesInAll * wanted * sizeof(u32x4) > (4ull << 30)) { wanted /= 2; }
+    // the instance for the network's tiles, sources and postsynaptic models whose entries come closest to that
+    struct Instance { uint32_t tile; bool walkers, poisson; uint32_t psm, quads; decltype(r->resKernel) kernel; };
+    constexpr uint32_t MAX = GENNMI_MAX_PSM;
+    static const Instance instances[] = {
+        {256, true, false, 2, 4, residentKernel<false, 4, 2, 256, WALK>}, {256, true, true, 2, 4, residentKernel<true, 4, 2, 256, WALK>},
+        {320, true, false, 2, 4, residentKernel<false, 4, 2, 320, WALK>}, {320, true, true, 2, 4, residentKernel<true, 4, 2, 320, WALK>},
+        {512, true, false, 2, 4, residentKernel<false, 4, 2, 512, WALK>}, {512, true, true, 2, 4, residentKernel<true, 4, 2, 512, WALK>},
+        {256, false, false, 2, 2, residentKernel<false, 2, 2, 256, 0>}, {256, false, false, 2, 4, residentKernel<false, 4, 2, 256, 0>},
+        {256, false, false, 2, 8, residentKernel<false, 8, 2, 256, 0>}, {256, false, true, 2, 4, residentKernel<true, 4, 2, 256, 0>},
+        {512, false, false, 2, 2, residentKernel<false, 2, 2, 512, 0>}, {512, false, false, 2, 4, residentKernel<false, 4, 2, 512, 0>},
+        {512, false, true, 2, 4, residentKernel<true, 4, 2, 512, 0>},
+        {1024, false, false, 2, 2, residentKernel<false, 2, 2, 1024, 0>}, {1024, false, false, 2, 4, residentKernel<false, 4, 2, 1024, 0>},
+        {1024, false, true, 2, 4, residentKernel<true, 4, 2, 1024, 0>},
+        {256, false, true, MAX, 4, residentKernel<true, 4, MAX, 256, 0>}, {512, false, true, MAX, 4, residentKernel<true, 4, MAX, 512, 0>},
+        {1024, false, true, MAX, 2, residentKernel<true, 2, MAX, 1024, 0>}};
+    decltype(r->resKernel) residentInstance = nullptr;
+    uint32_t quads = 0;
+    for(const auto &c : instances) {
+        if(c.tile != tileSize || c.walkers != walkers || c.psm != (maxPSM <= 2 ? 2u : MAX) || (maxPSM <= 2 && c.poisson != poisson)) { continue; }
+        if(!residentInstance || (c.quads <= wanted && c.quads > quads) || (quads > wanted && c.quads < quads)) { residentInstance = c.kernel; quads = c.quads; }
+    }
+    if(!residentInstance) { return GENNMI_OK; }
+    const void *kernel = reinterpret_cast<const void*>(residentInstance);
+    if(ldsBytes > 32 * 1024) {
+        HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
+    }
+    int perCU = 0;
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, (int)residentThreads, ldsBytes));
+    if((size_t)perCU * numCU < tiles.size()) { return GENNMI_OK; }
     for(size_t k = 0; k < r->pre.size(); k++) {
         const auto &q = r->pre[k].g;
         const Link &l = links[k];
@@ -877,14 +896,12 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         const size_t entries = (size_t)q.numSrcNeurons * tilesInGroup;
         if(q.rowStride > 0xFFFFu) { return GENNMI_OK; }         // a segment's length is a 16-bit field (device allocations made so far stay owned)
         u32x4 *dSeg = nullptr;
-        const uint32_t wide = wideEntries(q, tilesInGroup) ? 1u : 0u;
-        HIP_TRY(poolMalloc(&dSeg, entries * (wide ? RES_WIDE_QUADS : 2u) * sizeof(u32x4)));
+        HIP_TRY(poolMalloc(&dSeg, entries * quads * sizeof(u32x4)));
         r->owned.push_back(dSeg);
         const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d,
-                                                                                                     depth, tileSize, tilesInGroup, wide, dSeg);
+                                                                                                     depth, tileSize, tilesInGroup, quads, dSeg);
         r->resSegs.push_back(dSeg);
-        r->resSegWide.push_back(wide);
         r->resSegTiles.push_back(tilesInGroup);
         HIP_TRY(hipGetLastError());
         const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
@@ -900,7 +917,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         }
         r->resPacked.push_back(dPacked);
         ResProj proj{};
-        proj.packed = dPacked; proj.seg = dSeg; proj.wide = wide;
+        proj.packed = dPacked; proj.seg = dSeg;
         proj.D = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         proj.srcGroup = (uint32_t)l.src;
         for(uint32_t t = firstTile[l.trg]; t < firstTile[l.trg] + tilesInGroup; t++) {
@@ -931,7 +948,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     r->resTiles = (uint32_t)tiles.size();
     r->resLdsBytes = ldsBytes;
     r->resKernel = residentInstance;
-    r->resThreads = residentThreads; r->resTileSize = tileSize;
+    r->resThreads = residentThreads; r->resTileSize = tileSize; r->resQuads = quads;
     r->resident = true;
     return GENNMI_OK;
 }
@@ -957,7 +974,7 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
             const size_t entries = (size_t)q.numSrcNeurons * r->resSegTiles[k];
             const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
             residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(
-                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resTileSize, r->resSegTiles[k], r->resSegWide[k], r->resSegs[k]);
+                q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d, depth, r->resTileSize, r->resSegTiles[k], r->resQuads, r->resSegs[k]);
             const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
             if(padded) {
                 residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, r->stream>>>(padded, q.ind, q.g, q.d, depth, r->resTileSize, r->resPacked[k]);

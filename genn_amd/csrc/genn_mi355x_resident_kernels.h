@@ -33,13 +33,15 @@ constexpr uint32_t RES_MAX_TILE = 1024;
 constexpr uint32_t RES_MAX_PROJ = 16;        // projections into one population
 constexpr uint32_t RES_MAX_GROUPS = 64;      // neuron groups
 constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs a tile lists per exchange
-constexpr uint32_t RES_FRONT_MAX = 4;        // front-slot synapses held inline in a segment entry
-// Without a ring every synapse of a row part is due at once.  Where the parts are short they go into the entry whole: up to four into 32
-// bytes, up to 22 into a wide entry of 128 — one cache line, read where 32 bytes of it were — and the step is spared the second trip to
-// memory, to the records, and a barrier.  us a step of a balanced network: 100,000 neurons x 80 targets 8.1 -> 6.7, 40,000 x 80 4.7 -> 4.3
-// (ordinary entries); 12,000 x 100 4.19 -> 4.00, 4,000 x 80 3.79 -> 3.62 (wide ones; 4.19 and 3.70 without), and 2.85 -> 2.47 since
-// eight lanes read a wide entry, a quad each, instead of one lane all of it.
-constexpr uint32_t RES_WIDE_QUADS = 8, RES_WIDE_MAX = 22, RES_WIDE_COUNT = 30;       // (shift of a quad's number of synapses)
+// A segment entry says where a row's part inside a tile is and holds its due synapses, those that land in the slot the target reads in the
+// very step that delivers them (without a ring all of the part): a step waits for nothing else, and the dependent trip to the records is
+// spared.  Entries of a network are of 2, 4 or 8 quads of 16 bytes, which hold 4, 10 or 22 of them; a part with more is walked before the update,
+// and every tile waits for the one that does.  us a step of a balanced network, without / with synapses inside entries: 100,000 neurons x
+// 80 targets 8.1 / 6.7, 40,000 x 80 4.7 / 4.3 (2 quads), 12,000 x 100 4.19 / 4.00, 4,000 x 80 3.79 / 3.62 (8, which one lane read then), and 2.85 -> 2.47
+// since eight lanes read an entry of 8, a quad each; with 2 / with what the host's rule takes now: 4,000 x 80 2.66 / 2.24 (8), 20,000 x 100
+// 3.13 / 2.43 and 40,000 x 80 3.52 / 3.26 (4); the microcircuit's rings have few that are due, 4.22 with 2 and with 4.
+constexpr uint32_t residentInside(uint32_t quads) { return 3 * quads - 2; }
+constexpr uint32_t RES_MAX_QUADS = 8, RES_COUNT_SHIFT = 30;       // a quad's last word: targets, 10 bits each, and the number of its synapses
 constexpr uint32_t RES_SEG_OVERFLOW = 1u << 24, RES_SEG_NO_DELAY = 1u << 25;
 constexpr uint32_t RES_SEG_PROJ_SHIFT = 26;  // in the kernel's list of pairs: the projection, above an entry's flags
 // word: upper half sequence number << 11 | count, lower half up to three tile-local neuron indices, 10 bits each
@@ -56,8 +58,7 @@ struct ResProj
     uint32_t D;                         // ring depth; 0 = no dendritic delay, events add to inSyn
     uint32_t lds;                       // float offset of the ring (D x tile size, slot-major) or inSyn row in the tile's LDS
     uint32_t srcGroup;
-    uint32_t wide;                      // != 0: entries of RES_WIDE_QUADS x 16 bytes instead of two
-    uint32_t pad_[2];
+    uint32_t pad_[3];
 };
 
 struct ResTile
@@ -70,16 +71,12 @@ struct ResTile
     ResProj proj[RES_MAX_PROJ];
 };
 
-// One 32-byte entry per (row, tile of the target population): word 0 = first idSyn of the row's part inside the tile,
-// word 1 = its length | number of inline synapses << 16 | flags, words 2-5 = weights and words 6 and 7 = the tile-local
-// targets (byte offsets, 16 bits each) of up to four synapses whose delay is a multiple of the ring depth.  Those land in the slot the target reads in
-// the very step that delivers them, so they are the only ones a step has to wait for; carrying them inside the entry
-// saves that step the dependent read of the row.  RES_SEG_OVERFLOW: the segment has more of them than fit (the row part
-// is then read at once); RES_SEG_NO_DELAY: the projection has no ring, every synapse is due at once.  A wide entry is eight quads that
-// lanes read one each: the first has words 0 and 1, a weight and what the last word of every quad is, the targets (10 bits each)
-// and the number of the quad's synapses; the others have three weights and such a word.
+// One entry per (row, tile of the target population).  Its first quad: first idSyn of the row's part inside the tile; its length | number of
+// synapses inside << 16 | flags; a weight; targets and count as in every quad's last word.  The others: three weights, targets and count.
+// RES_SEG_OVERFLOW: the part has more due synapses than fit (none is inside, the row part is walked before the update);
+// RES_SEG_NO_DELAY: the projection has no ring, every synapse is due at once.
 __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLength, const uint32_t *ind, const float *weight,
-                                  const uint8_t *delay, uint32_t depth, uint32_t tileSize, uint32_t tilesInGroup, uint32_t wide, u32x4 *seg)
+                                  const uint8_t *delay, uint32_t depth, uint32_t tileSize, uint32_t tilesInGroup, uint32_t quads, u32x4 *seg)
 {
     const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if(id >= (size_t)numSrc * tilesInGroup) { return; }
@@ -93,40 +90,36 @@ __global__ void residentSegKernel(uint32_t numSrc, uint32_t rowStride, const uin
     };
     const uint32_t a = lowerBound(tile * tileSize), b = lowerBound((tile + 1) * tileSize);
     const uint32_t start = row * rowStride + a;
-    uint32_t flags = depth ? 0u : RES_SEG_NO_DELAY, numFront = 0;
-    if(wide) {
-        const uint32_t inside = (b - a <= RES_WIDE_MAX) ? b - a : 0u;
-        if(b - a > RES_WIDE_MAX) { flags |= RES_SEG_OVERFLOW; }
-        uint32_t j = 0;
-        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) {
-            uint32_t x[4] = {0u, 0u, 0u, 0u};
-            if(q == 0) { x[0] = start; x[1] = min(b - a, 0xFFFFu) | (inside << 16) | flags; }
-            uint32_t n = 0;
-            for(uint32_t f = q ? 0u : 2u; f < 3 && j < inside; f++, j++, n++) {
-                x[f] = __float_as_uint(weight[(size_t)row * rowStride + a + j]);
-                x[3] |= (r[a + j] - tile * tileSize) << (RES_ID_BITS * n);
-            }
-            x[3] |= n << RES_WIDE_COUNT;
-            seg[RES_WIDE_QUADS * id + q] = u32x4{x[0], x[1], x[2], x[3]};
+    uint32_t flags = depth ? 0u : RES_SEG_NO_DELAY;
+    auto due = [&](uint32_t j) { return !depth || delay[(size_t)row * rowStride + j] % depth == 0; };
+    uint32_t inside = 0;
+    for(uint32_t j = a; j < b && inside <= residentInside(quads); j++) { inside += due(j) ? 1u : 0u; }
+    if(inside > residentInside(quads)) { flags |= RES_SEG_OVERFLOW; inside = 0; }
+    uint32_t j = a, done = 0;
+    for(uint32_t q = 0; q < quads; q++) {
+        uint32_t x0 = 0, x1 = 0, x2 = 0, last = 0, n = 0;
+        if(q == 0) { x0 = start; x1 = min(b - a, 0xFFFFu) | (inside << 16) | flags; }
+        for(uint32_t f = q ? 0u : 2u; f < 3 && done < inside; f++, j++, n++, done++) {
+            while(!due(j)) { j++; }
+            const uint32_t w = __float_as_uint(weight[(size_t)row * rowStride + j]);
+            if(f == 0) { x0 = w; } else if(f == 1) { x1 = w; } else { x2 = w; }
+            last |= (r[j] - tile * tileSize) << (RES_ID_BITS * n);
         }
-        return;
+        seg[quads * id + q] = u32x4{x0, x1, x2, last | (n << RES_COUNT_SHIFT)};
     }
-    uint32_t w[RES_FRONT_MAX] = {0, 0, 0, 0}, at[2] = {0, 0};
-    if(!depth && b - a > RES_FRONT_MAX) { flags |= RES_SEG_OVERFLOW; }
-    else {
-        for(uint32_t j = a; j < b; j++) {
-            if(depth && delay[(size_t)row * rowStride + j] % depth != 0) { continue; }
-            if(numFront == RES_FRONT_MAX) { flags |= RES_SEG_OVERFLOW; numFront = 0; break; }    // the row walk adds all of them
-            w[numFront] = __float_as_uint(weight[(size_t)row * rowStride + j]);
-            at[numFront / 2] |= 4u * (r[j] - tile * tileSize) << (16 * (numFront & 1));
-            numFront++;
-        }
-    }
-    u32x4 lo4, hi4;
-    lo4.x = start; lo4.y = min(b - a, 0xFFFFu) | (numFront << 16) | flags; lo4.z = w[0]; lo4.w = w[1];
-    hi4.x = w[2]; hi4.y = w[3]; hi4.z = at[0]; hi4.w = at[1];
-    seg[2 * id] = lo4;
-    seg[2 * id + 1] = hi4;
+}
+
+// How many of a sample of a projection's synapses are due: counts[0] of counts[1] (64 rows across the source population, a work-group each)
+__global__ __launch_bounds__(BLOCK)
+void residentDueKernel(uint32_t numSrc, uint32_t rowStride, const uint32_t *rowLength, const uint8_t *delay, uint32_t depth, uint32_t *counts)
+{
+    const size_t row = (size_t)blockIdx.x * numSrc / gridDim.x;
+    const uint32_t len = rowLength[row];
+    uint32_t due = 0;
+    for(uint32_t j = threadIdx.x; j < len; j += BLOCK) { due += (delay[row * rowStride + j] % depth == 0) ? 1u : 0u; }
+    for(int off = WAVE / 2; off > 0; off >>= 1) { due += __shfl_down(due, off, WAVE); }
+    if((threadIdx.x & (WAVE - 1)) == 0 && due) { atomicAdd(&counts[0], due); }
+    if(threadIdx.x == 0) { atomicAdd(&counts[1], len); }
 }
 
 // The synapses as the row walk reads them: where in the tile's ring they land, in bytes from its front slot (slots of a float a
@@ -181,12 +174,12 @@ __device__ __forceinline__ void ldsBarrier()
 // What consecutive exchanges share exists once for each of them: pair lists twice, counters and ring fronts four times (those of the
 // exchange after the next are prepared behind the barrier, so no thread meets them half prepared).
 // POISSON: some population has a PoissonExp current source (its state then lives in a register per source and neuron);
-// the instantiation without it carries neither the registers nor the generator.  WIDE: some projection may have wide entries.
+// the instantiation without it carries neither the registers nor the generator.  QUADS: of a segment entry.
 // NPSM: postsynaptic models of any group.  TILE: neurons of a tile, and threads that own one.  WALK: wavefronts beyond those that
 // own the tile's neurons; 0: these walk too, once they have published.  With walkers nothing holds a wavefront back between its
 // update and the next exchange, so every projection must have a ring of two slots or more: what an early wavefront adds then goes to another slot
 // than the one a late one is reading and clearing.  Without, a barrier behind the update keeps them apart, and inSyn itself can be added to.
-template<bool POISSON, bool WIDE, uint32_t NPSM, uint32_t TILE, uint32_t WALK>
+template<bool POISSON, uint32_t QUADS, uint32_t NPSM, uint32_t TILE, uint32_t WALK>
 __global__ __launch_bounds__(TILE + WALK * WAVE, (TILE + WALK * WAVE + 4 * WAVE - 1) / (4 * WAVE))
 void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const NeuronGroupDev * __restrict__ groups,
                     const uint8_t * __restrict__ tileGroup, unsigned long long *tags, unsigned long long *side,
@@ -196,8 +189,8 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
 {
     extern __shared__ float lds[];                       // inSyn rows and ring slices of this tile
     __shared__ uint2 shSeg[2][RES_PAIR_CAP];             // (first idSyn, length | flags | projection) of each listed pair
-    // of an exchange: pairs claimed; listed pairs whose row has to be walked before the update; pairs were left over; a wait expired
-    struct Taken { uint32_t pairs, flagged, left, failed; };
+    // of an exchange: listed pairs whose row has to be walked before the update; pairs were left over; a wait expired
+    struct Taken { uint32_t flagged, left, failed, pad; };
     __shared__ __align__(16) Taken shTaken[4];
     __shared__ uint32_t shDone[4];                       // of the update an exchange feeds: wavefronts done << 16 | spikes
     __shared__ ResProj shProj[RES_MAX_PROJ];
@@ -207,6 +200,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     __shared__ uint32_t shOwn[TILE];                    // this tile's spikes of the last step, in no particular order
     constexpr uint32_t THREADS = TILE + WALK * WAVE, WAVES = THREADS / WAVE, MAIN = TILE / WAVE;
     __shared__ uint32_t shWave[WAVES];
+    __shared__ uint32_t shListed[4][MAIN];               // pairs each wavefront has listed of an exchange, in its own part of the list
     __shared__ uint32_t shScalar[4];
 
     // every tile publishes its word into all copies of the word array and reads the copy of its own XCD
@@ -352,12 +346,12 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // The source tile this thread watches and the spikes it takes of it: all of them, or, where there are fewer tiles than half the threads,
     // those that fall to it among the threads that watch the same one.
     uint32_t perTile = 1, perShift = 0, watchTile = tid, watchSub = 0;
-    // (wide entries are read by eight lanes each: with few enough tiles the eight watch the same one, `grouped`)
-    bool grouped = WIDE && numProj != 0 && numTiles <= TILE / RES_WIDE_QUADS;
-    for(uint32_t q = 0; grouped && q < numProj; q++) { grouped = shProj[q].wide != 0; }
+    // (entries of eight quads are read by eight lanes each: with few enough tiles the eight watch the same one, `grouped`)
+    bool grouped = QUADS == RES_MAX_QUADS && numTiles <= TILE / RES_MAX_QUADS;
+    for(uint32_t q = 0; grouped && q < numProj; q++) { grouped = shProj[q].D == 0; }
     if(grouped) {
-        const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u), group = tid / RES_WIDE_QUADS;
-        perTile = (TILE / RES_WIDE_QUADS) >> shift;
+        const uint32_t shift = 32u - (uint32_t)__clz(max(numTiles, 2u) - 1u), group = tid / RES_MAX_QUADS;
+        perTile = (TILE / RES_MAX_QUADS) >> shift;
         watchTile = group & ((1u << shift) - 1u); watchSub = group >> shift;
     }
     else if((TILE & (TILE - 1)) == 0 && numTiles <= TILE / 2) {
@@ -366,10 +360,13 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         watchTile = tid & ((1u << shift) - 1u); watchSub = tid >> shift;
     }
     const bool watching = main && watchTile < numTiles;
-    const uint32_t narrowStride = 2u * tilesInGroup;     // entries of consecutive rows, in quads
+    // The list is shared out between the wavefronts that watch: a pair's place depends on the spikes alone and not on when their words
+    // arrive, and so does the order in which the walk adds the synapses of an exchange (out of the order of arrival, two runs of the full
+    // microcircuit parted at every neuron that comes within a rounding of its threshold).
+    const uint32_t watchWaves = (perTile == 1) ? (numTiles + WAVE - 1) / WAVE : MAIN, listCap = RES_PAIR_CAP / watchWaves;
+    const uint32_t rowQuads = QUADS * tilesInGroup;     // entries of consecutive rows, in quads
     const uint32_t watchFirst = watching ? tiles[watchTile].first : 0u;
     uint32_t watchProj0 = 0, watchNumProj = 0, watchLds = 0, watchFlags = 0;             // (flags: the first projection's number << 26)
-    bool watchWide = false;
     GLOBAL_AS const u32x4 *watchSeg = nullptr;           // entry of the tile's first neuron under its group's first projection into this tile
     if(watching) {
         const uint32_t s = tileGroup[watchTile];
@@ -377,15 +374,14 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         watchNumProj = shProjStart[s + 1] - watchProj0;
         if(watchNumProj) {
             const uint32_t p = shProjIdx[watchProj0];
-            watchWide = WIDE && shProj[p].wide;
-            watchSeg = asGlobal(shProj[p].seg) + (watchWide ? RES_WIDE_QUADS : 2u) * ((size_t)watchFirst * tilesInGroup + tileInGroup);
+            watchSeg = asGlobal(shProj[p].seg) + QUADS * ((size_t)watchFirst * tilesInGroup + tileInGroup);
             watchFlags = p << RES_SEG_PROJ_SHIFT;
             watchLds = shProj[p].lds;
         }
     }
 
-    // spikes of a word whose entries a thread has in flight at a time
-    constexpr uint32_t FLIGHT = (THREADS <= 512) ? 3 : 1;
+    // entries of a side list that are asked for at a time
+    constexpr uint32_t FLIGHT = 3;
     // Entries e0, e0 + perTile, ... (FLIGHT of them, below c) of the watched tile's side list of the exchange `full`: waits, bounded, until each says so
     auto sideIds = [&](uint32_t e0, uint32_t c, unsigned long long full, uint32_t parity, uint32_t (&local)[FLIGHT]) -> bool {
         const unsigned long long *base = side + ((size_t)parity * numTiles + watchTile) * TILE + e0;
@@ -411,69 +407,52 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
 
     constexpr uint32_t PASS_ALL = 0, PASS_LATER = 1, PASS_DUE = 2, PASS_NONE = 3;      // which synapses a pass adds: see process()
 
-    // What one ordinary segment entry says: lists the pair and — unless `skipInline` — adds the entry's inline synapses to the front slot
-    auto takeNarrow = [&](u32x4 lo4, u32x4 hi4, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
-        shSeg[slot & 1][pos] = make_uint2(lo4.x, lo4.y | flags);
-        if(lo4.y & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
-        if(count) { events += lo4.y & 0xFFFFu; }
-        const uint32_t numFront = skipInline ? 0u : (lo4.y >> 16) & 0xFFu;
-        if(!__any(numFront != 0u)) { return; }
-        const uint32_t w[RES_FRONT_MAX] = {lo4.z, lo4.w, hi4.x, hi4.y};
+    struct Entry { u32x4 quad[QUADS]; };
+    auto readEntry = [&](GLOBAL_AS const u32x4 *entry) -> Entry {
+        Entry e;
         #pragma unroll
-        for(uint32_t f = 0; f < RES_FRONT_MAX; f++) {
-            if(f < numFront) { unsafeAtomicAdd(reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + (4u * frontBase + (((f & 2) ? hi4.w : hi4.z) >> (16 * (f & 1)) & 0xFFFFu))), __uint_as_float(w[f])); }
+        for(uint32_t q = 0; q < QUADS; q++) { e.quad[q] = entry[q]; }
+        return e;
+    };
+    // What a segment entry says: lists the pair and — unless `skipInline` — adds the synapses inside to the front slot
+    auto takeEntry = [&](const Entry &e, uint32_t flags, uint32_t frontBase, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
+        const uint32_t head = e.quad[0].y;
+        shSeg[slot & 1][pos] = make_uint2(e.quad[0].x, head | flags);
+        if(head & RES_SEG_OVERFLOW) { atomicAdd(&shTaken[slot].flagged, 1u); }
+        if(count) { events += head & 0xFFFFu; }
+        const uint32_t inside = skipInline ? 0u : (head >> 16) & 0xFFu;
+        #pragma unroll
+        for(uint32_t q = 0; q < QUADS; q++) {
+            if(!__any((q ? 3 * q - 2 : 0u) < inside)) { break; }
+            const u32x4 x = e.quad[q];
+            const float w[3] = {__uint_as_float(q ? x.x : x.z), __uint_as_float(x.y), __uint_as_float(x.z)};
+            #pragma unroll
+            for(uint32_t f = 0; f < (q ? 3u : 1u); f++) {
+                if((q ? 3 * q - 2 : 0u) + f < inside) { unsafeAtomicAdd(&lds[frontBase + ((x.w >> (RES_ID_BITS * f)) & RES_ID_MASK)], w[f]); }
+            }
         }
     };
-    // A wide entry, by eight consecutive lanes with the same arguments: a quad each, and each adds its synapses.  A row part that is longer than
-    // an entry is walked on the spot (without a ring all of it is due).  (Nothing is listed: there is nothing left for later.)
-    auto takeWide = [&](uint32_t id, uint32_t p, bool skipInline, bool count) {
+    // An entry of eight quads, by eight consecutive lanes with the same arguments: a quad each, and each adds its synapses.  A row part that is longer
+    // than an entry is walked on the spot (without a ring all of it is due).  (Nothing is listed: there is nothing left for later.)
+    auto takeTogether = [&](uint32_t id, uint32_t p, bool skipInline, bool count) {
         const ResProj &P = shProj[p];
-        const uint32_t u = lane & (RES_WIDE_QUADS - 1), base = P.lds;
-        const u32x4 x = (asGlobal(P.seg) + RES_WIDE_QUADS * ((size_t)id * tilesInGroup + tileInGroup))[u];
-        const uint32_t n = skipInline ? 0u : x.w >> RES_WIDE_COUNT;
+        const uint32_t u = lane & (RES_MAX_QUADS - 1), base = P.lds;
+        const u32x4 x = (asGlobal(P.seg) + RES_MAX_QUADS * ((size_t)id * tilesInGroup + tileInGroup))[u];
+        const uint32_t n = skipInline ? 0u : x.w >> RES_COUNT_SHIFT;
         const float w[3] = {__uint_as_float(u ? x.x : x.z), __uint_as_float(x.y), __uint_as_float(x.z)};
         #pragma unroll
         for(uint32_t f = 0; f < 3; f++) {
             if(f < n) { unsafeAtomicAdd(&lds[base + ((x.w >> (RES_ID_BITS * f)) & RES_ID_MASK)], w[f]); }
         }
         if(count && u == 0) { events += x.y & 0xFFFFu; }
-        const uint32_t head = __shfl(x.y, 0, RES_WIDE_QUADS), start = __shfl(x.x, 0, RES_WIDE_QUADS);
+        const uint32_t head = __shfl(x.y, 0, RES_MAX_QUADS), start = __shfl(x.x, 0, RES_MAX_QUADS);
         if((head & RES_SEG_OVERFLOW) && !skipInline) {
             GLOBAL_AS const u32x2 *packed = asGlobal(P.packed) + start;
-            for(uint32_t r = u; r < (head & 0xFFFFu); r += RES_WIDE_QUADS) {
+            for(uint32_t r = u; r < (head & 0xFFFFu); r += RES_MAX_QUADS) {
                 const u32x2 rec = packed[r];
                 unsafeAtomicAdd(&lds[base + rec.x / 4u], __uint_as_float(rec.y));
             }
         }
-    };
-    // The same by one lane, where eight cannot watch one tile: all quads' loads together, as far as any lane's entry goes.
-    auto takeWideAlone = [&](GLOBAL_AS const u32x4 *entry, const ResProj &P, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
-        u32x4 x[RES_WIDE_QUADS];
-        #pragma unroll
-        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) { x[q] = entry[q]; }
-        const bool flagged = (x[0].y & RES_SEG_OVERFLOW) != 0;
-        shSeg[slot & 1][pos] = make_uint2(flagged ? x[0].x : 0u, flagged ? x[0].y | ((uint32_t)(&P - shProj) << RES_SEG_PROJ_SHIFT) : 0u);
-        if(flagged) { atomicAdd(&shTaken[slot].flagged, 1u); }
-        if(count) { events += x[0].y & 0xFFFFu; }
-        #pragma unroll
-        for(uint32_t q = 0; q < RES_WIDE_QUADS; q++) {
-            const uint32_t n = skipInline ? 0u : x[q].w >> RES_WIDE_COUNT;
-            if(!__any(n != 0u)) { break; }
-            const float w[3] = {__uint_as_float(q ? x[q].x : x[q].z), __uint_as_float(x[q].y), __uint_as_float(x[q].z)};
-            #pragma unroll
-            for(uint32_t f = 0; f < 3; f++) {
-                if(f < n) { unsafeAtomicAdd(&lds[P.lds + ((x[q].w >> (RES_ID_BITS * f)) & RES_ID_MASK)], w[f]); }
-            }
-        }
-    };
-    // entry of (neuron, projection), read where a pair is not taken by the thread that saw its word
-    auto takeEntry = [&](uint32_t id, uint32_t p, uint32_t slot, uint32_t pos, bool skipInline, bool count) {
-        const ResProj &P = shProj[p];
-        const size_t row = (size_t)id * tilesInGroup + tileInGroup;
-        const uint32_t frontBase = P.lds + shProjPtr[slot][p];
-        if(WIDE && P.wide) { takeWideAlone(asGlobal(P.seg) + RES_WIDE_QUADS * row, P, slot, pos, skipInline, count); return; }
-        GLOBAL_AS const u32x4 *entry = asGlobal(P.seg) + 2 * row;
-        takeNarrow(entry[0], entry[1], p << RES_SEG_PROJ_SHIFT, frontBase, slot, pos, skipInline, count);
     };
 
     // Waits for every tile's word of exchange `step` (main threads; shTaken says when the bounded wait expired somewhere) and takes the
@@ -483,6 +462,13 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     bool left = false;
     auto spikesOf = [&]() -> uint32_t { return (uint32_t)(word >> 32) & RES_COUNT_MASK; };
     auto idOf = [&](uint32_t e) -> uint32_t { return ((uint32_t)word >> (RES_ID_BITS * e)) & RES_ID_MASK; };        // (e < RES_WORD_IDS)
+    // Cycles from a tile's own word to its first look for the others'.  A look that comes too early costs its whole trip to memory again, and
+    // the looks of all the waiting tiles slow the words down.  us a step without / with the wait (of 1,000 cycles, from 129 tiles on of 1,300: 1,000 and
+    // 1,500 gave 3.29 and 3.24 at 40,000 x 80, 4.30 and 4.04 at 100,000 x 80, 2.37 and 2.42 at 20,000 x 100): 20,000 x 100 2.76 / 2.43,
+    // 40,000 x 80 3.79 / 3.26, 100,000 x 80 4.83 / 4.15, 250,000 x 200 6.2 / 4.3, the full microcircuit 4.66 / 4.12.  A handful of tiles are too quick for it (1,000 x 80 2.10 / 2.17).
+    // Drawing of Poisson sources takes longer than the wait.
+    const uint32_t firstLook = (numTiles <= 8) ? 0u : (numTiles <= 128) ? 1000u : 1300u;
+    uint32_t published = (uint32_t)__builtin_readcyclecounter();
     auto poll = [&](uint32_t step, uint32_t convention) {
         const uint32_t seq = (uint32_t)(seqBase + step) & RES_SEQ_MASK;
         const uint32_t parity = seq & 1u, slot = seq & 3u;
@@ -493,6 +479,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         if(watching) {
             const unsigned long long *mine_ = myTags + (parity ? numTiles : 0u) + watchTile;
             uint32_t spins = 0;
+            while((uint32_t)__builtin_readcyclecounter() - published < firstLook) { __builtin_amdgcn_s_sleep(1); }
             while(true) {
                 word = __hip_atomic_load(mine_, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if((uint32_t)(word >> (32 + RES_COUNT_BITS)) == seq) { break; }
@@ -502,88 +489,69 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             }
         }
         const uint32_t c = spikesOf();
+        uint32_t listed = 0;
         if(convention != PASS_NONE && __any(c != 0u)) {
             if(grouped) {
                 for(uint32_t e = watchSub; e < c && ok; e += perTile) {
                     uint32_t local[FLIGHT] = {};
                     if(c <= RES_WORD_IDS) { local[0] = idOf(e); }
                     else if(!sideIds(e, min(c, e + 1), seqBase + step, parity, local)) { ok = false; }
-                    for(uint32_t j = 0; ok && j < watchNumProj; j++) { takeWide(watchFirst + local[0], shProjIdx[watchProj0 + j], skipInline, count); }
-                }
-                if(!ok) { shTaken[slot].failed = 1u; }
-                return;
-            }
-            // this thread's pairs
-            const uint32_t mineCount = (c > watchSub && watchNumProj != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u, total = mineCount * watchNumProj;
-            if(__any(total != 0u && (c > RES_WORD_IDS || watchNumProj > 1 || mineCount > FLIGHT))) {
-                // Some thread of the wavefront has many pairs: the wavefront lists its pairs first and every
-                // lane then takes as many of them as every other, so that their entries are one trip to memory and not one after another.
-                const uint32_t inclusive = waveInclusiveScanU32(total, lane);
-                const uint32_t waveTotal = (uint32_t)__builtin_amdgcn_readlane((int)inclusive, WAVE - 1);
-                uint32_t base = 0;
-                if(lane == 0) { base = atomicAdd(&shTaken[slot].pairs, waveTotal); }
-                base = __builtin_amdgcn_readfirstlane(base);
-                const bool fits = (base + waveTotal <= RES_PAIR_CAP);
-                uint32_t pos = base + inclusive - total;
-                left = !fits && total != 0;
-                for(uint32_t e0 = watchSub; total != 0 && e0 < c && ok; e0 += FLIGHT * perTile) {
-                    uint32_t local[FLIGHT];
-                    #pragma unroll
-                    for(uint32_t u = 0; u < FLIGHT; u++) { local[u] = (e0 + u * perTile < RES_WORD_IDS) ? idOf(e0 + u * perTile) : 0u; }
-                    // (also when the pairs do not fit and leftOver() will read the list again: once seen here, an entry is there
-                    // for every later read of this thread)
-                    if(c > RES_WORD_IDS && !sideIds(e0, c, seqBase + step, parity, local)) { ok = false; }
-                    #pragma unroll
-                    for(uint32_t u = 0; u < FLIGHT; u++) {
-                        if(!fits || e0 + u * perTile >= c) { break; }
-                        for(uint32_t j = 0; j < watchNumProj; j++) { shSeg[slot & 1][pos++] = make_uint2(watchFirst + local[u], shProjIdx[watchProj0 + j]); }
-                    }
-                }
-                if(!fits) {
-                    // (a claim across the list's end: the places it does not use say "no synapses")
-                    for(uint32_t r = base + lane; r < RES_PAIR_CAP; r += WAVE) { shSeg[slot & 1][r] = make_uint2(0u, 0u); }
-                    if(lane == 0) { shTaken[slot].left = 1u; }
-                }
-                else if(!__any(!ok)) {
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-                    for(uint32_t x = base + lane; x < base + waveTotal; x += WAVE) {
-                        const uint2 pr = shSeg[slot & 1][x];
-                        takeEntry(pr.x, pr.y, slot, x, skipInline, count);
-                    }
+                    for(uint32_t j = 0; ok && j < watchNumProj; j++) { takeTogether(watchFirst + local[0], shProjIdx[watchProj0 + j], skipInline, count); }
                 }
             }
-            else if(total) {
-                // up to FLIGHT spikes of the tile under one projection: their entries are asked for before they have their place in the list
-                uint32_t local[FLIGHT];
-                u32x4 lo4[FLIGHT], hi4[FLIGHT];
-                #pragma unroll
-                for(uint32_t u = 0; u < FLIGHT; u++) {
-                    const uint32_t e = watchSub + u * perTile;
-                    local[u] = (e < RES_WORD_IDS) ? idOf(e) : 0u;
-                    if(!watchWide && u < total) {
-                        GLOBAL_AS const u32x4 *entry = watchSeg + (size_t)local[u] * narrowStride;
-                        lo4[u] = entry[0]; hi4[u] = entry[1];
+            else {
+                // this thread's pairs
+                const uint32_t mineCount = (c > watchSub && watchNumProj != 0) ? ((c - watchSub + perTile - 1) >> perShift) : 0u, total = mineCount * watchNumProj;
+                const uint32_t listBase = wave * listCap;
+                const unsigned long long busy = __ballot(total != 0u);
+                listed = __popcll(busy);
+                if(__any(total > 1u || (total != 0u && c > RES_WORD_IDS))) {         // (beyond RES_WORD_IDS the ids are in the side list)
+                    // Some thread of the wavefront has many pairs: the wavefront lists its pairs first and every
+                    // lane then takes as many of them as every other, so that their entries are one trip to memory and not one after another.
+                    const uint32_t inclusive = waveInclusiveScanU32(total, lane);
+                    listed = (uint32_t)__builtin_amdgcn_readlane((int)inclusive, WAVE - 1);
+                    const bool fits = (listed <= listCap);
+                    uint32_t pos = listBase + inclusive - total;
+                    left = !fits && total != 0;
+                    for(uint32_t e0 = watchSub; total != 0 && e0 < c && ok; e0 += FLIGHT * perTile) {
+                        uint32_t local[FLIGHT];
+                        #pragma unroll
+                        for(uint32_t u = 0; u < FLIGHT; u++) { local[u] = (e0 + u * perTile < RES_WORD_IDS) ? idOf(e0 + u * perTile) : 0u; }
+                        // (also when the pairs do not fit and leftOver() will read the list again: once seen here, an entry is there
+                        // for every later read of this thread)
+                        if(c > RES_WORD_IDS && !sideIds(e0, c, seqBase + step, parity, local)) { ok = false; }
+                        #pragma unroll
+                        for(uint32_t u = 0; u < FLIGHT; u++) {
+                            if(!fits || e0 + u * perTile >= c) { break; }
+                            for(uint32_t j = 0; j < watchNumProj; j++) { shSeg[slot & 1][pos++] = make_uint2(watchFirst + local[u], shProjIdx[watchProj0 + j]); }
+                        }
                     }
-                }
-                const uint32_t pos = atomicAdd(&shTaken[slot].pairs, total);
-                if(pos + total <= RES_PAIR_CAP) {
-                    const uint32_t frontBase = watchLds + shProjPtr[slot][watchFlags >> RES_SEG_PROJ_SHIFT];
-                    #pragma unroll
-                    for(uint32_t u = 0; u < FLIGHT; u++) {
-                        if(u >= total) { break; }
-                        if(!watchWide) { takeNarrow(lo4[u], hi4[u], watchFlags, frontBase, slot, pos + u, skipInline, count); }
-                        else if(WIDE) { takeWideAlone(watchSeg + (size_t)local[u] * (RES_WIDE_QUADS * tilesInGroup), shProj[watchFlags >> RES_SEG_PROJ_SHIFT], slot, pos + u, skipInline, count); }
+                    if(!fits) {
+                        listed = 0;
+                        if(lane == 0) { shTaken[slot].left = 1u; }
+                    }
+                    else if(!__any(!ok)) {
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                        for(uint32_t x = listBase + lane; x < listBase + listed; x += WAVE) {
+                            const uint2 pr = shSeg[slot & 1][x];
+                            const ResProj &P = shProj[pr.y];
+                            takeEntry(readEntry(asGlobal(P.seg) + QUADS * ((size_t)pr.x * tilesInGroup + tileInGroup)), pr.y << RES_SEG_PROJ_SHIFT, P.lds + shProjPtr[slot][pr.y], slot, x, skipInline, count);
+                        }
                     }
                 }
                 else {
-                    left = true;
-                    for(uint32_t r = pos; r < RES_PAIR_CAP; r++) { shSeg[slot & 1][r] = make_uint2(0u, 0u); }
-                    shTaken[slot].left = 1u;
+                    // (what nearly every quiet step has: at most one pair a thread.  Handling up to three here, unrolled or in a loop, made the
+                    // step slower whether it had them or not)
+                    if(total) {
+                        takeEntry(readEntry(watchSeg + (size_t)idOf(watchSub) * rowQuads), watchFlags, watchLds + shProjPtr[slot][watchFlags >> RES_SEG_PROJ_SHIFT],
+                                  slot, listBase + __popcll(busy & ((1ull << lane) - 1ull)), skipInline, count);
+                    }
                 }
             }
         }
+        if(lane == 0) { shListed[slot][wave] = listed; }
         if(!ok) { shTaken[slot].failed = 1u; }
     };
 
@@ -595,17 +563,17 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     // A synapse is "due" when it lands in the slot read this step (delay a multiple of the ring depth, or no ring).
     // PASS_ALL adds every synapse, PASS_LATER those not due, PASS_DUE the due ones; `flaggedOnly` restricts the walk to
     // segments whose due synapses are not all inline in their entry.
-    // (wavefront `first` of the `count` that call)
-    auto process = [&](const uint2 *segs, const uint32_t *fronts, uint32_t numPairs, uint32_t pass, bool flaggedOnly, uint32_t first, uint32_t count) {
+    // (wavefront `first` of the `count` that call; pair q is in segs[place(q)], which all lanes ask for together)
+    auto process = [&](const uint2 *segs, auto place, const uint32_t *fronts, uint32_t numPairs, uint32_t pass, bool flaggedOnly, uint32_t first, uint32_t count) {
         constexpr uint32_t TRIP = 4, DUE_END = 4 * TILE;
         const uint32_t from = (pass == PASS_LATER) ? DUE_END : 0u, span = (pass == PASS_DUE) ? DUE_END : 0xFFFFFFFFu - from;      // offsets that are added
         const uint32_t shift = (numPairs <= 4 * count) ? 4u : (numPairs <= 8 * count) ? 3u : 2u;
         const uint32_t lanesPerPair = 1u << shift, pairsPerGroup = WAVE >> shift;
         for(uint32_t q0 = first * pairsPerGroup; q0 < numPairs; q0 += count * pairsPerGroup) {
-            const uint32_t q = q0 + (lane >> shift);
+            const uint32_t q = q0 + (lane >> shift), at = place(min(q, numPairs - 1u));
             uint32_t len = 0, start = 0, proj = 0;
             if(q < numPairs) {
-                const uint2 sg = segs[q];
+                const uint2 sg = segs[at];
                 proj = sg.y >> RES_SEG_PROJ_SHIFT;
                 const bool flagged = (sg.y & RES_SEG_OVERFLOW) != 0;
                 const bool skip = (flaggedOnly && !flagged) || (pass == PASS_LATER && (sg.y & RES_SEG_NO_DELAY));
@@ -661,33 +629,52 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             for(uint32_t q = tid; q < numPairs; q += THREADS) {
                 const uint2 pr = shSeg[other][q];
                 const ResProj &P = shProj[pr.y];
-                const u32x4 lo4 = (asGlobal(P.seg) + ((WIDE && P.wide) ? RES_WIDE_QUADS : 2u) * ((size_t)pr.x * tilesInGroup + tileInGroup))[0];
+                const u32x4 lo4 = (asGlobal(P.seg) + QUADS * ((size_t)pr.x * tilesInGroup + tileInGroup))[0];
                 shSeg[other][q] = make_uint2(lo4.x, (lo4.y & ~(0x3Fu << RES_SEG_PROJ_SHIFT)) | (pr.y << RES_SEG_PROJ_SHIFT));
                 if(count) { events += lo4.y & 0xFFFFu; }
             }
             __syncthreads();
-            process(shSeg[other], shProjPtr[slot], numPairs, pass, false, wave, WAVES);
+            process(shSeg[other], [](uint32_t q) { return q; }, shProjPtr[slot], numPairs, pass, false, wave, WAVES);
             __syncthreads();
         }
     };
 
     // After poll(), by all threads: the barrier, and whatever the listed entries could not deliver at once.  `convention` is PASS_ALL
     // normally, PASS_LATER when a previous launch has already delivered the due synapses of these spikes, PASS_DUE when only those
-    // are wanted.  False: some wait expired.  `later`: listed pairs whose remaining synapses are to be added before the next update.
-    uint32_t later = 0;
+    // are wanted.  False: some wait expired.
+    auto walkListed = [&](uint32_t slot, uint32_t pass, bool flaggedOnly, uint32_t first, uint32_t count) {
+        // (pair q of the wavefronts' parts one after the other)
+        uint32_t upTo = (lane < watchWaves) ? shListed[slot][lane] : 0u;
+        #pragma unroll
+        for(uint32_t d = 1; d < MAIN; d <<= 1) {
+            const uint32_t below = __shfl_up(upTo, d);
+            upTo += (lane >= d) ? below : 0u;
+        }
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)upTo, MAIN - 1);
+        auto place = [&](uint32_t q) {
+            uint32_t part = 0, before = 0;
+            #pragma unroll
+            for(uint32_t half = (MAIN > 8) ? 8 : (MAIN > 4) ? 4 : 2; half != 0; half /= 2) {
+                const uint32_t x = __shfl(upTo, part + half - 1);
+                before = (x <= q) ? x : before;
+                part = (x <= q) ? part + half : part;
+            }
+            return part * listCap + q - before;
+        };
+        if(total) { process(shSeg[slot & 1], place, shProjPtr[slot], total, pass, flaggedOnly, first, count); }
+    };
     auto deliverDue = [&](uint32_t step, uint32_t convention) -> bool {
         const uint32_t slot = (uint32_t)(seqBase + step) & 3u;
         ldsBarrier();
         Taken taken = shTaken[slot];
-        taken.pairs = __builtin_amdgcn_readfirstlane(taken.pairs); taken.flagged = __builtin_amdgcn_readfirstlane(taken.flagged);
+        taken.flagged = __builtin_amdgcn_readfirstlane(taken.flagged);
         taken.left = __builtin_amdgcn_readfirstlane(taken.left); taken.failed = __builtin_amdgcn_readfirstlane(taken.failed);
-        later = min(taken.pairs, RES_PAIR_CAP);
         if(taken.flagged | taken.left | taken.failed) {
             if(taken.failed) {
                 if(tid == 0) { raiseErrorFlag(errorFlag); }
                 return false;
             }
-            if(convention != PASS_LATER && taken.flagged) { process(shSeg[slot & 1], shProjPtr[slot], later, PASS_DUE, true, wave, WAVES); ldsBarrier(); }
+            if(convention != PASS_LATER && taken.flagged) { walkListed(slot, PASS_DUE, true, wave, WAVES); ldsBarrier(); }
             if(taken.left) { leftOver(step, convention, convention != PASS_DUE); }
         }
         return true;
@@ -784,6 +771,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             ldsBarrier();
             if(wave == 0) { publish(k + 2, shDone[slot]); }
         }
+        published = (uint32_t)__builtin_readcyclecounter();
         // while the words of this step travel: the step's recording words, and (next) the synapses of the previous step's spikes
         // that are not due yet
         if(recordHere) { *recordAt = (lane & 32) ? (uint32_t)(ballot >> 32) : (uint32_t)ballot; }
@@ -796,8 +784,8 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
             psmAt[m] = (next >= psmEnd[m]) ? psmAt[m] + (psmRing[m] ? TILE - psmRing[m] : 0u) : next;
         }
         }
-        if((WALK == 0 || !main) && anyRing && later) {       // (without a ring nothing is: the next word is looked for at once)
-            process(shSeg[slot & 1], shProjPtr[slot], later, PASS_LATER, false, WALK ? wave - MAIN : wave, WALK ? WALK : MAIN);
+        if((WALK == 0 || !main) && anyRing) {       // (without a ring nothing is: the next word is looked for at once)
+            walkListed(slot, PASS_LATER, false, WALK ? wave - MAIN : wave, WALK ? WALK : MAIN);
         }
     }
 
@@ -828,7 +816,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
     }
-    uint32_t offset = (watching && watchSub == 0 && !(grouped && (lane & (RES_WIDE_QUADS - 1)) != 0) && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
+    uint32_t offset = (watching && watchSub == 0 && !(grouped && (lane & (RES_MAX_QUADS - 1)) != 0) && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
     if(tid == 0) { shScalar[2] = 0; }
     __syncthreads();
     if(offset) { atomicAdd(&shScalar[2], offset); }

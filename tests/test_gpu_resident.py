@@ -389,3 +389,24 @@ def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
     model, oracle, spikes = _run_chunks(net, (14, -2, 14), check)
     assert spikes > n_a // 16
     model.unload()
+
+
+@pytest.mark.parametrize("together", [1, 3, 4, 5, 8, 33, 256])
+@pytest.mark.parametrize("depth", [0, 5])
+def test_spikes_of_one_tile_in_one_step(together, depth):
+    """Of a tile of 256 neurons `together` fire in the first step: up to three travel in the tile's word and more in its side list, and the
+    128 threads that watch the tile of so small a network take one, some or none of them each."""
+    n_a, n_b = 256, 200
+    net = Net(name="resident_together", dt=1.0, steps=40)
+    net.pops.append(_pop("A", n_a, 0.62, np.where(np.arange(n_a) * 97 % 256 < together, -50.01, -60.0)))
+    net.pops.append(_pop("B", n_b, 0.3, np.full(n_b, -58.0)))
+    net.pops[0].params["Ioffset"] = 0.55
+    net.syns.append(_projection("AB", "A", "B", n_a, n_b, 20, 0.3, 21, depth, 0.3))
+    net.syns.append(_projection("AA", "A", "A", n_a, n_a, 9, 0.2, 22, depth, 0.3))
+
+    def check(model, oracle):
+        compare_state(net, model, oracle, f"after {model.timestep} steps", exact=True)
+
+    model, oracle, spikes = _run_chunks(net, (6, 34), check)
+    assert int(np.unpackbits(oracle.record("A", 40).reshape(40, -1)[0].view(np.uint8)).sum()) == together
+    model.unload()
