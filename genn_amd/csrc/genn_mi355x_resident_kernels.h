@@ -463,11 +463,11 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     auto spikesOf = [&]() -> uint32_t { return (uint32_t)(word >> 32) & RES_COUNT_MASK; };
     auto idOf = [&](uint32_t e) -> uint32_t { return ((uint32_t)word >> (RES_ID_BITS * e)) & RES_ID_MASK; };        // (e < RES_WORD_IDS)
     // Cycles from a tile's own word to its first look for the others'.  A look that comes too early costs its whole trip to memory again, and
-    // the looks of all the waiting tiles slow the words down.  us a step without / with the wait (of 1,000 cycles, from 129 tiles on of 1,300: 1,000 and
-    // 1,500 gave 3.29 and 3.24 at 40,000 x 80, 4.30 and 4.04 at 100,000 x 80, 2.37 and 2.42 at 20,000 x 100): 20,000 x 100 2.76 / 2.43,
-    // 40,000 x 80 3.79 / 3.26, 100,000 x 80 4.83 / 4.15, 250,000 x 200 6.2 / 4.3, the full microcircuit 4.66 / 4.12.  A handful of tiles are too quick for it (1,000 x 80 2.10 / 2.17).
-    // Drawing of Poisson sources takes longer than the wait.
-    const uint32_t firstLook = (numTiles <= 8) ? 0u : (numTiles <= 128) ? 1000u : 1300u;
+    // the looks of all the waiting tiles slow the words down: the more tiles, the longer the words take.  us a step without the wait / with 1,000 /
+    // 1,500 / 2,000 cycles / as below: 20,000 x 100 (79 tiles) 2.76 / 2.37 / 2.42 / 2.62 / 2.35, 40,000 x 80 (157) 3.79 / 3.29 / 3.24 / 3.41 / 3.25,
+    // 100,000 x 80 (196) 4.83 / 4.30 / 4.04 / 4.05 / 4.05, the full microcircuit (243) 4.66 / 4.23 / - / - / 4.09.  A handful of tiles are too quick for it
+    // (1,000 x 80 2.10 / 2.17).  Drawing of Poisson sources takes longer than the wait.
+    const uint32_t firstLook = (numTiles <= 8) ? 0u : min(800u + 4u * numTiles, 1700u);
     uint32_t published = (uint32_t)__builtin_readcyclecounter();
     auto poll = [&](uint32_t step, uint32_t convention) {
         const uint32_t seq = (uint32_t)(seqBase + step) & RES_SEQ_MASK;
