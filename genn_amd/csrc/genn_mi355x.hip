@@ -831,36 +831,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         for(const auto &l : links) { incoming += (l.trg == gi) ? 1 : 0; }
         if(incoming > RES_MAX_PROJ) { return GENNMI_OK; }
     }
-    // are rows sorted by target, and how many of a sample of each projection's synapses are due (words 1 + 2 k: of 2 + 2 k)
-    uint32_t *dSeen = nullptr;
-    std::vector<uint32_t> seen(1 + 2 * r->pre.size(), 0u);
-    HIP_TRY(poolMalloc(&dSeen, seen.size() * sizeof(uint32_t)));
-    HIP_TRY(hipMemset(dSeen, 0, seen.size() * sizeof(uint32_t)));
-    for(size_t k = 0; k < r->pre.size(); k++) {
-        const auto &q = r->pre[k].g;
-        const size_t entries = (size_t)q.numSrcNeurons * q.rowStride;
-        residentSortedKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, dSeen);
-        if(q.maxDenDelay) { residentDueKernel<<<dim3(std::min(64u, q.numSrcNeurons)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.d, q.maxDenDelay, dSeen + 1 + 2 * k); }
-    }
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpy(seen.data(), dSeen, seen.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(poolFree(dSeen));
-    if(seen[0]) { return GENNMI_OK; }
-    // Quads of a segment entry, by the largest mean number of synapses of a row part that are due (rowStride is a little more than a row's
-    // mean): an entry should hold what all but one part in thousands has.  Where eight lanes can watch a tile, one of eight costs what
-    // a smaller one does; nowhere more than 4 GiB of them, and not where the parts are too long for any.
-    double due = 0.0;
-    uint64_t entriesInAll = 0;
-    for(size_t k = 0; k < r->pre.size(); k++) {
-        const auto &q = r->pre[k].g;
-        const double share = q.maxDenDelay ? (double)seen[1 + 2 * k] / std::max(1u, seen[2 + 2 * k]) : 1.0;
-        due = std::max(due, share * q.rowStride * tileSize / q.numTrgNeurons);
-        entriesInAll += (uint64_t)q.numSrcNeurons * numTilesOf[links[k].trg];
-    }
-    uint32_t wanted = (due <= 1.0 || due > 16.0) ? 2u : (due <= 5.0 && (anyRing || tiles.size() > tileSize / RES_MAX_QUADS)) ? 4u : 8u;
-    if(const char *envQuads = getenv("GENNMI_RESIDENT_QUADS")) { wanted = (uint32_t)atoi(envQuads); }
-    while(wanted > 2 && entriesInAll * wanted * sizeof(u32x4) > (4ull << 30)) { wanted /= 2; }
-    // the instance for the network's tiles, sources and postsynaptic models whose entries come closest to that
+    // the instances for the network's tiles, sources and postsynaptic models: one for each size of segment entry, smallest first
     struct Instance { uint32_t tile; bool walkers, poisson; uint32_t psm, quads; decltype(r->resKernel) kernel; };
     constexpr uint32_t MAX = GENNMI_MAX_PSM;
     static const Instance instances[] = {
@@ -875,13 +846,52 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         {1024, false, true, 2, 4, residentKernel<true, 4, 2, 1024, 0>},
         {256, false, true, MAX, 4, residentKernel<true, 4, MAX, 256, 0>}, {512, false, true, MAX, 4, residentKernel<true, 4, MAX, 512, 0>},
         {1024, false, true, MAX, 2, residentKernel<true, 2, MAX, 1024, 0>}};
-    decltype(r->resKernel) residentInstance = nullptr;
-    uint32_t quads = 0;
+    std::vector<Instance> choices;
     for(const auto &c : instances) {
-        if(c.tile != tileSize || c.walkers != walkers || c.psm != (maxPSM <= 2 ? 2u : MAX) || (maxPSM <= 2 && c.poisson != poisson)) { continue; }
-        if(!residentInstance || (c.quads <= wanted && c.quads > quads) || (quads > wanted && c.quads < quads)) { residentInstance = c.kernel; quads = c.quads; }
+        if(c.tile == tileSize && c.walkers == walkers && c.psm == (maxPSM <= 2 ? 2u : MAX) && (maxPSM > 2 || c.poisson == poisson)) { choices.push_back(c); }
     }
-    if(!residentInstance) { return GENNMI_OK; }
+    if(choices.empty()) { return GENNMI_OK; }
+    // are rows sorted by target, and, where there is a choice of entries, how many of a sample of each projection's synapses are due
+    // (words 1 + 2 k: of 2 + 2 k)
+    uint32_t *dSeen = nullptr;
+    std::vector<uint32_t> seen(1 + 2 * r->pre.size(), 0u);
+    HIP_TRY(poolMalloc(&dSeen, seen.size() * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(dSeen, 0, seen.size() * sizeof(uint32_t)));
+    for(size_t k = 0; k < r->pre.size(); k++) {
+        const auto &q = r->pre[k].g;
+        const size_t entries = (size_t)q.numSrcNeurons * q.rowStride;
+        residentSortedKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, dSeen);
+        if(q.maxDenDelay && choices.size() > 1) {
+            residentDueKernel<<<dim3(std::min(64u, q.numSrcNeurons)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.d, q.maxDenDelay, dSeen + 1 + 2 * k);
+        }
+    }
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpy(seen.data(), dSeen, seen.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    HIP_TRY(poolFree(dSeen));
+    if(seen[0]) { return GENNMI_OK; }
+    // Quads of a segment entry, where there is a choice: by the largest mean number of synapses of a row part that are due (rowStride is a
+    // little more than a row's mean), an entry should hold what all but one part in thousands has.  A population smaller than a tile gets the
+    // whole of a row and no more; a projection whose parts are too long for any entry is walked whatever the entries are, and has no say but that
+    // eight lanes that share an entry of eight quads would walk it alone.  Where eight lanes can watch a tile, one of eight quads
+    // costs what a smaller one does; and larger ones than the smallest only up to 4 GiB of them.  us a step of a balanced network that projects onto a small
+    // population besides, with entries of 2 / 4 / 8 quads: 4,000 x 80, onto 5 of 20 neurons 2.55 / 2.26 / 2.18 (8 is taken), onto 60 of 100 2.58 / 2.40 / 3.08
+    // (4); 20,000 x 100 2.96 / 2.18 / 2.30 (4) and 3.84 / 3.86 / 3.92 (4).
+    double due = 0.0;
+    bool beyond = false;
+    uint64_t entriesInAll = 0;
+    for(size_t k = 0; k < r->pre.size(); k++) {
+        const auto &q = r->pre[k].g;
+        const double share = q.maxDenDelay ? (double)seen[1 + 2 * k] / std::max(1u, seen[2 + 2 * k]) : 1.0;
+        const double part = share * q.rowStride * std::min(1.0, (double)tileSize / q.numTrgNeurons);
+        if(part <= 16.0) { due = std::max(due, part); } else { beyond = true; }
+        entriesInAll += (uint64_t)q.numSrcNeurons * numTilesOf[links[k].trg];
+    }
+    uint32_t wanted = (due <= 1.0) ? 2u : (beyond || (due <= 5.0 && (anyRing || tiles.size() > tileSize / RES_MAX_QUADS))) ? 4u : 8u;
+    if(const char *envQuads = getenv("GENNMI_RESIDENT_QUADS")) { wanted = (uint32_t)atoi(envQuads); }
+    size_t choice = 0;
+    while(choice + 1 < choices.size() && choices[choice + 1].quads <= wanted && entriesInAll * choices[choice + 1].quads * sizeof(u32x4) <= (4ull << 30)) { choice++; }
+    const auto residentInstance = choices[choice].kernel;
+    const uint32_t quads = choices[choice].quads;
     const void *kernel = reinterpret_cast<const void*>(residentInstance);
     if(ldsBytes > 32 * 1024) {
         HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
@@ -2434,7 +2444,8 @@ int gennmi_runner_get_info(gennmi_runner *r, uint32_t info[4])
     if(!r || !info) { return fail(GENNMI_EINVAL, "runner_get_info: null argument"); }
     if(!r->finalised) { return fail(GENNMI_ESTATE, "runner_get_info: runner not finalised"); }
     info[0] = (r->fusedStep ? 1u : 0u) | (r->resident ? 2u : 0u) | (r->neuronsPerLane > 1 ? 4u : 0u) | (r->ordered ? 8u : 0u)
-              | (r->combineSynapses ? 16u : 0u) | ((r->combineSynapses && r->combinePost) ? 32u : 0u) | (r->convMfmaBlocks ? 64u : 0u) | (r->convStep ? 128u : 0u) | (r->ahead ? 256u : 0u); info[1] = r->neuronBlocks; info[2] = r->preBlocks; info[3] = r->postBlocks;
+              | (r->combineSynapses ? 16u : 0u) | ((r->combineSynapses && r->combinePost) ? 32u : 0u) | (r->convMfmaBlocks ? 64u : 0u) | (r->convStep ? 128u : 0u) | (r->ahead ? 256u : 0u)
+              | (r->resident ? (r->resThreads > r->resTileSize ? 512u : 0u) | (r->resQuads << 12) | (r->resTileSize << 16) : 0u); info[1] = r->neuronBlocks; info[2] = r->preBlocks; info[3] = r->postBlocks;
     return GENNMI_OK;
 }
 

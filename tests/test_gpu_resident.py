@@ -357,6 +357,31 @@ def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypat
     model.unload()
 
 
+@pytest.mark.parametrize("n_c, targets, quads", [(None, 0, 8), (20, 5, 8), (100, 60, 4)])
+def test_one_projection_does_not_set_every_entry(n_c, targets, quads, monkeypatch):
+    """Two populations whose row parts want entries of eight quads (14 targets over 2.3 tiles: 6 a part).  A third one smaller than a tile has the
+    whole of a row, 5 targets, in its only part, which asks for no more than the others; parts of 60 are too long for any entry: four quads."""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
+    n_a, n_b = 700, 600
+    net = Net(name="resident_entries", dt=1.0, steps=120)
+    net.pops.append(_pop("A", n_a, 0.62, -60.0 + 9.5 * rng.uniform(5, 1, 0, n_a)))
+    net.pops.append(_pop("B", n_b, 0.45, -60.0 + 9.5 * rng.uniform(5, 2, 0, n_b)))
+    net.syns.append(_projection("AB", "A", "B", n_a, n_b, 14, 0.2, 21))
+    net.syns.append(_projection("BA", "B", "A", n_b, n_a, 14, -0.15, 22))
+    if n_c:
+        net.pops.append(_pop("C", n_c, 0.3, -60.0 + 9.5 * rng.uniform(5, 3, 0, n_c)))
+        net.syns.append(_projection("AC", "A", "C", n_a, n_c, targets, 0.01, 23))
+
+    def check(model, oracle):
+        compare_state(net, model, oracle, f"after {model.timestep} steps", exact=True)
+
+    model, oracle, spikes = _run_chunks(net, (60, 60), check)
+    info = model.runner_info()
+    assert (info["resident_tile"], info["resident_quads"], info["resident_walkers"]) == (256, quads, False)
+    assert spikes > 700
+    model.unload()
+
+
 @pytest.mark.parametrize("n_a, n_b, depth, models, poisson", [
     (256, 1, 0, 1, False), (250, 255, 1, 1, False), (32760, 3, 0, 1, False), (32760, 260, 2, 1, False),            # few tiles, threads share a tile's word
     (65000, 300, 3, 2, False), (65500, 200, 5, 1, True), (65530, 300, 0, 2, True), (65530, 300, 4, 2, False),      # up to, and one beyond, 256 tiles of 256
