@@ -810,7 +810,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     for(const auto &p : r->pre) {
         const auto &q = p.g;
         if(q.matrix != GENNMI_MATRIX_SPARSE || (q.wum != GENNMI_WUM_STATIC_PULSE && q.wum != GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY)) { return GENNMI_OK; }
-        if((unsigned long long)q.numSrcNeurons * q.rowStride > 0xFFFFFFFFull) { return GENNMI_OK; }
+        if((unsigned long long)q.numSrcNeurons * q.rowStride > 0xFFFFFFFFull || q.rowStride > 0xFFFFu) { return GENNMI_OK; }      // (a row part's length is a 16-bit field)
         const bool delayed = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY);
         Link l{r->neuron.size(), r->neuron.size(), 0};
         for(size_t gi = 0; gi < r->neuron.size(); gi++) {
@@ -899,14 +899,21 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     int perCU = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, residentInstance, (int)residentThreads, ldsBytes));
     if((size_t)perCU * numCU < tiles.size()) { return GENNMI_OK; }
+    // no room for the tables and the second copy of the synapses: the network steps with the other plans
+    auto noRoom = [r]() -> int {
+        (void)hipGetLastError();
+        for(auto *q : r->resSegs) { r->owned.erase(std::find(r->owned.begin(), r->owned.end(), (void*)q)); HIP_TRY(poolFree(q)); }
+        for(auto *q : r->resPacked) { r->owned.erase(std::find(r->owned.begin(), r->owned.end(), (void*)q)); HIP_TRY(poolFree(q)); }
+        r->resSegs.clear(); r->resPacked.clear(); r->resSegTiles.clear();
+        return GENNMI_OK;
+    };
     for(size_t k = 0; k < r->pre.size(); k++) {
         const auto &q = r->pre[k].g;
         const Link &l = links[k];
         const uint32_t tilesInGroup = numTilesOf[l.trg];
         const size_t entries = (size_t)q.numSrcNeurons * tilesInGroup;
-        if(q.rowStride > 0xFFFFu) { return GENNMI_OK; }         // a segment's length is a 16-bit field (device allocations made so far stay owned)
         u32x4 *dSeg = nullptr;
-        HIP_TRY(poolMalloc(&dSeg, entries * quads * sizeof(u32x4)));
+        if(poolMalloc(&dSeg, entries * quads * sizeof(u32x4)) != hipSuccess) { return noRoom(); }
         r->owned.push_back(dSeg);
         const uint32_t depth = (q.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? q.maxDenDelay : 0u;
         residentSegKernel<<<dim3((unsigned int)((entries + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(q.numSrcNeurons, q.rowStride, q.rowLength, q.ind, q.g, q.d,
@@ -916,10 +923,7 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
         HIP_TRY(hipGetLastError());
         const size_t padded = (size_t)q.numSrcNeurons * q.rowStride;
         u32x2 *dPacked = nullptr;
-        if(poolMalloc(&dPacked, std::max<size_t>(padded, 1) * sizeof(u32x2)) != hipSuccess) {
-            (void)hipGetLastError();            // no room for the second copy of the synapses: the network steps with the other plans
-            return GENNMI_OK;
-        }
+        if(poolMalloc(&dPacked, std::max<size_t>(padded, 1) * sizeof(u32x2)) != hipSuccess) { return noRoom(); }
         r->owned.push_back(dPacked);
         if(padded) {
             residentPackKernel<<<dim3((unsigned int)((padded + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, 0>>>(padded, q.ind, q.g, q.d, depth, tileSize, dPacked);
