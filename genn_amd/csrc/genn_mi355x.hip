@@ -96,6 +96,9 @@ struct gennmi_runner
     uint32_t resTiles = 0, resReplicaStride = 0; unsigned long long resSeq = 0; size_t resLdsBytes = 0;
     decltype(&residentKernel<false, 2, 2, 256, 0>) resKernel = nullptr;      // the instantiation its sources, segment entries and tiles need
     uint32_t resThreads = BLOCK, resTileSize = BLOCK;     // ... its work-group, and neurons of a tile
+    uint32_t resRoom[2] = {0, 0}; int resDevice = 0;      // ... compute units, its work-groups on one at most; where they are
+    hipEvent_t resDone = nullptr;       // see residentRoom(): what others wait for
+    unsigned long long resOrder = 0;    // number of its last resident launch, 0: it has none in flight
     std::vector<u32x4*> resSegs;        // segment table of each presynaptic group, in push order
     std::vector<uint32_t> resSegTiles;  // tiles of its target population
     uint32_t resQuads = 2;              // 16-byte quads of an entry
@@ -141,6 +144,10 @@ struct gennmi_runner
 // overlaps one of their projections' arrays makes them rebuild the tables before the next resident launch.
 static std::mutex g_runnersMutex;
 static std::vector<gennmi_runner*> g_runners;
+// Runners on the resident plan, and the number of the last resident launch (held from the look for room to the launch, see residentRoom()).
+static std::mutex g_residentMutex;
+static std::vector<gennmi_runner*> g_residents;
+static unsigned long long g_residentOrder = 0;
 
 static void noteDeviceWrite(const void *dev, size_t bytes)
 {
@@ -545,12 +552,17 @@ int gennmi_runner_destroy(gennmi_runner *r)
     if(!r) { return GENNMI_OK; }
     if(!r->queued.empty()) { r->queued.clear(); g_queuedRunners--; }      // nothing can observe these steps any more
     {
+        std::lock_guard<std::mutex> lock(g_residentMutex);
+        g_residents.erase(std::remove(g_residents.begin(), g_residents.end(), r), g_residents.end());
+    }
+    {
         std::lock_guard<std::mutex> lock(g_runnersMutex);
         g_runners.erase(std::remove(g_runners.begin(), g_runners.end(), r), g_runners.end());
     }
     hipStreamSynchronize(r->stream);
     for(hipEvent_t e : r->eventPool) { hipEventDestroy(e); }
     for(hipEvent_t e : r->marks) { if(e) { hipEventDestroy(e); } }
+    if(r->resDone) { hipEventDestroy(r->resDone); }
     for(void *q : r->owned) { poolFree(q); }
     for(void *q : r->zeroOwned) { poolFree(q); }
     for(void *q : r->orderedOwned) { poolFree(q); }
@@ -963,7 +975,36 @@ static int setupResident(gennmi_runner *r, uint32_t numCU)
     r->resLdsBytes = ldsBytes;
     r->resKernel = residentInstance;
     r->resThreads = residentThreads; r->resTileSize = tileSize; r->resQuads = quads;
+    r->resRoom[0] = numCU; r->resRoom[1] = (uint32_t)perCU;
+    HIP_TRY(hipGetDevice(&r->resDevice));
+    HIP_TRY(hipEventCreateWithFlags(&r->resDone, hipEventDisableTiming));
     r->resident = true;
+    std::lock_guard<std::mutex> lock(g_residentMutex);
+    g_residents.push_back(r);
+    return GENNMI_OK;
+}
+
+// Room for a resident launch (g_residentMutex held): two whose work-groups do not all fit on the chip can each get a part of them there and
+// wait for the rest until the bound of the wait, so a launch waits for as many of the other runners' streams, the one that launched first
+// first, as leave it room beside the others.  Any compute unit with fewer work-groups than the smallest of their limits takes one more.
+static int residentRoom(gennmi_runner *r)
+{
+    std::vector<gennmi_runner*> others;
+    for(auto *o : g_residents) {
+        if(o == r || !o->resOrder || o->resDevice != r->resDevice) { continue; }
+        if(hipStreamQuery(o->stream) == hipSuccess) { o->resOrder = 0; }
+        else { (void)hipGetLastError(); others.push_back(o); }
+    }
+    std::sort(others.begin(), others.end(), [](const gennmi_runner *a, const gennmi_runner *b) { return a->resOrder < b->resOrder; });
+    for(size_t first = 0; first < others.size(); first++) {
+        size_t tiles = r->resTiles;
+        uint32_t perCU = r->resRoom[1];
+        for(size_t k = first; k < others.size(); k++) { tiles += others[k]->resTiles; perCU = std::min(perCU, others[k]->resRoom[1]); }
+        if(tiles <= (size_t)perCU * r->resRoom[0]) { break; }
+        HIP_TRY(hipEventRecord(others[first]->resDone, others[first]->stream));
+        HIP_TRY(hipStreamWaitEvent(r->stream, others[first]->resDone, 0));
+    }
+    r->resOrder = ++g_residentOrder;
     return GENNMI_OK;
 }
 
@@ -999,6 +1040,8 @@ static int launchResident(gennmi_runner *r, unsigned long long timestep, unsigne
     for(unsigned long long done = 0; done < numSteps; ) {
         const uint32_t chunk = (uint32_t)std::min(MAX_STEPS, numSteps - done);
         const auto launch = r->resKernel;
+        std::lock_guard<std::mutex> lock(g_residentMutex);
+        { const int rc = residentRoom(r); if(rc) { return rc; } }
         launch<<<dim3(r->resTiles), dim3(r->resThreads), r->resLdsBytes, r->stream>>>(
             r->dResTiles, r->resTiles, r->dResGroups, r->dResTileGroup, r->dResTags, r->dResSide, timestep + done, r->epoch, numRecordingTimesteps,
             chunk, r->dt, r->fusedStep ? 1u : 0u, r->dError, r->dEvents, r->resReplicaStride, r->resSeq);

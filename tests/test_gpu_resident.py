@@ -6,6 +6,8 @@ stages at once, tiles with many spikes in one step (side buffer), weights pushed
 Weights are one value per projection and every postsynaptic model has one incoming projection, so no fp32 sum depends
 on the order of its additions and everything — state, rings, spike queues, recordings, event counts — must be identical.
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -435,3 +437,56 @@ def test_spikes_of_one_tile_in_one_step(together, depth):
     model, oracle, spikes = _run_chunks(net, (6, 34), check)
     assert int(np.unpackbits(oracle.record("A", 40).reshape(40, -1)[0].view(np.uint8)).sum()) == together
     model.unload()
+
+
+@pytest.mark.parametrize("threads", [False, True])
+def test_networks_that_do_not_fit_together(threads):
+    """Two networks of 158 tiles, each a compute unit's worth, do not fit on the chip together, and a third of 13 fits beside one of them.
+    Stepped at the same time, a launch behind the other's without a wait between them or from a thread each, every one is as if alone."""
+    steps, chunk = 48, 4
+    sizes = (40000, 40000, 3000)
+    nets = []
+    for k, n in enumerate(sizes):
+        net = Net(name=f"resident_beside{k}", dt=1.0, steps=steps)
+        net.pops.append(_pop("A", n, 0.62, -60.0 + 9.9 * rng.uniform(5, 1 + k, 0, n)))
+        net.pops.append(_pop("B", 300, 0.45, -60.0 + 9.9 * rng.uniform(6, 1 + k, 0, 300)))
+        net.syns.append(_projection("AB", "A", "B", n, 300, 4, 0.002, 31 + k, 4, 0.3))
+        net.syns.append(_projection("BA", "B", "A", 300, n, 40, 0.2, 41 + k, 4, 0.3))
+        nets.append(net)
+    models = [model_from_net(net) for net in nets]
+    for model, n in zip(models, sizes):
+        model.load(num_recording_timesteps=steps)
+        info = model.runner_info()
+        assert info["resident_plan"] and info["resident_tile"] == 256 and info["resident_walkers"]
+    if threads:
+        failed = []
+
+        def work(model):
+            try:
+                for _ in range(steps // chunk):
+                    model.run(chunk)
+                model.synchronize()
+            except Exception as e:
+                failed.append(e)
+
+        workers = [threading.Thread(target=work, args=(model,)) for model in models]
+        for w in workers:
+            w.start()
+        for w in workers:
+            w.join()
+        assert not failed
+    else:
+        for _ in range(steps // chunk):
+            for model in models:
+                model.run(chunk)
+        for model in models:
+            model.synchronize()
+    for net, model in zip(nets, models):
+        oracle = OracleNet(net, num_recording_timesteps=steps)
+        oracle.run(steps)
+        compare_state(net, model, oracle, f"of {net.name}", exact=True)
+        model.pull_recording_buffers_from_device()
+        for p in net.pops:
+            assert np.array_equal(model.neuron_populations[p.name].vars["recordSpk"].view, oracle.record(p.name, steps)), f"recording of {p.name} differs"
+        assert model.synaptic_event_count == oracle.events() > 0
+        model.unload()
