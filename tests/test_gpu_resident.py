@@ -113,17 +113,17 @@ def test_more_pairs_than_a_tile_stages(depth):
     model.unload()
 
 
-@pytest.mark.parametrize("n_a, ioffset", [(400, 1.0), (24, 0.62), (12, 0.62)])
-def test_long_row_parts_take_several_trips(n_a, ioffset):
-    """Rows of 120 targets inside one tile of 200 neurons: a pair's part is longer than what its group of lanes reads in
-    one trip to memory when many pairs are staged (400 sources crossing threshold together: 4 lanes per pair, 32 synapses
-    per trip), and fits one trip when few are (24 or 12 sources firing now and then: 8 or 16 lanes per pair)."""
+@pytest.mark.parametrize("n_a, ioffset, targets", [(400, 1.0, 120), (24, 0.62, 120), (12, 0.62, 120), (400, 1.0, 14), (24, 0.62, 64), (12, 0.62, 50), (12, 0.62, 65)])
+def test_long_row_parts_take_several_trips(n_a, ioffset, targets):
+    """Rows inside one tile of 200 neurons.  A lane reads four synapses of its pair's part in one trip to memory: a pair has 4 lanes and 16 synapses
+    a trip when many pairs are listed (400 sources crossing threshold together), 16 lanes and 64 synapses when few are (24 or 12 sources firing
+    now and then).  Parts of 120 and 65 take several trips, parts of 14, 50 and 64 take one."""
     n_b, depth = 200, 6
     net = Net(name="resident_long_parts", dt=1.0, steps=0)
     v0 = np.full(n_a, -50.4) if n_a == 400 else -60.0 + 9.5 * rng.uniform(41, 1, 0, n_a)
     net.pops.append(_pop("A", n_a, ioffset, v0))
     net.pops.append(_pop("B", n_b, 0.3, np.full(n_b, -58.0)))
-    net.syns.append(_projection("AB", "A", "B", n_a, n_b, 120, 0.004 if n_a == 400 else 0.05, 42, depth, 0.1))
+    net.syns.append(_projection("AB", "A", "B", n_a, n_b, targets, 0.004 if n_a == 400 else 0.05, 42, depth, 0.1))
     net.steps = 90
 
     def check(model, oracle):
@@ -326,8 +326,8 @@ def test_expired_wait_is_reported_not_hung(resident, monkeypatch):
 
 @pytest.mark.parametrize("stride,crowded", [(2, 0.0), (5, 0.0), (14, 0.0), (30, 0.5), (30, 1.0), (90, 0.0)])
 def test_row_parts_without_delay_inside_their_entries(stride, crowded, monkeypatch):
-    """Projections without a ring: a row's part in a tile is up to four synapses in an ordinary entry (stride 2), up to 24 in a wide one (5, 14),
-    longer than that (30 targets crowded into one tile, in some or in all rows) or walked as before (90).  Weights are pushed between
+    """Projections without a ring: a row's part in a tile is up to four synapses in an entry of two quads (stride 2), up to 22 in one of eight (5, 14),
+    longer than that (30 targets crowded into one tile, in some or in all rows) or too long for any entry (90).  Weights are pushed between
     launches, so that the entries' copies of them are rebuilt.  (The tile path adds a step's sums, not its weights one by one: the single
     steps in between go without it.)"""
     monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
@@ -388,7 +388,7 @@ def test_one_projection_does_not_set_every_entry(n_c, targets, quads, monkeypatc
     (256, 1, 0, 1, False), (250, 255, 1, 1, False), (32760, 3, 0, 1, False), (32760, 260, 2, 1, False),            # few tiles, threads share a tile's word
     (65000, 300, 3, 2, False), (65500, 200, 5, 1, True), (65530, 300, 0, 2, True), (65530, 300, 4, 2, False),      # up to, and one beyond, 256 tiles of 256
     (130000, 1000, 3, 1, False), (130800, 500, 2, 1, True), (130800, 500, 0, 1, False),                           # tiles of 512 and 1024
-    (2000, 300, 0, 1, True), (9000, 300, 0, 1, False), (9000, 300, 0, 1, True), (9000, 300, 0, 2, False),          # wide entries: all, or under one projection
+    (2000, 300, 0, 1, True), (9000, 300, 0, 1, False), (9000, 300, 0, 1, True), (9000, 300, 0, 2, False),          # entries of all sizes
     (5000, 700, 0, 3, False), (5000, 700, 6, 3, False), (70000, 700, 3, 3, True), (131000, 600, 0, 3, False)])     # more than two postsynaptic models
 def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
     """Which of the kernel's instances runs depends on how many neurons a tile needs (256, 320, 512 or 1024 for a tile a compute unit), rings,
@@ -414,6 +414,72 @@ def test_every_number_of_tiles(n_a, n_b, depth, models, poisson, monkeypatch):
         compare_state(net, model, oracle, f"after {model.timestep} steps", exact=True)
 
     model, oracle, spikes = _run_chunks(net, (14, -2, 14), check)
+    assert spikes > n_a // 16
+    model.unload()
+
+
+@pytest.mark.parametrize("sizes, targets, depth, models, poisson, chosen", [
+    ((4000,), 80, 0, 1, False, (256, 8, False)), ((8000, 400), 20, 0, 1, False, (256, 8, False)), ((8000, 400), 60, 0, 1, False, (256, 4, False)),
+    ((8000, 400), 20, 0, 1, True, (256, 4, False)), ((20000,), 100, 0, 1, False, (256, 4, False)), ((60000,), 80, 0, 1, False, (256, 2, False)),
+    ((100000,), 80, 0, 1, False, (512, 2, False)), ((70000,), 150, 0, 1, False, (512, 4, False)), ((70000,), 8, 0, 3, False, (512, 4, False)),
+    ((250000,), 20, 0, 1, False, (1024, 2, False)), ((200000, 3000), 10, 0, 1, False, (1024, 4, False)), ((250000,), 20, 0, 1, True, (1024, 4, False)),
+    ((40000,), 20, 5, 1, False, (256, 4, True)), ((78000,), 8, 5, 1, False, (320, 4, True)), ((78000,), 8, 35, 2, True, (320, 4, True)),
+    ((78000,), 8, 5, 3, False, (512, 4, False)), ((120000,), 8, 5, 2, True, (512, 4, True)), ((240000,), 8, 5, 1, False, (1024, 2, False)),
+    ((6200,) * 40, 2, 0, 1, False, (0, 0, False)), ((2000,) * 40, 2, 0, 1, False, (512, 2, False))])
+def test_tiles_and_entries_by_rule(sizes, targets, depth, models, poisson, chosen):
+    """Which tile, entry and walkers a network gets: the smallest tile with a compute unit for each and room for the rings (tiles of 320 have
+    walkers only), entries by the due synapses of a row part where there are instances to choose from.  40 populations of 6,200 are 280 tiles
+    of 1,024 and step with the other plans."""
+    net = Net(name="resident_rule", dt=1.0, steps=8)
+    for p, n in enumerate(sizes):
+        net.pops.append(_pop(f"P{p}", n, 0.62, np.full(n, -60.0)))
+        if poisson and p == 0:
+            net.css.append(CurrentSource("bg", "poisson_exp", "P0", params=dict(weight=0.2, tauSyn=2.0, rate=800.0)))
+        for k in range(models):
+            net.syns.append(_projection(f"S{p}_{k}", f"P{(p + 1) % len(sizes)}", f"P{p}", sizes[(p + 1) % len(sizes)], n, targets, 0.01, 11 + k, depth, 0.2, tau=5.0 + k))
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=net.steps)
+    info = model.runner_info()
+    assert (info["resident_tile"], info["resident_quads"], info["resident_walkers"]) == chosen
+    model.unload()
+
+
+@pytest.mark.parametrize("tile, quads, rings, models, poisson, tiles", [
+    (256, 4, "all", 2, False, 3), (256, 4, "all", 1, True, 3), (320, 4, "all", 2, False, 3), (320, 4, "all", 2, True, 3),             # walkers
+    (512, 4, "all", 2, False, 3), (512, 4, "all", 2, True, 3),
+    (256, 2, "none", 2, False, 3), (256, 2, "some", 2, False, 130), (256, 4, "none", 2, False, 3), (256, 4, "some", 2, True, 3),
+    (256, 8, "none", 2, False, 3), (256, 8, "none", 2, False, 31), (256, 8, "none", 2, False, 33), (256, 8, "some", 2, False, 3),      # eight lanes an entry, or one
+    (512, 2, "none", 2, False, 3), (512, 2, "some", 1, False, 3), (512, 4, "none", 2, False, 3), (512, 4, "some", 2, False, 3), (512, 4, "none", 2, True, 3),
+    (1024, 2, "none", 2, False, 3), (1024, 2, "all", 2, False, 3), (1024, 4, "none", 1, False, 3), (1024, 4, "all", 2, False, 3), (1024, 4, "some", 2, True, 3),
+    (256, 4, "all", 3, False, 3), (512, 4, "some", 3, True, 3), (1024, 2, "none", 3, False, 3)])                                       # any number of postsynaptic models
+def test_every_instance(tile, quads, rings, models, poisson, tiles, monkeypatch):
+    """Every instance of the kernel, tile and entry size given by environment.  Row parts between none and forty synapses: inside entries of any
+    size or too long for them."""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
+    monkeypatch.setenv("GENNMI_RESIDENT_TILE", str(tile))
+    monkeypatch.setenv("GENNMI_RESIDENT_QUADS", str(quads))
+    n_a, n_b, depth = tiles * tile - 5, 200, 5
+    net = Net(name="resident_instance", dt=1.0, steps=30)
+    net.pops.append(_pop("A", n_a, 0.62, -60.0 + 9.9 * rng.uniform(5, 1, 0, n_a)))
+    net.pops.append(_pop("B", n_b, 0.45, -60.0 + 9.9 * rng.uniform(5, 2, 0, n_b)))
+    if poisson:
+        net.css.append(CurrentSource("A_bg", "poisson_exp", "A", params=dict(weight=0.2, tauSyn=2.0, rate=800.0)))
+    def ring(k):
+        return dict(depth=depth, due_share=0.3) if rings == "all" or (rings == "some" and k == 0) else dict(depth=0)
+    for k in range(models):
+        net.syns.append(_projection(f"BA{k}", "B", "A", n_b, n_a, (40, 8, 16)[k], 0.21 / (k + 1), 11 + k, tau=5.0 + k, **ring(k)))
+    net.syns.append(_projection("AB", "A", "B", n_a, n_b, 40, 0.002, 31, **ring(models)))
+    net.syns.append(_projection("BB", "B", "B", n_b, n_b, 6, 0.02, 32, tau=9.0, **ring(models)))
+    for s in net.syns:
+        s.row_length[::7] = s.row_stride // 2
+        s.row_length[::49] = 0
+
+    def check(model, oracle):
+        compare_state(net, model, oracle, f"after {model.timestep} steps", exact=True)
+
+    model, oracle, spikes = _run_chunks(net, (14, -2, 14), check)
+    info = model.runner_info()
+    assert (info["resident_tile"], info["resident_quads"], info["resident_walkers"]) == (tile, quads, rings == "all" and models <= 2 and tile <= 512)
     assert spikes > n_a // 16
     model.unload()
 
