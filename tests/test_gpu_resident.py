@@ -6,13 +6,15 @@ stages at once, tiles with many spikes in one step (side buffer), weights pushed
 Weights are one value per projection and every postsynaptic model has one incoming projection, so no fp32 sum depends
 on the order of its additions and everything — state, rings, spike queues, recordings, event counts — must be identical.
 """
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
+import torch
 
-from genn_amd import rng
-from genn_amd.genn_model import model_from_net
+from genn_amd import _abi, rng
+from genn_amd.genn_model import model_from_net, release_cached_memory
 from genn_amd.netspec import CurrentSource, Net, Pop, Syn
 from oracle.genn_cpu import OracleNet
 from parity import compare_state
@@ -556,3 +558,34 @@ def test_networks_that_do_not_fit_together(threads):
             assert np.array_equal(model.neuron_populations[p.name].vars["recordSpk"].view, oracle.record(p.name, steps)), f"recording of {p.name} differs"
         assert model.synaptic_event_count == oracle.events() > 0
         model.unload()
+
+
+def test_no_room_for_the_tables_means_another_plan(monkeypatch):
+    """A network whose segment tables take 2 GB a projection, on a card with 3 GiB free: the second table finds no room, the first goes back, and
+    the network steps with the other plans."""
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")
+    n, gib = 250000, 1 << 30
+    net = Net(name="resident_no_room", dt=1.0, steps=12)
+    net.pops.append(_pop("A", n, 0.62, -60.0 + 9.9 * rng.uniform(5, 1, 0, n)))
+    for k in range(2):
+        net.syns.append(_projection(f"AA{k}", "A", "A", n, n, 2, 0.1, 11 + k, tau=5.0 + k))
+    model = model_from_net(net)
+    release_cached_memory()
+    free, _ = torch.cuda.mem_get_info()
+    taken = C.c_void_p()
+    _abi.check(_abi.load().gennmi_malloc(C.byref(taken), free - 3 * gib))
+    try:
+        model.load(num_recording_timesteps=net.steps)
+        assert not model.runner_info()["resident_plan"]
+        release_cached_memory()
+        assert torch.cuda.mem_get_info()[0] > 2.5 * gib
+    finally:
+        _abi.check(_abi.load().gennmi_free(taken))
+        release_cached_memory()
+    oracle = OracleNet(net, num_recording_timesteps=net.steps)
+    model.run(net.steps)
+    oracle.run(net.steps)
+    model.synchronize()
+    compare_state(net, model, oracle, "with the other plans", exact=True)
+    assert model.synaptic_event_count == oracle.events() > 0
+    model.unload()
