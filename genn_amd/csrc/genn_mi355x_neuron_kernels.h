@@ -6,7 +6,7 @@ namespace
 {
 // State a step leaves behind goes through the L2 to memory at once: what is dirty when a kernel ends is written back then, and the next
 // kernel waits for it.  us a step, written back at the end / through: 10^6 Izhikevich neurons 20.8 / 20.1, the microcircuit at 35 % with PoissonExp
-// sources, a launch a step, 7.5 / 7.25, 100,000 neurons with plastic synapses 20.4 / 20.0, 300,000 LIF neurons 13.1 / 13.0.
+// sources, a launch a step, 7.5 / 7.25, 100,000 neurons with plastic synapses 20.4 / 20.0; 300,000 LIF neurons 13.1 / 13.0, no more than two runs differ.
 template<typename T>
 __device__ __forceinline__ void storeThrough(GLOBAL_AS T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 

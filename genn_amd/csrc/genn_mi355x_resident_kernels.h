@@ -12,8 +12,8 @@
 // state -> spike count -> spike ids -> rows -> ~10^5 scattered fp32 atomics that retire at ~20 G/s on the memory
 // side.  Here one work-group owns a tile of neurons for a whole run: their state stays in registers, their
 // postsynaptic input (inSyn) and their slice of every dendritic-delay ring stay in LDS, and the only thing
-// work-groups exchange is each step's spikes — one 64-bit word per tile (sequence number, count, and the id
-// itself when a single neuron fired; longer lists go through a side buffer).  Every tile reads the words of
+// work-groups exchange is each step's spikes — one 64-bit word per tile (sequence number, count, and up to three
+// ids; longer lists go through a side buffer).  Every tile reads the words of
 // all tiles, looks up which part of each spiking row targets its own neurons (a per-(row, tile) segment table
 // built once; rows are sorted by target), and adds those synapses into its LDS ring: no global atomics, no
 // global read-modify-write of the ring, no kernel boundary.  The words are double-buffered by step parity: a
@@ -21,13 +21,20 @@
 // it can publish its own word of step s+1.
 //
 // The wait for the other tiles' words is bounded (c_spinLimit polls) and also watches the error flag, so a launch
-// whose work-groups are not all resident ends with an error instead of hanging.
+// whose work-groups are not all resident ends with an error instead of hanging.  Launches of several runners that do not fit on the
+// chip together take turns (residentRoom() on the host).
 // ------------------------------------------------------------------------------------------------
 // Neurons of a tile.  A network takes the smallest of these with which its tiles have a compute unit each: work-groups that share one take twice
 // as long around their loop, and every tile waits for the slowest; and with T x T neurons at most each of a tile's T threads has
 // one other tile's word to look for.  us a step with tiles of 256, two and four to a compute unit / with these: the full microcircuit 4.4 / 4.1
 // (320), 100,000 x 80 5.9 / 5.0 (512), 180,000 x 100 9.0 / 5.7 and 250,000 x 200 10.5 / 4.9 (1024).  Larger ones than needed do not pay: 4,000 x 80
 // to 40,000 x 80 within 3 % with 512, up to 20 % more with 1024; the microcircuit at half size 2.8 -> 3.3 with 512.
+// Tiles of 320 are for networks with walkers, 65,500 to 82,000 neurons.  us a step with tiles of 256 that share units / 320 / 512: with row parts of eight
+// synapses and more the microcircuit with PoissonExp sources at full size - / 4.00 / 5.03 and at 0.86 - / 3.65 / 4.47, 8 x 8,600 neurons x 800 - / 11.8 / 14.0,
+// 2 x 40,000 x 1,000 - / 27.3 / 28.1; with a few, 512 would be the better one: 4 x 19,000 x 200 9.7 / 6.2 / 5.4, 4 x 19,000 x 40 6.8 / 4.4 / 3.9,
+// 8 x 8,600 x 100 6.1 / 4.4 / 3.9.
+// Some networks of many populations have no tile that fits, since every population is rounded up to whole tiles: 40 x 6,200 neurons are 280 tiles of
+// 1024.  They step with the other plans, where tiles of 256, four to a unit, once took them: us a step then / now, 80 targets each 11.0 / 11.4, 800 targets 34 / 24.
 constexpr uint32_t RES_TILES[] = {256, 320, 512, 1024};
 constexpr uint32_t RES_MAX_TILE = 1024;
 constexpr uint32_t RES_MAX_PROJ = 16;        // projections into one population
@@ -39,7 +46,8 @@ constexpr uint32_t RES_PAIR_CAP = 1024;      // (spike, projection) pairs a tile
 // and every tile waits for the one that does.  us a step of a balanced network, without / with synapses inside entries: 100,000 neurons x
 // 80 targets 8.1 / 6.7, 40,000 x 80 4.7 / 4.3 (2 quads), 12,000 x 100 4.19 / 4.00, 4,000 x 80 3.79 / 3.62 (8, which one lane read then), and 2.85 -> 2.47
 // since eight lanes read an entry of 8, a quad each; with 2 / with what the host's rule takes now: 4,000 x 80 2.66 / 2.24 (8), 20,000 x 100
-// 3.13 / 2.43 and 40,000 x 80 3.52 / 3.26 (4); the microcircuit's rings have few that are due, 4.22 with 2 and with 4.
+// 3.13 / 2.43 and 40,000 x 80 3.52 / 3.26 (4).  Networks with walkers have entries of 4 and no others (the microcircuit, whose rings have few that are
+// due, took 4.22 with 2 and with 4), and so have most with PoissonExp sources or more than two postsynaptic models: the host's table of instances.
 constexpr uint32_t residentInside(uint32_t quads) { return 3 * quads - 2; }
 constexpr uint32_t RES_MAX_QUADS = 8, RES_COUNT_SHIFT = 30;       // a quad's last word: targets, 10 bits each, and the number of its synapses
 constexpr uint32_t RES_SEG_OVERFLOW = 1u << 24, RES_SEG_NO_DELAY = 1u << 25;
@@ -54,7 +62,7 @@ constexpr uint32_t RES_REPLICAS = 8;         // copies of the word array, one pe
 struct ResProj
 {
     const u32x2 *packed;                // one record per (padded) synapse, see residentPackKernel
-    const u32x4 *seg;                   // [numSrc * tilesInGroup][2]: the row's part inside a tile, see residentSegKernel
+    const u32x4 *seg;                   // [numSrc * tilesInGroup][QUADS]: the row's part inside a tile, see residentSegKernel
     uint32_t D;                         // ring depth; 0 = no dendritic delay, events add to inSyn
     uint32_t lds;                       // float offset of the ring (D x tile size, slot-major) or inSyn row in the tile's LDS
     uint32_t srcGroup;
@@ -361,8 +369,10 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     }
     const bool watching = main && watchTile < numTiles;
     // The list is shared out between the wavefronts that watch: a pair's place depends on the spikes alone and not on when their words
-    // arrive, and so does the order in which the walk adds the synapses of an exchange (out of the order of arrival, two runs of the full
-    // microcircuit parted at every neuron that comes within a rounding of its threshold).
+    // arrive, so a wavefront that walks adds the synapses of an exchange in the same order every time.  Between wavefronts there is no order, nor for
+    // the due synapses, which the thread that sees a word adds: sums that round differ from run to run.  (Where places followed the words' arrival,
+    // two runs of the full microcircuit parted at every neuron that comes within a rounding of its threshold.  As it is, 24 runs of 10,000 steps, four
+    // of each of six seeds, had the same rasters and membranes that differ by 1.5e-5 mV.)
     const uint32_t watchWaves = (perTile == 1) ? (numTiles + WAVE - 1) / WAVE : MAIN, listCap = RES_PAIR_CAP / watchWaves;
     const uint32_t rowQuads = QUADS * tilesInGroup;     // entries of consecutive rows, in quads
     const uint32_t watchFirst = watching ? tiles[watchTile].first : 0u;
@@ -556,9 +566,9 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
     };
 
     // Walks the row segments of the listed pairs: a group of lanes per pair, a lane taking every n-th synapse of its
-    // pair's segment, eight of them per trip to memory.  Sixteen lanes per pair when the pairs are few (a quiet step: one
-    // trip covers 128 synapses of each of a wavefront's four pairs), four when they are many (a synchronous burst).
-    // (Segments of a tile are short — a row's share of 256 targets — so lanes idle in the longest segment's last trip
+    // pair's segment, four of them per trip to memory.  Sixteen lanes per pair when the pairs are few (a quiet step: one
+    // trip covers 64 synapses of each of a wavefront's four pairs), four when they are many (a synchronous burst).
+    // (Segments are short — a row's share of a tile's targets — so lanes idle in the longest segment's last trip
     // cost less than finding, for every lane, its place in a list of all the segments' synapses would.)
     // A synapse is "due" when it lands in the slot read this step (delay a multiple of the ring depth, or no ring).
     // PASS_ALL adds every synapse, PASS_LATER those not due, PASS_DUE the due ones; `flaggedOnly` restricts the walk to
