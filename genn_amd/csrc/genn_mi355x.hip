@@ -1323,12 +1323,27 @@ static int refreshTables(gennmi_runner *r)
 // Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
 // plain population it feeds, so that no spike ever comes back.
 constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input over the steps of a launch
-constexpr size_t AHEAD_MAX_LDS = 64 * 1024;
+// A work-group of the convolution takes no more output rows than leave two of them to a compute unit; a single row may take a little more.
+constexpr size_t AHEAD_ROWS_LDS = 64 * 1024, AHEAD_MAX_LDS = 82 * 1024;
 // Runs (and remainders of runs) shorter than this are stepped one by one: a pass costs a good part of a pass of 32 steps however few it is given.  us
 // at once / one by one for 5 and for 8 steps: Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, at 20 %, 2.5 % and 0.25 % activity 239 / 174 and
 // 259 / 273, 125 / 152 and 144 / 238, 93 / 146 and 98 / 228; 40x40x16 -> 40x40x4 5x5, batch 16, at 0.25 % 185 / 131 and 189 / 204; DENSE 8192 x 8192
 // (5 %; 4 and 8 steps) 35 / 45 and 43 / 85, the same with batch 16 195 / 175 and 231 / 346.
 constexpr uint32_t AHEAD_MIN_STEPS = 8;
+// (the kernels of the target's neuron model and postsynaptic model)
+static auto aheadConvInstance(const gennmi_neuron_update_group_t &g)
+{
+    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
+    const bool lif = (g.model == LIF), exponential = (g.psm[0].kind == EXP);
+    return lif ? (exponential ? aheadConvKernel<LIF, EXP> : aheadConvKernel<LIF, DELTA>) : (exponential ? aheadConvKernel<IZH, EXP> : aheadConvKernel<IZH, DELTA>);
+}
+static auto aheadNeuronInstance(const gennmi_neuron_update_group_t &g)
+{
+    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
+    const bool lif = (g.model == LIF), exponential = (g.psm[0].kind == EXP);
+    return lif ? (exponential ? aheadNeuronKernel<LIF, EXP> : aheadNeuronKernel<LIF, DELTA>) : (exponential ? aheadNeuronKernel<IZH, EXP> : aheadNeuronKernel<IZH, DELTA>);
+}
+
 static int setupAhead(gennmi_runner *r, uint32_t numCU)
 {
     const char *env = getenv("GENNMI_AHEAD");
@@ -1346,17 +1361,20 @@ static int setupAhead(gennmi_runner *r, uint32_t numCU)
     if(conv) {
         const int32_t *c = p.conv;
         AheadConv &C = r->aheadConv;
-        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 0u, 1u};
-        C.rowPitch = (uint32_t)(c[6] - 1 + c[1]) * (uint32_t)c[4] + 1;      // (an odd number of taps is read as pairs: one word beyond)
-        C.pairsPerRow = ((uint32_t)(c[1] * c[4]) + 1) / 2;
+        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 1u};
+        C.rowPitch = (uint32_t)(c[6] - 1 + c[1]) * (uint32_t)c[4];
+        const uint32_t inputs = (uint32_t)(c[0] * c[1] * c[4]);
         // as many output rows per work-group as leave four work-groups to a compute unit
         const uint64_t rowsInAll = (uint64_t)c[5] * r->batch * (((uint32_t)c[7] + 31) / 32);
         C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (4 * numCU)));
         for(;; C.rowsPerBlock--) {
-            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)c[0] * 2 * C.pairsPerRow * 32) * sizeof(uint32_t);
-            if(r->aheadConvBytes <= AHEAD_MAX_LDS || C.rowsPerBlock == 1) { break; }
+            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)inputs * 32 + (size_t)(inputs + 1) / 2 + (size_t)(BLOCK / WAVE) * 2 * aheadConvList(inputs)) * sizeof(uint32_t);
+            if(r->aheadConvBytes <= AHEAD_ROWS_LDS || C.rowsPerBlock == 1) { break; }
         }
         if(r->aheadConvBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
+        if(r->aheadConvBytes > 48 * 1024) {
+            HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(aheadConvInstance(g)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)r->aheadConvBytes));
+        }
     }
     else if((size_t)r->batch * AHEAD_WORD * p.numTrgNeurons * sizeof(float) > AHEAD_MAX_SPACE || (uint64_t)r->batch * (AHEAD_MAX_STEPS / AHEAD_WORD) > 65535) { return GENNMI_OK; }
     if(!src.spikeBitmap) {
@@ -1413,12 +1431,9 @@ static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned l
     uint8_t *input = r->aheadSpace + wordBytes + bitBytes;
     const NeuronGroupDev *target = r->dAhead + 1, &src = r->neuron[r->aheadSource];
     const AheadArgs a{timestep, r->epoch, steps, B, (uint32_t)std::max<unsigned long long>(1, numRecordingTimesteps), r->dt};
-    // (the kernels of the target's neuron model and postsynaptic model)
     const gennmi_neuron_update_group_t &g = r->neuron[r->aheadTarget].g;
-    const bool lif = (g.model == GENNMI_NEURON_LIF), exponential = (g.psm[0].kind == GENNMI_PSM_EXPCURR);
-    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
-    const auto convKernel = lif ? (exponential ? aheadConvKernel<LIF, EXP> : aheadConvKernel<LIF, DELTA>) : (exponential ? aheadConvKernel<IZH, EXP> : aheadConvKernel<IZH, DELTA>);
-    const auto neuronKernel = lif ? (exponential ? aheadNeuronKernel<LIF, EXP> : aheadNeuronKernel<LIF, DELTA>) : (exponential ? aheadNeuronKernel<IZH, EXP> : aheadNeuronKernel<IZH, DELTA>);
+    const auto convKernel = aheadConvInstance(g);
+    const auto neuronKernel = aheadNeuronInstance(g);
     aheadSourceKernel<<<dim3((numSrc + BLOCK - 1) / BLOCK, B), dim3(BLOCK), 0, r->stream>>>(r->dAhead, a, r->aheadConv, numTrg, words, r->dEvents);
     if(conv) {
         const AheadConv &C = r->aheadConv;

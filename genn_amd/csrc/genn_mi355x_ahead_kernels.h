@@ -14,7 +14,7 @@
 // What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
 //
 // run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 205 us;
-// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 1040 us, of which 500 move 26 MB between host and device.
+// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 940 us, of which 500 move 26 MB between host and device.
 #pragma once
 
 namespace
@@ -32,9 +32,12 @@ struct AheadArgs
 struct AheadConv
 {
     int32_t kh, kw, ih, iw, ic, oh, ow, oc, PH, PW;
-    uint32_t rowsPerBlock, rowPitch, pairsPerRow;       // patch row in words; (tap, channel) pairs of one kernel row
+    uint32_t rowsPerBlock, rowPitch;                    // patch row in words
     uint32_t isConv;
 };
+
+// entries of a pixel's list of active inputs: all of them and what fills the last pair
+__host__ __device__ constexpr uint32_t aheadConvList(uint32_t inputs) { return inputs + 1u; }
 
 __device__ __forceinline__ size_t aheadRecordingRow(const AheadArgs &A, uint32_t step) { return (size_t)((A.timestep + step) % A.recordingRows); }
 
@@ -367,30 +370,40 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
 }
 
 // ---- 2b, 3b. Conv2D and its neurons, up to 32 steps.  A work-group owns some output rows of one batch and 32 output channels: the
-// words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes four output pixels at a
-// time: the rows of its four products are timesteps, the inner dimension the (tap, channel) pairs — consecutive words of the patch
-// for one kernel row — and a kernel weight read once serves all four.  The products stay in registers; one swap of half-wavefronts
-// per register pair puts a neuron's 32 inputs into one lane, which takes the neuron through the steps and leaves its spikes as one word.
-// The products are those of the step kernel, v_mfma_f32_32x32x2_f32 over taps and channels in the same order, so that a layer's sums are the
-// same bits whether its steps are taken at once or one by one (with weights in three bfloat16 parts, as in aheadDenseKernel, the kernel
-// takes 88 us instead of 204 and one spike in 10^6 moves by a step).  Bound by the fp32 matrix rate: 64x64x16 -> 64x64x32 3x3, batch 16 takes
-// 204 us for 32 steps and 154 for 18; at that rate the products take 123 without the silent pairs left out.
+// words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes two output pixels at a
+// time: the rows of its two products are timesteps, the inner dimension the pixel's (tap, channel) inputs that have a spike in any of the
+// steps, packed into a list in LDS in their order (45 % of them are silent at 2.5 % activity and 32 steps).  The products stay in registers; one
+// swap of half-wavefronts per register pair puts a neuron's 32 inputs into one lane, which takes the neuron through the steps and leaves
+// its spikes as one word.
+// The products are those of the step kernel, v_mfma_f32_32x32x2_f32 over taps and channels in the same order, which adds one input after
+// the other: leaving out inputs whose bits are all 0 changes no bit of a sum, whichever two then share an instruction, so a layer's sums are
+// the same bits whether its steps are taken at once or one by one.  (With weights in three bfloat16 parts, as in aheadDenseKernel, one spike in
+// 10^6 moves by a step.)
+// us for 32 steps of 64x64x16 -> 64x64x32 3x3, batch 16, at 2.5 %: 198 with pairs left out that are silent together and a weight read once for
+// four pixels, 183 packed with a branch around each product (the sixteen sums are copied wherever the paths meet), 144 packed and straight.
+// Of that the matrix cores are busy 60 and the vector units 64 (counters), the neurons' steps half of these.  run() with all its launches, packed
+// against paired, other shapes and rates: 40x37x16 -> 4 5x5 batch 16, 32 steps, 0.5 / 5 / 40 / 100 % 124 / 248 / 385 / 422 against 244 / 398 / 481 / 507; 24x24x16 -> 32
+// 5x5, 45 steps 96 / 165 / 270 / 298 against 189 / 283 / 358 / 375; the shape above, 50 steps 179 / 318 / 549 / 746 against 243 / 416 / 586 / 771.
 template<uint32_t MODEL, uint32_t PSM>
 __global__ __launch_bounds__(BLOCK, 4)
 void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
                      const float * __restrict__ kernel, uint32_t *spikeWords)
 {
-    extern __shared__ uint32_t shAhead[];
+    extern __shared__ __align__(16) uint32_t shAhead[];
     const gennmi_neuron_update_group_t &g = target->g;
     const uint32_t n = g.numNeurons, batch = blockIdx.y, oc = (uint32_t)C.oc, ow = (uint32_t)C.ow;
     const uint32_t lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), half = lane >> 5, col = lane & 31;
     const uint32_t y0 = blockIdx.x * C.rowsPerBlock, rows = min(C.rowsPerBlock, (uint32_t)C.oh - y0), pixels = rows * ow;
     const uint32_t o = blockIdx.z * 32 + col;
     const uint32_t steps = min(A.steps - wordBlock * AHEAD_WORD, AHEAD_WORD);
-    const AheadNeuron<MODEL, PSM> neuron(g, A.dt);
-    const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), pairs = C.pairsPerRow;
-    uint32_t *patch = shAhead;
-    float *kern = reinterpret_cast<float*>(shAhead + (C.rowsPerBlock + (uint32_t)C.kh - 1) * rowPitch);        // [kh][2 * pairs][32]
+    AheadNeuron<MODEL, PSM> neuron(g, A.dt);
+    asm volatile("" : "+v"(neuron.constants.p[5]), "+v"(neuron.constants.p[6]));       // (selected between in every step: from scalar registers that is a copy first)
+    const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), inputs = (uint32_t)C.kh * rowWords;
+    const uint32_t listed = aheadConvList(inputs);
+    uint2 *list = reinterpret_cast<uint2*>(shAhead) + wave * listed;                                // (word, byte of its weights) of a pixel's active inputs
+    float *kern = reinterpret_cast<float*>(reinterpret_cast<uint2*>(shAhead) + (BLOCK / WAVE) * listed);       // [input][32]
+    uint16_t *place = reinterpret_cast<uint16_t*>(kern + inputs * 32);                              // [input] its word behind the pixel's first
+    uint32_t *patch = reinterpret_cast<uint32_t*>(kern + inputs * 32) + (inputs + 1) / 2;
     // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
     GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
     const int inRowWords = C.iw * C.ic;
@@ -402,104 +415,93 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
         }
     }
     bool nonFinite = false;
-    for(uint32_t e = threadIdx.x; e < (uint32_t)C.kh * 2 * pairs * 32; e += BLOCK) {
-        const uint32_t k = e / 32, a = k / (2 * pairs), c = k - a * 2 * pairs, oo = blockIdx.z * 32 + (e & 31);
-        float weight = (c < rowWords && oo < oc) ? asGlobal(kernel)[((size_t)a * rowWords + c) * oc + oo] : 0.0f;
+    for(uint32_t e = threadIdx.x; e < inputs * 32; e += BLOCK) {
+        const uint32_t k = e / 32, oo = blockIdx.z * 32 + (e & 31);
+        float weight = (oo < oc) ? asGlobal(kernel)[(size_t)k * oc + oo] : 0.0f;
         if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
         kern[e] = weight;
     }
+    for(uint32_t k = threadIdx.x; k < inputs; k += BLOCK) { place[k] = (uint16_t)(k / rowWords * rowPitch + k % rowWords); }
     nonFinite = __syncthreads_or(nonFinite);
-    const uint32_t *patchOfHalf = patch + half;
 
     GLOBAL_AS float *var0 = asGlobal(g.var0) + (size_t)batch * n, *var1 = asGlobal(g.var1) + (size_t)batch * n, *outPost = asGlobal(g.psm[0].outPost) + (size_t)batch * n;
     GLOBAL_AS uint32_t *spikes = asGlobal(spikeWords) + (size_t)batch * n;
-    for(uint32_t first = wave * 4; first < pixels; first += (BLOCK / WAVE) * 4) {
-        uint32_t base[4];
+    const char *weights = reinterpret_cast<const char*>(kern + col);
+    const uint2 *entries = list + half;
+    for(uint32_t first = wave * 2; first < pixels; first += (BLOCK / WAVE) * 2) {
+        // state of the lane's neuron (pixel first + half, channel o), asked for ahead of the products
+        const uint32_t own = first + half;
+        const bool valid = (own < pixels && o < oc);
+        const size_t at = valid ? ((size_t)y0 * ow + own) * oc + o : 0;
+        float v0 = var0[at], v1 = var1[at], lin = outPost[at];
+        uint32_t base[2];
+        f32x16 acc[2];
         #pragma unroll
-        for(uint32_t j = 0; j < 4; j++) {
+        for(int j = 0; j < 2; j++) {
             const uint32_t p = min(first + j, pixels - 1), r = p / ow;
             base[j] = r * rowPitch + (p - r * ow) * (uint32_t)C.ic;
-        }
-        f32x16 acc[4];
-        #pragma unroll
-        for(int j = 0; j < 4; j++) { acc[j] = f32x16{}; }
-        const float *weight = kern + half * 32 + col;
-        for(uint32_t a = 0; a < (uint32_t)C.kh; a++) {
-            // four pairs a round: their reads from LDS are issued together, ahead of the sixteen products
-            uint32_t c = 0;
-            for(; c + 4 <= pairs; c += 4) {
-                float b[4]; uint32_t bits[4][4];
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) {
-                    b[u] = weight[(c + u) * 64];
-                    #pragma unroll
-                    for(int j = 0; j < 4; j++) { bits[u][j] = patchOfHalf[base[j] + 2 * (c + u)]; }
-                }
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) {
-                    #pragma unroll
-                    for(int j = 0; j < 4; j++) {
-                        // (two inputs silent in all steps add nothing: a fifth of the pairs at 2.5 % and 32 steps, two fifths at 18)
-                        if(__ballot(bits[u][j] != 0)) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(bits[u][j], col), b[u], acc[j], 0, 0, 0); }
-                    }
-                }
+            acc[j] = f32x16{};
+            // the inputs that have a spike in any of the steps, in their order
+            uint32_t count = 0;
+            for(uint32_t k0 = 0; k0 < inputs; k0 += WAVE) {
+                const uint32_t k = k0 + lane;
+                const uint32_t behind = place[min(k, inputs - 1)], there = patch[base[j] + behind], word = (k < inputs) ? there : 0u;
+                const unsigned long long active = __ballot(word != 0u);
+                if(word) { list[count + __popcll(active & ((1ull << lane) - 1ull))] = make_uint2(word, k * 128); }
+                count += __popcll(active);
             }
-            for(; c < pairs; c++) {
-                const float b = weight[c * 64];
+            if(lane == 0) { list[count] = make_uint2(0u, 0u); }         // (fills the last pair)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            // (no branch inside a round: the compiler copies the sixteen sums where paths with and without a product meet)
+            uint32_t m = 0;
+            for(; m + 8 <= count; m += 8) {
+                uint2 e[4]; float w[4];
                 #pragma unroll
-                for(int j = 0; j < 4; j++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(patchOfHalf[base[j] + 2 * c], col), b, acc[j], 0, 0, 0); }
+                for(uint32_t u = 0; u < 4; u++) { e[u] = entries[m + 2 * u]; }
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) { w[u] = *reinterpret_cast<const float*>(weights + e[u].y); }
+                #pragma unroll
+                for(uint32_t u = 0; u < 4; u++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e[u].x, col), w[u], acc[j], 0, 0, 0); }
             }
-            weight += pairs * 64;
-            #pragma unroll
-            for(int j = 0; j < 4; j++) { base[j] += rowPitch; }
+            for(; m < count; m += 2) {
+                const uint2 e = entries[m];
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e.x, col), *reinterpret_cast<const float*>(weights + e.y), acc[j], 0, 0, 0);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
         if(nonFinite) {
             // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
-            for(uint32_t k = 0; k < (uint32_t)C.kh * rowWords; k++) {
+            for(uint32_t k = 0; k < inputs; k++) {
                 const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
                 if(aheadFinite(b)) { continue; }
-                const uint32_t a = k / rowWords;
                 #pragma unroll
-                for(int j = 0; j < 4; j++) {
-                    const uint32_t bits = patch[base[j] - ((uint32_t)C.kh - a) * rowPitch + (k - a * rowWords)];
+                for(int j = 0; j < 2; j++) {
+                    const uint32_t bits = patch[base[j] + place[k]];
                     #pragma unroll
                     for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
                 }
             }
         }
-        // state of the lane's two neurons (pixels first + half and first + 2 + half, channel o), asked for behind the products: held across them, it and its addresses do not fit
-        // the registers
-        bool valid[2]; size_t at[2]; float v0[2], v1[2], lin[2];
+        // lower half: all steps of the first pixel, upper half: of the second
+        float x[16], y[16];
         #pragma unroll
-        for(uint32_t m = 0; m < 2; m++) {
-            const uint32_t p = first + 2 * m + half;
-            valid[m] = (p < pixels && o < oc);
-            at[m] = valid[m] ? ((size_t)y0 * ow + p) * oc + o : 0;
-            v0[m] = var0[at[m]]; v1[m] = var1[at[m]]; lin[m] = outPost[at[m]];
+        for(int v = 0; v < 16; v++) {
+            const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
+            x[v] = __uint_as_float(swapped[0]); y[v] = __uint_as_float(swapped[1]);
         }
+        uint32_t fired = 0;
         #pragma unroll
-        for(int m = 0; m < 2; m++) {
-            // lower half: all steps of the first pixel of the pair, upper half: of the second
-            float x[16], y[16];
-            #pragma unroll
-            for(int v = 0; v < 16; v++) {
-                const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[2 * m][v]), __float_as_uint(acc[2 * m + 1][v]), false, false);
-                x[v] = __uint_as_float(swapped[0]); y[v] = __uint_as_float(swapped[1]);
+        for(uint32_t t = 0; t < AHEAD_WORD; t++) {
+            // (kept a comparison and a branch: computed ahead for all steps, the conditions are 32 masks, spilled)
+            uint32_t end = steps;
+            asm volatile("" : "+s"(end));
+            if(t < end) {
+                asm volatile("" : "+v"(lin));
+                const float input = (t & 4) ? y[4 * (t / 8) + (t & 3)] : x[4 * (t / 8) + (t & 3)];
+                fired |= neuron.step(input, lin, v0, v1) ? 1u << t : 0u;
             }
-            uint32_t fired = 0;
-            #pragma unroll
-            for(uint32_t t = 0; t < AHEAD_WORD; t++) {
-                // (kept a comparison and a branch: computed ahead for all steps, the conditions are 32 masks, spilled)
-                uint32_t end = steps;
-                asm volatile("" : "+s"(end));
-                if(t < end) {
-                    asm volatile("" : "+v"(lin[m]));
-                    const float input = (t & 4) ? y[4 * (t / 8) + (t & 3)] : x[4 * (t / 8) + (t & 3)];
-                    fired |= neuron.step(input, lin[m], v0[m], v1[m]) ? 1u << t : 0u;
-                }
-            }
-            if(valid[m]) { var0[at[m]] = v0[m]; var1[at[m]] = v1[m]; outPost[at[m]] = lin[m]; spikes[at[m]] = fired; }
         }
+        if(valid) { var0[at] = v0; var1[at] = v1; outPost[at] = lin; spikes[at] = fired; }
     }
 }
 

@@ -203,3 +203,31 @@ def test_a_written_queue_that_names_a_neuron_twice(monkeypatch):
         got.append((model.neuron_populations["Out"].vars["V"].pull_from_device().copy(), model.synaptic_event_count))
         model.unload()
     assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+
+
+# few and many inputs a pixel (one round of 64, seven), an odd number of them, more LDS than 64 KiB, channels beyond a product's 32
+@pytest.mark.parametrize("shape,rate", [((8, 8, 16, 32, 3), 400.0), ((6, 9, 16, 8, 5), 250.0), ((4, 9, 17, 3, 5), 100.0), ((5, 7, 8, 33, 3), 300.0), ((5, 7, 3, 40, 3), 1000.0), ((9, 4, 13, 5, 2), 400.0)])
+def test_convolutions_sum_to_the_same_bits_at_once_and_step_by_step(shape, rate, monkeypatch):
+    """Weights of full precision: which inputs share a product must not change a bit.  (At these rates every step with spikes is one for the
+    matrix cores when taken by itself; a kernel that its step kernel has no LDS for has weights whose sums are exact in any order.)"""
+    h, w, ic, oc, k = shape
+    steps = 41
+    net = configs.conv_toeplitz(h=h, w=w, ic=ic, oc=oc, k=k, steps=steps, w_sd=1.0 / k, max_rate=rate, ioffset=0.3)
+    exact = k * k * ic >= 400
+    if exact:
+        net.syns[0].g = (np.rint(net.syns[0].g * 256.0) / 256.0).astype(np.float32)
+        net.syns[0].psm = "deltacurr"
+    states = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1") and (exact or model.runner_info()["conv_on_matrix_cores"])
+        model.run(steps)
+        model.pull_recording_buffers_from_device()
+        out, layer = model.neuron_populations["Out"], list(model.synapse_populations.values())[0]
+        states.append([out.vars["recordSpk"].view.copy(), out.vars["V"].pull_from_device().copy(), layer.vars["outPost"].pull_from_device().copy(), model.synaptic_event_count])
+        model.unload()
+    assert states[0][3] == states[1][3] > 0 and np.any(states[0][0])
+    for a, b in zip(states[0][:3], states[1][:3]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
