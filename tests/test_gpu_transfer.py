@@ -73,3 +73,19 @@ def test_spike_queues_of_every_length(model, n, batch, slots):
                 assert np.array_equal(got[b, :counts[b]], spk.view.reshape(batch, slots, n)[b, slot, :counts[b]])
                 assert np.all(got[b, counts[b]:] == 0xFFFFFFFF)
     _abi.check(lib.gennmi_runner_destroy(runner))
+
+
+# a work-group's 4,096 floats, 256 work-groups' and what is copied by up to 512 of them; ends and beginnings off 16 bytes
+@pytest.mark.parametrize("count", [1, 3, 4095, 4097, 256 * 4096 + 1, (1 << 22), (1 << 22) + 7])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_copies_on_the_device_touch_what_they_name(model, count, offset):
+    lib = _abi.load()
+    a, b = model._alloc(count + 8, np.float32), model._alloc(count + 8, np.float32)
+    a.view[:] = np.arange(count + 8)
+    a.push_to_device()
+    b.view[:] = -1.0
+    b.push_to_device()
+    _abi.check(lib.gennmi_runner_copy_f32(model._runner, b.ptr + 4 * offset, a.ptr + 4, count))
+    got = b.pull_from_device()
+    assert np.array_equal(got[offset:offset + count], np.arange(1, count + 1, dtype=np.float32))
+    assert np.all(got[:offset] == -1.0) and np.all(got[offset + count:] == -1.0)
