@@ -309,3 +309,31 @@ def test_column_view_of_columns_longer_than_the_lds_sort():
     assert np.array_equal(got_length, [len(c) for c in want])
     for j in range(num_trg):
         assert np.array_equal(got[j, :len(want[j])], np.asarray(want[j], dtype=np.uint32)), f"column {j}"
+
+
+# 64 blocks of a population and one more, 2,048 and one more, with one and with four neurons a lane: where the way to a block's place in the queue changes
+@pytest.mark.parametrize("per_lane", [1, 4])
+@pytest.mark.parametrize("blocks", [64, 65, 2048, 2049])
+def test_spike_queue_is_ascending_and_complete_at_any_number_of_blocks(blocks, per_lane, monkeypatch):
+    monkeypatch.setenv("GENNMI_NEURON_BULK", "4" if per_lane == 4 else "0")
+    n = (blocks - 1) * 256 * per_lane + 3
+    model = GeNNModel("float", "queues", dt=1.0)
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.55, TauRefrac=2.0)
+    rng = np.random.default_rng(blocks)
+    v = rng.uniform(-52.0, -49.9, n).astype(np.float32)
+    v[n // 3:n // 2] = -60.0            # (blocks without spikes)
+    pop = model.add_neuron_population("N", n, "LIF", lif, {"V": v, "RefracTime": 0.0})
+    pop.spike_recording_enabled = True
+    model.build()
+    model.load(num_recording_timesteps=4)
+    assert model.runner_info()["neuron_blocks"] == blocks
+    queues = []
+    for _ in range(4):
+        model.step_time()
+        queues.append(pop.current_spikes[0])
+    model.pull_recording_buffers_from_device()
+    bits = np.unpackbits(pop.vars["recordSpk"].view.view(np.uint8).reshape(4, -1), axis=1, bitorder="little")[:, :n]
+    assert sum(len(q) for q in queues) > n // 10
+    for step, queue in enumerate(queues):
+        assert np.array_equal(queue, np.nonzero(bits[step])[0])
+    model.unload()
