@@ -521,6 +521,7 @@ __device__ __forceinline__ unsigned long long tileRecordLoop(const TileGroupDev 
     return events;
 }
 
+constexpr uint32_t TILE_SEGMENTS = 2;                   // spikes whose segments a sub-group of the tile kernel takes together
 constexpr uint32_t TILE_NO_CHANGE = 0x7FC0DEADu;        // (a NaN no computation makes) the presynaptic-spike rule leaves this target's synapses alone
 __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float *shTile, const StepArgs &args, float dt, unsigned long long *eventCounter)
 {
@@ -586,9 +587,6 @@ __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float
         if(paired && ((bits >> (idPost & 31u)) & 1u)) { nw = learnPostOnSynapseWith(G.learn, g, rowST, rowTrace, nw, t, dt); }
         return nw;
     };
-    auto depress = [&](uint32_t idPre, uint32_t idPost, float w) -> float {
-        return depressWith(idPre, idPost, w, trgST[idPost], additive ? 0.0f : postTrace[idPost], paired ? trgBitmap[idPost >> 5] : 0u);
-    };
     // What the presynaptic-spike rule takes off a synapse depends on its target alone (times, trace and constants): in a busy step a block works
     // it out once per target of its tile and keeps it in LDS behind the tile, with the targets' bits of the spike bitmap.  Three gathers
     // over the chip's memory per synapse, a cache line each, are what a burst otherwise spends its time on (and, under the
@@ -641,47 +639,87 @@ __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float
     const uint32_t stride = perBlock * G.numSplits;
     const uint32_t lastSrc = g.numSrcNeurons - 1;
     unsigned long long events = 0;
-    // software pipeline over this sub-group's spikes: the spike id is fetched two iterations ahead and the
-    // segment boundaries one iteration ahead (spk holds numSrcNeurons entries, so clamped indices are readable)
-    uint32_t s = G.split * perBlock + threadIdx.x / L;
-    uint32_t id0 = spk[min(s, lastSrc)], id1 = spk[min(s + stride, lastSrc)];
-    size_t o0 = (size_t)id0 * (G.numTiles + 1) + G.tile;
-    uint32_t a0 = off[o0], b0 = off[o0 + 1];
+    // TILE_SEGMENTS spikes of a sub-group at a time: their segments' synapses are asked for together.  The spike ids are fetched two rounds ahead
+    // and the segments' boundaries one (spk holds numSrcNeurons entries, so clamped indices are readable).
+    const size_t total = (size_t)g.numSrcNeurons * g.rowStride;
     GLOBAL_AS const float *srcST = asGlobal(G.learn.srcST) + (size_t)batch * g.numSrcNeurons;
     GLOBAL_AS const float *preTrace = asGlobal(G.learn.preTrace) + (size_t)batch * g.numSrcNeurons;
     const bool rowTraceWanted = paired && !(G.learn.tauPlus > 0.0f);
-    float st0 = paired ? srcST[id0] : 0.0f, tr0 = rowTraceWanted ? preTrace[id0] : 0.0f;
-    for(; s < numSpikes; s += stride) {
-        const uint32_t idPre = id0, a = a0, b = b0;
-        rowST = st0; rowTrace = tr0;
-        id0 = id1;
-        id1 = spk[min(s + 2 * stride, lastSrc)];
-        o0 = (size_t)id0 * (G.numTiles + 1) + G.tile;
-        a0 = off[o0]; b0 = off[o0 + 1];
-        if(paired) { st0 = srcST[id0]; }
-        if(rowTraceWanted) { tr0 = preTrace[id0]; }
-        const size_t rowBase = (size_t)idPre * g.rowStride;
-        for(uint32_t j = a + 4 * lis; j < b; j += 4 * L) {
-            if(j + 4 <= b) {
-                const u32x4u ip = *reinterpret_cast<GLOBAL_AS const u32x4u*>(ind + rowBase + j);
-                const f32x4u w = *reinterpret_cast<GLOBAL_AS const f32x4u*>(weight + rowBase + j);
-                if(stdp) { *reinterpret_cast<GLOBAL_AS f32x4u*>(weight + rowBase + j) = factors ? depressLds4(ip, w) : depress4(idPre, ip, w); }
-                ldsAddF32x4(&shTile[ip.x - tileStart], w.x, true, &shTile[ip.y - tileStart], w.y, true,
-                            &shTile[ip.z - tileStart], w.z, true, &shTile[ip.w - tileStart], w.w, true);
+    uint32_t s = G.split * perBlock + threadIdx.x / L;
+    uint32_t id0[TILE_SEGMENTS], id1[TILE_SEGMENTS], a0[TILE_SEGMENTS], b0[TILE_SEGMENTS];
+    float st0[TILE_SEGMENTS], tr0[TILE_SEGMENTS];
+    auto bounds = [&]() {
+        #pragma unroll
+        for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+            const size_t o0 = (size_t)id0[q] * (G.numTiles + 1) + G.tile;
+            a0[q] = off[o0]; b0[q] = off[o0 + 1];
+            st0[q] = paired ? srcST[id0[q]] : 0.0f;
+            tr0[q] = rowTraceWanted ? preTrace[id0[q]] : 0.0f;
+        }
+    };
+    #pragma unroll
+    for(uint32_t q = 0; q < TILE_SEGMENTS; q++) { id0[q] = spk[min(s + q * stride, lastSrc)]; id1[q] = spk[min(s + (TILE_SEGMENTS + q) * stride, lastSrc)]; }
+    bounds();
+    for(; s < numSpikes; s += TILE_SEGMENTS * stride) {
+        uint32_t idPre[TILE_SEGMENTS], j[TILE_SEGMENTS], b[TILE_SEGMENTS];
+        float rowSTs[TILE_SEGMENTS], rowTraces[TILE_SEGMENTS];
+        uint32_t longest = 0;
+        #pragma unroll
+        for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+            const bool there = (s + q * stride < numSpikes);
+            idPre[q] = id0[q]; rowSTs[q] = st0[q]; rowTraces[q] = tr0[q];
+            b[q] = there ? b0[q] : 0u;
+            j[q] = a0[q] + 4 * lis;
+            if(there && lis == 0) { events += b0[q] - a0[q]; }
+            longest = max(longest, there ? b0[q] - a0[q] : 0u);
+            id0[q] = id1[q];
+        }
+        #pragma unroll
+        for(uint32_t q = 0; q < TILE_SEGMENTS; q++) { id1[q] = spk[min(s + (2 * TILE_SEGMENTS + q) * stride, lastSrc)]; }
+        bounds();
+        for(uint32_t done = 0; done < longest; done += 4 * L) {
+            // a lane's four synapses of each segment, whole quads whether the segment ends within them or not (what follows it in the matrix
+            // is read and not used); a quad that would reach beyond the matrix is read word by word
+            u32x4u ip[TILE_SEGMENTS]; f32x4u w[TILE_SEGMENTS]; uint32_t n[TILE_SEGMENTS]; size_t at[TILE_SEGMENTS]; bool beyond = false;
+            #pragma unroll
+            for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+                n[q] = (j[q] < b[q]) ? min(4u, b[q] - j[q]) : 0u;
+                at[q] = n[q] ? (size_t)idPre[q] * g.rowStride + j[q] : (size_t)0;
+                beyond = beyond || at[q] + 4 > total;
             }
-            else {
-                for(uint32_t jj = j; jj < b; jj++) {
-                    const uint32_t idPost = ind[rowBase + jj];
-                    const float w = weight[rowBase + jj];
-                    if(stdp) {
-                        const uint32_t local = idPost - tileStart;
-                        weight[rowBase + jj] = factors ? depressLds(w, shFactor[local], (shFired[local >> 5] >> (local & 31u)) & 1u) : depress(idPre, idPost, w);
-                    }
-                    ldsAddF32(&shTile[idPost - tileStart], w);
+            if(!beyond) {
+                #pragma unroll
+                for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+                    ip[q] = *reinterpret_cast<GLOBAL_AS const u32x4u*>(ind + at[q]);
+                    w[q] = *reinterpret_cast<GLOBAL_AS const f32x4u*>(weight + at[q]);
                 }
             }
+            else {
+                #pragma unroll
+                for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+                    #pragma unroll
+                    for(uint32_t k = 0; k < 4; k++) { const size_t e = min(at[q] + k, total - 1); ip[q][k] = ind[e]; w[q][k] = weight[e]; }
+                }
+            }
+            #pragma unroll
+            for(uint32_t q = 0; q < TILE_SEGMENTS; q++) {
+                #pragma unroll
+                for(uint32_t k = 0; k < 4; k++) { ip[q][k] = (k < n[q]) ? ip[q][k] : tileStart; }
+                if(stdp) {
+                    rowST = rowSTs[q]; rowTrace = rowTraces[q];
+                    const f32x4u nw = factors ? depressLds4(ip[q], w[q]) : depress4(idPre[q], ip[q], w[q]);
+                    if(n[q] == 4) { *reinterpret_cast<GLOBAL_AS f32x4u*>(weight + at[q]) = nw; }
+                    else {
+                        if(n[q] > 0) { weight[at[q]] = nw.x; }
+                        if(n[q] > 1) { weight[at[q] + 1] = nw.y; }
+                        if(n[q] > 2) { weight[at[q] + 2] = nw.z; }
+                    }
+                }
+                ldsAddF32x4(&shTile[ip[q].x - tileStart], w[q].x, n[q] > 0, &shTile[ip[q].y - tileStart], w[q].y, n[q] > 1,
+                            &shTile[ip[q].z - tileStart], w[q].z, n[q] > 2, &shTile[ip[q].w - tileStart], w[q].w, n[q] > 3);
+                j[q] += 4 * L;
+            }
         }
-        if(lis == 0) { events += b - a; }
     }
     __syncthreads();
     GLOBAL_AS float *outPost = asGlobal(g.outPost) + (size_t)batch * g.numTrgNeurons + tileStart;
@@ -1161,35 +1199,76 @@ __device__ __forceinline__ void postsynapticBody(const PostGroupDev &G, uint32_t
         const uint32_t lane = threadIdx.x & (WAVE - 1);
         const uint32_t numWaves = G.numBlocks * (BS / WAVE);
         GLOBAL_AS const uint32_t *ind = asGlobal(g.ind);
-        // per-row scalars of the NEXT row are fetched while the current one is processed (indices clamped: readable)
+        // A wavefront looks at 64 rows at a time, a lane each: what the rule reads of a row's own neuron, and whether there is anything to do.  It
+        // then takes the rows that have, ROWS at a time, with ROW_QUADS quads of synapses a lane and row asked for together; whole quads, whether
+        // the row ends within them or not (what follows it in the matrix is read and not used).  Nobody else writes these rows in this
+        // step, so a quad is written back whole.
+        constexpr uint32_t ROWS = 2, ROW_QUADS = 2, PARTS = ROWS * ROW_QUADS;
         const uint32_t lastRow = g.numSrcNeurons - 1;
-        uint32_t row = localBlock * (BS / WAVE) + threadIdx.x / WAVE;
-        uint32_t lenNext = asGlobal(g.rowLength)[min(row, lastRow)];
-        float stNext = srcST[min(row, lastRow)], traceNext = additive ? 0.0f : preTrace[min(row, lastRow)];
-        for(; row < g.numSrcNeurons; row += numWaves) {
-            const uint32_t len = lenNext;
-            const float stPre = dt + stNext;
-            const float trace = traceNext;
-            const uint32_t nextRow = min(row + numWaves, lastRow);
-            lenNext = asGlobal(g.rowLength)[nextRow]; stNext = srcST[nextRow];
-            if(!additive) { traceNext = preTrace[nextRow]; }
-            const float dtSpike = st.t - stPre;
-            if(!(dtSpike > 0) || len == 0 || (paired && bitmapTest(srcBitmap, row))) { continue; }
-            const float step = g.aPlus * (additive ? (float)exp((double)(-dtSpike / g.tauPlus)) : trace);
-            const size_t rowBase = (size_t)row * g.rowStride;
-            // up to four strides of the row in flight per lane
-            for(uint32_t j0 = lane; j0 < len; j0 += 4 * WAVE) {
-                uint32_t idPost[4]; float w[4];
+        const size_t total = (size_t)g.numSrcNeurons * g.rowStride;
+        for(unsigned long long base = localBlock * (BS / WAVE) + threadIdx.x / WAVE; base < g.numSrcNeurons; base += (unsigned long long)WAVE * numWaves) {
+            const unsigned long long own = base + (unsigned long long)lane * numWaves;
+            const uint32_t r = (uint32_t)min(own, (unsigned long long)lastRow);
+            const uint32_t ownLen = asGlobal(g.rowLength)[r];
+            const float ownTrace = additive ? 0.0f : preTrace[r];
+            const bool fired = paired && bitmapTest(srcBitmap, r);
+            const float dtSpike = st.t - (dt + srcST[r]);
+            const float ownStep = g.aPlus * (additive ? (float)exp((double)(-dtSpike / g.tauPlus)) : ownTrace);
+            unsigned long long rows = __ballot(own < g.numSrcNeurons && dtSpike > 0 && ownLen != 0 && !fired);
+            while(rows) {
+                uint32_t len[ROWS], longest = 0;
+                float step[ROWS];
+                size_t rowBase[ROWS];
                 #pragma unroll
-                for(int u = 0; u < 4; u++) {
-                    const uint32_t j = j0 + u * WAVE;
-                    idPost[u] = (j < len) ? ind[rowBase + j] : 0xFFFFFFFFu;
-                    w[u] = (j < len) ? weight[rowBase + j] : 0.0f;
+                for(uint32_t q = 0; q < ROWS; q++) {
+                    const int l = rows ? __ffsll((long long)rows) - 1 : 0;
+                    len[q] = rows ? (uint32_t)__builtin_amdgcn_readlane((int)ownLen, l) : 0u;
+                    step[q] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ownStep), l));
+                    rowBase[q] = (size_t)(uint32_t)__builtin_amdgcn_readlane((int)r, l) * g.rowStride;
+                    longest = max(longest, len[q]);
+                    rows &= rows - 1;           // (0 stays 0)
                 }
-                #pragma unroll
-                for(int u = 0; u < 4; u++) {
-                    if(idPost[u] != 0xFFFFFFFFu && ((shBits[idPost[u] >> 5] >> (idPost[u] & 31)) & 1u)) {
-                        weight[rowBase + j0 + u * WAVE] = fminf(g.wMax, fmaxf(g.wMin, w[u] + step));
+                const uint32_t quads = (longest + 3) / 4;
+                for(uint32_t quad = lane; quad < quads; quad += ROW_QUADS * WAVE) {
+                    u32x4u ip[PARTS]; f32x4u w[PARTS]; uint32_t n[PARTS]; size_t at[PARTS]; bool beyond = false;
+                    #pragma unroll
+                    for(uint32_t q = 0; q < PARTS; q++) {
+                        const uint32_t j = 4 * (quad + WAVE * (q % ROW_QUADS)), length = len[q / ROW_QUADS];
+                        n[q] = (j < length) ? min(4u, length - j) : 0u;
+                        at[q] = n[q] ? rowBase[q / ROW_QUADS] + j : (size_t)0;
+                        beyond = beyond || at[q] + 4 > total;
+                    }
+                    if(!beyond) {
+                        #pragma unroll
+                        for(uint32_t q = 0; q < PARTS; q++) {
+                            ip[q] = *reinterpret_cast<GLOBAL_AS const u32x4u*>(ind + at[q]);
+                            w[q] = *reinterpret_cast<GLOBAL_AS const f32x4u*>(weight + at[q]);
+                        }
+                    }
+                    else {
+                        #pragma unroll
+                        for(uint32_t q = 0; q < PARTS; q++) {
+                            #pragma unroll
+                            for(uint32_t k = 0; k < 4; k++) { const size_t e = min(at[q] + k, total - 1); ip[q][k] = ind[e]; w[q][k] = weight[e]; }
+                        }
+                    }
+                    #pragma unroll
+                    for(uint32_t q = 0; q < PARTS; q++) {
+                        bool hit[4];
+                        #pragma unroll
+                        for(uint32_t k = 0; k < 4; k++) {
+                            const uint32_t idPost = (k < n[q]) ? ip[q][k] : 0u;
+                            hit[k] = ((shBits[idPost >> 5] >> (idPost & 31u)) & 1u) && k < n[q];
+                            const float changed = fminf(g.wMax, fmaxf(g.wMin, w[q][k] + step[q / ROW_QUADS]));
+                            w[q][k] = hit[k] ? changed : w[q][k];
+                        }
+                        if(n[q] == 4) {
+                            if(hit[0] || hit[1] || hit[2] || hit[3]) { *reinterpret_cast<GLOBAL_AS f32x4u*>(weight + at[q]) = w[q]; }
+                        }
+                        else {
+                            #pragma unroll
+                            for(uint32_t k = 0; k < 3; k++) { if(hit[k]) { weight[at[q] + k] = w[q][k]; } }
+                        }
                     }
                 }
             }

@@ -106,6 +106,47 @@ def test_tile_path_segment_records(m, fan, tile_floats, records, monkeypatch):
     model.unload()
 
 
+# rows of fewer synapses than a quad (the last one ends the matrix), of more than a wavefront takes at once, more rows than a wavefront looks at at once,
+# a matrix smaller than a quad; several tiles, and what the rule takes off kept beside the tile or not
+@pytest.mark.parametrize("factors", ["0", "2"])
+@pytest.mark.parametrize("rule", ["stdp_trace", "stdp_additive"])
+@pytest.mark.parametrize("n, m, fan", [(64, 300, 3), (5003, 40, 37), (300, 1500, 1203), (2, 1, 1), (700, 900, 130)])
+def test_busy_steps_of_ragged_plastic_rows(n, m, fan, rule, factors, monkeypatch):
+    """Every step with spikes walks the rows on both sides; weights, rasters and event counts must be the oracle's."""
+    from genn_amd.netspec import Net, Pop, Syn
+    from genn_amd import netgen
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "512")
+    monkeypatch.setenv("GENNMI_TILE_FACTORS", factors)
+    monkeypatch.setenv("GENNMI_POST_DENSE_DIVISOR", "1000000")
+    steps = 50
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.8, TauRefrac=2.0)
+    net = Net(name="ragged", dt=1.0, steps=steps)
+    for name, size, step in (("A", n, 17), ("B", m, 29)):
+        v0 = (-60.0 + 10.0 * ((np.arange(size) // 3 * step) % 101) / 101.0).astype(np.float32)
+        net.pops.append(Pop(name, "lif", size, dict(lif), {"V": v0, "RefracTime": np.zeros(size, np.float32)}))
+    rl, ind = netgen.fixed_number_post(11, 3, n, m, fan)
+    rl[:-1][::7] = (rl[:-1][::7] * 2) // 3
+    rl[:-1][3::11] = 0
+    g = netgen.rows_uniform(11, 4, rl, fan, n, 0.5 / fan, 0.0, 0.5 / fan, 0.0)
+    net.syns.append(Syn("AB", "A", "B", wum=rule, wum_params=dict(tauPlus=20.0, tauMinus=20.0, aPlus=0.1 / fan, aMinus=0.12 / fan, wMin=0.0, wMax=1.0 / fan), psm="deltacurr",
+                        row_stride=fan, row_length=rl, ind=ind, g=g))
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=steps)
+    oracle = OracleNet(net, col_stride={"AB": model.synapse_populations["AB"].col_stride}, num_recording_timesteps=steps)
+    model.run(steps)
+    oracle.run(steps)
+    model.pull_recording_buffers_from_device()
+    for p in net.pops:
+        words = (p.n + 31) // 32
+        assert np.array_equal(model.neuron_populations[p.name].vars["recordSpk"].view.reshape(steps, words), oracle.record(p.name, steps).reshape(steps, words)), p.name
+    got, want = model.synapse_populations["AB"].vars["g"].pull_from_device().reshape(n, -1), oracle.syn_g("AB").reshape(n, -1)
+    inside = np.arange(got.shape[1])[None, :] < rl[:, None]
+    assert np.array_equal(got[~inside], want[~inside])
+    assert np.max(np.abs(got - want)) <= 2e-7 * np.max(np.abs(want))        # (the additive rule's exponentials: a unit in the last place)
+    assert model.synaptic_event_count == oracle.events() > 0
+    model.unload()
+
+
 def test_izhikevich_fanout_noise():
     """C3 shape: Izhikevich neurons, fixed fanout with replacement (multapses), DeltaCurr input,
     per-step noise current from a pregenerated array.  dt = 1 ms, first 100 ms = 100 steps."""
