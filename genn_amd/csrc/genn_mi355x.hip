@@ -2089,8 +2089,7 @@ static int refreshSpikeSources(gennmi_runner *r)
             const uint32_t words = (n.g.numNeurons + 31) / 32;
             // (of two copies, the one the coming step reads: the update after k completed steps writes copy (k + 1) & 1)
             uint32_t *bitmap = n.spikeBitmap + (r->epoch & 1) * n.bitmapStride;
-            spikeBitmapFromQueueKernel<<<dim3((words + BLOCK - 1) / BLOCK, r->batch), dim3(BLOCK), 0, r->stream>>>(n.g.spkCnt, n.g.spk, bitmap, n.g.numNeurons, 1u);
-            spikeBitmapFromQueueKernel<<<dim3((n.g.numNeurons + BLOCK - 1) / BLOCK, r->batch), dim3(BLOCK), 0, r->stream>>>(n.g.spkCnt, n.g.spk, bitmap, n.g.numNeurons, 0u);
+            spikeBitmapFromQueueKernel<<<dim3((words + BITMAP_WORDS - 1) / BITMAP_WORDS, r->batch), dim3(BITMAP_WORDS), 0, r->stream>>>(n.g.spkCnt, n.g.spk, bitmap, n.g.numNeurons);
             HIP_TRY(hipGetLastError());
         }
     }

@@ -1147,13 +1147,31 @@ void presynapticConvMfmaKernel(const ConvMfmaDev * __restrict__ blocks, uint32_t
     convMfmaBlock<CONV_MFMA_THREADS>(G, blockIdx.x / numBatches, batch, st.epoch, shConvM, epilogue, eventCounter);
 }
 
-// bitmap of a population's spike queue, for callers that wrote the queue themselves (the neuron update keeps it otherwise)
-__global__ void spikeBitmapFromQueueKernel(const uint32_t *spkCnt, const uint32_t *spk, uint32_t *bitmap, uint32_t numNeurons, uint32_t clear)
+// Bitmap of a population's spike queue, for callers that wrote the queue themselves (the neuron update keeps it otherwise).  A work-group
+// owns BITMAP_WORDS words and looks through the whole queue for them: no word is added to from two sides, and clearing and setting are one launch.
+// A queue is empty or holds a few per cent of the population; one that names all of 10^6 neurons is read by 31 work-groups, 4 MB each.
+constexpr uint32_t BITMAP_WORDS = 1024;
+__global__ __launch_bounds__(BITMAP_WORDS)
+void spikeBitmapFromQueueKernel(const uint32_t *spkCnt, const uint32_t *spk, uint32_t *bitmap, uint32_t numNeurons)
 {
-    const uint32_t batch = blockIdx.y, words = (numNeurons + 31) / 32;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(clear) { if(i < words) { bitmap[(size_t)batch * words + i] = 0u; } return; }
-    if(i < spkCnt[batch]) { const uint32_t id = spk[(size_t)batch * numNeurons + i]; atomicOr(&bitmap[(size_t)batch * words + (id >> 5)], 1u << (id & 31)); }
+    __shared__ uint32_t shWords[BITMAP_WORDS];
+    const uint32_t batch = blockIdx.y, words = (numNeurons + 31) / 32, first = blockIdx.x * BITMAP_WORDS;
+    const uint32_t count = min(spkCnt[batch], numNeurons);
+    const uint32_t *queue = spk + (size_t)batch * numNeurons;
+    shWords[threadIdx.x] = 0u;
+    __syncthreads();
+    for(uint32_t k = threadIdx.x; k < count; k += 4 * BITMAP_WORDS) {
+        uint32_t id[4];
+        #pragma unroll
+        for(uint32_t u = 0; u < 4; u++) { id[u] = queue[min(k + u * BITMAP_WORDS, count - 1)]; }
+        #pragma unroll
+        for(uint32_t u = 0; u < 4; u++) {
+            const uint32_t word = (id[u] >> 5) - first;
+            if(word < BITMAP_WORDS) { atomicOr(&shWords[word], 1u << (id[u] & 31)); }
+        }
+    }
+    __syncthreads();
+    if(first + threadIdx.x < words) { bitmap[(size_t)batch * words + first + threadIdx.x] = shWords[threadIdx.x]; }
 }
 
 __global__ __launch_bounds__(1024)

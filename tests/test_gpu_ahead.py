@@ -231,3 +231,84 @@ def test_convolutions_sum_to_the_same_bits_at_once_and_step_by_step(shape, rate,
     assert states[0][3] == states[1][3] > 0 and np.any(states[0][0])
     for a, b in zip(states[0][:3], states[1][:3]):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# one spike and none, exactly four (the times a lane asks for at once) and one more, as many as steps; the step's length as a float and not, counts of
+# steps that floats hold exactly, that they round to even ones, and beyond 32 bits
+@pytest.mark.parametrize("dt,first_step", [(1.0, 0), (0.1, 3), (0.1, 1 << 22), (0.7, (1 << 24) + 5), (1.0, (1 << 25) + 1), (1.0, (1 << 32) - 40)])
+def test_spike_times_off_the_grid_of_steps(dt, first_step, monkeypatch):
+    """Times between steps, on them, next to them, several in one step (each is emitted a step later than the one before), in the past, not a number and
+    infinite: the steps of their spikes are those of the network stepped one by one."""
+    steps, n = 100, 130
+    rng = np.random.default_rng(5)
+    start = np.float32(first_step) * np.float32(dt)
+    grid = (np.arange(first_step, first_step + steps + 10).astype(np.float32) * np.float32(dt)).astype(np.float32)
+    trains = []
+    for i in range(n):
+        count = [0, 1, 3, 4, 5, 8, 9, 40, steps + 5][i % 9]
+        kind = (i // 9) % 4
+        if kind == 0:
+            times = rng.choice(grid, count)
+        elif kind == 1:
+            times = np.nextafter(rng.choice(grid, count), np.float32(rng.choice([-np.inf, np.inf])))
+        elif kind == 2:
+            times = start + np.float32(dt) * (rng.integers(-3, steps // 10, count) * 10 + 0.5)
+        else:
+            times = start + np.float32(dt) * rng.uniform(-5.0, steps, count)
+        times = np.sort(times.astype(np.float32))
+        if count and i % 5 == 0:
+            times[count // 2] = np.nan
+        if count and i % 5 == 1:
+            times[-1] = np.inf
+        trains.append(times)
+    end = np.cumsum([len(t) for t in trains])
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        net = _net("dense", (n, 33), steps)
+        source = net.pop("In")
+        source.spike_times = np.concatenate(trains).astype(np.float32)
+        source.vars = {"startSpike": np.concatenate([[0], end[:-1]]).astype(np.uint32), "endSpike": end.astype(np.uint32)}
+        net.dt = dt
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        model.timestep = first_step
+        model.run(steps)
+        model.pull_recording_buffers_from_device()
+        pops = [model.neuron_populations[name] for name in ("In", "Out")]
+        got.append([p.vars["recordSpk"].view.copy() for p in pops] + [pops[0].vars["startSpike"].pull_from_device().copy(), pops[1].vars["V"].pull_from_device().copy()])
+        model.unload()
+    assert np.any(got[0][0])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+# a word, one work-group's words and a few beyond, more spikes than its threads take in a round
+@pytest.mark.parametrize("n", [1, 40, 32767, 32801, 70001])
+def test_a_queue_cut_short_between_runs(n, monkeypatch):
+    """A count written between two runs: the source's bitmap is made from the queue's first entries."""
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        net = _net("dense", (n, 3), 40)
+        source = net.pop("In")
+        # every third neuron does not fire in the run's last step
+        offset = np.where(np.arange(n) % 3 == 1, 0.0, 9.0).astype(np.float32)
+        source.spike_times = np.stack([np.full(n, 4.0, np.float32), np.maximum(offset, 5.0)], axis=1).reshape(-1).astype(np.float32)
+        source.vars = {"startSpike": np.arange(0, 2 * n, 2, dtype=np.uint32), "endSpike": np.arange(2, 2 * n + 2, 2, dtype=np.uint32)}
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=40)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        model.run(10)
+        source = model.neuron_populations["In"]
+        left = len(source.current_spikes[0])
+        assert left == np.count_nonzero(offset)
+        source.vars["spkCnt"].view[:] = max(left - 3, left // 2)
+        source.vars["spkCnt"].push_to_device()
+        events = model.synaptic_event_count
+        model.run(10)
+        got.append((model.neuron_populations["Out"].vars["V"].pull_from_device().copy(), model.synaptic_event_count - events))
+        model.unload()
+    assert got[0][1] == got[1][1] == 3 * max(left - 3, left // 2)
+    assert np.array_equal(got[0][0], got[1][0])
