@@ -13,8 +13,8 @@
 //   4. aheadQueueKernel: the spike queues as the last step leaves them, in ascending neuron index.
 // What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
 //
-// run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 205 us;
-// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 940 us, of which 500 move 26 MB between host and device.
+// run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 180 us;
+// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 865 us, of which 500 move 26 MB between host and device.
 #pragma once
 
 namespace
@@ -162,6 +162,16 @@ __device__ __forceinline__ bool aheadOrdinary(float w)
     const uint32_t bits = __float_as_uint(w);
     return ((bits & 0x7F800000u) - (37u << 23)) < ((255u - 37u) << 23) || (bits << 1) == 0u;
 }
+// smallest of eight weights' patterns without sign, moved so that infinities and NaN (from 0), 0 (2^24) and whatever is below 2^-90 lie under
+// AHEAD_ORDINARY and all else above: one comparison tells that every one of them can be split as it is
+constexpr uint32_t AHEAD_ORDINARY = 38u << 24;
+__device__ __forceinline__ uint32_t aheadLeast(const float w[8])
+{
+    uint32_t q[8];
+    #pragma unroll
+    for(int k = 0; k < 8; k++) { q[k] = (__float_as_uint(w[k]) << 1) + (1u << 24); }
+    return min(min(min(min(q[0], q[1]), q[2]), min(min(q[3], q[4]), q[5])), min(q[6], q[7]));
+}
 // top 16 bits of two words, packed; what the top 16 bits leave of a float (exact)
 __device__ __forceinline__ uint32_t aheadTop(float lower, float upper) { return __builtin_amdgcn_perm(__float_as_uint(upper), __float_as_uint(lower), 0x07060302u); }
 __device__ __forceinline__ float aheadRest(float w) { return w - __uint_as_float(__float_as_uint(w) & 0xFFFF0000u); }
@@ -183,36 +193,45 @@ __device__ __forceinline__ uint32_t aheadRow(uint32_t v, uint32_t half) { return
 // source; its wavefronts deal the slice's chunks of 64 source neurons among themselves and add their tiles up in LDS in a fixed order.
 // Source neurons that are silent in all of the group's steps are dropped first (a ballot packs the others), so what is
 // read and multiplied follows the activity: at 5 % and 128 steps all rows remain, at 0.1 % one in eight.  Bound by reading the weights:
-// 8192 x 8192 for 100 steps takes 75 us, 3.6 TB/s (152 us with v_mfma_f32_32x32x2_f32, bound by the matrix rate).  Error of outPost after
+// 8192 x 8192 for 100 steps takes 55 us, 4.9 TB/s.  That needs loads under way all the time (75 us where a group's were asked for behind the
+// group before it and every chunk began with a trip for its words and one for its first weights) and fewer instructions than the loads leave
+// room for: 32-bit offsets of rows in the list instead of 64-bit products, one comparison for eight weights that can be split.  128
+// registers: four wavefronts a SIMD.  (152 us with v_mfma_f32_32x32x2_f32, bound by the matrix rate.)  Error of outPost after
 // 100 steps against 64 bits, one by one -> here (2-norm, relative): 8192 sources 2.0e-7 -> 1.4e-7, 300 sources 1.6e-7 -> 0.8e-7, weights of
 // one sign 1.4e-7 -> 0.7e-7.
 template<int MT>
-__global__ __launch_bounds__(AHEAD_DENSE_THREADS)
+__global__ __launch_bounds__(AHEAD_DENSE_THREADS, 4)
 void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint32_t mGroups, const float * __restrict__ weights, uint32_t numSrc, uint32_t numTrg,
                       uint32_t sourcesPerSlice, float * __restrict__ partial)
 {
     constexpr uint32_t LIST_WORDS = WAVE * (MT + 1), TILE = MT * 32 * 32;
-    __shared__ __align__(16) uint32_t lds[(AHEAD_DENSE_WAVES * LIST_WORDS > AHEAD_TILE_COPIES * TILE) ? AHEAD_DENSE_WAVES * LIST_WORDS : AHEAD_TILE_COPIES * TILE];
-    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, col = lane & 31;
+    static_assert(AHEAD_DENSE_WAVES * 2 * LIST_WORDS <= AHEAD_TILE_COPIES * TILE, "lists and tiles share LDS");
+    __shared__ __align__(16) uint32_t lds[AHEAD_TILE_COPIES * TILE];
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), half = lane >> 5, col = lane & 31;
     const uint32_t mGroup = blockIdx.y % mGroups, slice = blockIdx.y / mGroups;
     const uint32_t firstTile = mGroup * MT;
-    const uint32_t column = blockIdx.x * 32 + col, readColumn = min(column, numTrg - 1);
-    const uint32_t sliceBegin = slice * sourcesPerSlice, sliceEnd = min(numSrc, sliceBegin + sourcesPerSlice);
+    const uint32_t column = blockIdx.x * 32 + col, columnByte = min(column, numTrg - 1) * 4, rowBytes = numTrg * 4;
+    const uint32_t sliceBegin = slice * sourcesPerSlice, sliceEnd = min(numSrc, sliceBegin + sourcesPerSlice), sliceFirst = sliceBegin + wave * WAVE;
     GLOBAL_AS const uint32_t *in = asGlobal(words);
-    GLOBAL_AS const float *w = asGlobal(weights) + readColumn;
-    // [64] source neurons, then per tile [64] lower and [64] upper halves of their words, 16 bits each
-    uint32_t *list = lds + wave * LIST_WORDS;
-    uint16_t *halves = reinterpret_cast<uint16_t*>(list + WAVE);
+    // two lists of [64] source neurons, as byte offsets of their rows behind the chunk's first (below 2^32: a layer's input of 32 steps fits
+    // AHEAD_MAX_SPACE, and a row is a 32nd of that), then per tile [64] lower and [64] upper halves of their words, 16 bits each
+    uint32_t *lists = lds + wave * 2 * LIST_WORDS;
     f32x16 acc[MT];
     #pragma unroll
     for(int q = 0; q < MT; q++) { acc[q] = f32x16{}; }
+    auto fetch = [&](uint32_t base, uint32_t mine[MT]) {
+        const uint32_t readable = min(base + lane, numSrc - 1);
+        #pragma unroll
+        for(int q = 0; q < MT; q++) { mine[q] = in[(size_t)min(firstTile + q, mTiles - 1) * numSrc + readable]; }
+    };
     // the active ones of 64 source neurons, packed and filled up to a multiple of 16 with entries without spikes; returns how many
-    auto pack = [&](uint32_t base) -> uint32_t {
-        const uint32_t i = base + lane;
-        uint32_t mine[MT], any = 0;
+    auto pack = [&](uint32_t base, uint32_t mine[MT], uint32_t *list) -> uint32_t {
+        uint16_t *halves = reinterpret_cast<uint16_t*>(list + WAVE);
+        const uint32_t inside = (base + lane < sliceEnd) ? 0xFFFFFFFFu : 0u;
+        uint32_t any = 0;
         #pragma unroll
         for(int q = 0; q < MT; q++) {
-            mine[q] = (i < sliceEnd && firstTile + q < mTiles) ? in[(size_t)(firstTile + q) * numSrc + i] : 0u;
+            mine[q] &= (firstTile + q < mTiles) ? inside : 0u;
             any |= mine[q];
         }
         const unsigned long long active = __ballot(any != 0);
@@ -221,7 +240,7 @@ void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint
         const uint32_t at = any ? __popcll(active & ((1ull << lane) - 1ull)) : count + __popcll(~active & ((1ull << lane) - 1ull));
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");      // (16-bit stores, 128-bit loads: the compiler must not move either across)
         if(at < filled) {
-            list[at] = min(i, sliceEnd - 1);
+            list[at] = min(lane, sliceEnd - 1 - base) * rowBytes;
             #pragma unroll
             for(int q = 0; q < MT; q++) {
                 halves[(2 * q) * WAVE + at] = (uint16_t)mine[q];
@@ -231,53 +250,85 @@ void aheadDenseKernel(const uint32_t * __restrict__ words, uint32_t mTiles, uint
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         return filled;
     };
-    // a lane's rows are the steps of its column number: the lower or the upper halves
-    const u32x4 *bits = reinterpret_cast<const u32x4*>(list + WAVE + (col >> 4) * (WAVE / 2)) + half;
-    const u32x4 *sources = reinterpret_cast<const u32x4*>(list) + 2 * half;
+    auto rowsOf = [&](uint32_t base) { return asGlobal(reinterpret_cast<const char*>(weights + (size_t)base * numTrg)); };
+    // Groups of 16 packed sources, a chunk's and then the next one's: a group's weights are asked for before the group ahead of it is worked off, a
+    // chunk's words before the chunk ahead of it.  (A chunk's list is made when the last group of the one before is still being read: two lists.)
+    uint32_t base = sliceFirst, groups = 0, group = 0, other = 0, mine[MT];
+    uint32_t *list = lists;
+    GLOBAL_AS const char *rows = nullptr;
     bool special = false;
-    for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
-        const uint32_t groups = pack(base) / 16;
-        float b[8], bNext[8];
-        auto load = [&](uint32_t g, float x[8]) {
-            const u32x4 first = sources[4 * g], second = sources[4 * g + 1];
-            #pragma unroll
-            for(int k = 0; k < 4; k++) { x[k] = w[(size_t)first[k] * numTrg]; x[4 + k] = w[(size_t)second[k] * numTrg]; }
-        };
-        if(groups) { load(0, b); }
-        for(uint32_t g = 0; g < groups; g++) {
-            if(g + 1 < groups) { load(g + 1, bNext); }
-            u32x4 top, middle, low;
+    // moves on to the next group; false: there is none, and the list's first one stands in for it
+    auto advance = [&]() -> bool {
+        if(++group < groups) { return true; }
+        group = 0;
+        uint32_t found = 0;
+        while(base < sliceEnd && found == 0) {
+            found = pack(base, mine, lists + other) / 16;
+            base += AHEAD_DENSE_THREADS;
+            fetch(base, mine);
+        }
+        if(found == 0) { return false; }
+        groups = found;
+        rows = rowsOf(base - AHEAD_DENSE_THREADS);
+        list = lists + other;
+        other = LIST_WORDS - other;
+        return true;
+    };
+    auto load = [&](float x[8]) {
+        const u32x4 *sources = reinterpret_cast<const u32x4*>(list) + 4 * group + 2 * half;
+        const u32x4 first = sources[0], second = sources[1];
+        #pragma unroll
+        for(int k = 0; k < 4; k++) {
+            x[k] = *reinterpret_cast<GLOBAL_AS const float*>(rows + (first[k] + columnByte));
+            x[4 + k] = *reinterpret_cast<GLOBAL_AS const float*>(rows + (second[k] + columnByte));
+        }
+    };
+    // works the group off whose weights are in b, those of the next one on their way into `following`; false: it was the last
+    auto work = [&](float b[8], float following[8]) -> bool {
+        // a lane's rows are the steps of its column number: the lower or the upper halves
+        const u32x4 *bits = reinterpret_cast<const u32x4*>(list + WAVE + (col >> 4) * (WAVE / 2)) + half + 2 * group;
+        const bool more = advance();
+        load(following);            // (not behind a branch: b is then waited for while these are under way)
+        if(__ballot(aheadLeast(b) < AHEAD_ORDINARY)) {
             #pragma unroll
             for(int k = 0; k < 8; k++) {
                 const bool ordinary = aheadOrdinary(b[k]);
                 special = special || !ordinary;
                 b[k] = ordinary ? b[k] : 0.0f;
             }
-            #pragma unroll
-            for(int k = 0; k < 4; k++) {
-                const float r0 = aheadRest(b[2 * k]), r1 = aheadRest(b[2 * k + 1]);
-                top[k] = aheadTop(b[2 * k], b[2 * k + 1]);
-                middle[k] = aheadTop(r0, r1);
-                low[k] = aheadTop(aheadRest(r0), aheadRest(r1));
-            }
-            bf16x8 a[MT];
-            #pragma unroll
-            for(int q = 0; q < MT; q++) { a[q] = aheadBits(bits[q * (WAVE / 4) + 2 * g], col & 15); }
-            #pragma unroll
-            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, low), acc[q]); }
-            #pragma unroll
-            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, middle), acc[q]); }
-            #pragma unroll
-            for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, top), acc[q]); }
-            #pragma unroll
-            for(int k = 0; k < 8; k++) { b[k] = bNext[k]; }
         }
+        u32x4 top, middle, low;
+        #pragma unroll
+        for(int k = 0; k < 4; k++) {
+            const float r0 = aheadRest(b[2 * k]), r1 = aheadRest(b[2 * k + 1]);
+            top[k] = aheadTop(b[2 * k], b[2 * k + 1]);
+            middle[k] = aheadTop(r0, r1);
+            low[k] = aheadTop(aheadRest(r0), aheadRest(r1));
+        }
+        bf16x8 a[MT];
+        #pragma unroll
+        for(int q = 0; q < MT; q++) { a[q] = aheadBits(bits[q * (WAVE / 4)], col & 15); }
+        #pragma unroll
+        for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, low), acc[q]); }
+        #pragma unroll
+        for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, middle), acc[q]); }
+        #pragma unroll
+        for(int q = 0; q < MT; q++) { acc[q] = aheadProduct(a[q], __builtin_bit_cast(bf16x8, top), acc[q]); }
+        return more;
+    };
+    fetch(base, mine);
+    if(advance()) {
+        float even[8], odd[8];
+        load(even);
+        while(work(even, odd) && work(odd, even)) {}
     }
     if(__ballot(special)) {
-        for(uint32_t base = sliceBegin + wave * WAVE; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
-            const uint32_t count = pack(base);
+        for(base = sliceFirst; base < sliceEnd; base += AHEAD_DENSE_THREADS) {
+            fetch(base, mine);
+            const uint32_t count = pack(base, mine, lists);
+            const uint16_t *halves = reinterpret_cast<const uint16_t*>(lists + WAVE);
             for(uint32_t k = 0; k < count; k++) {
-                const float x = w[(size_t)list[k] * numTrg];
+                const float x = *reinterpret_cast<GLOBAL_AS const float*>(rowsOf(base) + (lists[k] + columnByte));
                 if(aheadOrdinary(x)) { continue; }
                 #pragma unroll
                 for(int q = 0; q < MT; q++) {

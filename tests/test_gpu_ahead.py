@@ -312,3 +312,33 @@ def test_a_queue_cut_short_between_runs(n, monkeypatch):
         model.unload()
     assert got[0][1] == got[1][1] == 3 * max(left - 3, left // 2)
     assert np.array_equal(got[0][0], got[1][0])
+
+
+# one, two and four words of rows a work-group; chunks of 64 sources without a spike at the beginning, between others, at the end and throughout
+@pytest.mark.parametrize("steps", [20, 40, 100])
+@pytest.mark.parametrize("active", [(), (0,), (1999,), (700, 701, 1290), tuple(range(512, 600)) + (1500,), tuple(range(0, 2000, 63))])
+def test_dense_layers_of_sources_most_of_which_are_silent(steps, active, monkeypatch):
+    """Every spike of the few sources counts once; among their weights are zeros, infinite ones and ones that are not a number, which keep the others
+    of their groups as they are.  Sums of multiples of 2^-8 are exact: the state is that of the network stepped one by one."""
+    n = 2000
+    net = _net("dense", (n, 70), steps)
+    source, g = net.pop("In"), net.syns[0].g.reshape(n, 70)
+    trains = [np.arange(i % 3, steps - 1, 1 + i % 5, dtype=np.float32) if i in active else np.zeros(0, np.float32) for i in range(n)]
+    end = np.cumsum([len(t) for t in trains])
+    source.spike_times = np.concatenate(trains + [np.zeros(1, np.float32)])
+    source.vars = {"startSpike": np.concatenate([[0], end[:-1]]).astype(np.uint32), "endSpike": end.astype(np.uint32)}
+    for k, i in enumerate(active):
+        g[i, k % 70] = [0.0, -0.0, np.inf, np.nan][k % 4]
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        model = model_from_net(net)
+        model.load(num_recording_timesteps=steps)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        model.run(steps)
+        model.pull_recording_buffers_from_device()
+        out = model.neuron_populations["Out"]
+        got.append((out.vars["V"].pull_from_device().copy(), out.vars["recordSpk"].view.copy(), model.synaptic_event_count))
+        model.unload()
+    assert np.array_equal(got[0][0], got[1][0], equal_nan=True) and np.array_equal(got[0][1], got[1][1])
+    assert got[0][2] == got[1][2] == 70 * end[-1]
