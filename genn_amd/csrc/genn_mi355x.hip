@@ -1779,14 +1779,19 @@ int gennmi_runner_finalise(gennmi_runner *r)
             const char *envSplit = getenv("GENNMI_TILE_BLOCKS_PER_CU");
             const uint32_t blocksPerCUTile = envSplit ? (uint32_t)std::max(1, atoi(envSplit)) : 4u;
             const uint32_t budget = blocksPerCUTile * numCU * BLOCK / r->tileThreads;
-            // ... several groups share two such rounds in proportion to their synapse counts: a launch's floor is the
-            // dispatch of its blocks, and the quiet steps of a network with many projections should not pay for a round each
+            // ... several groups share such rounds in proportion to their synapse counts: a launch's floor is the
+            // dispatch of its blocks, and the quiet steps of a network with many projections should not pay for a round each.
+            // Those with records share two (fewer of their blocks take part in a calm step, below; with one, the bursts of 10^6 neurons x 1000
+            // take 816 us instead of 645), the others one: each of their blocks clears, flushes and (plastic) works out the
+            // factors of a whole tile, and the second round waits for the first.  us of synapse kernels in 400 steps with two / one / half a round:
+            // plastic networks 100,000 x 500 5652 / 5326 / 5487, 100,000 x 100 7334 / 6542 / 6079, 40,000 x 300 3020 / 2767 / 2675, 17,011 x 300
+            // 2276 / 2220 / 2163, 9,000 x 300 1969 / 1949 / 1982; 200 steps of the balanced network 300,007 x 1000 1852 / 1723 / 1696.
             const char *envPerSplit = getenv("GENNMI_TILE_SPIKES_PER_SPLIT");
             const uint32_t spikesPerSplit = envPerSplit ? (uint32_t)std::max(1, atoi(envPerSplit)) : 4096u;
             double totalWeight = 0.0;
             for(const auto &t : tileGroups) { totalWeight += (double)t.g.numSrcNeurons * t.g.rowStride; }
             for(auto &t : tileGroups) {
-                const double share = (tileGroups.size() == 1) ? 1.0 : 2.0 * ((double)t.g.numSrcNeurons * t.g.rowStride) / totalWeight;
+                const double share = (tileGroups.size() == 1) ? 1.0 : (t.recLanes ? 2.0 : 1.0) * ((double)t.g.numSrcNeurons * t.g.rowStride) / totalWeight;
                 const uint32_t groupBudget = std::max(t.numTiles, (uint32_t)(share * budget));
                 const uint32_t numSplits = std::max(1u, std::min(256u, groupBudget / t.numTiles));
                 t.numSplits = numSplits;
