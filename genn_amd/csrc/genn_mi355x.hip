@@ -1731,7 +1731,13 @@ int gennmi_runner_finalise(gennmi_runner *r)
             const uint32_t tileSize = offsets[candidate].tileSize, numTiles = offsets[candidate].numTiles, unsorted = unsortedFlags[candidate];
             uint16_t *dOff = offsets[candidate++].off;
             if(unsorted) { continue; }          // rows not sorted by target: the scatter kernel handles every step
+            // Events from which a step goes to the tiles: one per target, but 49,152 (scattered one by one, 2 us) if that is more, and then no more
+            // than four per target (additions to one address follow each other).  us of synapse kernels with one per target -> now: 400
+            // steps of plastic networks 6,000 x 100 3604 -> 2395, 17,011 x 300 2234 -> 2147, 80 of Izhikevich networks 30,000 x 300 696 -> 665,
+            // 12,000 x 500 647 -> 602.  (Half a one per target: balanced 300,000 x 1000 1810 -> 1723 but the steps of a pass no faster.)  Projections with
+            // records, and where the tile size is given: one per target.
             p.tileThreshold = std::max(1u, p.g.numTrgNeurons);
+            if(!envTile) { p.tileThreshold = std::max(p.tileThreshold, (uint32_t)std::min<uint64_t>(49152, 4ull * p.g.numTrgNeurons)); }
             r->tileTables.push_back({(size_t)(&p - r->pre.data()), dOff, tileSize, numTiles});
             const uint32_t avgSeg = std::max(1u, p.g.rowStride / numTiles);
             TileGroupDev t{};
@@ -1765,6 +1771,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
                     { const int rc = buildTileRecords(r, table); if(rc) { return rc; } }
                     r->recordTables.push_back(table);
                     t.records = records; t.recLanes = lanes; t.overflow = overflow;
+                    t.threshold = p.tileThreshold = std::max(1u, p.g.numTrgNeurons);
                 }
             }
             t.segLength = avgSeg;

@@ -147,6 +147,29 @@ def test_busy_steps_of_ragged_plastic_rows(n, m, fan, rule, factors, monkeypatch
     model.unload()
 
 
+# four events per target; 49,152 events; one event per target: steps on either side of each
+@pytest.mark.parametrize("m, fan, at", [(1, 1, 4), (1000, 40, 4000), (20000, 80, 49152), (150000, 800, 150000)])
+def test_steps_around_the_tile_path_s_threshold(m, fan, at):
+    """As many events as send a step to the tile kernel, one spike more and one fewer: both paths add the same multiples of 2^-3."""
+    from genn_amd.netspec import Net, Pop, Syn
+    from genn_amd import netgen
+    least = (at + fan - 1) // fan
+    n = least + 1
+    net = Net(name="threshold", dt=1.0, steps=12)
+    # neuron i fires in steps 2, 5 and 8, but for the last two and the last one in two of them
+    times = [[2.0] * (i < least - 1) + [5.0] * (i < least) + [8.0] for i in range(n)]
+    end = np.cumsum([len(t) for t in times]).astype(np.uint32)
+    net.pops.append(Pop("A", "ssa", n, {}, {"startSpike": np.concatenate([[0], end[:-1]]).astype(np.uint32), "endSpike": end}, spike_times=np.concatenate(times).astype(np.float32)))
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.0, TauRefrac=2.0)
+    net.pops.append(Pop("B", "lif", m, lif, {"V": np.full(m, -60.0, np.float32), "RefracTime": np.zeros(m, np.float32)}))
+    rl, ind = netgen.fixed_number_post(7, 3, n, m, fan)
+    g = (np.arange(n * fan) % 9 - 3).astype(np.float32).reshape(n, fan) / 8.0
+    net.syns.append(Syn("AB", "A", "B", wum="static", psm="deltacurr", row_stride=fan, row_length=rl, ind=ind, g=g))
+    model, oracle, counts = run_side_by_side(net, check_every=1, exact=True)
+    assert counts["A"] == 3 * least and model.synaptic_event_count == oracle.events()
+    model.unload()
+
+
 def test_izhikevich_fanout_noise():
     """C3 shape: Izhikevich neurons, fixed fanout with replacement (multapses), DeltaCurr input,
     per-step noise current from a pregenerated array.  dt = 1 ms, first 100 ms = 100 steps."""
