@@ -193,6 +193,7 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
 // (tagged with the step so nothing ever needs clearing) the cross-block offset.  Only blocks that
 // emitted spikes, and the last block of each population (which stores spkCnt), look back.
 // ------------------------------------------------------------------------------------------------
+template<bool DIRECT = true>
 __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                            const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
@@ -391,7 +392,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     }
     storeState();
     const bool last = (localBlock == G.numBlocks - 1);
-    const bool direct = queueDirect(G.numBlocks), groupLeader = (!direct && (localBlock % WAVE) == WAVE - 1) || last;
+    const bool direct = DIRECT && queueDirect(G.numBlocks), groupLeader = (!direct && (localBlock % WAVE) == WAVE - 1) || last;
     if(blockCount == 0 && !groupLeader) { return; }
 
     // Synapses with d % D == 0 of the neurons that just fired belong in the slot their targets read in the
@@ -745,7 +746,8 @@ void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t 
         // the neuron blocks are the critical path (other blocks wait for their spike counts): let their
         // instructions issue ahead of the presynaptic blocks that share the compute unit
         __builtin_amdgcn_s_setprio(3);
-        neuronBody(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
+        // (offsets in two levels: 50 steps of the full microcircuit 562 us, with sumOfEarlierBlocks in this kernel 569; at 0.35 of it 682 either way)
+        neuronBody<false>(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
     }
     else { presynapticBody(preBlocks[blockIdx.x - numNeuronBlocks], blockIdx.x - numNeuronBlocks, blockIdx.y, gridDim.y, st, dt, eventCounter); }
 }
