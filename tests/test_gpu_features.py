@@ -337,3 +337,38 @@ def test_spike_queue_is_ascending_and_complete_at_any_number_of_blocks(blocks, p
     for step, queue in enumerate(queues):
         assert np.array_equal(queue, np.nonzero(bits[step])[0])
     model.unload()
+
+
+# a row's parts are read by neighbouring lanes whatever number of them a spike is given: one lane a spike took 1.5 times as long as eight when its row's
+# synapses were dealt to the work-groups one by one (their cache lines are then fetched by as many of them)
+def test_one_lane_a_spike_reads_rows_as_well_as_eight_do(monkeypatch):
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "0")          # (busy steps too are the scatter kernel's)
+    n, fan, steps = 10000, 1000, 100
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=1.0, TauRefrac=5.0)
+    rng = np.random.default_rng(5)
+    pre, post = np.repeat(np.arange(n), fan), rng.integers(0, n, n * fan)
+    v = rng.uniform(-60.0, -50.0, n).astype(np.float32)
+    took, sums = {}, {}
+    for hint, lanes in (("WAVE", 1), ("PRESYNAPTIC", 1), ("PRESYNAPTIC", 8)):
+        model = GeNNModel("float", "lanes", dt=0.5)
+        model.timing_enabled = True
+        a = model.add_neuron_population("A", n, "LIF", lif, {"V": v, "RefracTime": 0.0})
+        b = _silent_pop(model, "B", n)
+        s = model.add_synapse_population("AB", "SPARSE", a, b, init_weight_update("StaticPulse", {}, {"g": 0.125}), init_postsynaptic("ExpCurr", {"tau": 5.0}))
+        s.set_sparse_connections(pre, post)
+        s.parallelism_hint, s.num_threads_per_spike = hint, lanes
+        model.build()
+        model.load()
+        rounds = []
+        for _ in range(5):
+            before = model.presynaptic_update_time
+            for _ in range(steps):
+                model.step_time()
+            rounds.append(model.presynaptic_update_time - before)
+        took[hint, lanes] = min(rounds)
+        sums[hint, lanes] = b.vars["V"].pull_from_device().copy()
+        model.unload()
+    # (V is a sum of up to 500 steps' inputs in fp32, in any order: 500 * 2^-24)
+    for key in took:
+        assert np.max(np.abs(sums[key] - sums["WAVE", 1])) <= 500 * 2.0 ** -24 * np.max(np.abs(sums["WAVE", 1] + 60.0)), key
+    assert took["PRESYNAPTIC", 1] < 1.25 * took["PRESYNAPTIC", 8], took
