@@ -53,10 +53,12 @@ __device__ __forceinline__ float poissonExpInject(const gennmi_cs_t &cs, GLOBAL_
 // 0xFFFFFFFF after a bounded wait expired (error flag raised).
 // ------------------------------------------------------------------------------------------------
 // Populations of more blocks than a wavefront has lanes and of no more than this: one trip after the last count instead of the three of two
-// levels (counts of the group, its total out, totals in).  us a pass: 300,000 neurons stepped 50 times 645 -> 608, 10^6 Izhikevich neurons 20 times
-// 360 -> 349 (the kernel 10.5 -> 9.5), 100,000 plastic ones 100 times 1949 -> 1924.  Beyond, a step in which every block has spikes would
-// read more counts than spikes.
-constexpr uint32_t QUEUE_DIRECT_BLOCKS = 2048;
+// levels (counts of the group, its total out, totals in).  Beyond, a step in which every block has spikes would read more counts than spikes.
+// Counts that have not arrived at the first look are asked for again together; eight at once instead of four cost registers (300,000 neurons 6.0 -> 8.5).
+// us a step of neurons alone, two levels -> counts asked for again one by one -> together, no spike / one in 20,000 / one in 200 of the neurons: 20,000
+// neurons 4.64 -> 4.36 -> 4.34, 4.67 -> 4.42 -> 4.38, 4.89 -> 4.58 -> 4.58; 140,000 4.73 -> 4.80 -> 4.78, 5.03 -> 4.83 -> 4.78, 6.12 -> 5.02 -> 4.99; 300,000
+// 5.40 -> 5.70 -> 5.54, 5.67 -> 5.82 -> 5.67, 7.07 -> 6.01 -> 5.84; 520,000 7.25 -> 7.40 -> 7.31, 7.66 -> 7.57 -> 7.46, 10.87 -> 8.23 -> 8.07.
+constexpr uint32_t QUEUE_DIRECT_BLOCKS = 2048, COUNTS_AT_ONCE = 4;
 __device__ __forceinline__ bool queueDirect(uint32_t numBlocks) { return numBlocks > WAVE && numBlocks <= QUEUE_DIRECT_BLOCKS; }
 __device__ __forceinline__ uint32_t sumOfEarlierBlocks(uint32_t localBlock, const unsigned long long *counts, uint32_t tag, uint32_t *errorFlag)
 {
@@ -64,20 +66,31 @@ __device__ __forceinline__ uint32_t sumOfEarlierBlocks(uint32_t localBlock, cons
     const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, threads = blockDim.x;
     uint32_t sum = 0, spins = 0;
     bool ok = true;
-    for(uint32_t base = threadIdx.x; base < localBlock; base += 4 * threads) {
-        unsigned long long word[4];
+    for(uint32_t first = 0; first < localBlock && ok; first += COUNTS_AT_ONCE * threads) {
+        unsigned long long word[COUNTS_AT_ONCE];
+        uint32_t pending = 0;
+        // (a count that is not there to be read: 0 with the step's tag)
         #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) { word[u] = __hip_atomic_load(&counts[min(base + u * threads, localBlock - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-        #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) {
-            if(base + u * threads >= localBlock) { continue; }
-            while(ok && (uint32_t)(word[u] >> 32) != tag) {
-                if(++spins > c_spinLimit) { ok = false; break; }
-                __builtin_amdgcn_s_sleep(1);
-                word[u] = __hip_atomic_load(&counts[base + u * threads], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            sum += (uint32_t)word[u];
+        for(uint32_t u = 0; u < COUNTS_AT_ONCE; u++) {
+            const uint32_t k = first + u * threads + threadIdx.x;
+            word[u] = (unsigned long long)tag << 32;
+            if(k < localBlock) { word[u] = __hip_atomic_load(&counts[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
         }
+        // (those that had not arrived are asked for again together, not one after the other)
+        while(true) {
+            pending = 0;
+            #pragma unroll
+            for(uint32_t u = 0; u < COUNTS_AT_ONCE; u++) { pending |= ((uint32_t)(word[u] >> 32) != tag) ? 1u << u : 0u; }
+            if(pending == 0) { break; }
+            if(++spins > c_spinLimit) { ok = false; break; }
+            __builtin_amdgcn_s_sleep(1);
+            #pragma unroll
+            for(uint32_t u = 0; u < COUNTS_AT_ONCE; u++) {
+                if((pending >> u) & 1u) { word[u] = __hip_atomic_load(&counts[first + u * threads + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+            }
+        }
+        #pragma unroll
+        for(uint32_t u = 0; u < COUNTS_AT_ONCE; u++) { sum += (uint32_t)word[u]; }
     }
     if(!ok) { raiseErrorFlag(errorFlag); }
     for(int off = WAVE / 2; off > 0; off >>= 1) { sum += __shfl_down(sum, off, WAVE); }

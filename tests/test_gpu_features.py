@@ -339,6 +339,38 @@ def test_spike_queue_is_ascending_and_complete_at_any_number_of_blocks(blocks, p
     model.unload()
 
 
+@pytest.mark.parametrize("per_lane", [1, 4])
+@pytest.mark.parametrize("blocks", [65, 1300, 2048])
+def test_a_count_that_does_not_come_is_reported_not_waited_for(blocks, per_lane, monkeypatch):
+    """With a wait bound of zero polls the first count of an earlier block that is not there when it is looked at raises the device error flag; the
+    kernels end normally, and the next synchronisation reports it."""
+    from genn_amd._abi import GennmiError
+    monkeypatch.setenv("GENNMI_NEURON_BULK", "4" if per_lane == 4 else "0")
+    monkeypatch.setenv("GENNMI_RESIDENT", "0")
+    n = (blocks - 1) * 256 * per_lane + 3
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.55, TauRefrac=2.0)
+    v = np.random.default_rng(blocks).uniform(-60.0, -50.0, n).astype(np.float32)
+
+    def run(steps):
+        model = GeNNModel("float", "wait", dt=1.0)
+        model.add_neuron_population("N", n, "LIF", lif, {"V": v, "RefracTime": 0.0})
+        model.build()
+        model.load()
+        assert model.runner_info()["neuron_blocks"] == blocks
+        try:
+            model.run(steps)
+            model.synchronize()
+        finally:
+            model.unload()
+
+    monkeypatch.setenv("GENNMI_SPIN_LIMIT", "0")
+    with pytest.raises(GennmiError, match="bounded wait"):
+        run(500)
+    # the bound is per process: restore the default for whatever runs next
+    monkeypatch.delenv("GENNMI_SPIN_LIMIT")
+    run(100)
+
+
 # a row's parts are read by neighbouring lanes whatever number of them a spike is given: one lane a spike took 1.5 times as long as eight when its row's
 # synapses were dealt to the work-groups one by one (their cache lines are then fetched by as many of them)
 def test_one_lane_a_spike_reads_rows_as_well_as_eight_do(monkeypatch):
