@@ -82,22 +82,33 @@ void pullSpikesKernel(const uint32_t *spkCnt, const uint32_t *spk, uint32_t numN
     signalWhenLast(counter, flag, seq);
 }
 
+// Elements ahead of the first that lies on 16 bytes in both arrays (all of them: there is none)
+__host__ __device__ __forceinline__ size_t copyHead(const float *dst, const float *src, size_t n)
+{
+    const uintptr_t to = reinterpret_cast<uintptr_t>(dst), from = reinterpret_cast<uintptr_t>(src);
+    if(((to ^ from) & 15) || (to & 3)) { return n; }
+    return std::min<size_t>(n, ((16 - (to & 15)) & 15) / 4);
+}
+
 __global__ __launch_bounds__(BLOCK)
 void copySignalKernel(float *dst, const float *src, size_t n, uint32_t *counter, uint32_t *flag, uint32_t seq)
 {
-    const size_t threads = (size_t)gridDim.x * BLOCK;
-    const bool aligned = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
-    const size_t quads = aligned ? n / 4 : 0;
-    const u32x4 *from = reinterpret_cast<const u32x4*>(src);
-    u32x4 *to = reinterpret_cast<u32x4*>(dst);
-    for(size_t k = (size_t)blockIdx.x * BLOCK + threadIdx.x; k < quads; k += 4 * threads) {
-        u32x4 v[4];
-        #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) { v[u] = from[min(k + u * threads, quads - 1)]; }
-        #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) { if(k + u * threads < quads) { storeThrough(to + k + u * threads, v[u]); } }
-    }
-    for(size_t k = quads * 4 + (size_t)blockIdx.x * BLOCK + threadIdx.x; k < n; k += threads) { storeThrough(dst + k, src[k]); }
+    const size_t threads = (size_t)gridDim.x * BLOCK, thread = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    // `count` elements, four of them under way a thread
+    auto copy = [&](auto *to, const auto *from, size_t count) {
+        for(size_t k = thread; k < count; k += 4 * threads) {
+            std::remove_const_t<std::remove_reference_t<decltype(*from)>> v[4];
+            #pragma unroll
+            for(uint32_t u = 0; u < 4; u++) { v[u] = from[min(k + u * threads, count - 1)]; }
+            #pragma unroll
+            for(uint32_t u = 0; u < 4; u++) { if(k + u * threads < count) { storeThrough(to + k + u * threads, v[u]); } }
+        }
+    };
+    // quads from the first 16-byte boundary on, where both sides have theirs at the same element
+    const size_t head = copyHead(dst, src, n), quads = (n - head) / 4, done = head + 4 * quads;
+    copy(reinterpret_cast<u32x4*>(dst + head), reinterpret_cast<const u32x4*>(src + head), quads);
+    copy(dst, src, head);
+    copy(dst + done, src + done, n - done);
     signalWhenLast(counter, flag, seq);
 }
 
@@ -419,11 +430,16 @@ int copyOnDevice(float *dst, const float *src, size_t count, hipStream_t stream)
     }
     uint32_t slot;
     { const int rc = nextSlot(lease.ring, stream, &slot); if(rc) { return rc; } }
-    // Four quads a thread, and no more work-groups than keep memory busy: each ends with an addition to one counter, one after the other, 8 ns
-    // each.  us a copy with 2048 / 1024 / 512 / 256 / 128 at most: 300,000 floats 12.0 / 11.8 / 12.0 / 11.4 / 10.1, 10^6 19.8 / 19.5 / 14.2 / 11.6 / 11.0,
-    // 2.1 x 10^6 32.1 / 20.4 / 15.0 / 13.0 / 13.4, 8 x 10^6 34.6 / 23.8 / 18.7 / 19.1 / 25.9, 10^8 175 / 150 / 149 / 201 / 354.
-    const size_t most = (count > (size_t(1) << 22)) ? 512 : 256;
-    const uint32_t blocks = (uint32_t)std::min<size_t>(most, (count + 16 * BLOCK - 1) / (16 * BLOCK));
+    // Four quads (elements, where there are no quads) a thread, and no more work-groups than keep memory busy: each ends with an addition to one
+    // counter, one after the other, 8 ns each.  Up to 64 work-groups a thread has one of them (30,000 floats 16.4 -> 15.6 us a call).  us a copy
+    // with 2048 / 1024 / 512 / 256 / 128 at most: 300,000 floats 12.0 / 11.8 / 12.0 / 11.4 / 10.1, 10^6 19.8 / 19.5 / 14.2 / 11.6 / 11.0, 2.1 x 10^6 32.1
+    // / 20.4 / 15.0 / 13.0 / 13.4, 8 x 10^6 34.6 / 23.8 / 18.7 / 19.1 / 25.9, 10^8 175 / 150 / 149 / 201 / 354.  us a call without quads with 2048 / 1024
+    // / 512 / 256: 10^6 - / 26.8 / 21.8 / 19.5, 2.1 x 10^6 - / 27.9 / 23.0 / 21.8, 8 x 10^6 42.7 / 32.9 / 31.6 / -, 10^8 169 / 160 / 227 / -; with 2048 and
+    // one element a thread under way 27.2, 39.6, 44.0 and 180, with 512 48 and 571 for the last two.
+    const bool quads = copyHead(dst, src, count) < count;
+    const size_t most = (count <= (size_t(1) << 22)) ? 256 : (quads ? 512 : 1024);
+    const size_t one = ((quads ? (count + 3) / 4 : count) + BLOCK - 1) / BLOCK;
+    const uint32_t blocks = (uint32_t)std::min<size_t>(most, std::max<size_t>(std::min<size_t>(one, 64), (one + 3) / 4));
     copySignalKernel<<<dim3(blocks), dim3(BLOCK), 0, stream>>>(dst, src, count, lease.ring->counters + slot, lease.ring->flag(slot), lease.ring->seq[slot] + 1);
     HIP_TRY(hipGetLastError());
     lease.ring->seq[slot]++;
