@@ -1152,25 +1152,38 @@ void presynapticConvMfmaKernel(const ConvMfmaDev * __restrict__ blocks, uint32_t
 
 // Bitmap of a population's spike queue, for callers that wrote the queue themselves (the neuron update keeps it otherwise).  A work-group
 // owns BITMAP_WORDS words and looks through the whole queue for them: no word is added to from two sides, and clearing and setting are one launch.
-// A queue is empty or holds a few per cent of the population; one that names all of 10^6 neurons is read by 31 work-groups, 4 MB each.
+// Bound by the trips a work-group makes through the queue, so 16 entries a thread are under way.  us for a count pushed and 8 steps, two launches
+// -> four entries under way -> 16: 10^6 neurons, 0 / 10,000 / 100,000 / all of them in the queue 130 -> 127 -> 127, 155 -> 146 -> 143, 161 -> 168 -> 144
+// and 230 -> 287 -> 214; 100,000 neurons, 1000 / all 86 -> 80 -> 79 and 100 -> 113 -> 90.
 constexpr uint32_t BITMAP_WORDS = 1024;
 __global__ __launch_bounds__(BITMAP_WORDS)
 void spikeBitmapFromQueueKernel(const uint32_t *spkCnt, const uint32_t *spk, uint32_t *bitmap, uint32_t numNeurons)
 {
+    constexpr uint32_t QUADS = 4;
     __shared__ uint32_t shWords[BITMAP_WORDS];
     const uint32_t batch = blockIdx.y, words = (numNeurons + 31) / 32, first = blockIdx.x * BITMAP_WORDS;
     const uint32_t count = min(spkCnt[batch], numNeurons);
-    const uint32_t *queue = spk + (size_t)batch * numNeurons;
+    GLOBAL_AS const uint32_t *queue = asGlobal(spk) + (size_t)batch * numNeurons;
     shWords[threadIdx.x] = 0u;
     __syncthreads();
-    for(uint32_t k = threadIdx.x; k < count; k += 4 * BITMAP_WORDS) {
-        uint32_t id[4];
-        #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) { id[u] = queue[min(k + u * BITMAP_WORDS, count - 1)]; }
-        #pragma unroll
-        for(uint32_t u = 0; u < 4; u++) {
-            const uint32_t word = (id[u] >> 5) - first;
-            if(word < BITMAP_WORDS) { atomicOr(&shWords[word], 1u << (id[u] & 31)); }
+    auto set = [&](uint32_t id) {
+        const uint32_t word = (id >> 5) - first;
+        if(word < BITMAP_WORDS) { atomicOr(&shWords[word], 1u << (id & 31)); }
+    };
+    if(count < 4) {
+        if(threadIdx.x < count) { set(queue[threadIdx.x]); }
+    }
+    else {
+        for(uint32_t k = 4 * threadIdx.x; k < count; k += QUADS * 4 * BITMAP_WORDS) {
+            // (a quad beyond the last stands for the last: it sets the same bits again)
+            u32x4u ids[QUADS];
+            #pragma unroll
+            for(uint32_t u = 0; u < QUADS; u++) { ids[u] = *reinterpret_cast<GLOBAL_AS const u32x4u*>(queue + min(k + u * 4 * BITMAP_WORDS, count - 4)); }
+            #pragma unroll
+            for(uint32_t u = 0; u < QUADS; u++) {
+                #pragma unroll
+                for(uint32_t j = 0; j < 4; j++) { set(ids[u][j]); }
+            }
         }
     }
     __syncthreads();

@@ -314,6 +314,37 @@ def test_a_queue_cut_short_between_runs(n, monkeypatch):
     assert np.array_equal(got[0][0], got[1][0])
 
 
+# fewer entries than a quad, quads that the queue's end cuts, a round of all threads' quads and one more entry, several rounds; one word, several work-groups'
+# words; a second batch's queue off 16 bytes
+@pytest.mark.parametrize("n, counts", [(3, (0, 1, 2, 3)), (7, (3, 4, 5, 7)), (33001, (1, 4098, 16384, 16385, 33001)), (70001, (65537, 70001))])
+def test_a_queue_written_in_any_order(n, counts, monkeypatch):
+    got = []
+    for ahead in ("1", "0"):
+        monkeypatch.setenv("GENNMI_AHEAD", ahead)
+        net = _net("dense", (n, 3), 40)
+        source = net.pop("In")
+        source.spike_times = np.zeros(1, np.float32)
+        source.vars = {"startSpike": np.zeros(n, np.uint32), "endSpike": np.zeros(n, np.uint32)}
+        model = model_from_net(net, batch_size=2)
+        model.load(num_recording_timesteps=40)
+        assert model.runner_info()["feed_forward_ahead"] == (ahead == "1")
+        source = model.neuron_populations["In"]
+        rng, states = np.random.default_rng(n), []
+        for count in counts:
+            source.vars["spk"].view.reshape(2, n)[:] = [rng.permutation(n), rng.permutation(n)]
+            source.vars["spkCnt"].view[:] = [count, n - count]
+            source.vars["spk"].push_to_device()
+            source.vars["spkCnt"].push_to_device()
+            events = model.synaptic_event_count
+            model.run(8)
+            states.append(model.neuron_populations["Out"].vars["V"].pull_from_device().copy())
+            assert model.synaptic_event_count - events == 3 * n
+        got.append(states)
+        model.unload()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
 # one, two and four words of rows a work-group; chunks of 64 sources without a spike at the beginning, between others, at the end and throughout
 @pytest.mark.parametrize("steps", [20, 40, 100])
 @pytest.mark.parametrize("active", [(), (0,), (1999,), (700, 701, 1290), tuple(range(512, 600)) + (1500,), tuple(range(0, 2000, 63))])
