@@ -170,6 +170,47 @@ def test_steps_around_the_tile_path_s_threshold(m, fan, at):
     model.unload()
 
 
+# the line at four events per target, at 49,152 events, at one event per target; at one per target too for projections with segment records (rows of 10
+# synapses) and where the tile size is given
+@pytest.mark.parametrize("wum", ["static", "stdp_trace", "stdp_additive"])
+@pytest.mark.parametrize("m, fan, at, tile_floats", [(1, 1, 4, None), (1000, 40, 4000, None), (20000, 80, 49152, None), (60000, 600, 60000, None), (1000, 10, 1000, None), (1000, 40, 1000, "512")])
+def test_which_steps_the_tile_path_takes(m, fan, at, tile_floats, wum, monkeypatch):
+    """Into inputs of 2^24 a single weight of 1 is rounded away: what the scatter path adds one by one leaves no trace, what the tile path adds up first
+    does.  One spike fewer than the line asks for, and as many."""
+    from genn_amd.netspec import Net, Pop, Syn
+    from genn_amd import netgen
+    if tile_floats:
+        monkeypatch.setenv("GENNMI_TILE_FLOATS", tile_floats)
+    if (m, fan) == (1000, 10) and wum != "static":
+        at = 4 * m              # (plastic projections have no records)
+    n = (at + fan - 1) // fan
+    net = Net(name="line", dt=1.0, steps=12)
+    times = [[2.0] * (i < n - 1) + [5.0] for i in range(n)]        # (all but one of the neurons in step 2, all in step 5)
+    end = np.cumsum([len(t) for t in times]).astype(np.uint32)
+    net.pops.append(Pop("A", "ssa", n, {}, {"startSpike": np.concatenate([[0], end[:-1]]).astype(np.uint32), "endSpike": end}, spike_times=np.concatenate(times).astype(np.float32)))
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=1e9, Ioffset=0.0, TauRefrac=2.0)
+    net.pops.append(Pop("B", "lif", m, lif, {"V": np.full(m, -60.0, np.float32), "RefracTime": np.zeros(m, np.float32)}))
+    rl, ind = netgen.fixed_number_post(7, 3, n, m, fan)
+    rule = {} if wum == "static" else dict(tauPlus=20.0, tauMinus=20.0, aPlus=0.0, aMinus=0.0, wMin=0.0, wMax=1.0)
+    net.syns.append(Syn("AB", "A", "B", wum=wum, wum_params=rule, psm="deltacurr", row_stride=fan, row_length=rl, ind=ind, g=np.ones((n, fan), np.float32)))
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=12)
+    inputs = model.synapse_populations["AB"].vars["outPost"]
+    added = {}
+    for step in range(8):
+        inputs.view[:] = 2.0 ** 24
+        inputs.push_to_device()
+        model.update_synapses()
+        left = inputs.pull_from_device().copy()
+        if step in (3, 6):
+            added[step] = float(np.max(left)) - 2.0 ** 24
+        inputs.view[:] = 0.0
+        inputs.push_to_device()
+        model.update_neurons()
+    assert added[3] == 0.0 and added[6] >= 2.0, added
+    model.unload()
+
+
 def test_izhikevich_fanout_noise():
     """C3 shape: Izhikevich neurons, fixed fanout with replacement (multapses), DeltaCurr input,
     per-step noise current from a pregenerated array.  dt = 1 ms, first 100 ms = 100 steps."""
