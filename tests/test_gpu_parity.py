@@ -211,6 +211,53 @@ def test_which_steps_the_tile_path_takes(m, fan, at, tile_floats, wum, monkeypat
     model.unload()
 
 
+@pytest.mark.parametrize("wum", ["static", "stdp_trace"])
+def test_as_many_spikes_as_sub_groups_of_the_tile_kernel(wum, monkeypatch):
+    """A sub-group with one spike takes two parts of its row's segment at a time, one with more of them two spikes' segments: as many spikes as
+    sub-groups, one fewer, one more, twice as many and one more.  Segments of up to 60 synapses around the 32 of a round."""
+    import torch
+    from genn_amd.netspec import Net, Pop, Syn
+    from genn_amd import netgen
+    for name, value in (("TILE_FLOATS", "64"), ("TILE_THREADS", "64"), ("TILE_LANES", "4"), ("TILE_RECORDS", "0"), ("TILE_FACTORS", "0")):
+        monkeypatch.setenv("GENNMI_" + name, value)
+    m, fan, tiles = 2560, 1200, 40
+    splits = min(256, 4 * torch.cuda.get_device_properties(0).multi_processor_count * 256 // 64 // tiles)
+    stride = (64 // 4) * splits
+    n = 2 * stride + 1
+    net = Net(name="alone", dt=1.0, steps=16)
+    times = [[t for t, most in ((2.0, stride - 1), (4.0, stride), (6.0, stride + 1), (8.0, 2 * stride), (10.0, n)) if i < most] for i in range(n)]
+    end = np.cumsum([len(t) for t in times]).astype(np.uint32)
+    net.pops.append(Pop("A", "ssa", n, {}, {"startSpike": np.concatenate([[0], end[:-1]]).astype(np.uint32), "endSpike": end}, spike_times=np.concatenate(times).astype(np.float32)))
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.8, TauRefrac=2.0)
+    v0 = (-60.0 + 10.0 * ((np.arange(m) * 29) % 101) / 101.0).astype(np.float32)
+    net.pops.append(Pop("B", "lif", m, lif, {"V": v0, "RefracTime": np.zeros(m, np.float32)}))
+    rl, ind = netgen.fixed_number_post(7, 3, n, m, fan)
+    rl[::7] = (rl[::7] * 2) // 3
+    if wum == "static":
+        rule, g = {}, ((np.arange(n * fan) % 9 - 3).astype(np.float32) / 64.0).reshape(n, fan)
+    else:           # (weights too small to move a spike, whatever order they are added in)
+        rule, g = dict(tauPlus=20.0, tauMinus=20.0, aPlus=1e-9, aMinus=1.2e-9, wMin=0.0, wMax=1e-8), netgen.rows_uniform(7, 4, rl, fan, n, 1e-8, 0.0, 1e-8, 0.0)
+    net.syns.append(Syn("AB", "A", "B", wum=wum, wum_params=rule, psm="deltacurr", row_stride=fan, row_length=rl, ind=ind, g=g))
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=16)
+    plastic = {} if wum == "static" else {"col_stride": {"AB": model.synapse_populations["AB"].col_stride}}
+    oracle = OracleNet(net, num_recording_timesteps=16, **plastic)
+    model.run(16)
+    oracle.run(16)
+    model.pull_recording_buffers_from_device()
+    for p in net.pops:
+        words = (p.n + 31) // 32
+        assert np.array_equal(model.neuron_populations[p.name].vars["recordSpk"].view.reshape(16, words), oracle.record(p.name, 16).reshape(16, words)), p.name
+    assert model.synaptic_event_count == oracle.events()
+    if wum == "static":
+        compare_state(net, model, oracle, "after 16 steps", exact=True)
+    else:
+        got, want = model.synapse_populations["AB"].vars["g"].pull_from_device().reshape(n, -1)[:, :fan], oracle.syn_g("AB").reshape(n, -1)[:, :fan]
+        inside = np.arange(fan)[None, :] < rl[:, None]
+        assert np.max(np.abs(got - want)[inside]) <= 2e-7 * 1e-8 and (np.abs(want - g)[inside] > 0.0).any()
+    model.unload()
+
+
 def test_izhikevich_fanout_noise():
     """C3 shape: Izhikevich neurons, fixed fanout with replacement (multapses), DeltaCurr input,
     per-step noise current from a pregenerated array.  dt = 1 ms, first 100 ms = 100 steps."""
