@@ -1732,12 +1732,14 @@ int gennmi_runner_finalise(gennmi_runner *r)
             uint16_t *dOff = offsets[candidate++].off;
             if(unsorted) { continue; }          // rows not sorted by target: the scatter kernel handles every step
             // Events from which a step goes to the tiles: one per target, but 49,152 (scattered one by one, 2 us) if that is more, and then no more
-            // than four per target (additions to one address follow each other).  us of synapse kernels with one per target -> now: 400
-            // steps of plastic networks 6,000 x 100 3604 -> 2395, 17,011 x 300 2234 -> 2147, 80 of Izhikevich networks 30,000 x 300 696 -> 665,
-            // 12,000 x 500 647 -> 602.  (Half a one per target: balanced 300,000 x 1000 1810 -> 1723 but the steps of a pass no faster.)  Projections with
-            // records, and where the tile size is given: one per target.
+            // than two per target, four where weights change (additions to one address follow each other; a plastic tile step costs more).  us of synapse
+            // kernels with one per target -> now: 400 steps of plastic networks 6,000 x 100 3604 -> 2395, 17,011 x 300 2234 -> 2147.  us a step at 1.2 events per
+            // target and at 2.6, with one / two / four: 10,000 static x 100 11.3 / 10.5 / 10.5 and 10.5 / 10.5 / 11.6, 3,000 x 100 10.0 / 10.0 / 10.0 and
+            // 9.6 / 9.6 / 10.5; plastic, one / four: 10,000 x 100 15.9 / 11.8 and 14.2 / 12.5, 3,000 x 100 13.5 / 10.7 and 12.8 / 11.8.  (Half a one per target:
+            // balanced 300,000 x 1000 1810 -> 1723 but the steps of a pass no faster.)  Projections with records, and where GENNMI_TILE_FLOATS gives the
+            // tile size (which tests do to reach the tiles with small networks): one per target.
             p.tileThreshold = std::max(1u, p.g.numTrgNeurons);
-            if(!envTile) { p.tileThreshold = std::max(p.tileThreshold, (uint32_t)std::min<uint64_t>(49152, 4ull * p.g.numTrgNeurons)); }
+            if(!envTile) { p.tileThreshold = std::max(p.tileThreshold, (uint32_t)std::min<uint64_t>(49152, (p.g.wum == GENNMI_WUM_STATIC_PULSE ? 2ull : 4ull) * p.g.numTrgNeurons)); }
             r->tileTables.push_back({(size_t)(&p - r->pre.data()), dOff, tileSize, numTiles});
             const uint32_t avgSeg = std::max(1u, p.g.rowStride / numTiles);
             TileGroupDev t{};

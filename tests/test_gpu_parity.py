@@ -147,8 +147,8 @@ def test_busy_steps_of_ragged_plastic_rows(n, m, fan, rule, factors, monkeypatch
     model.unload()
 
 
-# four events per target; 49,152 events; one event per target: steps on either side of each
-@pytest.mark.parametrize("m, fan, at", [(1, 1, 4), (1000, 40, 4000), (20000, 80, 49152), (150000, 800, 150000)])
+# two and four events per target; 49,152 events; one event per target: steps on either side of each
+@pytest.mark.parametrize("m, fan, at", [(1, 1, 4), (1000, 40, 4000), (20000, 80, 49152), (150000, 800, 150000), (1, 1, 2), (1000, 40, 2000), (30000, 80, 49152)])
 def test_steps_around_the_tile_path_s_threshold(m, fan, at):
     """As many events as send a step to the tile kernel, one spike more and one fewer: both paths add the same multiples of 2^-3."""
     from genn_amd.netspec import Net, Pop, Syn
@@ -170,20 +170,19 @@ def test_steps_around_the_tile_path_s_threshold(m, fan, at):
     model.unload()
 
 
-# the line at four events per target, at 49,152 events, at one event per target; at one per target too for projections with segment records (rows of 10
-# synapses) and where the tile size is given
+# the line at two events per target (four where weights change), at 49,152 events, at one event per target; at one per target too for projections with
+# segment records (static rows of 10 synapses) and where the tile size is given
 @pytest.mark.parametrize("wum", ["static", "stdp_trace", "stdp_additive"])
-@pytest.mark.parametrize("m, fan, at, tile_floats", [(1, 1, 4, None), (1000, 40, 4000, None), (20000, 80, 49152, None), (60000, 600, 60000, None), (1000, 10, 1000, None), (1000, 40, 1000, "512")])
-def test_which_steps_the_tile_path_takes(m, fan, at, tile_floats, wum, monkeypatch):
+@pytest.mark.parametrize("m, fan, static, plastic, tile_floats", [(1, 1, 2, 4, None), (1000, 40, 2000, 4000, None), (20000, 80, 40000, 49152, None), (30000, 80, 49152, 49152, None),
+                                                                  (60000, 600, 60000, 60000, None), (1000, 10, 1000, 4000, None), (1000, 40, 1000, 1000, "512")])
+def test_which_steps_the_tile_path_takes(m, fan, static, plastic, tile_floats, wum, monkeypatch):
     """Into inputs of 2^24 a single weight of 1 is rounded away: what the scatter path adds one by one leaves no trace, what the tile path adds up first
     does.  One spike fewer than the line asks for, and as many."""
     from genn_amd.netspec import Net, Pop, Syn
     from genn_amd import netgen
     if tile_floats:
         monkeypatch.setenv("GENNMI_TILE_FLOATS", tile_floats)
-    if (m, fan) == (1000, 10) and wum != "static":
-        at = 4 * m              # (plastic projections have no records)
-    n = (at + fan - 1) // fan
+    n = ((static if wum == "static" else plastic) + fan - 1) // fan
     net = Net(name="line", dt=1.0, steps=12)
     times = [[2.0] * (i < n - 1) + [5.0] for i in range(n)]        # (all but one of the neurons in step 2, all in step 5)
     end = np.cumsum([len(t) for t in times]).astype(np.uint32)
