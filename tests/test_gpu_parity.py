@@ -107,10 +107,11 @@ def test_tile_path_segment_records(m, fan, tile_floats, records, monkeypatch):
 
 
 # rows of fewer synapses than a quad (the last one ends the matrix), of more than a wavefront takes at once, more rows than a wavefront looks at at once,
+# rows that share a wavefront (of 2, 10, 16 and 32 quads),
 # a matrix smaller than a quad; several tiles, and what the rule takes off kept beside the tile or not
 @pytest.mark.parametrize("factors", ["0", "2"])
 @pytest.mark.parametrize("rule", ["stdp_trace", "stdp_additive"])
-@pytest.mark.parametrize("n, m, fan", [(64, 300, 3), (5003, 40, 37), (300, 1500, 1203), (2, 1, 1), (700, 900, 130)])
+@pytest.mark.parametrize("n, m, fan", [(64, 300, 3), (5003, 40, 37), (300, 1500, 1203), (2, 1, 1), (700, 900, 130), (5003, 40, 5), (3001, 500, 61), (1500, 600, 128)])
 def test_busy_steps_of_ragged_plastic_rows(n, m, fan, rule, factors, monkeypatch):
     """Every step with spikes walks the rows on both sides; weights, rasters and event counts must be the oracle's."""
     from genn_amd.netspec import Net, Pop, Syn

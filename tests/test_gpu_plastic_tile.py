@@ -49,3 +49,30 @@ def test_weights_are_the_same_with_and_without(rule, tile_floats, n, monkeypatch
         assert np.array_equal(g.reshape(-1)[valid], got[0][0].reshape(-1)[valid])
         assert np.abs(g.reshape(-1)[valid] - want).max() <= 1e-5
     assert (np.abs(want - np.asarray(ee.g).reshape(-1)[valid]) > 1e-3).mean() > 0.5
+
+
+def test_short_rows_are_walked_about_as_fast_as_long_ones():
+    """A burst of the targets walks every row.  Three million synapses in rows of 30 took 10 times as long as in rows of 300 when a wavefront looked at
+    rows far apart and took two of them at a time, whatever their length."""
+    from genn_amd.genn_model import GeNNModel, init_postsynaptic, init_sparse_connectivity, init_var, init_weight_update
+    m, took = 1000, {}
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, TauRefrac=5.0)
+    rule = dict(tauPlus=20.0, tauMinus=20.0, aPlus=1e-6, aMinus=1e-6, wMin=0.0, wMax=1.0)
+    for n, fan in ((100000, 30), (10000, 300)):
+        model = GeNNModel("float", "rows", dt=0.5)
+        model.seed, model.timing_enabled = 7, True
+        a = model.add_neuron_population("A", n, "LIF", dict(lif, Ioffset=0.0), {"V": -60.0, "RefracTime": 0.0})
+        b = model.add_neuron_population("B", m, "LIF", dict(lif, Ioffset=4.0), {"V": init_var("Uniform", {"min": -60.0, "max": -50.0}), "RefracTime": 0.0})
+        model.add_synapse_population("AB", "SPARSE", a, b, init_weight_update("STDPTrace", rule, {"g": init_var("Uniform", {"min": 0.0, "max": 0.5})}, {"preTrace": 0.0}, {"postTrace": 0.0}),
+                                     init_postsynaptic("ExpCurr", {"tau": 5.0}), init_sparse_connectivity("FixedNumberPostWithReplacement", {"num": fan}))
+        model.build()
+        model.load()
+        rounds = []
+        for _ in range(5):
+            before = model.postsynaptic_update_time
+            for _ in range(40):
+                model.step_time()
+            rounds.append(model.postsynaptic_update_time - before)
+        took[n] = min(rounds)
+        model.unload()
+    assert 0.0 < took[100000] < 4.0 * took[10000], took
