@@ -59,11 +59,9 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
     // a wavefront stay neighbours: with few lanes a spike they read neighbouring parts of one row.  us a step with wavefronts numbered block by
     // block / sub-groups across the blocks / as here, about 3 % of 10,000 and of 100,000 neurons x 1000 spiking, one lane a spike: 19.3 / 29.6 / 19.3
     // and 138 / 153 / 138, 100,000 x 100 with 1, 2 and 4 lanes 22.3 / 25.3 / 22.4, 22.3 / 24.1 / 22.4 and 22.3 / 23.4 / 22.4.
-    // A convolution's are numbered block by block: a work-group's wavefronts then take neighbouring parts of one spike's kernel, which every spike
-    // reads again (steps in which all of 4 x 2,880 inputs of a 12x12x20 -> 40 5x5 layer spike 66.5 -> 63.8 us).
-    const uint32_t wavefront = (g.matrix == GENNMI_MATRIX_TOEPLITZ_CONV2D) ? localBlock * (blockDim.x / WAVE) + threadIdx.x / WAVE : (threadIdx.x / WAVE) * G.numBlocks + localBlock;
-    const uint32_t subGroup = wavefront * (WAVE / W) + (threadIdx.x & (WAVE - 1)) / W;
-    const uint32_t numSubGroups = (G.numBlocks * blockDim.x) / W;
+    const uint32_t shift = (uint32_t)__ffs((int)W) - 1u;        // (W is a power of two; divisions by it are on the way to the first spike)
+    const uint32_t subGroup = ((((threadIdx.x / WAVE) * G.numBlocks + localBlock) * WAVE) >> shift) + ((threadIdx.x & (WAVE - 1)) >> shift);
+    const uint32_t numSubGroups = (G.numBlocks * blockDim.x) >> shift;
     // spikes of the previous step: the population's own queue, or (when this launch may run next to the
     // neuron update that refills that queue) the shadow copy written one step ago
     const uint32_t parity = (uint32_t)((st.epoch + 1) & 1);
@@ -93,10 +91,13 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
         const uint32_t numDiag = (uint32_t)(kh * kw * oc);
         const uint32_t chunksPerRow = (numDiag + W - 1) / W;
         GLOBAL_AS const float *kernel = asGlobal(g.g);
-        // item = subGroup + k*numSubGroups, split into (spike, chunk) incrementally: no division in the loop
+        // numbered block by block: a work-group's wavefronts then take neighbouring parts of one spike's kernel, which every spike reads again (steps in
+        // which all of 4 x 2,880 inputs of a 12x12x20 -> 40 5x5 layer spike 66.5 -> 64.8 us).
+        const uint32_t along = (localBlock * blockDim.x + threadIdx.x) >> shift;
+        // item = along + k*numSubGroups, split into (spike, chunk) incrementally: no division in the loop
         const uint32_t stepSpike = numSubGroups / chunksPerRow, stepChunk = numSubGroups % chunksPerRow;
-        uint32_t chunk = subGroup % chunksPerRow;
-        for(unsigned long long s = subGroup / chunksPerRow; s < numSpikes; ) {
+        uint32_t chunk = along % chunksPerRow;
+        for(unsigned long long s = along / chunksPerRow; s < numSpikes; ) {
             const uint32_t j = chunk * W + lis;
             const uint32_t ipre = spk[s];
             s += stepSpike; chunk += stepChunk;
