@@ -112,6 +112,7 @@ __device__ __forceinline__ void publishBlockCount(uint32_t blockCount, uint32_t 
         __hip_atomic_store(&counts[aggBase + localBlock], ((unsigned long long)tag << 32) | blockCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
+template<bool DIRECT = true>
 __device__ __forceinline__ uint32_t blockQueueOffset(uint32_t blockCount, uint32_t localBlock, uint32_t numBlocks, size_t aggBase,
                                                     unsigned long long *counts, unsigned long long *groupTotals, uint32_t tag,
                                                     uint32_t *shOffset, uint32_t *errorFlag, bool published = false)
@@ -122,7 +123,7 @@ __device__ __forceinline__ uint32_t blockQueueOffset(uint32_t blockCount, uint32
         __hip_atomic_store(&counts[aggBase + localBlock], ((unsigned long long)tag << 32) | blockCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const bool last = (localBlock == numBlocks - 1);
-    if(queueDirect(numBlocks)) {
+    if(DIRECT && queueDirect(numBlocks)) {
         // (a block without spikes that is not the last needs no offset)
         return (blockCount != 0 || last) ? sumOfEarlierBlocks(localBlock, counts + aggBase, tag, errorFlag) : 0u;
     }
@@ -169,6 +170,7 @@ __device__ __forceinline__ uint32_t blockQueueOffset(uint32_t blockCount, uint32
 // with the step, blocks in groups of 64 with a published group total), as a function every block of the population
 // calls with all its threads.  `counts` and `groupTotals` hold one entry per (batch, neuron block of the launch).
 // ------------------------------------------------------------------------------------------------
+template<bool DIRECT = true>
 __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t localBlock, uint32_t numBlocks, size_t aggBase,
                                               unsigned long long *counts, unsigned long long *groupTotals, uint32_t tag,
                                               uint32_t *queue, uint32_t *queueCount, uint32_t *errorFlag,
@@ -191,7 +193,7 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
         if(w < wave) { waveOffset += c; }
         blockCount += c;
     }
-    const uint32_t prefix = blockQueueOffset(blockCount, localBlock, numBlocks, aggBase, counts, groupTotals, tag, &shOffset, errorFlag);
+    const uint32_t prefix = blockQueueOffset<DIRECT>(blockCount, localBlock, numBlocks, aggBase, counts, groupTotals, tag, &shOffset, errorFlag);
     if(prefix != 0xFFFFFFFFu) {
         if(flag) { queue[prefix + waveOffset + laneRank] = id; }
         if(localBlock == numBlocks - 1 && threadIdx.x == 0) { *queueCount = prefix + blockCount; }
@@ -365,7 +367,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
         const size_t perArea = (size_t)totalNeuronBlocks * gridDim.y;
         for(uint32_t e = 0; e < g.numSpkEvent; e++) {
             unsigned long long *counts = G.aggEvent + (size_t)e * 2 * perArea;
-            appendOrdered(i < n && vEvent > g.spkEvent[e].threshold, i, localBlock, G.numBlocks, (size_t)batch * totalNeuronBlocks + G.startBlock,
+            appendOrdered<DIRECT>(i < n && vEvent > g.spkEvent[e].threshold, i, localBlock, G.numBlocks, (size_t)batch * totalNeuronBlocks + G.startBlock,
                           counts, counts + perArea, (uint32_t)(st.epoch + 1), g.spkEvent[e].spkEvent + (size_t)batch * n,
                           g.spkEvent[e].spkCntEvent + batch, errorFlag,
                           g.spkEvent[e].recordSpkEvent ? g.spkEvent[e].recordSpkEvent + ((size_t)st.recordingTimestep * gridDim.y + batch) * ((n + 31) / 32) : nullptr, i < n);
@@ -759,7 +761,8 @@ void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t 
         // the neuron blocks are the critical path (other blocks wait for their spike counts): let their
         // instructions issue ahead of the presynaptic blocks that share the compute unit
         __builtin_amdgcn_s_setprio(3);
-        // (offsets in two levels: 50 steps of the full microcircuit 562 us, with sumOfEarlierBlocks in this kernel 569; at 0.35 of it 682 either way)
+        // (offsets in two levels throughout: 50 steps of the full microcircuit 562 us, with sumOfEarlierBlocks in this kernel 569.  2000 steps of 0.35 of it
+        // 13.50 ms in this kernel before there was a sumOfEarlierBlocks, 13.66 with it for spike-like events only, which no step there has, 13.27 without)
         neuronBody<false>(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
     }
     else { presynapticBody(preBlocks[blockIdx.x - numNeuronBlocks], blockIdx.x - numNeuronBlocks, blockIdx.y, gridDim.y, st, dt, eventCounter); }
