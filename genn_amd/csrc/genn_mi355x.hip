@@ -1797,12 +1797,42 @@ int gennmi_runner_finalise(gennmi_runner *r)
             // 2276 / 2220 / 2163, 9,000 x 300 1969 / 1949 / 1982; 200 steps of the balanced network 300,007 x 1000 1852 / 1723 / 1696.
             const char *envPerSplit = getenv("GENNMI_TILE_SPIKES_PER_SPLIT");
             const uint32_t spikesPerSplit = envPerSplit ? (uint32_t)std::max(1, atoi(envPerSplit)) : 4096u;
-            double totalWeight = 0.0;
-            for(const auto &t : tileGroups) { totalWeight += (double)t.g.numSrcNeurons * t.g.rowStride; }
+            // Work-groups of a tile: as many as make the largest share of synapses any work-group has the smallest, within the budget (a launch ends with
+            // the work-group that has most: dealt out in proportion and rounded down, a projection of 1.8 work-groups a tile got one).  Where two rounds'
+            // shares come out more even, by a twentieth, it is two after all.  us of the longest step of a burst, two rounds rounded down / one rounded
+            // down / as here: Izhikevich 932,087 x 107 606 / 783 / 608 (one round as even as can be 660), 600,000 x 100 372 / 337 / 327, 500,000 x 300 160 / 162 / 155.
+            auto weight = [&](const TileGroupDev &t) { return (tileGroups.size() > 1 && t.recLanes ? 2.0 : 1.0) * (double)t.g.numSrcNeurons * t.g.rowStride; };
+            auto splitsOf = [&](const TileGroupDev &t, double most) { return (uint32_t)std::min(256.0, std::max(1.0, std::ceil(weight(t) / (t.numTiles * most)))); };
+            double totalWeight = 0.0, shared = 0.0;
+            for(const auto &t : tileGroups) { totalWeight += (double)t.g.numSrcNeurons * t.g.rowStride; shared += weight(t); }
+            auto leastShare = [&](double rounds) {
+                double fits = std::max(1.0, shared), tooSmall = 0.0;
+                for(int k = 0; k < 64; k++) {
+                    const double most = 0.5 * (fits + tooSmall);
+                    double blocks = 0.0;
+                    for(const auto &t : tileGroups) { blocks += (double)t.numTiles * splitsOf(t, most); }
+                    if(blocks <= rounds * budget * (shared / std::max(1.0, totalWeight))) { fits = most; } else { tooSmall = most; }
+                }
+                return fits;
+            };
+            double rounds = 1.0, fits = leastShare(1.0);
+            if(tileGroups.size() > 1 && shared == totalWeight) { const double two = leastShare(2.0); if(2.0 * two < 0.95 * fits) { rounds = 2.0; fits = two; } }
+            // (what the budget leaves goes to whoever's share is largest and has room for one more work-group a tile)
+            std::vector<uint32_t> splits;
+            double left = rounds * budget * (shared / std::max(1.0, totalWeight));
+            for(const auto &t : tileGroups) { splits.push_back(splitsOf(t, fits)); left -= (double)t.numTiles * splits.back(); }
+            while(true) {
+                size_t most = tileGroups.size();
+                auto share = [&](size_t k) { return weight(tileGroups[k]) / ((double)tileGroups[k].numTiles * splits[k]); };
+                for(size_t k = 0; k < tileGroups.size(); k++) {
+                    if(splits[k] < 256u && tileGroups[k].numTiles <= left && (most == tileGroups.size() || share(k) > share(most))) { most = k; }
+                }
+                if(most == tileGroups.size()) { break; }
+                splits[most]++;
+                left -= tileGroups[most].numTiles;
+            }
             for(auto &t : tileGroups) {
-                const double share = (tileGroups.size() == 1) ? 1.0 : (t.recLanes ? 2.0 : 1.0) * ((double)t.g.numSrcNeurons * t.g.rowStride) / totalWeight;
-                const uint32_t groupBudget = std::max(t.numTiles, (uint32_t)(share * budget));
-                const uint32_t numSplits = std::max(1u, std::min(256u, groupBudget / t.numTiles));
+                const uint32_t numSplits = splits[(size_t)(&t - tileGroups.data())];
                 t.numSplits = numSplits;
                 t.spikesPerSplit = spikesPerSplit;
                 // (worth it from one event per two targets of a block's tile)

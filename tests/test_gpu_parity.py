@@ -258,6 +258,29 @@ def test_as_many_spikes_as_sub_groups_of_the_tile_kernel(wum, monkeypatch):
     model.unload()
 
 
+# more tiles than work-groups; one projection of seven times the other's synapses a tile; a projection too small for a second work-group a tile; one of two
+# where two rounds' shares are the more even
+@pytest.mark.parametrize("sizes", [((3000, 40000, 60), (500, 40000, 50)), ((3000, 1000, 200), (500, 3000, 60)), ((5000, 2000, 100), (60, 30000, 700)), ((4000, 12000, 100), (1000, 12000, 100))])
+def test_projections_share_the_tile_kernel_s_work_groups(sizes, monkeypatch):
+    """However the work-groups are shared out, every synapse of a spike is added once (multiples of 1/64: sums are exact)."""
+    from genn_amd.netspec import Net, Pop, Syn
+    from genn_amd import netgen
+    monkeypatch.setenv("GENNMI_TILE_FLOATS", "64")
+    monkeypatch.setenv("GENNMI_TILE_RECORDS", "0")
+    lif = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=0.8, TauRefrac=2.0)
+    net = Net(name="shared", dt=1.0, steps=30)
+    for k, (n, m, fan) in enumerate(sizes):
+        for name, size in (("S", n), ("T", m)):
+            v0 = (-60.0 + 10.0 * ((np.arange(size) * 29) % 13) / 13.0).astype(np.float32)          # (a thirteenth of them in a step)
+            net.pops.append(Pop(f"{name}{k}", "lif", size, dict(lif), {"V": v0, "RefracTime": np.zeros(size, np.float32)}))
+        rl, ind = netgen.fixed_number_post(7, 3 + k, n, m, fan)
+        g = ((np.arange(n * fan) % 9 - 3).astype(np.float32) / 64.0).reshape(n, fan)
+        net.syns.append(Syn(f"P{k}", f"S{k}", f"T{k}", wum="static", psm="deltacurr", row_stride=fan, row_length=rl, ind=ind, g=g))
+    model, oracle, counts = run_side_by_side(net, check_every=5, exact=True)
+    assert all(counts[p.name] > p.n // 13 for p in net.pops) and model.synaptic_event_count == oracle.events()
+    model.unload()
+
+
 def test_izhikevich_fanout_noise():
     """C3 shape: Izhikevich neurons, fixed fanout with replacement (multapses), DeltaCurr input,
     per-step noise current from a pregenerated array.  dt = 1 ms, first 100 ms = 100 steps."""
