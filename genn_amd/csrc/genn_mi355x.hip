@@ -1801,12 +1801,17 @@ int gennmi_runner_finalise(gennmi_runner *r)
             // the work-group that has most: dealt out in proportion and rounded down, a projection of 1.8 work-groups a tile got one).  Where two rounds'
             // shares come out more even, by a twentieth, it is two after all.  us of the longest step of a burst, two rounds rounded down / one rounded
             // down / as here: Izhikevich 932,087 x 107 606 / 783 / 608 (one round as even as can be 660), 600,000 x 100 372 / 337 / 327, 500,000 x 300 160 / 162 / 155.
+            constexpr uint32_t MOST_SPLITS = 256;
             auto weight = [&](const TileGroupDev &t) { return (tileGroups.size() > 1 && t.recLanes ? 2.0 : 1.0) * (double)t.g.numSrcNeurons * t.g.rowStride; };
-            auto splitsOf = [&](const TileGroupDev &t, double most) { return (uint32_t)std::min(256.0, std::max(1.0, std::ceil(weight(t) / (t.numTiles * most)))); };
-            double totalWeight = 0.0, shared = 0.0;
-            for(const auto &t : tileGroups) { totalWeight += (double)t.g.numSrcNeurons * t.g.rowStride; shared += weight(t); }
+            auto splitsOf = [&](const TileGroupDev &t, double most) { return (uint32_t)std::min((double)MOST_SPLITS, std::max(1.0, std::ceil(weight(t) / (t.numTiles * most)))); };
+            double totalWeight = 0.0, shared = 0.0, least = 0.0;
+            for(const auto &t : tileGroups) {
+                totalWeight += (double)t.g.numSrcNeurons * t.g.rowStride;
+                shared += weight(t);
+                least = std::max(least, weight(t) / ((double)t.numTiles * MOST_SPLITS));        // (the others gain nothing by smaller shares than this)
+            }
             auto leastShare = [&](double rounds) {
-                double fits = std::max(1.0, shared), tooSmall = 0.0;
+                double fits = std::max(1.0, shared), tooSmall = least * (1.0 - 1e-9);
                 for(int k = 0; k < 64; k++) {
                     const double most = 0.5 * (fits + tooSmall);
                     double blocks = 0.0;
@@ -1825,7 +1830,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
                 size_t most = tileGroups.size();
                 auto share = [&](size_t k) { return weight(tileGroups[k]) / ((double)tileGroups[k].numTiles * splits[k]); };
                 for(size_t k = 0; k < tileGroups.size(); k++) {
-                    if(splits[k] < 256u && tileGroups[k].numTiles <= left && (most == tileGroups.size() || share(k) > share(most))) { most = k; }
+                    if(share(k) > least && tileGroups[k].numTiles <= left && (most == tileGroups.size() || share(k) > share(most))) { most = k; }
                 }
                 if(most == tileGroups.size()) { break; }
                 splits[most]++;

@@ -259,8 +259,8 @@ def test_as_many_spikes_as_sub_groups_of_the_tile_kernel(wum, monkeypatch):
 
 
 # more tiles than work-groups; one projection of seven times the other's synapses a tile; a projection too small for a second work-group a tile; one of two
-# where two rounds' shares are the more even
-@pytest.mark.parametrize("sizes", [((3000, 40000, 60), (500, 40000, 50)), ((3000, 1000, 200), (500, 3000, 60)), ((5000, 2000, 100), (60, 30000, 700)), ((4000, 12000, 100), (1000, 12000, 100))])
+# where two rounds' shares are the more even; one with as many work-groups as a tile may have
+@pytest.mark.parametrize("sizes", [((3000, 40000, 60), (500, 40000, 50)), ((20000, 60, 40), (800, 60, 40)), ((3000, 1000, 200), (500, 3000, 60)), ((5000, 2000, 100), (60, 30000, 700)), ((4000, 12000, 100), (1000, 12000, 100))])
 def test_projections_share_the_tile_kernel_s_work_groups(sizes, monkeypatch):
     """However the work-groups are shared out, every synapse of a spike is added once (multiples of 1/64: sums are exact)."""
     from genn_amd.netspec import Net, Pop, Syn
