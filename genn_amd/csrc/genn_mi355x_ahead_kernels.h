@@ -455,7 +455,7 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
         const uint32_t step = first + voteStep;
         if(voteLane && step < A.steps) {
             // (of the steps of this launch that share a recording row only the last writes it)
-            if(recordSpk && step + A.recordingRows >= A.steps) { recordSpk[(aheadRecordingRow(A, step) * A.batch + batch) * bitmapWords + voteWord] = votes; }
+            if(recordSpk && A.steps - step <= A.recordingRows) { recordSpk[(aheadRecordingRow(A, step) * A.batch + batch) * bitmapWords + voteWord] = votes; }
             if(step + 1 == A.steps) { lastBits[(size_t)batch * bitmapWords + voteWord] = votes; }
         }
     };
@@ -642,7 +642,7 @@ void aheadTransposeKernel(const NeuronGroupDev * __restrict__ target, AheadArgs 
         const uint32_t t = e / 32, word = blockIdx.x * 32 + e % 32, step = wordBlock * AHEAD_WORD + t;
         if(t >= steps || word >= bitmapWords) { continue; }
         // (of the steps of this launch that share a recording row only the last writes it)
-        if(g.recordSpk && t + A.recordingRows >= steps) { g.recordSpk[(aheadRecordingRow(A, step) * A.batch + batch) * bitmapWords + word] = rows[t][e % 32]; }
+        if(g.recordSpk && steps - t <= A.recordingRows) { g.recordSpk[(aheadRecordingRow(A, step) * A.batch + batch) * bitmapWords + word] = rows[t][e % 32]; }
         if(step + 1 == A.steps) { lastBits[(size_t)batch * bitmapWords + word] = rows[t][e % 32]; }
     }
 }

@@ -6,7 +6,7 @@ import copy
 import numpy as np
 import pytest
 
-from genn_amd import configs
+from genn_amd import _abi, configs
 from genn_amd.genn_model import model_from_net
 from oracle.genn_cpu import OracleNet
 from parity import compare_state
@@ -312,6 +312,21 @@ def test_a_queue_cut_short_between_runs(n, monkeypatch):
         model.unload()
     assert got[0][1] == got[1][1] == 3 * max(left - 3, left // 2)
     assert np.array_equal(got[0][0], got[1][0])
+
+
+@pytest.mark.parametrize("kind,shape", [("dense", (65, 33)), ("conv", (5, 7, 3, 4, 3))], ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_a_recording_buffer_of_almost_2_to_the_32_rows(kind, shape):
+    """The rows of a run that starts at step 0 are the first ones, however many there are said to be: steps and rows are not added up in 32 bits."""
+    steps = 40
+    net = _net(kind, shape, steps)
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=steps)
+    assert model.runner_info()["feed_forward_ahead"]
+    oracle = OracleNet(net, num_recording_timesteps=steps)
+    _abi.check(_abi.load().gennmi_run_steps(model._runner, 0, steps, 0xFFFFFFFF))
+    oracle.run(steps)
+    _same_rasters(net, model, oracle, steps)
+    model.unload()
 
 
 # fewer entries than a quad, quads that the queue's end cuts, a round of all threads' quads and one more entry, several rounds; one word, several work-groups'
