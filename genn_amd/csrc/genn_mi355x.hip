@@ -104,6 +104,7 @@ struct gennmi_runner
     uint32_t resQuads = 2;              // 16-byte quads of an entry
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
+    bool queuesDirect = false;          // a population's blocks sum the counts of all earlier ones (queueDirect)
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
     bool sourcesStale = false;          // startSpike / endSpike / spikeTimes of a spike source were written since nextSpikeTime was built
     bool failed = false;                // a queued step failed part-way: what was queued behind it is lost, the runner refuses to go on
@@ -1563,6 +1564,7 @@ int gennmi_runner_finalise(gennmi_runner *r)
         block += n.numBlocks;
     }
     r->neuronBlocks = block;
+    r->queuesDirect = std::any_of(r->neuron.begin(), r->neuron.end(), [](const NeuronGroupDev &n) { return queueDirect(n.numBlocks); });
 
 
     // DENSE / BITMASK projections: one lane per postsynaptic neuron; a group owns its outPost unless another dense or
@@ -2237,7 +2239,8 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed)
     if(r->neuronsPerLane == 2) { neuronBulkKernel<2><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
     else if(r->neuronsPerLane == 4) { neuronBulkKernel<4><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
     else if(r->neuronsPerLane == 8) { neuronBulkKernel<8><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
-    else { neuronUpdateKernel<<<dim3(r->neuronBlocks, r->batch), dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
+    else if(r->queuesDirect) { neuronUpdateKernel<true><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
+    else { neuronUpdateKernel<false><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
     if(timed) { const int rc = stamp(r, &e1); if(rc) { return rc; } r->pending.push_back({e0, e1, 2}); }
     HIP_TRY(hipGetLastError());
     return GENNMI_OK;

@@ -59,7 +59,7 @@ __device__ __forceinline__ float poissonExpInject(const gennmi_cs_t &cs, GLOBAL_
 // neurons 4.64 -> 4.36 -> 4.34, 4.67 -> 4.42 -> 4.38, 4.89 -> 4.58 -> 4.58; 140,000 4.73 -> 4.80 -> 4.78, 5.03 -> 4.83 -> 4.78, 6.12 -> 5.02 -> 4.99; 300,000
 // 5.40 -> 5.70 -> 5.54, 5.67 -> 5.82 -> 5.67, 7.07 -> 6.01 -> 5.84; 520,000 7.25 -> 7.40 -> 7.31, 7.66 -> 7.57 -> 7.46, 10.87 -> 8.23 -> 8.07.
 constexpr uint32_t QUEUE_DIRECT_BLOCKS = 2048, COUNTS_AT_ONCE = 4;
-__device__ __forceinline__ bool queueDirect(uint32_t numBlocks) { return numBlocks > WAVE && numBlocks <= QUEUE_DIRECT_BLOCKS; }
+__host__ __device__ __forceinline__ bool queueDirect(uint32_t numBlocks) { return numBlocks > WAVE && numBlocks <= QUEUE_DIRECT_BLOCKS; }
 __device__ __forceinline__ uint32_t sumOfEarlierBlocks(uint32_t localBlock, const unsigned long long *counts, uint32_t tag, uint32_t *errorFlag)
 {
     __shared__ uint32_t shSum[1024 / WAVE];
@@ -497,11 +497,14 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     if(G.zeroStart && wave == 0) { deliverZeroDelay(); }
 }
 
+// (DIRECT: one of the populations is queueDirect.  Where none is, a step that has that code compiled in is slower: DENSE 8192 x 8192 stepped 9.75 us a step
+// before there was such code, 9.91 with it, 9.79 without; 1000 x 500 batch 4 8.85, 9.02 and 8.88)
+template<bool DIRECT>
 __global__ __launch_bounds__(BLOCK)
 void neuronUpdateKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args, float dt,
                         unsigned long long *agg, uint32_t *errorFlag)
 {
-    neuronBody(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag);
+    neuronBody<DIRECT>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag);
 }
 
 // ------------------------------------------------------------------------------------------------
