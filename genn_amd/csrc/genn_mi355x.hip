@@ -79,7 +79,7 @@ struct gennmi_runner
     ConvMfmaDev convMfma{}; size_t convSource = 0;      // host copy of its descriptor; index of its source population in `neuron`
     // a convolutional layer's whole step in one launch (convStepKernel): the layer's target population is updated on the accumulators
     bool convStep = false;
-    NeuronGroupDev *dConvTarget = nullptr, *dConvRest = nullptr; uint32_t convRestBlocks = 0; size_t convStepBytes = 0;
+    NeuronGroupDev *dConvTarget = nullptr, *dConvRest = nullptr; uint32_t convRestBlocks = 0; size_t convStepBytes = 0; bool convQueuesDirect = false;
     unsigned long long *dConvAgg = nullptr, *dConvRestAgg = nullptr;
     // a feed-forward layer, many steps per launch (genn_mi355x_ahead_kernels.h): its source population, its target population and the layer
     bool ahead = false;
@@ -1321,6 +1321,8 @@ static int refreshTables(gennmi_runner *r)
     return GENNMI_OK;
 }
 
+static auto convStepInstance(const gennmi_runner *r) { return r->convQueuesDirect ? convStepKernel<true> : convStepKernel<false>; }
+
 // Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
 // plain population it feeds, so that no spike ever comes back.
 constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input over the steps of a launch
@@ -2053,8 +2055,9 @@ int gennmi_runner_finalise(gennmi_runner *r)
             HIP_TRY(hipMemset(r->dConvRestAgg, 0, restCount * sizeof(unsigned long long)));
             for(void *q : {(void*)r->dConvRest, (void*)r->dConvTarget, (void*)r->dConvAgg, (void*)r->dConvRestAgg}) { if(q) { r->owned.push_back(q); } }
             r->convStepBytes = bytes;
+            r->convQueuesDirect = queueDirect(r->convMfmaBlocks) || std::any_of(rest.begin(), rest.end(), [](const NeuronGroupDev &n) { return queueDirect(n.numBlocks); });
             if(bytes > 48 * 1024) {
-                HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(convStepKernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+                HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(convStepInstance(r)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
             }
             r->convStep = true;
         }
@@ -2225,7 +2228,8 @@ static int launchFusedStep(gennmi_runner *r, const StepArgs &a)
 
 static int launchConvStep(gennmi_runner *r, const StepArgs &a)
 {
-    convStepKernel<<<dim3((r->convMfmaBlocks + r->convRestBlocks) * r->batch), dim3(CONV_STEP_THREADS), r->convStepBytes, r->stream>>>(
+    const auto kernel = convStepInstance(r);
+    kernel<<<dim3((r->convMfmaBlocks + r->convRestBlocks) * r->batch), dim3(CONV_STEP_THREADS), r->convStepBytes, r->stream>>>(
         r->dConvMfma, r->dConvTarget, r->dConvRest, r->batch, a, r->dt, r->dConvAgg, r->dConvRestAgg, r->dError, r->dEvents);
     HIP_TRY(hipGetLastError());
     return GENNMI_OK;

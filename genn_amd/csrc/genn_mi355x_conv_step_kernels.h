@@ -86,6 +86,9 @@ struct ConvStepEpilogue
 
 constexpr int CONV_STEP_THREADS = BLOCK;
 
+// (DIRECT: one of the populations is queueDirect.  us a step with that code / without: 64x64x16 -> 64x64x32 batch 16, where none is, 29.9 / 29.6,
+// 160x160x8 -> 160x160x8 batch 2, where the layer's 80 row groups are, 31.1 / 31.3)
+template<bool DIRECT>
 __global__ __launch_bounds__(CONV_STEP_THREADS, 3)
 void convStepKernel(const ConvMfmaDev * __restrict__ conv, const NeuronGroupDev * __restrict__ target, const NeuronGroupDev * __restrict__ rest,
                     uint32_t numBatches, StepArgs args, float dt, unsigned long long *agg, unsigned long long *restAgg, uint32_t *errorFlag,
@@ -103,10 +106,10 @@ void convStepKernel(const ConvMfmaDev * __restrict__ conv, const NeuronGroupDev 
         // ---- every other population: the code of the several-neurons-per-lane neuron kernel
         const uint32_t id = blockIdx.x - convBlocks * numBatches;
         const uint32_t batch = id / G.restBlocks, b = id - batch * G.restBlocks;
-        if(G.restNeuronsPerLane == 8) { neuronBulkBody<8, CONV_STEP_THREADS>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
-        else if(G.restNeuronsPerLane == 4) { neuronBulkBody<4, CONV_STEP_THREADS>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
-        else if(G.restNeuronsPerLane == 2) { neuronBulkBody<2, CONV_STEP_THREADS>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
-        else { neuronBulkBody<1, CONV_STEP_THREADS>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
+        if(G.restNeuronsPerLane == 8) { neuronBulkBody<8, CONV_STEP_THREADS, DIRECT>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
+        else if(G.restNeuronsPerLane == 4) { neuronBulkBody<4, CONV_STEP_THREADS, DIRECT>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
+        else if(G.restNeuronsPerLane == 2) { neuronBulkBody<2, CONV_STEP_THREADS, DIRECT>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
+        else { neuronBulkBody<1, CONV_STEP_THREADS, DIRECT>(rest[b], b, G.restBlocks, st, dt, restAgg, errorFlag, batch, numBatches); }
         return;
     }
     // ---- the layer (consecutive work-groups, which go to consecutive XCDs, differ in batch)
@@ -148,7 +151,7 @@ void convStepKernel(const ConvMfmaDev * __restrict__ conv, const NeuronGroupDev 
         blockCount += c;
     }
     unsigned long long *groupAgg = agg + (size_t)convBlocks * numBatches;
-    const uint32_t prefix = blockQueueOffset(blockCount, rowGroup, convBlocks, (size_t)batch * convBlocks, agg, groupAgg, (uint32_t)(st.epoch + 1), &shPrefix, errorFlag);
+    const uint32_t prefix = blockQueueOffset<DIRECT>(blockCount, rowGroup, convBlocks, (size_t)batch * convBlocks, agg, groupAgg, (uint32_t)(st.epoch + 1), &shPrefix, errorFlag);
     if(prefix == 0xFFFFFFFFu) { return; }
     uint32_t position = prefix + waveOffset + scan - mine;
     GLOBAL_AS uint32_t *queue = asGlobal(t.spk) + (size_t)batch * n;

@@ -565,7 +565,7 @@ __device__ __forceinline__ bool plainNeuronStep(const PlainNeuron &c, float Isyn
 }
 
 // (THREADS: threads of the calling work-group, all of which call; batch / numBatches: the grid's second dimension in the neuron kernels)
-template<int NPL, int THREADS = BLOCK>
+template<int NPL, int THREADS = BLOCK, bool DIRECT = true>
 __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                                const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag,
                                                uint32_t batch, uint32_t numBatches)
@@ -733,8 +733,8 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
         if(psm.maxDenDelay && psm.denDelayPtr) { *psm.denDelayPtr = modStep(st.epoch + 1, psm.maxDenDelay); }
     }
 
-    const uint32_t prefix = blockQueueOffset(blockCount, localBlock, groupBlocks, aggBase, agg, groupAgg,
-                                             (uint32_t)(st.epoch + 1), &shPrefix, errorFlag, true);
+    const uint32_t prefix = blockQueueOffset<DIRECT>(blockCount, localBlock, groupBlocks, aggBase, agg, groupAgg,
+                                                     (uint32_t)(st.epoch + 1), &shPrefix, errorFlag, true);
     if(prefix == 0xFFFFFFFFu) { return; }
     #pragma unroll
     for(int j = 0; j < NPL; j++) {
