@@ -1329,9 +1329,9 @@ constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input 
 // A work-group of the convolution takes no more output rows than leave two of them to a compute unit; a single row may take a little more.
 constexpr size_t AHEAD_ROWS_LDS = 64 * 1024, AHEAD_MAX_LDS = 82 * 1024;
 // Runs (and remainders of runs) shorter than this are stepped one by one: a pass costs a good part of a pass of 32 steps however few it is given.  us
-// at once / one by one for 5 and for 8 steps: Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, at 20 %, 2.5 % and 0.25 % activity 239 / 174 and
-// 259 / 273, 125 / 152 and 144 / 238, 93 / 146 and 98 / 228; 40x40x16 -> 40x40x4 5x5, batch 16, at 0.25 % 185 / 131 and 189 / 204; DENSE 8192 x 8192
-// (5 %; 4 and 8 steps) 35 / 45 and 43 / 85, the same with batch 16 195 / 175 and 231 / 346.
+// at once / one by one for 5 and for 8 steps: Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, at 20 %, 2.5 % and 0.25 % activity 187 / 173 and
+// 211 / 268, 97 / 164 and 110 / 251, 76 / 159 and 81 / 244; 40x40x16 -> 40x40x4 5x5, batch 16, at 0.25 % 87 / 143 and 91 / 223; DENSE 8192 x 8192
+// (5 %; 4 and 8 steps) 40 / 54 and 48 / 91, the same with batch 16 153 / 181 and 180 / 352.
 constexpr uint32_t AHEAD_MIN_STEPS = 8;
 // (the kernels of the target's neuron model and postsynaptic model)
 static auto aheadConvInstance(const gennmi_neuron_update_group_t &g)
