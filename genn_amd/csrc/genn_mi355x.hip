@@ -1804,8 +1804,8 @@ int gennmi_runner_finalise(gennmi_runner *r)
             // Work-groups of a tile: as many as make the largest share of synapses any work-group has the smallest, within the budget (a launch ends with
             // the work-group that has most: dealt out in proportion and rounded down, a projection of 1.8 work-groups a tile got one).  Where two rounds'
             // shares come out more even, by a twentieth, it is two after all.  us of the longest step of a burst, two rounds rounded down / one rounded
-            // down / as here: Izhikevich 932,087 x 107 606 / 783 / 608 (one round as even as can be 660), 600,000 x 100 372 / 337 / 327, 500,000 x 300 160 / 162 / 155.
-            constexpr uint32_t MOST_SPLITS = 256;
+            // down / as here, dealt out tile by tile: Izhikevich 932,087 x 107 606 / 783 / 608 (one round as even as can be 660), 600,000 x 100 372 / 337 / 327, 500,000 x 300 160 / 162 / 155.
+            constexpr uint32_t MOST_SPLITS = 256, NUM_XCD = 8;
             auto weight = [&](const TileGroupDev &t) { return (tileGroups.size() > 1 && t.recLanes ? 2.0 : 1.0) * (double)t.g.numSrcNeurons * t.g.rowStride; };
             auto splitsOf = [&](const TileGroupDev &t, double most) { return (uint32_t)std::min((double)MOST_SPLITS, std::max(1.0, std::ceil(weight(t) / (t.numTiles * most)))); };
             double totalWeight = 0.0, shared = 0.0, least = 0.0;
@@ -1846,8 +1846,22 @@ int gennmi_runner_finalise(gennmi_runner *r)
                 t.spikesPerSplit = spikesPerSplit;
                 // (worth it from one event per two targets of a block's tile)
                 if(t.factorEvents && factorMode == 1) { t.factorEvents = std::max(1ull, (unsigned long long)numSplits * t.tileSize / 2); }
-                for(uint32_t tile = 0; tile < t.numTiles; tile++) {
-                    for(uint32_t split = 0; split < numSplits; split++) { t.tile = tile; t.split = split; tiles.push_back(t); }
+                // Work-groups go to the XCDs in turn.  The parts of a row that different tiles read share cache lines where they are short, so the work-groups that
+                // read the same spikes' rows, one of every tile, are given to as few XCDs as an even deal allows, and find those lines in an L2.  (Dealt out tile by
+                // tile they did so only where a tile had a multiple of 8 work-groups, and a time depended on that number more than on their shares.)  us of
+                // the longest step of a burst, with two rounds of work-groups rounded down, dealt out tile by tile / with these numbers of them, tile by
+                // tile / as here: Izhikevich 720,000 x 9 176 / 188 / 103, 690,000 x 20 219 / 263 / 115, 860,000 x 40 442 / 452 / 282, 780,000 x 60 260 / 304 / 284,
+                // 932,087 x 107 622 / 612 / 366, 600,000 x 100 394 / 334 / 223; long parts: plastic 100,000 x 500 308 / 254 / 255, balanced 300,007 x 1000 33 throughout.
+                const uint32_t count = t.numTiles * numSplits;
+                for(uint32_t k = 0; k < count; k++) {
+                    uint32_t at = k;
+                    if(t.recLanes) { t.tile = at / numSplits; t.split = at % numSplits; }       // (in a calm step only the first few have work)
+                    else {
+                        const uint32_t xcd = k % NUM_XCD;
+                        at = k / NUM_XCD + xcd * (count / NUM_XCD) + std::min(xcd, count % NUM_XCD);
+                        t.split = at / t.numTiles; t.tile = at % t.numTiles;
+                    }
+                    tiles.push_back(t);
                 }
             }
         }

@@ -76,3 +76,30 @@ def test_short_rows_are_walked_about_as_fast_as_long_ones():
         took[n] = min(rounds)
         model.unload()
     assert 0.0 < took[100000] < 4.0 * took[10000], took
+
+
+def test_bursts_of_short_rows_do_not_depend_on_how_many_work_groups_a_tile_gets():
+    """Rows of 9 synapses over 40 tiles share cache lines between the tiles' work-groups.  Dealt out tile by tile, those of one line met in one L2 only where a
+    tile had a multiple of 8 or 4 of them: a step of 720,000 neurons (17 to a tile) took 1.5 times as long as one of 650,000 (20), now 1.1 times."""
+    from genn_amd.genn_model import GeNNModel, init_postsynaptic, init_sparse_connectivity, init_var, init_weight_update
+    lif, took = dict(C=1.0, TauM=20.0, Vrest=-60.0, Vreset=-60.0, Vthresh=-50.0, Ioffset=4.0, TauRefrac=2.0), {}
+    for n in (650000, 720000):
+        model = GeNNModel("float", "burst", dt=1.0)
+        model.seed, model.timing_enabled = 11, True
+        size = {"E": n * 4 // 5, "I": n // 5}
+        pops = {k: model.add_neuron_population(k, size[k], "LIF", lif, {"V": init_var("Uniform", {"min": -60.0, "max": -50.0}), "RefracTime": 0.0}) for k in "EI"}
+        for src in "EI":
+            for trg, num in (("E", 7), ("I", 2)):
+                model.add_synapse_population(src + trg, "SPARSE", pops[src], pops[trg], init_weight_update("StaticPulse", {}, {"g": init_var("Uniform", {"min": 0.0, "max": 1e-4})}),
+                                             init_postsynaptic("DeltaCurr"), init_sparse_connectivity("FixedNumberPostWithReplacement", {"num": num}))
+        model.build()
+        model.load()
+        rounds = []
+        for _ in range(5):
+            before = model.presynaptic_update_time
+            for _ in range(20):
+                model.step_time()
+            rounds.append(model.presynaptic_update_time - before)
+        took[n] = min(rounds)
+        model.unload()
+    assert 0.0 < took[720000] < 1.3 * took[650000], took
