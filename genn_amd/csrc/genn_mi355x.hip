@@ -1370,11 +1370,13 @@ static int setupAhead(gennmi_runner *r, uint32_t numCU)
         // as many output rows per work-group as leave four work-groups to a compute unit
         const uint64_t rowsInAll = (uint64_t)c[5] * r->batch * (((uint32_t)c[7] + 31) / 32);
         C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (4 * numCU)));
+        size_t ldsBytes = 0;        // (the lists of steps, up to 7 KiB more, change neither how many fit: 64 KiB and 82)
         for(;; C.rowsPerBlock--) {
-            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)inputs * 32 + (size_t)(inputs + 1) / 2 + (size_t)(BLOCK / WAVE) * 2 * aheadConvList(inputs)) * sizeof(uint32_t);
-            if(r->aheadConvBytes <= AHEAD_ROWS_LDS || C.rowsPerBlock == 1) { break; }
+            ldsBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)inputs * 32 + (size_t)(inputs + 1) / 2 + (size_t)(BLOCK / WAVE) * 2 * (inputs + 1)) * sizeof(uint32_t);
+            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)(inputs + 1) * 32 + (size_t)(inputs + 1) / 2) * sizeof(uint32_t) + (size_t)(BLOCK / WAVE) * aheadConvListBytes(inputs);
+            if(ldsBytes <= AHEAD_ROWS_LDS || C.rowsPerBlock == 1) { break; }
         }
-        if(r->aheadConvBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
+        if(ldsBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
         if(r->aheadConvBytes > 48 * 1024) {
             HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(aheadConvInstance(g)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)r->aheadConvBytes));
         }

@@ -36,8 +36,24 @@ struct AheadConv
     uint32_t isConv;
 };
 
-// entries of a pixel's list of active inputs: all of them and what fills the last pair
-__host__ __device__ constexpr uint32_t aheadConvList(uint32_t inputs) { return inputs + 1u; }
+// bytes of a wavefront's lists: of a pixel's active inputs, all of them and what fills the last pair; or of the active inputs of its two pixels in each of
+// 32 steps, 16 bits each
+constexpr uint32_t AHEAD_CONV_MOST = 16;
+__host__ __device__ constexpr uint32_t aheadConvListBytes(uint32_t inputs)
+{
+    const uint32_t pixel = (8u * (inputs + 1u) + 15u) / 16u * 16u, steps = 2u * AHEAD_WORD * AHEAD_CONV_MOST * 2u;
+    return (pixel > steps) ? pixel : steps;
+}
+// How many inputs of a pixel may have a spike in a step for its sum to be made one by one, by how many of a patch's words have spikes and how many those have (of
+// the steps of a launch).  0: sums are products throughout.  (The line's figures: aheadConvKernel.)
+__host__ __device__ constexpr uint32_t aheadConvMost(uint32_t inputs, uint32_t steps, uint32_t active, uint32_t spikes, uint32_t words)
+{
+    // (above 511 a weight's place does not fit the list's 16 bits)
+    const uint32_t most = (inputs > 511u) ? 0u : (inputs / 16u * 4u < AHEAD_CONV_MOST) ? inputs / 16u * 4u : AHEAD_CONV_MOST;
+    const unsigned long long all = words, spikesOfAll = (unsigned long long)spikes * inputs;
+    const bool few = (32u * spikesOfAll <= 13u * most * steps * all), worth = (8ull * inputs * active > all * (4u * steps + 25u * ((inputs + 31u) / 32u)) + spikesOfAll);
+    return (few && worth) ? most : 0u;
+}
 
 __device__ __forceinline__ size_t aheadRecordingRow(const AheadArgs &A, uint32_t step) { return (size_t)((A.timestep + step) % A.recordingRows); }
 
@@ -469,6 +485,43 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
     if(i < n) { var0[bi] = v0; var1[bi] = v1; outPost[bi] = lin; }
 }
 
+// 32 x 32 bits per half-wave, transposed by exchanging ever smaller blocks across the diagonal.  A lane's neighbours are reached without LDS, and a block is
+// moved by a rotation and put in place by a bit select: 17 instructions.
+struct Transpose32
+{
+    uint32_t keep[5], turn[5];
+    __device__ __forceinline__ explicit Transpose32(uint32_t lane)
+    {
+        // (low: the bits b with b & j == 0; a lane with lane & j keeps the others and takes its neighbour's, moved down)
+        constexpr uint32_t low[5] = {0x0000FFFFu, 0x00FF00FFu, 0x0F0F0F0Fu, 0x33333333u, 0x55555555u};
+        #pragma unroll
+        for(uint32_t k = 0; k < 5; k++) {
+            const uint32_t j = 16u >> k;
+            keep[k] = (lane & j) ? ~low[k] : low[k];
+            turn[k] = (lane & j) ? j : 32u - j;
+        }
+    }
+    __device__ __forceinline__ uint32_t operator()(uint32_t x) const
+    {
+        const auto rows = __builtin_amdgcn_permlane16_swap(x, x, false, false);             // the lower row's and the upper row's, in both
+        exchange<0>(x, (keep[0] == 0xFFFF0000u) ? rows[0] : rows[1]);
+        exchange<1>(x, dpp<0x128>(x));                                                      // row_ror:8
+        exchange<2>(x, dpp<0x1B>(dpp<0x141>(x)));                                           // row_half_mirror, quad_perm:[3,2,1,0]
+        exchange<3>(x, dpp<0x4E>(x));                                                       // quad_perm:[2,3,0,1]
+        exchange<4>(x, dpp<0xB1>(x));                                                       // quad_perm:[1,0,3,2]
+        return x;
+    }
+private:
+    template<int K>
+    __device__ __forceinline__ void exchange(uint32_t &x, uint32_t other) const
+    {
+        const uint32_t turned = __builtin_amdgcn_alignbit(other, other, turn[K]);
+        x = (x & keep[K]) | (turned & ~keep[K]);
+    }
+    template<int CTRL>
+    static __device__ __forceinline__ uint32_t dpp(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false); }
+};
+
 // ---- 2b, 3b. Conv2D and its neurons, up to 32 steps.  A work-group owns some output rows of one batch and 32 output channels: the
 // words of the input pixels they reach (zero outside the input) and the kernel wait in LDS.  A wavefront takes two output pixels at a
 // time: the rows of its two products are timesteps, the inner dimension the pixel's (tap, channel) inputs that have a spike in any of the
@@ -484,6 +537,13 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
 // Of that the matrix cores are busy 60 and the vector units 64 (counters), the neurons' steps half of these.  run() with all its launches, packed
 // against paired, other shapes and rates: 40x37x16 -> 4 5x5 batch 16, 32 steps, 0.5 / 5 / 40 / 100 % 124 / 248 / 385 / 422 against 244 / 398 / 481 / 507; 24x24x16 -> 32
 // 5x5, 45 steps 96 / 165 / 270 / 298 against 189 / 283 / 358 / 375; the shape above, 50 steps 179 / 318 / 549 / 746 against 243 / 416 / 586 / 771.
+// Where few of a pixel's inputs have a spike in a step (2.5 %: 3.6 of 144), most of a product's rows add nothing, and a sum is made one weight after the
+// other instead, in the same order and so with the same bits: the words of 32 inputs, transposed, give each lane one step's, which it lists in LDS, and the
+// pixel's lanes add up the weights listed for step after step, four at a time.  A product of two inputs is 64 clocks of the matrix unit whatever they hold;
+// a listed weight is two or three vector instructions, so the rule (aheadConvMost) compares 48 clocks an active input with 48 a step, 300 a transposed word and 6 a
+// spike, and leaves patches of more than 6.5 spikes a pixel and step (a list holds 16; one that is full means products for its two pixels) to the products.
+// run() of 50 steps, products only -> now, at 0.5 / 2.5 / 10 / 30 / 75 %: 64x64x16 -> 32 3x3 batch 16 196 / 308 / 440 / 540 / 687 -> 197 / 235 / 440 / 540 / 687; 48x48x3 ->
+// 20 5x5 batch 8 90 / 116 / 145 / 164 / 172 -> 89 / 108 / 144 / 164 / 172; 40x37x16 -> 4 5x5 batch 16, 24x24x16 -> 32 5x5 batch 4, 64x64 from one channel, 33x47x2: no change.
 template<uint32_t MODEL, uint32_t PSM>
 __global__ __launch_bounds__(BLOCK, 4)
 void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
@@ -499,25 +559,33 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     AheadNeuron<MODEL, PSM> neuron(g, A.dt);
     asm volatile("" : "+v"(neuron.constants.p[5]), "+v"(neuron.constants.p[6]));       // (selected between in every step: from scalar registers that is a copy first)
     const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), inputs = (uint32_t)C.kh * rowWords;
-    const uint32_t listed = aheadConvList(inputs);
-    uint2 *list = reinterpret_cast<uint2*>(shAhead) + wave * listed;                                // (word, byte of its weights) of a pixel's active inputs
-    float *kern = reinterpret_cast<float*>(reinterpret_cast<uint2*>(shAhead) + (BLOCK / WAVE) * listed);       // [input][32]
-    uint16_t *place = reinterpret_cast<uint16_t*>(kern + inputs * 32);                              // [input] its word behind the pixel's first
-    uint32_t *patch = reinterpret_cast<uint32_t*>(kern + inputs * 32) + (inputs + 1) / 2;
+    uint8_t *lists = reinterpret_cast<uint8_t*>(shAhead) + wave * aheadConvListBytes(inputs);
+    uint2 *list = reinterpret_cast<uint2*>(lists);                                                  // (word, byte of its weights) of a pixel's active inputs
+    uint16_t *stepList = reinterpret_cast<uint16_t*>(lists);                                        // [pixel][step][AHEAD_CONV_MOST] bytes of weights
+    float *kern = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(shAhead) + (BLOCK / WAVE) * aheadConvListBytes(inputs));     // [input][32], one more of zeros
+    uint16_t *place = reinterpret_cast<uint16_t*>(kern + (inputs + 1) * 32);                        // [input] its word behind the pixel's first
+    uint32_t *patch = reinterpret_cast<uint32_t*>(kern + (inputs + 1) * 32) + (inputs + 1) / 2;
     // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
     GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
     const int inRowWords = C.iw * C.ic;
+    uint32_t active = 0, spiked = 0;
     for(uint32_t r = 0; r < rows + (uint32_t)C.kh - 1; r++) {
         const int y = (int)(y0 + r) - C.PH;
         for(uint32_t e = threadIdx.x; e < rowPitch; e += BLOCK) {
             const int x = (int)e - C.PW * C.ic;
-            patch[r * rowPitch + e] = (y >= 0 && y < C.ih && x >= 0 && x < inRowWords) ? in[(size_t)y * inRowWords + x] : 0u;
+            const uint32_t word = (y >= 0 && y < C.ih && x >= 0 && x < inRowWords) ? in[(size_t)y * inRowWords + x] : 0u;
+            patch[r * rowPitch + e] = word;
+            active += (word != 0u) ? 1u : 0u;
+            spiked += __popc(word);
         }
     }
+    for(int off = WAVE / 2; off > 0; off >>= 1) { active += __shfl_down(active, off, WAVE); spiked += __shfl_down(spiked, off, WAVE); }
+    __shared__ uint32_t seen[2][BLOCK / WAVE];
+    if(lane == 0) { seen[0][wave] = active; seen[1][wave] = spiked; }
     bool nonFinite = false;
-    for(uint32_t e = threadIdx.x; e < inputs * 32; e += BLOCK) {
+    for(uint32_t e = threadIdx.x; e < (inputs + 1) * 32; e += BLOCK) {
         const uint32_t k = e / 32, oo = blockIdx.z * 32 + (e & 31);
-        float weight = (oo < oc) ? asGlobal(kernel)[(size_t)k * oc + oo] : 0.0f;
+        float weight = (oo < oc && k < inputs) ? asGlobal(kernel)[(size_t)k * oc + oo] : 0.0f;
         if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
         kern[e] = weight;
     }
@@ -528,6 +596,45 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     GLOBAL_AS uint32_t *spikes = asGlobal(spikeWords) + (size_t)batch * n;
     const char *weights = reinterpret_cast<const char*>(kern + col);
     const uint2 *entries = list + half;
+    // Lists, for each of 32 steps, the inputs that have a spike in it, in their order: lane (half, t) those of the half's pixel in step t.  32 inputs at a
+    // time, a lane each, their words transposed.  false: a step has more than `most`.
+    active = spiked = 0;
+    #pragma unroll
+    for(uint32_t w = 0; w < BLOCK / WAVE; w++) { active += seen[0][w]; spiked += seen[1][w]; }
+    // (of the patch's words those that are input: a work-group at the edge has no more to add up for most of its pixels than any other)
+    const int firstRow = max((int)y0 - C.PH, 0), endRow = min((int)(y0 + rows) + C.kh - 1 - C.PH, C.ih), firstWord = max(C.PW * C.ic, 0), endWord = min(C.PW * C.ic + inRowWords, (int)rowPitch);
+    const uint32_t inputWords = (uint32_t)max(endRow - firstRow, 0) * (uint32_t)max(endWord - firstWord, 0);
+    const uint32_t most = nonFinite ? 0u : aheadConvMost(inputs, steps, active, spiked, inputWords);
+    const Transpose32 transposed(lane);
+    auto listSteps = [&](uint32_t pixel, uint32_t &count) -> bool {
+        auto word = [&](uint32_t k) -> uint32_t {
+            const uint32_t there = patch[pixel + place[min(k, inputs - 1)]];
+            return (k < inputs) ? there : 0u;
+        };
+        uint32_t bits = word(col), following = word(32 + col);
+        bits = transposed(bits);
+        uint16_t *mine = stepList + lane * AHEAD_CONV_MOST;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        #pragma unroll
+        for(uint32_t q = 0; q < AHEAD_CONV_MOST / 4; q++) { reinterpret_cast<u32x2*>(mine)[q] = u32x2{inputs * 0x800080u, inputs * 0x800080u}; }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for(uint32_t k0 = 0; ; ) {
+            if(__ballot(count + __popc(bits) > most)) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                return false;
+            }
+            while(bits) {
+                mine[count++] = (uint16_t)((k0 + __ffs(bits) - 1) * 128);
+                bits &= bits - 1;
+            }
+            k0 += 32;
+            if(k0 >= inputs) { break; }
+            bits = transposed(following);
+            following = word(k0 + 32 + col);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        return true;
+    };
     for(uint32_t first = wave * 2; first < pixels; first += (BLOCK / WAVE) * 2) {
         // state of the lane's neuron (pixel first + half, channel o), asked for ahead of the products
         const uint32_t own = first + half;
@@ -535,71 +642,121 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
         const size_t at = valid ? ((size_t)y0 * ow + own) * oc + o : 0;
         float v0 = var0[at], v1 = var1[at], lin = outPost[at];
         uint32_t base[2];
-        f32x16 acc[2];
         #pragma unroll
         for(int j = 0; j < 2; j++) {
             const uint32_t p = min(first + j, pixels - 1), r = p / ow;
             base[j] = r * rowPitch + (p - r * ow) * (uint32_t)C.ic;
-            acc[j] = f32x16{};
-            // the inputs that have a spike in any of the steps, in their order
-            uint32_t count = 0;
-            for(uint32_t k0 = 0; k0 < inputs; k0 += WAVE) {
-                const uint32_t k = k0 + lane;
-                const uint32_t behind = place[min(k, inputs - 1)], there = patch[base[j] + behind], word = (k < inputs) ? there : 0u;
-                const unsigned long long active = __ballot(word != 0u);
-                if(word) { list[count + __popcll(active & ((1ull << lane) - 1ull))] = make_uint2(word, k * 128); }
-                count += __popcll(active);
-            }
-            if(lane == 0) { list[count] = make_uint2(0u, 0u); }         // (fills the last pair)
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            // (no branch inside a round: the compiler copies the sixteen sums where paths with and without a product meet)
-            uint32_t m = 0;
-            for(; m + 8 <= count; m += 8) {
-                uint2 e[4]; float w[4];
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) { e[u] = entries[m + 2 * u]; }
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) { w[u] = *reinterpret_cast<const float*>(weights + e[u].y); }
-                #pragma unroll
-                for(uint32_t u = 0; u < 4; u++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e[u].x, col), w[u], acc[j], 0, 0, 0); }
-            }
-            for(; m < count; m += 2) {
-                const uint2 e = entries[m];
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e.x, col), *reinterpret_cast<const float*>(weights + e.y), acc[j], 0, 0, 0);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        if(nonFinite) {
-            // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
-            for(uint32_t k = 0; k < inputs; k++) {
-                const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
-                if(aheadFinite(b)) { continue; }
-                #pragma unroll
-                for(int j = 0; j < 2; j++) {
-                    const uint32_t bits = patch[base[j] + place[k]];
-                    #pragma unroll
-                    for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
-                }
-            }
-        }
-        // lower half: all steps of the first pixel, upper half: of the second
-        float x[16], y[16];
-        #pragma unroll
-        for(int v = 0; v < 16; v++) {
-            const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
-            x[v] = __uint_as_float(swapped[0]); y[v] = __uint_as_float(swapped[1]);
-        }
-        uint32_t fired = 0;
-        #pragma unroll
-        for(uint32_t t = 0; t < AHEAD_WORD; t++) {
-            // (kept a comparison and a branch: computed ahead for all steps, the conditions are 32 masks, spilled)
+        // (kept a comparison and a branch: computed ahead for all steps, the conditions are 32 masks, spilled)
+        uint32_t fired = 0, count = 0;
+        auto step = [&](uint32_t t, float input) {
             uint32_t end = steps;
             asm volatile("" : "+s"(end));
             if(t < end) {
                 asm volatile("" : "+v"(lin));
-                const float input = (t & 4) ? y[4 * (t / 8) + (t & 3)] : x[4 * (t / 8) + (t & 3)];
                 fired |= neuron.step(input, lin, v0, v1) ? 1u << t : 0u;
             }
+        };
+        if(most != 0 && listSteps(half ? base[1] : base[0], count)) {
+            // four of a step's inputs at a time, both halves as many rounds as the one that has more needs
+            uint32_t more[AHEAD_CONV_MOST / 4];
+            #pragma unroll
+            for(uint32_t q = 0; q < AHEAD_CONV_MOST / 4; q++) {
+                const unsigned long long ballot = __ballot(count > 4 * q);
+                more[q] = (uint32_t)ballot | (uint32_t)(ballot >> 32);
+            }
+            const u32x2 *mine = reinterpret_cast<const u32x2*>(stepList + half * AHEAD_WORD * AHEAD_CONV_MOST);
+            auto load = [&](u32x2 four, float w[4]) {
+                w[0] = *reinterpret_cast<const float*>(weights + (four[0] & 0xFFFFu)); w[1] = *reinterpret_cast<const float*>(weights + (four[0] >> 16));
+                w[2] = *reinterpret_cast<const float*>(weights + (four[1] & 0xFFFFu)); w[3] = *reinterpret_cast<const float*>(weights + (four[1] >> 16));
+            };
+            // (the first four of a group of steps are asked for ahead of the group before; a loop, for the instruction cache's sake)
+            constexpr uint32_t GROUP = 4;
+            float w[GROUP][4], next[GROUP][4];
+            #pragma unroll
+            for(uint32_t u = 0; u < GROUP; u++) { load(mine[u * (AHEAD_CONV_MOST / 4)], w[u]); }
+            #pragma unroll 1
+            for(uint32_t t0 = 0; t0 < steps; t0 += GROUP) {
+                const uint32_t ahead = min(t0 + GROUP, AHEAD_WORD - GROUP);
+                #pragma unroll
+                for(uint32_t u = 0; u < GROUP; u++) { load(mine[(ahead + u) * (AHEAD_CONV_MOST / 4)], next[u]); }
+                __builtin_amdgcn_sched_barrier(0);
+                #pragma unroll
+                for(uint32_t u = 0; u < GROUP; u++) {
+                    const uint32_t t = t0 + u;
+                    float input = (((0.0f + w[u][0]) + w[u][1]) + w[u][2]) + w[u][3];
+                    #pragma unroll
+                    for(uint32_t q = 1; q < AHEAD_CONV_MOST / 4; q++) {
+                        if(!((more[q] >> t) & 1u)) { break; }
+                        float x[4];
+                        load(mine[t * (AHEAD_CONV_MOST / 4) + q], x);
+                        input = (((input + x[0]) + x[1]) + x[2]) + x[3];
+                    }
+                    step(t, input);
+                }
+                #pragma unroll
+                for(uint32_t u = 0; u < GROUP; u++) {
+                    #pragma unroll
+                    for(uint32_t k = 0; k < 4; k++) { w[u][k] = next[u][k]; }
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+        else {
+            f32x16 acc[2];
+            #pragma unroll
+            for(int j = 0; j < 2; j++) {
+                acc[j] = f32x16{};
+                // the inputs that have a spike in any of the steps, in their order
+                uint32_t count = 0;
+                for(uint32_t k0 = 0; k0 < inputs; k0 += WAVE) {
+                    const uint32_t k = k0 + lane;
+                    const uint32_t behind = place[min(k, inputs - 1)], there = patch[base[j] + behind], word = (k < inputs) ? there : 0u;
+                    const unsigned long long active = __ballot(word != 0u);
+                    if(word) { list[count + __popcll(active & ((1ull << lane) - 1ull))] = make_uint2(word, k * 128); }
+                    count += __popcll(active);
+                }
+                if(lane == 0) { list[count] = make_uint2(0u, 0u); }         // (fills the last pair)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                // (no branch inside a round: the compiler copies the sixteen sums where paths with and without a product meet)
+                uint32_t m = 0;
+                for(; m + 8 <= count; m += 8) {
+                    uint2 e[4]; float w[4];
+                    #pragma unroll
+                    for(uint32_t u = 0; u < 4; u++) { e[u] = entries[m + 2 * u]; }
+                    #pragma unroll
+                    for(uint32_t u = 0; u < 4; u++) { w[u] = *reinterpret_cast<const float*>(weights + e[u].y); }
+                    #pragma unroll
+                    for(uint32_t u = 0; u < 4; u++) { acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e[u].x, col), w[u], acc[j], 0, 0, 0); }
+                }
+                for(; m < count; m += 2) {
+                    const uint2 e = entries[m];
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(aheadBit(e.x, col), *reinterpret_cast<const float*>(weights + e.y), acc[j], 0, 0, 0);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+            if(nonFinite) {
+                // weights that are not finite, to the steps that have their spike only (see aheadDenseKernel)
+                for(uint32_t k = 0; k < inputs; k++) {
+                    const float b = (o < oc) ? asGlobal(kernel)[(size_t)k * oc + o] : 0.0f;
+                    if(aheadFinite(b)) { continue; }
+                    #pragma unroll
+                    for(int j = 0; j < 2; j++) {
+                        const uint32_t bits = patch[base[j] + place[k]];
+                        #pragma unroll
+                        for(uint32_t v = 0; v < 16; v++) { acc[j][v] += ((bits >> aheadRow(v, half)) & 1u) ? b : 0.0f; }
+                    }
+                }
+            }
+            // lower half: all steps of the first pixel, upper half: of the second
+            float x[16], y[16];
+            #pragma unroll
+            for(int v = 0; v < 16; v++) {
+                const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
+                x[v] = __uint_as_float(swapped[0]); y[v] = __uint_as_float(swapped[1]);
+            }
+            #pragma unroll
+            for(uint32_t t = 0; t < AHEAD_WORD; t++) { step(t, (t & 4) ? y[4 * (t / 8) + (t & 3)] : x[4 * (t / 8) + (t & 3)]); }
         }
         if(valid) { var0[at] = v0; var1[at] = v1; outPost[at] = lin; spikes[at] = fired; }
     }
@@ -620,22 +777,11 @@ void aheadTransposeKernel(const NeuronGroupDev * __restrict__ target, AheadArgs 
         const uint32_t i = blockIdx.x * 1024 + (wave * 4 + q) * WAVE + lane;
         mine[q] = (i < n) ? asGlobal(spikeWords)[(size_t)batch * n + i] : 0u;
     }
-    // (low: the bits b with b & j == 0)
-    auto exchange = [&](uint32_t &x, uint32_t j, uint32_t low) {
-        const uint32_t other = (uint32_t)__shfl_xor((int)x, (int)j, WAVE);
-        x = (lane & j) ? ((x & ~low) | ((other & ~low) >> j)) : ((x & low) | ((other & low) << j));
-    };
+    const Transpose32 transposed(lane);
     #pragma unroll
     for(uint32_t q = 0; q < 4; q++) {
-        // 32 x 32 bits per half-wave, transposed by exchanging ever smaller blocks across the diagonal (32 ballots and selects: 18 us
-        // for 2.1 x 10^6 neurons)
-        uint32_t x = mine[q];
-        exchange(x, 16, 0x0000FFFFu);
-        exchange(x, 8, 0x00FF00FFu);
-        exchange(x, 4, 0x0F0F0F0Fu);
-        exchange(x, 2, 0x33333333u);
-        exchange(x, 1, 0x55555555u);
-        rows[lane & 31][(wave * 4 + q) * 2 + (lane >> 5)] = x;
+        // (32 ballots and selects instead: 18 us for 2.1 x 10^6 neurons)
+        rows[lane & 31][(wave * 4 + q) * 2 + (lane >> 5)] = transposed(mine[q]);
     }
     __syncthreads();
     for(uint32_t e = threadIdx.x; e < AHEAD_WORD * 32; e += BLOCK) {

@@ -388,3 +388,47 @@ def test_dense_layers_of_sources_most_of_which_are_silent(steps, active, monkeyp
         model.unload()
     assert np.array_equal(got[0][0], got[1][0], equal_nan=True) and np.array_equal(got[0][1], got[1][1])
     assert got[0][2] == got[1][2] == 70 * end[-1]
+
+
+# 32 and 64 inputs a pixel and numbers off a round of 32, up to what LDS holds; few enough spikes for a list of each step, too many, and about as many as the
+# rule allows; channels of one product and of two
+@pytest.mark.parametrize("h,w,ic,oc,k,rate", [(9, 11, 16, 32, 3, 0.025), (9, 11, 16, 32, 3, 0.045), (12, 6, 8, 7, 3, 0.04), (10, 9, 7, 34, 3, 0.06), (8, 9, 16, 3, 2, 0.05),
+                                              (7, 7, 13, 5, 5, 0.012), (7, 8, 19, 4, 5, 0.01), (9, 9, 8, 32, 2, 0.05), (11, 33, 4, 33, 5, 0.03)])
+@pytest.mark.parametrize("steps", [8, 32, 45])
+def test_sums_of_convolutions_with_few_spikes(h, w, ic, oc, k, rate, steps):
+    """A step's sum is that of its inputs' weights in the kernel's order, whichever way it is made: outPost bit for bit as 32-bit sums in that order give it.
+    Two pixels have steps with 15, 16 and 17 inputs (a list holds 16), and one step has no spike at all."""
+    rng = np.random.default_rng(h * w + steps)
+    net = configs.conv_toeplitz(h=h, w=w, ic=ic, oc=oc, k=k, steps=steps, w_sd=0.1, ioffset=0.3)
+    fire = rng.random((steps, h, w, ic)) < rate
+    before, after = (k - 1) - (k - 1) // 2, (k - 1) // 2
+    for step, y, x, count in ((1, 4, 4, 15), (3, 4, 4, 16), (5, 4, 4, 17), (5, 5, 3, 16), (6, 2, 4, 17)):
+        patch = np.zeros((min(k, 4), min(k, 4), ic), bool).reshape(-1)
+        patch[rng.permutation(len(patch))[:count]] = True
+        side = min(k, 4)
+        fire[step, y - before:y - before + side, x - before:x - before + side] = patch.reshape(side, side, ic)
+    fire[2] = False
+    trains = fire.reshape(steps, -1).T
+    end = np.cumsum(trains.sum(axis=1)).astype(np.uint32)
+    source = net.pop("In")
+    source.vars = {"startSpike": (end - trains.sum(axis=1)).astype(np.uint32), "endSpike": end}
+    source.spike_times = np.nonzero(trains)[1].astype(np.float32)
+    model = model_from_net(net)
+    model.load(num_recording_timesteps=steps)
+    assert model.runner_info()["feed_forward_ahead"]
+    model.run(steps)
+    got = model.synapse_populations["Conv"].vars["outPost"].pull_from_device().copy()
+    model.unload()
+    want = np.zeros((h, w, oc), np.float32)
+    decay = np.float32(np.exp(-1.0 / 5.0))
+    kernel = net.syns[0].g
+    for step in range(steps):
+        sums = np.zeros((h, w, oc), np.float32)
+        if step:
+            padded = np.pad(fire[step - 1], ((before, after), (before, after), (0, 0)))
+            for a in range(k):
+                for b in range(k):
+                    for channel in range(ic):
+                        sums += np.where(padded[a:a + h, b:b + w, channel, None], kernel[a, b, channel], np.float32(0))
+        want = (want + sums) * decay
+    assert np.array_equal(got.reshape(want.shape).view(np.uint32), want.view(np.uint32))
