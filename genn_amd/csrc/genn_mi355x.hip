@@ -1340,13 +1340,6 @@ static auto aheadConvInstance(const gennmi_neuron_update_group_t &g)
     const bool lif = (g.model == LIF), exponential = (g.psm[0].kind == EXP);
     return lif ? (exponential ? aheadConvKernel<LIF, EXP> : aheadConvKernel<LIF, DELTA>) : (exponential ? aheadConvKernel<IZH, EXP> : aheadConvKernel<IZH, DELTA>);
 }
-static auto aheadNeuronInstance(const gennmi_neuron_update_group_t &g)
-{
-    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
-    const bool lif = (g.model == LIF), exponential = (g.psm[0].kind == EXP);
-    return lif ? (exponential ? aheadNeuronKernel<LIF, EXP> : aheadNeuronKernel<LIF, DELTA>) : (exponential ? aheadNeuronKernel<IZH, EXP> : aheadNeuronKernel<IZH, DELTA>);
-}
-
 static int setupAhead(gennmi_runner *r, uint32_t numCU)
 {
     const char *env = getenv("GENNMI_AHEAD");
@@ -1438,7 +1431,7 @@ static int launchAhead(gennmi_runner *r, unsigned long long timestep, unsigned l
     const AheadArgs a{timestep, r->epoch, steps, B, (uint32_t)std::max<unsigned long long>(1, numRecordingTimesteps), r->dt};
     const gennmi_neuron_update_group_t &g = r->neuron[r->aheadTarget].g;
     const auto convKernel = aheadConvInstance(g);
-    const auto neuronKernel = aheadNeuronInstance(g);
+    const auto neuronKernel = (slices == 1) ? aheadNeuronInstance<1>(g) : (slices == 2) ? aheadNeuronInstance<2>(g) : aheadNeuronInstance<0>(g);
     aheadSourceKernel<<<dim3((numSrc + BLOCK - 1) / BLOCK, B), dim3(BLOCK), 0, r->stream>>>(r->dAhead, a, r->aheadConv, numTrg, words, r->dEvents);
     if(conv) {
         const AheadConv &C = r->aheadConv;

@@ -415,7 +415,8 @@ struct AheadNeuron
         if(MODEL != GENNMI_NEURON_LIF) { return plainNeuronStep(constants, Isyn, dt, v0, v1); }
         const float alpha = ((Isyn + constants.p[0]) * constants.p[1]) + constants.p[2];
         const bool free = (v1 <= 0.0f);
-        const float moved = alpha - (constants.p[3] * (alpha - v0)), waited = v1 - dt;
+        float moved = alpha - (constants.p[3] * (alpha - v0)), waited = v1 - dt;
+        asm volatile("" : "+v"(moved), "+v"(waited));       // (the compiler would make a branch around them again)
         v0 = free ? moved : v0;
         v1 = free ? v1 : waited;
         const bool spiked = (v1 <= 0.0f && v0 >= constants.p[4]);
@@ -428,43 +429,59 @@ struct AheadNeuron
 // ---- 3a. the neurons behind a DENSE projection: one lane each, 16 steps' inputs asked for while the 16 before are worked off (a
 // population of 8192 is 128 wavefronts: the chain of steps bounds it, so work-groups are single wavefronts, spread over the chip).
 // The 16 steps are straight code (both paths of a LIF neuron computed, votes kept in a register, stored once a group): 100 steps of 8192
-// neurons 21.4 us with a branch for the refractory neurons, the last step and the recorder in every step, 16.4 without.
-template<uint32_t MODEL, uint32_t PSM>
+// neurons 21.4 us with a branch for the refractory neurons, the last step and the recorder in every step, 16.4 without.  The compiler had put the
+// branch back and waited for a group's inputs as soon as it had asked for them, to add up the slices: with both paths kept apart from that, and one
+// or two slices added up when they are used (SLICES), 16.6 -> 13.2 us.
+template<uint32_t MODEL, uint32_t PSM, uint32_t SLICES>
 __global__ __launch_bounds__(WAVE)
 void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, const float * __restrict__ partial, uint32_t slices, uint32_t mTiles, uint32_t *lastBits)
 {
     const gennmi_neuron_update_group_t &g = target->g;
     const uint32_t n = g.numNeurons, batch = blockIdx.y, lane = threadIdx.x, i = blockIdx.x * WAVE + lane;
     const uint32_t bitmapWords = (n + 31) / 32;
-    const AheadNeuron<MODEL, PSM, true> neuron(g, A.dt);
+    AheadNeuron<MODEL, PSM, true> neuron(g, A.dt);
+    asm volatile("" : "+v"(neuron.constants.p[5]), "+v"(neuron.constants.p[6]));       // (selected between in every step: from scalar registers that is a copy first)
     const size_t bi = (size_t)batch * n + min(i, n - 1);
     uint32_t *recordSpk = g.recordSpk;
     constexpr uint32_t GROUP = 16;
     GLOBAL_AS float *var0 = asGlobal(g.var0), *var1 = asGlobal(g.var1), *outPost = asGlobal(g.psm[0].outPost);
     float v0 = var0[bi], v1 = var1[bi], lin = outPost[bi];
     GLOBAL_AS const float *input = asGlobal(partial) + min(i, n - 1);
-    auto load = [&](uint32_t first, float x[GROUP]) {
+    // a group's inputs, on their way where the source is cut into one or two slices (added up when they are used), or already added up
+    struct Inputs { float x[GROUP], y[SLICES == 2 ? GROUP : 1]; };
+    auto load = [&](uint32_t first, Inputs &to) {
+        const size_t row = ((size_t)(first / 32) * A.batch + batch) * 32 + first % 32, slice = (size_t)mTiles * 32;
+        if(SLICES != 0) {
+            #pragma unroll
+            for(uint32_t u = 0; u < GROUP; u++) {
+                to.x[u] = input[(row + u) * n];
+                if(SLICES == 2) { to.y[u] = input[(row + slice + u) * n]; }
+            }
+            return;
+        }
         #pragma unroll
-        for(uint32_t u = 0; u < GROUP; u++) { x[u] = 0.0f; }
+        for(uint32_t u = 0; u < GROUP; u++) { to.x[u] = 0.0f; }
         #pragma unroll 2
         for(uint32_t k = 0; k < slices; k++) {
-            const size_t row = (((size_t)k * mTiles + (size_t)(first / 32) * A.batch + batch) * 32 + first % 32) * n;
             #pragma unroll
-            for(uint32_t u = 0; u < GROUP; u++) { x[u] += input[row + (size_t)u * n]; }
+            for(uint32_t u = 0; u < GROUP; u++) { to.x[u] += input[(k * slice + row + u) * n]; }
         }
     };
+    auto inputOf = [&](const Inputs &from, uint32_t u) {
+        const float x = (SLICES == 0) ? from.x[u] : 0.0f + from.x[u];
+        return (SLICES == 2) ? x + from.y[u] : x;
+    };
     // A step's votes go to two lanes of `votes`, and a group's steps leave with one store: lane u (16 + u) has the lower (upper) word of step u.
+    const unsigned long long present = __builtin_amdgcn_ballot_w64(i < n);
     const uint32_t voteStep = lane & 15, voteWord = (blockIdx.x * WAVE >> 5) + ((lane >> 4) & 1);
     const bool voteLane = lane < 32 && voteWord < bitmapWords;
-    float now[GROUP], next[GROUP];
-    load(0, now);
     // (`all`: 1, and the steps of the group are one straight piece of code; 0: some of them are beyond the last)
-    auto group = [&](uint32_t first, auto all) {
+    auto group = [&](uint32_t first, const Inputs &now, auto all) {
         uint32_t votes = 0;
         #pragma unroll
         for(uint32_t u = 0; u < GROUP; u++) {
             if(all.value || first + u < A.steps) {
-                const unsigned long long ballot = __ballot(neuron.step(now[u], lin, v0, v1) && i < n);
+                const unsigned long long ballot = __builtin_amdgcn_ballot_w64(neuron.step(inputOf(now, u), lin, v0, v1)) & present;
                 votes = (voteStep == u) ? ((lane & 16) ? (uint32_t)(ballot >> 32) : (uint32_t)ballot) : votes;
             }
         }
@@ -475,13 +492,16 @@ void aheadNeuronKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, 
             if(step + 1 == A.steps) { lastBits[(size_t)batch * bitmapWords + voteWord] = votes; }
         }
     };
-    for(uint32_t first = 0; first < A.steps; first += GROUP) {
+    // (two groups' inputs that change places, not values)
+    auto work = [&](uint32_t first, const Inputs &now, Inputs &next) -> bool {
         if(first + GROUP < A.steps) { load(first + GROUP, next); }
-        if(first + GROUP <= A.steps) { group(first, std::integral_constant<uint32_t, 1>()); }
-        else { group(first, std::integral_constant<uint32_t, 0>()); }
-        #pragma unroll
-        for(uint32_t u = 0; u < GROUP; u++) { now[u] = next[u]; }
-    }
+        if(first + GROUP <= A.steps) { group(first, now, std::integral_constant<uint32_t, 1>()); }
+        else { group(first, now, std::integral_constant<uint32_t, 0>()); }
+        return first + GROUP < A.steps;
+    };
+    Inputs even, odd;
+    load(0, even);
+    for(uint32_t first = 0; work(first, even, odd) && work(first + GROUP, odd, even); first += 2 * GROUP) {}
     if(i < n) { var0[bi] = v0; var1[bi] = v1; outPost[bi] = lin; }
 }
 
@@ -760,6 +780,16 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
         }
         if(valid) { var0[at] = v0; var1[at] = v1; outPost[at] = lin; spikes[at] = fired; }
     }
+}
+
+// (the kernel of the target's neuron model and postsynaptic model)
+template<uint32_t SLICES>
+auto aheadNeuronInstance(const gennmi_neuron_update_group_t &g)
+{
+    constexpr uint32_t LIF = GENNMI_NEURON_LIF, IZH = GENNMI_NEURON_IZHIKEVICH, EXP = GENNMI_PSM_EXPCURR, DELTA = GENNMI_PSM_DELTACURR;
+    const bool lif = (g.model == LIF), exponential = (g.psm[0].kind == EXP);
+    return lif ? (exponential ? aheadNeuronKernel<LIF, EXP, SLICES> : aheadNeuronKernel<LIF, DELTA, SLICES>)
+               : (exponential ? aheadNeuronKernel<IZH, EXP, SLICES> : aheadNeuronKernel<IZH, DELTA, SLICES>);
 }
 
 // The layer's spikes turned from one word per neuron (32 steps) into one word per step (32 neurons): the recording rows and the bitmap of

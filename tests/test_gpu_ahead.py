@@ -40,7 +40,7 @@ def _same_rasters(net, model, oracle, steps):
 
 # sizes around a product's 32 columns, a chunk of 64 sources, a work-group's 512; output pixels around the four of a wavefront, channel
 # counts that make an odd number of taps, more than 32 output channels, an even kernel
-SHAPES = [("dense", (1, 1)), ("dense", (63, 31)), ("dense", (65, 33)), ("dense", (512, 64)), ("dense", (1300, 70)), ("dense", (300, 1000)),
+SHAPES = [("dense", (1, 1)), ("dense", (63, 31)), ("dense", (65, 33)), ("dense", (512, 64)), ("dense", (1300, 70)), ("dense", (300, 1000)), ("dense", (900, 40)),
           ("conv", (1, 1, 1, 1, 3)), ("conv", (5, 7, 3, 4, 3)), ("conv", (9, 6, 1, 33, 5)), ("conv", (8, 8, 16, 32, 3)), ("conv", (6, 5, 2, 40, 1))]
 
 
