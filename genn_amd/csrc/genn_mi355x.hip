@@ -104,6 +104,7 @@ struct gennmi_runner
     uint32_t resQuads = 2;              // 16-byte quads of an entry
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
+    bool leanNeurons = false, ringNeurons = false;      // the populations fit LeanNeurons, RingNeurons
     bool queuesDirect = false;          // a population's blocks sum the counts of all earlier ones (queueDirect)
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
     bool sourcesStale = false;          // startSpike / endSpike / spikeTimes of a spike source were written since nextSpikeTime was built
@@ -2076,6 +2077,8 @@ int gennmi_runner_finalise(gennmi_runner *r)
         const NeuronGroupDev both[2] = {r->neuron[r->aheadSource], r->neuron[r->aheadTarget]};
         HIP_TRY(upload(r->dAhead, both, sizeof(both)));
     }
+    r->leanNeurons = neuronsFit<LeanNeurons>(r->neuron);
+    r->ringNeurons = neuronsFit<RingNeurons>(r->neuron);
     HIP_TRY(uploadPerBlock(r->neuron, r->neuronBlocks, &r->dNeuron));
     HIP_TRY(uploadPerBlock(r->pre, r->preBlocks, &r->dPre));
     HIP_TRY(uploadPerBlock(r->post, r->postBlocks, &r->dPost));
@@ -2229,7 +2232,8 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed);
 
 static int launchFusedStep(gennmi_runner *r, const StepArgs &a)
 {
-    stepFusedKernel<<<dim3(r->neuronBlocks + r->preBlocks, r->batch), dim3(BLOCK), 0, r->stream>>>(
+    const auto kernel = r->ringNeurons ? stepFusedKernel<RingNeurons> : stepFusedKernel<AnyNeurons>;
+    kernel<<<dim3(r->neuronBlocks + r->preBlocks, r->batch), dim3(BLOCK), 0, r->stream>>>(
         r->dNeuron, r->neuronBlocks, r->dPre, a, r->dt, r->dAgg, r->dError, r->dEvents);
     HIP_TRY(hipGetLastError());
     return GENNMI_OK;
@@ -2252,8 +2256,11 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed)
     if(r->neuronsPerLane == 2) { neuronBulkKernel<2><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
     else if(r->neuronsPerLane == 4) { neuronBulkKernel<4><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
     else if(r->neuronsPerLane == 8) { neuronBulkKernel<8><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
-    else if(r->queuesDirect) { neuronUpdateKernel<true><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
-    else { neuronUpdateKernel<false><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
+    else {
+        const auto kernel = r->queuesDirect ? (r->leanNeurons ? neuronUpdateKernel<LeanNeurons, true> : neuronUpdateKernel<AnyNeurons, true>)
+                                            : (r->leanNeurons ? neuronUpdateKernel<LeanNeurons, false> : neuronUpdateKernel<AnyNeurons, false>);
+        kernel<<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError);
+    }
     if(timed) { const int rc = stamp(r, &e1); if(rc) { return rc; } r->pending.push_back({e0, e1, 2}); }
     HIP_TRY(hipGetLastError());
     return GENNMI_OK;

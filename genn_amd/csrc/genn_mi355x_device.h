@@ -45,7 +45,7 @@ struct StepArgs              // per launch: what a step's kernels know of time
 // counter fits 32 bits for the first 4e9 steps
 __device__ __forceinline__ uint32_t modStep(unsigned long long x, uint32_t d)
 {
-    return (x >> 32) ? (uint32_t)(x % d) : ((uint32_t)x % d);
+    return __builtin_expect((x >> 32) != 0, 0) ? (uint32_t)(x % d) : ((uint32_t)x % d);
 }
 
 // Synapses whose dendritic delay is a multiple of the ring depth land in the slot the target reads in

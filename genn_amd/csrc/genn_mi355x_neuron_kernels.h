@@ -201,6 +201,37 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
     __syncthreads();            // the shared words are reused by the next call
 }
 
+// What the populations of a launch may have.  A launch fetches its instructions anew, and a path that jumps over what a population does not have fetches a
+// little of each; an instance without it is 840 to 1,200 instructions instead of 5,400 to 6,300.  us a launch, AnyNeurons / LeanNeurons: 4,000 LIF neurons 4.57 / 4.16,
+// 17,011 4.92 / 4.52, 100,000 5.72 / 5.44, 300,007 6.02 / 5.68; stepFusedKernel on the microcircuit at 0.35 with Poisson sources, AnyNeurons / RingNeurons 6.60 / 6.00.
+struct AnyNeurons       // whatever a description can say
+{
+    static constexpr uint32_t PSM = GENNMI_MAX_PSM, CS = GENNMI_MAX_CS;
+    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = true;     // dendritic delays; sources other than DC; shadow queues and zero delays; events, presynaptic output, axonal delays
+};
+struct LeanNeurons      // few inputs without delays, at most a constant current
+{
+    static constexpr uint32_t PSM = 4, CS = 1;
+    static constexpr bool RINGS = false, SOURCES = false, SHADOW = false, REST = false;
+};
+struct RingNeurons      // the single-launch step's
+{
+    static constexpr uint32_t PSM = 2, CS = 1;
+    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = false;
+};
+template<typename HAS>
+inline bool neuronsFit(const std::vector<NeuronGroupDev> &groups)
+{
+    return std::all_of(groups.begin(), groups.end(), [](const NeuronGroupDev &n) {
+        const gennmi_neuron_update_group_t &g = n.g;
+        bool fits = g.numPSM <= HAS::PSM && g.numCS <= HAS::CS && (HAS::SHADOW || (!n.zeroStart && !n.shadowSpk))
+                    && (HAS::REST || (g.numPreOutput == 0 && g.numSpkEvent == 0 && g.numDelaySlots <= 1));
+        for(uint32_t m = 0; m < g.numPSM; m++) { fits = fits && (HAS::RINGS || g.psm[m].maxDenDelay == 0); }
+        for(uint32_t c = 0; c < g.numCS; c++) { fits = fits && (HAS::SOURCES || g.cs[c].kind == GENNMI_CS_DC); }
+        return fits;
+    });
+}
+
 // ------------------------------------------------------------------------------------------------
 // Neuron update.  One lane per neuron.  Spikes are emitted in ascending neuron index (the CPU
 // backend's order, single_threaded_cpu/backend.cc:321, 2119-2133): wave ballot gives the in-wave
@@ -208,7 +239,7 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
 // (tagged with the step so nothing ever needs clearing) the cross-block offset.  Only blocks that
 // emitted spikes, and the last block of each population (which stores spkCnt), look back.
 // ------------------------------------------------------------------------------------------------
-template<bool DIRECT = true>
+template<typename HAS, bool DIRECT = true>
 __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                            const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
@@ -224,16 +255,18 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint32_t wave = threadIdx.x / WAVE;
     const float t = st.t;
+    constexpr uint32_t MAX_PSM = HAS::PSM, MAX_CS = HAS::CS;
 
     bool spiked = false;
     float vEvent = 0.0f;
     uint32_t z0 = 0, z1 = 0;
-    if(G.zeroStart && i < n) { z0 = asGlobal(G.zeroStart)[i]; z1 = asGlobal(G.zeroStart)[i + 1]; }
+    if(HAS::SHADOW && G.zeroStart && i < n) { z0 = asGlobal(G.zeroStart)[i]; z1 = asGlobal(G.zeroStart)[i + 1]; }
     // what the update leaves to be stored (see storeState below)
     float l0 = 0, l1 = 0, preTrace = 0, postTrace = 0;
-    float lin[GENNMI_MAX_PSM];
+    float lin[MAX_PSM];
+    uint32_t ringSlot[MAX_PSM];
     #pragma unroll
-    for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) { lin[m] = 0.0f; }
+    for(uint32_t m = 0; m < MAX_PSM; m++) { lin[m] = 0.0f; }
     if(i < n) {
         // order of operations: neuronUpdateGroupMerged.cc:552-773 — PSMs, current sources, sim code,
         // WU pre/post dynamics, threshold, then (on a spike) WU pre/post spike code, sT, reset
@@ -248,36 +281,39 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
             // descriptor in memory, so a store in between would force the compiler to re-read the descriptor
             // and would serialise the loads, and each dependent access costs about a microsecond at the start of
             // a launch (nothing is cached yet).  Sums keep the reference's order (PSMs, then current sources).
-            float front[GENNMI_MAX_PSM], inj[GENNMI_MAX_CS], rev[GENNMI_MAX_PRE_OUTPUT];
-            const uint32_t numPSM = g.numPSM, numCS = g.numCS, numRev = g.numPreOutput;
+            float front[MAX_PSM], inj[MAX_CS], rev[GENNMI_MAX_PRE_OUTPUT];
+            const uint32_t numPSM = g.numPSM, numCS = g.numCS, numRev = HAS::REST ? g.numPreOutput : 0u;
             #pragma unroll
             for(uint32_t q = 0; q < GENNMI_MAX_PRE_OUTPUT; q++) { rev[q] = (q < numRev) ? asGlobal(g.outPre[q])[bi] : 0.0f; }
             l0 = asGlobal(g.var0)[bi]; l1 = asGlobal(g.var1)[bi];
             #pragma unroll
-            for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) {
+            for(uint32_t m = 0; m < MAX_PSM; m++) {
                 lin[m] = 0.0f; front[m] = 0.0f;
                 if(m < numPSM) {
                     lin[m] = asGlobal(g.psm[m].outPost)[bi];
-                    const uint32_t D = g.psm[m].maxDenDelay;
-                    if(D) { front[m] = asGlobal(g.psm[m].denDelay)[((size_t)batch * D + modStep(st.epoch + 1, D)) * n + i]; }
+                    const uint32_t D = HAS::RINGS ? g.psm[m].maxDenDelay : 0u;
+                    if(D) {
+                        ringSlot[m] = modStep(st.epoch + 1, D);
+                        front[m] = asGlobal(g.psm[m].denDelay)[((size_t)batch * D + ringSlot[m]) * n + i];
+                    }
                 }
             }
             #pragma unroll
-            for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) {
+            for(uint32_t c = 0; c < MAX_CS; c++) {
                 inj[c] = 0.0f;
                 if(c < numCS) {
-                    inj[c] = (g.cs[c].kind == GENNMI_CS_DC) ? g.cs[c].amp
+                    inj[c] = (!HAS::SOURCES || g.cs[c].kind == GENNMI_CS_DC) ? g.cs[c].amp
                            : (g.cs[c].kind == GENNMI_CS_ARRAY) ? asGlobal(g.cs[c].array)[(size_t)modStep(st.epoch, g.cs[c].arraySteps) * n + i]
                                                                : poissonExpInject(g.cs[c], asGlobal(g.cs[c].current), bi, st.epoch);
                 }
             }
             float Isyn = 0;
             #pragma unroll
-            for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) {
+            for(uint32_t m = 0; m < MAX_PSM; m++) {
                 if(m < numPSM) {
                     // read and clear the front slot of the ring (neuronUpdateGroupMerged.cc:84-101)
                     float linSyn = lin[m];
-                    const uint32_t D = g.psm[m].maxDenDelay;
+                    const uint32_t D = HAS::RINGS ? g.psm[m].maxDenDelay : 0u;
                     if(D) { linSyn += front[m]; }
                     if(g.psm[m].kind == GENNMI_PSM_EXPCURR) {
                         Isyn += g.psm[m].init * linSyn;
@@ -294,7 +330,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
             #pragma unroll
             for(uint32_t q = 0; q < GENNMI_MAX_PRE_OUTPUT; q++) { if(q < numRev) { Isyn += rev[q]; } }
             #pragma unroll
-            for(uint32_t c = 0; c < GENNMI_MAX_CS; c++) { if(c < numCS) { Isyn += inj[c]; } }
+            for(uint32_t c = 0; c < MAX_CS; c++) { if(c < numCS) { Isyn += inj[c]; } }
             if(g.model == GENNMI_NEURON_LIF) {
                 if(l1 <= 0.0f) {
                     const float alpha = ((Isyn + g.params[0]) * g.params[1]) + g.params[2];
@@ -338,14 +374,14 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
                 }
             }
             else {
-                const uint32_t numPSM = g.numPSM, numRev = g.numPreOutput;
+                const uint32_t numPSM = g.numPSM, numRev = HAS::REST ? g.numPreOutput : 0u;
                 #pragma unroll
                 for(uint32_t q = 0; q < GENNMI_MAX_PRE_OUTPUT; q++) { if(q < numRev) { storeThrough(&asGlobal(g.outPre[q])[bi], 0.0f); } }
                 #pragma unroll
-                for(uint32_t m = 0; m < GENNMI_MAX_PSM; m++) {
+                for(uint32_t m = 0; m < MAX_PSM; m++) {
                     if(m < numPSM) {
-                        const uint32_t D = g.psm[m].maxDenDelay;
-                        if(D) { storeThrough(&asGlobal(g.psm[m].denDelay)[((size_t)batch * D + modStep(st.epoch + 1, D)) * n + i], 0.0f); }
+                        const uint32_t D = HAS::RINGS ? g.psm[m].maxDenDelay : 0u;
+                        if(D) { storeThrough(&asGlobal(g.psm[m].denDelay)[((size_t)batch * D + ringSlot[m]) * n + i], 0.0f); }
                         storeThrough(&asGlobal(g.psm[m].outPost)[bi], lin[m]);
                     }
                 }
@@ -356,14 +392,14 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
             if(g.postTrace) { storeThrough(&asGlobal(g.postTrace)[bi], postTrace); }
         }
         // keep the user-visible ring pointers current (nothing in the kernels reads them)
-        if(localBlock == 0 && batch == 0 && threadIdx.x < g.numPSM) {
+        if(HAS::RINGS && localBlock == 0 && batch == 0 && threadIdx.x < g.numPSM) {
             const gennmi_psm_t &psm = g.psm[threadIdx.x];
             if(psm.maxDenDelay && psm.denDelayPtr) { *psm.denDelayPtr = modStep(st.epoch + 1, psm.maxDenDelay); }
         }
     };
 
     // ---- spike-like events: one ordered queue per event condition ----------------------------------
-    if(g.numSpkEvent) {
+    if(HAS::REST && g.numSpkEvent) {
         const size_t perArea = (size_t)totalNeuronBlocks * gridDim.y;
         for(uint32_t e = 0; e < g.numSpkEvent; e++) {
             unsigned long long *counts = G.aggEvent + (size_t)e * 2 * perArea;
@@ -427,7 +463,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
             }
         }
     };
-    if(G.zeroStart && wave != 0) { deliverZeroDelay(); }
+    if(HAS::SHADOW && G.zeroStart && wave != 0) { deliverZeroDelay(); }
 
     if(!direct && wave == 0) {
         // Two-level offset: blocks of a population form groups of 64.  The last block of a group sums the
@@ -479,7 +515,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     if(prefix == 0xFFFFFFFFu) { return; }       // bounded wait expired: flagged, nothing written
     // with axonal delay the queue is a ring of slots and this step writes slot (epoch + 1) % slots: the reference's
     // spkQuePtr after the increment at the start of its updateNeurons (neuronUpdateGroupMerged.cc:947-953)
-    const uint32_t delaySlots = max(1u, g.numDelaySlots);
+    const uint32_t delaySlots = HAS::REST ? max(1u, g.numDelaySlots) : 1u;
     const size_t queue = (size_t)batch * delaySlots + ((delaySlots > 1) ? modStep(st.epoch + 1, delaySlots) : 0u);
     if(spiked) { g.spk[queue * n + prefix + waveOffset + laneRank] = i; }
     if(last && threadIdx.x == 0) { g.spkCnt[queue] = prefix + blockCount; }
@@ -489,22 +525,22 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
         if(spiked) { g.extraSpk[q][(size_t)batch * n + prefix + waveOffset + laneRank] = i; }
         if(last && threadIdx.x == 0) { g.extraSpkCnt[q][batch] = prefix + blockCount; }
     }
-    if(G.shadowSpk) {
+    if(HAS::SHADOW && G.shadowSpk) {
         const uint32_t parity = (uint32_t)(st.epoch & 1);
         if(spiked) { G.shadowSpk[((size_t)parity * gridDim.y + batch) * n + prefix + waveOffset + laneRank] = i; }
         if(last && threadIdx.x == 0) { G.shadowCnt[(size_t)parity * gridDim.y + batch] = prefix + blockCount; }
     }
-    if(G.zeroStart && wave == 0) { deliverZeroDelay(); }
+    if(HAS::SHADOW && G.zeroStart && wave == 0) { deliverZeroDelay(); }
 }
 
 // (DIRECT: one of the populations is queueDirect.  Where none is, a step that has that code compiled in is slower: DENSE 8192 x 8192 stepped 9.75 us a step
 // before there was such code, 9.91 with it, 9.79 without; 1000 x 500 batch 4 8.85, 9.02 and 8.88)
-template<bool DIRECT>
+template<typename HAS, bool DIRECT>
 __global__ __launch_bounds__(BLOCK)
 void neuronUpdateKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args, float dt,
                         unsigned long long *agg, uint32_t *errorFlag)
 {
-    neuronBody<DIRECT>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag);
+    neuronBody<HAS, DIRECT>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -755,6 +791,7 @@ void neuronBulkKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args,
 // synapses are delivered by the spiking neuron itself, and the presynaptic update reads the shadow spike
 // queue of step t-1 while the neuron update refills the visible one.  Neuron blocks come first so that
 // their look-back chain starts early.
+template<typename HAS>
 __global__ __launch_bounds__(BLOCK)
 void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t numNeuronBlocks, const PreGroupDev * __restrict__ preBlocks,
                      StepArgs args, float dt, unsigned long long *agg, uint32_t *errorFlag, unsigned long long *eventCounter)
@@ -766,7 +803,7 @@ void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t 
         __builtin_amdgcn_s_setprio(3);
         // (offsets in two levels throughout: 50 steps of the full microcircuit 562 us, with sumOfEarlierBlocks in this kernel 569.  2000 steps of 0.35 of it
         // 13.50 ms in this kernel before there was a sumOfEarlierBlocks, 13.66 with it for spike-like events only, which no step there has, 13.27 without)
-        neuronBody<false>(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
+        neuronBody<HAS, false>(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
     }
     else { presynapticBody(preBlocks[blockIdx.x - numNeuronBlocks], blockIdx.x - numNeuronBlocks, blockIdx.y, gridDim.y, st, dt, eventCounter); }
 }
