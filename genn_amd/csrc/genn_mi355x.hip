@@ -104,6 +104,7 @@ struct gennmi_runner
     uint32_t resQuads = 2;              // 16-byte quads of an entry
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
+    bool staticRows = false, plasticRows = false;       // the scatter path's projections fit StaticRows (and nothing learns), PlasticRows
     bool leanNeurons = false, ringNeurons = false;      // the populations fit LeanNeurons, RingNeurons
     bool queuesDirect = false;          // a population's blocks sum the counts of all earlier ones (queueDirect)
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
@@ -1322,6 +1323,10 @@ static int refreshTables(gennmi_runner *r)
     return GENNMI_OK;
 }
 
+static auto combinedInstance(const gennmi_runner *r)
+{
+    return r->staticRows ? synapseCombinedKernel<StaticRows> : r->plasticRows ? synapseCombinedKernel<PlasticRows> : synapseCombinedKernel<AnyRows>;
+}
 static auto convStepInstance(const gennmi_runner *r) { return r->convQueuesDirect ? convStepKernel<true> : convStepKernel<false>; }
 
 // Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
@@ -1985,8 +1990,10 @@ int gennmi_runner_finalise(gennmi_runner *r)
         const char *envCombined = getenv("GENNMI_COMBINED");
         r->combineSynapses = !r->ordered && !(envCombined && atoi(envCombined) == 0) && (r->tileBlocks != 0 || r->combinePost);
         r->combinedLdsBytes = std::max<size_t>(r->tileBlocks ? (size_t)r->tileFloats * sizeof(float) : 0, r->combinePost ? r->postLdsBytes : 0);
+        r->staticRows = r->post.empty() && rowsFit<StaticRows>(r->pre);
+        r->plasticRows = rowsFit<PlasticRows>(r->pre);
         if(r->combineSynapses && r->combinedLdsBytes > 48 * 1024) {
-            HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(synapseCombinedKernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)r->combinedLdsBytes));
+            HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(combinedInstance(r)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)r->combinedLdsBytes));
         }
     }
     if(r->ordered && r->batch != 1 && !r->post.empty()) { return fail(GENNMI_EUNSUPPORTED, "runner_finalise: ordered accumulation of plastic projections needs batch size 1"); }
@@ -2197,7 +2204,8 @@ static int launchSynapses(gennmi_runner *r, const StepArgs &a, bool timed)
             const uint32_t scatterBlocks = (r->preBlocks && r->scatterNeeded) ? r->preBlocks : 0u;
             const uint32_t postBlocks = r->combinePost ? r->postBlocks : 0u;
             postInCombined = (postBlocks != 0);
-            synapseCombinedKernel<<<dim3(scatterBlocks + r->tileBlocks + postBlocks, r->batch), dim3(r->synapseThreads), r->combinedLdsBytes, r->stream>>>(
+            const auto kernel = combinedInstance(r);
+            kernel<<<dim3(scatterBlocks + r->tileBlocks + postBlocks, r->batch), dim3(r->synapseThreads), r->combinedLdsBytes, r->stream>>>(
                 r->dPre, scatterBlocks, r->dTile, r->tileBlocks, r->dPost, a, r->dt, r->dEvents);
         }
         else if(r->preBlocks && r->scatterNeeded && !(r->convMfmaBlocks && !timed)) {
@@ -2232,7 +2240,7 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed);
 
 static int launchFusedStep(gennmi_runner *r, const StepArgs &a)
 {
-    const auto kernel = r->ringNeurons ? stepFusedKernel<RingNeurons> : stepFusedKernel<AnyNeurons>;
+    const auto kernel = r->ringNeurons ? stepFusedKernel<RingNeurons, DelayRows> : stepFusedKernel<AnyNeurons, DelayRows>;
     kernel<<<dim3(r->neuronBlocks + r->preBlocks, r->batch), dim3(BLOCK), 0, r->stream>>>(
         r->dNeuron, r->neuronBlocks, r->dPre, a, r->dt, r->dAgg, r->dError, r->dEvents);
     HIP_TRY(hipGetLastError());

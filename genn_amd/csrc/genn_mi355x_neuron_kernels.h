@@ -791,7 +791,7 @@ void neuronBulkKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args,
 // synapses are delivered by the spiking neuron itself, and the presynaptic update reads the shadow spike
 // queue of step t-1 while the neuron update refills the visible one.  Neuron blocks come first so that
 // their look-back chain starts early.
-template<typename HAS>
+template<typename HAS, typename ROWS>
 __global__ __launch_bounds__(BLOCK)
 void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t numNeuronBlocks, const PreGroupDev * __restrict__ preBlocks,
                      StepArgs args, float dt, unsigned long long *agg, uint32_t *errorFlag, unsigned long long *eventCounter)
@@ -805,7 +805,7 @@ void stepFusedKernel(const NeuronGroupDev * __restrict__ neuronBlocks, uint32_t 
         // 13.50 ms in this kernel before there was a sumOfEarlierBlocks, 13.66 with it for spike-like events only, which no step there has, 13.27 without)
         neuronBody<HAS, false>(neuronBlocks[blockIdx.x], blockIdx.x, numNeuronBlocks, st, dt, agg, errorFlag);
     }
-    else { presynapticBody(preBlocks[blockIdx.x - numNeuronBlocks], blockIdx.x - numNeuronBlocks, blockIdx.y, gridDim.y, st, dt, eventCounter); }
+    else { presynapticBody<ROWS>(preBlocks[blockIdx.x - numNeuronBlocks], blockIdx.x - numNeuronBlocks, blockIdx.y, gridDim.y, st, dt, eventCounter); }
 }
 
 // Per row: count the synapses with d % D == 0 and, when `entries` is given, append them at offset[row].

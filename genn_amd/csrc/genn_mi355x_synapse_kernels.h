@@ -45,6 +45,38 @@ __device__ __forceinline__ bool bitmapTest(GLOBAL_AS const uint32_t *bitmap, uin
 // round-robin to the sub-groups of the synapse group's blocks, so the launch geometry is fixed
 // while the spike count lives on the device.
 // ------------------------------------------------------------------------------------------------
+// What the projections of a launch may have (as for the neuron kernels: a launch fetches its instructions anew, and a path that jumps over what there is none of
+// fetches a little of each).  us a launch of quiet steps, AnyRows for all / as here: 4,000 LIF neurons x 80 4.3 / 3.6, 300,007 x 1000 3.2 / 2.64, plastic 17,011 x 300 3.7 / 3.24,
+// 100,000 x 500 5.4 / 4.96; the combined kernel has 6,300 instructions for static rows, 11,300 with plastic ones, 12,500 with everything.
+struct AnyRows          // whatever the scatter path takes
+{
+    static constexpr bool CONV = true, STATIC = true, DELAY = true, REVERSE = true, GRADED = true, PLASTIC = true, AXONAL = true, SHADOW = true;
+};
+struct StaticRows       // stored rows of weights that do not change, nothing delayed
+{
+    static constexpr bool CONV = false, STATIC = true, DELAY = false, REVERSE = false, GRADED = false, PLASTIC = false, AXONAL = false, SHADOW = false;
+};
+struct PlasticRows      // the same, and rows that learn
+{
+    static constexpr bool CONV = false, STATIC = true, DELAY = false, REVERSE = false, GRADED = false, PLASTIC = true, AXONAL = false, SHADOW = false;
+};
+struct DelayRows        // the single-launch step's: dendritic delays, sources with a shadow queue
+{
+    static constexpr bool CONV = false, STATIC = false, DELAY = true, REVERSE = false, GRADED = false, PLASTIC = false, AXONAL = false, SHADOW = true;
+};
+template<typename HAS>
+inline bool rowsFit(const std::vector<PreGroupDev> &groups)
+{
+    return std::all_of(groups.begin(), groups.end(), [](const PreGroupDev &p) {
+        const gennmi_presynaptic_update_group_t &g = p.g;
+        const bool conv = (g.matrix == GENNMI_MATRIX_TOEPLITZ_CONV2D);
+        const bool kind = (g.wum == GENNMI_WUM_STATIC_PULSE) ? (conv ? HAS::CONV : HAS::STATIC) : (g.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) ? HAS::DELAY
+                        : (g.wum == GENNMI_WUM_STATIC_PULSE_REVERSE) ? HAS::REVERSE : (g.wum == GENNMI_WUM_STATIC_GRADED) ? HAS::GRADED : HAS::PLASTIC;
+        return kind && (g.matrix == GENNMI_MATRIX_SPARSE || (conv && HAS::CONV)) && (HAS::AXONAL || g.numSrcDelaySlots <= 1) && (HAS::SHADOW || !p.shadowSpk);
+    });
+}
+
+template<typename HAS>
 __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t blockInKernel, uint32_t batch, uint32_t numBatches,
                                                 const StepArgs &st, float dt, unsigned long long *eventCounter)
 {
@@ -67,23 +99,23 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
     const uint32_t parity = (uint32_t)((st.epoch + 1) & 1);
     // axonal delay: the source's queue is a ring of slots; this projection reads the slot written axonalDelaySteps + 1
     // updates ago, (spkQuePtr + slots - delay) % slots with spkQuePtr = epoch % slots (backendBase.cc:207-216)
-    const uint32_t slots = max(1u, g.numSrcDelaySlots);
+    const uint32_t slots = HAS::AXONAL ? max(1u, g.numSrcDelaySlots) : 1u;
     const uint32_t readSlot = (slots > 1) ? modStep(st.epoch + slots - g.axonalDelaySteps, slots) : 0u;
-    GLOBAL_AS const uint32_t *cntPtr = G.shadowSpk ? asGlobal(G.shadowCnt) + (size_t)parity * numBatches + batch
+    GLOBAL_AS const uint32_t *cntPtr = (HAS::SHADOW && G.shadowSpk) ? asGlobal(G.shadowCnt) + (size_t)parity * numBatches + batch
                                                    : asGlobal(g.srcSpkCnt) + ((size_t)batch * slots + readSlot);
-    GLOBAL_AS const uint32_t *spk = G.shadowSpk ? asGlobal(G.shadowSpk) + ((size_t)parity * numBatches + batch) * g.numSrcNeurons
+    GLOBAL_AS const uint32_t *spk = (HAS::SHADOW && G.shadowSpk) ? asGlobal(G.shadowSpk) + ((size_t)parity * numBatches + batch) * g.numSrcNeurons
                                                 : asGlobal(g.srcSpk) + ((size_t)batch * slots + readSlot) * g.numSrcNeurons;
     // the first spike id this sub-group would handle is fetched together with the count, not after it (the
     // queue always holds numSrcNeurons entries, so any index below that is readable)
     const uint32_t sparseSpan = W * (G.vec4 ? 4u : 1u);
     const uint32_t sparseChunksPerRow = (g.rowStride + sparseSpan - 1) / sparseSpan;
-    const uint32_t firstSpike = (g.matrix == GENNMI_MATRIX_SPARSE) ? spk[min(subGroup / max(sparseChunksPerRow, 1u), g.numSrcNeurons - 1)] : 0u;
+    const uint32_t firstSpike = (!HAS::CONV || g.matrix == GENNMI_MATRIX_SPARSE) ? spk[min(subGroup / max(sparseChunksPerRow, 1u), g.numSrcNeurons - 1)] : 0u;
     const uint32_t numSpikes = cntPtr[0];
     if(G.tileThreshold && (unsigned long long)numSpikes * G.workPerSpike >= G.tileThreshold) { return; }
     GLOBAL_AS float *outPost = asGlobal(g.outPost) + (size_t)batch * g.numTrgNeurons;
     unsigned long long events = 0;
 
-    if(g.matrix == GENNMI_MATRIX_TOEPLITZ_CONV2D) {
+    if(HAS::CONV && g.matrix == GENNMI_MATRIX_TOEPLITZ_CONV2D) {
         // initToeplitzConnectivitySnippet.h:116-137; lanes span the kh*kw*oc diagonals, so
         // consecutive lanes hit consecutive output channels (consecutive outPost addresses)
         const int kh = g.conv[0], kw = g.conv[1], iw = g.conv[3], ic = g.conv[4];
@@ -121,7 +153,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
         }
     }
     else {
-        const uint32_t D = g.maxDenDelay;
+        const uint32_t D = HAS::DELAY ? g.maxDenDelay : 0u;
         // *denDelayPtr = (*denDelayPtr + 1) % D happens at the start of updateSynapses
         // (synapseUpdateGroupMerged.cc:480-483); st.epoch counts completed steps, so the pointer
         // in force during this step is (epoch + 1) % D.
@@ -155,7 +187,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
             const uint32_t j = chunk * span + lis * perLane;
             const bool inRow = (j < g.rowStride);
             const uint32_t npost = rowLength[idPre];
-            if(g.wum == GENNMI_WUM_STATIC_PULSE) {
+            if(HAS::STATIC && g.wum == GENNMI_WUM_STATIC_PULSE) {
                 if(G.vec4) {
                     u32x4 ip = {0, 0, 0, 0}; f32x4 w = {0, 0, 0, 0};
                     if(inRow) {
@@ -173,7 +205,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
                     if(j < npost) { atomicAddF32(&outPost[ip], w); }
                 }
             }
-            else if(g.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) {
+            else if(HAS::DELAY && g.wum == GENNMI_WUM_STATIC_PULSE_DENDRITIC_DELAY) {
                 // addToPostDelay(g, d): denDelay[((ptr + d) % D) * numPost + idPost] += g  (synapseUpdateGroupMerged.cc:245-251)
                 if(G.vec4) {
                     u32x4 ip = {0, 0, 0, 0}; f32x4 w = {0, 0, 0, 0}; u8x4 dl = {0, 0, 0, 0};
@@ -196,7 +228,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
                     if(j < npost && !(G.skipZeroDelay && slot == denPtr)) { atomicAddF32(&denDelay[(size_t)slot * numTrg + ip], w); }
                 }
             }
-            else if(g.wum == GENNMI_WUM_STATIC_PULSE_REVERSE) {
+            else if(HAS::REVERSE && g.wum == GENNMI_WUM_STATIC_PULSE_REVERSE) {
                 // addToPre(g): the weights of the row go to the spiking neuron itself; a lane sums its share, the lanes of the
                 // (spike, chunk) item combine theirs, one atomic per item
                 float sum = 0.0f;
@@ -204,7 +236,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
                 for(uint32_t off = W / 2; off > 0; off >>= 1) { sum += __shfl_xor(sum, off, WAVE); }
                 if(lis == 0 && sum != 0.0f) { atomicAddF32(asGlobal(g.outPre) + (size_t)batch * g.numSrcNeurons + idPre, sum); }
             }
-            else if(g.wum == GENNMI_WUM_STATIC_GRADED) {
+            else if(HAS::GRADED && g.wum == GENNMI_WUM_STATIC_GRADED) {
                 // event code of weightUpdateModels.h:318: addToPost(fmax(0.0, g * tanh((V_pre - Epre) / Vslope) * dt)).  The CPU
                 // backend's generated code evaluates tanh, the products and the maximum in double (only the double versions of
                 // tanh and fmax are in scope there); so does this, rounding once before the fp32 atomic.
@@ -216,7 +248,7 @@ __device__ __forceinline__ void presynapticBody(const PreGroupDev &G, uint32_t b
                     }
                 }
             }
-            else {
+            else if(HAS::PLASTIC) {
                 // trace STDP presynaptic-spike code (pygenn/genn_model.py:1456-1463); every synapse of
                 // the row is owned by exactly one lane, so the read-modify-write of g needs no atomic
                 // (plastic weights, spike times and traces are per batch: VarAccess::READ_WRITE variables are duplicated).
@@ -530,6 +562,7 @@ __device__ __forceinline__ unsigned long long tileRecordLoop(const TileGroupDev 
 
 constexpr uint32_t TILE_SEGMENTS = 2;                   // spikes whose segments a sub-group of the tile kernel takes together
 constexpr uint32_t TILE_NO_CHANGE = 0x7FC0DEADu;        // (a NaN no computation makes) the presynaptic-spike rule leaves this target's synapses alone
+template<bool PLASTIC>
 __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float *shTile, const StepArgs &args, float dt, unsigned long long *eventCounter)
 {
     const gennmi_presynaptic_update_group_t &g = G.g;
@@ -571,13 +604,13 @@ __device__ __forceinline__ void presynapticTileBody(const TileGroupDev &G, float
     // synapse (pygenn/genn_model.py:1456-1463); a synapse belongs to exactly one tile, so g needs no atomic here either.
     // Plastic weights, spike times and traces are per batch.
     const bool additive = (g.wum == GENNMI_WUM_STDP);
-    const bool stdp = (g.wum == GENNMI_WUM_STDP_TRACE) || additive;
+    const bool stdp = PLASTIC && ((g.wum == GENNMI_WUM_STDP_TRACE) || additive);
     GLOBAL_AS float *weight = asGlobal(g.g) + (stdp ? (size_t)batch * g.numSrcNeurons * g.rowStride : (size_t)0);
     const float t = stdp ? args.t : 0.0f;
     GLOBAL_AS const float *trgST = asGlobal(g.trgST) + (size_t)batch * g.numTrgNeurons;
     GLOBAL_AS const float *postTrace = asGlobal(g.postTrace) + (size_t)batch * g.numTrgNeurons;
     GLOBAL_AS const uint32_t *trgBitmap = asGlobal(G.learn.trgBitmap) + (size_t)batch * ((g.numTrgNeurons + 31) / 32);
-    const bool paired = (G.learn.enabled != 0);
+    const bool paired = PLASTIC && (G.learn.enabled != 0);
     // the rule on one synapse, given what it reads of its target: last spike time, trace, word of the spike bitmap
     // (what the postsynaptic-spike rule reads of the row's own neuron — rowST, rowTrace — is loaded once per row, one row ahead:
     // in a burst most targets have just fired, and two dependent loads per synapse were the longest chain of such a step)
@@ -747,7 +780,7 @@ __global__ __launch_bounds__(1024)
 void presynapticTileKernel(const TileGroupDev * __restrict__ blocks, StepArgs args, float dt, unsigned long long *eventCounter)
 {
     extern __shared__ float shTile[];
-    presynapticTileBody(blocks[blockIdx.x], shTile, args, dt, eventCounter);
+    presynapticTileBody<true>(blocks[blockIdx.x], shTile, args, dt, eventCounter);
 }
 
 // Toeplitz Conv2D counterpart of the tile kernel: every block finds the run of spikes whose kernel footprint touches
@@ -1149,7 +1182,7 @@ void presynapticConvMfmaKernel(const ConvMfmaDev * __restrict__ blocks, uint32_t
     const StepArgs st = args;
     if(blockIdx.x >= mfmaBlocks) {
         const uint32_t b = (blockIdx.x - mfmaBlocks) / numBatches;
-        presynapticBody(scatter[b], b, batch, numBatches, st, dt, eventCounter);
+        presynapticBody<AnyRows>(scatter[b], b, batch, numBatches, st, dt, eventCounter);
         return;
     }
     const uint32_t numDiag = (uint32_t)(g.conv[0] * g.conv[1] * g.conv[7]);
@@ -1202,7 +1235,7 @@ void spikeBitmapFromQueueKernel(const uint32_t *spkCnt, const uint32_t *spk, uin
 __global__ __launch_bounds__(1024)
 void presynapticUpdateKernel(const PreGroupDev * __restrict__ blocks, StepArgs args, float dt, unsigned long long *eventCounter)
 {
-    presynapticBody(blocks[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
+    presynapticBody<AnyRows>(blocks[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1409,18 +1442,19 @@ void postsynapticUpdateKernel(const PostGroupDev * __restrict__ blocks, StepArgs
 // have one (a projection's step is taken by one or the other, decided on the device from its spike count) and the
 // postsynaptic passes whose projections are paired with their presynaptic halves (LearnPostDev: no synapse is written by
 // both, so nothing orders the passes).  Block ranges [0, preBlocks), [preBlocks, preBlocks + tileBlocks), then the rest.
+template<typename ROWS>
 __global__ __launch_bounds__(1024)
 void synapseCombinedKernel(const PreGroupDev * __restrict__ pre, uint32_t preBlocks, const TileGroupDev * __restrict__ tiles, uint32_t tileBlocks,
                            const PostGroupDev * __restrict__ post, StepArgs args, float dt, unsigned long long *eventCounter)
 {
     extern __shared__ float shDynamic[];
     if(blockIdx.x < preBlocks) {
-        presynapticBody(pre[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
+        presynapticBody<ROWS>(pre[blockIdx.x], blockIdx.x, blockIdx.y, gridDim.y, args, dt, eventCounter);
     }
     else if(blockIdx.x < preBlocks + tileBlocks) {
-        presynapticTileBody(tiles[blockIdx.x - preBlocks], shDynamic, args, dt, eventCounter);
+        presynapticTileBody<ROWS::PLASTIC>(tiles[blockIdx.x - preBlocks], shDynamic, args, dt, eventCounter);
     }
-    else {
+    else if(ROWS::PLASTIC) {
         const uint32_t b = blockIdx.x - preBlocks - tileBlocks;
         postsynapticBody(post[b], b, reinterpret_cast<uint32_t*>(shDynamic), args, dt);
     }
