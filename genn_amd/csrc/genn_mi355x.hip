@@ -105,6 +105,7 @@ struct gennmi_runner
     std::vector<u32x2*> resPacked;      // its synapses as the resident kernel reads them
     uint32_t neuronsPerLane = 1;        // 2, 4 or 8: neuronBulkKernel instead of neuronUpdateKernel
     bool staticRows = false, plasticRows = false;       // the scatter path's projections fit StaticRows (and nothing learns), PlasticRows
+    bool leanBulk = false;              // ... neuronBulkBody<LEAN>
     bool leanNeurons = false, ringNeurons = false;      // the populations fit LeanNeurons, RingNeurons
     bool queuesDirect = false;          // a population's blocks sum the counts of all earlier ones (queueDirect)
     bool plainGroups = false;           // every group is one the several-neurons-per-lane neuron update covers
@@ -2086,6 +2087,11 @@ int gennmi_runner_finalise(gennmi_runner *r)
     }
     r->leanNeurons = neuronsFit<LeanNeurons>(r->neuron);
     r->ringNeurons = neuronsFit<RingNeurons>(r->neuron);
+    r->leanBulk = std::all_of(r->neuron.begin(), r->neuron.end(), [](const NeuronGroupDev &n) {
+        bool rings = false;
+        for(uint32_t m = 0; m < n.g.numPSM; m++) { rings = rings || n.g.psm[m].maxDenDelay != 0; }
+        return n.g.model != GENNMI_NEURON_SPIKE_SOURCE_ARRAY && !rings;
+    });
     HIP_TRY(uploadPerBlock(r->neuron, r->neuronBlocks, &r->dNeuron));
     HIP_TRY(uploadPerBlock(r->pre, r->preBlocks, &r->dPre));
     HIP_TRY(uploadPerBlock(r->post, r->postBlocks, &r->dPost));
@@ -2261,9 +2267,10 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed)
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if(timed) { const int rc = stamp(r, &e0); if(rc) { return rc; } }
     const dim3 neuronGrid(r->neuronBlocks, r->batch);
-    if(r->neuronsPerLane == 2) { neuronBulkKernel<2><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
-    else if(r->neuronsPerLane == 4) { neuronBulkKernel<4><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
-    else if(r->neuronsPerLane == 8) { neuronBulkKernel<8><<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); }
+    auto bulk = [&](auto any, auto lean) { (r->leanBulk ? lean : any)<<<neuronGrid, dim3(BLOCK), 0, r->stream>>>(r->dNeuron, a, r->dt, r->dAgg, r->dError); };
+    if(r->neuronsPerLane == 2) { bulk(neuronBulkKernel<2, false>, neuronBulkKernel<2, true>); }
+    else if(r->neuronsPerLane == 4) { bulk(neuronBulkKernel<4, false>, neuronBulkKernel<4, true>); }
+    else if(r->neuronsPerLane == 8) { bulk(neuronBulkKernel<8, false>, neuronBulkKernel<8, true>); }
     else {
         const auto kernel = r->queuesDirect ? (r->leanNeurons ? neuronUpdateKernel<LeanNeurons, true> : neuronUpdateKernel<AnyNeurons, true>)
                                             : (r->leanNeurons ? neuronUpdateKernel<LeanNeurons, false> : neuronUpdateKernel<AnyNeurons, false>);

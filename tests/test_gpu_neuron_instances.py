@@ -45,3 +45,12 @@ def test_populations_and_projections_on_either_side_of_what_an_instance_has(inpu
     model, _, counts = run_side_by_side(net)
     model.unload()
     assert counts["S"] > 0 and counts["T"] > 0
+
+
+@pytest.mark.parametrize("sources", [(), ("dc",), ("noise",)])
+@pytest.mark.parametrize("kinds", [S, D, D + S])
+def test_several_neurons_a_lane_with_delays_and_without(sources, kinds, monkeypatch):
+    monkeypatch.setenv("GENNMI_NEURON_BULK", "1")
+    model, _, counts = run_side_by_side(_net(2, sources, kinds, n_trg=1333))
+    assert model.runner_info()["bulk_neuron_kernel"] and counts["T"] > 0
+    model.unload()
