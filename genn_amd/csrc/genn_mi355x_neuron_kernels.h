@@ -601,7 +601,8 @@ __device__ __forceinline__ bool plainNeuronStep(const PlainNeuron &c, float Isyn
 }
 
 // (THREADS: threads of the calling work-group, all of which call; batch / numBatches: the grid's second dimension in the neuron kernels)
-// (LEAN: no population is a spike source or has dendritic delays; see AnyNeurons.  1,780 instead of 5,850 instructions for four chunks: 10^6 Izhikevich neurons 8.8 -> 7.8 us a launch)
+// (LEAN: no population is a spike source or has dendritic delays; see AnyNeurons.  1,650 instructions for four chunks instead of 2,660, and of 5,850 while what is
+// uniform was decided chunk by chunk: 10^6 Izhikevich neurons 8.8 -> 7.8 us a launch with LEAN alone, 6.8 with straight loads and one decision besides)
 template<int NPL, int THREADS = BLOCK, bool DIRECT = true, bool LEAN = false>
 __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                                const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag,
@@ -631,7 +632,9 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
         psmD[m] = (!LEAN && have) ? g.psm[m].maxDenDelay : 0u; psmKind[m] = have ? g.psm[m].kind : 0u;
         psmInit[m] = have ? g.psm[m].init : 0.0f; psmDecay[m] = have ? g.psm[m].expDecay : 0.0f;
     }
-    // (once, not chunk by chunk)
+    uint32_t ringSlot[BULK_MAX_PSM];
+    #pragma unroll
+    for(uint32_t m = 0; m < BULK_MAX_PSM; m++) { ringSlot[m] = psmD[m] ? modStep(st.epoch + 1, psmD[m]) : 0u; }
     const uint32_t csKind = numCS ? g.cs[0].kind : 0u, csRow = (numCS && csKind == GENNMI_CS_ARRAY) ? modStep(st.epoch, g.cs[0].arraySteps) : 0u;
     const float csAmp = numCS ? g.cs[0].amp : 0.0f;
     GLOBAL_AS const float *csArray = numCS ? asGlobal(g.cs[0].array) : nullptr;
@@ -644,33 +647,45 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
 
     float l0[NPL], l1[NPL], lin[NPL][BULK_MAX_PSM], front[NPL][BULK_MAX_PSM], inj[NPL];
     bool spiked[NPL];
-    // ---- every input of every chunk first
+    // ---- every input of every chunk first.  What is uniform is decided once for all chunks, so that a launch runs through few instructions (see AnyNeurons); a
+    // lane beyond the population reads its last neuron and keeps nothing of it.
+    uint32_t ids[NPL];
     #pragma unroll
     for(int j = 0; j < NPL; j++) {
-        const uint32_t i = first + j * WAVE;
-        const size_t bi = (size_t)batch * n + i;
+        ids[j] = min(first + j * WAVE, n - 1);
         l0[j] = l1[j] = inj[j] = 0.0f;
         #pragma unroll
         for(uint32_t m = 0; m < BULK_MAX_PSM; m++) { lin[j][m] = front[j][m] = 0.0f; }
-        spiked[j] = false;
-        if(i < n) {
-            if(source) {
-                l0[j] = asGlobal(nextSpikeTime)[bi];
-            }
-            else {
-                l0[j] = var0[bi]; l1[j] = var1[bi];
+    }
+    const size_t batchBase = (size_t)batch * n;
+    if(source) {
+        #pragma unroll
+        for(int j = 0; j < NPL; j++) { l0[j] = asGlobal(nextSpikeTime)[batchBase + ids[j]]; }
+    }
+    else {
+        #pragma unroll
+        for(int j = 0; j < NPL; j++) { l0[j] = var0[batchBase + ids[j]]; l1[j] = var1[batchBase + ids[j]]; }
+        #pragma unroll
+        for(uint32_t m = 0; m < BULK_MAX_PSM; m++) {
+            if(m < numPSM) {
                 #pragma unroll
-                for(uint32_t m = 0; m < BULK_MAX_PSM; m++) {
-                    if(m < numPSM) {
-                        lin[j][m] = psmOut[m][bi];
-                        const uint32_t D = psmD[m];
-                        if(D) { front[j][m] = psmRing[m][((size_t)batch * D + modStep(st.epoch + 1, D)) * n + i]; }
-                    }
-                }
-                if(numCS) {
-                    inj[j] = (csKind == GENNMI_CS_DC) ? csAmp : csArray[(size_t)csRow * n + i];
+                for(int j = 0; j < NPL; j++) { lin[j][m] = psmOut[m][batchBase + ids[j]]; }
+                const uint32_t D = psmD[m];
+                if(D) {
+                    GLOBAL_AS const float *slot = psmRing[m] + ((size_t)batch * D + ringSlot[m]) * n;
+                    #pragma unroll
+                    for(int j = 0; j < NPL; j++) { front[j][m] = slot[ids[j]]; }
                 }
             }
+        }
+        if(csKind == GENNMI_CS_ARRAY && numCS) {
+            GLOBAL_AS const float *row = csArray + (size_t)csRow * n;
+            #pragma unroll
+            for(int j = 0; j < NPL; j++) { inj[j] = row[ids[j]]; }
+        }
+        else {
+            #pragma unroll
+            for(int j = 0; j < NPL; j++) { inj[j] = csAmp; }
         }
     }
     // ---- update, chunk by chunk (operations and their order as in neuronBody); results stay in registers until the block's
@@ -678,40 +693,37 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
     // behind the store traffic of the whole chip before it can vote would keep them waiting
     float outLin[NPL][BULK_MAX_PSM];
     uint32_t newStart[NPL];
-    #pragma unroll
-    for(int j = 0; j < NPL; j++) {
-        const uint32_t i = first + j * WAVE;
-        const size_t bi = (size_t)batch * n + i;
-        newStart[j] = 0;
+    auto update = [&](auto model) {
+        PlainNeuron neuron = constants;
+        neuron.model = model.value;
         #pragma unroll
-        for(uint32_t m = 0; m < BULK_MAX_PSM; m++) { outLin[j][m] = 0.0f; }
-        if(i >= n) { continue; }
-        if(source) {
-            spiked[j] = (t >= l0[j]);
-            if(spiked[j]) { newStart[j] = startSpikeArr[bi] + 1; }
-            continue;
-        }
-        float Isyn = 0;
-        #pragma unroll
-        for(uint32_t m = 0; m < BULK_MAX_PSM; m++) {
-            if(m < numPSM) {
-                float linSyn = lin[j][m];
-                const uint32_t D = psmD[m];
-                if(D) { linSyn += front[j][m]; }
-                if(psmKind[m] == GENNMI_PSM_EXPCURR) {
-                    Isyn += psmInit[m] * linSyn;
-                    linSyn *= psmDecay[m];
+        for(int j = 0; j < NPL; j++) {
+            float Isyn = 0;
+            #pragma unroll
+            for(uint32_t m = 0; m < BULK_MAX_PSM; m++) {
+                outLin[j][m] = 0.0f;
+                if(m < numPSM) {
+                    float linSyn = lin[j][m];
+                    const uint32_t D = psmD[m];
+                    if(D) { linSyn += front[j][m]; }
+                    const bool exponential = (psmKind[m] == GENNMI_PSM_EXPCURR);
+                    Isyn += exponential ? psmInit[m] * linSyn : linSyn;
+                    outLin[j][m] = exponential ? linSyn * psmDecay[m] : 0.0f;
                 }
-                else {
-                    Isyn += linSyn;
-                    linSyn = 0.0f;
-                }
-                outLin[j][m] = linSyn;
             }
+            if(numCS) { Isyn += inj[j]; }
+            spiked[j] = plainNeuronStep(neuron, Isyn, dt, l0[j], l1[j]) && first + j * WAVE < n;
         }
-        if(numCS) { Isyn += inj[j]; }
-        spiked[j] = plainNeuronStep(constants, Isyn, dt, l0[j], l1[j]);
+    };
+    if(source) {
+        #pragma unroll
+        for(int j = 0; j < NPL; j++) {
+            spiked[j] = (t >= l0[j]) && first + j * WAVE < n;
+            newStart[j] = spiked[j] ? startSpikeArr[batchBase + ids[j]] + 1 : 0u;
+        }
     }
+    else if(constants.model == GENNMI_NEURON_LIF) { update(std::integral_constant<uint32_t, GENNMI_NEURON_LIF>()); }
+    else { update(std::integral_constant<uint32_t, GENNMI_NEURON_IZHIKEVICH>()); }
 
     // ---- ordered compaction: rank = spikes of the wave's earlier chunks + spikes of lower lanes in this chunk
     uint32_t rank[NPL];
@@ -758,7 +770,7 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
         for(uint32_t m = 0; m < BULK_MAX_PSM; m++) {
             if(m < numPSM) {
                 const uint32_t D = psmD[m];
-                if(D) { storeThrough(&psmRing[m][((size_t)batch * D + modStep(st.epoch + 1, D)) * n + i], 0.0f); }
+                if(D) { storeThrough(&psmRing[m][((size_t)batch * D + ringSlot[m]) * n + i], 0.0f); }
                 // (an input that is the same bits as it was read — a DeltaCurr input that received nothing: zero in, zero out —
                 // is not written again: in a quiet step that is most of a population's 4 bytes per neuron)
                 if(__float_as_uint(outLin[j][m]) != __float_as_uint(lin[j][m])) { storeThrough(&psmOut[m][bi], outLin[j][m]); }
