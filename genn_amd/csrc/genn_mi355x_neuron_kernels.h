@@ -204,20 +204,22 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
 // What the populations of a launch may have.  A launch fetches its instructions anew, and a path that jumps over what a population does not have fetches a
 // little of each; an instance without it is 840 to 1,200 instructions instead of 5,400 to 6,300.  us a launch, AnyNeurons / LeanNeurons: 4,000 LIF neurons 4.57 / 4.16,
 // 17,011 4.92 / 4.52, 100,000 5.72 / 5.44, 300,007 6.02 / 5.68; stepFusedKernel on the microcircuit at 0.35 with Poisson sources, AnyNeurons / RingNeurons 6.60 / 6.00.
+// OWN: the path reads what it needs of the descriptor at once and its inputs without a branch, instead of a dozen trips to the scalar cache in between: 17,011
+// neurons 4.52 -> 4.27, the others no change.
 struct AnyNeurons       // whatever a description can say
 {
     static constexpr uint32_t PSM = GENNMI_MAX_PSM, CS = GENNMI_MAX_CS;
-    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = true;     // dendritic delays; sources other than DC; shadow queues and zero delays; events, presynaptic output, axonal delays
+    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = true, OWN = false;     // dendritic delays; sources other than DC; shadow queues and zero delays; events, presynaptic output, axonal delays
 };
 struct LeanNeurons      // few inputs without delays, at most a constant current
 {
     static constexpr uint32_t PSM = 4, CS = 1;
-    static constexpr bool RINGS = false, SOURCES = false, SHADOW = false, REST = false;
+    static constexpr bool RINGS = false, SOURCES = false, SHADOW = false, REST = false, OWN = true;
 };
 struct RingNeurons      // the single-launch step's
 {
     static constexpr uint32_t PSM = 2, CS = 1;
-    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = false;
+    static constexpr bool RINGS = true, SOURCES = true, SHADOW = true, REST = false, OWN = false;
 };
 template<typename HAS>
 inline bool neuronsFit(const std::vector<NeuronGroupDev> &groups)
@@ -240,18 +242,22 @@ inline bool neuronsFit(const std::vector<NeuronGroupDev> &groups)
 // emitted spikes, and the last block of each population (which stores spkCnt), look back.
 // ------------------------------------------------------------------------------------------------
 template<typename HAS, bool DIRECT = true>
-__device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
+__device__ __forceinline__ void neuronBody(const NeuronGroupDev &descriptor, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                            const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
     __shared__ uint32_t shWaveCount[BLOCK / WAVE];
     __shared__ uint32_t shPrefix;
 
+    // (OWN: what the path needs of the descriptor is read at its beginning, at once, instead of where it is needed)
+    typename std::conditional<HAS::OWN, const NeuronGroupDev, const NeuronGroupDev&>::type G = descriptor;
     const gennmi_neuron_update_group_t &g = G.g;
     const uint32_t batch = blockIdx.y;
     const uint32_t localBlock = blockInKernel - G.startBlock;
     const uint32_t n = g.numNeurons;
     const uint32_t i = localBlock * BLOCK + threadIdx.x;
-    const size_t bi = (size_t)batch * n + i;
+    // (a lane beyond the population reads its last neuron and keeps nothing of it)
+    const bool present = (i < n);
+    const size_t bi = (size_t)batch * n + (HAS::OWN ? min(i, n - 1) : i);
     const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint32_t wave = threadIdx.x / WAVE;
     const float t = st.t;
@@ -267,7 +273,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     uint32_t ringSlot[MAX_PSM];
     #pragma unroll
     for(uint32_t m = 0; m < MAX_PSM; m++) { lin[m] = 0.0f; }
-    if(i < n) {
+    if(HAS::OWN || present) {
         // order of operations: neuronUpdateGroupMerged.cc:552-773 — PSMs, current sources, sim code,
         // WU pre/post dynamics, threshold, then (on a spike) WU pre/post spike code, sT, reset
         float nextTime = 0.0f;
@@ -356,6 +362,7 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
         if(g.model == GENNMI_NEURON_LIF) { spiked = (l1 <= 0.0f && l0 >= g.params[4]); }
         else if(g.model == GENNMI_NEURON_IZHIKEVICH) { spiked = (l0 >= 29.99f); }
         else { spiked = (t >= nextTime); }       // startSpike != endSpike && t >= spikeTimes[startSpike] (neuronModels.h:274-286)
+        spiked = spiked && present;
         vEvent = l0;           // spike-like event conditions see the updated V before any reset (neuronUpdateGroupMerged.cc:677-683)
         if(spiked) {
             preTrace += 1.0f; postTrace += 1.0f;
@@ -521,9 +528,12 @@ __device__ __forceinline__ void neuronBody(const NeuronGroupDev &G, uint32_t blo
     if(last && threadIdx.x == 0) { g.spkCnt[queue] = prefix + blockCount; }
     // further copies of the queue (one population can feed several spike arrays: its own outgoing projections
     // and, for learnPost, the incoming plastic ones; runtime.cc:267-278)
-    for(uint32_t q = 0; q < g.numExtraSpk; q++) {
-        if(spiked) { g.extraSpk[q][(size_t)batch * n + prefix + waveOffset + laneRank] = i; }
-        if(last && threadIdx.x == 0) { g.extraSpkCnt[q][batch] = prefix + blockCount; }
+    #pragma unroll
+    for(uint32_t q = 0; q < GENNMI_MAX_EXTRA_SPK; q++) {
+        if(q < g.numExtraSpk) {
+            if(spiked) { g.extraSpk[q][(size_t)batch * n + prefix + waveOffset + laneRank] = i; }
+            if(last && threadIdx.x == 0) { g.extraSpkCnt[q][batch] = prefix + blockCount; }
+        }
     }
     if(HAS::SHADOW && G.shadowSpk) {
         const uint32_t parity = (uint32_t)(st.epoch & 1);
