@@ -25,6 +25,7 @@
 #include <string>
 
 #include "genn_mi355x.h"
+#define GENNMI_ROWS_THROUGHPUT
 #include "genn_mi355x_rows.h"
 
 namespace gennmi_detail

@@ -20,6 +20,31 @@ struct Words { uint32_t w[4]; };
 
 __host__ __device__ inline uint32_t mulHi(uint32_t a, uint32_t b) { return (uint32_t)(((unsigned long long)a * b) >> 32); }
 
+// Where a kernel has wavefronts enough its instructions bound it: the initialisation unit asks for one per product both halves of which are wanted, and one per
+// two exclusive ors (GENNMI_ROWS_THROUGHPUT; the compiler makes two of each).  10^8 calls by 2048 work-groups 213 us, 142 so; targets and weights of 10^8 synapses, us:
+// 213 -> 186 and 139 -> 105, a network's unloading, description and load 1,200 -> 1,160.  The kernels of a step have few wavefronts and keep the compiler's form (10^6
+// neurons with procedural rows, 20 steps: 406 us, 426 so).
+#if defined(__HIP_DEVICE_COMPILE__) && defined(GENNMI_ROWS_THROUGHPUT)
+__host__ __device__ inline Words philox4x32(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1)
+{
+    auto product = [](uint32_t a, uint32_t b) { uint64_t p = (uint64_t)a * b; asm("" : "+v"(p)); return p; };
+    auto xor3 = [](uint32_t a, uint32_t b, uint32_t c) { return (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, c, 0x96); };
+    #pragma unroll
+    for(int round = 0; round < 10; round++) {
+        // (counters differ between lanes in c0, most in nothing else: what depends on the others alone is left to the scalar unit)
+        const uint64_t p0 = (round == 1) ? (uint64_t)0xD2511F53u * c0 : product(0xD2511F53u, c0);
+        const uint64_t p1 = (round == 0) ? (uint64_t)0xCD9E8D57u * c2 : product(0xCD9E8D57u, c2);
+        const uint32_t hi0 = (uint32_t)(p0 >> 32), hi1 = (uint32_t)(p1 >> 32);
+        c0 = (round == 0) ? hi1 ^ c1 ^ k0 : xor3(hi1, c1, k0);
+        c1 = (uint32_t)p1;
+        c2 = xor3(hi0, c3, k1);
+        c3 = (uint32_t)p0;
+        k0 += 0x9E3779B9u;
+        k1 += 0xBB67AE85u;
+    }
+    return Words{{c0, c1, c2, c3}};
+}
+#else
 __host__ __device__ inline Words philox4x32(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1)
 {
     #pragma unroll
@@ -35,6 +60,7 @@ __host__ __device__ inline Words philox4x32(uint32_t c0, uint32_t c1, uint32_t c
     }
     return Words{{c0, c1, c2, c3}};
 }
+#endif
 
 // One of four values by an index the compiler does not know.  Indexing an array does the same through memory: the compiler puts the
 // array into scratch or, where it can, into 16 KB of LDS, and every access waits for it.
