@@ -47,6 +47,11 @@ __device__ __forceinline__ uint32_t modStep(unsigned long long x, uint32_t d)
 {
     return __builtin_expect((x >> 32) != 0, 0) ? (uint32_t)(x % d) : ((uint32_t)x % d);
 }
+// (the resident kernel's, which goes through it once a launch and has its loop laid out by the compiler's own guess: 1,000 steps of 4,000 neurons 2,436 us so, 2,448 with the other)
+__device__ __forceinline__ uint32_t modStepOnce(unsigned long long x, uint32_t d)
+{
+    return (x >> 32) ? (uint32_t)(x % d) : ((uint32_t)x % d);
+}
 
 // Synapses whose dendritic delay is a multiple of the ring depth land in the slot the target reads in
 // the very step that delivers them.  When a runner handles them in the neuron update (see

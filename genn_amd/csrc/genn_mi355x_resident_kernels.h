@@ -251,11 +251,11 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         }
         shProjIdx[below + before] = (uint8_t)tid;
         const uint32_t D = shProj[tid].D;
-        for(uint32_t e = 1; e <= 2; e++) { shProjPtr[(seqBase + e) & 3][tid] = D ? modStep(epoch0 + e, D) * TILE : 0u; }
+        for(uint32_t e = 1; e <= 2; e++) { shProjPtr[(seqBase + e) & 3][tid] = D ? modStepOnce(epoch0 + e, D) * TILE : 0u; }
     }
     // (lane p < numProj of the last wavefront, which prepares what the exchange after the next needs) front slot of projection p's ring then
     const uint32_t ptrDepth = (wave == WAVES - 1 && lane < numProj) ? max(1u, shProj[lane].D) : 1u;
-    uint32_t ptrNext = modStep(epoch0 + 3, ptrDepth);
+    uint32_t ptrNext = modStepOnce(epoch0 + 3, ptrDepth);
 
     // ---- state: neuron variables in registers, inSyn in registers (in LDS where synapses add to it) and ring slices in LDS
     float l0 = 0, l1 = 0;
@@ -279,7 +279,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         psmExp[m] = inVector(exponential ? 1u : 0u); psmRing[m] = inVector(D ? D * TILE : 0u);
         psmInit[m] = inVector(exponential ? g.psm[m].init : 1.0f); psmDecay[m] = inVector(exponential ? g.psm[m].expDecay : 0.0f);
         // this neuron's element of the slot the coming step reads, and one beyond the last slot's; without a ring inSyn itself, in LDS
-        psmAt[m] = on ? (D ? T.ldsRing[m] + modStep(epoch0 + 1, D) * TILE : T.ldsIn[m]) + tid : 0u;
+        psmAt[m] = on ? (D ? T.ldsRing[m] + modStepOnce(epoch0 + 1, D) * TILE : T.ldsIn[m]) + tid : 0u;
         psmEnd[m] = on ? (D ? T.ldsRing[m] + D * TILE : T.ldsIn[m] + 1u) + tid : 0u;
         lin[m] = (on && mine) ? asGlobal(g.psm[m].outPost)[i] : 0.0f;
     }
@@ -824,7 +824,7 @@ void residentKernel(const ResTile * __restrict__ tiles, uint32_t numTiles, const
         for(uint32_t slot = 0; slot < D; slot++) {
             if(mine) { asGlobal(g.psm[m].denDelay)[(size_t)slot * n + i] = lds[T.ldsRing[m] + slot * TILE + tid]; }
         }
-        if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStep(epochEnd, D); }
+        if(tileInGroup == 0 && tid == 0 && D && g.psm[m].denDelayPtr) { *g.psm[m].denDelayPtr = modStepOnce(epochEnd, D); }
     }
     uint32_t offset = (watching && watchSub == 0 && !(grouped && (lane & (RES_MAX_QUADS - 1)) != 0) && watchTile >= T.firstTileOfGroup && watchTile < T.firstTileOfGroup + tileInGroup) ? spikesOf() : 0u;
     if(tid == 0) { shScalar[2] = 0; }
