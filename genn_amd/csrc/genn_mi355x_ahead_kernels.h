@@ -13,8 +13,8 @@
 //   4. aheadQueueKernel: the spike queues as the last step leaves them, in ascending neuron index.
 // What the next step, of whichever plan, finds is what step-by-step execution leaves: state, queues, recording rows, next spike times.
 //
-// run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 182 us;
-// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 865 us, of which 500 move 26 MB between host and device.
+// run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 178 us;
+// Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 795 us, of which 500 move 26 MB between host and device.
 #pragma once
 
 namespace
