@@ -1333,8 +1333,6 @@ static auto convStepInstance(const gennmi_runner *r) { return r->convQueuesDirec
 // Many steps of a feed-forward layer per launch: possible when the model is a spike source array, one DENSE or Conv2D projection and the
 // plain population it feeds, so that no spike ever comes back.
 constexpr size_t AHEAD_MAX_SPACE = 512ull << 20;        // of the layer's input over the steps of a launch
-// A work-group of the convolution takes no more output rows than leave two of them to a compute unit; a single row may take a little more.
-constexpr size_t AHEAD_ROWS_LDS = 64 * 1024, AHEAD_MAX_LDS = 82 * 1024;
 // Runs (and remainders of runs) shorter than this are stepped one by one: a pass costs a good part of a pass of 32 steps however few it is given.  us
 // at once / one by one for 5 and for 8 steps: Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, at 20 %, 2.5 % and 0.25 % activity 187 / 173 and
 // 211 / 268, 97 / 164 and 110 / 251, 76 / 159 and 81 / 244; 40x40x16 -> 40x40x4 5x5, batch 16, at 0.25 % 87 / 143 and 91 / 223; DENSE 8192 x 8192
@@ -1364,19 +1362,11 @@ static int setupAhead(gennmi_runner *r, uint32_t numCU)
     if(conv) {
         const int32_t *c = p.conv;
         AheadConv &C = r->aheadConv;
-        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 1u};
-        C.rowPitch = (uint32_t)(c[6] - 1 + c[1]) * (uint32_t)c[4];
-        const uint32_t inputs = (uint32_t)(c[0] * c[1] * c[4]);
-        // as many output rows per work-group as leave four work-groups to a compute unit
-        const uint64_t rowsInAll = (uint64_t)c[5] * r->batch * (((uint32_t)c[7] + 31) / 32);
-        C.rowsPerBlock = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)c[5], rowsInAll / (4 * numCU)));
-        size_t ldsBytes = 0;        // (the lists of steps, up to 7 KiB more, change neither how many fit: 64 KiB and 82)
-        for(;; C.rowsPerBlock--) {
-            ldsBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)inputs * 32 + (size_t)(inputs + 1) / 2 + (size_t)(BLOCK / WAVE) * 2 * (inputs + 1)) * sizeof(uint32_t);
-            r->aheadConvBytes = ((size_t)(C.rowsPerBlock + c[0] - 1) * C.rowPitch + (size_t)(inputs + 1) * 32 + (size_t)(inputs + 1) / 2) * sizeof(uint32_t) + (size_t)(BLOCK / WAVE) * aheadConvListBytes(inputs);
-            if(ldsBytes <= AHEAD_ROWS_LDS || C.rowsPerBlock == 1) { break; }
-        }
-        if(ldsBytes > AHEAD_MAX_LDS || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
+        C = AheadConv{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[0] - 1 - r->pre[0].convBH, c[1] - 1 - r->pre[0].convBW, 0u, 0u, 0u, 1u};
+        const AheadConvLayout layout = aheadConvLayout(c[0], c[1], c[4], c[5], c[6], c[7], r->batch, numCU);
+        if(!layout.fits || ((uint32_t)c[7] + 31) / 32 > 65535) { return GENNMI_OK; }
+        C.rowsPerBlock = layout.rowsPerBlock; C.rowPitch = layout.rowPitch; C.listDepth = layout.listDepth;
+        r->aheadConvBytes = layout.bytes;
         if(r->aheadConvBytes > 48 * 1024) {
             HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(aheadConvInstance(g)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)r->aheadConvBytes));
         }

@@ -16,10 +16,11 @@
 // run() with its launches, copies and waits, one by one -> at once: DENSE 8192 -> 8192 at 5 % activity, 100 steps: 1107 -> 178 us;
 // Conv2D 64x64x16 -> 64x64x32 3x3, batch 16, 2.5 %, 50 steps: 2125 -> 795 us, of which 500 move 26 MB between host and device.
 #pragma once
+#include "genn_mi355x_ahead_layout.h"
 
 namespace
 {
-constexpr uint32_t AHEAD_MAX_STEPS = 128, AHEAD_WORD = 32;      // steps per pass over the source; steps per word (rows of a product)
+constexpr uint32_t AHEAD_MAX_STEPS = 128;                       // steps per pass over the source
 constexpr uint32_t AHEAD_DENSE_THREADS = 512, AHEAD_DENSE_WAVES = AHEAD_DENSE_THREADS / WAVE, AHEAD_TILE_COPIES = 4;
 
 struct AheadArgs
@@ -32,28 +33,9 @@ struct AheadArgs
 struct AheadConv
 {
     int32_t kh, kw, ih, iw, ic, oh, ow, oc, PH, PW;
-    uint32_t rowsPerBlock, rowPitch;                    // patch row in words
+    uint32_t rowsPerBlock, rowPitch, listDepth;         // see AheadConvLayout
     uint32_t isConv;
 };
-
-// bytes of a wavefront's lists: of a pixel's active inputs, all of them and what fills the last pair; or of the active inputs of its two pixels in each of
-// 32 steps, 16 bits each
-constexpr uint32_t AHEAD_CONV_MOST = 16;
-__host__ __device__ constexpr uint32_t aheadConvListBytes(uint32_t inputs)
-{
-    const uint32_t pixel = (8u * (inputs + 1u) + 15u) / 16u * 16u, steps = 2u * AHEAD_WORD * AHEAD_CONV_MOST * 2u;
-    return (pixel > steps) ? pixel : steps;
-}
-// How many inputs of a pixel may have a spike in a step for its sum to be made one by one, by how many of a patch's words have spikes and how many those have (of
-// the steps of a launch).  0: sums are products throughout.  (The line's figures: aheadConvKernel.)
-__host__ __device__ constexpr uint32_t aheadConvMost(uint32_t inputs, uint32_t steps, uint32_t active, uint32_t spikes, uint32_t words)
-{
-    // (above 511 a weight's place does not fit the list's 16 bits)
-    const uint32_t most = (inputs > 511u) ? 0u : (inputs / 16u * 4u < AHEAD_CONV_MOST) ? inputs / 16u * 4u : AHEAD_CONV_MOST;
-    const unsigned long long all = words, spikesOfAll = (unsigned long long)spikes * inputs;
-    const bool few = (32u * spikesOfAll <= 13u * most * steps * all), worth = (8ull * inputs * active > all * (4u * steps + 25u * ((inputs + 31u) / 32u)) + spikesOfAll);
-    return (few && worth) ? most : 0u;
-}
 
 __device__ __forceinline__ size_t aheadRecordingRow(const AheadArgs &A, uint32_t step) { return (size_t)((A.timestep + step) % A.recordingRows); }
 
@@ -561,9 +543,11 @@ private:
 // other instead, in the same order and so with the same bits: the words of 32 inputs, transposed, give each lane one step's, which it lists in LDS, and the
 // pixel's lanes add up the weights listed for step after step, four at a time.  A product of two inputs is 64 clocks of the matrix unit whatever they hold;
 // a listed weight is two or three vector instructions, so the rule (aheadConvMost) compares 48 clocks an active input with 48 a step, 300 a transposed word and 6 a
-// spike, and leaves patches of more than 6.5 spikes a pixel and step (a list holds 16; one that is full means products for its two pixels) to the products.
+// spike, and leaves to the products patches of more spikes a pixel and step than 13/32 of what a list holds (6.5 where it holds 16; one that is full means products
+// for its two pixels).  A list holds a quarter of the inputs, 16 at most, and no more than leaves a compute unit its work-groups (aheadConvLayout).
 // run() of 50 steps, products only -> now, at 0.5 / 2.5 / 10 / 30 / 75 %: 64x64x16 -> 32 3x3 batch 16 196 / 308 / 440 / 540 / 687 -> 197 / 235 / 440 / 540 / 687; 48x48x3 ->
-// 20 5x5 batch 8 90 / 116 / 145 / 164 / 172 -> 89 / 108 / 144 / 164 / 172; 40x37x16 -> 4 5x5 batch 16, 24x24x16 -> 32 5x5 batch 4, 64x64 from one channel, 33x47x2: no change.
+// 20 5x5 batch 8 90 / 116 / 145 / 164 / 172 -> 89 / 108 / 144 / 164 / 172; 40x37x16 -> 4 5x5 batch 16, 24x24x16 -> 32 5x5 batch 4, 64x64 from one channel, 33x47x2: no change; 64x72x16 -> 32 3x3
+// batch 16, at 0.5 / 2.5 / 10 / 30 %, lists of 12: 206 / 329 / 500 / 620 -> 205 / 253 / 498 / 620.
 template<uint32_t MODEL, uint32_t PSM>
 __global__ __launch_bounds__(BLOCK, 4)
 void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, AheadConv C, uint32_t wordBlock, const uint32_t * __restrict__ words,
@@ -579,12 +563,13 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     AheadNeuron<MODEL, PSM> neuron(g, A.dt);
     asm volatile("" : "+v"(neuron.constants.p[5]), "+v"(neuron.constants.p[6]));       // (selected between in every step: from scalar registers that is a copy first)
     const uint32_t rowPitch = C.rowPitch, rowWords = (uint32_t)(C.kw * C.ic), inputs = (uint32_t)C.kh * rowWords;
-    uint8_t *lists = reinterpret_cast<uint8_t*>(shAhead) + wave * aheadConvListBytes(inputs);
+    const uint32_t depth = C.listDepth, quads = depth / 4, listBytes = aheadConvListBytes(inputs, depth), zeroRow = depth ? 1u : 0u;
+    uint8_t *lists = reinterpret_cast<uint8_t*>(shAhead) + wave * listBytes;
     uint2 *list = reinterpret_cast<uint2*>(lists);                                                  // (word, byte of its weights) of a pixel's active inputs
-    uint16_t *stepList = reinterpret_cast<uint16_t*>(lists);                                        // [pixel][step][AHEAD_CONV_MOST] bytes of weights
-    float *kern = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(shAhead) + (BLOCK / WAVE) * aheadConvListBytes(inputs));     // [input][32], one more of zeros
-    uint16_t *place = reinterpret_cast<uint16_t*>(kern + (inputs + 1) * 32);                        // [input] its word behind the pixel's first
-    uint32_t *patch = reinterpret_cast<uint32_t*>(kern + (inputs + 1) * 32) + (inputs + 1) / 2;
+    uint16_t *stepList = reinterpret_cast<uint16_t*>(lists);                                        // [pixel][step][depth] bytes of weights
+    float *kern = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(shAhead) + (BLOCK / WAVE) * listBytes);     // [input][32], with lists of steps one more of zeros
+    uint16_t *place = reinterpret_cast<uint16_t*>(kern + (inputs + zeroRow) * 32);                        // [input] its word behind the pixel's first
+    uint32_t *patch = reinterpret_cast<uint32_t*>(kern + (inputs + zeroRow) * 32) + (inputs + 1) / 2;
     // ---- the patch: row r, word e is word e - PW * ic of input row y0 - PH + r
     GLOBAL_AS const uint32_t *in = asGlobal(words) + ((size_t)wordBlock * A.batch + batch) * ((size_t)C.ih * C.iw * C.ic);
     const int inRowWords = C.iw * C.ic;
@@ -603,7 +588,7 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     __shared__ uint32_t seen[2][BLOCK / WAVE];
     if(lane == 0) { seen[0][wave] = active; seen[1][wave] = spiked; }
     bool nonFinite = false;
-    for(uint32_t e = threadIdx.x; e < (inputs + 1) * 32; e += BLOCK) {
+    for(uint32_t e = threadIdx.x; e < (inputs + zeroRow) * 32; e += BLOCK) {
         const uint32_t k = e / 32, oo = blockIdx.z * 32 + (e & 31);
         float weight = (oo < oc && k < inputs) ? asGlobal(kernel)[(size_t)k * oc + oo] : 0.0f;
         if(!aheadFinite(weight)) { nonFinite = true; weight = 0.0f; }
@@ -624,7 +609,7 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
     // (of the patch's words those that are input: a work-group at the edge has no more to add up for most of its pixels than any other)
     const int firstRow = max((int)y0 - C.PH, 0), endRow = min((int)(y0 + rows) + C.kh - 1 - C.PH, C.ih), firstWord = max(C.PW * C.ic, 0), endWord = min(C.PW * C.ic + inRowWords, (int)rowPitch);
     const uint32_t inputWords = (uint32_t)max(endRow - firstRow, 0) * (uint32_t)max(endWord - firstWord, 0);
-    const uint32_t most = nonFinite ? 0u : aheadConvMost(inputs, steps, active, spiked, inputWords);
+    const uint32_t most = nonFinite ? 0u : aheadConvMost(depth, inputs, steps, active, spiked, inputWords);
     const Transpose32 transposed(lane);
     auto listSteps = [&](uint32_t pixel, uint32_t &count) -> bool {
         auto word = [&](uint32_t k) -> uint32_t {
@@ -633,10 +618,9 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
         };
         uint32_t bits = word(col), following = word(32 + col);
         bits = transposed(bits);
-        uint16_t *mine = stepList + lane * AHEAD_CONV_MOST;
+        uint16_t *mine = stepList + lane * depth;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        #pragma unroll
-        for(uint32_t q = 0; q < AHEAD_CONV_MOST / 4; q++) { reinterpret_cast<u32x2*>(mine)[q] = u32x2{inputs * 0x800080u, inputs * 0x800080u}; }
+        for(uint32_t q = 0; q < quads; q++) { reinterpret_cast<u32x2*>(mine)[q] = u32x2{inputs * 0x800080u, inputs * 0x800080u}; }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         for(uint32_t k0 = 0; ; ) {
             if(__ballot(count + __popc(bits) > most)) {
@@ -685,7 +669,7 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
                 const unsigned long long ballot = __ballot(count > 4 * q);
                 more[q] = (uint32_t)ballot | (uint32_t)(ballot >> 32);
             }
-            const u32x2 *mine = reinterpret_cast<const u32x2*>(stepList + half * AHEAD_WORD * AHEAD_CONV_MOST);
+            const u32x2 *mine = reinterpret_cast<const u32x2*>(stepList + half * AHEAD_WORD * depth);
             auto load = [&](u32x2 four, float w[4]) {
                 w[0] = *reinterpret_cast<const float*>(weights + (four[0] & 0xFFFFu)); w[1] = *reinterpret_cast<const float*>(weights + (four[0] >> 16));
                 w[2] = *reinterpret_cast<const float*>(weights + (four[1] & 0xFFFFu)); w[3] = *reinterpret_cast<const float*>(weights + (four[1] >> 16));
@@ -694,12 +678,12 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
             constexpr uint32_t GROUP = 4;
             float w[GROUP][4], next[GROUP][4];
             #pragma unroll
-            for(uint32_t u = 0; u < GROUP; u++) { load(mine[u * (AHEAD_CONV_MOST / 4)], w[u]); }
+            for(uint32_t u = 0; u < GROUP; u++) { load(mine[u * quads], w[u]); }
             #pragma unroll 1
             for(uint32_t t0 = 0; t0 < steps; t0 += GROUP) {
                 const uint32_t ahead = min(t0 + GROUP, AHEAD_WORD - GROUP);
                 #pragma unroll
-                for(uint32_t u = 0; u < GROUP; u++) { load(mine[(ahead + u) * (AHEAD_CONV_MOST / 4)], next[u]); }
+                for(uint32_t u = 0; u < GROUP; u++) { load(mine[(ahead + u) * quads], next[u]); }
                 __builtin_amdgcn_sched_barrier(0);
                 #pragma unroll
                 for(uint32_t u = 0; u < GROUP; u++) {
@@ -709,7 +693,7 @@ void aheadConvKernel(const NeuronGroupDev * __restrict__ target, AheadArgs A, Ah
                     for(uint32_t q = 1; q < AHEAD_CONV_MOST / 4; q++) {
                         if(!((more[q] >> t) & 1u)) { break; }
                         float x[4];
-                        load(mine[t * (AHEAD_CONV_MOST / 4) + q], x);
+                        load(mine[t * quads + q], x);
                         input = (((input + x[0]) + x[1]) + x[2]) + x[3];
                     }
                     step(t, input);

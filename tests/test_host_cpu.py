@@ -3,6 +3,7 @@ import ctypes as C
 import math
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -155,3 +156,41 @@ def test_max_row_length_follows_the_snippets():
             assert max_row_length("FixedProbability", {"prob": prob}, size, size) == stride
     assert max_row_length("FixedNumberPostWithReplacement", {"num": 37}, 100, 100) == 37
     assert max_row_length("OneToOne", {}, 100, 100) == 1
+
+
+def test_lists_of_a_convolution_cost_no_work_group(tmp_path):
+    """A layer of a feed-forward network lists its steps' inputs in LDS only where as many work-groups stay on a compute unit as without the lists, or as the
+    launch has: four by their registers, and by 160 KiB of LDS in parts of 1,280 bytes.  Which layers are taken, and their rows, do not depend on the lists."""
+    (tmp_path / "layout.cc").write_text("""#include "genn_mi355x_ahead_layout.h"
+extern "C" void layout(const int *c, unsigned batch, unsigned units, unsigned long long *out)
+{
+    const AheadConvLayout l = aheadConvLayout(c[0], c[1], c[2], c[3], c[4], c[5], batch, units);
+    out[0] = l.fits; out[1] = l.rowsPerBlock; out[2] = l.listDepth; out[3] = l.bytes;
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "genn_amd", "csrc"), "-o", str(tmp_path / "layout.so"), str(tmp_path / "layout.cc")], check=True)
+    layout = C.CDLL(str(tmp_path / "layout.so")).layout
+
+    def resident(size):
+        return min(4, 163840 // (-(-(size + 288) // 1280) * 1280))
+
+    units, listed, shallower = 256, 0, 0
+    shapes = [(64, w, 8, 32, 5, 16) for w in range(36, 44)] + [(64, 72, 16, 32, 3, 16), (16, 16, 9, 32, 5, 16), (64, 64, 1, 32, 3, 16), (64, 64, 16, 32, 3, 16)]
+    shapes += [(h, w, ic, oc, k, b) for h, w in ((5, 7), (33, 47), (64, 64), (200, 31)) for ic in (1, 2, 3, 5, 8, 13, 16, 20, 40, 60) for oc, b in ((1, 1), (33, 2), (64, 16), (1056, 3)) for k in (1, 3, 5)]
+    for h, w, ic, oc, k, b in shapes:
+        out = (C.c_ulonglong * 4)()
+        layout((C.c_int * 6)(k, k, ic, h, w, oc), b, units, out)
+        fits, rows, depth, size = out
+        inputs, columns = k * k * ic, b * (-(-oc // 32))
+        bare = lambda r: 4 * ((r + k - 1) * (w - 1 + k) * ic + 32 * inputs + (inputs + 1) // 2 + 8 * (inputs + 1))
+        most = max(1, min(h, h * columns // (4 * units)))
+        while bare(most) > 65536 and most > 1:
+            most -= 1
+        assert (bool(fits), rows) == (bare(most) <= 83968, most), (h, w, ic, oc, k, b)
+        if not fits:
+            continue
+        needed = -(-(-(-h // rows) * columns) // units)
+        assert resident(size) >= min(needed, resident(bare(rows))), (h, w, ic, oc, k, b, depth, size)
+        assert depth % 4 == 0 and depth <= min(16, inputs // 16 * 4) and (depth or size == bare(rows)) and size >= 4 * 128 * depth and inputs * 128 < 65536
+        listed, shallower = listed + (depth != 0), shallower + (depth < min(16, inputs // 16 * 4))
+    assert listed > 100 and shallower > 5
