@@ -613,7 +613,10 @@ __device__ __forceinline__ bool plainNeuronStep(const PlainNeuron &c, float Isyn
 // (THREADS: threads of the calling work-group, all of which call; batch / numBatches: the grid's second dimension in the neuron kernels)
 // (LEAN: no population is a spike source or has dendritic delays; see AnyNeurons.  1,650 instructions for four chunks instead of 2,660, and of 5,850 while what is
 // uniform was decided chunk by chunk: 10^6 Izhikevich neurons 8.8 -> 7.8 us a launch with LEAN alone, 6.8 with straight loads and one decision besides)
-template<int NPL, int THREADS = BLOCK, bool DIRECT = true, bool LEAN = false>
+// (STRAIGHT: a chunk's spiking sources are looked up without a branch, so that a lane's chunks do not wait for one another: a step of a convolution 64x64x16 -> 32,
+// batch 16, whose neurons have a kernel of their own, 38.6 us -> 31.3 with eight chunks, 30.3 -> 29.4 with four, 37.2 -> 36.2 with two; 1.4 x 10^6 neurons with delays, eight chunks,
+// 25.8 -> 22.4.  The convolution's one-launch step, whose other work-groups wait for memory as well, is slower with it: 28.3 -> 29.4)
+template<int NPL, int THREADS = BLOCK, bool DIRECT = true, bool LEAN = false, bool STRAIGHT = false>
 __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t blockInKernel, uint32_t totalNeuronBlocks,
                                                const StepArgs &st, float dt, unsigned long long *agg, uint32_t *errorFlag,
                                                uint32_t batch, uint32_t numBatches)
@@ -729,7 +732,8 @@ __device__ __forceinline__ void neuronBulkBody(const NeuronGroupDev &G, uint32_t
         #pragma unroll
         for(int j = 0; j < NPL; j++) {
             spiked[j] = (t >= l0[j]) && first + j * WAVE < n;
-            newStart[j] = spiked[j] ? startSpikeArr[batchBase + ids[j]] + 1 : 0u;
+            if(STRAIGHT) { newStart[j] = asGlobal(startSpikeArr)[batchBase + (spiked[j] ? ids[j] : ids[0])] + 1; }
+            else { newStart[j] = spiked[j] ? startSpikeArr[batchBase + ids[j]] + 1 : 0u; }
         }
     }
     else if(constants.model == GENNMI_NEURON_LIF) { update(std::integral_constant<uint32_t, GENNMI_NEURON_LIF>()); }
@@ -807,7 +811,7 @@ template<int NPL, bool LEAN>
 __global__ __launch_bounds__(BLOCK)
 void neuronBulkKernel(const NeuronGroupDev * __restrict__ blocks, StepArgs args, float dt, unsigned long long *agg, uint32_t *errorFlag)
 {
-    neuronBulkBody<NPL, BLOCK, true, LEAN>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag, blockIdx.y, gridDim.y);
+    neuronBulkBody<NPL, BLOCK, true, LEAN, true>(blocks[blockIdx.x], blockIdx.x, gridDim.x, args, dt, agg, errorFlag, blockIdx.y, gridDim.y);
 }
 
 // One launch per timestep for networks whose projections all go through the dendritic-delay ring: the
