@@ -1176,7 +1176,8 @@ class GeNNModel:
         return {"single_launch_step": bool(info[0] & 1), "resident_plan": bool(info[0] & 2), "bulk_neuron_kernel": bool(info[0] & 4), "ordered_accumulation": bool(info[0] & 8),
                 "combined_synapse_launch": bool(info[0] & 16), "postsynaptic_in_combined_launch": bool(info[0] & 32),
                 "conv_on_matrix_cores": bool(info[0] & 64), "conv_step_in_one_launch": bool(info[0] & 128),
-                "feed_forward_ahead": bool(info[0] & 256), "resident_walkers": bool(info[0] & 512), "resident_quads": (info[0] >> 12) & 15,
+                "feed_forward_ahead": bool(info[0] & 256), "resident_walkers": bool(info[0] & 512), "lean_neuron_kernel": bool(info[0] & 1024),
+                "narrow_synapse_kernel": bool(info[0] & 2048), "resident_quads": (info[0] >> 12) & 15,
                 "resident_tile": info[0] >> 16, "neuron_blocks": info[1], "presyn_blocks": info[2], "postsyn_blocks": info[3]}
 
     # timing counters under PyGeNN's names (pygenn/genn_model.py:292-326), in seconds, accumulated while `timing_enabled`
