@@ -2236,7 +2236,7 @@ static int launchNeurons(gennmi_runner *r, const StepArgs &a, bool timed);
 
 static int launchFusedStep(gennmi_runner *r, const StepArgs &a)
 {
-    const auto kernel = r->ringNeurons ? stepFusedKernel<RingNeurons, DelayRows> : stepFusedKernel<AnyNeurons, DelayRows>;
+    const auto kernel = r->ringNeurons ? stepFusedKernel<RingNeurons, DelayRows> : stepFusedKernel<AnyNeurons, AnyRows>;     // (see stepFusedKernel)
     kernel<<<dim3(r->neuronBlocks + r->preBlocks, r->batch), dim3(BLOCK), 0, r->stream>>>(
         r->dNeuron, r->neuronBlocks, r->dPre, a, r->dt, r->dAgg, r->dError, r->dEvents);
     HIP_TRY(hipGetLastError());
@@ -2583,7 +2583,7 @@ int gennmi_runner_get_info(gennmi_runner *r, uint32_t info[4])
     if(!r->finalised) { return fail(GENNMI_ESTATE, "runner_get_info: runner not finalised"); }
     // (of the kernels that step a network in one launch or in two)
     const bool lean = r->fusedStep ? r->ringNeurons : (r->neuronsPerLane > 1) ? r->leanBulk : r->leanNeurons;
-    const bool narrow = r->fusedStep || (r->combineSynapses && (r->staticRows || r->plasticRows));
+    const bool narrow = r->fusedStep ? r->ringNeurons : (r->combineSynapses && (r->staticRows || r->plasticRows));
     info[0] = (r->fusedStep ? 1u : 0u) | (r->resident ? 2u : 0u) | (r->neuronsPerLane > 1 ? 4u : 0u) | (r->ordered ? 8u : 0u)
               | (r->combineSynapses ? 16u : 0u) | ((r->combineSynapses && r->combinePost) ? 32u : 0u) | (r->convMfmaBlocks ? 64u : 0u) | (r->convStep ? 128u : 0u) | (r->ahead ? 256u : 0u) | (lean ? 1024u : 0u) | (narrow ? 2048u : 0u)
               | (r->resident ? (r->resThreads > r->resTileSize ? 512u : 0u) | (r->resQuads << 12) | (r->resTileSize << 16) : 0u); info[1] = r->neuronBlocks; info[2] = r->preBlocks; info[3] = r->postBlocks;

@@ -131,3 +131,14 @@ def test_batches_of_spike_sources_and_few_inputs(n_src, n_trg):
     for b, oracle in enumerate(oracles):
         assert np.array_equal(v[b], oracle.var("T", 0))
     model.unload()
+
+
+@pytest.mark.parametrize("inputs,sources", [(3, ()), (2, ("dc", "noise")), (1, ("dc", "dc")), (8, ("noise",))])
+def test_single_launch_steps_of_more_inputs_or_sources(inputs, sources):
+    """What the lean neuron instance of the single-launch step does not take runs beside the synapse code for everything: the instance for delayed rows
+    alone made such a step up to 8 % longer."""
+    model, _, counts = run_side_by_side(_net(inputs, sources, D))
+    info = model.runner_info()
+    assert info["single_launch_step"] and not info["lean_neuron_kernel"] and not info["narrow_synapse_kernel"]
+    assert counts["S"] > 0 and counts["T"] > 0
+    model.unload()
