@@ -1538,9 +1538,11 @@ int gennmi_runner_finalise(gennmi_runner *r)
             plain = plain && g.numPSM <= BULK_MAX_PSM && g.numCS <= BULK_MAX_CS && !g.preTrace && !g.postTrace && !g.sT && g.numExtraSpk == 0
                     && g.numDelaySlots <= 1 && g.numSpkEvent == 0 && g.numPreOutput == 0;
         }
-        // measured: four per lane from one round of work-groups up (10^6 Izhikevich neurons: 20.1 us with one, 18.0 with two,
-        // 16.4 with four), eight beyond five rounds (3.1 x 10^6 lanes of the batched convolution layer: 57 / 38 / 29 / 24 us
-        // with one / two / four / eight); GENNMI_NEURON_BULK = 0 (never), 2, 4 or 8 forces the choice
+        // Four per lane from one round of work-groups up, eight beyond five rounds: the lines of a kernel for several neurons that took twice as long as today's (10^6
+        // Izhikevich neurons 20.1 / 18.0 / 16.4 us with one / two / four a lane, 3.1 x 10^6 lanes of the batched convolution layer 57 / 38 / 29 / 24 with eight).  Today's, us with
+        // one / two / four / eight: Izhikevich neurons with noise, 3 x 10^6 34.8 / 23.2 / 18.1 / 16.8, 10^6 14.2 / 6.8 / 6.6 / 7.4, 600,000 9.9 / 5.9 / 5.8 / 6.7; LIF neurons with two inputs,
+        // 600,000 8.1 / 6.8 / 6.1 / 6.9; the convolution layer's lanes in a kernel of their own 29.3 / 16.2 / 13.2 / 15.9.  The first line could lie lower (300,007 Izhikevich neurons 6.4 / 4.7 / 5.0 /
+        // 5.9, LIF 5.8 / 5.2 / 5.2 / 6.0; 17,011 LIF neurons 4.2 / 4.0 / 4.6 / 5.5).  GENNMI_NEURON_BULK = 0 (never), 2, 4 or 8 forces the choice
         const unsigned long long round = 1ull * numCU * 8 * BLOCK;
         uint32_t perLane = (lanes <= round) ? 1u : (2 * lanes <= 5 * round) ? 4u : 8u;
         if(const char *envBulk = getenv("GENNMI_NEURON_BULK")) {

@@ -202,10 +202,13 @@ __device__ __forceinline__ void appendOrdered(bool flag, uint32_t id, uint32_t l
 }
 
 // What the populations of a launch may have.  A launch fetches its instructions anew, and a path that jumps over what a population does not have fetches a
-// little of each; an instance without it is 840 to 1,200 instructions instead of 5,400 to 6,300.  us a launch, AnyNeurons / LeanNeurons: 4,000 LIF neurons 4.57 / 4.16,
+// little of each; neuronUpdateKernel is 5,430 and 6,380 instructions (DIRECT) with AnyNeurons, 845 and 1,250 with LeanNeurons.  us a launch, AnyNeurons / LeanNeurons: 4,000 LIF neurons 4.57 / 4.16,
 // 17,011 4.92 / 4.52, 100,000 5.72 / 5.44, 300,007 6.02 / 5.68; stepFusedKernel on the microcircuit at 0.35 with Poisson sources, AnyNeurons / RingNeurons 6.60 / 6.00.
 // OWN: the path reads what it needs of the descriptor at once and its inputs without a branch, instead of a dozen trips to the scalar cache in between: 17,011
 // neurons 4.52 -> 4.27, the others no change.
+// The lines, us a step of two launches / of one: LeanNeurons for eight inputs costs networks with two of them, 17,011 neurons 7.4 -> 7.5, 300,007 11.8 -> 13.0 (and what has five 17,011 8.3 -> 7.6,
+// 200,000 11.2 -> 12.2), for four sources 11.8 -> 12.4 (two constant currents, 17,011 8.1 -> 7.4); RingNeurons for four inputs 77,000 neurons with Poisson sources 8.2 -> 8.4 (three inputs
+// 8.4 -> 8.3, 27,000 6.8 -> 6.5), for four sources nothing (two sources 10,007 6.2 -> 6.0, 50,021 7.5 -> 7.2, 77,000 the same).
 struct AnyNeurons       // whatever a description can say
 {
     static constexpr uint32_t PSM = GENNMI_MAX_PSM, CS = GENNMI_MAX_CS;
@@ -611,7 +614,7 @@ __device__ __forceinline__ bool plainNeuronStep(const PlainNeuron &c, float Isyn
 }
 
 // (THREADS: threads of the calling work-group, all of which call; batch / numBatches: the grid's second dimension in the neuron kernels)
-// (LEAN: no population is a spike source or has dendritic delays; see AnyNeurons.  1,650 instructions for four chunks instead of 2,660, and of 5,850 while what is
+// (LEAN: no population is a spike source or has dendritic delays; see AnyNeurons.  1,660 instructions for four chunks instead of 2,690, and of 5,890 while what is
 // uniform was decided chunk by chunk: 10^6 Izhikevich neurons 8.8 -> 7.8 us a launch with LEAN alone, 6.8 with straight loads and one decision besides)
 // (STRAIGHT: a chunk's spiking sources are looked up without a branch, so that a lane's chunks do not wait for one another: a step of a convolution 64x64x16 -> 32,
 // batch 16, whose neurons have a kernel of their own, 38.6 us -> 31.3 with eight chunks, 30.3 -> 29.4 with four, 37.2 -> 36.2 with two; 1.4 x 10^6 neurons with delays, eight chunks,

@@ -13,6 +13,10 @@
 
 namespace gennmi_rows
 {
+#if defined(GENNMI_ROWS_THROUGHPUT)
+inline namespace throughput         // (what calls the generator's other form goes by another name)
+{
+#endif
 constexpr int WAVE = 64;
 
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw: "Parallel random numbers: as easy as 1, 2, 3", SC'11)
@@ -23,7 +27,7 @@ __host__ __device__ inline uint32_t mulHi(uint32_t a, uint32_t b) { return (uint
 // Where a kernel has wavefronts enough its instructions bound it: the initialisation unit asks for one per product both halves of which are wanted, and one per
 // two exclusive ors (GENNMI_ROWS_THROUGHPUT; the compiler makes two of each).  10^8 calls by 2048 work-groups 213 us, 142 so; targets and weights of 10^8 synapses, us:
 // 213 -> 186 and 139 -> 105, a network's unloading, description and load 1,200 -> 1,160.  The kernels of a step have few wavefronts and keep the compiler's form (10^6
-// neurons with procedural rows, 20 steps: 406 us, 426 so).
+// neurons with procedural rows, 20 steps: 406 us, 426 so).  Both forms are the same ten rounds, and the same words.
 #if defined(__HIP_DEVICE_COMPILE__) && defined(GENNMI_ROWS_THROUGHPUT)
 __host__ __device__ inline Words philox4x32(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1)
 {
@@ -401,6 +405,9 @@ __device__ __forceinline__ bool fixedNumberPostRowBlock(uint32_t row, uint32_t n
     __syncthreads();            // roundTotal is reused by the next row
     return true;
 }
+#if defined(GENNMI_ROWS_THROUGHPUT)
+}
+#endif
 }   // namespace gennmi_rows
 
 #endif

@@ -361,7 +361,7 @@ void presynapticDenseKernel(const DenseGroupDev * __restrict__ blocks, unsigned 
 // ------------------------------------------------------------------------------------------------
 // PROCEDURAL connectivity (the reference's PostSpan/PreSpan procedural strategies, presynapticUpdateStrategySIMT.cc:391-560,
 // re-run the connectivity snippet with a per-row generator state).  Here a wavefront regenerates the row of a spiking
-// neuron with exactly the code and draws the initialisation kernels use (genn_mi355x_rows.h), so a procedural projection
+// neuron with the draws of the initialisation kernels (genn_mi355x_rows.h), so a procedural projection
 // behaves synapse for synapse like the stored matrix the same seed would have produced — without reading a byte of
 // connectivity: the only memory traffic of an event is its atomic.
 // What bounds it is the chain of arithmetic that makes a row (generator, logarithms, scan, division).  Nothing in it may index a
