@@ -36,24 +36,28 @@ BYTES_PER_EVENT = {"dense": 4,          # one weight read per (spike, target); o
 # produced them in profiles/<kernel>_<workload>.md.  A counter run is a separate invocation of this script, so the figure
 # is only attached to a run of the very command line it was measured on (same workload, steps and warm-up: the network,
 # its seed and therefore its activity are then identical); any other run reports null.
-# The kernel's source is named with a digest: a figure measured on another version of the kernel is not attached.
+# The files that a kernel's code comes from are named with a digest: a figure measured on another version of them is not attached.
 MEASURED_TRAFFIC_BYTES = {
-    ("potjans", 20, 5): {"plan": "resident", "bytes_per_launch": 172079712,
-                         "kernel_source": ("genn_amd/csrc/genn_mi355x_resident_kernels.h", "03cc94d209a8d753"),
-                         "source": "rocprofv3 --pmc FETCH_SIZE (76117.31 x 2 KiB) + WRITE_SIZE (15811.97 x 1 KiB) of the timed 20-step "
+    ("potjans", 20, 5): {"plan": "resident", "bytes_per_launch": 171992965,
+                         "kernel_source": (("resident_kernels", "device"), "a5e8ada1b523d856"),
+                         "source": "rocprofv3 --pmc FETCH_SIZE (76074.94 x 2 KiB) + WRITE_SIZE (15812.00 x 1 KiB) of the timed 20-step "
                                    "launch, profiles/residentKernel_potjans_full.md"},
-    ("conv", 1000, 100): {"plan": "stepped", "requires": "conv_step_in_one_launch", "bytes_per_launch": 66118287,
-                          "kernel_source": ("genn_amd/csrc/genn_mi355x_conv_step_kernels.h", "b33aec4cfae473d9"),
-                          "source": "rocprofv3 --pmc FETCH_SIZE (18888.04 x 2 KiB) + WRITE_SIZE (26792.56 x 1 KiB), average over the "
-                                    "run's 1,100 launches, profiles/convStepKernel_conv_batch16.md"},
+    ("conv", 1000, 100): {"plan": "stepped", "requires": "conv_step_in_one_launch", "bytes_per_launch": 65796803,
+                          "kernel_source": (("conv_step_kernels", "neuron_kernels", "synapse_kernels", "device"), "d1bca87f7214890f"),
+                          "source": "rocprofv3 --pmc FETCH_SIZE (18734.37 x 2 KiB) + WRITE_SIZE (26785.95 x 1 KiB), average over the "
+                                    "1,100 launches of a run with GENNMI_AHEAD=0, profiles/convStepKernel_conv_batch16.md"},
 }
 FP32_MFMA_PEAK_TFLOPS = 157.3
 
 
-def source_digest(path):
+def source_digest(headers):
+    """Of the kernel headers of these names together."""
     import hashlib
-    with open(os.path.join(ROOT, path), "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()[:16]
+    digest = hashlib.sha256()
+    for name in headers:
+        with open(os.path.join(ROOT, "genn_amd", "csrc", f"genn_mi355x_{name}.h"), "rb") as f:
+            digest.update(f.read())
+    return digest.hexdigest()[:16]
 
 
 def build_net(name, steps):
@@ -357,7 +361,7 @@ def run_net_workload(args, workload, steps, warmup, profile_steps, with_cpu, wit
             roofline["traffic"] = measured["bytes_per_launch"]
             roofline["traffic_source"] = measured["source"]
         else:
-            roofline["traffic_source"] = "not attached: " + measured["kernel_source"][0] + " has changed since the counters were read"
+            roofline["traffic_source"] = "not attached: the kernel's source (" + ", ".join(measured["kernel_source"][0]) + ") has changed since the counters were read"
 
     # ---- the running network: short runs only (see the module docstring)
     steady = None

@@ -194,3 +194,22 @@ extern "C" void layout(const int *c, unsigned batch, unsigned units, unsigned lo
         assert depth % 4 == 0 and depth <= min(16, inputs // 16 * 4) and (depth or size == bare(rows)) and size >= 4 * 128 * depth and inputs * 128 < 65536
         listed, shallower = listed + (depth != 0), shallower + (depth < min(16, inputs // 16 * 4))
     assert listed > 100 and shallower > 5
+
+
+def test_counters_are_attached_to_the_code_they_were_read_on(tmp_path, monkeypatch):
+    """The benchmark's figures of hardware counters go with every file that their kernel's code comes from: the convolution's step has its neurons' update
+    and its products from the other kernel files."""
+    import shutil
+    import bench
+    files = {key: measured["kernel_source"][0] for key, measured in bench.MEASURED_TRAFFIC_BYTES.items()}
+    assert {"conv_step_kernels", "neuron_kernels", "synapse_kernels", "device"} <= set(files["conv", 1000, 100])
+    assert {"resident_kernels", "device"} <= set(files["potjans", 20, 5])
+    shutil.copytree(os.path.join(ROOT, "genn_amd", "csrc"), tmp_path / "genn_amd" / "csrc")
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    for names in files.values():
+        seen = [bench.source_digest(names)]
+        for name in names:
+            with open(tmp_path / "genn_amd" / "csrc" / f"genn_mi355x_{name}.h", "a") as f:
+                f.write("//")
+            seen.append(bench.source_digest(names))
+        assert len(set(seen)) == len(names) + 1
