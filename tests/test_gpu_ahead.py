@@ -390,15 +390,14 @@ def test_dense_layers_of_sources_most_of_which_are_silent(steps, active, monkeyp
     assert got[0][2] == got[1][2] == 70 * end[-1]
 
 
-# 32 and 64 inputs a pixel and numbers off a round of 32, up to what LDS holds, and fewer than 32 (lists of four); two output rows a work-group; few enough spikes for a list of each step, too many, and about as many as the
+# 32 and 64 inputs a pixel and numbers off a round of 32, up to what LDS holds; few enough spikes for a list of each step, too many, and about as many as the
 # rule allows; channels of one product and of two
 @pytest.mark.parametrize("h,w,ic,oc,k,rate", [(9, 11, 16, 32, 3, 0.025), (9, 11, 16, 32, 3, 0.045), (12, 6, 8, 7, 3, 0.04), (10, 9, 7, 34, 3, 0.06), (8, 9, 16, 3, 2, 0.05),
-                                              (7, 7, 13, 5, 5, 0.012), (7, 8, 19, 4, 5, 0.01), (9, 9, 8, 32, 2, 0.05), (11, 33, 4, 33, 5, 0.03),
-                                              (9, 11, 1, 5, 5, 0.06), (9, 11, 2, 32, 3, 0.08), (64, 6, 4, 1056, 3, 0.03)])
+                                              (7, 7, 13, 5, 5, 0.012), (7, 8, 19, 4, 5, 0.01), (9, 9, 8, 32, 2, 0.05), (11, 33, 4, 33, 5, 0.03)])
 @pytest.mark.parametrize("steps", [8, 32, 45])
 def test_sums_of_convolutions_with_few_spikes(h, w, ic, oc, k, rate, steps):
     """A step's sum is that of its inputs' weights in the kernel's order, whichever way it is made: outPost bit for bit as 32-bit sums in that order give it.
-    Two pixels have steps with 15, 16 and 17 inputs (a list holds 16 at most), and one step has no spike at all."""
+    Two pixels have steps with 15, 16 and 17 inputs (a list holds 16), and one step has no spike at all."""
     rng = np.random.default_rng(h * w + steps)
     net = configs.conv_toeplitz(h=h, w=w, ic=ic, oc=oc, k=k, steps=steps, w_sd=0.1, ioffset=0.3)
     fire = rng.random((steps, h, w, ic)) < rate
@@ -433,3 +432,11 @@ def test_sums_of_convolutions_with_few_spikes(h, w, ic, oc, k, rate, steps):
                         sums += np.where(padded[a:a + h, b:b + w, channel, None], kernel[a, b, channel], np.float32(0))
         want = (want + sums) * decay
     assert np.array_equal(got.reshape(want.shape).view(np.uint32), want.view(np.uint32))
+
+
+# fewer than 32 inputs a pixel (lists of four), and two output rows a work-group
+@pytest.mark.parametrize("h,w,ic,oc,k,rate", [(9, 11, 1, 5, 5, 0.06), (9, 11, 2, 32, 3, 0.08), (64, 6, 4, 1056, 3, 0.03)])
+@pytest.mark.parametrize("steps", [8, 32, 45])
+def test_sums_of_convolutions_with_short_lists(h, w, ic, oc, k, rate, steps):
+    """The same where a list holds fewer than 16 inputs."""
+    test_sums_of_convolutions_with_few_spikes(h, w, ic, oc, k, rate, steps)
